@@ -1,85 +1,118 @@
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias) in true float32: float32 products,
-// float32 sums, no matrix-core mode of reduced precision.
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias) in true float32: float32 products, float32 sums (the matrix
+// instructions whose operands are float32), no mode of reduced precision.
 //
-// A 64x64 tile of C per block of 256 threads, each thread a 4x4 patch; K is walked in
-// steps of 16 through LDS.  Every element of C is one accumulator that takes its
-// products in the order k = 0, 1, ..., K-1, so its value does not depend on M, on the
-// tile it falls in or on its row's place in the batch.
+// Every element of C is made in one way, whatever M, its tile or its row's place in the batch: K is cut into
+// chunks of 32; wave w of a block's eight adds up the chunks w, w + 8, ... in order (a chunk is eight
+// 16 x 16 x 4 instructions, of which number j takes the values k + j, k + 8 + j, k + 16 + j, k + 24 + j); the
+// eight sums are added in wave order, then the bias.  So the tile may follow the sizes of a call and the bits
+// do not.
+//
+// A block takes NT x MT tiles of 16 columns x 16 rows of C and all its waves take all of them, each its part
+// of K: the operands go from memory to registers (a lane 32 contiguous bytes, the four lanes of a row 128), a
+// fetched weight meets 16 MT rows and a fetched row 16 NT columns.  Bound by the float32 matrix rate
+// (157 TFLOP/s) from some 30 rows on and by reading W below that.  Against a tile of 64 x 64 through LDS whose
+// threads multiplied and added: 122 rows of 16384 x 2048 262 -> 118 us (70 TFLOP/s), of 2048 x 8192 875 -> 62;
+// 2,048 rows of 16384 x 2048 3.64 -> 1.68 ms (82 TFLOP/s); one row of 16384 x 2048 196 -> 33 us (4.0 TB/s).
 
 #include <hip/hip_runtime.h>
 
 #include "device_utils.h"
+#include "gemm_common.h"
 #include "kvcore_hip.h"
+
+using namespace kvc;
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16;
+constexpr int kWaves = 8;
+constexpr int kChunk = 32;
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ C,
-                                                       const float* __restrict__ A,
-                                                       const float* __restrict__ W,
-                                                       const float* __restrict__ bias, int M,
-                                                       int N, int K, int64_t lda, int64_t ldc) {
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Ws[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid & 15;   // column patch
-  const int ty = tid >> 4;   // row patch
-  const int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
+// Eight values of a row from k on.  VEC: K a multiple of 8 and 16-byte aligned rows, so a lane's eight are in or
+// out as a whole; `whole` (the same for the wave): the chunk lies inside K.
+template <int VEC>
+__device__ __forceinline__ void load8(f32x4_t* v, const float* row, int k, int K, bool whole) {
+  if constexpr (VEC) {
+    const float* p = row + (k < K ? k : 0);
+    v[0] = *reinterpret_cast<const f32x4_t*>(p);
+    v[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
+    if (!whole && k >= K) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = k + i < K ? row[k + i] : 0.f;
+  }
+}
 
-  float acc[4][4];
+template <int NT, int MT, int AHEAD, int VEC>
+__global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict__ C, const float* __restrict__ A,
+                                                               const float* __restrict__ W,
+                                                               const float* __restrict__ bias, int M, int N, int K,
+                                                               int64_t lda, int64_t ldc) {
+  __shared__ f32x4_t part[kWaves][MT][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  // columns and rows beyond the matrix read its last ones and are not stored
+  const float* wp[NT];
+  const float* ap[MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int n = 0; n < NT; ++n) wp[n] = W + static_cast<int64_t>(n0 + 16 * n + li < N ? n0 + 16 * n + li : N - 1) * K;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-  // loader mapping: 256 threads fetch 64 rows x 16 k: thread -> (row = tid / 4, k4 = tid % 4)
-  const int lrow = tid >> 2;
-  const int lk = (tid & 3) * 4;
-
-  for (int k0 = 0; k0 < K; k0 += BK) {
-    float a[4], w[4];
-    const int am = m0 + lrow;
-    const int wn = n0 + lrow;
+  for (int m = 0; m < MT; ++m) ap[m] = A + static_cast<int64_t>(m0 + 16 * m + li < M ? m0 + 16 * m + li : M - 1) * lda;
+  f32x4_t acc[NT][MT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int k = k0 + lk + i;
-      a[i] = (am < M && k < K) ? A[static_cast<int64_t>(am) * lda + k] : 0.f;
-      w[i] = (wn < N && k < K) ? W[static_cast<int64_t>(wn) * K + k] : 0.f;
-    }
-    __syncthreads();
+  for (int n = 0; n < NT; ++n)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      As[lk + i][lrow] = a[i];
-      Ws[lk + i][lrow] = w[i];
-    }
-    __syncthreads();
+    for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int chunks = (K + kChunk - 1) / kChunk;
+  f32x4_t wv[AHEAD][NT][2], av[AHEAD][MT][2];
+  // no branch around the loads: a chunk that is not there is one that reads zeros
+  auto fetch = [&](int slot, int c) {
+    const int k = c * kChunk + 8 * lk;
+    const bool whole = (c + 1) * kChunk <= K;
 #pragma unroll
-    for (int k = 0; k < BK; ++k) {
-      float av[4], wv[4];
+    for (int n = 0; n < NT; ++n) load8<VEC>(wv[slot][n], wp[n], k, K, whole);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = As[k][ty * 4 + i];
+    for (int m = 0; m < MT; ++m) load8<VEC>(av[slot][m], ap[m], k, K, whole);
+  };
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wv[j] = Ws[k][tx * 4 + j];
+  for (int s = 0; s < AHEAD; ++s) fetch(s, wave + kWaves * s);
+  for (int c = wave; c < chunks; c += kWaves * AHEAD) {  // scalar
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int s = 0; s < AHEAD; ++s) {
+      f32x4_t w[NT][2], a[MT][2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
+      for (int n = 0; n < NT; ++n) w[n][0] = wv[s][n][0], w[n][1] = wv[s][n][1];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m][0] = av[s][m][0], a[m][1] = av[s][m][1];
+      fetch(s, c + kWaves * (s + AHEAD));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n][j >> 2][j & 3], a[m][j >> 2][j & 3], acc[n][m], 0, 0, 0);
     }
   }
-
+  // the waves' sums, 16 columns at a time: lane holds row li, columns 4 lk .. of its tiles
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+  for (int n = 0; n < NT; ++n) {
+    if (n > 0) __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float v = acc[i][j];
-      if (bias != nullptr) v += bias[n];
-      C[static_cast<int64_t>(m) * ldc + n] = v;
+    for (int m = 0; m < MT; ++m) part[wave][m][lane] = acc[n][m];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < MT * 64; idx += kWaves * 64) {
+      const int m = idx >> 6, l = idx & 63;
+      f32x4_t v = part[0][m][l];
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w) v += part[w][m][l];
+      const int row = m0 + 16 * m + (l & 15), col = n0 + 16 * n + 4 * (l >> 4);
+      if (row >= M || col >= N) continue;
+      if (bias != nullptr) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += bias[col + i < N ? col + i : N - 1];
+      }
+      store4<float>(C + static_cast<int64_t>(row) * ldc + col, v, N - col);
     }
   }
 }
@@ -90,9 +123,44 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
                             int N, int K, int64_t lda, int64_t ldc, kvc_stream stream) {
   if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N) return kvc_fail("kvc_gemm_f32: bad sizes");
   if (M == 0) return 0;
-  const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+  // tiles of 64 x 64 where they give every compute unit a block, narrower ones otherwise (122 rows of 2048 x 2048
+  // are 64 blocks of 64 x 64 and 256 of 32 x 32); rows in sixteens up to the batch's size
+  const int64_t units = kvc_device_compute_units();
+  int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  if (mt == 4 && M < 256 && (M + 63) / 64 * 64 >= M + 32) mt = 2;  // the last 64 rows would be half empty
+  int nt = 4;
+  auto blocks = [&]() { return static_cast<int64_t>((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt)); };
+  while (blocks() < units && (nt > 1 || mt > 2)) {
+    if (nt >= mt && nt > 1) nt /= 2;
+    else if (mt > 2) mt /= 2;
+    else nt /= 2;
+  }
+  const dim3 grid((N + 16 * nt - 1) / (16 * nt), (M + 16 * mt - 1) / (16 * mt));
   if (grid.y > 65535) return kvc_fail("kvc_gemm_f32: M too large for one launch");
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     C, A, W, bias, M, N, K, lda, ldc);
+  const bool vec = K % 8 == 0 && lda % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
+#define KVC_F32(NT, MT, AHEAD)                                                                                 \
+  do {                                                                                                         \
+    if (vec)                                                                                                   \
+      hipLaunchKernelGGL((gemm_f32_kernel<NT, MT, AHEAD, 1>), grid, dim3(kWaves * 64), 0,                      \
+                         reinterpret_cast<hipStream_t>(stream), C, A, W, bias, M, N, K, lda, ldc);             \
+    else                                                                                                       \
+      hipLaunchKernelGGL((gemm_f32_kernel<NT, MT, 1, 0>), grid, dim3(kWaves * 64), 0,                          \
+                         reinterpret_cast<hipStream_t>(stream), C, A, W, bias, M, N, K, lda, ldc);             \
+  } while (0)
+  if (mt == 4) {
+    if (nt == 4) KVC_F32(4, 4, 1);
+    else if (nt == 2) KVC_F32(2, 4, 1);
+    else KVC_F32(1, 4, 1);
+  } else if (mt == 2) {
+    if (nt == 4) KVC_F32(4, 2, 1);
+    else if (nt == 2) KVC_F32(2, 2, 2);
+    else KVC_F32(1, 2, 2);
+  } else {
+    if (nt == 4) KVC_F32(4, 1, 2);
+    else if (nt == 2) KVC_F32(2, 1, 2);
+    else KVC_F32(1, 1, 4);
+  }
+#undef KVC_F32
   return kvc_check_launch("kvc_gemm_f32");
 }

@@ -442,7 +442,7 @@ int kvc_hyper_step(void* out, int out_dtype, float* streams, const void* y, int 
 int kvc_spread_streams(float* streams, const float* rows, int T, int H, int copies, kvc_stream stream);
 
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float32 with float32 products and sums;
-// each element is one running sum over k = 0..K-1, whatever M is.
+// each element is the sum of eight running sums over fixed parts of K, whatever M is.
 int kvc_gemm_f32(float* C, const float* A, const float* W, const float* bias, int M, int N,
                  int K, int64_t lda, int64_t ldc, kvc_stream stream);
 

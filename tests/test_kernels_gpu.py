@@ -121,6 +121,22 @@ def test_gemm_f32_is_true_float32_and_does_not_depend_on_the_batch(ops, M, N, K)
     assert torch.all(wide_out[:, N:] == 0)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (2, 4100, 2048), (16, 17, 264), (17, 8200, 520), (33, 2048, 1024),
+                                   (65, 515, 2056), (122, 2048, 8192), (122, 16384, 264), (130, 100, 40), (300, 1000, 72)])
+def test_gemm_f32_tiles_give_the_same_bits(ops, M, N, K):
+    """Every tile shape that the sizes choose: the sums of a 64-bit product, and a row's bits as it has them alone."""
+    a, w = rnd(M, K, seed=4), rnd(N, K, seed=5)
+    out = torch.full((M, N), 7.0, device=DEV)
+    ops.gemm_f32(out, a, w, None)
+    # eight chains of K / 8 products each and seven sums: sqrt(K) * 2^-24 of the summed magnitudes, as for one chain
+    bound = 4 * math.sqrt(K) * 2 ** -24 * (a.double().abs() @ w.double().abs().T)
+    assert ((out.double() - a.double() @ w.double().T).abs() <= bound + 1e-7).all()
+    single = torch.empty(1, N, device=DEV)
+    for i in {0, M // 2, M - 1}:
+        ops.gemm_f32(single, a[i:i + 1].contiguous(), w, None)
+        assert torch.equal(single[0], out[i])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (5, 100, 200), (8, 4096, 4096), (16, 130, 1032),
                                    (17, 6144, 512), (33, 48, 14336), (64, 1000, 2048),
                                    # the longest sum and the widest output of the 70B shape
