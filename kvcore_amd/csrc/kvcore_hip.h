@@ -313,8 +313,8 @@ int kvc_head_rmsnorm_gate(void* out, int out_dtype, const float* o, const void* 
 int kvc_moe_route(int32_t* choice, float* weight, const float* logits, int T, int E, int top,
                   int groups, int keep, int score_fn, const float* bias, const float* correction,
                   int group_best, int renormalize, float weight_scale, kvc_stream stream);
-// Tiles hold up to tile_rows rows, 16 or 64 (kvc_moe_tile_rows says which a step's size asks
-// for; 64 is for bfloat16 with K a multiple of 32).
+// Tiles hold up to tile_rows rows, 16, 64 or 128 (kvc_moe_tile_rows says which a step's size asks
+// for; 64 and 128 are for bfloat16 with K a multiple of 32).
 int kvc_moe_tile_rows(int pairs, int E);
 // The router's logits (x [T, H] of x_dtype times router [E, H] float32, float32 sums in one fixed order)
 // and the choice of kvc_moe_route in one kernel.  With gate [T] (may be null) the matrix is [E + 1, H]
@@ -323,6 +323,15 @@ int kvc_moe_router(int32_t* choice, float* weight, const void* x, int64_t x_stri
                    const float* router, float* gate, int T, int H, int E, int top, int groups, int keep,
                    int score_fn, const float* bias, const float* correction, int group_best, int renormalize,
                    float weight_scale, kvc_stream stream);
+// The same and kvc_moe_align for at most kvc_moe_router_spread_tokens() tokens and 64 experts, by kernels that spread
+// the product over the chip; the same bits.  parts: kvc_moe_router_spread_floats(T, E) float32, 16-byte aligned.
+int kvc_moe_router_spread_tokens(void);
+int kvc_moe_router_spread_floats(int T, int E);
+int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32_t* tiles, int32_t* num_tiles,
+                       int max_tiles, int tile_rows, float* parts, int64_t parts_floats, const void* x,
+                       int64_t x_stride, int x_dtype, const float* router, float* gate, int T, int H, int E,
+                       int top, int groups, int keep, int score_fn, const float* bias, const float* correction,
+                       int group_best, int renormalize, float weight_scale, kvc_stream stream);
 int kvc_moe_max_tiles(int pairs, int E, int tile_rows);
 int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
                   int pairs, int E, int max_tiles, int tile_rows, kvc_stream stream);

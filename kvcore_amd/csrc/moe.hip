@@ -16,8 +16,9 @@
 //   kvc_moe_router   the router's product (float32 sums in one fixed order over rows of either dtype)
 //                    and the choice in one kernel; a further row of the router's matrix may give one
 //                    number a token, a sigmoid gate for an expert that every token runs.
+//   kvc_moe_router_spread  the same and kvc_moe_align in kernels that spread the product over the chip.
 //   kvc_moe_align    pairs sorted by expert: sorted[i] = pair index (token * top + choice), and a
-//                    list of tiles of up to 16 (or 64) sorted rows that belong to one expert each.
+//                    list of tiles of up to 16 (or 64, or 128) sorted rows that belong to one expert each.
 //   kvc_moe_gemm     for every tile, rows x that expert's matrix.  Gated: gate and up rows of the
 //                    expert side by side in one pass, and the activation
 //                    min(g, limit) * sigmoid(alpha * g) * (clamp(u, -limit, limit) + up_shift) on the way
@@ -44,7 +45,8 @@ namespace {
 #define S(stream) reinterpret_cast<hipStream_t>(stream)
 
 constexpr int kTileRows = 16;
-constexpr int kBigTileRows = 64;
+constexpr int kMidTileRows = 64;
+constexpr int kBigTileRows = 128;
 
 // What happens to the sums of an ungated product on their way out (the codes of kvc_activation; -1: nothing).
 __device__ __forceinline__ float plain_act(float v, int act) {
@@ -184,6 +186,88 @@ __device__ __forceinline__ void route_one(int32_t* __restrict__ choice, float* _
   }
 }
 
+// The same choice for at most 64 experts, one a lane (`z`: the lane's logit, lanes beyond E anything): an expert's
+// place among the choices is the number of experts that come before it, counted against each in turn, so no
+// wave-wide maximum has to be found choice by choice.
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ void route_lanes(int32_t* choice, float* weight, float z, int lane, int E, const RouteRule& rule) {
+  const int top = rule.top, groups = rule.groups, keep = rule.keep;
+  const bool live = lane < E;
+  const int le = live ? lane : 0;
+  if (rule.bias != nullptr) z += rule.bias[le];
+  float sc = 0.f;
+  if (rule.score_fn == 0) {
+    const float mx = wave_max(live ? z : -INFINITY);
+    const float p = live ? expf(z - mx) : 0.f;
+    sc = p * (1.f / wave_sum(p));
+  } else if (rule.score_fn == 1) {
+    sc = 1.f / (1.f + expf(-z));
+  } else {
+    sc = z;
+  }
+  float pk = live ? sc + (rule.correction != nullptr ? rule.correction[le] : 0.f) : -INFINITY;
+  if (keep < groups) {  // the same for the whole grid
+    const int per = E / groups;
+    const int base = lane < groups ? lane * per : 0;
+    float best = -INFINITY, second = -INFINITY;  // lane g: of group g
+    for (int i = 0; i < per; ++i) {
+      const float s = __shfl(pk, base + i, kWave);
+      if (s > best) {
+        second = best;
+        best = s;
+      } else if (s > second) {
+        second = s;
+      }
+    }
+    const float worth = (rule.group_best >= 2 && per >= 2) ? best + second : best;
+    int before = 0;
+    for (int g = 0; g < groups; ++g) {
+      const float s = lane_value(worth, g);
+      before += s != INFINITY && (s > worth || (s == worth && g < lane));
+    }
+    const int kept = lane < groups && (worth == INFINITY || (worth == worth && before < keep));
+    if (!__shfl(kept, le / per, kWave)) pk = -INFINITY;  // choice scores may be negative: minus infinity, not zero
+  }
+  int before = 0;
+#pragma unroll 8
+  for (int e = 0; e < E; ++e) {
+    const float s = lane_value(pk, e);
+    before += s > pk || (s == pk && e < lane);
+  }
+  const bool allowed = live && pk > -INFINITY;  // not for a score that is no number
+  const int count = __popcll(__ballot(allowed));
+  const uint64_t numbers = __ballot(live && pk == pk);
+  const int spare = numbers ? __ffsll(static_cast<unsigned long long>(numbers)) - 1 : 0;
+  float total = 0.f, mine = 0.f;  // lane c keeps the c-th choice's score
+  int mine_idx = 0;
+  bool mine_ok = false;
+  for (int c = 0; c < top; ++c) {  // scalar
+    // fewer allowed experts than choices: a weight of zero
+    const bool ok = c < count;
+    const uint64_t who = __ballot(allowed && before == c);
+    const int idx = ok && who ? __ffsll(static_cast<unsigned long long>(who)) - 1 : spare;
+    const float plain = ok ? lane_value(sc, idx) : 0.f;
+    total += plain;
+    if (lane == c) {
+      mine = plain;
+      mine_idx = idx;
+      mine_ok = ok;
+    }
+  }
+  float norm = rule.renormalize ? rule.weight_scale / (total + 1e-20f) : rule.weight_scale;
+  if (rule.score_fn == 2) {  // the softmax over the chosen logits alone
+    const float mx = wave_max(mine_ok ? mine : -INFINITY);
+    mine = mine_ok ? expf(mine - mx) : 0.f;
+    norm = rule.weight_scale / wave_sum(mine);
+  }
+  if (lane < top) {
+    choice[lane] = mine_idx;
+    weight[lane] = mine * norm;
+  }
+}
+
 __global__ __launch_bounds__(256) void moe_route_kernel(int32_t* __restrict__ choice, float* __restrict__ weight,
                                                         const float* __restrict__ logits, int T, int E,
                                                         RouteRule rule) {
@@ -192,8 +276,11 @@ __global__ __launch_bounds__(256) void moe_route_kernel(int32_t* __restrict__ ch
   float* sc = lds + wave * (2 * E + rule.groups);  // scores, choice scores, then the groups' worth
   const int t = blockIdx.x * 4 + wave;
   if (t >= T) return;  // the whole wave
-  route_one(choice + static_cast<int64_t>(t) * rule.top, weight + static_cast<int64_t>(t) * rule.top,
-            logits + static_cast<int64_t>(t) * E, sc, sc + E, sc + 2 * E, lane, E, rule);
+  int32_t* ct = choice + static_cast<int64_t>(t) * rule.top;
+  float* wt = weight + static_cast<int64_t>(t) * rule.top;
+  const float* zt = logits + static_cast<int64_t>(t) * E;
+  if (E <= kWave) route_lanes(ct, wt, zt[lane < E ? lane : 0], lane, E, rule);  // the same for the whole grid
+  else route_one(ct, wt, zt, sc, sc + E, sc + 2 * E, lane, E, rule);
 }
 
 // The router whole: logits = x W^T with float32 products and sums (x of either dtype, its values as
@@ -315,20 +402,20 @@ __global__ __launch_bounds__(kRouterWaves * 64) void moe_router_kernel(
     gate[t] = 1.f / (1.f + expf(-sum));
   }
   float* zr = z + wave * zrow;
-  route_one(choice + static_cast<int64_t>(t) * rule.top, weight + static_cast<int64_t>(t) * rule.top, zr, zr, zr + E,
-            zr + 2 * E, lane, E, rule);
+  int32_t* ct = choice + static_cast<int64_t>(t) * rule.top;
+  float* wt = weight + static_cast<int64_t>(t) * rule.top;
+  if (E <= kWave) route_lanes(ct, wt, zr[lane < E ? lane : 0], lane, E, rule);  // the same for the whole grid
+  else route_one(ct, wt, zr, zr, zr + E, zr + 2 * E, lane, E, rule);
 }
 
-// One block.  counts -> offsets and tiles (a thread an expert, which adds up the counts before its own)
-// -> sorted pairs.
-__global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
-                                                         int32_t* __restrict__ num_tiles,
-                                                         const int32_t* __restrict__ choice, int pairs, int E,
-                                                         int max_tiles, int tile_rows) {
-  extern __shared__ int32_t ilds[];
+// One block.  counts -> offsets and tiles (a thread an expert) -> sorted pairs.  `ilds`: [4 E] in LDS.
+__device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
+                                            int32_t* __restrict__ num_tiles, const int32_t* choice, int pairs, int E,
+                                            int max_tiles, int tile_rows, int32_t* ilds) {
   int32_t* count = ilds;           // [E]
   int32_t* offset = count + E;     // [E]
   int32_t* cursor = offset + E;    // [E]
+  int32_t* ntiles = cursor + E;    // [E]
   for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
@@ -336,20 +423,52 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ s
     if (e >= 0 && e < E) atomicAdd(&count[e], 1);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < E; e += blockDim.x) {
-    int at = 0, nt = 0;
-    for (int p = 0; p < e; ++p) {
-      at += count[p];
-      nt += (count[p] + tile_rows - 1) / tile_rows;
-    }
+  // an expert's rows in as few tiles as hold them, all of about one size (in sixteens): no tile is left with a few
+  const int shift = 31 - __clz(tile_rows);
+  auto rows_each = [&](int n) {
+    const int tiles_of = (n + tile_rows - 1) >> shift;
+    return tiles_of < 2 ? tile_rows : ((n + tiles_of - 1) / tiles_of + 15) & ~15;
+  };
+  auto list = [&](int e, int n, int each, int at, int nt) {
     offset[e] = at;
     cursor[e] = 0;
-    for (int r = 0; r < count[e] && nt < max_tiles; r += tile_rows, ++nt) {
+    for (int r = 0; r < n && nt < max_tiles; r += each, ++nt) {
       tiles[3 * nt] = e;
       tiles[3 * nt + 1] = at + r;
-      tiles[3 * nt + 2] = (count[e] - r < tile_rows) ? count[e] - r : tile_rows;
+      tiles[3 * nt + 2] = (n - r < each) ? n - r : each;
     }
     if (e == E - 1) *num_tiles = nt;
+  };
+  if (E <= kWave) {  // a lane an expert: running sums over the lanes
+    if (threadIdx.x < kWave) {
+      const int e = threadIdx.x;
+      const int n = e < E ? count[e] : 0;
+      const int each = rows_each(n), mine = (n + each - 1) / each;
+      int at = n, nt = mine;
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int pa = __shfl_up(at, o, kWave), pt = __shfl_up(nt, o, kWave);
+        if (e >= o) {
+          at += pa;
+          nt += pt;
+        }
+      }
+      if (e < E) list(e, n, each, at - n, nt - mine);
+    }
+  } else {
+    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+      const int each = rows_each(count[e]);
+      ntiles[e] = (count[e] + each - 1) / each;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+      int at = 0, nt = 0;
+      for (int p = 0; p < e; ++p) {
+        at += count[p];
+        nt += ntiles[p];
+      }
+      list(e, count[e], rows_each(count[e]), at, nt);
+    }
   }
   __syncthreads();
   // an expert's pairs take their places in the order in which their threads arrive: a row's sums
@@ -362,28 +481,164 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ s
   }
 }
 
-// bfloat16: a block of four waves takes one tile of rows and 64 columns (16 a wave).  A pass covers
-// 64 values along K: lane (li, lk) fetches the 16 values from 16 lk of its weight row and of its
-// token row (32 contiguous bytes, so that the four lanes of a row read one 128-byte line) and the two
-// matrix instructions of the pass take its first and its second eight (both operands are dealt the
-// same way, so each product still sums over all of K); the values of the next two passes are asked for
-// before this pass's products.
+__global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
+                                                         int32_t* __restrict__ num_tiles,
+                                                         const int32_t* __restrict__ choice, int pairs, int E,
+                                                         int max_tiles, int tile_rows) {
+  extern __shared__ int32_t ilds[];
+  align_pairs(sorted, tiles, num_tiles, choice, pairs, E, max_tiles, tile_rows, ilds);
+}
+
+// The router spread over the chip (at most kRouterSpread tokens and 64 experts), with the arrangement of its pairs.
+// One block reads its 260 KB of router and rows at what a compute unit draws (50 GB/s), so the sixteen parts of K
+// that moe_router_kernel's waves take go to as many blocks here, which leave their sums in `parts` [16][T][row]
+// (the gate's behind the experts'); they are added in the same order by the wave that chooses for a token.  Up to
+// kChooseInOne tokens the block that lists the tiles chooses too, a token a wave; with more of them a choice costs
+// that one compute unit 0.3 us a token, so a kernel of its own deals the tokens out.  With 32 experts and rows of
+// 2,048, 8 tokens 26.4 -> 12.6 us (router and tiles together), 64 tokens
+// 23.8 -> 15.7, 300 tokens 23.6 -> 15.7; 2,030 tokens fill the chip either way (27.2 and 26.5).
+constexpr int kRouterSpread = 1024;
+constexpr int kChooseInOne = 16;
+__host__ __device__ __forceinline__ int router_part_row(int E) { return ((E + 3) & ~3) + 4; }
+
+template <typename T, int VEC>
+__global__ __launch_bounds__(64) void moe_router_parts_kernel(float* __restrict__ parts, const T* __restrict__ x,
+                                                              int64_t x_stride, const float* __restrict__ wr,
+                                                              int with_gate_row, int T_, int H, int E) {
+  constexpr int NT = kRouterRows / 16;
+  const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+  const int part = blockIdx.y, e0 = blockIdx.z * kRouterRows, t0 = blockIdx.x * kRouterTokens;
+  const T* xr = x + static_cast<int64_t>(t0 + li < T_ ? t0 + li : T_ - 1) * x_stride;  // rows beyond are dropped
+  const int ne = (E - e0 < kRouterRows) ? E - e0 : kRouterRows;
+  const bool with_gate = with_gate_row && e0 == 0;
+  const float* wp[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) wp[n] = wr + static_cast<int64_t>(e0 + (16 * n + li < ne ? 16 * n + li : 0)) * H;
+  const float* wg = wr + static_cast<int64_t>(with_gate ? E : e0) * H;
+  f32x4_t acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float acc_g = 0.f;
+  constexpr int kAhead = 2;  // pieces on their way
+  float xn[kAhead][8], wn[kAhead][NT][8], gn[kAhead][8];
+  auto fetch = [&](int slot, int k) {  // no branch around the loads: a piece beyond H reads the row's last values
+    router_load<VEC>(xr, k + 8 * lk, H, xn[slot]);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) router_load<VEC>(wp[n], k + 8 * lk, H, wn[slot][n]);
+    router_load<VEC>(wg, k + 8 * lk, H, gn[slot]);
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) fetch(s, 32 * (part + kRouterWaves * s));
+  for (int k0 = 32 * part; k0 < H; k0 += 32 * kRouterWaves * kAhead) {  // scalar
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      const int k = k0 + 32 * kRouterWaves * s;
+      if (k >= H) break;  // scalar
+      float xc[8], wc[NT][8];
+      const bool in = !VEC || k + 8 * lk < H;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        xc[i] = in ? xn[s][i] : 0.f;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) wc[n][i] = wn[s][n][i];
+        if (with_gate) acc_g = fmaf(xc[i], gn[s][i], acc_g);
+      }
+      fetch(s, k + 32 * kRouterWaves * kAhead);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[n][i], xc[i], acc[n], 0, 0, 0);
+    }
+  }
+  acc_g += __shfl_xor(acc_g, 16, kWave);
+  acc_g += __shfl_xor(acc_g, 32, kWave);
+  if (t0 + li >= T_) return;
+  const int row = router_part_row(E);
+  float* dst = parts + (static_cast<int64_t>(part) * T_ + t0 + li) * row;
+  // lane holds token li, experts 16 n + 4 lk + i
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+    if (e0 + 16 * n + 4 * lk < row - 4) *reinterpret_cast<f32x4_t*>(dst + e0 + 16 * n + 4 * lk) = acc[n];
+  if (with_gate && lk == 0) dst[row - 4] = acc_g;
+}
+
+// One token's choice from the parts of its logits, by one wave.
+__device__ __forceinline__ void choose_from_parts(int32_t* choice, float* weight, float* __restrict__ gate,
+                                                  const float* __restrict__ parts, int t, int T_, int E, int lane,
+                                                  const RouteRule& rule) {
+  const int row = router_part_row(E);
+  const int64_t step = static_cast<int64_t>(T_) * row;
+  const float* p = parts + static_cast<int64_t>(t) * row;
+  const int at = lane < E ? lane : 0;
+  float v[kRouterWaves], g[kRouterWaves];
+#pragma unroll
+  for (int w = 0; w < kRouterWaves; ++w) v[w] = p[w * step + at];
+  if (gate != nullptr) {  // the same for the whole grid
+#pragma unroll
+    for (int w = 0; w < kRouterWaves; ++w) g[w] = p[w * step + row - 4];
+  }
+  float z = 0.f;
+#pragma unroll
+  for (int w = 0; w < kRouterWaves; ++w) z += v[w];
+  if (gate != nullptr) {
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kRouterWaves; ++w) sum += g[w];
+    if (lane == 0) gate[t] = 1.f / (1.f + expf(-sum));
+  }
+  route_lanes(choice, weight, z, lane, E, rule);
+}
+
+__global__ __launch_bounds__(256) void moe_choose_kernel(int32_t* __restrict__ choice, float* __restrict__ weight,
+                                                         float* __restrict__ gate, const float* __restrict__ parts, int T_,
+                                                         int E, RouteRule rule) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int t = blockIdx.x * 4 + wave;
+  if (t >= T_) return;  // scalar
+  choose_from_parts(choice + static_cast<int64_t>(t) * rule.top, weight + static_cast<int64_t>(t) * rule.top, gate, parts,
+                    t, T_, E, lane, rule);
+}
+
+__global__ __launch_bounds__(1024) void moe_choose_align_kernel(
+    int32_t* __restrict__ choice, float* __restrict__ weight, float* __restrict__ gate, int32_t* __restrict__ sorted,
+    int32_t* __restrict__ tiles, int32_t* __restrict__ num_tiles, const float* __restrict__ parts, int T_, int E,
+    int max_tiles, int tile_rows, RouteRule rule) {
+  extern __shared__ int32_t ilds[];  // [T top] choices, then [4 E]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  if (wave < T_)  // scalar
+    choose_from_parts(ilds + wave * rule.top, weight + static_cast<int64_t>(wave) * rule.top, gate, parts, wave, T_, E, lane,
+                      rule);
+  __syncthreads();
+  const int pairs = T_ * rule.top;
+  for (int i = threadIdx.x; i < pairs; i += blockDim.x) choice[i] = ilds[i];
+  align_pairs(sorted, tiles, num_tiles, ilds, pairs, E, max_tiles, tile_rows, ilds + pairs);
+}
+
+// bfloat16, few rows: a block of four waves takes one tile of up to 16 rows and 16 columns (gated: of gate and of
+// up), and its waves share K: wave w takes the passes w, w + 4, ... of 64 values, four of them on their way, and
+// the four sums are added in wave order.  In a pass lane (li, lk) fetches the 16 values from 16 lk of its weight
+// row and of its token row (32 contiguous bytes, so that the four lanes of a row read one 128-byte line) and the
+// two matrix instructions take its first and its second eight (both operands are dealt the same way, so each
+// product still sums over all of K).  Bound by reading the weights of the experts that were chosen: with a whole K
+// a wave and 64 columns a block, one token of four experts of 2048 x 2048 had 128 blocks.  Gated and ungated, packed:
+// one token 22.0 and 13.4 -> 13.8 and 11.8 us, eight tokens 75 and 46 -> 64 and 34 us (5.6 TB/s).
 template <int GATED, typename TO, int PACKED>
-__global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
+__global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
     int act, const float* __restrict__ row_scale) {
-  const int tile = blockIdx.x;
+  constexpr int kWavesK = 4, kStages = 4;
+  __shared__ f32x4_t part[(kWavesK - 1) * (GATED ? 2 : 1)][64];
+  const int tile = blockIdx.y;
   if (tile >= *num_tiles) return;
   const int e = tiles[3 * tile], r0 = tiles[3 * tile + 1], nr = tiles[3 * tile + 2];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-  const int n0 = (blockIdx.y * 4 + wave) * 16;
-  if (n0 >= N) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int n0 = blockIdx.x * 16;
   const int li = lane & 15, lk = lane >> 4;
   // B operand: token row li of the tile; A operand: the expert's row n0 + li
   const bool row_ok = li < nr;
-  const int pair = sorted[r0 + (row_ok ? li : 0)];
+  const int pair = sorted[r0 + (row_ok ? li : 0)];  // a row that is not there reads the tile's first and is dropped
   const int64_t in_row = in_div > 0 ? pair / in_div : r0 + (row_ok ? li : 0);
   // PACKED: w is the copy that `kvc_pack_weight` makes, tiles of 16 rows x 32 values of K in one
   // piece of 1 KB each, so a wave's load of an operand is one contiguous kilobyte instead of 128 bytes
@@ -396,53 +651,46 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
                             : w + (static_cast<int64_t>(e) * rows_per_expert + wrow) * K + 16 * lk;
   const bf16_t* wr2 = wr + static_cast<int64_t>(N) * K;  // the up rows follow the gate rows (in either order of storage)
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
-  const int k_main = K & ~63;
-  // two passes are on their way while one is multiplied
-  bf16x8_t an[2][2], a2n[2][2], bn[2][2];
-  auto fetch = [&](int k, int slot) {
+  const int passes = K / 64;
+  // blocks walk K round from places of their own, as in the kernel for more rows
+  const int turn = passes > 0 ? (e * 5 + static_cast<int>(blockIdx.x) * 3) % passes : 0;
+  bf16x8_t an[kStages][2], a2n[kStages][2], bn[kStages][2];
+  auto fetch = [&](int slot, int pass) {  // no branch around the loads: a pass that is not there repeats the last
+    int p = pass < passes ? pass + turn : passes - 1 + turn;
+    p = p < passes ? p : p - passes;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int64_t wo = PACKED ? static_cast<int64_t>(k / 32 + h) * 512 : k + 8 * h;
+      const int64_t wo = PACKED ? static_cast<int64_t>(2 * p + h) * 512 : 64 * p + 8 * h;
       an[slot][h] = *reinterpret_cast<const bf16x8_t*>(wr + wo);
       if (GATED) a2n[slot][h] = *reinterpret_cast<const bf16x8_t*>(wr2 + wo);
-      // a row that is not there reads the tile's first
-      bn[slot][h] = *reinterpret_cast<const bf16x8_t*>(xr + k + (PACKED ? 32 : 8) * h);
+      bn[slot][h] = *reinterpret_cast<const bf16x8_t*>(xr + 64 * p + (PACKED ? 32 : 8) * h);
     }
   };
-  if (k_main > 0) fetch(0, 0);
-  if (k_main > 64) fetch(64, 1);
-  for (int k = 0; k < k_main; k += 128) {
-    // slot 0 holds pass k, slot 1 pass k + 64; each is asked for again as soon as it has been used
-    bf16x8_t a0[2], a20[2], b0[2];
+  if (wave < passes) {  // scalar
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      a0[h] = an[0][h];
-      if (GATED) a20[h] = a2n[0][h];
-      b0[h] = row_ok ? bn[0][h] : zero8();
-    }
-    if (k + 128 < k_main) fetch(k + 128, 0);
+    for (int s = 0; s < kStages; ++s) fetch(s, wave + kWavesK * s);
+    for (int p = wave; p < passes; p += kWavesK * kStages) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[h], b0[h], acc, 0, 0, 0);
-      if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a20[h], b0[h], acc2, 0, 0, 0);
-    }
-    if (k + 64 < k_main) {
-      bf16x8_t a1[2], a21[2], b1[2];
+      for (int s = 0; s < kStages; ++s) {
+        if (p + kWavesK * s >= passes) break;  // scalar
+        bf16x8_t a[2], a2[2], b[2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        a1[h] = an[1][h];
-        if (GATED) a21[h] = a2n[1][h];
-        b1[h] = row_ok ? bn[1][h] : zero8();
-      }
-      if (k + 192 < k_main) fetch(k + 192, 1);
+        for (int h = 0; h < 2; ++h) {
+          a[h] = an[s][h];
+          if (GATED) a2[h] = a2n[s][h];
+          b[h] = bn[s][h];
+        }
+        if (p + kWavesK * kStages < passes) fetch(s, p + kWavesK * (s + kStages));
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[h], b1[h], acc, 0, 0, 0);
-        if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a21[h], b1[h], acc2, 0, 0, 0);
+        for (int h = 0; h < 2; ++h) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], b[h], acc, 0, 0, 0);
+          if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[h], b[h], acc2, 0, 0, 0);
+        }
       }
     }
   }
-  if (k_main < K) {  // a ragged end along K (a multiple of 8): element by element, zeros beyond
+  const int k_main = 64 * passes;
+  if (wave == 0 && k_main < K) {  // a ragged end along K (a multiple of 8): element by element, zeros beyond
     bf16x8_t a[2], a2[2], b[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -452,12 +700,23 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
         if (off + 16 * lk < K) {
           a[h][i] = reinterpret_cast<const __bf16*>(wr)[off];
           if (GATED) a2[h][i] = reinterpret_cast<const __bf16*>(wr2)[off];
-          if (row_ok) b[h][i] = reinterpret_cast<const __bf16*>(xr)[off];
+          b[h][i] = reinterpret_cast<const __bf16*>(xr)[off];
         }
       }
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], b[h], acc, 0, 0, 0);
       if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[h], b[h], acc2, 0, 0, 0);
     }
+  }
+  if (wave > 0) {
+    part[wave - 1][lane] = acc;
+    if (GATED) part[kWavesK - 2 + wave][lane] = acc2;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int v = 0; v < kWavesK - 1; ++v) {
+    acc += part[v][lane];
+    if (GATED) acc2 += part[kWavesK - 1 + v][lane];
   }
   // lane holds column (token) li, rows (features) n0 + 4 * lk + i
   if (!row_ok) return;
@@ -470,35 +729,62 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(
   if (nf < N) store4<TO>(out + out_row * out_stride + nf, acc, N - nf);
 }
 
-// bfloat16, tiles of 64 rows: a block of four waves takes the tile's rows and 128 columns (gated;
-// 256 otherwise).  The rows' chunk of 64 values along K goes through LDS, which all waves read as
-// the B operand (four row blocks of 16); every wave fetches the weight rows of its own columns
-// straight into registers as the A operand (NF blocks of 16 columns, for gate and for up), one
-// chunk ahead of the products.  Every fetched weight meets 64 rows, every row 128 or 256 columns.
-template <int GATED, typename TO, int PACKED>
-__global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(
+// bfloat16, tiles of 64 or 128 rows (NR row blocks of 16; the last ones of a tile may be empty and are not
+// multiplied): a block of four waves takes the tile's rows and 128 columns (gated; 256 otherwise).  The rows'
+// chunk of 64 values along K goes through LDS (two buffers, one barrier a chunk), which all waves read as the B
+// operand; every wave fetches the weight rows of its own columns straight into registers as the A operand
+// (NF blocks of 16 columns, for gate and for up), one chunk ahead of the products.  Bound by the weights' way to
+// the compute units: a fetched weight meets 16 NR rows, a row 128 or 256 columns, and the blocks that read the
+// same weights or the same rows run on one die at the same time (see `place`), so its L2 is asked twice and
+// memory once.  Packed, 32 experts of 2048 x 2048, gated and ungated: 8,192 pairs 397 and 232 us with tiles of 64
+// rows dealt to the dies in turn, 202 and 123 us this way (0.68 PFLOP/s); 1,200 pairs 226 and 143 us in tiles of 16
+// rows, 102 and 52 us here (5.3 TB/s of weights); 256 pairs 113 and 61 us, 95 and 46 us (5.8 TB/s), of which
+// 14 and 7 us are the turn that every block starts K at.
+struct TilePlace {
+  int tile, col;
+};
+// Which row tile and which column block the block `id` takes (tile -1: none).  Blocks are dealt to the eight
+// dies in turn, so `id % 8` is the die.  Where the column blocks divide by eight, a die keeps its share of them
+// for every tile, its own columns of a tile side by side (they share the rows); otherwise a die takes a run of
+// (column, tile) pairs, a column's tiles side by side (an expert's share the weights).
+__device__ __forceinline__ TilePlace place(int id, int tiles, int cols) {
+  const int die = id & 7, idx = id >> 3;
+  if ((cols & 7) == 0) {
+    const int own = cols >> 3, tile = idx / own;
+    return {tile < tiles ? tile : -1, die * own + (idx - tile * own)};
+  }
+  const int total = tiles * cols, chunk = (total + 7) >> 3;
+  const int at = die * chunk + idx;
+  if (idx >= chunk || at >= total) return {-1, 0};
+  const int col = at / tiles;
+  return {at - col * tiles, col};
+}
+
+template <int GATED, int NR, typename TO, int PACKED>
+__global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
     int act, const float* __restrict__ row_scale) {
   constexpr int NF = GATED ? 2 : 4;   // column blocks of 16 a wave
-  constexpr int NR = kBigTileRows / 16;
   constexpr int KC = 64;              // values of K a pass (two matrix instructions deep)
   constexpr int KROW = KC + 8;        // a row's chunk in LDS, padded against bank conflicts
-  __shared__ __attribute__((aligned(16))) bf16_t x_s[kBigTileRows * KROW];
-  const int tile = blockIdx.x;
-  if (tile >= *num_tiles) return;
-  const int e = tiles[3 * tile], r0 = tiles[3 * tile + 1], nr = tiles[3 * tile + 2];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  constexpr int CH = NR / 2;          // pieces of eight values that a thread stages a pass
+  __shared__ __attribute__((aligned(16))) bf16_t x_s[2][16 * NR * KROW];
+  const TilePlace at = place(blockIdx.x, *num_tiles, (N + 64 * NF - 1) / (64 * NF));
+  if (at.tile < 0) return;
+  const int e = tiles[3 * at.tile], r0 = tiles[3 * at.tile + 1];
+  const int nr = __builtin_amdgcn_readfirstlane(tiles[3 * at.tile + 2]);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   const int li = lane & 15, lk = lane >> 4;
-  const int n0 = (blockIdx.y * 4 + wave) * 16 * NF;
+  const int n0 = (at.col * 4 + wave) * 16 * NF;
   const bool wave_live = n0 < N;  // the same for the whole wave
-  // staging: thread t brings 16 values of row t / 4 of the tile
-  const int srow = threadIdx.x >> 2, spart = threadIdx.x & 3;
+  // staging: a thread brings 8 CH values of one row of the tile
+  const int srow = threadIdx.x / (8 / CH), spart = threadIdx.x % (8 / CH);
   const bool srow_ok = srow < nr;
   const int srow_safe = srow_ok ? srow : 0;  // a row that is not there reads the tile's first, and is set to zero
   const int64_t in_row = in_div > 0 ? sorted[r0 + srow_safe] / in_div : r0 + srow_safe;
-  const bf16_t* xp = x + in_row * x_stride + 16 * spart;
+  const bf16_t* xp = x + in_row * x_stride + 8 * CH * spart;
   const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
   const bf16_t* wp[NF];
 #pragma unroll
@@ -518,60 +804,89 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(
       acc[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (GATED) acc2[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-  uint4 x_next[2] = {uint4{0u, 0u, 0u, 0u}, uint4{0u, 0u, 0u, 0u}};
+  uint4 x_next[CH];
   bf16x8_t w_next[2][NF], w2_next[2][GATED ? NF : 1];
-  // a pass's second half may lie beyond K (K a multiple of 32 only): it then reads the first half
-  // again and is not multiplied
-  auto fetch = [&](int k) {
-    const bool two = k + 32 < K;
-    const int c0 = (two || spart < 2) ? 0 : -16 * spart;  // columns beyond K read the pass's first instead
-    x_next[0] = *reinterpret_cast<const uint4*>(xp + k + c0);
-    x_next[1] = *reinterpret_cast<const uint4*>(xp + k + c0 + 8);
-    if (wave_live) {
+  // a pass's second half may lie beyond K (K a multiple of 32 only): the first half is then read
+  // again and not multiplied
+  auto fetch_x = [&](int k) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int kk = k + ((h && two) ? 32 : 0);
+    for (int c = 0; c < CH; ++c) {
+      const int col = 8 * (CH * spart + c);
+      x_next[c] = *reinterpret_cast<const uint4*>(xp + k + 8 * c - (k + col < K ? 0 : 32));
+    }
+  };
+  auto fetch_w = [&](int k) {
 #pragma unroll
-        for (int f = 0; f < NF; ++f) {
-          const int64_t wo = PACKED ? static_cast<int64_t>(kk / 32) * 512 : kk;
-          w_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + wo);
-          if (GATED) w2_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + up_off + wo);
-        }
+    for (int h = 0; h < 2; ++h) {
+      const int kk = k + 32 * h < K ? k + 32 * h : k;
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        const int64_t wo = PACKED ? static_cast<int64_t>(kk / 32) * 512 : kk;
+        w_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + wo);
+        if (GATED) w2_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + up_off + wo);
       }
     }
   };
-  fetch(0);
-  for (int k = 0; k < K; k += KC) {
-    const bool two = k + 32 < K;
-    __syncthreads();  // the chunk before has been read by every wave
-    // thread t's 16 values: columns 16 spart .. of the pass; K shorter than a whole pass leaves zeros
-    const bool keep = srow_ok && (two || spart < 2);
-    *reinterpret_cast<uint4*>(x_s + srow * KROW + 16 * spart) = keep ? x_next[0] : uint4{0u, 0u, 0u, 0u};
-    *reinterpret_cast<uint4*>(x_s + srow * KROW + 16 * spart + 8) = keep ? x_next[1] : uint4{0u, 0u, 0u, 0u};
-    bf16x8_t wa[2][NF], wa2[2][GATED ? NF : 1];
+  auto stash = [&](int buffer) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int c = 0; c < CH; ++c)
+      *reinterpret_cast<uint4*>(x_s[buffer] + srow * KROW + 8 * (CH * spart + c)) = srow_ok ? x_next[c] : uint4{0u, 0u, 0u, 0u};
+  };
+  // Every block walks K round from a place of its own (which its expert and columns decide, so a row's sums do
+  // not depend on its tile): blocks that start at the same place of rows that lie a power of two apart would ask
+  // the same memory channels at the same time.
+  const int turn = K % KC == 0 ? (e * 5 + at.col * 11) % (K / KC) * KC : 0;
+  auto round = [&](int k) { return k + turn < K ? k + turn : k + turn - K; };
+  fetch_x(round(0));
+  fetch_w(round(0));
+  stash(0);
+  if (KC < K) fetch_x(round(KC));
+  __syncthreads();
+  for (int k0 = 0; k0 < K; k0 += 2 * KC) {
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        wa[h][f] = w_next[h][f];
-        if (GATED) wa2[h][f] = w2_next[h][f];
-      }
-    if (k + KC < K) fetch(k + KC);
-    __syncthreads();
-    if (wave_live) {  // scalar: matrix instructions are skipped by a branch, never by a lane mask
+    for (int s = 0; s < 2; ++s) {  // the chunk is in LDS buffer s
+      const int k = k0 + KC * s;
+      if (k >= K) break;  // scalar
+      const bool two = k + 32 < K;
+      bf16x8_t wa[2][NF], wa2[2][GATED ? NF : 1];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (h == 1 && !two) break;  // scalar
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(x_s + (16 * r + li) * KROW + 32 * h + 8 * lk);
+        for (int f = 0; f < NF; ++f) {
+          wa[h][f] = w_next[h][f];
+          if (GATED) wa2[h][f] = w2_next[h][f];
+        }
+      fetch_w(round(k + KC < K ? k + KC : k));  // no branch around the loads: the last one repeats
+      if (k + KC < K) stash(s ^ 1);  // the chunk after this one, asked for a pass ago
+      if (k + 2 * KC < K) fetch_x(round(k + 2 * KC));
+      if (wave_live) {  // scalar: matrix instructions are skipped by a branch, never by a lane mask
+        const bf16_t* xb = x_s[s] + li * KROW + 8 * lk;
 #pragma unroll
-          for (int f = 0; f < NF; ++f) {
-            acc[f][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[h][f], b, acc[f][r], 0, 0, 0);
-            if (GATED) acc2[f][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa2[h][f], b, acc2[f][r], 0, 0, 0);
+        for (int h = 0; h < 2; ++h) {
+          if (h == 1 && !two) break;  // scalar
+          bf16x8_t b[2][2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) b[0][i] = *reinterpret_cast<const bf16x8_t*>(xb + 16 * i * KROW + 32 * h);
+#pragma unroll
+          for (int g = 0; g < NR / 2; ++g) {  // two row blocks at a time, the next two on their way from LDS
+            if (g + 1 < NR / 2)
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                b[(g + 1) & 1][i] = *reinterpret_cast<const bf16x8_t*>(xb + 16 * (2 * g + 2 + i) * KROW + 32 * h);
+            if (32 * g < nr) {  // scalar
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                  acc[f][2 * g + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[h][f], b[g & 1][i], acc[f][2 * g + i], 0, 0, 0);
+                  if (GATED)
+                    acc2[f][2 * g + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa2[h][f], b[g & 1][i], acc2[f][2 * g + i], 0, 0, 0);
+                }
+            }
           }
         }
       }
+      __syncthreads();  // this chunk has been read by every wave, the next one is there
     }
   }
   if (!wave_live) return;
@@ -628,22 +943,40 @@ __global__ __launch_bounds__(256) void moe_gemm_plain_kernel(
   }
 }
 
-template <typename TA>
+// VEC columns a thread (4 where rows and pointers allow 16-byte loads): bound by reading the experts' rows.
+// 2,030 tokens of 2,048 columns with four choices: 37 us with one column a thread, 21 us.
+template <typename TA, int VEC>
 __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ out, const float* __restrict__ y,
                                                           const float* __restrict__ weight, int top,
                                                           const TA* __restrict__ add0, const float* __restrict__ add1,
                                                           const float* __restrict__ add1_gate, int T, int H,
                                                           int accumulate) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t idx = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * VEC;
   if (idx >= static_cast<int64_t>(T) * H) return;
   const int t = static_cast<int>(idx / H), c = static_cast<int>(idx - static_cast<int64_t>(t) * H);
-  float acc = 0.f;
-  for (int j = 0; j < top; ++j)
-    acc = fmaf(weight != nullptr ? weight[static_cast<int64_t>(t) * top + j] : 1.f,
-               y[(static_cast<int64_t>(t) * top + j) * H + c], acc);
-  if (add0 != nullptr) acc += to_float(add0[idx]);
-  if (add1 != nullptr) acc = add1_gate != nullptr ? fmaf(add1_gate[t], add1[idx], acc) : acc + add1[idx];
-  out[idx] = accumulate ? out[idx] + acc : acc;
+  typedef float vec_t __attribute__((ext_vector_type(VEC)));
+  auto load = [](const float* p) { return *reinterpret_cast<const vec_t*>(p); };
+  const float* yt = y + static_cast<int64_t>(t) * top * H + c;
+  vec_t acc = 0.f;
+#pragma unroll 4
+  for (int j = 0; j < top; ++j) {
+    const float w = weight != nullptr ? weight[static_cast<int64_t>(t) * top + j] : 1.f;
+    const vec_t v = load(yt + static_cast<int64_t>(j) * H);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) acc[i] = fmaf(w, v[i], acc[i]);
+  }
+  if (add0 != nullptr) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) acc[i] += to_float(add0[idx + i]);
+  }
+  if (add1 != nullptr) {
+    const vec_t v = load(add1 + idx);
+    const float g = add1_gate != nullptr ? add1_gate[t] : 0.f;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) acc[i] = add1_gate != nullptr ? fmaf(g, v[i], acc[i]) : acc[i] + v[i];
+  }
+  vec_t* o = reinterpret_cast<vec_t*>(out + idx);
+  *o = accumulate ? *o + acc : acc;
 }
 
 }  // namespace
@@ -702,20 +1035,73 @@ extern "C" int kvc_moe_router(int32_t* choice, float* weight, const void* x, int
   return kvc_check_launch("kvc_moe_router");
 }
 
-extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
-  return (pairs + tile_rows - 1) / tile_rows + E;
+extern "C" int kvc_moe_router_spread_tokens(void) { return kRouterSpread; }
+extern "C" int kvc_moe_router_spread_floats(int T, int E) { return kRouterWaves * T * router_part_row(E); }
+
+extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32_t* tiles, int32_t* num_tiles,
+                                  int max_tiles, int tile_rows, float* parts, int64_t parts_floats, const void* x,
+                                  int64_t x_stride, int x_dtype, const float* router, float* gate, int T, int H, int E,
+                                  int top, int groups, int keep, int score_fn, const float* bias, const float* correction,
+                                  int group_best, int renormalize, float weight_scale, kvc_stream stream) {
+  if (T < 0 || H <= 0 || E <= 0 || top <= 0 || top > E || groups <= 0 || E % groups || keep <= 0 || keep > groups ||
+      x_stride < H)
+    return kvc_fail("kvc_moe_router_spread: bad sizes (the experts in equal groups)");
+  if (T > kRouterSpread || E > kWave) return kvc_fail("kvc_moe_router_spread: at most 1024 tokens and 64 experts");
+  if (score_fn < 0 || score_fn > 2 || (group_best != 1 && group_best != 2))
+    return kvc_fail("kvc_moe_router_spread: scores by softmax (0), sigmoid (1) or logit (2); a group is worth its best 1 or 2");
+  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
+    return kvc_fail("kvc_moe_router_spread: tiles of 16, 64 or 128 rows");
+  if (max_tiles < kvc_moe_max_tiles(T * top, E, tile_rows))
+    return kvc_fail("kvc_moe_router_spread: room for fewer tiles than the routing may need");
+  if (parts_floats < kvc_moe_router_spread_floats(T, E) || (reinterpret_cast<uintptr_t>(parts) & 15) != 0)
+    return kvc_fail("kvc_moe_router_spread: the workspace is too small or not 16-byte aligned");
+  if (x_dtype != 0 && x_dtype != 1) return kvc_fail("kvc_moe_router_spread: unknown dtype code");
+  if (T == 0) return 0;
+  const RouteRule rule{top, groups, keep, score_fn, group_best, renormalize, bias, correction, weight_scale};
+  const dim3 grid((T + kRouterTokens - 1) / kRouterTokens, kRouterWaves, (E + kRouterRows - 1) / kRouterRows);
+  // 16-byte loads where the rows allow
+  const bool vectors = H % 8 == 0 && x_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(router) & 15) == 0 &&
+                       (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+#define KVC_PARTS(Tp, VEC)                                                                                       \
+  hipLaunchKernelGGL((moe_router_parts_kernel<Tp, VEC>), grid, dim3(kWave), 0, S(stream), parts,                 \
+                     static_cast<const Tp*>(x), x_stride, router, gate != nullptr ? 1 : 0, T, H, E)
+  if (x_dtype == 1 && vectors) KVC_PARTS(bf16_t, 1);
+  else if (x_dtype == 1) KVC_PARTS(bf16_t, 0);
+  else if (vectors) KVC_PARTS(float, 1);
+  else KVC_PARTS(float, 0);
+#undef KVC_PARTS
+  if (T <= kChooseInOne) {
+    hipLaunchKernelGGL(moe_choose_align_kernel, dim3(1), dim3(1024), sizeof(int32_t) * (T * top + 4 * E), S(stream),
+                       choice, weight, gate, sorted, tiles, num_tiles, parts, T, E, max_tiles, tile_rows, rule);
+    return kvc_check_launch("kvc_moe_router_spread");
+  }
+  hipLaunchKernelGGL(moe_choose_kernel, dim3((T + 3) / 4), dim3(256), 0, S(stream), choice, weight, gate, parts, T, E, rule);
+  return kvc_moe_align(sorted, tiles, num_tiles, choice, T * top, E, max_tiles, tile_rows, stream);
 }
 
-// Tiles of 64 rows where the experts have that many rows on average (portions of prompts): the
-// tiled kernel then uses every fetched weight four times as often; tiles of 16 otherwise.
-extern "C" int kvc_moe_tile_rows(int pairs, int E) { return pairs >= 64 * E ? kBigTileRows : kTileRows; }
+extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
+  const int most = (pairs + tile_rows - 1) / tile_rows + E;
+  return pairs < most ? pairs : most;  // no tile is empty
+}
+
+// Tiles that hold an expert's rows as a rule, so that a fetched weight meets all of them.  Measured over 32 experts of
+// 2048 x 2048, both products: 2 rows an expert 119 us in tiles of 16 and 120 in tiles of 64, 4 rows 137 and 135; 37
+// rows 156 us in tiles of 64 and 155 in tiles of 128, 64 rows 182 and 166.  From 104 to 150 rows many an expert has a
+// few more than 128, and two tiles of half the size cost more than smaller ones: 128 rows 232 us in tiles of 64, 253
+// in tiles of 128; 192 rows 287 and 247.
+extern "C" int kvc_moe_tile_rows(int pairs, int E) {
+  const int64_t e = E;
+  if (pairs >= 150 * e || (pairs >= 40 * e && pairs < 104 * e)) return kBigTileRows;
+  return pairs >= 3 * e ? kMidTileRows : kTileRows;
+}
 
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
                              int pairs, int E, int max_tiles, int tile_rows, kvc_stream stream) {
-  if (tile_rows != kTileRows && tile_rows != kBigTileRows) return kvc_fail("kvc_moe_align: tiles of 16 or 64 rows");
+  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
+    return kvc_fail("kvc_moe_align: tiles of 16, 64 or 128 rows");
   if (pairs < 0 || E <= 0 || max_tiles < kvc_moe_max_tiles(pairs, E, tile_rows))
     return kvc_fail("kvc_moe_align: bad sizes, or room for fewer tiles than the routing may need");
-  const size_t lds = sizeof(int32_t) * 3 * E;
+  const size_t lds = sizeof(int32_t) * 4 * E;
   if (lds > 60000) return kvc_fail("kvc_moe_align: too many experts");
   hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), lds, S(stream), sorted, tiles, num_tiles, choice,
                      pairs, E, max_tiles, tile_rows);
@@ -729,7 +1115,8 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
                             const float* row_scale, int packed, kvc_stream stream) {
   if (max_tiles < 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N)
     return kvc_fail("kvc_moe_gemm: bad sizes");
-  if (tile_rows != kTileRows && tile_rows != kBigTileRows) return kvc_fail("kvc_moe_gemm: tiles of 16 or 64 rows");
+  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
+    return kvc_fail("kvc_moe_gemm: tiles of 16, 64 or 128 rows");
   if (act < -1 || act > 0 || (gated && act != -1))
     return kvc_fail("kvc_moe_gemm: an ungated product has no activation (-1) or the square of relu (0)");
   if (max_tiles == 0) return 0;
@@ -744,34 +1131,45 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
     // the matrix cores read 16 bytes at a time: rows of a multiple of 8 values, 16-byte aligned
     const bool vectors = K % 8 == 0 && x_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(w) & 15) == 0;
-    if (tile_rows == kBigTileRows) {
-      if (!vectors || K % 32) return kvc_fail("kvc_moe_gemm: tiles of 64 rows need K to be a multiple of 32");
+    if (tile_rows != kTileRows) {
+      if (!vectors || K % 32) return kvc_fail("kvc_moe_gemm: tiles of 64 and 128 rows need K to be a multiple of 32");
       if (packed && (N % 16 || K % 64))
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
-      grid.y = gated ? (N + 127) / 128 : (N + 255) / 256;
-      if (packed) {
-        if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, bf16_t, 1>), bf16_t, bf16_t);
-        else if (gated) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, float, 1>), bf16_t, float);
-        else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, bf16_t, 1>), bf16_t, bf16_t);
-        else KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, float, 1>), bf16_t, float);
+      const int64_t cols = gated ? (N + 127) / 128 : (N + 255) / 256;
+      const int64_t blocks = 8 * ((cols * max_tiles + 7) / 8);  // every die gets its share of the pairs
+      if (blocks > 0x7fffffff) return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
+      grid = dim3(static_cast<unsigned>(blocks));
+#define KVC_MOE_TILED(NR, PACKED)                                                                               \
+  do {                                                                                                          \
+    if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, NR, bf16_t, PACKED>), bf16_t, bf16_t); \
+    else if (gated) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, NR, float, PACKED>), bf16_t, float);               \
+    else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, NR, bf16_t, PACKED>), bf16_t, bf16_t);    \
+    else KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, NR, float, PACKED>), bf16_t, float);                          \
+  } while (0)
+      if (tile_rows == kBigTileRows) {
+        if (packed) KVC_MOE_TILED(8, 1);
+        else KVC_MOE_TILED(8, 0);
       } else {
-        if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, bf16_t, 0>), bf16_t, bf16_t);
-        else if (gated) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, float, 0>), bf16_t, float);
-        else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, bf16_t, 0>), bf16_t, bf16_t);
-        else KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, float, 0>), bf16_t, float);
+        if (packed) KVC_MOE_TILED(4, 1);
+        else KVC_MOE_TILED(4, 0);
       }
+#undef KVC_MOE_TILED
+    } else if (vectors && max_tiles > 65535) {
+      return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
     } else if (packed) {
+      grid = dim3((N + 15) / 16, max_tiles);
       if (!vectors || N % 16 || K % 64)
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
-      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<1, bf16_t, 1>), bf16_t, bf16_t);
-      else if (gated) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<1, float, 1>), bf16_t, float);
-      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<0, bf16_t, 1>), bf16_t, bf16_t);
-      else KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<0, float, 1>), bf16_t, float);
+      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, 1>), bf16_t, bf16_t);
+      else if (gated) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, float, 1>), bf16_t, float);
+      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, bf16_t, 1>), bf16_t, bf16_t);
+      else KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, float, 1>), bf16_t, float);
     } else if (vectors) {
-      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<1, bf16_t, 0>), bf16_t, bf16_t);
-      else if (gated) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<1, float, 0>), bf16_t, float);
-      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<0, bf16_t, 0>), bf16_t, bf16_t);
-      else KVC_MOE_LAUNCH((moe_gemm_bf16_kernel<0, float, 0>), bf16_t, float);
+      grid = dim3((N + 15) / 16, max_tiles);
+      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, 0>), bf16_t, bf16_t);
+      else if (gated) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, float, 0>), bf16_t, float);
+      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, bf16_t, 0>), bf16_t, bf16_t);
+      else KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, float, 0>), bf16_t, float);
     } else {
       if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_plain_kernel<1, bf16_t, bf16_t>), bf16_t, bf16_t);
       else if (gated) KVC_MOE_LAUNCH((moe_gemm_plain_kernel<1, bf16_t, float>), bf16_t, float);
@@ -797,13 +1195,19 @@ extern "C" int kvc_moe_combine(float* out, const float* y, const float* weight, 
   if (T < 0 || H <= 0 || top < 0) return kvc_fail("kvc_moe_combine: bad sizes");
   if (T == 0) return 0;
   const int64_t n = static_cast<int64_t>(T) * H;
-  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+  const bool vec = H % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(y) |
+                                   reinterpret_cast<uintptr_t>(add1) | reinterpret_cast<uintptr_t>(add0)) & 15) == 0;
+  const dim3 grid(static_cast<unsigned>((n / (vec ? 4 : 1) + 255) / 256));
+#define KVC_COMBINE(TA, VEC)                                                                                \
+  hipLaunchKernelGGL((moe_combine_kernel<TA, VEC>), grid, dim3(256), 0, S(stream), out, y, weight, top,     \
+                     static_cast<const TA*>(add0), add1, add1_gate, T, H, accumulate)
   if (add0_dtype == 1) {
-    hipLaunchKernelGGL((moe_combine_kernel<bf16_t>), grid, dim3(256), 0, S(stream), out, y, weight, top,
-                       static_cast<const bf16_t*>(add0), add1, add1_gate, T, H, accumulate);
+    if (vec) KVC_COMBINE(bf16_t, 4);
+    else KVC_COMBINE(bf16_t, 1);
   } else {
-    hipLaunchKernelGGL((moe_combine_kernel<float>), grid, dim3(256), 0, S(stream), out, y, weight, top,
-                       static_cast<const float*>(add0), add1, add1_gate, T, H, accumulate);
+    if (vec) KVC_COMBINE(float, 4);
+    else KVC_COMBINE(float, 1);
   }
+#undef KVC_COMBINE
   return kvc_check_launch("kvc_moe_combine");
 }

@@ -69,6 +69,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_head_rmsnorm_gate": [P, I, P, P, L, I, P, F, I, I, I, I, P],
         "kvc_moe_route": [P, P, P, I, I, I, I, I, I, P, P, I, I, F, P],
         "kvc_moe_router": [P, P, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
+        "kvc_moe_router_spread": [P, P, P, P, P, I, I, P, L, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
+        "kvc_moe_router_spread_floats": [I, I],
         "kvc_moe_max_tiles": [I, I, I],
         "kvc_moe_tile_rows": [I, I],
         "kvc_moe_align": [P, P, P, P, I, I, I, I, P],
@@ -122,6 +124,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvc_last_variant.argtypes = [c_int]
     lib.kvc_argmax_static_capacity.restype = c_int
     lib.kvc_argmax_static_capacity.argtypes = []
+    lib.kvc_moe_router_spread_tokens.restype = c_int
+    lib.kvc_moe_router_spread_tokens.argtypes = []
     lib.kvc_ssm_scan_max_state.restype = c_int
     lib.kvc_ssm_scan_max_state.argtypes = []
     lib.kvc_fixed_decay_chunk_tokens.restype = c_int
@@ -1917,9 +1921,47 @@ def moe_router(choice: torch.Tensor, weight: torch.Tensor, x: torch.Tensor, rout
            "kvc_moe_router")
 
 
+def moe_router_spread_tokens() -> int:
+    """The most tokens that ``moe_router_spread`` serves."""
+    return int(load().kvc_moe_router_spread_tokens())
+
+
+def moe_router_spread_supported(tokens: int, experts: int) -> bool:
+    """Whether ``moe_router_spread`` serves a step of this size."""
+    return tokens <= moe_router_spread_tokens() and experts <= 64
+
+
+def moe_router_spread_floats(tokens: int, experts: int) -> int:
+    """float32 values of workspace that ``moe_router_spread`` needs."""
+    return int(load().kvc_moe_router_spread_floats(tokens, experts))
+
+
+def moe_router_spread(choice: torch.Tensor, weight: torch.Tensor, sorted_pairs: torch.Tensor, tiles: torch.Tensor,
+                   num_tiles: torch.Tensor, x: torch.Tensor, router: torch.Tensor, work: torch.Tensor, *, top: int,
+                   tile_rows: int, groups: int = 1, keep: int = 1, score: str = "softmax",
+                   correction: torch.Tensor | None = None, group_best: int = 1, weight_scale: float = 1.0,
+                   bias: torch.Tensor | None = None, gate: torch.Tensor | None = None, renormalize: bool = True) -> None:
+    """:func:`moe_router` and :func:`moe_align` where ``moe_router_spread_supported``, with the same results; ``work`` float32, ``moe_router_spread_floats`` values."""
+    T, H = x.shape
+    E = router.shape[0] - (1 if gate is not None else 0)
+    if gate is not None and gate.numel() != T:
+        raise KernelError("moe_router_spread: a gate value a token")
+    if router.dim() != 2 or router.shape[1] != H or E < 1 or choice.shape != (T, top) or weight.shape != (T, top) or x.stride(1) != 1:
+        raise KernelError("moe_router_spread: shapes do not match")
+    if sorted_pairs.numel() < T * top or tiles.dim() != 2 or tiles.shape[1] != 3 or num_tiles.numel() < 1:
+        raise KernelError("moe_router_spread: buffers too small")
+    _check(load().kvc_moe_router_spread(
+        _dev(choice, "choice", torch.int32), _dev(weight, "weight", torch.float32), _dev(sorted_pairs, "sorted", torch.int32),
+        _dev(tiles, "tiles", torch.int32), _dev(num_tiles, "num_tiles", torch.int32), tiles.shape[0], tile_rows,
+        _dev(work, "work", torch.float32), work.numel(), x.data_ptr(), x.stride(0), _code(x, "x"),
+        _dev(router, "router", torch.float32), None if gate is None else _dev(gate, "gate", torch.float32), T, H, E, top,
+        groups, keep, *_route_rule(E, score, bias, correction, group_best, weight_scale, renormalize), _stream()),
+        "kvc_moe_router_spread")
+
+
 def moe_tile_rows(pairs: int, experts: int, x: torch.Tensor | None = None, k_sizes: tuple[int, ...] = ()) -> int:
-    """Rows a tile of the experts' products holds for a step of this size: 64 where the experts
-    have that many rows on average and the operands allow (bfloat16, every K a multiple of 32), else 16."""
+    """Rows a tile of the experts' products holds for a step of this size: 128 or 64 where the experts have
+    many rows on average and the operands allow (bfloat16, every K a multiple of 32), else 16."""
     rows = int(load().kvc_moe_tile_rows(pairs, experts))
     if rows > 16 and (x is None or x.dtype != torch.bfloat16 or any(k % 32 for k in k_sizes)):
         return 16

@@ -146,10 +146,9 @@ class RoutedExperts(FeedForward):
         choice = ctx.buf(f"moe_choice:{top}", top, torch.int32)
         weight = ctx.buf(f"moe_weight:{top}", top, torch.float32)
         gate = ctx.buf("moe_shared_gate", 1, torch.float32) if self.has_shared_gate else None
-        ops.moe_router(choice, weight, x, p["router.weight"], top=top, groups=self.groups, keep=self.keep,
-                       score=self.score, correction=p.get("correction"), group_best=self.group_best,
-                       weight_scale=self.weight_scale, bias=p.get("router.bias"), gate=gate,
-                       renormalize=self.renormalize)
+        rule = dict(top=top, groups=self.groups, keep=self.keep, score=self.score, correction=p.get("correction"),
+                    group_best=self.group_best, weight_scale=self.weight_scale, bias=p.get("router.bias"), gate=gate,
+                    renormalize=self.renormalize)
         cap = ctx.buffers.token_capacity
         sorted_pairs = ctx.buffers.get(f"moe_sorted:{top}", pairs, 1, torch.int32, reserve=cap * top).view(-1)
         # portions of prompts give the experts rows enough for tiles of 64, single tokens tiles of 16
@@ -158,7 +157,14 @@ class RoutedExperts(FeedForward):
         tiles = ctx.buffers.get(f"moe_tiles:{top}:{E}", max_tiles, 3, torch.int32,
                                 reserve=ops.moe_max_tiles(cap * top, E, 16))
         num_tiles = ctx.buffers.get("moe_num_tiles", 1, 1, torch.int32).view(-1)
-        ops.moe_align(sorted_pairs, tiles, num_tiles, choice, E, tile_rows)
+        if ops.moe_router_spread_supported(T, E):
+            work = ctx.buffers.get(f"moe_router_parts:{E}", T, ops.moe_router_spread_floats(1, E), torch.float32,
+                                   reserve=min(cap, ops.moe_router_spread_tokens()))
+            ops.moe_router_spread(choice, weight, sorted_pairs, tiles, num_tiles, x, p["router.weight"], work,
+                               tile_rows=tile_rows, **rule)
+        else:
+            ops.moe_router(choice, weight, x, p["router.weight"], **rule)
+            ops.moe_align(sorted_pairs, tiles, num_tiles, choice, E, tile_rows)
         act = ctx.buffers.get(f"moe_act:{I}", pairs, I, ctx.dtype, reserve=cap * top)
         ops.moe_gemm(act, x, p[f"experts.{self.first}"], sorted_pairs, tiles, num_tiles, pairs=pairs, experts=E,
                      in_div=top, out_sorted=True, gated=self.gated, limit=self.limit, alpha=self.alpha,

@@ -472,6 +472,93 @@ def test_the_feed_forward_of_routed_experts(dtype, E, top, groups, keep, H, I, s
         assert rel(again, first[perm].double()) < 1e-6
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("E,top,groups,keep,H,T,score,gated", [
+    (32, 4, 8, 4, 2048, 8, "softmax", False), (64, 8, 1, 1, 520, 64, "logit", True), (33, 5, 3, 2, 100, 17, "sigmoid", True),
+    (2, 2, 2, 1, 8, 1, "sigmoid", False), (40, 3, 10, 9, 2040, 256, "softmax", True), (1, 1, 1, 1, 32, 16, "logit", False), (16, 2, 4, 2, 64, 1000, "softmax", False)])
+def test_spread_router_and_tiles_are_those_of_the_two_kernels(dtype, E, top, groups, keep, H, T, score, gated):
+    """The same bits for choices, weights and gates, and the same tiles; a tile's pairs may stand in any order."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(E + T)
+    x = gpu(torch.randn(T, H, generator=gen), dtype)
+    x[T // 2] = 0  # every expert alike: the lowest indices
+    w = gpu(torch.randn(E + gated, H, generator=gen) * H ** -0.5)
+    bias = gpu(torch.randn(E, generator=gen) * 0.1) if score != "softmax" else None
+    correction = gpu(torch.randn(E, generator=gen)) if score == "sigmoid" else None
+    rule = dict(top=top, groups=groups, keep=keep, score=score, bias=bias, correction=correction, weight_scale=1.5,
+                group_best=2 if score == "sigmoid" else 1, renormalize=score != "sigmoid")
+    i32 = dict(dtype=torch.int32, device=DEV)
+    results = []
+    for few in (False, True):
+        choice, weight = torch.full((T, top), -1, **i32), torch.full((T, top), float("nan"), device=DEV)
+        gate = torch.full((T,), float("nan"), device=DEV) if gated else None
+        sorted_pairs, num = torch.full((T * top,), -1, **i32), torch.empty(1, **i32)
+        tiles = torch.full((ops.moe_max_tiles(T * top, E, 16), 3), -1, **i32)
+        if few:
+            work = torch.full((ops.moe_router_spread_floats(T, E),), float("nan"), device=DEV)
+            ops.moe_router_spread(choice, weight, sorted_pairs, tiles, num, x, w, work, tile_rows=16, gate=gate, **rule)
+        else:
+            ops.moe_router(choice, weight, x, w, gate=gate, **rule)
+            ops.moe_align(sorted_pairs, tiles, num, choice, E, 16)
+        listed = tiles[: int(num)].tolist()
+        pairs = sorted_pairs.tolist()
+        starts = {e: min(a for f, a, _ in listed if f == e) for e, _, _ in listed}
+        held = {e: sorted(pairs[starts[e]: starts[e] + sum(n for f, _, n in listed if f == e)]) for e in starts}
+        results.append((choice, weight, gate, listed, held))
+    (c0, w0, g0, l0, h0), (c1, w1, g1, l1, h1) = results
+    assert torch.equal(c0, c1) and torch.equal(w0, w1) and l0 == l1 and h0 == h1
+    assert g0 is None or torch.equal(g0, g1)
+    assert sum(len(v) for v in h1.values()) == T * top
+
+
+@pytest.mark.parametrize("tile_rows", [16, 64, 128])
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "packed"])
+@pytest.mark.parametrize("gated,N,K,out_dtype", [(True, 1024, 64, torch.bfloat16), (True, 176, 192, torch.bfloat16),
+                                                 (False, 2048, 128, torch.float32), (False, 48, 64, torch.float32),
+                                                 (True, 40, 96, torch.float32), (False, 300, 160, torch.bfloat16)])
+def test_products_of_experts_over_tiles_of_many_rows(tile_rows, packed, gated, N, K, out_dtype):
+    """Experts with no row, one, a few, exactly a tile's, one more and several tiles' worth; columns that end
+    inside a block; sums that end inside a pass (a packed matrix has none of the two)."""
+    from kvcore_amd.ops import library as ops
+
+    if packed and (N % 16 or K % 64):
+        pytest.skip("a packed matrix has experts of a multiple of 16 rows of a multiple of 64")
+    gen = torch.Generator().manual_seed(N + K)
+    counts = [0, 1, 16, 17, tile_rows - 1, tile_rows, tile_rows + 1, 3, 2 * tile_rows + 5, 0]
+    E, T = len(counts), sum(counts)
+    choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=gen)]
+    x = torch.randn(T, K, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(E * N * (2 if gated else 1), K, generator=gen) * K ** -0.5).to(torch.bfloat16)
+    scale = torch.rand(T, generator=gen) + 0.5
+    wg = gpu(w, torch.bfloat16)
+    if packed:
+        ops.pack_weight(wg)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+    tiles = torch.empty(ops.moe_max_tiles(T, E, tile_rows), 3, **i32)
+    ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32).view(T, 1), E, tile_rows)
+    listed = tiles[: int(num)].tolist()
+    assert all(1 <= n <= tile_rows for _, _, n in listed)
+    assert [sum(n for e, _, n in listed if e == which) for which in range(E)] == counts
+    out = torch.full((T, N), float("nan"), dtype=out_dtype, device=DEV)
+    ops.moe_gemm(out, gpu(x, torch.bfloat16), wg, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1, out_sorted=False,
+                 gated=gated, limit=1.2, alpha=1.702, up_shift=1.0, tile_rows=tile_rows, row_scale=gpu(scale),
+                 act=None if gated else "relu_squared")
+    want = torch.empty(T, N, dtype=torch.float64)
+    per = w.double().view(E, -1, K)
+    for e in range(E):
+        at = choice == e
+        y = (x[at].double() @ per[e].T) * scale[at, None].double()
+        if gated:
+            g, u = y[:, :N].clamp(max=1.2), y[:, N:].clamp(-1.2, 1.2)
+            want[at] = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            want[at] = y.clamp(min=0) ** 2
+    # float32 sums of exact products; a bfloat16 result adds one rounding of 2^-9
+    assert rel(out, want) < (2e-6 if out_dtype == torch.float32 else 3e-3)
+
+
 def test_offset_norm_keeps_a_gain_of_one_plus_the_stored_weight():
     from kvcore_amd.parts.base import Runtime
     from kvcore_amd.parts.rmsnorm import RMSNorm
