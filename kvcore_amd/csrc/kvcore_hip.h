@@ -229,7 +229,7 @@ int kvc_ssm_scan(float* y, const float* xbc, int64_t xbc_stride, const void* dt_
                  int64_t dt_stride, int dt_dtype, const float* dt_bias, const float* a_log,
                  const float* d_skip, float* state, const int32_t* positions,
                  const int32_t* token_req, const int32_t* q_start, const int32_t* slots, int R,
-                 int nh, int P, int N, int G, kvc_stream stream);
+                 int nh, int P, int N, int G, int below, kvc_stream stream);
 // out[t, c] = gain[c] * v / sqrt(mean of v^2 over c's part + eps), v = y[t, c] * silu(z[t, c]),
 // the width cut into `groups` equal parts.
 int kvc_gated_group_rmsnorm(void* out, int out_dtype, const float* y, const void* z,
@@ -248,13 +248,14 @@ int kvc_gated_group_rmsnorm(void* out, int out_dtype, const float* y, const void
 // beta are float32 rows with strides.  d at most 256.  With ones_column the rows of v hold dv - 1
 // values a head and column dv - 1 of every head takes a one for each token: a normaliser that is
 // gated and read like the matrix, out[t, h, dv - 1] being its product with the query.  silu_in: q, k and v
-// pass through silu on their way in (q before its scale; delta_rule 2 without beta only).
+// pass through silu on their way in (q before its scale; delta_rule 2 without beta only).  below > 0: requests of
+// that many tokens and more in the step are left alone (so for kvc_ssm_scan).
 int kvc_linear_state_scan(float* out, const float* q, int64_t q_stride, const float* k,
                           int64_t k_stride, const float* v, int64_t v_stride, const float* decay,
                           int64_t decay_stride, const float* beta, int64_t beta_stride, float* state,
                           const int32_t* positions, const int32_t* token_req, const int32_t* q_start,
                           const int32_t* slots, int R, int nh, int nqk, int d, int dv, int delta_rule,
-                          float q_scale, int ones_column, int silu_in, kvc_stream stream);
+                          float q_scale, int ones_column, int silu_in, int below, kvc_stream stream);
 // delta_rule 2 with a fixed decay per head (decay [nh], no beta) over portions of prompts, in chunks of
 // kvc_fixed_decay_chunk_tokens() tokens side by side (chunked_state.hip): the same results as the scan's, up to
 // the order of sums.  work: work_chunks >= min(T, T / chunk + R) chunks of nh * dpad * dv floats each.
@@ -264,6 +265,23 @@ int kvc_fixed_decay_chunks(float* out, const float* q, int64_t q_stride, const f
                            int64_t work_chunks, const int32_t* positions, const int32_t* token_req,
                            const int32_t* q_start, const int32_t* slots, int T, int R, int nh, int nqk, int d,
                            int dv, float q_scale, int silu_in, kvc_stream stream);
+// The same for gates that change from token to token (gated_chunks.hip): kvc_linear_state_scan with delta_rule 2
+// (keep = decay, take = beta), and kvc_ssm_scan, for the requests of at least `from` tokens in the step, whose
+// tokens make `chunks` chunks of kvc_gated_chunk_tokens(); states of at most 128 rows.  work: kvc_gated_chunk_floats
+// floats (of nh heads, nqk or G of which have keys of their own, and states of d x dv) a chunk.
+int kvc_gated_chunk_tokens(void);
+int64_t kvc_gated_chunk_floats(int nh, int nqk, int d, int dv);
+int kvc_scalar_gate_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride,
+                           const float* v, int64_t v_stride, const float* keep, int64_t keep_stride,
+                           const float* take, int64_t take_stride, float* state, float* work, int64_t work_floats,
+                           const int32_t* positions, const int32_t* token_req, const int32_t* q_start,
+                           const int32_t* slots, int chunks, int from, int R, int nh, int nqk, int d, int dv,
+                           float q_scale, int ones_column, kvc_stream stream);
+int kvc_ssm_chunks(float* y, const float* xbc, int64_t xbc_stride, const void* dt_raw, int64_t dt_stride,
+                   int dt_dtype, const float* dt_bias, const float* a_log, const float* d_skip, float* state,
+                   float* work, int64_t work_floats, const int32_t* positions, const int32_t* token_req,
+                   const int32_t* q_start, const int32_t* slots, int chunks, int from, int R, int nh, int P, int N,
+                   int G, kvc_stream stream);
 // The gates of a matrix memory with log gates and a running maximum m (mLSTM), per request in
 // token order: i = cap tanh((i_raw + i_bias) / cap), f = logsigmoid(cap tanh((f_raw + f_bias) / cap)),
 // m_t = max(f + m_(t-1), i), keep[t, h] = exp(f + m_(t-1) - m_t), take[t, h] = exp(i - m_t),

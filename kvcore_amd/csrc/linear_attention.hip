@@ -66,7 +66,7 @@ __global__ __launch_bounds__(256) void linear_state_scan_kernel(
     int64_t decay_stride, const float* __restrict__ beta, int64_t beta_stride, float* __restrict__ state,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, int nh, int nqk, int d,
-    int dv, float q_scale, int scalar_gates, int ones_column, int silu_in) {
+    int dv, float q_scale, int scalar_gates, int ones_column, int silu_in, int below) {
   constexpr int VT = 256 / NSL;  // value channels a block
   // with ones_column the rows of v hold dv - 1 values a head and the last column of the state's dv
   // takes a one for every token (a normaliser kept beside the matrix)
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256) void linear_state_scan_kernel(
   const bool c_ok = c < dv;
   const int width = nh * dv;
   const int b = q_start[r], e = q_start[r + 1];
-  if (e <= b) return;
+  if (e <= b || e - b >= below) return;
   if (token_req[b] < 0) {  // padding rows: zeros out, no state touched
     for (int idx = tid; idx < (e - b) * VT; idx += nthreads) {
       const int tt = idx / VT, cc = c0 + idx - tt * VT;
@@ -576,7 +576,7 @@ extern "C" int kvc_linear_state_scan(float* out, const float* q, int64_t q_strid
                                      int64_t beta_stride, float* state, const int32_t* positions,
                                      const int32_t* token_req, const int32_t* q_start,
                                      const int32_t* slots, int R, int nh, int nqk, int d, int dv,
-                                     int rule, float q_scale, int ones_column, int silu_in,
+                                     int rule, float q_scale, int ones_column, int silu_in, int below,
                                      kvc_stream stream) {
   ones_column = ones_column ? 1 : 0;
   if (rule < 0 || rule > 2) return kvc_fail("kvc_linear_state_scan: the rule is 0 (key decay), 1 (delta) or 2 (scalar gates)");
@@ -608,7 +608,7 @@ extern "C" int kvc_linear_state_scan(float* out, const float* q, int64_t q_strid
   hipLaunchKernelGGL((linear_state_scan_kernel<NPT, DELTA, NSL_, FULL_, PF_>), grid, dim3(256),               \
                      lds*(PF_ ? 2 : 1), S(stream), out, q, q_stride, k, k_stride, v, v_stride, decay,         \
                      decay_stride, beta, beta_stride, state, positions, token_req, q_start, slots, nh, nqk, d, \
-                     dv, q_scale, scalar_gates, ones_column, silu_in)
+                     dv, q_scale, scalar_gates, ones_column, silu_in, below > 0 ? below : 0x7fffffff)
   // two sets of LDS buffers (the next stage fetched while one is worked on) where a stage's values
   // deal out evenly to the threads and both sets fit the 64 KB a block may take
 #define KVC_LSCAN(NPT, DELTA, NSL_)                                                  \

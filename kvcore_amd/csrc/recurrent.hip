@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(
     const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, int nh, int P, int N,
-    int G, int PT) {
+    int G, int PT, int below) {
   extern __shared__ float lds[];
   float* b_s = lds;                    // [SC][N]
   float* c_s = b_s + SC * N;           // [SC][N]
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(
   const bool p_ok = p < P;
   const int inner = nh * P;
   const int b = q_start[r], e = q_start[r + 1];
-  if (e <= b) return;
+  if (e <= b || e - b >= below) return;
   if (token_req[b] < 0) {
     for (int idx = tid; idx < (e - b) * PT; idx += nthreads) {
       const int tt = idx / PT, q = p0 + idx - tt * PT;
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(
     const float* __restrict__ a_log, const float* __restrict__ d_skip, float* __restrict__ state,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, int nh, int P, int N,
-    int G) {
+    int G, int below) {
   constexpr int NSL = 256 / PT;            // threads that share a column of the state
   constexpr int NP = NSL * NPT;            // padded rows of the state
   constexpr int NB = SC * NP / 256;        // values of B (and of C) a thread fetches per stage
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(
   const bool p_ok = p < P;
   const int inner = nh * P;
   const int b = q_start[r], e = q_start[r + 1];
-  if (e <= b) return;
+  if (e <= b || e - b >= below) return;
   if (token_req[b] < 0) {
     for (int idx = tid; idx < (e - b) * PT; idx += 256) {
       const int tt = idx / PT, q = p0 + idx - tt * PT;
@@ -721,7 +721,8 @@ extern "C" int kvc_ssm_scan(float* y, const float* xbc, int64_t xbc_stride, cons
                             const float* a_log, const float* d_skip, float* state,
                             const int32_t* positions, const int32_t* token_req,
                             const int32_t* q_start, const int32_t* slots, int R, int nh, int P, int N,
-                            int G, kvc_stream stream) {
+                            int G, int below, kvc_stream stream) {
+  if (below <= 0) below = 0x7fffffff;
   if (R < 0 || nh <= 0 || P <= 0 || N <= 0 || G <= 0 || nh % G)
     return kvc_fail("kvc_ssm_scan: bad sizes");
   if (N > NS * 64) return kvc_fail("kvc_ssm_scan: a state of more than 256 rows a head");
@@ -739,14 +740,14 @@ extern "C" int kvc_ssm_scan(float* y, const float* xbc, int64_t xbc_stride, cons
                      hipLaunchKernelGGL((ssm_scan_kernel<NPT, TD>), grid, block, lds, S(stream), y, \
                                         xbc, xbc_stride, static_cast<const TD*>(dt_raw), dt_stride, \
                                         dt_bias, a_log, d_skip, state, positions, token_req,       \
-                                        q_start, slots, nh, P, N, G, PT))
+                                        q_start, slots, nh, P, N, G, PT, below))
 #define KVC_SSM_LAUNCH_WIDE(NPT, PTW)                                                              \
   KVC_DISPATCH_DTYPE(dt_dtype, TD,                                                                 \
                      hipLaunchKernelGGL((ssm_scan_wide_kernel<NPT, PTW, TD>),                      \
                                         dim3(R, nh, (P + PTW - 1) / PTW), dim3(256), 0, S(stream), \
                                         y, xbc, xbc_stride, static_cast<const TD*>(dt_raw),        \
                                         dt_stride, dt_bias, a_log, d_skip, state, positions,       \
-                                        token_req, q_start, slots, nh, P, N, G))
+                                        token_req, q_start, slots, nh, P, N, G, below))
   // tiles of 16 value channels (sixteen threads a column of the state) where tiles of 64 would
   // give fewer blocks than the chip has compute units
   const int64_t wide_blocks = static_cast<int64_t>(R) * nh * ((P + 63) / 64);

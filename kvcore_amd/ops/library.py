@@ -61,8 +61,10 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_kv_slots": [P, P, P, P, P, I, I, I, I, P],
         "kvc_rope_kv_write": [P, P, P, P, P, I, I, P, I, I, I, I, I, I, I, I, P],
         "kvc_paged_attention": [P, P, L, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P, I, P, F, P, L, I, I, P],
-        "kvc_linear_state_scan": [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P],
+        "kvc_linear_state_scan": [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, I, I, P],
         "kvc_fixed_decay_chunks": [P, P, L, P, L, P, L, P, P, P, L, P, P, P, P, I, I, I, I, I, I, F, I, P],
+        "kvc_scalar_gate_chunks": [P, P, L, P, L, P, L, P, L, P, L, P, P, L, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
+        "kvc_ssm_chunks": [P, P, L, P, L, I, P, P, P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, P],
         "kvc_sigmoid_power": [P, P, L, P, F, I, I, P],
         "kvc_decay_and_write_gates": [P, P, P, L, P, L, P, P, I, I, P],
         "kvc_unit_heads": [P, L, I, I, I, F, F, I, F, P],
@@ -84,7 +86,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_causal_conv": [P, L, I, P, L, I, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "kvc_rglru_gates": [P, P, P, P, P, P, P, P, F, I, I, I, P],
         "kvc_rglru_scan": [P, I, P, P, P, L, I, P, P, P, P, P, I, I, I, P, L, P],
-        "kvc_ssm_scan": [P, P, L, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
+        "kvc_ssm_scan": [P, P, L, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P],
         "kvc_gated_group_rmsnorm": [P, I, P, P, L, I, P, F, I, I, I, P],
         "kvc_decode_attention": [P, P, P, P, L, P, P, P, I, P, P, P, P, P, P, I, I, P, P, F, I, I, I, I, I, I,
                                  I, I, F, I, P, I, P, F, P, L, I, I, I, P],
@@ -130,6 +132,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvc_ssm_scan_max_state.argtypes = []
     lib.kvc_fixed_decay_chunk_tokens.restype = c_int
     lib.kvc_fixed_decay_chunk_tokens.argtypes = []
+    lib.kvc_gated_chunk_floats.restype = c_int64
+    lib.kvc_gated_chunk_floats.argtypes = [c_int] * 4
+    lib.kvc_gated_chunk_tokens.restype = c_int
+    lib.kvc_gated_chunk_tokens.argtypes = []
     lib.kvc_rglru_scan_segment.restype = c_int
     lib.kvc_rglru_scan_segment.argtypes = []
 
@@ -1539,11 +1545,11 @@ def ssm_scan_max_state() -> int:
 def ssm_scan(y: torch.Tensor, xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor,
              a_log: torch.Tensor, d_skip: torch.Tensor, state: torch.Tensor, *, positions: torch.Tensor,
              token_req: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, num_reqs: int,
-             heads: int, head_dim: int, state_size: int, groups: int) -> None:
+             heads: int, head_dim: int, state_size: int, groups: int, below: int = 0) -> None:
     """The state-space recurrence with a scalar decay per head (see the C header): ``xbc [T, heads
     * head_dim + 2 * groups * state_size]`` float32 (x, B, C after their convolution), ``dt_raw
     [T, heads]`` (a column view is fine), ``state [slots, heads, state_size, head_dim]`` float32,
-    ``y [T, heads * head_dim]`` float32."""
+    ``y [T, heads * head_dim]`` float32.  ``below`` > 0: requests of that many tokens and more are left alone."""
     T = xbc.shape[0]
     inner = heads * head_dim
     if y.shape != (T, inner) or not y.is_contiguous() or y.dtype != torch.float32:
@@ -1562,7 +1568,81 @@ def ssm_scan(y: torch.Tensor, xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: 
         _dev(a_log, "a_log", f), _dev(d_skip, "d_skip", f), _dev(state, "state"),
         _dev(positions, "positions", torch.int32), _dev(token_req, "token_req", torch.int32),
         _dev(q_start, "q_start", torch.int32), _dev(slots, "slots", torch.int32), num_reqs, heads,
-        head_dim, state_size, groups, _stream()), "kvc_ssm_scan")
+        head_dim, state_size, groups, below, _stream()), "kvc_ssm_scan")
+
+
+def gated_chunk_count(lengths, start: int) -> int:
+    """Chunks that the requests of at least ``start`` tokens among ``lengths`` (tokens in the step) are cut into."""
+    chunk = int(load().kvc_gated_chunk_tokens())
+    return sum(-(-n // chunk) for n in lengths if n >= start)
+
+
+def gated_chunk_work(buffers, name: str, chunks: int, start: int, heads: int, key_heads: int, rows: int,
+                     cols: int) -> torch.Tensor:
+    """The step buffer that ``ssm_chunks`` and ``scalar_gate_chunks`` work in: a row for each of ``chunks`` chunks (of
+    requests of at least ``start`` tokens), for states of ``rows x cols`` a head."""
+    lib = load()
+    each = int(lib.kvc_gated_chunk_floats(heads, key_heads, rows, cols))
+    capacity = buffers.token_capacity  # every request of at least `start` tokens may end in a ragged chunk
+    most = capacity // int(lib.kvc_gated_chunk_tokens()) + capacity // max(start, 1) + 1
+    return buffers.get(f"{name}:{each}", chunks, each, torch.float32, reserve=most)
+
+
+def ssm_chunks(y: torch.Tensor, xbc: torch.Tensor, dt_raw: torch.Tensor, dt_bias: torch.Tensor, a_log: torch.Tensor,
+               d_skip: torch.Tensor, state: torch.Tensor, work: torch.Tensor, *, positions: torch.Tensor,
+               token_req: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, num_reqs: int, heads: int,
+               head_dim: int, state_size: int, groups: int, chunks: int, start: int = 1) -> None:
+    """:func:`ssm_scan` for the requests of at least ``start`` tokens, ``chunks`` chunks of tokens side by side
+    (:func:`gated_chunk_count`); ``work``: :func:`gated_chunk_work`."""
+    T = xbc.shape[0]
+    inner = heads * head_dim
+    if y.shape != (T, inner) or not y.is_contiguous() or y.dtype != torch.float32:
+        raise KernelError("ssm_chunks: y must be contiguous float32 [T, heads * head_dim]")
+    if tuple(state.shape[1:]) != (heads, state_size, head_dim) or state.dtype != torch.float32:
+        raise KernelError("ssm_chunks: state must be float32 [slots, heads, state_size, head_dim]")
+    if dt_bias.numel() != heads or a_log.numel() != heads or d_skip.numel() != heads or dt_raw.shape[0] < T:
+        raise KernelError("ssm_chunks: a value per head for dt_bias, a_log and d_skip, a row of dt_raw a token")
+    if positions.numel() < T or token_req.numel() < T or q_start.numel() < num_reqs + 1:
+        raise KernelError("ssm_chunks: index arrays too short")
+    x_ptr, x_stride, x_code = _rows(xbc, "xbc", inner + 2 * groups * state_size)
+    if x_code != 0:
+        raise KernelError("ssm_chunks: xbc must be float32")
+    d_ptr, d_stride, d_code = _rows(dt_raw, "dt_raw", heads)
+    f, i32 = torch.float32, torch.int32
+    _check(load().kvc_ssm_chunks(
+        y.data_ptr(), x_ptr, x_stride, d_ptr, d_stride, d_code, _dev(dt_bias, "dt_bias", f), _dev(a_log, "a_log", f),
+        _dev(d_skip, "d_skip", f), _dev(state, "state"), _dev(work, "work", f), work.numel(),
+        _dev(positions, "positions", i32), _dev(token_req, "token_req", i32), _dev(q_start, "q_start", i32),
+        _dev(slots, "slots", i32), chunks, start, num_reqs, heads, head_dim, state_size, groups, _stream()), "kvc_ssm_chunks")
+
+
+def scalar_gate_chunks(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, keep: torch.Tensor,
+                       take: torch.Tensor, state: torch.Tensor, work: torch.Tensor, *, positions: torch.Tensor,
+                       token_req: torch.Tensor, q_start: torch.Tensor, slots: torch.Tensor, num_reqs: int, heads: int,
+                       qk_heads: int, dim: int, vdim: int, chunks: int, start: int = 1, q_scale: float = 1.0,
+                       ones_column: bool = False) -> None:
+    """:func:`linear_state_scan` with ``scalar_gates`` for the requests of at least ``start`` tokens, ``chunks`` chunks
+    of tokens side by side (:func:`gated_chunk_count`); ``work``: :func:`gated_chunk_work`."""
+    T = out.shape[0]
+    if out.shape != (T, heads * vdim) or not out.is_contiguous() or out.dtype != torch.float32:
+        raise KernelError("scalar_gate_chunks: out must be contiguous float32 [T, heads * vdim]")
+    if tuple(state.shape[1:]) != (heads, linear_state_rows(dim), vdim) or state.dtype != torch.float32 \
+            or not state.is_contiguous():
+        raise KernelError("scalar_gate_chunks: state must be float32 [slots, heads, linear_state_rows(dim), vdim]")
+    if min(q.shape[0], k.shape[0], v.shape[0], keep.shape[0], take.shape[0]) < T or positions.numel() < T \
+            or token_req.numel() < T or q_start.numel() < num_reqs + 1:
+        raise KernelError("scalar_gate_chunks: rows or index arrays too short")
+    qp, qs = _f32_rows(q, "q", qk_heads * dim)
+    kp, ks = _f32_rows(k, "k", qk_heads * dim)
+    vp, vs = _f32_rows(v, "v", heads * (vdim - 1 if ones_column else vdim))
+    gp, gs = _f32_rows(keep, "keep", heads)
+    tp, ts = _f32_rows(take, "take", heads)
+    f, i32 = torch.float32, torch.int32
+    _check(load().kvc_scalar_gate_chunks(
+        out.data_ptr(), qp, qs, kp, ks, vp, vs, gp, gs, tp, ts, _dev(state, "state"), _dev(work, "work", f), work.numel(),
+        _dev(positions, "positions", i32), _dev(token_req, "token_req", i32), _dev(q_start, "q_start", i32),
+        _dev(slots, "slots", i32), chunks, start, num_reqs, heads, qk_heads, dim, vdim, float(q_scale),
+        int(bool(ones_column)), _stream()), "kvc_scalar_gate_chunks")
 
 
 def gated_group_rmsnorm(out: torch.Tensor, y: torch.Tensor, z: torch.Tensor, gain: torch.Tensor,
@@ -1597,7 +1677,8 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
                       positions: torch.Tensor, token_req: torch.Tensor, q_start: torch.Tensor,
                       slots: torch.Tensor, num_reqs: int, heads: int, qk_heads: int, dim: int,
                       vdim: int, delta_rule: bool = False, q_scale: float = 1.0,
-                      scalar_gates: bool = False, ones_column: bool = False, silu_in: bool = False) -> None:
+                      scalar_gates: bool = False, ones_column: bool = False, silu_in: bool = False,
+                      below: int = 0) -> None:
     """The recurrence of a matrix state per head (see the C header): ``q, k [T, qk_heads * dim]``,
     ``v [T, heads * vdim]``, all float32 rows (column views are fine); ``decay [T, heads * dim]``
     (a factor per key channel) or, with ``delta_rule``, ``decay`` and ``beta [T, heads]``; with
@@ -1607,7 +1688,7 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
     columns takes a one for every token (a normaliser beside the matrix);
     ``state [slots, heads, linear_state_rows(dim), vdim]`` float32, in an order of the kernel's own;
     ``out [T, heads * vdim]`` float32.  ``q_scale``
-    multiplies every q on its way in."""
+    multiplies every q on its way in.  ``below`` > 0: requests of that many tokens and more are left alone."""
     T = out.shape[0]
     if out.shape != (T, heads * vdim) or not out.is_contiguous() or out.dtype != torch.float32:
         raise KernelError("linear_state_scan: out must be contiguous float32 [T, heads * vdim]")
@@ -1637,7 +1718,7 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
         _dev(positions, "positions", torch.int32), _dev(token_req, "token_req", torch.int32),
         _dev(q_start, "q_start", torch.int32), _dev(slots, "slots", torch.int32), num_reqs, heads,
         qk_heads, dim, vdim, 2 if scalar_gates else int(bool(delta_rule)), float(q_scale), int(bool(ones_column)),
-        int(bool(silu_in)), _stream()),
+        int(bool(silu_in)), below, _stream()),
         "kvc_linear_state_scan")
 
 

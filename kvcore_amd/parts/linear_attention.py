@@ -37,6 +37,10 @@ from .base import Mixer, ParamSource, ParamSpec, StateNeed, register_mixer
 
 # from so many tokens of one request in a step on, lightning attention works in chunks
 CHUNKED_FROM = 48
+# and a bfloat16 model's matrix memories (16 heads of 64 x 129: 128 tokens 28 us token by token and 31 in chunks, eight
+# requests of 128 tokens 67 and 47, 2,048 tokens 405 and 57); a float32 model walks every token, so that its results
+# do not depend on how a request is cut into steps
+GATED_CHUNKED_FROM = 128
 
 
 def _src(name: str, rows: int) -> tuple[ParamSource, ...]:
@@ -274,9 +278,17 @@ class MaxGatedMatrixMemory(_MatrixStateMixer):
                       maxima, **batch)
         wide = nh * (self.vdim + 1)
         o = ctx.buf(f"mm_o:{wide}", wide, torch.float32)
-        ops.linear_state_scan(o, proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], keep, take, state,
-                              heads=nh, qk_heads=nh, dim=self.dim, vdim=self.vdim + 1, scalar_gates=True,
-                              ones_column=True, q_scale=self.q_scale, **batch)
+        rows = (proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], keep, take, state)
+        sizes = dict(heads=nh, qk_heads=nh, dim=self.dim, vdim=self.vdim + 1, ones_column=True, q_scale=self.q_scale)
+        chunks = 0
+        if ctx.dtype == torch.bfloat16 and self.dim <= 128:
+            chunks = ops.gated_chunk_count(ctx.host_query_lens, GATED_CHUNKED_FROM)
+        if chunks:
+            work = ops.gated_chunk_work(ctx.buffers, "mm_chunks", chunks, GATED_CHUNKED_FROM, nh, nh, self.dim,
+                                        self.vdim + 1)
+            ops.scalar_gate_chunks(o, *rows, work, chunks=chunks, start=GATED_CHUNKED_FROM, **sizes, **batch)
+        if not chunks or min(ctx.host_query_lens) < GATED_CHUNKED_FROM:
+            ops.linear_state_scan(o, *rows, scalar_gates=True, below=GATED_CHUNKED_FROM if chunks else 0, **sizes, **batch)
         normed = ctx.buf(f"ms_normed:{inner}", inner)
         ops.max_gated_finish(normed, o, m, proj[:, 2 * qk + inner:2 * qk + 2 * inner], p["norm"], self.eps,
                              self.den_eps, nh, self.vdim)

@@ -36,6 +36,12 @@ def _src(name: str, rows: int) -> tuple[ParamSource, ...]:
     return (ParamSource(name, 0, rows),)
 
 
+# from so many tokens of one request in a step on, a bfloat16 model's state-space layers work in chunks (64 heads of
+# 128 x 64: 128 tokens 27 us token by token and 37 in chunks, 256 tokens 49 and 41, 2,048 tokens 383 and 127); a
+# float32 model walks every token, so that its results do not depend on how a request is cut into steps
+SSM_CHUNKED_FROM = 192
+
+
 class GatedLinearRecurrence(Mixer):
     """``width`` channels in ``blocks`` equal parts for the gates, a convolution of ``conv``
     taps, decay constant ``decay_scale`` (the c above).  ``tensor_names`` renames checkpoint
@@ -191,8 +197,17 @@ class StateSpaceMixer(Mixer):
         ops.causal_conv(xbc, xbc_raw, p["conv.weight"], p["conv.bias"], conv_state, act="silu",
                         single_tokens=ctx.max_query_len == 1, **batch)
         y = ctx.buf(f"ssm_y:{self.inner}", self.inner, torch.float32)
-        ops.ssm_scan(y, xbc, dt_raw, p["dt_bias"], p["A_log"], p["D"], ssm_state, heads=self.heads,
-                     head_dim=self.head_dim, state_size=self.state_size, groups=self.groups, **batch)
+        sizes = dict(heads=self.heads, head_dim=self.head_dim, state_size=self.state_size, groups=self.groups)
+        chunks = 0
+        if ctx.dtype == torch.bfloat16 and self.state_size <= 128:
+            chunks = ops.gated_chunk_count(ctx.host_query_lens, SSM_CHUNKED_FROM)
+        rows = (y, xbc, dt_raw, p["dt_bias"], p["A_log"], p["D"], ssm_state)
+        if chunks:
+            work = ops.gated_chunk_work(ctx.buffers, "ssm_chunks", chunks, SSM_CHUNKED_FROM, self.heads, self.groups,
+                                        self.state_size, self.head_dim)
+            ops.ssm_chunks(*rows, work, chunks=chunks, start=SSM_CHUNKED_FROM, **sizes, **batch)
+        if not chunks or min(ctx.host_query_lens) < SSM_CHUNKED_FROM:
+            ops.ssm_scan(*rows, below=SSM_CHUNKED_FROM if chunks else 0, **sizes, **batch)
         normed = ctx.buf(f"ssm_normed:{self.inner}", self.inner)
         ops.gated_group_rmsnorm(normed, y, z, p["norm.weight"], self.eps, self.norm_groups)
         out = ctx.buf("mixer_out", self.hidden_size)
