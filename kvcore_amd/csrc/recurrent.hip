@@ -151,97 +151,131 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
 // The channels are cut into nb blocks of bw; in block b, r = sigmoid(Wa[b] u_b + ba) and
 // i = sigmoid(Wi[b] u_b + bi) with square matrices [out, in].  Then log a = -c r softplus(lam),
 // a = exp(log a), and the driven input sqrt(1 - a^2) i u, with 1 - a^2 taken as
-// -expm1(2 log a).  A block of 256 threads owns 16 tokens x 64 outputs of one channel block
-// and walks the inputs 32 at a time through LDS; each thread sums two dot products for four
-// tokens in the order k = 0, 1, ...
-constexpr int GT = 16, GK = 32;
+// -expm1(2 log a).
+//
+// A wave takes 16 outputs of both matrices x TT tiles of 16 tokens along the whole of a channel
+// block, on the float32 matrix instructions (float32 products, float32 sums), its operands from
+// memory to registers AHEAD chunks of 32 inputs ahead (a lane 32 contiguous bytes).  A result is
+// made in the same order whatever the tile: chunk by chunk, and within one eight 16 x 16 x 4
+// instructions, of which number j takes the inputs k + j, k + 8 + j, k + 16 + j, k + 24 + j.
+// A block's waves are neighbours along the tokens and share the matrices' rows through the
+// cache.  2,048 tokens of 2,560 channels in blocks of 256: 92 us, of which the products take 34
+// at the matrix rate and the exponentials, quotients and roots of the results some 30 (blocks
+// of 16 channels, 38 us); two tiles of outputs or four of tokens a wave 89 to 160 us, with the
+// fewer waves in flight that their registers leave no better over other sizes.  Through LDS with
+// a multiply and an add a step it took 129 us.
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+constexpr int GK = 32;
 
-// GO outputs a block and TPT = GO / 16 tokens a thread: 64 and 4 for many tokens; 16 and 1 for
-// steps of few tokens, whose blocks are then four times as many (the weights, read once, are
-// all the work there, and a launch of a few dozen blocks leaves most of the chip idle).
-template <int GO, int TPT>
+// eight inputs of a row from k on, zeros beyond the block (VEC: whole 16-byte pieces)
+template <int VEC>
+__device__ __forceinline__ void gate_load8(f32x4_t* v, const float* row, int k, int bw) {
+  if constexpr (VEC) {
+    const float* p = row + (k < bw ? k : 0);
+    v[0] = *reinterpret_cast<const f32x4_t*>(p);
+    v[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
+    if (k >= bw) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = k + i < bw ? row[k + i] : 0.f;
+  }
+}
+
+template <int TT, int AHEAD, int VEC>
 __global__ __launch_bounds__(256) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
     int bw, int out_tiles) {
-  static_assert(GO * (GT / TPT) == 256, "a thread per (output, group of tokens)");
-  __shared__ float wa_s[GO][GK + 1];
-  __shared__ float wi_s[GO][GK + 1];
-  __shared__ float u_s[GT][GK];
-  const int tid = threadIdx.x;
-  const int t0 = blockIdx.x * GT;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int t0 = (blockIdx.x * (blockDim.x >> 6) + wave) * 16 * TT;
+  if (t0 >= T) return;
   const int blk = blockIdx.y / out_tiles;
-  const int o0 = (blockIdx.y - blk * out_tiles) * GO;
-  const int ol = tid % GO;
-  const int tg = tid / GO;
-  const float* wa_b = wa + static_cast<int64_t>(blk) * bw * bw;
-  const float* wi_b = wi + static_cast<int64_t>(blk) * bw * bw;
-  float acc_a[TPT], acc_i[TPT];
+  const int o0 = (blockIdx.y - blk * out_tiles) * 16;
+  // outputs and tokens beyond the last read the last one and are not stored
+  const int64_t row = (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
+  const float *wa_row = wa + row, *wi_row = wi + row, *u_row[TT];
 #pragma unroll
-  for (int tt = 0; tt < TPT; ++tt) acc_a[tt] = acc_i[tt] = 0.f;
-  // a stage of 32 inputs is fetched into registers while the stage before it is multiplied
-  constexpr int NW = GO * GK / 256, NU = GT * GK / 256;
-  float wa_r[NW], wi_r[NW], u_r[NU];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / GK, col = idx - row * GK;
-      const bool ok = o0 + row < bw && k0 + col < bw;
-      const int64_t off = static_cast<int64_t>(o0 + row) * bw + k0 + col;
-      wa_r[i] = ok ? wa_b[off] : 0.f;
-      wi_r[i] = ok ? wi_b[off] : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      const int idx = tid + i * 256;
-      const int row = idx / GK, col = idx - row * GK;
-      const bool ok = t0 + row < T && k0 + col < bw;
-      u_r[i] = ok ? u[static_cast<int64_t>(t0 + row) * W + blk * bw + k0 + col] : 0.f;
-    }
-  };
-  fetch(0);
-  for (int k0 = 0; k0 < bw; k0 += GK) {
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      const int idx = tid + i * 256;
-      wa_s[idx / GK][idx % GK] = wa_r[i];
-      wi_s[idx / GK][idx % GK] = wi_r[i];
-    }
-#pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      const int idx = tid + i * 256;
-      u_s[idx / GK][idx % GK] = u_r[i];
-    }
-    __syncthreads();
-    if (k0 + GK < bw) fetch(k0 + GK);
-#pragma unroll 8
-    for (int k = 0; k < GK; ++k) {
-      const float va = wa_s[ol][k], vi = wi_s[ol][k];
-#pragma unroll
-      for (int tt = 0; tt < TPT; ++tt) {
-        const float uv = u_s[tg * TPT + tt][k];
-        acc_a[tt] = fmaf(va, uv, acc_a[tt]);
-        acc_i[tt] = fmaf(vi, uv, acc_i[tt]);
-      }
-    }
-    __syncthreads();
+  for (int t = 0; t < TT; ++t) {
+    const int tok = t0 + 16 * t + li;
+    u_row[t] = u + static_cast<int64_t>(tok < T ? tok : T - 1) * W + blk * bw;
   }
-  if (o0 + ol >= bw) return;
-  const int c = blk * bw + o0 + ol;
-  const float sp = softplus_f(lam[c]);
-  const float b_a = ba[c], b_i = bi[c];
+  f32x4_t acc_a[TT], acc_i[TT];
 #pragma unroll
-  for (int tt = 0; tt < TPT; ++tt) {
-    const int t = t0 + tg * TPT + tt;
-    if (t >= T) continue;
-    const float r = sigmoid_f(acc_a[tt] + b_a);
-    const float g = sigmoid_f(acc_i[tt] + b_i);
-    const float log_a = -c_decay * r * sp;
-    const int64_t at = static_cast<int64_t>(t) * W + c;
-    a_out[at] = expf(log_a);
-    drive[at] = sqrtf(-expm1f(2.f * log_a)) * g * u[at];
+  for (int t = 0; t < TT; ++t) acc_a[t] = acc_i[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t av[AHEAD][2], iv[AHEAD][2], uv[AHEAD][TT][2];
+  auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
+    const int k = k0 + 8 * lk;
+    gate_load8<VEC>(av[slot], wa_row, k, bw);
+    gate_load8<VEC>(iv[slot], wi_row, k, bw);
+#pragma unroll
+    for (int t = 0; t < TT; ++t) gate_load8<VEC>(uv[slot][t], u_row[t], k, bw);
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) fetch(s, GK * s);
+  for (int k0 = 0; k0 < bw; k0 += GK * AHEAD) {
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      f32x4_t a_now[2], i_now[2], u_now[TT][2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        a_now[h] = av[s][h];
+        i_now[h] = iv[s][h];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) u_now[t][h] = uv[s][t][h];
+      }
+      fetch(s, k0 + GK * (s + AHEAD));
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          acc_a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_a[t], 0, 0, 0);
+          acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
+        }
+    }
+  }
+  // a lane holds token li, outputs 4 lk .. of its tiles
+  const int out = o0 + 4 * lk;
+  const int left = bw - out;
+  if (left <= 0) return;
+  const int c = blk * bw + out;
+  float sp[4], b_a[4], b_i[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int ce = e < left ? c + e : c;
+    sp[e] = softplus_f(lam[ce]);
+    b_a[e] = ba[ce];
+    b_i[e] = bi[ce];
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    const int tok = t0 + 16 * t + li;
+    if (tok >= T) continue;
+    const int64_t at = static_cast<int64_t>(tok) * W + c;
+    f32x4_t a4, d4, u4;
+    if (VEC) {
+      u4 = *reinterpret_cast<const f32x4_t*>(u + at);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) u4[e] = u[e < left ? at + e : at];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float r = sigmoid_f(acc_a[t][e] + b_a[e]);
+      const float g = sigmoid_f(acc_i[t][e] + b_i[e]);
+      const float log_a = -c_decay * r * sp[e];
+      a4[e] = expf(log_a);
+      d4[e] = sqrtf(-expm1f(2.f * log_a)) * g * u4[e];
+    }
+    if (VEC) {
+      *reinterpret_cast<f32x4_t*>(a_out + at) = a4;
+      *reinterpret_cast<f32x4_t*>(drive + at) = d4;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < left) a_out[at + e] = a4[e], drive[at + e] = d4[e];
+    }
   }
 }
 
@@ -666,17 +700,24 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
   if (T < 0 || W <= 0 || nb <= 0 || W % nb) return kvc_fail("kvc_rglru_gates: bad sizes");
   if (T == 0) return 0;
   const int bw = W / nb;
-  const bool few = T <= 16 * GT;  // few tokens: smaller tiles of outputs, four times the blocks
-  const int go = few ? 16 : 64;
-  const int out_tiles = (bw + go - 1) / go;
-  const dim3 grid((T + GT - 1) / GT, nb * out_tiles);  // tokens on x, which has no 16-bit limit
-  if (grid.y > 65535u) return kvc_fail("kvc_rglru_gates: too many channel tiles");
-  if (few)
-    hipLaunchKernelGGL((rglru_gates_kernel<16, 1>), grid, dim3(256), 0, S(stream), a_out, drive, u, wa,
-                       wi, ba, bi, lam, c_decay, T, W, bw, out_tiles);
+  const int out_tiles = (bw + 15) / 16;
+  if (static_cast<int64_t>(nb) * out_tiles > 65535) return kvc_fail("kvc_rglru_gates: too many channel tiles");
+  const bool vec = bw % 8 == 0 && ((reinterpret_cast<uintptr_t>(u) | reinterpret_cast<uintptr_t>(wa) |
+                                    reinterpret_cast<uintptr_t>(wi) | reinterpret_cast<uintptr_t>(a_out) |
+                                    reinterpret_cast<uintptr_t>(drive)) & 15) == 0;
+#define KVC_GATES(TT, AHEAD, VEC, WAVES)                                                                   \
+  hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC>),                                                 \
+                     dim3((T + 16 * TT * WAVES - 1) / (16 * TT * WAVES), nb * out_tiles), dim3(64 * WAVES), \
+                     0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles)
+  // few tokens: a wave a block, so that every compute unit has some, and more of a row on its way (8 tokens
+  // 9.8 against 11.2 us, 40 tokens 10.3 against 12.8; 100 tokens 16.9 against 14.8)
+  if (!vec)
+    KVC_GATES(2, 1, 0, 4);
+  else if (T <= 64)
+    KVC_GATES(1, 4, 1, 1);
   else
-    hipLaunchKernelGGL((rglru_gates_kernel<64, 4>), grid, dim3(256), 0, S(stream), a_out, drive, u, wa,
-                       wi, ba, bi, lam, c_decay, T, W, bw, out_tiles);
+    KVC_GATES(2, 2, 1, 4);
+#undef KVC_GATES
   return kvc_check_launch("kvc_rglru_gates");
 }
 

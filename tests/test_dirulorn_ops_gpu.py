@@ -218,6 +218,33 @@ def test_gated_linear_recurrence_whole_and_in_steps(ops, W, nb):
         close(state[2], last, 2e-5, 2e-5)
 
 
+@pytest.mark.parametrize("W,nb", [(512, 2), (96, 3), (128, 8), (66, 3), (20, 1)])
+def test_gates_of_a_token_do_not_depend_on_the_step(ops, W, nb):
+    """Tiles of 16 and of 32 tokens and their edges, channel blocks that fill tiles of 16 and chunks of 32 and
+    that do not, rows that are and are not 16-byte aligned: 64-bit results, and one token's bits in any step."""
+    T, bw = 131, W // nb
+    u = rnd(T, W, seed=1)
+    wa, wi = (rnd(nb, bw, bw, seed=s, std=bw ** -0.5) for s in (2, 3))
+    ba, bi, lam = rnd(nb, bw, seed=4), rnd(nb, bw, seed=5), rnd(W, seed=6)
+    ud, d = u.double().view(T, nb, bw), [t.to(DEV) for t in (wa, wi, ba, bi, lam)]
+    r, g = (torch.sigmoid(torch.einsum("tbi,boi->tbo", ud, w.double()) + b.double()).reshape(T, W)
+            for w, b in ((wa, ba), (wi, bi)))
+    log_a = -8.0 * r * torch.nn.functional.softplus(lam.double())
+
+    def run(first, n):
+        # the last row's end is the buffer's end: a read beyond it would leave the allocation
+        a, drive = torch.empty(n, W, device=DEV), torch.empty(n, W, device=DEV)
+        ops.rglru_gates(a, drive, u[first: first + n].to(DEV), *d, 8.0)
+        return a.cpu(), drive.cpu()
+
+    whole = run(0, T)
+    close(whole[0], log_a.exp(), 1e-5, 1e-5)
+    close(whole[1], torch.sqrt(-torch.expm1(2 * log_a)) * g * u.double(), 1e-5, 1e-5)
+    for first, n in ((0, 1), (5, 16), (3, 17), (2, 64), (60, 65), (1, 130)):
+        for got, want in zip(run(first, n), whole):
+            assert torch.equal(got, want[first: first + n])
+
+
 def test_long_portions_are_scanned_in_segments_side_by_side(ops):
     """With a workspace, requests longer than a segment are cut into segments that are scanned
     side by side and joined in order: the same results, whatever the portions, beside short
