@@ -42,7 +42,7 @@ constexpr int kRun = 16;        // tokens whose decays are multiplied one by one
 constexpr int kRuns = kChunk / kRun;
 constexpr int kPad = 4;         // floats between rows in LDS
 constexpr int kMostKeys = 128;  // rows of a state
-constexpr int kScalar = 1, kSpace = 2;
+constexpr int kScalar = 1, kSpace = 2, kChannel = 3;
 
 __device__ __forceinline__ float softplus_of(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
@@ -54,9 +54,9 @@ struct GatedArgs {
   int64_t k_stride;
   const float* v;     // rows of nh heads of dv - ones values
   int64_t v_stride;
-  const float* keep;  // kScalar: g [T, nh]
+  const float* keep;  // kScalar: g [T, nh]; kChannel: [T, nh * d]
   int64_t keep_stride;
-  const float* take;  // kScalar: b [T, nh]
+  const float* take;  // kScalar: b [T, nh], none: ones
   int64_t take_stride;
   const void* dt;     // kSpace: [T, nh] float32 or bfloat16
   int64_t dt_stride;
@@ -65,7 +65,10 @@ struct GatedArgs {
   const float* a_log;
   const float* skip;
   float* work;        // [chunks][nh][dpad / 4][dv][4], then the chunks' whole decays [chunks][nh]
-  float* decays;
+  float* decays;      // kChannel: [chunks][nh][dpad]
+  float* solved_k;    // the delta rule's: [T][nh * d], [T][nh * dv], [T][nh]
+  float* solved_v;
+  float* ends;
   float* scores;      // [chunks][nqk][64 queries][64 keys]: k . q of the heads that share both (else unused)
   float* state;       // [slots][nh][dpad / 4][dv][4]; kSpace: [slots][nh][d][dv]
   const int32_t* positions;
@@ -120,7 +123,7 @@ __device__ __forceinline__ void gates_of(const GatedArgs& a, const ChunkPlace& a
     g = expf(-expf(a.a_log[h]) * b);
   } else {
     g = a.keep[t * a.keep_stride + h];
-    b = a.take[t * a.take_stride + h];
+    b = a.take != nullptr ? a.take[t * a.take_stride + h] : 1.f;
   }
 }
 
@@ -278,16 +281,22 @@ __global__ __launch_bounds__(256) void gated_walk_kernel(const GatedArgs a) {
   }
   const int64_t step = static_cast<int64_t>(a.nh) * a.dpad * a.dv;
   float* w = a.work + (static_cast<int64_t>(first) * a.nh + h) * a.dpad * a.dv + static_cast<int64_t>(idx) * 4;
-  const float* whole = a.decays + static_cast<int64_t>(first) * a.nh + h;
+  constexpr bool kFours = GATES == kChannel;  // a factor for each of the four rows
+  const float* whole = kFours ? a.decays + (static_cast<int64_t>(first) * a.nh + h) * a.dpad + n
+                              : a.decays + static_cast<int64_t>(first) * a.nh + h;
   constexpr int kAhead = 8;
   for (int c0 = 0; c0 < chunks; c0 += kAhead) {
-    f32x4_t own[kAhead];
-    float g[kAhead];
+    f32x4_t own[kAhead], g[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int c = c0 + i < chunks ? c0 + i : chunks - 1;
       own[i] = *reinterpret_cast<const f32x4_t*>(w + c * step);
-      g[i] = whole[static_cast<int64_t>(c) * a.nh];
+      if (kFours) {
+        g[i] = *reinterpret_cast<const f32x4_t*>(whole + static_cast<int64_t>(c) * a.nh * a.dpad);
+      } else {
+        const float one = whole[static_cast<int64_t>(c) * a.nh];
+        g[i] = f32x4_t{one, one, one, one};
+      }
     }
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
@@ -328,24 +337,22 @@ __device__ __forceinline__ void fetch_query(f32x4_t* qv, const GatedArgs& a, con
     for (int e = 0; e < 4; ++e) qv[s][e] = live ? qv[s][e] * a.q_scale : 0.f;
   }
 }
-// k . q of sixteen keys (k_s: the first one's row) and the wave's sixteen queries; two running sums, so that an
-// instruction does not wait for the one before it.  Lane holds query li, keys 4 lk + i.
+// k . q of sixteen keys (k_s: the first one's row) and the wave's sixteen queries; eight running sums: an instruction
+// does not wait for the one before it, and no sum is long.  Lane holds query li, keys 4 lk + i.
 template <int NS>
 __device__ __forceinline__ f32x4_t score_tile(const float* k_s, const f32x4_t* qv, int d, int li, int lk) {
   constexpr int krow = 16 * NS + kPad;
-  f32x4_t even = {0.f, 0.f, 0.f, 0.f}, odd = even;
+  f32x4_t sum[4][2] = {};
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     if (16 * s < d) {  // scalar
       const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(k_s + li * krow + 16 * s + 4 * lk);
 #pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        even = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], qv[s][i], even, 0, 0, 0);
-        odd = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i + 1], qv[s][i + 1], odd, 0, 0, 0);
-      }
+      for (int i = 0; i < 4; ++i)
+        sum[s & 3][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], qv[s][i], sum[s & 3][i & 1], 0, 0, 0);
     }
   }
-  return even + odd;
+  return ((sum[0][0] + sum[0][1]) + (sum[1][0] + sum[1][1])) + ((sum[2][0] + sum[2][1]) + (sum[3][0] + sum[3][1]));
 }
 
 // ---- the scores of a chunk for heads that share queries and keys, once for all of them
@@ -370,6 +377,21 @@ __global__ __launch_bounds__(256) void gated_scores_kernel(const GatedArgs a) {
   float* dst = a.scores + ((static_cast<int64_t>(blockIdx.x) * a.nqk + hk) * kChunk + 16 * wave + li) * kChunk + 4 * lk;
   for (int kt = 0; kt <= wave; ++kt)  // scalar
     *reinterpret_cast<f32x4_t*>(dst + 16 * kt) = score_tile<NS>(lds + 16 * kt * krow, qv, a.d, li, lk);
+}
+
+// For token `tid` of a chunk: the factors between it and each later token of its run (`inside`, a row a later token),
+// those from the run's start on (`from_start`) and those behind it (`to_end`).
+__device__ __forceinline__ void run_products(const float* g_s, float* inside, float* from_start, float* to_end, int tid) {
+  const int run = tid / kRun * kRun, j = tid - run;
+  const double first = g_s[run];
+  double p = 1.0;
+#pragma unroll
+  for (int i = 0; i < kRun; ++i) {
+    if (i > j) p *= static_cast<double>(g_s[run + i]);
+    inside[(run + i) * (kRun + 1) + j] = i >= j ? static_cast<float>(p) : 0.f;
+    if (j == 0) from_start[run + i] = static_cast<float>(first * p);
+  }
+  to_end[tid] = static_cast<float>(p);
 }
 
 // ---- every chunk's results.  Wave w takes the queries 16 w .. 16 w + 15 (an operand's columns).  SHARED: the
@@ -418,18 +440,7 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
     bad = values.stash(v_s, at, a.ones ? dvin - c0 : -1);
   }
   bad = __syncthreads_or(bad);  // the same for the whole block
-  if (tid < kChunk) {
-    const int run = tid / kRun * kRun, j = tid - run;
-    const double first = g_s[run];
-    double p = 1.0;
-#pragma unroll
-    for (int i = 0; i < kRun; ++i) {
-      if (i > j) p *= static_cast<double>(g_s[run + i]);
-      inside[(run + i) * (kRun + 1) + j] = i >= j ? static_cast<float>(p) : 0.f;
-      if (j == 0) from_start[run + i] = static_cast<float>(first * p);
-    }
-    to_end[tid] = static_cast<float>(p);
-  }
+  if (tid < kChunk) run_products(g_s, inside, from_start, to_end, tid);
   __syncthreads();
   if (16 * wave >= at.n) return;  // scalar; no barrier follows
 
@@ -511,6 +522,318 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
   }
 }
 
+// ================================================= a factor per key channel: S <- diag(a_t) S + k_t v_t^T
+// The same three kernels.  A wave takes a run of 16 tokens into registers as an operand lies (lane: token li, channels
+// 16 s + 4 lk + e), so that products of factors along the run are scans over the 16 lanes of a row.  Scores of a run
+// with an earlier one: (q . factors from the run's start) (k . factors to its run's end) with the whole runs between
+// multiplied into the query on the way; inside a run, pair by pair on the vector unit, the key's row multiplied by one
+// more factor for each later query.  Products of factors and the pairs' sums are made in 64 bits and rounded once, and
+// no product's sum has more than eight terms in a row: in 32 bits and in long sums the results' error was 1.7 times the
+// scan's, so they are the same (0.95e-7 and 0.94e-7 at 683 tokens of 64 x 128 with factors sigmoid(z)^(1/8)).
+//
+// 16 heads of 64 x 128, three requests of 683 tokens: 152 -> 82 us (sums 22, walk 9, results 50), 2,048 tokens of one
+// 357 -> 68, 512 tokens 88 -> 39; bound by what a block does one after the other (a single chunk's results take 20 us,
+// half of it the pairs) on two blocks a compute unit.
+
+template <int NS, int VEC>
+__device__ __forceinline__ void fetch_lane(f32x4_t* x, const float* row, bool live, int lk, int size, float none) {
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    x[s] = f32x4_t{none, none, none, none};
+    const int n = 16 * s + 4 * lk;
+    if (!live) continue;
+    if (VEC) {
+      if (n < size) x[s] = *reinterpret_cast<const f32x4_t*>(row + n);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < size) x[s][e] = row[n + e];
+    }
+  }
+}
+// a value from another lane of the row of 16, one where there is none
+template <int CTRL>
+__device__ __forceinline__ double row_or_one(double v) {
+  const int64_t bits = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(bits), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0x3ff00000, static_cast<int>(bits >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double(static_cast<int64_t>(hi) << 32 | static_cast<uint32_t>(lo));
+}
+__device__ __forceinline__ double product_up_to(double v) {  // of this lane's value and those before it in its row
+  v *= row_or_one<0x111>(v);  // row_shr 1, 2, 4, 8
+  v *= row_or_one<0x112>(v);
+  v *= row_or_one<0x114>(v);
+  v *= row_or_one<0x118>(v);
+  return v;
+}
+__device__ __forceinline__ double product_behind(double v) {  // of the values behind this lane's in its row
+  v = row_or_one<0x101>(v);  // row_shl 1, then 1, 2, 4, 8
+  v *= row_or_one<0x101>(v);
+  v *= row_or_one<0x102>(v);
+  v *= row_or_one<0x104>(v);
+  v *= row_or_one<0x108>(v);
+  return v;
+}
+
+// Sixteen terms of a product's sums, four of each lane's, in two sums of eight (all of a result's terms in a row would
+// round too often).
+template <typename TA, typename TB>
+__device__ __forceinline__ f32x4_t sixteen_terms(const TA& x, const TB& y) {
+  f32x4_t t[2] = {};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], t[i & 1], 0, 0, 0);
+  return t[0] + t[1];
+}
+
+template <int NS, int NC, int VEC>
+__global__ __launch_bounds__(256) void channel_sums_kernel(const GatedArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  constexpr int kCols = 16 * NC, kVRow = kCols + kPad, kKeys = 16 * NS, krow = kKeys + kPad, NM = NS / 4;
+  const ChunkPlace at = find_chunk(a, blockIdx.x);
+  if (at.n == 0 || a.token_req[at.t0] < 0) return;
+  const int h = blockIdx.y, c0 = blockIdx.z * kCols, hk = h / (a.nh / a.nqk);
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cols = a.dv - c0 < kCols ? a.dv - c0 : kCols;
+  float* k_s = lds;                      // [64][krow], times the factors behind each token in the chunk
+  float* v_s = k_s + kChunk * krow;      // [64][kVRow]
+  double* whole = reinterpret_cast<double*>(v_s + kChunk * kVRow);  // [4][kKeys] a run's factors
+  {
+    const bool live = 16 * wave + li < at.n;
+    const int64_t t = at.t0 + (live ? 16 * wave + li : 0);
+    f32x4_t kv[NS], av[NS];
+    fetch_lane<NS, VEC>(kv, a.k + t * a.k_stride + static_cast<int64_t>(hk) * a.d, live, lk, a.d, 0.f);
+    fetch_lane<NS, VEC>(av, a.keep + t * a.keep_stride + static_cast<int64_t>(h) * a.d, live, lk, a.d, 1.f);
+    Staged<VEC, kCols> values;
+    values.fetch(a.v + static_cast<int64_t>(h) * a.dv + c0, a.v_stride, at, cols);
+    double behind[NS][4];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        behind[s][e] = product_behind(av[s][e]);
+        if (li == 0) whole[wave * kKeys + 16 * s + 4 * lk + e] = av[s][e] * behind[s][e];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        for (int r = wave + 1; r < kRuns; ++r) behind[s][e] *= whole[r * kKeys + 16 * s + 4 * lk + e];  // scalar
+        kv[s][e] = static_cast<float>(kv[s][e] * behind[s][e]);
+      }
+      *reinterpret_cast<f32x4_t*>(k_s + (16 * wave + li) * krow + 16 * s + 4 * lk) = kv[s];
+    }
+    values.stash(v_s, at, -1);
+  }
+  __syncthreads();
+  f32x4_t acc[NM][NC];
+#pragma unroll
+  for (int m = 0; m < NM; ++m)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[m][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; 16 * s < at.n; ++s) {  // scalar
+    float ka[4][NM];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = 0; m < NM; ++m) ka[i][m] = k_s[(16 * s + 4 * lk + i) * krow + 16 * (wave + 4 * m) + li];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float vb[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vb[i] = v_s[(16 * s + 4 * lk + i) * kVRow + 16 * c + li];
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const float mine[4] = {ka[0][m], ka[1][m], ka[2][m], ka[3][m]};
+        acc[m][c] += sixteen_terms(mine, vb);
+      }
+    }
+  }
+  const int64_t place = static_cast<int64_t>(blockIdx.x) * a.nh + h;
+  float* dst = a.work + place * a.dpad * a.dv;
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const int tile = 16 * (wave + 4 * m);
+    if (blockIdx.z == 0 && lk == 0 && tile + li < a.dpad) {
+      const double* w = whole + tile + li;
+      a.decays[place * a.dpad + tile + li] = static_cast<float>(w[0] * w[kKeys] * (w[2 * kKeys] * w[3 * kKeys]));
+    }
+    if (tile + 4 * lk >= a.dpad) continue;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int col = c0 + 16 * c + li;
+      if (col < a.dv) *reinterpret_cast<f32x4_t*>(dst + (static_cast<int64_t>((tile >> 2) + lk) * a.dv + col) * 4) = acc[m][c];
+    }
+  }
+}
+
+// The pairs of a run whose query lies BY tokens behind the key, key li in lane li, over 64 channels: its row p takes that
+// query's factors, and its products with the query are added up, in 64 bits.  (Lanes whose query would lie outside the
+// run end up with zeros.)
+template <int BY>
+__device__ __forceinline__ void pair_step(float* sums, double (&p)[4][4], const f32x4_t* av, const f32x4_t* qv) {
+  if constexpr (BY < kRun) {
+    double sum[2] = {0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float query = qv[s][e];
+        if constexpr (BY > 0) {  // row_shl: from the lane BY further on
+          p[s][e] *= __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(av[s][e]), 0x100 + BY, 0xF, 0xF, true));
+          query = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(query), 0x100 + BY, 0xF, 0xF, true));
+        }
+        sum[e & 1] = fma(p[s][e], static_cast<double>(query), sum[e & 1]);
+      }
+    float v = static_cast<float>(sum[0] + sum[1]);
+    v += __shfl_xor(v, 16, kWave);
+    v += __shfl_xor(v, 32, kWave);
+    sums[BY] += v;
+    pair_step<BY + 1>(sums, p, av, qv);
+  }
+}
+
+template <int NS, int NC, int VEC>
+__global__ __launch_bounds__(256) void channel_results_kernel(const GatedArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  constexpr int kCols = 16 * NC, kVRow = kCols + kPad, kKeys = 16 * NS, krow = kKeys + kPad, kPairRow = kRun + 4;
+  const ChunkPlace at = find_chunk(a, blockIdx.x);
+  if (at.n == 0) return;
+  const int h = blockIdx.y, c0 = blockIdx.z * kCols, hk = h / (a.nh / a.nqk);
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int cols = a.dv - c0 < kCols ? a.dv - c0 : kCols;
+  const int width = a.nh * a.dv;
+  if (a.token_req[at.t0] < 0) {  // padding rows: zeros
+    for (int idx = tid; idx < at.n * cols; idx += blockDim.x) {
+      const int i = idx / cols, c = idx - i * cols;
+      a.out[static_cast<int64_t>(at.t0 + i) * width + h * a.dv + c0 + c] = 0.f;
+    }
+    return;
+  }
+  float* k_s = lds;                        // [64][krow], times the factors behind each token in its run
+  float* v_s = k_s + kChunk * krow;        // [64][kVRow]
+  double* whole = reinterpret_cast<double*>(v_s + kChunk * kVRow);  // [4][kKeys] a run's factors
+  float* pairs = reinterpret_cast<float*>(whole + 4 * kKeys);  // [64][kPairRow] scores of a query with its run's keys
+  const int query = 16 * wave + li;
+  const bool live = query < at.n;
+  f32x4_t qv[NS];
+  double far_q[NS][4];  // the query times the factors from the run at hand to it
+  bool bad;
+  {
+    const int64_t t = at.t0 + (live ? query : 0);
+    f32x4_t kv[NS], av[NS];
+    fetch_lane<NS, VEC>(qv, a.q + t * a.q_stride + static_cast<int64_t>(hk) * a.d, live, lk, a.d, 0.f);
+    fetch_lane<NS, VEC>(kv, a.k + t * a.k_stride + static_cast<int64_t>(hk) * a.d, live, lk, a.d, 0.f);
+    fetch_lane<NS, VEC>(av, a.keep + t * a.keep_stride + static_cast<int64_t>(h) * a.d, live, lk, a.d, 1.f);
+    Staged<VEC, kCols> values;
+    values.fetch(a.v + static_cast<int64_t>(h) * a.dv + c0, a.v_stride, at, cols);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qv[s] = qv[s] * a.q_scale;
+    float sums[kRun] = {};
+#pragma unroll
+    for (int half = 0; half < NS / 4; ++half) {
+      double p[4][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[s][e] = kv[4 * half + s][e];
+      pair_step<0>(sums, p, av + 4 * half, qv + 4 * half);
+    }
+    // lane: key li of every query; of four neighbouring distances it stores number lk, and that distance's zeros for
+    // the queries before the key
+#pragma unroll
+    for (int i = 0; i < kRun; i += 4) {
+      const float mine = lk & 2 ? (lk & 1 ? sums[i + 3] : sums[i + 2]) : (lk & 1 ? sums[i + 1] : sums[i]);
+      const int by = i + lk;
+      if (li + by < kRun) pairs[(query + by) * kPairRow + li] = mine;
+      if (by > 0 && li - by >= 0) pairs[(query - by) * kPairRow + li] = 0.f;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double upto = product_up_to(av[s][e]);
+        far_q[s][e] = qv[s][e] * upto;
+        if (li == kRun - 1) whole[wave * kKeys + 16 * s + 4 * lk + e] = upto;
+        kv[s][e] = static_cast<float>(kv[s][e] * product_behind(av[s][e]));
+        qv[s][e] = static_cast<float>(far_q[s][e]);
+      }
+      *reinterpret_cast<f32x4_t*>(k_s + query * krow + 16 * s + 4 * lk) = kv[s];
+    }
+    bad = values.stash(v_s, at, -1);
+  }
+  bad = __syncthreads_or(bad);  // the same for the whole block
+  if (16 * wave >= at.n) return;  // scalar; no barrier follows
+  f32x4_t own[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) own[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int kt = wave; kt >= 0; --kt) {  // scalar
+    // lane holds query li, keys 4 lk + i of the run: the operand order of the next product
+    f32x4_t score;
+    if (kt == wave) {  // scalar
+      score = *reinterpret_cast<const f32x4_t*>(pairs + query * kPairRow + 4 * lk);
+      if (bad) {  // key by key: see gated_results_kernel
+        for (int j = 0; j < kRun; ++j) {
+          const float mine = pairs[query * kPairRow + j];
+          if (j <= li)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) own[c] += mine * *reinterpret_cast<const f32x4_t*>(v_s + (16 * kt + j) * kVRow + 16 * c + 4 * lk);
+        }
+        continue;
+      }
+    } else {
+      score = score_tile<NS>(k_s + 16 * kt * krow, qv, a.d, li, lk);
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          far_q[s][e] *= whole[kt * kKeys + 16 * s + 4 * lk + e];
+          qv[s][e] = static_cast<float>(far_q[s][e]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      float vb[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vb[i] = v_s[(16 * kt + 4 * lk + i) * kVRow + 16 * c + li];
+      own[c] += sixteen_terms(vb, score);
+    }
+  }
+  // the state before the chunk; the queries carry every factor since by now
+  const float* st = a.work + (static_cast<int64_t>(blockIdx.x) * a.nh + h) * a.dpad * a.dv;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (16 * s < a.d) {  // scalar
+      const int n = 16 * s + 4 * lk;
+      const int row = n < a.dpad ? n >> 2 : 0;  // rows beyond read the first: their q is zero
+      f32x4_t sv[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int col = c0 + 16 * c + li;
+        sv[c] = *reinterpret_cast<const f32x4_t*>(st + (static_cast<int64_t>(row) * a.dv + (col < a.dv ? col : c0)) * 4);
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) own[c] += sixteen_terms(sv[c], qv[s]);
+    }
+  }
+  if (!live) return;
+  float* o = a.out + static_cast<int64_t>(at.t0 + query) * width + static_cast<int64_t>(h) * a.dv + c0;
+  const bool vec_out = (a.dv & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int col = 16 * c + 4 * lk;
+    if (vec_out) {
+      if (col < cols) *reinterpret_cast<f32x4_t*>(o + col) = own[c];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < cols) o[col + e] = own[c][e];
+    }
+  }
+}
+
 size_t gated_lds(int keys, int nc) {
   return sizeof(float) * (kChunk * (keys + kPad) + kChunk * (16 * nc + kPad) + 4 * kChunk + kChunk * (kRun + 1));
 }
@@ -545,6 +868,19 @@ int run_chunks(const GatedArgs& a, int chunks, hipStream_t stream) {
   if (a.d <= 64) return run_results<GATES, 4, NC, VEC>(a, grid, stream);
   return run_results<GATES, 8, NC, VEC>(a, grid, stream);
 }
+
+template <int NS, int NC, int VEC>
+int run_channel(const GatedArgs& a, int chunks, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(chunks), a.nh, (a.dv + 16 * NC - 1) / (16 * NC));
+  const size_t lds = sizeof(float) * (kChunk * (16 * NS + kPad) + kChunk * (16 * NC + kPad) + 2 * 4 * 16 * NS);
+  int code = launch(channel_sums_kernel<NS, NC, VEC>, a, grid, lds, stream);
+  if (code) return code;
+  const int fours = a.dpad / 4 * a.dv;
+  hipLaunchKernelGGL(gated_walk_kernel<kChannel>, dim3(a.R, a.nh, (fours + 255) / 256), dim3(256), 0, stream, a);
+  return launch(channel_results_kernel<NS, NC, VEC>, a, grid, lds + sizeof(float) * kChunk * (kRun + 4), stream);
+}
+
+int64_t channel_floats(int nh, int d, int dv) { return nh * (static_cast<int64_t>((d + 3) & ~3) * (dv + 1)); }
 
 int64_t chunk_floats(int nh, int nqk, int d, int dv) {
   const int64_t all = nh * (static_cast<int64_t>((d + 3) & ~3) * dv + 1) + (nqk < nh ? static_cast<int64_t>(nqk) * kChunk * kChunk : 0);
@@ -599,6 +935,45 @@ extern "C" int kvc_scalar_gate_chunks(float* out, const float* q, int64_t q_stri
   a.positions = positions; a.token_req = token_req; a.q_start = q_start; a.slots = slots;
   a.from = from; a.R = R; a.nh = nh; a.nqk = nqk; a.d = d; a.dv = dv; a.dpad = (d + 3) & ~3; a.ones = ones; a.q_scale = q_scale;
   return run<kScalar>(a, work_floats, chunks, "kvc_scalar_gate_chunks", S(stream));
+}
+
+extern "C" int64_t kvc_channel_chunk_floats(int nh, int d, int dv) { return channel_floats(nh, d, dv); }
+
+extern "C" int kvc_channel_gate_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride,
+                                       const float* v, int64_t v_stride, const float* decay, int64_t decay_stride,
+                                       float* state, float* work, int64_t work_floats, const int32_t* positions,
+                                       const int32_t* token_req, const int32_t* q_start, const int32_t* slots, int chunks,
+                                       int from, int R, int nh, int nqk, int d, int dv, float q_scale, kvc_stream stream) {
+  if (chunks < 0 || R < 0 || nh <= 0 || nqk <= 0 || nh % nqk || d <= 0 || dv <= 0 || nh > 65535)
+    return kvc_fail("kvc_channel_gate_chunks: bad sizes");
+  if (d > kMostKeys) return kvc_fail("kvc_channel_gate_chunks: at most 128 key channels a head");
+  if (q_stride < static_cast<int64_t>(nqk) * d || k_stride < static_cast<int64_t>(nqk) * d ||
+      v_stride < static_cast<int64_t>(nh) * dv || decay_stride < static_cast<int64_t>(nh) * d)
+    return kvc_fail("kvc_channel_gate_chunks: rows too short for the heads");
+  if (chunks == 0 || R == 0) return 0;
+  if (work == nullptr || work_floats < chunks * channel_floats(nh, d, dv))
+    return kvc_fail("gated chunks: the workspace is too small");
+  if (((reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(work)) & 15) != 0)
+    return kvc_fail("gated chunks: state and workspace must be 16-byte aligned");
+  GatedArgs a{};
+  a.out = out; a.q = q; a.q_stride = q_stride; a.k = k; a.k_stride = k_stride; a.v = v; a.v_stride = v_stride;
+  a.keep = decay; a.keep_stride = decay_stride; a.work = work; a.state = state;
+  a.positions = positions; a.token_req = token_req; a.q_start = q_start; a.slots = slots;
+  a.from = from; a.R = R; a.nh = nh; a.nqk = nqk; a.d = d; a.dv = dv; a.dpad = (d + 3) & ~3; a.q_scale = q_scale;
+  a.decays = work + static_cast<int64_t>(chunks) * nh * a.dpad * dv;
+  const bool vec = d % 4 == 0 && dv % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
+                   decay_stride % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
+                     reinterpret_cast<uintptr_t>(decay)) & 15) == 0;
+  // all of a head's columns in one tile where it holds them: the pairs inside a run are then paid for once
+  int code;
+  if (d <= 64) {
+    if (dv <= 64) code = vec ? run_channel<4, 4, 1>(a, chunks, S(stream)) : run_channel<4, 4, 0>(a, chunks, S(stream));
+    else code = vec ? run_channel<4, 8, 1>(a, chunks, S(stream)) : run_channel<4, 8, 0>(a, chunks, S(stream));
+  } else {
+    code = vec ? run_channel<8, 8, 1>(a, chunks, S(stream)) : run_channel<8, 8, 0>(a, chunks, S(stream));
+  }
+  return code ? code : kvc_check_launch("kvc_channel_gate_chunks");
 }
 
 extern "C" int kvc_ssm_chunks(float* y, const float* xbc, int64_t xbc_stride, const void* dt_raw, int64_t dt_stride,

@@ -277,6 +277,14 @@ int kvc_scalar_gate_chunks(float* out, const float* q, int64_t q_stride, const f
                            const int32_t* positions, const int32_t* token_req, const int32_t* q_start,
                            const int32_t* slots, int chunks, int from, int R, int nh, int nqk, int d, int dv,
                            float q_scale, int ones_column, kvc_stream stream);
+// kvc_linear_state_scan with a factor per key channel the same way (decay [T, nh * d]); work:
+// kvc_channel_chunk_floats a chunk.
+int64_t kvc_channel_chunk_floats(int nh, int d, int dv);
+int kvc_channel_gate_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride,
+                            const float* v, int64_t v_stride, const float* decay, int64_t decay_stride,
+                            float* state, float* work, int64_t work_floats, const int32_t* positions,
+                            const int32_t* token_req, const int32_t* q_start, const int32_t* slots, int chunks,
+                            int from, int R, int nh, int nqk, int d, int dv, float q_scale, kvc_stream stream);
 int kvc_ssm_chunks(float* y, const float* xbc, int64_t xbc_stride, const void* dt_raw, int64_t dt_stride,
                    int dt_dtype, const float* dt_bias, const float* a_log, const float* d_skip, float* state,
                    float* work, int64_t work_floats, const int32_t* positions, const int32_t* token_req,

@@ -64,6 +64,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_linear_state_scan": [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, I, I, P],
         "kvc_fixed_decay_chunks": [P, P, L, P, L, P, L, P, P, P, L, P, P, P, P, I, I, I, I, I, I, F, I, P],
         "kvc_scalar_gate_chunks": [P, P, L, P, L, P, L, P, L, P, L, P, P, L, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
+        "kvc_channel_gate_chunks": [P, P, L, P, L, P, L, P, L, P, P, L, P, P, P, P, I, I, I, I, I, I, I, F, P],
         "kvc_ssm_chunks": [P, P, L, P, L, I, P, P, P, P, P, L, P, P, P, P, I, I, I, I, I, I, I, P],
         "kvc_sigmoid_power": [P, P, L, P, F, I, I, P],
         "kvc_decay_and_write_gates": [P, P, P, L, P, L, P, P, I, I, P],
@@ -134,6 +135,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvc_fixed_decay_chunk_tokens.argtypes = []
     lib.kvc_gated_chunk_floats.restype = c_int64
     lib.kvc_gated_chunk_floats.argtypes = [c_int] * 4
+    lib.kvc_channel_chunk_floats.restype = c_int64
+    lib.kvc_channel_chunk_floats.argtypes = [c_int] * 3
     lib.kvc_gated_chunk_tokens.restype = c_int
     lib.kvc_gated_chunk_tokens.argtypes = []
     lib.kvc_rglru_scan_segment.restype = c_int
@@ -1578,11 +1581,12 @@ def gated_chunk_count(lengths, start: int) -> int:
 
 
 def gated_chunk_work(buffers, name: str, chunks: int, start: int, heads: int, key_heads: int, rows: int,
-                     cols: int) -> torch.Tensor:
-    """The step buffer that ``ssm_chunks`` and ``scalar_gate_chunks`` work in: a row for each of ``chunks`` chunks (of
-    requests of at least ``start`` tokens), for states of ``rows x cols`` a head."""
+                     cols: int, per_channel: bool = False) -> torch.Tensor:
+    """The step buffer that ``ssm_chunks``, ``scalar_gate_chunks`` and (``per_channel``) ``channel_gate_chunks`` work in:
+    a row for each of ``chunks`` chunks (of requests of at least ``start`` tokens), for states of ``rows x cols`` a head."""
     lib = load()
-    each = int(lib.kvc_gated_chunk_floats(heads, key_heads, rows, cols))
+    each = int(lib.kvc_channel_chunk_floats(heads, rows, cols) if per_channel
+               else lib.kvc_gated_chunk_floats(heads, key_heads, rows, cols))
     capacity = buffers.token_capacity  # every request of at least `start` tokens may end in a ragged chunk
     most = capacity // int(lib.kvc_gated_chunk_tokens()) + capacity // max(start, 1) + 1
     return buffers.get(f"{name}:{each}", chunks, each, torch.float32, reserve=most)
@@ -1643,6 +1647,33 @@ def scalar_gate_chunks(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: t
         _dev(positions, "positions", i32), _dev(token_req, "token_req", i32), _dev(q_start, "q_start", i32),
         _dev(slots, "slots", i32), chunks, start, num_reqs, heads, qk_heads, dim, vdim, float(q_scale),
         int(bool(ones_column)), _stream()), "kvc_scalar_gate_chunks")
+
+
+def channel_gate_chunks(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor,
+                        state: torch.Tensor, work: torch.Tensor, *, positions: torch.Tensor, token_req: torch.Tensor,
+                        q_start: torch.Tensor, slots: torch.Tensor, num_reqs: int, heads: int, qk_heads: int, dim: int,
+                        vdim: int, chunks: int, start: int = 1, q_scale: float = 1.0) -> None:
+    """:func:`linear_state_scan` with a factor per key channel for the requests of at least ``start`` tokens, ``chunks``
+    chunks of tokens side by side (:func:`gated_chunk_count`); ``work``: :func:`gated_chunk_work` (``per_channel``)."""
+    T = out.shape[0]
+    if out.shape != (T, heads * vdim) or not out.is_contiguous() or out.dtype != torch.float32:
+        raise KernelError("channel_gate_chunks: out must be contiguous float32 [T, heads * vdim]")
+    if tuple(state.shape[1:]) != (heads, linear_state_rows(dim), vdim) or state.dtype != torch.float32 \
+            or not state.is_contiguous():
+        raise KernelError("channel_gate_chunks: state must be float32 [slots, heads, linear_state_rows(dim), vdim]")
+    if min(q.shape[0], k.shape[0], v.shape[0], decay.shape[0]) < T or positions.numel() < T or token_req.numel() < T \
+            or q_start.numel() < num_reqs + 1:
+        raise KernelError("channel_gate_chunks: rows or index arrays too short")
+    qp, qs = _f32_rows(q, "q", qk_heads * dim)
+    kp, ks = _f32_rows(k, "k", qk_heads * dim)
+    vp, vs = _f32_rows(v, "v", heads * vdim)
+    dp, ds = _f32_rows(decay, "decay", heads * dim)
+    f, i32 = torch.float32, torch.int32
+    _check(load().kvc_channel_gate_chunks(
+        out.data_ptr(), qp, qs, kp, ks, vp, vs, dp, ds, _dev(state, "state"), _dev(work, "work", f), work.numel(),
+        _dev(positions, "positions", i32), _dev(token_req, "token_req", i32), _dev(q_start, "q_start", i32),
+        _dev(slots, "slots", i32), chunks, start, num_reqs, heads, qk_heads, dim, vdim, float(q_scale), _stream()),
+        "kvc_channel_gate_chunks")
 
 
 def gated_group_rmsnorm(out: torch.Tensor, y: torch.Tensor, z: torch.Tensor, gain: torch.Tensor,

@@ -41,6 +41,9 @@ CHUNKED_FROM = 48
 # requests of 128 tokens 67 and 47, 2,048 tokens 405 and 57); a float32 model walks every token, so that its results
 # do not depend on how a request is cut into steps
 GATED_CHUNKED_FROM = 128
+# a factor a channel (16 heads of 64 x 128: 128 tokens 25 and 35 us, 192 tokens 35 and 36, 512 tokens 88 and 39, three
+# requests of 683 tokens 152 and 82, 2,048 tokens 357 and 68)
+CHANNEL_CHUNKED_FROM = 192
 
 
 def _src(name: str, rows: int) -> tuple[ParamSource, ...]:
@@ -134,9 +137,19 @@ class GatedLinearAttention(_MatrixStateMixer):
         decay = ctx.buf(f"gla_decay:{qk}", qk, torch.float32)
         ops.sigmoid_power(decay, z, p["a2.bias"], 1.0 / self.tau)
         o = ctx.buf(f"ms_o:{inner}", inner, torch.float32)
-        ops.linear_state_scan(o, proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], decay, None,
-                              state, heads=self.heads, qk_heads=self.heads, dim=self.dim, vdim=self.vdim,
-                              delta_rule=False, q_scale=self.q_scale, **self._batch(ctx))
+        rows = (proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner])
+        sizes = dict(heads=self.heads, qk_heads=self.heads, dim=self.dim, vdim=self.vdim, q_scale=self.q_scale,
+                     **self._batch(ctx))
+        chunks = 0
+        if ctx.dtype == torch.bfloat16 and self.dim <= 128:
+            chunks = ops.gated_chunk_count(ctx.host_query_lens, CHANNEL_CHUNKED_FROM)
+        if chunks:
+            work = ops.gated_chunk_work(ctx.buffers, "gla_chunks", chunks, CHANNEL_CHUNKED_FROM, self.heads, self.heads,
+                                        self.dim, self.vdim, per_channel=True)
+            ops.channel_gate_chunks(o, *rows, decay, state, work, chunks=chunks, start=CHANNEL_CHUNKED_FROM, **sizes)
+        if not chunks or min(ctx.host_query_lens) < CHANNEL_CHUNKED_FROM:
+            ops.linear_state_scan(o, *rows, decay, None, state, delta_rule=False,
+                                  below=CHANNEL_CHUNKED_FROM if chunks else 0, **sizes)
         return self._finish(o, proj[:, 2 * qk + inner:], ctx)
 
 

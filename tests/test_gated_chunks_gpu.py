@@ -204,3 +204,80 @@ def test_state_space_recurrence_in_chunks(heads, groups, N, P, dtype, start, fro
     (scan_y, scan_s), (chunk_y, chunk_s) = errors
     assert chunk_y < 1e-6 and chunk_s < 1e-6, errors
     assert chunk_y < 1.25 * scan_y + 2e-8 and chunk_s < 1.25 * scan_s + 2e-8, errors
+
+
+@pytest.mark.parametrize("start,from_", [(0, 1), (7, 1), (7, 64)])
+@pytest.mark.parametrize("heads,qk_heads,d,dv", [(2, 2, 64, 128), (3, 1, 24, 40), (2, 2, 100, 80), (1, 1, 7, 5),
+                                                  (2, 1, 128, 130), (2, 2, 30, 64)])
+def test_channel_factors_in_chunks(heads, qk_heads, d, dv, start, from_):
+    """Factors from zero to one, some channels that forget at once and some that keep for ever."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(d + dv)
+    reqs = requests(LENGTHS, start)
+    where, T = spans(reqs)
+    q, k = (torch.randn(T, qk_heads, d, generator=gen) for _ in range(2))
+    k = k * d ** -0.5
+    v = torch.randn(T, heads, dv, generator=gen)
+    a = torch.rand(T, heads, d, generator=gen) ** (10.0 ** (torch.rand(heads, d, generator=gen) * -3 + 1))
+    a[torch.rand(T, heads, d, generator=gen) < 0.02] = 0.0
+    a[:, 0, 0] = 1.0
+    rows = ops.linear_state_rows(d)
+    held = torch.randn(len(LENGTHS), heads, rows, dv, generator=gen)
+    state = gpu(torch.full_like(held, float("nan")) if start == 0 else held)
+    batch, _ = batch_tensors(reqs)
+    wide = torch.cat([q.flatten(1), k.flatten(1), v.flatten(1)], 1)
+    wide = gpu(torch.cat([wide, torch.zeros(T, -wide.shape[1] % 4)], 1))
+    c = qk_heads * d
+    views = (wide[:, :c], wide[:, c:2 * c], wide[:, 2 * c:2 * c + heads * dv])
+    sizes = dict(heads=heads, qk_heads=qk_heads, dim=d, vdim=dv, q_scale=0.5, **batch)
+    errors = []
+    for chunked in (False, True):
+        y, s = torch.full((T, heads * dv), float("nan"), device=DEV), state.clone()
+        if chunked:
+            chunks = ops.gated_chunk_count([1 if r is None else r[2] for r in reqs], from_)
+            work = torch.full((chunks, ops.load().kvc_channel_chunk_floats(heads, d, dv)), float("nan"), device=DEV)
+            ops.channel_gate_chunks(y, *views, gpu(a.flatten(1)), s, work, chunks=chunks, start=from_, **sizes)
+            if from_ > 1:
+                ops.linear_state_scan(y, *views, gpu(a.flatten(1)), None, s, below=from_, **sizes)
+        else:
+            ops.linear_state_scan(y, *views, gpu(a.flatten(1)), None, s, **sizes)
+        got, want, gs, ws = [], [], [], []
+        rep = heads // qk_heads
+        for slot, lo, hi in where:
+            S = held[slot].double().view(heads, rows // 4, dv, 4).permute(0, 1, 3, 2).reshape(heads, rows, dv)[:, :d]
+            S = S * (start > 0)
+            for t in range(lo, hi):
+                kt, qt = (x[t].double().repeat_interleave(rep, 0) for x in (k, q))
+                S = a[t].double()[:, :, None] * S + kt[:, :, None] * v[t].double()[:, None, :]
+                want.append(torch.einsum("hdv,hd->hv", S, qt * 0.5).flatten())
+            got.append(y[lo:hi])
+            gs.append(s[slot].view(heads, rows // 4, dv, 4).permute(0, 1, 3, 2).reshape(heads, rows, dv)[:, :d])
+            ws.append(S)
+        errors.append((rel(torch.cat(got), torch.stack(want)), rel(torch.stack(gs), torch.stack(ws))))
+        if None in reqs:
+            at = sum(r[2] for r in reqs[:4])
+            assert (y[at] == 0).all()
+    # the same number of products and sums is rounded either way: no worse than the scan but for chance (factors that
+    # forget at once leave the last few tokens' roundings, of which the scan has two a token and the chunks three)
+    assert errors[1][0] < 1.2 * errors[0][0] and errors[1][1] < 1.5 * errors[0][1], errors
+
+
+def test_channel_factors_in_chunks_keep_to_their_own_tokens():
+    """A value or key that is not finite reaches the tokens from its own on and no earlier one, and its own column or all."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(2)
+    T, d, dv = 100, 64, 128
+    q, k, v = (torch.randn(T, n, generator=gen) for n in (d, d, dv))
+    a = torch.rand(T, d, generator=gen)
+    v[37, 5], k[70, 3] = float("inf"), float("nan")
+    batch, _ = batch_tensors([(0, 0, T)])
+    y, s = torch.zeros(T, dv, device=DEV), torch.zeros(1, 1, d, dv, device=DEV)
+    work = torch.empty(2, ops.load().kvc_channel_chunk_floats(1, d, dv), device=DEV)
+    ops.channel_gate_chunks(y, gpu(q), gpu(k), gpu(v), gpu(a), s, work, chunks=2, heads=1, qk_heads=1, dim=d, vdim=dv,
+                            **batch)
+    fine = torch.isfinite(y.cpu())
+    assert fine[:37].all() and not fine[37:, 5].any() and not fine[70:].any()
+    others = torch.arange(dv) != 5
+    assert fine[37:70][:, others].all()
