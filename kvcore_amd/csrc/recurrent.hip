@@ -643,6 +643,69 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(
   }
 }
 
+template <typename T>
+__device__ __forceinline__ void take4(const T* p, float* v) {  // aligned to four values
+  if constexpr (sizeof(T) == 4) {
+    const float4 w = *reinterpret_cast<const float4*>(p);
+    v[0] = w.x, v[1] = w.y, v[2] = w.z, v[3] = w.w;
+  } else {
+    const uint2 w = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(w.x << 16), v[1] = __uint_as_float(w.x & 0xffff0000u);
+    v[2] = __uint_as_float(w.y << 16), v[3] = __uint_as_float(w.y & 0xffff0000u);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void put4(T* p, const float* v) {
+  alignas(16) T y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = from_float<T>(v[e]);
+  if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(p) = *reinterpret_cast<const float4*>(y);
+  else *reinterpret_cast<uint2*>(p) = *reinterpret_cast<const uint2*>(y);
+}
+
+// The same for parts of at most 1,024 channels in fours, aligned: a wave a (token, part), the gated values kept in
+// registers between the sum and the norm.  A block a part waits for its barriers and makes every gate twice: 2,048 tokens
+// of 8 parts of 512 34 -> 18 us.
+template <typename TZ, typename TO>
+__global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(
+    TO* __restrict__ out, const float* __restrict__ y, const TZ* __restrict__ z, int64_t z_stride,
+    const float* __restrict__ gain, float eps, int width, int groups, int64_t items) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
+  if (item >= items) return;
+  const int64_t t = item / groups;
+  const int n = width / groups, c0 = static_cast<int>(item - t * groups) * n;
+  const float* yr = y + t * width + c0;
+  const TZ* zr = z + t * z_stride + c0;
+  float v[4][4], ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = 4 * lane + 256 * k;
+    float zv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[k][e] = zv[e] = 0.f;
+    if (i < n) {
+      take4(yr + i, v[k]);
+      take4(zr + i, zv);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[k][e] = i < n ? v[k][e] * silu_f(zv[e]) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(v[k][e], v[k][e], ss);
+  }
+  const float inv = 1.f / sqrtf(wave_sum(ss) / static_cast<float>(n) + eps);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int i = 4 * lane + 256 * k;
+    if (i >= n) continue;
+    float g[4];
+    take4(gain + c0 + i, g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[k][e] = v[k][e] * inv * g[e];
+    put4(out + t * width + c0 + i, v[k]);
+  }
+}
+
 }  // namespace
 
 // dtype codes: 0 float32, 1 bfloat16.
@@ -828,6 +891,18 @@ extern "C" int kvc_gated_group_rmsnorm(void* out, int out_dtype, const float* y,
     return kvc_fail("kvc_gated_group_rmsnorm: bad sizes");
   if (T == 0) return 0;
   if (groups > 65535) return kvc_fail("kvc_gated_group_rmsnorm: too many parts");
+  const int n = width / groups;
+  const uintptr_t z_four = z_dtype == 0 ? 15 : 7, out_four = out_dtype == 0 ? 15 : 7;
+  if (n % 4 == 0 && n <= 1024 && z_stride % 4 == 0 &&
+      ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gain)) & 15) == 0 &&
+      (reinterpret_cast<uintptr_t>(z) & z_four) == 0 && (reinterpret_cast<uintptr_t>(out) & out_four) == 0) {
+    const int64_t items = static_cast<int64_t>(T) * groups;
+    KVC_DISPATCH_2(z_dtype, TZ, out_dtype, TO,
+                   hipLaunchKernelGGL((gated_group_rmsnorm_wave_kernel<TZ, TO>), dim3(static_cast<unsigned>((items + 3) / 4)),
+                                      dim3(256), 0, S(stream), static_cast<TO*>(out), y,
+                                      static_cast<const TZ*>(z), z_stride, gain, eps, width, groups, items));
+    return kvc_check_launch("kvc_gated_group_rmsnorm");
+  }
   KVC_DISPATCH_2(z_dtype, TZ, out_dtype, TO,
                  hipLaunchKernelGGL((gated_group_rmsnorm_kernel<TZ, TO>), dim3(T, groups), dim3(256),
                                     0, S(stream), static_cast<TO*>(out), y,

@@ -171,6 +171,20 @@ def test_convolution_reads_bfloat16_rows_and_writes_them(ops):
     assert torch.equal(state[0].cpu(), x[T - (K - 1):].float())
 
 
+@pytest.mark.parametrize("n,parts", [(4, 3), (252, 2), (512, 8), (1020, 1), (1024, 2), (1028, 1), (30, 2)])
+@pytest.mark.parametrize("shift", [0, 4, 1])
+def test_gated_norm_of_parts_that_a_wave_holds_and_does_not(ops, n, parts, shift):
+    T, width = 5, n * parts
+    y, g = rnd(T, width, seed=1), rnd(width, seed=2)
+    z = rnd(T, width + 8, seed=3, dtype=torch.bfloat16)
+    out = torch.empty(T, width, device=DEV)
+    ops.gated_group_rmsnorm(out, y.to(DEV), z.to(DEV)[:, shift: shift + width], g.to(DEV), 1e-5, parts)
+    v = y.double() * plain.silu(z[:, shift: shift + width].double())
+    v = v.view(T, parts, n)
+    want = (v / torch.sqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5)).reshape(T, width) * g.double()
+    close(out, want, 2e-6, 2e-6)  # a sum of n squares and a few products, each rounded to 24 bits
+
+
 # ------------------------------------------------------------ gated linear recurrence
 def plain_recurrence(u, y, wa, wi, ba, bi, lam, c):
     T, W = u.shape
