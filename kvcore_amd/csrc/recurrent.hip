@@ -186,13 +186,14 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
-    int bw, int out_tiles) {
+    int bw, int out_tiles, int token_tiles) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
-  const int t0 = (blockIdx.x * (blockDim.x >> 6) + wave) * 16 * TT;
+  const int channel_tile = blockIdx.x / token_tiles;
+  const int t0 = ((blockIdx.x - channel_tile * token_tiles) * (blockDim.x >> 6) + wave) * 16 * TT;
   if (t0 >= T) return;
-  const int blk = blockIdx.y / out_tiles;
-  const int o0 = (blockIdx.y - blk * out_tiles) * 16;
+  const int blk = channel_tile / out_tiles;
+  const int o0 = (channel_tile - blk * out_tiles) * 16;
   // outputs and tokens beyond the last read the last one and are not stored
   const int64_t row = (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
   const float *wa_row = wa + row, *wi_row = wi + row, *u_row[TT];
@@ -763,15 +764,20 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
   if (T < 0 || W <= 0 || nb <= 0 || W % nb) return kvc_fail("kvc_rglru_gates: bad sizes");
   if (T == 0) return 0;
   const int bw = W / nb;
-  const int out_tiles = (bw + 15) / 16;
-  if (static_cast<int64_t>(nb) * out_tiles > 65535) return kvc_fail("kvc_rglru_gates: too many channel tiles");
+  const int out_tiles = (bw + 15) / 16, wide = T <= 256 ? 16 : 64;
+  if (static_cast<int64_t>(nb) * ((bw + wide - 1) / wide) > 65535) return kvc_fail("kvc_rglru_gates: too many channel tiles");
   const bool vec = bw % 8 == 0 && ((reinterpret_cast<uintptr_t>(u) | reinterpret_cast<uintptr_t>(wa) |
                                     reinterpret_cast<uintptr_t>(wi) | reinterpret_cast<uintptr_t>(a_out) |
                                     reinterpret_cast<uintptr_t>(drive)) & 15) == 0;
-#define KVC_GATES(TT, AHEAD, VEC, WAVES)                                                                   \
-  hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC>),                                                 \
-                     dim3((T + 16 * TT * WAVES - 1) / (16 * TT * WAVES), nb * out_tiles), dim3(64 * WAVES), \
-                     0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles)
+#define KVC_GATES(TT, AHEAD, VEC, WAVES)                                                                     \
+  do {                                                                                                      \
+    const int token_tiles = (T + 16 * TT * WAVES - 1) / (16 * TT * WAVES);                                  \
+    const int64_t blocks = static_cast<int64_t>(token_tiles) * nb * out_tiles;                              \
+    if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");                           \
+    hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC>), dim3(static_cast<unsigned>(blocks)),           \
+                       dim3(64 * WAVES), 0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, \
+                       bw, out_tiles, token_tiles);                                                         \
+  } while (0)
   // few tokens: a wave a block, so that every compute unit has some, and more of a row on its way (8 tokens
   // 9.8 against 11.2 us, 40 tokens 10.3 against 12.8; 100 tokens 16.9 against 14.8)
   if (!vec)
