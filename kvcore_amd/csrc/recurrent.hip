@@ -899,10 +899,12 @@ extern "C" int kvc_gated_group_rmsnorm(void* out, int out_dtype, const float* y,
   if (groups > 65535) return kvc_fail("kvc_gated_group_rmsnorm: too many parts");
   const int n = width / groups;
   const uintptr_t z_four = z_dtype == 0 ? 15 : 7, out_four = out_dtype == 0 ? 15 : 7;
-  if (n % 4 == 0 && n <= 1024 && z_stride % 4 == 0 &&
+  const int64_t items = static_cast<int64_t>(T) * groups;
+  // a wave a part where that gives every compute unit a block of four (8 tokens of 8 parts: 5.3 us by waves, 4.6 by
+  // blocks, whose threads have two values each and not eight)
+  if (items >= 4 * static_cast<int64_t>(kvc_device_compute_units()) && n % 4 == 0 && n <= 1024 && z_stride % 4 == 0 &&
       ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(gain)) & 15) == 0 &&
       (reinterpret_cast<uintptr_t>(z) & z_four) == 0 && (reinterpret_cast<uintptr_t>(out) & out_four) == 0) {
-    const int64_t items = static_cast<int64_t>(T) * groups;
     KVC_DISPATCH_2(z_dtype, TZ, out_dtype, TO,
                    hipLaunchKernelGGL((gated_group_rmsnorm_wave_kernel<TZ, TO>), dim3(static_cast<unsigned>((items + 3) / 4)),
                                       dim3(256), 0, S(stream), static_cast<TO*>(out), y,

@@ -173,8 +173,9 @@ def test_convolution_reads_bfloat16_rows_and_writes_them(ops):
 
 @pytest.mark.parametrize("n,parts", [(4, 3), (252, 2), (512, 8), (1020, 1), (1024, 2), (1028, 1), (30, 2)])
 @pytest.mark.parametrize("shift", [0, 4, 1])
-def test_gated_norm_of_parts_that_a_wave_holds_and_does_not(ops, n, parts, shift):
-    T, width = 5, n * parts
+@pytest.mark.parametrize("T", [5, 1030])  # few parts take a block each
+def test_gated_norm_of_parts_that_a_wave_holds_and_does_not(ops, T, n, parts, shift):
+    width = n * parts
     y, g = rnd(T, width, seed=1), rnd(width, seed=2)
     z = rnd(T, width + 8, seed=3, dtype=torch.bfloat16)
     out = torch.empty(T, width, device=DEV)
