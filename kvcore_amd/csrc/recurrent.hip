@@ -181,8 +181,9 @@ __device__ __forceinline__ void gate_load8(f32x4_t* v, const float* row, int k, 
   }
 }
 
-template <int TT, int AHEAD, int VEC>
-__global__ __launch_bounds__(256) void rglru_gates_kernel(
+// SPLIT: a block of two waves, one a matrix, for the same tokens.
+template <int TT, int AHEAD, int VEC, int SPLIT>
+__global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
@@ -190,7 +191,8 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
   const int channel_tile = blockIdx.x / token_tiles;
-  const int t0 = ((blockIdx.x - channel_tile * token_tiles) * (blockDim.x >> 6) + wave) * 16 * TT;
+  const int token_tile = blockIdx.x - channel_tile * token_tiles;
+  const int t0 = (SPLIT ? token_tile : token_tile * 4 + wave) * 16 * TT;
   if (t0 >= T) return;
   const int blk = channel_tile / out_tiles;
   const int o0 = (channel_tile - blk * out_tiles) * 16;
@@ -208,8 +210,8 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
   f32x4_t av[AHEAD][2], iv[AHEAD][2], uv[AHEAD][TT][2];
   auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
     const int k = k0 + 8 * lk;
-    gate_load8<VEC>(av[slot], wa_row, k, bw);
-    gate_load8<VEC>(iv[slot], wi_row, k, bw);
+    gate_load8<VEC>(av[slot], SPLIT && wave ? wi_row : wa_row, k, bw);  // scalar
+    if constexpr (!SPLIT) gate_load8<VEC>(iv[slot], wi_row, k, bw);
 #pragma unroll
     for (int t = 0; t < TT; ++t) gate_load8<VEC>(uv[slot][t], u_row[t], k, bw);
   };
@@ -222,7 +224,7 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         a_now[h] = av[s][h];
-        i_now[h] = iv[s][h];
+        if constexpr (!SPLIT) i_now[h] = iv[s][h];
 #pragma unroll
         for (int t = 0; t < TT; ++t) u_now[t][h] = uv[s][t][h];
       }
@@ -232,9 +234,19 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
           acc_a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_a[t], 0, 0, 0);
-          acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
+          if constexpr (!SPLIT) acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
         }
     }
+  }
+  if constexpr (SPLIT) {
+    __shared__ f32x4_t other[TT][64];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+      if (wave) other[t][lane] = acc_a[t];
+    __syncthreads();
+    if (wave) return;
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc_i[t] = other[t][lane];
   }
   // a lane holds token li, outputs 4 lk .. of its tiles
   const int out = o0 + 4 * lk;
@@ -769,23 +781,24 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
   const bool vec = bw % 8 == 0 && ((reinterpret_cast<uintptr_t>(u) | reinterpret_cast<uintptr_t>(wa) |
                                     reinterpret_cast<uintptr_t>(wi) | reinterpret_cast<uintptr_t>(a_out) |
                                     reinterpret_cast<uintptr_t>(drive)) & 15) == 0;
-#define KVC_GATES(TT, AHEAD, VEC, WAVES)                                                                     \
+#define KVC_GATES(TT, AHEAD, VEC, SPLIT)                                                                     \
   do {                                                                                                      \
-    const int token_tiles = (T + 16 * TT * WAVES - 1) / (16 * TT * WAVES);                                  \
+    const int rows = 16 * TT * (SPLIT ? 1 : 4), token_tiles = (T + rows - 1) / rows;                                \
     const int64_t blocks = static_cast<int64_t>(token_tiles) * nb * out_tiles;                              \
     if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");                           \
-    hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC>), dim3(static_cast<unsigned>(blocks)),           \
-                       dim3(64 * WAVES), 0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, \
+    hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC, SPLIT>), dim3(static_cast<unsigned>(blocks)),           \
+                       dim3(SPLIT ? 128 : 256), 0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, \
                        bw, out_tiles, token_tiles);                                                         \
   } while (0)
-  // few tokens: a wave a block, so that every compute unit has some, and more of a row on its way (8 tokens
-  // 9.8 against 11.2 us, 40 tokens 10.3 against 12.8; 100 tokens 16.9 against 14.8)
+  // few tokens: a wave a matrix, so that every compute unit has some and a wave's chain of instructions is half as
+  // long, and more of a row on its way (8 tokens 8.4 against 11.2 us, 40 tokens 10.1 against 12.8; 100 tokens 16.9
+  // against 14.8; both matrices in one wave 9.8 and 10.3)
   if (!vec)
-    KVC_GATES(2, 1, 0, 4);
+    KVC_GATES(2, 1, 0, 0);
   else if (T <= 64)
     KVC_GATES(1, 4, 1, 1);
   else
-    KVC_GATES(2, 2, 1, 4);
+    KVC_GATES(2, 2, 1, 0);
 #undef KVC_GATES
   return kvc_check_launch("kvc_rglru_gates");
 }
