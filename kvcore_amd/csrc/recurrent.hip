@@ -678,7 +678,8 @@ __device__ __forceinline__ void put4(T* p, const float* v) {
 
 // The same for parts of at most 1,024 channels in fours, aligned: a wave a (token, part), the gated values kept in
 // registers between the sum and the norm.  A block a part waits for its barriers and makes every gate twice: 2,048 tokens
-// of 8 parts of 512 34 -> 18 us.
+// of 8 parts of 512 34 -> 18 us.  The squares are added in the block's order (its thread i takes the channels i, i + 256,
+// ...; lane l here stands for its threads 4 l .. 4 l + 3), so a row's bits do not depend on which of the two a step takes.
 template <typename TZ, typename TO>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(
     TO* __restrict__ out, const float* __restrict__ y, const TZ* __restrict__ z, int64_t z_stride,
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(
   const int n = width / groups, c0 = static_cast<int>(item - t * groups) * n;
   const float* yr = y + t * width + c0;
   const TZ* zr = z + t * z_stride + c0;
-  float v[4][4], ss = 0.f;
+  float v[4][4], ss[4] = {};
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int i = 4 * lane + 256 * k;
@@ -704,9 +705,18 @@ __global__ __launch_bounds__(256) void gated_group_rmsnorm_wave_kernel(
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[k][e] = i < n ? v[k][e] * silu_f(zv[e]) : 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) ss = fmaf(v[k][e], v[k][e], ss);
+    for (int e = 0; e < 4; ++e) ss[e] = fmaf(v[k][e], v[k][e], ss[e]);
   }
-  const float inv = 1.f / sqrtf(wave_sum(ss) / static_cast<float>(n) + eps);
+  // sixteen lanes stand for one wave of the block: its sum over the lanes, then the four waves' sums in order
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss[e] += __shfl_xor(ss[e], o, kWave);
+  const float mine = (ss[0] + ss[2]) + (ss[1] + ss[3]);
+  float sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) sum += __shfl(mine, 16 * w, kWave);
+  const float inv = 1.f / sqrtf(sum / static_cast<float>(n) + eps);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int i = 4 * lane + 256 * k;

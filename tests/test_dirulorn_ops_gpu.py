@@ -186,6 +186,25 @@ def test_gated_norm_of_parts_that_a_wave_holds_and_does_not(ops, T, n, parts, sh
     close(out, want, 2e-6, 2e-6)  # a sum of n squares and a few products, each rounded to 24 bits
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("n,parts", [(4, 8), (60, 8), (256, 8), (260, 4), (512, 8), (1000, 3), (1024, 8), (1028, 8), (30, 8)])
+def test_gated_norm_gives_a_token_the_same_bits_in_every_step(ops, n, parts, dtype):
+    """A token alone, in a small step and on either side of the step size from which waves take the parts."""
+    width, T = n * parts, 1100 // parts + 140
+    y, g, z = rnd(T, width, seed=4).to(DEV), rnd(width, seed=5).to(DEV), rnd(T, width, seed=6, dtype=dtype).to(DEV)
+
+    def norm(lo, hi):
+        out = torch.empty(hi - lo, width, device=DEV)
+        ops.gated_group_rmsnorm(out, y[lo:hi], z[lo:hi], g, 1e-5, parts)
+        return out
+
+    whole = norm(0, T)
+    edge = -(-4 * 256 // parts)  # four parts a compute unit
+    assert T > edge
+    for lo, hi in ((0, 1), (T - 1, T), (3, 11), (0, edge - 1), (0, edge), (T - edge, T), (T - edge + 1, T)):
+        assert torch.equal(norm(lo, hi), whole[lo:hi]), (lo, hi)
+
+
 # ------------------------------------------------------------ gated linear recurrence
 def plain_recurrence(u, y, wa, wi, ba, bi, lam, c):
     T, W = u.shape
