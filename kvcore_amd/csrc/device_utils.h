@@ -135,5 +135,6 @@ int kvc_device_compute_units(void);
 // Kernel families that have several variants to choose from at launch.  The entry points note
 // which one they launched (kvc_note_variant), and kvc_last_variant() tells the caller's thread:
 // for tests and tuning that must know which code ran.
-enum { kVariantPrefillAttention = 0, kVariantRopeKvWrite = 1, kVariantDecodeAttention = 2, kVariantFamilies = 3 };
+enum { kVariantPrefillAttention = 0, kVariantRopeKvWrite = 1, kVariantDecodeAttention = 2, kVariantMoeGemm = 3,
+       kVariantFamilies = 4 };
 void kvc_note_variant(int family, const char* name);

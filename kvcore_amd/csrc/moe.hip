@@ -614,27 +614,32 @@ __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
   align_pairs(sorted, tiles, num_tiles, ilds, pairs, E, max_tiles, tile_rows, ilds + pairs);
 }
 
-// bfloat16, few rows: a block of four waves takes one tile of up to 16 rows and 16 columns (gated: of gate and of
-// up), and its waves share K: wave w takes the passes w, w + 4, ... of 64 values, four of them on their way, and
-// the four sums are added in wave order.  In a pass lane (li, lk) fetches the 16 values from 16 lk of its weight
+// bfloat16, few rows: a wave takes one tile of up to 16 rows and 16 columns (gated: of gate and of up).  WK 4: the
+// four waves of a block share K: wave w takes the passes w, w + 4, ... of 64 values, four of them on their way, and
+// the four sums are added in wave order.  WK 1: each takes all of K of columns of its own.  In a pass lane (li, lk)
+// fetches the 16 values from 16 lk of its weight
 // row and of its token row (32 contiguous bytes, so that the four lanes of a row read one 128-byte line) and the
 // two matrix instructions take its first and its second eight (both operands are dealt the same way, so each
 // product still sums over all of K).  Bound by reading the weights of the experts that were chosen: with a whole K
 // a wave and 64 columns a block, one token of four experts of 2048 x 2048 had 128 blocks.  Gated and ungated, packed:
-// one token 22.0 and 13.4 -> 13.8 and 11.8 us, eight tokens 75 and 46 -> 64 and 34 us (5.6 TB/s).
-template <int GATED, typename TO, int PACKED>
+// one token 22.0 and 13.4 -> 13.8 and 11.8 us, eight tokens 75 and 46 -> 64 and 34 us (5.6 TB/s).  Where K is a few
+// passes long a share of it is one or two, and with many tiles four times the blocks cost more than they bring
+// (kvc_moe_gemm has the line): 128 experts of 1024 x 384, 8 rows each, down 37.0 us with WK 4, 20.8 with WK 1
+// (two passes on their way: with four 22.6).
+template <int GATED, typename TO, int PACKED, int WK>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
     int act, const float* __restrict__ row_scale) {
-  constexpr int kWavesK = 4, kStages = 4;
-  __shared__ f32x4_t part[(kWavesK - 1) * (GATED ? 2 : 1)][64];
+  constexpr int kStages = WK == 1 ? 2 : 4;
   const int tile = blockIdx.y;
   if (tile >= *num_tiles) return;
   const int e = tiles[3 * tile], r0 = tiles[3 * tile + 1], nr = tiles[3 * tile + 2];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
-  const int n0 = blockIdx.x * 16;
+  const int of_block = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int wave = WK == 1 ? 0 : of_block;  // whose share of K
+  const int n0 = (WK == 1 ? blockIdx.x * 4 + of_block : blockIdx.x) * 16;
+  if (n0 >= N) return;  // scalar; with WK 4 the whole block
   const int li = lane & 15, lk = lane >> 4;
   // B operand: token row li of the tile; A operand: the expert's row n0 + li
   const bool row_ok = li < nr;
@@ -653,7 +658,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
   const int passes = K / 64;
   // blocks walk K round from places of their own, as in the kernel for more rows
-  const int turn = passes > 0 ? (e * 5 + static_cast<int>(blockIdx.x) * 3) % passes : 0;
+  const int turn = passes > 0 ? (e * 5 + (n0 >> 4) * 3) % passes : 0;
   bf16x8_t an[kStages][2], a2n[kStages][2], bn[kStages][2];
   auto fetch = [&](int slot, int pass) {  // no branch around the loads: a pass that is not there repeats the last
     int p = pass < passes ? pass + turn : passes - 1 + turn;
@@ -668,11 +673,11 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   };
   if (wave < passes) {  // scalar
 #pragma unroll
-    for (int s = 0; s < kStages; ++s) fetch(s, wave + kWavesK * s);
-    for (int p = wave; p < passes; p += kWavesK * kStages) {
+    for (int s = 0; s < kStages; ++s) fetch(s, wave + WK * s);
+    for (int p = wave; p < passes; p += WK * kStages) {
 #pragma unroll
       for (int s = 0; s < kStages; ++s) {
-        if (p + kWavesK * s >= passes) break;  // scalar
+        if (p + WK * s >= passes) break;  // scalar
         bf16x8_t a[2], a2[2], b[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -680,7 +685,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
           if (GATED) a2[h] = a2n[s][h];
           b[h] = bn[s][h];
         }
-        if (p + kWavesK * kStages < passes) fetch(s, p + kWavesK * (s + kStages));
+        if (p + WK * kStages < passes) fetch(s, p + WK * (s + kStages));
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h], b[h], acc, 0, 0, 0);
@@ -707,16 +712,19 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
       if (GATED) acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[h], b[h], acc2, 0, 0, 0);
     }
   }
-  if (wave > 0) {
-    part[wave - 1][lane] = acc;
-    if (GATED) part[kWavesK - 2 + wave][lane] = acc2;
-  }
-  __syncthreads();
-  if (wave > 0) return;
+  if constexpr (WK > 1) {
+    __shared__ f32x4_t part[(WK - 1) * (GATED ? 2 : 1)][64];
+    if (wave > 0) {
+      part[wave - 1][lane] = acc;
+      if (GATED) part[WK - 2 + wave][lane] = acc2;
+    }
+    __syncthreads();
+    if (wave > 0) return;
 #pragma unroll
-  for (int v = 0; v < kWavesK - 1; ++v) {
-    acc += part[v][lane];
-    if (GATED) acc2 += part[kWavesK - 1 + v][lane];
+    for (int v = 0; v < WK - 1; ++v) {
+      acc += part[v][lane];
+      if (GATED) acc2 += part[WK - 1 + v][lane];
+    }
   }
   // lane holds column (token) li, rows (features) n0 + 4 * lk + i
   if (!row_ok) return;
@@ -1156,20 +1164,30 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
 #undef KVC_MOE_TILED
     } else if (vectors && max_tiles > 65535) {
       return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
-    } else if (packed) {
-      grid = dim3((N + 15) / 16, max_tiles);
-      if (!vectors || N % 16 || K % 64)
-        return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
-      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, 1>), bf16_t, bf16_t);
-      else if (gated) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, float, 1>), bf16_t, float);
-      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, bf16_t, 1>), bf16_t, bf16_t);
-      else KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, float, 1>), bf16_t, float);
     } else if (vectors) {
-      grid = dim3((N + 15) / 16, max_tiles);
-      if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, 0>), bf16_t, bf16_t);
-      else if (gated) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, float, 0>), bf16_t, float);
-      else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, bf16_t, 0>), bf16_t, bf16_t);
-      else KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, float, 0>), bf16_t, float);
+      if (packed && (N % 16 || K % 64))
+        return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
+      // A whole K a wave where a share of it is at most two passes and there are waves enough without: one a compute unit
+      // for each 256 of K.  Shares / whole: 64 experts of 2048 x 512 down, 8 rows each, 36.7 / 26.2 us; 8 experts of 512 x
+      // 512 gated, 1 row each (256 waves), 5.4 / 6.6 us, 32 rows (768 waves) 9.5 / 8.3; 4 experts of 256 x 320 gated, 48
+      // rows (320 waves), 7.1 / 5.8; 16 experts of 1024 x 1024 (sixteen passes), 64 rows, 27 / 33 us.
+      const bool whole = K <= 512 && static_cast<int64_t>(max_tiles) * ((N + 15) / 16) * 256 >= static_cast<int64_t>(K) * kvc_device_compute_units();
+      kvc_note_variant(kVariantMoeGemm, whole ? "moe_gemm_few_kernel, whole K" : "moe_gemm_few_kernel, shares of K");
+      grid = dim3(whole ? (N + 63) / 64 : (N + 15) / 16, max_tiles);
+#define KVC_MOE_FEW(PACKED, WK)                                                                                  \
+  do {                                                                                                          \
+    if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, PACKED, WK>), bf16_t, bf16_t);   \
+    else if (gated) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, float, PACKED, WK>), bf16_t, float);                 \
+    else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, bf16_t, PACKED, WK>), bf16_t, bf16_t);      \
+    else KVC_MOE_LAUNCH((moe_gemm_few_kernel<0, float, PACKED, WK>), bf16_t, float);                            \
+  } while (0)
+      if (packed && whole) KVC_MOE_FEW(1, 1);
+      else if (packed) KVC_MOE_FEW(1, 4);
+      else if (whole) KVC_MOE_FEW(0, 1);
+      else KVC_MOE_FEW(0, 4);
+#undef KVC_MOE_FEW
+    } else if (packed) {
+      return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
     } else {
       if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_plain_kernel<1, bf16_t, bf16_t>), bf16_t, bf16_t);
       else if (gated) KVC_MOE_LAUNCH((moe_gemm_plain_kernel<1, bf16_t, float>), bf16_t, float);

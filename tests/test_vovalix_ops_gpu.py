@@ -559,6 +559,50 @@ def test_products_of_experts_over_tiles_of_many_rows(tile_rows, packed, gated, N
     assert rel(out, want) < (2e-6 if out_dtype == torch.float32 else 3e-3)
 
 
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "packed"])
+@pytest.mark.parametrize("gated,N,K,whole", [
+    (True, 64, 2048, False),    # 32 passes of 64: eight a wave, more than are on their way at once
+    (False, 48, 1088, False),   # 17 passes
+    (True, 32, 1000, False),    # a ragged end along K
+    (False, 2048, 576, False),  # many waves, K too long for a whole one
+    (True, 336, 512, False), (False, 160, 256, False),  # 504 and 240 waves: just too few
+    (True, 352, 512, True), (False, 176, 256, True), (False, 1000, 456, True), (False, 1040, 64, True), (True, 999, 8, True)])
+def test_few_rows_take_shares_of_k_or_all_of_it(gated, N, K, whole, packed):
+    """Both sides of the line between the two, with 24 tiles of up to 16 rows (the line: a wave of 16 columns a unit for
+    each 256 of K, and K of at most 512)."""
+    from kvcore_amd.ops import library as ops
+
+    if packed and (N % 16 or K % 64):
+        pytest.skip("a packed matrix has experts of a multiple of 16 rows of a multiple of 64")
+    gen = torch.Generator().manual_seed(N + K)
+    E, T = 8, 16 * 16
+    choice = torch.randint(1, E, (T,), generator=gen)
+    choice[:17] = 3
+    x = torch.randn(T, K, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(E * N * (2 if gated else 1), K, generator=gen) * K ** -0.5).to(torch.bfloat16)
+    wg = gpu(w, torch.bfloat16)
+    if packed:
+        ops.pack_weight(wg)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+    tiles = torch.empty(ops.moe_max_tiles(T, E, 16), 3, **i32)
+    assert tiles.shape[0] == 24
+    ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32).view(T, 1), E, 16)
+    out = torch.full((T, N), float("nan"), device=DEV)
+    ops.moe_gemm(out, gpu(x, torch.bfloat16), wg, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1, out_sorted=False,
+                 gated=gated, limit=1.2, alpha=1.702, up_shift=1.0, tile_rows=16)
+    assert ops.last_variant("moe_gemm") == "moe_gemm_few_kernel, " + ("whole K" if whole else "shares of K")
+    per, want = w.double().view(E, -1, K), torch.empty(T, N, dtype=torch.float64)
+    for e in range(E):
+        at = choice == e
+        y = x[at].double() @ per[e].T
+        if gated:
+            g, u = y[:, :N].clamp(max=1.2), y[:, N:].clamp(-1.2, 1.2)
+            y = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        want[at] = y
+    assert rel(out, want) < 2e-6  # float32 sums of exact products
+
+
 def test_offset_norm_keeps_a_gain_of_one_plus_the_stored_weight():
     from kvcore_amd.parts.base import Runtime
     from kvcore_amd.parts.rmsnorm import RMSNorm
