@@ -1168,10 +1168,11 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
       if (packed && (N % 16 || K % 64))
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
       // A whole K a wave where a share of it is at most two passes and there are waves enough without: one a compute unit
-      // for each 256 of K.  Shares / whole: 64 experts of 2048 x 512 down, 8 rows each, 36.7 / 26.2 us; 8 experts of 512 x
-      // 512 gated, 1 row each (256 waves), 5.4 / 6.6 us, 32 rows (768 waves) 9.5 / 8.3; 4 experts of 256 x 320 gated, 48
-      // rows (320 waves), 7.1 / 5.8; 16 experts of 1024 x 1024 (sixteen passes), 64 rows, 27 / 33 us.
-      const bool whole = K <= 512 && static_cast<int64_t>(max_tiles) * ((N + 15) / 16) * 256 >= static_cast<int64_t>(K) * kvc_device_compute_units();
+      // up to K of 256, three up to 512.  Shares / whole: 64 experts of 2048 x 512 down, 8 rows each, 36.7 / 26.2 us; 8
+      // experts of 512 x 512 gated, 1 row each (256 waves), 5.4 / 6.6 us, 32 rows (768 waves) 9.5 / 8.3; 4 experts of
+      // 256 x 320 gated, 48 rows (320 waves), 7.1 / 5.8; 16 experts of 1024 x 1024 (sixteen passes), 64 rows, 27 / 33 us.
+      const int64_t waves = static_cast<int64_t>(max_tiles) * ((N + 15) / 16);
+      const bool whole = K <= 512 && waves >= (K <= 256 ? 1 : 3) * static_cast<int64_t>(kvc_device_compute_units());
       kvc_note_variant(kVariantMoeGemm, whole ? "moe_gemm_few_kernel, whole K" : "moe_gemm_few_kernel, shares of K");
       grid = dim3(whole ? (N + 63) / 64 : (N + 15) / 16, max_tiles);
 #define KVC_MOE_FEW(PACKED, WK)                                                                                  \

@@ -565,11 +565,11 @@ def test_products_of_experts_over_tiles_of_many_rows(tile_rows, packed, gated, N
     (False, 48, 1088, False),   # 17 passes
     (True, 32, 1000, False),    # a ragged end along K
     (False, 2048, 576, False),  # many waves, K too long for a whole one
-    (True, 336, 512, False), (False, 160, 256, False),  # 504 and 240 waves: just too few
-    (True, 352, 512, True), (False, 176, 256, True), (False, 1000, 456, True), (False, 1040, 64, True), (True, 999, 8, True)])
+    (True, 496, 512, False), (False, 160, 256, False),  # 744 and 240 waves: just too few
+    (True, 512, 512, True), (False, 176, 256, True), (False, 1000, 456, True), (False, 1040, 64, True), (True, 999, 8, True)])
 def test_few_rows_take_shares_of_k_or_all_of_it(gated, N, K, whole, packed):
-    """Both sides of the line between the two, with 24 tiles of up to 16 rows (the line: a wave of 16 columns a unit for
-    each 256 of K, and K of at most 512)."""
+    """Both sides of the line between the two, with 24 tiles of up to 16 rows (the line: K of at most 512, from a wave of
+    16 columns a unit on up to K of 256, from three beyond)."""
     from kvcore_amd.ops import library as ops
 
     if packed and (N % 16 or K % 64):
