@@ -34,6 +34,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "device_utils.h"
 #include "gemm_common.h"
 #include "kvcore_hip.h"
@@ -1092,15 +1094,36 @@ extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
   return pairs < most ? pairs : most;  // no tile is empty
 }
 
-// Tiles that hold an expert's rows as a rule, so that a fetched weight meets all of them.  Measured over 32 experts of
-// 2048 x 2048, both products: 2 rows an expert 119 us in tiles of 16 and 120 in tiles of 64, 4 rows 137 and 135; 37
-// rows 156 us in tiles of 64 and 155 in tiles of 128, 64 rows 182 and 166.  From 104 to 150 rows many an expert has a
-// few more than 128, and two tiles of half the size cost more than smaller ones: 128 rows 232 us in tiles of 64, 253
-// in tiles of 128; 192 rows 287 and 247.
-extern "C" int kvc_moe_tile_rows(int pairs, int E) {
-  const int64_t e = E;
-  if (pairs >= 150 * e || (pairs >= 40 * e && pairs < 104 * e)) return kBigTileRows;
-  return pairs >= 3 * e ? kMidTileRows : kTileRows;
+// How many rows a tile holds, for experts of matrices [I, H] ([2 I, H] if gated) and [H, I], by an estimate of both
+// products in us (routing taken as even).  Tiles of 16: every expert's matrices once at 5.6 TB/s, and again for each
+// further tile, of which there are some from 6 rows an expert on.  Tiles of 64: one fetch, but columns of 128 (ungated
+// 256) a block, so a step is no faster than a block's walk along K (0.8 us a pass of 64), and blocks that
+// come out uneven on the units wait for the last.  Both products of even routing, tiles of 16 / 64:
+//   32 experts of 2048 x 2048    8 rows an expert  136 / 139 us,   12  146 / 141,   64  444 / 188
+//   8 experts of 512 x 512      16 rows             14 /  21 us,   48   15 /  26,   64   22 /  25
+//   4 experts of 1024 x 2048     8 rows             16 /  38 us,   48   33 /  48
+//   128 experts of 1024 x 384    6 rows             56 /  63 us,   16   77 /  68
+// Tiles of 128 where experts have that many rows and the blocks still fill the chip (300 in either product if they held
+// 64 rows: the second of two blocks a unit keeps the matrix cores busy): 32 experts of 2048 x 2048, 64 rows each,
+// 188 / 165 us, 16 experts of 1024 x 1024 41 / 53.  From 104 to 150 rows many an expert has a few more than 128, and two
+// tiles of half the size cost more than smaller ones: 128 rows 227 us in tiles of 64, 249 in tiles of 128.
+extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
+  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0) return kTileRows;
+  const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
+  const double used = pairs < E ? pairs : E;  // experts with rows
+  const int first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, down_cols = (H + 255) / 256;
+  const double down_mb = 2e-6 * H * I, first_mb = gated ? 2 * down_mb : down_mb;
+  const double again = each > 6 ? (each - 6) / 16 * E : 0;
+  const double few = 8 + (first_mb + down_mb) * (used / 5.6 + again / 6);
+  const double mid_tiles = used + (each > 32 ? (each - 32) / 64 * E : 0);
+  auto product = [&](double mb, int k, int cols) {
+    const double a_unit = mid_tiles * cols / units;
+    const double uneven = a_unit > 1 ? ceil(a_unit) / a_unit : 1;
+    return 4 + fmax(0.8 * k / 64, used * mb / 5.6 * uneven);
+  };
+  if (each <= 64 && few <= product(first_mb, H, first_cols) + product(down_mb, I, down_cols)) return kTileRows;
+  const double blocks = (pairs / 64.0 + E / 2.0) * (first_cols < down_cols ? first_cols : down_cols);
+  return blocks >= 300 && (each >= 150 || (each >= 40 && each < 104)) ? kBigTileRows : kMidTileRows;
 }
 
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,

@@ -75,7 +75,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_moe_router_spread": [P, P, P, P, P, I, I, P, L, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
         "kvc_moe_router_spread_floats": [I, I],
         "kvc_moe_max_tiles": [I, I, I],
-        "kvc_moe_tile_rows": [I, I],
+        "kvc_moe_tile_rows": [I, I, I, I, I],
         "kvc_moe_align": [P, P, P, P, I, I, I, I, P],
         "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, I, P],
         "kvc_moe_combine": [P, P, P, I, P, I, P, P, I, I, I, P],
@@ -2071,13 +2071,14 @@ def moe_router_spread(choice: torch.Tensor, weight: torch.Tensor, sorted_pairs: 
         "kvc_moe_router_spread")
 
 
-def moe_tile_rows(pairs: int, experts: int, x: torch.Tensor | None = None, k_sizes: tuple[int, ...] = ()) -> int:
+def moe_tile_rows(pairs: int, experts: int, x: torch.Tensor | None = None, k_sizes: tuple[int, int] = (2048, 2048),
+                  gated: bool = True) -> int:
     """Rows a tile of the experts' products holds for a step of this size: 128 or 64 where the experts have
-    many rows on average and the operands allow (bfloat16, every K a multiple of 32), else 16."""
-    rows = int(load().kvc_moe_tile_rows(pairs, experts))
-    if rows > 16 and (x is None or x.dtype != torch.bfloat16 or any(k % 32 for k in k_sizes)):
+    rows enough for their matrices' sizes (``k_sizes``: K of the first product and of the second) and the operands
+    allow (bfloat16, every K a multiple of 32), else 16."""
+    if x is None or x.dtype != torch.bfloat16 or any(k % 32 for k in k_sizes):
         return 16
-    return rows
+    return int(load().kvc_moe_tile_rows(pairs, experts, *k_sizes, int(gated)))
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16) -> int:

@@ -5,6 +5,7 @@ be fastest, and a kernel whose operands do not fit is never chosen."""
 from __future__ import annotations
 
 import pytest
+import torch
 
 from kvcore_amd.ops.library import choose_product
 
@@ -45,3 +46,25 @@ def test_decode_graph_sizes(limit):
         assert padded <= limit and padded < 2 * live + (live == 1)
         if live > 16:
             assert padded - live < 32
+
+
+@pytest.mark.parametrize("experts,H,I,rows", [
+    (32, 2048, 2048, {1: 16, 4: 16, 16: 64, 40: 64, 64: 128, 128: 64, 192: 128, 512: 128}),
+    (8, 512, 512, {3: 16, 16: 16, 48: 16, 96: 64, 192: 64, 512: 64}),
+    (8, 2048, 512, {4: 16, 24: 16, 96: 64, 384: 64}),
+    (4, 1024, 2048, {3: 16, 32: 16, 96: 64, 256: 64}),
+    (4, 256, 320, {4: 16, 48: 16, 256: 64}),
+    (128, 1024, 384, {3: 16, 6: 16, 16: 64, 64: 128, 128: 64}),
+    (64, 4096, 1408, {2: 16, 8: 64, 32: 64, 96: 128}),
+    (16, 512, 2048, {4: 16, 8: 16, 32: 64, 192: 64})])
+def test_rows_a_tile_of_the_experts_products_holds(experts, H, I, rows):
+    """Experts of small matrices keep tiles of 16 until their rows fill larger ones, and none gets tiles of 128 whose
+    blocks would leave the chip idle: within a few percent of the fastest measured of the three."""
+    from kvcore_amd.ops import library as ops
+
+    x = torch.empty(1, H, dtype=torch.bfloat16)
+    for each, tile in rows.items():
+        assert ops.moe_tile_rows(each * experts, experts, x, (H, I)) == tile, each
+    assert ops.moe_tile_rows(512 * experts, experts, x.float(), (H, I)) == 16
+    assert ops.moe_tile_rows(512 * experts, experts, x, (H, I + 8)) == 16
+    assert ops.moe_max_tiles(0, experts, 64) == 0 and ops.moe_tile_rows(0, experts, x, (H, I)) == 16
