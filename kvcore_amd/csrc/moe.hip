@@ -410,14 +410,13 @@ __global__ __launch_bounds__(kRouterWaves * 64) void moe_router_kernel(
   else route_one(ct, wt, zr, zr, zr + E, zr + 2 * E, lane, E, rule);
 }
 
-// One block.  counts -> offsets and tiles (a thread an expert) -> sorted pairs.  `ilds`: [4 E] in LDS.
+// One block.  counts -> offsets and tiles (a thread an expert) -> sorted pairs.  `ilds`: [3 E] in LDS.
 __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
                                             int32_t* __restrict__ num_tiles, const int32_t* choice, int pairs, int E,
                                             int max_tiles, int tile_rows, int32_t* ilds) {
   int32_t* count = ilds;           // [E]
   int32_t* offset = count + E;     // [E]
-  int32_t* cursor = offset + E;    // [E]
-  int32_t* ntiles = cursor + E;    // [E]
+  int32_t* cursor = offset + E;    // [E]; at first the experts' numbers of tiles
   for (int e = threadIdx.x; e < E; e += blockDim.x) count[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
@@ -433,7 +432,6 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
   };
   auto list = [&](int e, int n, int each, int at, int nt) {
     offset[e] = at;
-    cursor[e] = 0;
     for (int r = 0; r < n && nt < max_tiles; r += each, ++nt) {
       tiles[3 * nt] = e;
       tiles[3 * nt + 1] = at + r;
@@ -460,18 +458,20 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
   } else {
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
       const int each = rows_each(count[e]);
-      ntiles[e] = (count[e] + each - 1) / each;
+      cursor[e] = (count[e] + each - 1) / each;
     }
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
       int at = 0, nt = 0;
       for (int p = 0; p < e; ++p) {
         at += count[p];
-        nt += ntiles[p];
+        nt += cursor[p];
       }
       list(e, count[e], rows_each(count[e]), at, nt);
     }
+    __syncthreads();
   }
+  for (int e = threadIdx.x; e < E; e += blockDim.x) cursor[e] = 0;
   __syncthreads();
   // an expert's pairs take their places in the order in which their threads arrive: a row's sums
   // do not depend on its place
@@ -605,7 +605,7 @@ __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
     int32_t* __restrict__ choice, float* __restrict__ weight, float* __restrict__ gate, int32_t* __restrict__ sorted,
     int32_t* __restrict__ tiles, int32_t* __restrict__ num_tiles, const float* __restrict__ parts, int T_, int E,
     int max_tiles, int tile_rows, RouteRule rule) {
-  extern __shared__ int32_t ilds[];  // [T top] choices, then [4 E]
+  extern __shared__ int32_t ilds[];  // [T top] choices, then [3 E]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   if (wave < T_)  // scalar
     choose_from_parts(ilds + wave * rule.top, weight + static_cast<int64_t>(wave) * rule.top, gate, parts, wave, T_, E, lane,
@@ -1081,7 +1081,7 @@ extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* so
   else KVC_PARTS(float, 0);
 #undef KVC_PARTS
   if (T <= kChooseInOne) {
-    hipLaunchKernelGGL(moe_choose_align_kernel, dim3(1), dim3(1024), sizeof(int32_t) * (T * top + 4 * E), S(stream),
+    hipLaunchKernelGGL(moe_choose_align_kernel, dim3(1), dim3(1024), sizeof(int32_t) * (T * top + 3 * E), S(stream),
                        choice, weight, gate, sorted, tiles, num_tiles, parts, T, E, max_tiles, tile_rows, rule);
     return kvc_check_launch("kvc_moe_router_spread");
   }
@@ -1132,7 +1132,7 @@ extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles
     return kvc_fail("kvc_moe_align: tiles of 16, 64 or 128 rows");
   if (pairs < 0 || E <= 0 || max_tiles < kvc_moe_max_tiles(pairs, E, tile_rows))
     return kvc_fail("kvc_moe_align: bad sizes, or room for fewer tiles than the routing may need");
-  const size_t lds = sizeof(int32_t) * 4 * E;
+  const size_t lds = sizeof(int32_t) * 3 * E;
   if (lds > 60000) return kvc_fail("kvc_moe_align: too many experts");
   hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), lds, S(stream), sorted, tiles, num_tiles, choice,
                      pairs, E, max_tiles, tile_rows);

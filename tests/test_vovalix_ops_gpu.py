@@ -603,6 +603,31 @@ def test_few_rows_take_shares_of_k_or_all_of_it(gated, N, K, whole, packed):
     assert rel(out, want) < 2e-6  # float32 sums of exact products
 
 
+@pytest.mark.parametrize("E", [65, 1500, 5000])
+def test_tiles_of_very_many_experts(E):
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(E)
+    T, top = 3000, 3
+    choice = torch.randint(0, E, (T, top), generator=gen)
+    choice[:200] = E - 1
+    i32 = dict(dtype=torch.int32, device=DEV)
+    sorted_pairs, num = torch.full((T * top,), -1, **i32), torch.empty(1, **i32)
+    tiles = torch.full((ops.moe_max_tiles(T * top, E, 64), 3), -1, **i32)
+    ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32), E, 64)
+    of_pair, at = choice.flatten(), 0
+    order = sorted_pairs.cpu().long()
+    assert torch.equal(order.sort().values, torch.arange(T * top))
+    assert torch.equal(of_pair[order], of_pair.sort().values)
+    for e, first, n in tiles[: int(num)].tolist():
+        assert first == at and 1 <= n <= 64 and (of_pair[order[first: first + n]] == e).all()
+        at += n
+    assert at == T * top
+    too_many = torch.zeros(1, 1, **i32)
+    with pytest.raises(ops.KernelError, match="too many experts"):
+        ops.moe_align(sorted_pairs, torch.empty(ops.moe_max_tiles(1, 5001, 16), 3, **i32), num, too_many, 5001, 16)
+
+
 def test_offset_norm_keeps_a_gain_of_one_plus_the_stored_weight():
     from kvcore_amd.parts.base import Runtime
     from kvcore_amd.parts.rmsnorm import RMSNorm
