@@ -635,7 +635,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
     int act, const float* __restrict__ row_scale) {
   constexpr int kStages = WK == 1 ? 2 : 4;
-  const int tile = blockIdx.y;
+  const int tile = blockIdx.z * gridDim.y + blockIdx.y;  // more tiles than a grid's second dimension takes
   if (tile >= *num_tiles) return;
   const int e = tiles[3 * tile], r0 = tiles[3 * tile + 1], nr = tiles[3 * tile + 2];
   const int of_block = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
@@ -1185,8 +1185,6 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
         else KVC_MOE_TILED(4, 0);
       }
 #undef KVC_MOE_TILED
-    } else if (vectors && max_tiles > 65535) {
-      return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
     } else if (vectors) {
       if (packed && (N % 16 || K % 64))
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
@@ -1197,7 +1195,8 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
       const int64_t waves = static_cast<int64_t>(max_tiles) * ((N + 15) / 16);
       const bool whole = K <= 512 && waves >= (K <= 256 ? 1 : 3) * static_cast<int64_t>(kvc_device_compute_units());
       kvc_note_variant(kVariantMoeGemm, whole ? "moe_gemm_few_kernel, whole K" : "moe_gemm_few_kernel, shares of K");
-      grid = dim3(whole ? (N + 63) / 64 : (N + 15) / 16, max_tiles);
+      const int layers = (max_tiles + 65534) / 65535;
+      grid = dim3(whole ? (N + 63) / 64 : (N + 15) / 16, (max_tiles + layers - 1) / layers, layers);
 #define KVC_MOE_FEW(PACKED, WK)                                                                                  \
   do {                                                                                                          \
     if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_few_kernel<1, bf16_t, PACKED, WK>), bf16_t, bf16_t);   \

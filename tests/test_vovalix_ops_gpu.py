@@ -603,6 +603,25 @@ def test_few_rows_take_shares_of_k_or_all_of_it(gated, N, K, whole, packed):
     assert rel(out, want) < 2e-6  # float32 sums of exact products
 
 
+def test_more_tiles_of_few_rows_than_a_grid_dimension_holds():
+    """K that tiles of 64 rows do not take, and 65,536 tiles of 16."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(1)
+    E, T, N, K = 3, 65536 * 16 - 40, 16, 8
+    choice = torch.randint(0, E, (T, 1), generator=gen).to(device=DEV, dtype=torch.int32)
+    x, w = (gpu(torch.randn(n, K, generator=gen), torch.bfloat16) for n in (T, E * N))
+    i32 = dict(dtype=torch.int32, device=DEV)
+    sorted_pairs, num, tiles = torch.empty(T, **i32), torch.empty(1, **i32), torch.empty(ops.moe_max_tiles(T, E, 16), 3, **i32)
+    assert tiles.shape[0] > 65535
+    ops.moe_align(sorted_pairs, tiles, num, choice, E, 16)
+    out = torch.full((T, N), float("nan"), device=DEV)
+    ops.moe_gemm(out, x, w, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1, out_sorted=False, gated=False, tile_rows=16)
+    every = (x.float() @ w.float().T).view(T, E, N)  # eight exact products a sum
+    want = every.gather(1, choice.long()[:, :, None].expand(-1, -1, N))[:, 0]
+    assert torch.allclose(out, want, atol=1e-5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("E", [65, 1500, 5000])
 def test_tiles_of_very_many_experts(E):
     from kvcore_amd.ops import library as ops
