@@ -11,6 +11,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "device_utils.h"
 #include "kvcore_hip.h"
 
@@ -165,25 +167,28 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
 // fewer waves in flight that their registers leave no better over other sizes.  Through LDS with
 // a multiply and an add a step it took 129 us.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-constexpr int GK = 32;
+constexpr int GT = 16, GK = 32;
 
-// eight inputs of a row from k on, zeros beyond the block (VEC: whole 16-byte pieces)
-template <int VEC>
-__device__ __forceinline__ void gate_load8(f32x4_t* v, const float* row, int k, int bw) {
-  if constexpr (VEC) {
-    const float* p = row + (k < bw ? k : 0);
-    v[0] = *reinterpret_cast<const f32x4_t*>(p);
-    v[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
-    if (k >= bw) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = k + i < bw ? row[k + i] : 0.f;
-  }
+// The results for one channel of a token from its two sums (biases added), softplus(lam) and its input.
+__device__ __forceinline__ void gate_results(float& a, float& drive, float sum_a, float sum_i, float sp, float c_decay,
+                                             float u) {
+  const float r = sigmoid_f(sum_a);
+  const float g = sigmoid_f(sum_i);
+  const float log_a = -c_decay * r * sp;
+  a = expf(log_a);
+  drive = sqrtf(-expm1f(2.f * log_a)) * g * u;
 }
 
-// SPLIT: a block of two waves, one a matrix, for the same tokens.
-template <int TT, int AHEAD, int VEC, int SPLIT>
-__global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
+// eight inputs of a row from k on, zeros beyond the block (bw a multiple of 8)
+__device__ __forceinline__ void gate_load8(f32x4_t* v, const float* row, int k, int bw) {
+  const float* p = row + (k < bw ? k : 0);
+  v[0] = *reinterpret_cast<const f32x4_t*>(p);
+  v[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
+  if (k >= bw) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+
+template <int TT, int AHEAD>
+__global__ __launch_bounds__(256) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
   const int li = lane & 15, lk = lane >> 4;
   const int channel_tile = blockIdx.x / token_tiles;
   const int token_tile = blockIdx.x - channel_tile * token_tiles;
-  const int t0 = (SPLIT ? token_tile : token_tile * 4 + wave) * 16 * TT;
+  const int t0 = (token_tile * 4 + wave) * 16 * TT;
   if (t0 >= T) return;
   const int blk = channel_tile / out_tiles;
   const int o0 = (channel_tile - blk * out_tiles) * 16;
@@ -210,10 +215,10 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
   f32x4_t av[AHEAD][2], iv[AHEAD][2], uv[AHEAD][TT][2];
   auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
     const int k = k0 + 8 * lk;
-    gate_load8<VEC>(av[slot], SPLIT && wave ? wi_row : wa_row, k, bw);  // scalar
-    if constexpr (!SPLIT) gate_load8<VEC>(iv[slot], wi_row, k, bw);
+    gate_load8(av[slot], wa_row, k, bw);
+    gate_load8(iv[slot], wi_row, k, bw);
 #pragma unroll
-    for (int t = 0; t < TT; ++t) gate_load8<VEC>(uv[slot][t], u_row[t], k, bw);
+    for (int t = 0; t < TT; ++t) gate_load8(uv[slot][t], u_row[t], k, bw);
   };
 #pragma unroll
   for (int s = 0; s < AHEAD; ++s) fetch(s, GK * s);
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         a_now[h] = av[s][h];
-        if constexpr (!SPLIT) i_now[h] = iv[s][h];
+        i_now[h] = iv[s][h];
 #pragma unroll
         for (int t = 0; t < TT; ++t) u_now[t][h] = uv[s][t][h];
       }
@@ -234,61 +239,175 @@ __global__ __launch_bounds__(SPLIT ? 128 : 256) void rglru_gates_kernel(
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
           acc_a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_a[t], 0, 0, 0);
-          if constexpr (!SPLIT) acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
+          acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
         }
     }
   }
-  if constexpr (SPLIT) {
-    __shared__ f32x4_t other[TT][64];
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-      if (wave) other[t][lane] = acc_a[t];
-    __syncthreads();
-    if (wave) return;
-#pragma unroll
-    for (int t = 0; t < TT; ++t) acc_i[t] = other[t][lane];
-  }
   // a lane holds token li, outputs 4 lk .. of its tiles
   const int out = o0 + 4 * lk;
-  const int left = bw - out;
-  if (left <= 0) return;
+  if (out >= bw) return;
   const int c = blk * bw + out;
   float sp[4], b_a[4], b_i[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int ce = e < left ? c + e : c;
-    sp[e] = softplus_f(lam[ce]);
-    b_a[e] = ba[ce];
-    b_i[e] = bi[ce];
+    sp[e] = softplus_f(lam[c + e]);
+    b_a[e] = ba[c + e];
+    b_i[e] = bi[c + e];
   }
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
     const int tok = t0 + 16 * t + li;
     if (tok >= T) continue;
     const int64_t at = static_cast<int64_t>(tok) * W + c;
-    f32x4_t a4, d4, u4;
-    if (VEC) {
-      u4 = *reinterpret_cast<const f32x4_t*>(u + at);
-    } else {
+    const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(u + at);
+    float a4[4], d4[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) u4[e] = u[e < left ? at + e : at];
+    for (int e = 0; e < 4; ++e) gate_results(a4[e], d4[e], acc_a[t][e] + b_a[e], acc_i[t][e] + b_i[e], sp[e], c_decay, u4[e]);
+    *reinterpret_cast<f32x4_t*>(a_out + at) = f32x4_t{a4[0], a4[1], a4[2], a4[3]};
+    *reinterpret_cast<f32x4_t*>(drive + at) = f32x4_t{d4[0], d4[1], d4[2], d4[3]};
+  }
+}
+
+// The same, with the same bits, for few blocks of 16 tokens x 16 outputs: the block's first wave takes one matrix, the
+// second the other, four chunks on their way, and then every thread the results of one channel of one token.  Where one
+// wave made all 256 of them, 8 tokens of 10 blocks of 32 channels took 5.8 us, this way 3.7, of 256 channels 8.2 and 6.1.
+__global__ __launch_bounds__(256) void rglru_gates_few_kernel(
+    float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
+    const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
+    const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
+    int bw, int out_tiles, int token_tiles) {
+  constexpr int AHEAD = 4, kRow = 20;
+  __shared__ __attribute__((aligned(16))) float sums[2][16 * kRow];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int channel_tile = blockIdx.x / token_tiles;
+  const int t0 = (blockIdx.x - channel_tile * token_tiles) * 16;
+  const int blk = channel_tile / out_tiles;
+  const int o0 = (channel_tile - blk * out_tiles) * 16;
+  // what this thread makes in the end
+  const int my_tok = threadIdx.x >> 4, my_out = threadIdx.x & 15;
+  const bool mine = t0 + my_tok < T && o0 + my_out < bw;
+  const int c = blk * bw + (mine ? o0 + my_out : 0);
+  const int64_t at = static_cast<int64_t>(mine ? t0 + my_tok : 0) * W + c;
+  const float sp = softplus_f(lam[c]), b_a = ba[c], b_i = bi[c], my_u = u[at];
+  if (wave < 2) {  // scalar
+    const int li = lane & 15, lk = lane >> 4;
+    // outputs and tokens beyond the last read the last one and are not stored
+    const float* w_row = (wave ? wi : wa) + (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
+    const float* u_row = u + static_cast<int64_t>(t0 + li < T ? t0 + li : T - 1) * W + blk * bw;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, wv[AHEAD][2], uv[AHEAD][2];
+    auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
+      gate_load8(wv[slot], w_row, k0 + 8 * lk, bw);
+      gate_load8(uv[slot], u_row, k0 + 8 * lk, bw);
+    };
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) fetch(s, GK * s);
+    for (int k0 = 0; k0 < bw; k0 += GK * AHEAD) {
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {
+        if (k0 + GK * s >= bw) break;  // scalar
+        f32x4_t w_now[2], u_now[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) w_now[h] = wv[s][h], u_now[h] = uv[s][h];
+        fetch(s, k0 + GK * (s + AHEAD));
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w_now[j >> 2][j & 3], u_now[j >> 2][j & 3], acc, 0, 0, 0);
+      }
+    }
+    *reinterpret_cast<f32x4_t*>(sums[wave] + li * kRow + 4 * lk) = acc;  // token li, outputs 4 lk ..
+  }
+  __syncthreads();
+  if (!mine) return;
+  const int s = my_tok * kRow + my_out;
+  gate_results(a_out[at], drive[at], sums[0][s] + b_a, sums[1][s] + b_i, sp, c_decay, my_u);
+}
+
+// Channel blocks of any width and alignment: 256 threads take 16 tokens x GO outputs and walk the inputs 32 at a time
+// through LDS, which deals out loads of four bytes side by side; a thread sums its products in the order k = 0, 1, ...
+// (Rows of 250 channels with such loads straight to the matrix instructions' registers: 2,048 tokens of 10 blocks
+// 255 us, this way 123; 8 tokens 14.0 and 9.4.)
+// GO outputs a block and TPT = GO / 16 tokens a thread: 64 and 4 for many tokens; 16 and 1 for
+// steps of few tokens, whose blocks are then four times as many (the weights, read once, are
+// all the work there, and a launch of a few dozen blocks leaves most of the chip idle).
+template <int GO, int TPT>
+__global__ __launch_bounds__(256) void rglru_gates_any_kernel(
+    float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
+    const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
+    const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
+    int bw, int out_tiles) {
+  static_assert(GO * (GT / TPT) == 256, "a thread per (output, group of tokens)");
+  __shared__ float wa_s[GO][GK + 1];
+  __shared__ float wi_s[GO][GK + 1];
+  __shared__ float u_s[GT][GK];
+  const int tid = threadIdx.x;
+  const int t0 = blockIdx.x * GT;
+  const int blk = blockIdx.y / out_tiles;
+  const int o0 = (blockIdx.y - blk * out_tiles) * GO;
+  const int ol = tid % GO;
+  const int tg = tid / GO;
+  const float* wa_b = wa + static_cast<int64_t>(blk) * bw * bw;
+  const float* wi_b = wi + static_cast<int64_t>(blk) * bw * bw;
+  float acc_a[TPT], acc_i[TPT];
+#pragma unroll
+  for (int tt = 0; tt < TPT; ++tt) acc_a[tt] = acc_i[tt] = 0.f;
+  // a stage of 32 inputs is fetched into registers while the stage before it is multiplied
+  constexpr int NW = GO * GK / 256, NU = GT * GK / 256;
+  float wa_r[NW], wi_r[NW], u_r[NU];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const int idx = tid + i * 256;
+      const int row = idx / GK, col = idx - row * GK;
+      const bool ok = o0 + row < bw && k0 + col < bw;
+      const int64_t off = static_cast<int64_t>(o0 + row) * bw + k0 + col;
+      wa_r[i] = ok ? wa_b[off] : 0.f;
+      wi_r[i] = ok ? wi_b[off] : 0.f;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float r = sigmoid_f(acc_a[t][e] + b_a[e]);
-      const float g = sigmoid_f(acc_i[t][e] + b_i[e]);
-      const float log_a = -c_decay * r * sp[e];
-      a4[e] = expf(log_a);
-      d4[e] = sqrtf(-expm1f(2.f * log_a)) * g * u4[e];
+    for (int i = 0; i < NU; ++i) {
+      const int idx = tid + i * 256;
+      const int row = idx / GK, col = idx - row * GK;
+      const bool ok = t0 + row < T && k0 + col < bw;
+      u_r[i] = ok ? u[static_cast<int64_t>(t0 + row) * W + blk * bw + k0 + col] : 0.f;
     }
-    if (VEC) {
-      *reinterpret_cast<f32x4_t*>(a_out + at) = a4;
-      *reinterpret_cast<f32x4_t*>(drive + at) = d4;
-    } else {
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < bw; k0 += GK) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (e < left) a_out[at + e] = a4[e], drive[at + e] = d4[e];
+    for (int i = 0; i < NW; ++i) {
+      const int idx = tid + i * 256;
+      wa_s[idx / GK][idx % GK] = wa_r[i];
+      wi_s[idx / GK][idx % GK] = wi_r[i];
     }
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int idx = tid + i * 256;
+      u_s[idx / GK][idx % GK] = u_r[i];
+    }
+    __syncthreads();
+    if (k0 + GK < bw) fetch(k0 + GK);
+#pragma unroll 8
+    for (int k = 0; k < GK; ++k) {
+      const float va = wa_s[ol][k], vi = wi_s[ol][k];
+#pragma unroll
+      for (int tt = 0; tt < TPT; ++tt) {
+        const float uv = u_s[tg * TPT + tt][k];
+        acc_a[tt] = fmaf(va, uv, acc_a[tt]);
+        acc_i[tt] = fmaf(vi, uv, acc_i[tt]);
+      }
+    }
+    __syncthreads();
+  }
+  if (o0 + ol >= bw) return;
+  const int c = blk * bw + o0 + ol;
+  const float sp = softplus_f(lam[c]);
+  const float b_a = ba[c], b_i = bi[c];
+#pragma unroll
+  for (int tt = 0; tt < TPT; ++tt) {
+    const int t = t0 + tg * TPT + tt;
+    if (t >= T) continue;
+    const int64_t at = static_cast<int64_t>(t) * W + c;
+    gate_results(a_out[at], drive[at], acc_a[tt] + b_a, acc_i[tt] + b_i, sp, c_decay, u[at]);
   }
 }
 
@@ -786,30 +905,44 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
   if (T < 0 || W <= 0 || nb <= 0 || W % nb) return kvc_fail("kvc_rglru_gates: bad sizes");
   if (T == 0) return 0;
   const int bw = W / nb;
-  const int out_tiles = (bw + 15) / 16, wide = T <= 256 ? 16 : 64;
-  if (static_cast<int64_t>(nb) * ((bw + wide - 1) / wide) > 65535) return kvc_fail("kvc_rglru_gates: too many channel tiles");
+  // the widths that have always been served: channel tiles of 16 up to 256 tokens, of 64 beyond, at most 65,535
+  const bool narrow = T <= 256;
+  const int wide_tiles = narrow ? (bw + 15) / 16 : (bw + 63) / 64;
+  if (static_cast<int64_t>(nb) * wide_tiles > 65535) return kvc_fail("kvc_rglru_gates: too many channel tiles");
   const bool vec = bw % 8 == 0 && ((reinterpret_cast<uintptr_t>(u) | reinterpret_cast<uintptr_t>(wa) |
                                     reinterpret_cast<uintptr_t>(wi) | reinterpret_cast<uintptr_t>(a_out) |
                                     reinterpret_cast<uintptr_t>(drive)) & 15) == 0;
-#define KVC_GATES(TT, AHEAD, VEC, SPLIT)                                                                     \
-  do {                                                                                                      \
-    const int rows = 16 * TT * (SPLIT ? 1 : 4), token_tiles = (T + rows - 1) / rows;                                \
-    const int64_t blocks = static_cast<int64_t>(token_tiles) * nb * out_tiles;                              \
-    if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");                           \
-    hipLaunchKernelGGL((rglru_gates_kernel<TT, AHEAD, VEC, SPLIT>), dim3(static_cast<unsigned>(blocks)),           \
-                       dim3(SPLIT ? 128 : 256), 0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, \
-                       bw, out_tiles, token_tiles);                                                         \
-  } while (0)
-  // few tokens: a wave a matrix, so that every compute unit has some and a wave's chain of instructions is half as
-  // long, and more of a row on its way (8 tokens 8.4 against 11.2 us, 40 tokens 10.1 against 12.8; 100 tokens 16.9
-  // against 14.8; both matrices in one wave 9.8 and 10.3)
-  if (!vec)
-    KVC_GATES(2, 1, 0, 0);
-  else if (T <= 64)
-    KVC_GATES(1, 4, 1, 1);
+  if (!vec) {
+    const dim3 grid((T + GT - 1) / GT, nb * wide_tiles);  // tokens on x, which has no 16-bit limit
+    if (narrow)
+      hipLaunchKernelGGL((rglru_gates_any_kernel<16, 1>), grid, dim3(256), 0, S(stream), a_out, drive, u, wa,
+                         wi, ba, bi, lam, c_decay, T, W, bw, wide_tiles);
+    else
+      hipLaunchKernelGGL((rglru_gates_any_kernel<64, 4>), grid, dim3(256), 0, S(stream), a_out, drive, u, wa,
+                         wi, ba, bi, lam, c_decay, T, W, bw, wide_tiles);
+    return kvc_check_launch("kvc_rglru_gates");
+  }
+  const int out_tiles = (bw + 15) / 16;
+  // Small blocks or large, whichever an estimate in us says: small ones share the units, a large one has its walk along
+  // the inputs to itself and a second on the same unit costs most of another.  Large / small blocks, both measured:
+  // 10 blocks of 256 channels, 64 tokens, 11.9 / 10.7 us, 100 tokens 14.8 / 15.1, 256 tokens 24.8 / 27.1; one block
+  // of 128, 256 tokens, 10.2 / 4.7, 2,048 tokens 10.7 / 8.1, 4,096 tokens 11.4 / 13.4; 10 blocks of 160, 256 tokens
+  // 13.5 / 14.3, 257 tokens 19.8 / 14.9.
+  const double units = kvc_device_compute_units();
+  const int64_t few_blocks = static_cast<int64_t>((T + 15) / 16) * nb * out_tiles;
+  const int64_t big_blocks = static_cast<int64_t>((T + 127) / 128) * nb * out_tiles;
+  const double few_us = 4 + few_blocks / units * (0.6 + 0.0065 * bw);
+  const double big_us = 4 + (0.25 + 0.75 * ceil(big_blocks / units)) * (4.5 + 0.029 * bw);
+  const bool few = few_us <= big_us;
+  const int token_tiles = few ? (T + 15) / 16 : (T + 127) / 128;
+  const int64_t blocks = few ? few_blocks : big_blocks;
+  if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");
+  if (few)
+    hipLaunchKernelGGL(rglru_gates_few_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out, drive,
+                       u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles, token_tiles);
   else
-    KVC_GATES(2, 2, 1, 0);
-#undef KVC_GATES
+    hipLaunchKernelGGL((rglru_gates_kernel<2, 2>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out,
+                       drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles, token_tiles);
   return kvc_check_launch("kvc_rglru_gates");
 }
 

@@ -279,6 +279,32 @@ def test_gates_of_a_token_do_not_depend_on_the_step(ops, W, nb):
             assert torch.equal(got, want[first: first + n])
 
 
+@pytest.mark.parametrize("W,nb", [(512, 2), (512, 8), (520, 13), (60, 2)])
+def test_gates_in_long_portions_are_those_of_short_steps(ops, W, nb):
+    """Steps long enough for the larger blocks, tokens that do not fill them and channels that do not fill tiles of
+    16: 64-bit results, and the bits of the same rows in steps that take the small ones."""
+    T, bw = 2100, W // nb
+    u = rnd(T, W, seed=1).to(DEV)
+    d = [rnd(nb, bw, bw, seed=s, std=bw ** -0.5).to(DEV) for s in (2, 3)]
+    d += [rnd(nb, bw, seed=4).to(DEV), rnd(nb, bw, seed=5).to(DEV), rnd(W, seed=6).to(DEV)]
+
+    def run(first, n):
+        a, drive = torch.empty(n, W, device=DEV), torch.empty(n, W, device=DEV)
+        ops.rglru_gates(a, drive, u[first: first + n], *d, 8.0)
+        return a, drive
+
+    whole = run(0, T)
+    ud = u.double().view(T, nb, bw)
+    r, g = (torch.sigmoid((torch.stack([ud[:, i] @ w[i].double().T for i in range(nb)], 1) + b.double()).view(T, W))
+            for w, b in ((d[0], d[2]), (d[1], d[3])))
+    log_a = -8.0 * r * torch.nn.functional.softplus(d[4].double())
+    close(whole[0], log_a.exp().cpu(), 1e-5, 1e-5)
+    close(whole[1], (torch.sqrt(-torch.expm1(2 * log_a)) * g * u.double()).cpu(), 1e-5, 1e-5)
+    for first, n in ((0, 1), (2080, 20), (500, 100), (7, 300)):
+        for got, want in zip(run(first, n), whole):
+            assert torch.equal(got, want[first: first + n]), (first, n)
+
+
 def test_long_portions_are_scanned_in_segments_side_by_side(ops):
     """With a workspace, requests longer than a segment are cut into segments that are scanned
     side by side and joined in order: the same results, whatever the portions, beside short
