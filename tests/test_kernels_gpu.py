@@ -137,6 +137,28 @@ def test_gemm_f32_tiles_give_the_same_bits(ops, M, N, K):
         assert torch.equal(single[0], out[i])
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 70000, 8), (16, 140003, 16), (16, 100, 32), (70, 515, 24), (2100, 4100, 30), (800, 1000, 64),
+                                   (2100, 5000, 96), (2100, 800, 100), (2100, 801, 99), (1030, 6200, 130), (1030, 2052, 192),
+                                   (2100, 2052, 256), (2100, 2052, 255), (2100, 2052, 257)])
+def test_gemm_f32_of_short_rows_gives_the_same_bits(ops, M, N, K):
+    """K of at most eight chunks and enough of C for a wave to take all of them: the sums of a 64-bit product, and a row's
+    bits as the other kernel (which takes a few rows from two chunks on) makes them; every tile shape and width of load."""
+    wide = rnd(M, K + 3, seed=4)
+    for a in (wide[:, :K].contiguous(), wide[:, 3:]):  # the second: rows at any 4 bytes
+        w, b = rnd(N, K, seed=5), rnd(N, seed=6)
+        out = torch.full((M, N + 1), 7.0, device=DEV)
+        ops.gemm_f32(out[:, :N], a, w, b)
+        assert (out[:, N] == 7.0).all()
+        rows = torch.randint(0, M, (40,), generator=torch.Generator().manual_seed(K)).tolist() + [0, M - 1]
+        some = a[rows].double()
+        bound = 4 * math.sqrt(K) * 2 ** -24 * (some.abs() @ w.double().abs().T + b.double().abs())
+        assert ((out[rows, :N].double() - (some @ w.double().T + b.double())).abs() <= bound + 1e-7).all()
+        single = torch.empty(1, N, device=DEV)
+        for i in {0, M // 2, M - 1}:
+            ops.gemm_f32(single, a[i:i + 1].contiguous(), w, b)
+            assert torch.equal(single[0], out[i, :N])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (5, 100, 200), (8, 4096, 4096), (16, 130, 1032),
                                    (17, 6144, 512), (33, 48, 14336), (64, 1000, 2048),
                                    # the longest sum and the widest output of the 70B shape
