@@ -807,7 +807,8 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, T* __restrict__ k_cach
 // contiguous, so a token alone stores its value two bytes at a time, d * nkv stores 32 bytes
 // apart; when the block's eight tokens lie side by side in one page (a portion of a prompt
 // mostly does), a thread gathers one element of all eight and stores them together; otherwise it
-// stores them one by one, all eight loads on their way first.  The tile's items are dealt to
+// stores them one by one, all eight loads on their way first.  Page and offset of the eight are made
+// by a lane each (by every lane for all eight, 2 kv heads of 16 took 0.7 us longer).  The tile's items are dealt to
 // gridDim.y blocks, about one of each kind a thread, since a chain of a few loads is all there is
 // to wait for: 122 tokens of 40 heads of 64 in float32 16.5 -> 5.5 us, 8 kv heads
 // of 64 in bfloat16 for a thousand tokens with decode tokens among them 15.3 -> 8.0, 8 of 128 for
@@ -874,37 +875,61 @@ __global__ __launch_bounds__(256) void rope_kv_write_tile_kernel(
     store8(k_cache + (static_cast<int64_t>(page) * nkv * page_size + off) * d + head * head_step + i, v);
   }
   // ---- v: element i of a head goes to V[page, head, i, off]
+  // lane i of every eight looks at token i
+  const int mine = threadIdx.x & (TILE - 1);
+  const int my_slot = mine < n_tok ? kv_slot[t0 + mine] : -1;
+  const int my_page = (my_slot >= 0 ? my_slot : 0) / page_size, my_off = (my_slot >= 0 ? my_slot : 0) - my_page * page_size;
+  const int s0 = __builtin_amdgcn_readlane(my_slot, 0);
+  const bool side_by_side = s0 >= 0 && (s0 & 7) == 0 && (page_size & 7) == 0 && __all(my_slot == s0 + mine);
+  // (eight slots from a multiple of eight stay within a page whose size is a multiple of eight)
+  auto head0 = [&](int ti) -> int64_t {  // where token ti's element 0 of head 0 goes
+    return static_cast<int64_t>(__builtin_amdgcn_readlane(my_page, ti)) * nkv * page_size * d + __builtin_amdgcn_readlane(my_off, ti);
+  };
+  if (side_by_side) {  // scalar
+    T* base = v_cache + head0(0);
+    for (int w = first; w < nkv * d; w += step) {
+      const int head = w / d;
+      const int i = w - head * d;
+      const T* src = qkv + t0 * row_elems + static_cast<int64_t>(nh + nkv) * d + w;
+      alignas(16) T vals[TILE];
+#pragma unroll
+      for (int ti = 0; ti < TILE; ++ti) vals[ti] = src[ti * row_elems];
+      T* dst = base + head * head_step + static_cast<int64_t>(i) * page_size;
+      *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(vals);
+      if constexpr (sizeof(T) == 4) *reinterpret_cast<uint4*>(dst + 4) = *reinterpret_cast<const uint4*>(vals + 4);
+    }
+    return;
+  }
+  if (nkv * d < 256) {
+    // fewer elements than threads: the tokens are dealt out too (1 kv head of 64, 64 tokens: 5.9 us eight a thread, 5.4)
+    for (int w = first; w < n_tok * nkv * d; w += step) {
+      const int ti = w / (nkv * d);
+      const int rest = w - ti * nkv * d;
+      const int head = rest / d;
+      const int i = rest - head * d;
+      const int slot = kv_slot[t0 + ti];
+      if (slot < 0) continue;
+      const int page = slot / page_size, off = slot - page * page_size;
+      v_cache[static_cast<int64_t>(page) * nkv * page_size * d + off + head * head_step + static_cast<int64_t>(i) * page_size] =
+          qkv[(t0 + ti) * row_elems + static_cast<int64_t>(nh + nkv) * d + rest];
+    }
+    return;
+  }
+  int64_t at[TILE];
   int slots[TILE];
 #pragma unroll
-  for (int ti = 0; ti < TILE; ++ti) slots[ti] = ti < n_tok ? kv_slot[t0 + ti] : -1;
-  const int s0 = slots[0];
-  bool side_by_side = s0 >= 0 && (s0 & 7) == 0 && (page_size & 7) == 0;
-#pragma unroll
-  for (int ti = 1; ti < TILE; ++ti) side_by_side = side_by_side && slots[ti] == s0 + ti;
-  // (eight slots from a multiple of eight stay within a page whose size is a multiple of eight)
-  int64_t at[TILE];  // of head 0, element 0
-#pragma unroll
-  for (int ti = 0; ti < TILE; ++ti) {
-    const int slot = slots[ti] >= 0 ? slots[ti] : 0;
-    const int page = slot / page_size, off = slot - page * page_size;
-    at[ti] = static_cast<int64_t>(page) * nkv * page_size * d + off;
-  }
+  for (int ti = 0; ti < TILE; ++ti) at[ti] = head0(ti), slots[ti] = __builtin_amdgcn_readlane(my_slot, ti);
   for (int w = first; w < nkv * d; w += step) {
     const int head = w / d;
     const int i = w - head * d;
     const T* src = qkv + t0 * row_elems + static_cast<int64_t>(nh + nkv) * d + w;
-    alignas(16) T vals[TILE];
+    T vals[TILE];
 #pragma unroll
     for (int ti = 0; ti < TILE; ++ti) vals[ti] = src[(ti < n_tok ? ti : 0) * row_elems];
     T* dst = v_cache + head * head_step + static_cast<int64_t>(i) * page_size;
-    if (side_by_side) {  // scalar
-      *reinterpret_cast<uint4*>(dst + at[0]) = *reinterpret_cast<const uint4*>(vals);
-      if constexpr (sizeof(T) == 4) *reinterpret_cast<uint4*>(dst + at[0] + 4) = *reinterpret_cast<const uint4*>(vals + 4);
-    } else {
 #pragma unroll
-      for (int ti = 0; ti < TILE; ++ti)
-        if (slots[ti] >= 0) dst[at[ti]] = vals[ti];  // scalar
-    }
+    for (int ti = 0; ti < TILE; ++ti)
+      if (slots[ti] >= 0) dst[at[ti]] = vals[ti];  // scalar
   }
 }
 

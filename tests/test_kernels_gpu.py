@@ -654,7 +654,9 @@ def test_rope_kv_write(ops, dtype, interleaved, rot_dim):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("nh,nkv,d,rot_dim,page", [(4, 2, 64, 64, 16), (3, 1, 32, 16, 8), (2, 2, 128, 64, 48)])
+@pytest.mark.parametrize("nh,nkv,d,rot_dim,page", [(4, 2, 64, 64, 16), (3, 1, 32, 16, 8), (2, 2, 128, 64, 48),
+                                                   # values on both sides of a block of 256, pages of no multiple of 8
+                                                   (2, 1, 248, 32, 16), (2, 1, 256, 32, 16), (1, 3, 24, 16, 12), (1, 9, 40, 32, 12)])
 @pytest.mark.parametrize("rotate_q", [True, False])
 def test_rope_kv_write_of_many_tokens_equals_token_by_token(ops, dtype, nh, nkv, d, rot_dim, page, rotate_q):
     """Steps of 16 tokens and more take a kernel that handles eight tokens a block and stores
