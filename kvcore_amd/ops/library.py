@@ -1580,6 +1580,18 @@ def gated_chunk_count(lengths, start: int) -> int:
     return sum(-(-n // chunk) for n in lengths if n >= start)
 
 
+def gated_chunk_start(lengths, start: int, ahead: float) -> int:
+    """Where chunks begin in a step of these request lengths: at requests of ``start`` tokens, or 0, nowhere.  The scan
+    of the shorter requests then follows the chunks instead of running beside the longest one's, so chunks are taken if
+    the longest request has ``ahead`` tokens more than the longest that stays with the scan (which, were it of single
+    tokens, still costs what 16 do)."""
+    longest = max(lengths, default=0)
+    if longest < start:
+        return 0
+    rest = max((n for n in lengths if n < start), default=None)
+    return start if longest - (0 if rest is None else max(rest, 16)) >= ahead else 0
+
+
 def gated_chunk_work(buffers, name: str, chunks: int, start: int, heads: int, key_heads: int, rows: int,
                      cols: int, per_channel: bool = False) -> torch.Tensor:
     """The step buffer that ``ssm_chunks``, ``scalar_gate_chunks`` and (``per_channel``) ``channel_gate_chunks`` work in:

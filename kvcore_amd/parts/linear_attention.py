@@ -37,13 +37,25 @@ from .base import Mixer, ParamSource, ParamSpec, StateNeed, register_mixer
 
 # from so many tokens of one request in a step on, lightning attention works in chunks
 CHUNKED_FROM = 48
-# and a bfloat16 model's matrix memories (16 heads of 64 x 129: 128 tokens 28 us token by token and 31 in chunks, eight
-# requests of 128 tokens 67 and 47, 2,048 tokens 405 and 57); a float32 model walks every token, so that its results
-# do not depend on how a request is cut into steps
+# requests of so many tokens may be cut into chunks by a bfloat16 model's matrix memories and by its states with a factor
+# a channel (see _chunk_start); a float32 model walks every token, so that its results do not depend on how a request is
+# cut into steps
 GATED_CHUNKED_FROM = 128
-# a factor a channel (16 heads of 64 x 128: 128 tokens 25 and 35 us, 192 tokens 35 and 36, 512 tokens 88 and 39, three
-# requests of 683 tokens 152 and 82, 2,048 tokens 357 and 68)
-CHANNEL_CHUNKED_FROM = 192
+CHANNEL_CHUNKED_FROM = 160
+
+
+def _chunk_start(lengths, start: int, floats: int, many: int, ahead: int) -> int:
+    """From how many tokens on a step's requests are cut into chunks (0: none are), for states of ``floats`` a request.
+
+    The scan takes as long as its longest request, some 0.18 us a token while its blocks have a compute unit to
+    themselves (``ahead`` tokens cost what chunks cost at least) and about twice that from ``many`` floats of states a
+    unit on.  Scan and chunks, us: matrix memories of 16 heads of 64 x 129, one request of 128 tokens 29 and 33, 192 tokens
+    41 and 33, 2,048 tokens 406 and 58, six of 128 tokens 67 and 40, 16 of 512 tokens 371 and 200; factors a channel, 16
+    heads of 64 x 128, one of 192 tokens 35 and 36, 512 tokens 86 and 39, eight of 192 tokens 82 and 60, 16 heads of 128 x
+    128, one of 192 tokens 77 and 59; beside eight requests of 100 tokens, one of 192 84 and 90, 111 and 113, of 256 106 and
+    90, 137 and 113, beside eight of single tokens, one of 192 69 and 40, 80 and 41."""
+    crowded = len(lengths) * floats >= many * ops.compute_units()
+    return ops.gated_chunk_start(lengths, start, 88 if crowded else ahead)
 
 
 def _src(name: str, rows: int) -> tuple[ParamSource, ...]:
@@ -124,6 +136,10 @@ class GatedLinearAttention(_MatrixStateMixer):
     def state_needs(self) -> tuple[StateNeed, ...]:
         return (StateNeed((self.heads, ops.linear_state_rows(self.dim), self.vdim)),)
 
+    def chunk_start(self, lengths) -> int:
+        return _chunk_start(lengths, CHANNEL_CHUNKED_FROM, self.heads * self.dim * self.vdim, 2560,
+                            152 if self.dim > 64 else 192)
+
     def forward(self, x, ctx, call, sink=None):
         p, qk, inner = self.params, self.qk, self.inner
         state = ctx.states[call.state_indices[0]]
@@ -140,16 +156,18 @@ class GatedLinearAttention(_MatrixStateMixer):
         rows = (proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner])
         sizes = dict(heads=self.heads, qk_heads=self.heads, dim=self.dim, vdim=self.vdim, q_scale=self.q_scale,
                      **self._batch(ctx))
-        chunks = 0
+        chunks = start = 0
         if ctx.dtype == torch.bfloat16 and self.dim <= 128:
             chunks = ops.gated_chunk_count(ctx.host_query_lens, CHANNEL_CHUNKED_FROM)
         if chunks:
+            # reserved by every step that has such requests, cut or not: an engine counts it before it sizes its cache
             work = ops.gated_chunk_work(ctx.buffers, "gla_chunks", chunks, CHANNEL_CHUNKED_FROM, self.heads, self.heads,
                                         self.dim, self.vdim, per_channel=True)
-            ops.channel_gate_chunks(o, *rows, decay, state, work, chunks=chunks, start=CHANNEL_CHUNKED_FROM, **sizes)
-        if not chunks or min(ctx.host_query_lens) < CHANNEL_CHUNKED_FROM:
-            ops.linear_state_scan(o, *rows, decay, None, state, delta_rule=False,
-                                  below=CHANNEL_CHUNKED_FROM if chunks else 0, **sizes)
+            start = self.chunk_start(ctx.host_query_lens)
+        if start:
+            ops.channel_gate_chunks(o, *rows, decay, state, work, chunks=chunks, start=start, **sizes)
+        if not start or min(ctx.host_query_lens) < start:
+            ops.linear_state_scan(o, *rows, decay, None, state, delta_rule=False, below=start, **sizes)
         return self._finish(o, proj[:, 2 * qk + inner:], ctx)
 
 
@@ -276,6 +294,10 @@ class MaxGatedMatrixMemory(_MatrixStateMixer):
         # the matrices with the normaliser as their last column, and the running maxima
         return (StateNeed((self.heads, ops.linear_state_rows(self.dim), self.vdim + 1)), StateNeed((self.heads,)))
 
+    def chunk_start(self, lengths) -> int:
+        return _chunk_start(lengths, GATED_CHUNKED_FROM, self.heads * self.dim * (self.vdim + 1), 3072,
+                            112 if self.dim > 64 else 152)
+
     def forward(self, x, ctx, call, sink=None):
         p, qk, inner, nh = self.params, self.qk, self.inner, self.heads
         state, maxima = (ctx.states[i] for i in call.state_indices)
@@ -293,15 +315,17 @@ class MaxGatedMatrixMemory(_MatrixStateMixer):
         o = ctx.buf(f"mm_o:{wide}", wide, torch.float32)
         rows = (proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + inner], keep, take, state)
         sizes = dict(heads=nh, qk_heads=nh, dim=self.dim, vdim=self.vdim + 1, ones_column=True, q_scale=self.q_scale)
-        chunks = 0
+        chunks = start = 0
         if ctx.dtype == torch.bfloat16 and self.dim <= 128:
             chunks = ops.gated_chunk_count(ctx.host_query_lens, GATED_CHUNKED_FROM)
-        if chunks:
+        if chunks:  # reserved cut or not, as for factors a channel
             work = ops.gated_chunk_work(ctx.buffers, "mm_chunks", chunks, GATED_CHUNKED_FROM, nh, nh, self.dim,
                                         self.vdim + 1)
-            ops.scalar_gate_chunks(o, *rows, work, chunks=chunks, start=GATED_CHUNKED_FROM, **sizes, **batch)
-        if not chunks or min(ctx.host_query_lens) < GATED_CHUNKED_FROM:
-            ops.linear_state_scan(o, *rows, scalar_gates=True, below=GATED_CHUNKED_FROM if chunks else 0, **sizes, **batch)
+            start = self.chunk_start(ctx.host_query_lens)
+        if start:
+            ops.scalar_gate_chunks(o, *rows, work, chunks=chunks, start=start, **sizes, **batch)
+        if not start or min(ctx.host_query_lens) < start:
+            ops.linear_state_scan(o, *rows, scalar_gates=True, below=start, **sizes, **batch)
         normed = ctx.buf(f"ms_normed:{inner}", inner)
         ops.max_gated_finish(normed, o, m, proj[:, 2 * qk + inner:2 * qk + 2 * inner], p["norm"], self.eps,
                              self.den_eps, nh, self.vdim)

@@ -36,10 +36,9 @@ def _src(name: str, rows: int) -> tuple[ParamSource, ...]:
     return (ParamSource(name, 0, rows),)
 
 
-# from so many tokens of one request in a step on, a bfloat16 model's state-space layers work in chunks (64 heads of
-# 128 x 64: 128 tokens 27 us token by token and 37 in chunks, 256 tokens 49 and 41, 2,048 tokens 383 and 127); a
-# float32 model walks every token, so that its results do not depend on how a request is cut into steps
-SSM_CHUNKED_FROM = 192
+# requests of so many tokens in a step may be cut into chunks by a bfloat16 model's state-space layers (see chunk_start);
+# a float32 model walks every token, so that its results do not depend on how a request is cut into steps
+SSM_CHUNKED_FROM = 160
 
 
 class GatedLinearRecurrence(Mixer):
@@ -182,6 +181,24 @@ class StateSpaceMixer(Mixer):
         if self.state_size > most:
             raise ValueError(f"a state of {self.state_size} rows a head: the recurrence kernel serves {most}")
 
+    def chunk_start(self, lengths) -> int:
+        """From how many tokens on a step's requests are cut into chunks (0: none are).
+
+        The scan takes as long as its longest request, on as many blocks as there are requests times heads times
+        tiles of 64 columns.  Below a block a compute unit it has 0.2 us a token and its fixed cost is less; from there
+        on 0.55 us; three blocks a unit fill the chip, and then it is the faster by a tenth, but for a fourth, which
+        starts another round.  Scan and chunks, 64 heads of 128 x 64 in 8 groups, us: one request of 192 tokens
+        39 and 40, 256 tokens 51 and 42, 2,048 tokens 376 and 125; four of 192 tokens 108 and 65, eight of 256 tokens
+        150 and 129, twelve of 512 tokens 351 and 384, sixteen of 256 tokens 288 and 258, 32 of 256 tokens 474 and 519;
+        one of 320 tokens beside one of 100 tokens 72 and 75, one of 256 beside eight of single tokens 142 and 53."""
+        units = ops.compute_units()
+        blocks = self.heads * -(-self.head_dim // 64)
+        full = blocks * sum(n >= SSM_CHUNKED_FROM for n in lengths) / units
+        if full >= 3 and not (self.state_size > 64 and 4 <= full < 5):
+            return 0
+        share = blocks * len(lengths) / units
+        return ops.gated_chunk_start(lengths, SSM_CHUNKED_FROM, 176 + 96 * share if share < 1 else 88)
+
     def forward(self, x, ctx, call, sink=None):
         p = self.params
         conv_state, ssm_state = (ctx.states[i] for i in call.state_indices)
@@ -198,16 +215,19 @@ class StateSpaceMixer(Mixer):
                         single_tokens=ctx.max_query_len == 1, **batch)
         y = ctx.buf(f"ssm_y:{self.inner}", self.inner, torch.float32)
         sizes = dict(heads=self.heads, head_dim=self.head_dim, state_size=self.state_size, groups=self.groups)
-        chunks = 0
+        rows = (y, xbc, dt_raw, p["dt_bias"], p["A_log"], p["D"], ssm_state)
+        chunks = start = 0
         if ctx.dtype == torch.bfloat16 and self.state_size <= 128:
             chunks = ops.gated_chunk_count(ctx.host_query_lens, SSM_CHUNKED_FROM)
-        rows = (y, xbc, dt_raw, p["dt_bias"], p["A_log"], p["D"], ssm_state)
         if chunks:
+            # reserved by every step that has such requests, cut or not: an engine counts it before it sizes its cache
             work = ops.gated_chunk_work(ctx.buffers, "ssm_chunks", chunks, SSM_CHUNKED_FROM, self.heads, self.groups,
                                         self.state_size, self.head_dim)
-            ops.ssm_chunks(*rows, work, chunks=chunks, start=SSM_CHUNKED_FROM, **sizes, **batch)
-        if not chunks or min(ctx.host_query_lens) < SSM_CHUNKED_FROM:
-            ops.ssm_scan(*rows, below=SSM_CHUNKED_FROM if chunks else 0, **sizes, **batch)
+            start = self.chunk_start(ctx.host_query_lens)
+        if start:
+            ops.ssm_chunks(*rows, work, chunks=chunks, start=start, **sizes, **batch)
+        if not start or min(ctx.host_query_lens) < start:
+            ops.ssm_scan(*rows, below=start, **sizes, **batch)
         normed = ctx.buf(f"ssm_normed:{self.inner}", self.inner)
         ops.gated_group_rmsnorm(normed, y, z, p["norm.weight"], self.eps, self.norm_groups)
         out = ctx.buf("mixer_out", self.hidden_size)

@@ -68,3 +68,32 @@ def test_rows_a_tile_of_the_experts_products_holds(experts, H, I, rows):
     assert ops.moe_tile_rows(512 * experts, experts, x.float(), (H, I)) == 16
     assert ops.moe_tile_rows(512 * experts, experts, x, (H, I + 8)) == 16
     assert ops.moe_max_tiles(0, experts, 64) == 0 and ops.moe_tile_rows(0, experts, x, (H, I)) == 16
+
+
+def _mixers():
+    from kvcore_amd.parts.linear_attention import GatedLinearAttention, MaxGatedMatrixMemory
+    from kvcore_amd.parts.recurrent import StateSpaceMixer
+
+    return {
+        "space": StateSpaceMixer(hidden_size=64, heads=64, head_dim=64, state_size=128, groups=8, conv=4, eps=1e-5,
+                                 norm_groups=8),
+        "channel": GatedLinearAttention(hidden_size=64, heads=16, dim=64, vdim=128, tau=8.0, decay_rank=8, eps=1e-5),
+        "wide": GatedLinearAttention(hidden_size=64, heads=16, dim=128, vdim=128, tau=8.0, decay_rank=8, eps=1e-5),
+        "memory": MaxGatedMatrixMemory(hidden_size=64, heads=16, dim=64, vdim=128, gate_cap=15.0, eps=1e-5)}
+
+
+@pytest.mark.parametrize("kind,lengths,cut", [
+    ("space", [199], 0), ("space", [256], 160), ("space", [2048], 160),                 # one request
+    ("space", [192] * 3, 0), ("space", [256] * 3, 160), ("space", [160] * 4, 160),      # until each unit has a block
+    ("space", [256] * 8, 160), ("space", [512] * 12, 0), ("space", [256] * 16, 160), ("space", [256] * 32, 0),
+    ("space", [100, 320], 0), ("space", [100, 384], 160), ("space", [1, 208], 0),       # the scan of the rest follows
+    ("space", [1] * 8 + [192], 160), ("space", [1] * 60 + [160] * 2, 160), ("space", [1] * 64, 0),
+    ("channel", [191], 0), ("channel", [192], 160), ("channel", [160] * 4, 0), ("channel", [160] * 8, 160),
+    ("channel", [100, 256], 0), ("channel", [100, 300], 160), ("channel", [100] * 8 + [180], 0),
+    ("channel", [100] * 8 + [256], 160), ("wide", [152], 0), ("wide", [160], 160),
+    ("memory", [151], 0), ("memory", [152], 128), ("memory", [128] * 4, 0), ("memory", [128] * 6, 128),
+    ("memory", [1] * 30 + [128], 128), ("memory", [127] * 30, 0)])
+def test_which_requests_are_cut_into_chunks(kind, lengths, cut):
+    """By the tokens of the requests, by how far they are ahead of those that stay with the scan, and by how full of
+    scans the chip is: the side that was measured to be the faster."""
+    assert _mixers()[kind].chunk_start(lengths) == cut
