@@ -14,16 +14,21 @@
 // workspace and the last one in the request's slot; every chunk's results.  Products are float32 matrix
 // instructions with float32 operands, and every decay between two tokens is a product of the factors between
 // them (inside a run of 16 tokens one by one, across runs by the runs' own products), never a quotient and never
-// an exponential of a sum, so no decay is too fast for a chunk and a factor of zero is one.  The products are made
-// in 64 bits and rounded once: a product's error is the same for all elements of a state and does not average out
-// as the scan's does (made in 32 bits they left 4e-7 of error where the scan has 2e-7).  Chunks are counted from a request's first token in the step.
+// an exponential of a sum, so no decay is too fast for a chunk and a factor of zero is one.  Inside a chunk the products
+// are made in 64 bits and rounded once, and no sum has more than eight terms in a row (a matrix instruction's four
+// count as one): in 32 bits the decays left 4e-7 of error where the scan has 2e-7, and with the runs' products in 32
+// bits and sums in one chain the results of 64 heads of 128 x 64 had 1.1 to 1.3 times the scan's error (256 tokens 0.90e-7
+// and 0.69e-7; now 0.69e-7; matrix memories of 64 x 129 1.77e-7 and 1.74e-7; now 1.20e-7).  The walk from chunk to
+// chunk rounds to 32 bits, once a chunk where the scan does once a token.  Chunks are counted from a request's first
+// token in the step.
 //
 // The scan walks 2,048 tokens one after the other, some 180 ns each, on as many blocks as there are heads times
-// tiles of values; here a chunk of a head is a block.  2,048 tokens of one request: 16 heads of 64 x 129 405 -> 57 us
-// (sums 16, walk 9, results 32), 64 heads of 128 x 64 in 8 groups 383 -> 127 us (sums 48, walk 24, scores 7, results
-// 48; the states' way to and from the workspace is 67 MB four times).  Loading the state before the chunk ahead of
+// tiles of values; here a chunk of a head is a block.  2,048 tokens of one request: 16 heads of 64 x 129 405 -> 59 us
+// (sums 16, walk 9, results 33), 64 heads of 128 x 64 in 8 groups 376 -> 133 us (sums 49, walk 24, scores 7, results
+// 53; the states' way to and from the workspace is 67 MB four times).  Loading the state before the chunk ahead of
 // the chunk's own keys cost more waves than it hid (results 105 -> 122 us); scores once for the heads that share
-// them brought 105 -> 56.
+// them brought 105 -> 56; two running sums for the state's part of the results, as the chunks' sums have them, instead
+// of sums of eight terms took registers that cost waves (16 heads of 64 x 129 58.6 -> 70.1 us).
 
 #include <hip/hip_runtime.h>
 
@@ -171,6 +176,16 @@ struct Staged {
   }
 };
 
+// Sixteen terms of a product's sums, four of each lane's, in two sums of eight (all of a result's terms in a row would
+// round too often).
+template <typename TA, typename TB>
+__device__ __forceinline__ f32x4_t sixteen_terms(const TA& x, const TB& y) {
+  f32x4_t t[2] = {};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) t[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], t[i & 1], 0, 0, 0);
+  return t[0] + t[1];
+}
+
 // ---- every chunk's own sum.  Wave w takes the key channels 16 (w + 4 m) .., all of the block's columns.
 template <int GATES, int NM, int NC, int VEC>
 __global__ __launch_bounds__(256) void gated_sums_kernel(const GatedArgs a) {
@@ -208,26 +223,27 @@ __global__ __launch_bounds__(256) void gated_sums_kernel(const GatedArgs a) {
   keys.stash(k_s, at, -1);
   values.stash(v_s, at, a.ones ? dvin - c0 : -1);
   __syncthreads();
-  f32x4_t acc[NM][NC];
-#pragma unroll
-  for (int m = 0; m < NM; ++m)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) acc[m][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t acc[NM][NC][2] = {};  // two sums, so that none has all of the terms in a row
   const int steps = (at.n + 15) / 16;
   for (int s = 0; s < steps; ++s) {
+    float ka[NM][4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int j = 16 * s + 4 * lk + i;
       const float w = pw[j];
-      float ka[NM], vb[NC];
 #pragma unroll
-      for (int m = 0; m < NM; ++m) ka[m] = k_s[j * krow + 16 * (wave + 4 * m) + li] * w;
+      for (int m = 0; m < NM; ++m) ka[m][i] = k_s[j * krow + 16 * (wave + 4 * m) + li] * w;
+    }
 #pragma unroll
-      for (int c = 0; c < NC; ++c) vb[c] = v_s[j * kVRow + 16 * c + li];
+    for (int i = 0; i < 4; ++i) {
+      float vb[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) vb[c] = v_s[(16 * s + 4 * lk + i) * kVRow + 16 * c + li];
 #pragma unroll
       for (int m = 0; m < NM; ++m)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[m], vb[c], acc[m][c], 0, 0, 0);
+        for (int c = 0; c < NC; ++c)
+          acc[m][c][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[m][i], vb[c], acc[m][c][i & 1], 0, 0, 0);
     }
   }
   // lane holds column li and key channels 4 lk .. of its tiles: four rows of one column, one 16-byte store
@@ -239,7 +255,7 @@ __global__ __launch_bounds__(256) void gated_sums_kernel(const GatedArgs a) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       const int col = c0 + 16 * c + li;
-      if (col < a.dv) *reinterpret_cast<f32x4_t*>(dst + (static_cast<int64_t>(n >> 2) * a.dv + col) * 4) = acc[m][c];
+      if (col < a.dv) *reinterpret_cast<f32x4_t*>(dst + (static_cast<int64_t>(n >> 2) * a.dv + col) * 4) = acc[m][c][0] + acc[m][c][1];
     }
   }
 }
@@ -381,7 +397,7 @@ __global__ __launch_bounds__(256) void gated_scores_kernel(const GatedArgs a) {
 
 // For token `tid` of a chunk: the factors between it and each later token of its run (`inside`, a row a later token),
 // those from the run's start on (`from_start`) and those behind it (`to_end`).
-__device__ __forceinline__ void run_products(const float* g_s, float* inside, float* from_start, float* to_end, int tid) {
+__device__ __forceinline__ void run_products(const float* g_s, float* inside, double* from_start, double* to_end, int tid) {
   const int run = tid / kRun * kRun, j = tid - run;
   const double first = g_s[run];
   double p = 1.0;
@@ -389,9 +405,9 @@ __device__ __forceinline__ void run_products(const float* g_s, float* inside, fl
   for (int i = 0; i < kRun; ++i) {
     if (i > j) p *= static_cast<double>(g_s[run + i]);
     inside[(run + i) * (kRun + 1) + j] = i >= j ? static_cast<float>(p) : 0.f;
-    if (j == 0) from_start[run + i] = static_cast<float>(first * p);
+    if (j == 0) from_start[run + i] = first * p;
   }
-  to_end[tid] = static_cast<float>(p);
+  to_end[tid] = p;
 }
 
 // ---- every chunk's results.  Wave w takes the queries 16 w .. 16 w + 15 (an operand's columns).  SHARED: the
@@ -419,9 +435,9 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
   float* v_s = lds;                      // [64][kVRow]
   float* g_s = v_s + kChunk * kVRow;     // [64] factors
   float* b_s = g_s + kChunk;             // [64] what a token writes with
-  float* from_start = b_s + kChunk;      // [64] factors from the run's start to the token
-  float* to_end = from_start + kChunk;   // [64] factors behind the token to the run's end
-  float* inside = to_end + kChunk;       // [64][17] factors between a token and each one before it in its run
+  double* from_start = reinterpret_cast<double*>(b_s + kChunk);  // [64] factors from the run's start to the token
+  double* to_end = from_start + kChunk;  // [64] factors behind the token to the run's end
+  float* inside = reinterpret_cast<float*>(to_end + kChunk);  // [64][17] factors between a token and each one before it in its run
   float* k_s = inside + kChunk * (kRun + 1);  // [64][krow], not with SHARED
   const int query = 16 * wave + li;
   const bool live = query < at.n;
@@ -461,9 +477,7 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
         sv[c] = *reinterpret_cast<const f32x4_t*>(st + (static_cast<int64_t>(row) * a.dv + (col < a.dv ? col : c0)) * 4);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) far[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[c][i], qv[s][i], far[c], 0, 0, 0);
+      for (int c = 0; c < NC; ++c) far[c] += sixteen_terms(sv[c], qv[s]);
     }
   }
   // the chunk's own keys up to the query, run by run, the query's own run first
@@ -471,7 +485,7 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
 #pragma unroll
   for (int c = 0; c < NC; ++c) own[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const float* shared = a.scores + ((static_cast<int64_t>(blockIdx.x) * a.nqk + hk) * kChunk + query) * kChunk + 4 * lk;
-  float reach = from_start[query];  // factors from the start of the run after kt to the query
+  double reach = from_start[query];  // factors from the start of the run after kt to the query
   for (int kt = wave; kt >= 0; --kt) {  // scalar
     // lane holds query li, keys 4 lk + i of the run: the operand order of the next product
     f32x4_t score = SHARED ? *reinterpret_cast<const f32x4_t*>(shared + 16 * kt)
@@ -492,24 +506,25 @@ __global__ __launch_bounds__(256) void gated_results_kernel(const GatedArgs a) {
         continue;
       }
     } else {
-      const f32x4_t end = *reinterpret_cast<const f32x4_t*>(to_end + 16 * kt + 4 * lk);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) score[i] = score[i] * reach * (end[i] * b[i]);
+      for (int i = 0; i < 4; ++i) score[i] *= static_cast<float>(reach * to_end[16 * kt + 4 * lk + i]) * b[i];
       reach *= from_start[16 * kt + kRun - 1];
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int c = 0; c < NC; ++c) {
+      float vb[4];
 #pragma unroll
-      for (int c = 0; c < NC; ++c)
-        own[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_s[(16 * kt + 4 * lk + i) * kVRow + 16 * c + li], score[i], own[c], 0, 0, 0);
+      for (int i = 0; i < 4; ++i) vb[i] = v_s[(16 * kt + 4 * lk + i) * kVRow + 16 * c + li];
+      own[c] += sixteen_terms(vb, score);
+    }
   }
   if (!live) return;
   float* o = a.out + static_cast<int64_t>(at.t0 + query) * width + static_cast<int64_t>(h) * a.dv + c0;
   const bool vec_out = (a.dv & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
-  const float skip = GATES == kSpace ? a.skip[h] : 0.f;
+  const float skip = GATES == kSpace ? a.skip[h] : 0.f, all = static_cast<float>(reach);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    f32x4_t y = far[c] * reach + own[c];
+    f32x4_t y = far[c] * all + own[c];
     const int col = 16 * c + 4 * lk;
     if (GATES == kSpace) y += skip * *reinterpret_cast<const f32x4_t*>(v_s + query * kVRow + col);
     if (vec_out) {
@@ -573,16 +588,6 @@ __device__ __forceinline__ double product_behind(double v) {  // of the values b
   v *= row_or_one<0x104>(v);
   v *= row_or_one<0x108>(v);
   return v;
-}
-
-// Sixteen terms of a product's sums, four of each lane's, in two sums of eight (all of a result's terms in a row would
-// round too often).
-template <typename TA, typename TB>
-__device__ __forceinline__ f32x4_t sixteen_terms(const TA& x, const TB& y) {
-  f32x4_t t[2] = {};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) t[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], t[i & 1], 0, 0, 0);
-  return t[0] + t[1];
 }
 
 template <int NS, int NC, int VEC>
@@ -835,7 +840,7 @@ __global__ __launch_bounds__(256) void channel_results_kernel(const GatedArgs a)
 }
 
 size_t gated_lds(int keys, int nc) {
-  return sizeof(float) * (kChunk * (keys + kPad) + kChunk * (16 * nc + kPad) + 4 * kChunk + kChunk * (kRun + 1));
+  return sizeof(float) * (kChunk * (keys + kPad) + kChunk * (16 * nc + kPad) + 6 * kChunk + kChunk * (kRun + 1));
 }
 
 template <typename K>

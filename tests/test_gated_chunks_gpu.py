@@ -135,6 +135,41 @@ def test_scalar_gates_in_chunks(heads, qk_heads, d, dv, ones, start, from_):
     assert chunk_y < 1.25 * scan_y + 2e-8 and chunk_s < 1.25 * scan_s + 2e-8, errors
 
 
+@pytest.mark.parametrize("heads,P,N,groups", [(16, 64, 128, 2), (16, 64, 64, 1), (8, 100, 30, 2)])
+def test_state_space_chunks_round_no_more_than_the_scan(heads, P, N, groups):
+    """Decays and steps as such layers have them; the mean of four draws, whose ratios scatter by some 3%."""
+    from kvcore_amd.ops import library as ops
+
+    T, inner, errors = 256, heads * P, []
+    for seed in range(4):
+        gen = torch.Generator().manual_seed(seed)
+        z = torch.randn(T, inner + 2 * groups * N, generator=gen)
+        xbc, dt = gpu(z * torch.sigmoid(z)), gpu(torch.randn(T, heads, generator=gen))
+        bias = gpu(torch.log(torch.expm1(0.001 * torch.exp(4.6 * torch.rand(heads, generator=gen)))))
+        a_log, skip = gpu(torch.log(1 + 15 * torch.rand(heads, generator=gen))), gpu(torch.ones(heads))
+        step = torch.nn.functional.softplus(dt.double() + bias.double(), threshold=100).cpu()
+        x = xbc[:, :inner].double().cpu().view(T, heads, P)
+        B, C = (xbc[:, inner + i * groups * N: inner + (i + 1) * groups * N].double().cpu().view(T, groups, N)
+                .repeat_interleave(heads // groups, 1) for i in (0, 1))
+        want, _ = walk(C, B, x, torch.exp(-torch.exp(a_log.double().cpu()) * step), step,
+                       torch.zeros(heads, N, P, dtype=torch.float64))
+        want = (want + x).reshape(T, inner)
+        batch, _ = batch_tensors([(0, 0, T)])
+        sizes = dict(heads=heads, head_dim=P, state_size=N, groups=groups)
+        both_ways = []
+        for chunked in (False, True):
+            y, s = torch.empty(T, inner, device=DEV), torch.zeros(1, heads, N, P, device=DEV)
+            if chunked:
+                work, cut = in_chunks([(0, 0, T)], 1, heads, groups, N, P)
+                ops.ssm_chunks(y, xbc, dt, bias, a_log, skip, s, work, **cut, **sizes, **batch)
+            else:
+                ops.ssm_scan(y, xbc, dt, bias, a_log, skip, s, **sizes, **batch)
+            both_ways.append(rel(y, want))
+        errors.append(both_ways)
+    scan, chunks = torch.tensor(errors).mean(0).tolist()
+    assert chunks < 1.08 * scan, errors
+
+
 def test_what_is_not_finite_reaches_no_earlier_token_and_no_other_request():
     gen = torch.Generator().manual_seed(4)
     heads, d, dv = 2, 16, 20
