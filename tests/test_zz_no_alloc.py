@@ -6,6 +6,7 @@ in the static array must not show)."""
 from __future__ import annotations
 
 import ctypes
+import gc
 
 import pytest
 import torch
@@ -67,6 +68,7 @@ def test_static_argmax_two_calls_in_a_row(lib):
     warm = torch.full((5,), -7, dtype=torch.int32, device=DEV)
     assert _static(lib, small, warm) == 0, lib.kvc_last_error()
     torch.cuda.synchronize()
+    gc.collect()  # tensors in reference cycles that earlier tests left must not go between the two readings
     # torch's counters see its own allocator only; the device's free memory sees every
     # hipMalloc of the process, the library's included
     before = torch.cuda.memory_allocated(), torch.cuda.memory_reserved(), torch.cuda.mem_get_info()[0]
