@@ -71,9 +71,6 @@ struct GatedArgs {
   const float* skip;
   float* work;        // [chunks][nh][dpad / 4][dv][4], then the chunks' whole decays [chunks][nh]
   float* decays;      // kChannel: [chunks][nh][dpad]
-  float* solved_k;    // the delta rule's: [T][nh * d], [T][nh * dv], [T][nh]
-  float* solved_v;
-  float* ends;
   float* scores;      // [chunks][nqk][64 queries][64 keys]: k . q of the heads that share both (else unused)
   float* state;       // [slots][nh][dpad / 4][dv][4]; kSpace: [slots][nh][d][dv]
   const int32_t* positions;

@@ -27,7 +27,10 @@
 //                    pair's input (the sums, before any activation).
 //                    bfloat16 operands go through the matrix cores (16 x 16 x 32, the expert's rows as
 //                    the A operand, the tokens as B) with float32 sums; float32 operands, and rows
-//                    that 16-byte loads do not divide, are summed in float32 in index order.  A row's sums do not depend on which tile it is in.
+//                    that 16-byte loads do not divide, are summed in float32 in index order.  A row's sums do
+//                    not depend on its place in a tile or on the rows beside it.  In bfloat16 their order is that of
+//                    the kernel which the step's size chose (four shares of K added up, or one chain that starts at
+//                    a place its expert and columns decide); in float32 it is the same in every step.
 //   kvc_moe_combine  out[t] = sum_c weight[t, c] * y[t * top + c] (without weights: the plain sum) (+ up to two more row sets, the second
 //                    times a number a token where one is given), float32, in the order of the
 //                    choices; or added into out (the residual stream).
