@@ -1098,33 +1098,39 @@ extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
 }
 
 // How many rows a tile holds, for experts of matrices [I, H] ([2 I, H] if gated) and [H, I], by an estimate of both
-// products in us (routing taken as even).  Tiles of 16: every expert's matrices once at 5.6 TB/s, and again for each
-// further tile, of which there are some from 6 rows an expert on.  Tiles of 64: one fetch, but columns of 128 (ungated
-// 256) a block, so a step is no faster than a block's walk along K (0.8 us a pass of 64), and blocks that
-// come out uneven on the units wait for the last.  Both products of even routing, tiles of 16 / 64:
-//   32 experts of 2048 x 2048    8 rows an expert  136 / 139 us,   12  146 / 141,   64  444 / 188
-//   8 experts of 512 x 512      16 rows             14 /  21 us,   48   15 /  26,   64   22 /  25
-//   4 experts of 1024 x 2048     8 rows             16 /  38 us,   48   33 /  48
-//   128 experts of 1024 x 384    6 rows             56 /  63 us,   16   77 /  68
-// Tiles of 128 where experts have that many rows and the blocks still fill the chip (300 in either product if they held
+// products in us, for tokens that choose their experts at random.  Tiles of 16: the matrices of the experts that are
+// chosen at 6.6 TB/s, and again for each further tile, of which there are some from 4.5 rows an expert on.  Tiles of 64:
+// one fetch, at 6.1 TB/s gated and 7.2 otherwise, but columns of 128 (ungated 256) a block, so a product is no faster than
+// a block's walk along K (1.05 us a pass of 64), and blocks that come out uneven on the units wait for the last.  Both
+// products, tiles of 16 / 64, by rows an expert, gated:
+//   32 experts of 2048 x 2048     1   90 / 101 us    4  141 / 139    8  146 / 139   16  177 / 145
+//   16 experts of 1024 x 1024     4   21 /  27       8   21 /  27   16   27 /  30   32   39 /  34
+//   4 experts of 1024 x 2048      8   15 /  36      32   20 /  38   64   33 /  46
+//   128 experts of 1024 x 384     4   52 /  60      12   63 /  65   16   74 /  68
+// and not gated:
+//   32 experts of 2048 x 2048     1   54 /  62       4   97 /  90    8  100 /  91
+//   16 experts of 2048 x 2048     8   45 /  56      12   52 /  57   24   87 /  61
+// Over 428 such steps of fourteen sizes, gated and not, the tiles it takes are 1.001 x the faster in the mean and 1.09 x
+// at most.  Tiles of 128 where experts have that many rows and the blocks still fill the chip (300 in either product if they held
 // 64 rows: the second of two blocks a unit keeps the matrix cores busy): 32 experts of 2048 x 2048, 64 rows each,
 // 188 / 165 us, 16 experts of 1024 x 1024 41 / 53.  From 104 to 150 rows many an expert has a few more than 128, and two
 // tiles of half the size cost more than smaller ones: 128 rows 227 us in tiles of 64, 249 in tiles of 128.
 extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
   if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0) return kTileRows;
   const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
-  const double used = pairs < E ? pairs : E;  // experts with rows
+  const double used = E * -expm1(-each);  // experts with rows
   const int first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, down_cols = (H + 255) / 256;
   const double down_mb = 2e-6 * H * I, first_mb = gated ? 2 * down_mb : down_mb;
-  const double again = each > 6 ? (each - 6) / 16 * E : 0;
-  const double few = 8 + (first_mb + down_mb) * (used / 5.6 + again / 6);
+  const double again = each > 4.5 ? (each - 4.5) / 16 * E : 0;
+  const double few = 10 + (first_mb + down_mb) * (used / 6.6 + again / 6.5);
   const double mid_tiles = used + (each > 32 ? (each - 32) / 64 * E : 0);
-  auto product = [&](double mb, int k, int cols) {
+  auto product = [&](double mb, double rate, int k, int cols) {
     const double a_unit = mid_tiles * cols / units;
     const double uneven = a_unit > 1 ? ceil(a_unit) / a_unit : 1;
-    return 4 + fmax(0.8 * k / 64, used * mb / 5.6 * uneven);
+    return 5 + fmax(1.05 * k / 64, used * mb / rate * uneven);
   };
-  if (each <= 64 && few <= product(first_mb, H, first_cols) + product(down_mb, I, down_cols)) return kTileRows;
+  const double mid = product(first_mb, gated ? 6.1 : 7.2, H, first_cols) + product(down_mb, 7.2, I, down_cols);
+  if (each <= 64 && few <= mid) return kTileRows;
   const double blocks = (pairs / 64.0 + E / 2.0) * (first_cols < down_cols ? first_cols : down_cols);
   return blocks >= 300 && (each >= 150 || (each >= 40 && each < 104)) ? kBigTileRows : kMidTileRows;
 }

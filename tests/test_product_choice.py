@@ -56,7 +56,7 @@ def test_decode_graph_sizes(limit):
     (4, 256, 320, {4: 16, 48: 16, 256: 64}),
     (128, 1024, 384, {3: 16, 6: 16, 16: 64, 64: 128, 128: 64}),
     (64, 4096, 1408, {2: 16, 8: 64, 32: 64, 96: 128}),
-    (16, 512, 2048, {4: 16, 8: 16, 32: 64, 192: 64})])
+    (16, 512, 2048, {4: 16, 8: 16, 32: 16, 48: 64, 192: 64})])  # 32 rows: 40 us in tiles of 16, 44 of 64
 def test_rows_a_tile_of_the_experts_products_holds(experts, H, I, rows):
     """Experts of small matrices keep tiles of 16 until their rows fill larger ones, and none gets tiles of 128 whose
     blocks would leave the chip idle: within a few percent of the fastest measured of the three."""
@@ -68,6 +68,21 @@ def test_rows_a_tile_of_the_experts_products_holds(experts, H, I, rows):
     assert ops.moe_tile_rows(512 * experts, experts, x.float(), (H, I)) == 16
     assert ops.moe_tile_rows(512 * experts, experts, x, (H, I + 8)) == 16
     assert ops.moe_max_tiles(0, experts, 64) == 0 and ops.moe_tile_rows(0, experts, x, (H, I)) == 16
+
+
+def test_rows_a_tile_of_few_rows_and_without_a_gate():
+    """No step of as many pairs as experts or fewer leaves tiles of 16, whose estimate and that of larger tiles lie close
+    there; without a gate a product has half the columns of weights a block, and larger tiles pay from fewer rows on."""
+    from kvcore_amd.ops import library as ops
+
+    x = torch.empty(1, 8, dtype=torch.bfloat16)
+    for E, H, I in ((128, 2048, 768), (64, 2048, 1408), (64, 4096, 1408), (32, 2048, 2048), (8, 4096, 4096), (4, 256, 320)):
+        for gated in (True, False):
+            assert {ops.moe_tile_rows(p, E, x, (H, I), gated) for p in range(1, E + 1)} == {16}, (E, H, I, gated)
+    for (E, H, I), rows in {(32, 2048, 2048): {1: 16, 4: 64, 6: 64, 16: 64}, (128, 2048, 768): {2: 16, 6: 64, 8: 64},
+                            (64, 4096, 1408): {2: 16, 8: 64}, (16, 2048, 2048): {8: 16, 12: 16, 24: 64}}.items():
+        for each, tile in rows.items():
+            assert ops.moe_tile_rows(each * E, E, x, (H, I), False) == tile, (E, H, I, each)
 
 
 def _mixers():
