@@ -25,6 +25,8 @@ run in the model dtype with float32 sums.
 
 from __future__ import annotations
 
+import math
+
 import torch
 
 from kvcore_amd.ops import library as ops
@@ -182,22 +184,47 @@ class StateSpaceMixer(Mixer):
             raise ValueError(f"a state of {self.state_size} rows a head: the recurrence kernel serves {most}")
 
     def chunk_start(self, lengths) -> int:
-        """From how many tokens on a step's requests are cut into chunks (0: none are).
+        """From how many tokens on a step's requests are cut into chunks (0: none are): there if the chunks and the scan
+        of the shorter requests behind them are estimated to take less time than the scan of all.
 
-        The scan takes as long as its longest request, on as many blocks as there are requests times heads times
-        tiles of 64 columns.  Below a block a compute unit it has 0.2 us a token and its fixed cost is less; from there
-        on 0.55 us; three blocks a unit fill the chip, and then it is the faster by a tenth, but for a fourth, which
-        starts another round.  Scan and chunks, 64 heads of 128 x 64 in 8 groups, us: one request of 192 tokens
-        39 and 40, 256 tokens 51 and 42, 2,048 tokens 376 and 125; four of 192 tokens 108 and 65, eight of 256 tokens
-        150 and 129, twelve of 512 tokens 351 and 384, sixteen of 256 tokens 288 and 258, 32 of 256 tokens 474 and 519;
-        one of 320 tokens beside one of 100 tokens 72 and 75, one of 256 beside eight of single tokens 142 and 53."""
-        units = ops.compute_units()
-        blocks = self.heads * -(-self.head_dim // 64)
-        full = blocks * sum(n >= SSM_CHUNKED_FROM for n in lengths) / units
-        if full >= 3 and not (self.state_size > 64 and 4 <= full < 5):
+        Both are fitted to 740 steps of 27 sizes (2 to 128 heads, states of 8 to 128 rows by 16 to 128 columns): the
+        side taken is 1.008 x the faster in the mean, more than a tenth behind it in 22 of them and at most 1.32 x.  Scan and chunks,
+        us, 64 heads of 128 x 64 in 8 groups: one request of 192 tokens 38 and 43, 256 tokens 50 and 46, 2,048 tokens
+        379 and 133; four of 200 tokens 113 and 76, eight of 256 tokens 153 and 135, twelve of 512 tokens 351 and 384,
+        32 of 256 tokens 480 and 553; one of 256 beside eight of single tokens 142 and 53.  80 heads of 64 x 32: one of
+        256 tokens 40 and 32, four of 200 tokens 40 and 61, eight of 160 tokens 47 and 72."""
+        long = [n for n in lengths if n >= SSM_CHUNKED_FROM]
+        if not long:
             return 0
-        share = blocks * len(lengths) / units
-        return ops.gated_chunk_start(lengths, SSM_CHUNKED_FROM, 176 + 96 * share if share < 1 else 88)
+        if self.head_dim < 16:  # the scan's general kernel: 0.4 to 1.3 us a token
+            return SSM_CHUNKED_FROM
+        rest = [n for n in lengths if n < SSM_CHUNKED_FROM]
+        return SSM_CHUNKED_FROM if self._chunks_us(long) + self._scan_us(rest) < self._scan_us(lengths) else 0
+
+    def _scan_us(self, lengths) -> float:
+        """The scan: the chain of its longest request's tokens or the work of all, whichever is more; tiles of 16 columns
+        with shorter steps where tiles of 64 would leave units idle.  A block more than the three that a unit of large
+        states holds starts another round, and single tokens' states come and go beside a long request's."""
+        if not lengths:
+            return 0.0
+        units, state, longest = ops.compute_units(), self.state_size / 128, max(lengths)
+        blocks = len(lengths) * self.heads * -(-self.head_dim // 64) / units
+        work = sum(lengths) * self.heads * self.head_dim / 64 / units
+        if self.head_dim < 64 or blocks < 1:
+            chain, work = longest * (0.115 + 0.056 * state), work * (0.102 + 0.158 * state)
+        else:
+            chain, work = longest * (0.154 + 0.264 * state), work * (0.022 + 0.121 * state)
+            if 4 <= blocks < 5 and self.state_size > 64:
+                work *= 1.8
+        singles = sum(n <= 16 for n in lengths) if longest > 16 else 0
+        return 5 + math.hypot(chain, work) + 0.52e-6 * singles * 8 * self.heads * self.state_size * self.head_dim
+
+    def _chunks_us(self, lengths) -> float:
+        """The chunks: their four launches and a block's own way, then every block's work."""
+        state = self.state_size / 128
+        chunks = ops.gated_chunk_count(lengths, SSM_CHUNKED_FROM)
+        work = self.heads * (3 + 9 * state * -(-self.head_dim // 16) / 4) + 1.4 * self.groups * state
+        return 21.3 + 13.2 * state + chunks * work / ops.compute_units()
 
     def forward(self, x, ctx, call, sink=None):
         p = self.params

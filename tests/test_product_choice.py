@@ -92,6 +92,8 @@ def _mixers():
     return {
         "space": StateSpaceMixer(hidden_size=64, heads=64, head_dim=64, state_size=128, groups=8, conv=4, eps=1e-5,
                                  norm_groups=8),
+        "narrow": StateSpaceMixer(hidden_size=64, heads=80, head_dim=32, state_size=64, groups=1, conv=4, eps=1e-5,
+                                  norm_groups=1),
         "channel": GatedLinearAttention(hidden_size=64, heads=16, dim=64, vdim=128, tau=8.0, decay_rank=8, eps=1e-5),
         "wide": GatedLinearAttention(hidden_size=64, heads=16, dim=128, vdim=128, tau=8.0, decay_rank=8, eps=1e-5),
         "memory": MaxGatedMatrixMemory(hidden_size=64, heads=16, dim=64, vdim=128, gate_cap=15.0, eps=1e-5)}
@@ -103,6 +105,9 @@ def _mixers():
     ("space", [256] * 8, 160), ("space", [512] * 12, 0), ("space", [256] * 16, 160), ("space", [256] * 32, 0),
     ("space", [100, 320], 0), ("space", [100, 384], 160), ("space", [1, 208], 0),       # the scan of the rest follows
     ("space", [1] * 8 + [192], 160), ("space", [1] * 60 + [160] * 2, 160), ("space", [1] * 64, 0),
+    # heads of fewer columns than a tile of the scan: chunks cost as much a head, the scan less
+    ("narrow", [160], 0), ("narrow", [256], 160), ("narrow", [200] * 4, 0), ("narrow", [160] * 8, 0), ("narrow", [256] * 8, 0),
+    ("narrow", [2048] * 2, 160), ("narrow", [1] * 8 + [160], 0),
     ("channel", [191], 0), ("channel", [192], 160), ("channel", [160] * 4, 0), ("channel", [160] * 8, 160),
     ("channel", [100, 256], 0), ("channel", [100, 300], 160), ("channel", [100] * 8 + [180], 0),
     ("channel", [100] * 8 + [256], 160), ("wide", [152], 0), ("wide", [160], 160),
