@@ -1,19 +1,16 @@
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias) in true float32: float32 products, float32 sums (the matrix
-// instructions whose operands are float32), no mode of reduced precision.
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias) in float32, its products on the bfloat16 matrix instructions: an operand is
+// the sum of three bfloat16 values, and the six products of parts that float32 can tell are added up in float32.  That
+// is no mode of reduced precision: over 1 to 2,048 rows and K of 64 to 8,192 the error against 64 bits is 0.43 to 0.89 of
+// what the float32 matrix instructions leave (122 rows of 16384 x 2048: 2.4e-7 and 2.9e-7 of the result, of 2048 x 8192
+// 5.1e-7 and 5.7e-7), and a chunk of 32 values takes 96 cycles of a matrix core, not 256.
 //
 // Every element of C is made in one way, whatever M, its tile or its row's place in the batch: K is cut into
-// chunks of 32; wave w of a block's eight adds up the chunks w, w + 8, ... in order (a chunk is eight
-// 16 x 16 x 4 instructions, of which number j takes the values k + j, k + 8 + j, k + 16 + j, k + 24 + j); the
-// eight sums are added in wave order, then the bias.  So the tile may follow the sizes of a call and the bits
-// do not.
+// chunks of 32; eight chains take the chunks w, w + 8, ... in order (a chunk is six 16 x 16 x 32 instructions); the
+// eight sums are added in order, then the bias.  So the tile may follow the sizes of a call and the bits do not.
 //
-// A block takes NT x MT tiles of 16 columns x 16 rows of C and all its waves take all of them, each its part
-// of K: the operands go from memory to registers (a lane 32 contiguous bytes, the four lanes of a row 128), a
-// fetched weight meets 16 MT rows and a fetched row 16 NT columns.  Bound by the float32 matrix rate
-// (157 TFLOP/s) from some 30 rows on and by reading W below that.  Against a tile of 64 x 64 through LDS whose
-// threads multiplied and added: 122 rows of 16384 x 2048 262 -> 118 us (70 TFLOP/s), of 2048 x 8192 875 -> 62;
-// 2,048 rows of 16384 x 2048 3.64 -> 1.68 ms (82 TFLOP/s); one row of 16384 x 2048 196 -> 33 us (4.0 TB/s).  It was
-// the faster only for hundreds of rows whose K is short and no multiple of 8 (300 rows of 8192 x 100 17 and 23 us).
+// Few rows: a block takes NT x MT tiles of 16 columns x 16 rows of C and all its waves take all of them, each a chain
+// of K: the operands go from memory to registers (the four lanes of a row read 64 contiguous bytes at a time).  Bound by
+// reading W (one row of 16384 x 2048 31 us, 4.4 TB/s).  More than 32 rows: gemm_f32_shared_kernel.
 
 #include <hip/hip_runtime.h>
 
@@ -28,27 +25,111 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kChunk = 32;
 
-// Eight values of a row from k on, loaded in pieces of PIECE (8: two of four): K a multiple of PIECE and the rows
-// aligned to it (16 bytes at most), so a piece is in or out as a whole; `whole` (the same for the wave): the chunk
-// lies inside K.
+// Read by lanes whose values lie beyond K: an address, so that no select stands between a load and its use (one that
+// does makes the compiler wait for every load in flight).
+__device__ f32x4_t kNothing[2];
+
+// A lane's eight values of a chunk, four from k = 4 lk on and four from k + 16 on, so that the four lanes of a row read
+// 64 contiguous bytes at a time; loaded in pieces of PIECE (8: two of four): K a multiple of PIECE and the rows aligned to
+// it (16 bytes at most), so a piece is in or out as a whole; `whole` (the same for the wave): the chunk lies inside K.
 template <int PIECE>
 __device__ __forceinline__ void load8(f32x4_t* v, const float* row, int k, int K, bool whole) {
   if constexpr (PIECE == 8) {
-    const float* p = row + (k < K ? k : 0);
-    v[0] = *reinterpret_cast<const f32x4_t*>(p);
-    v[1] = *reinterpret_cast<const f32x4_t*>(p + 4);
-    if (!whole && k >= K) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    v[0] = *(k < K ? reinterpret_cast<const f32x4_t*>(row + k) : kNothing);
+    v[1] = *(k + 16 < K ? reinterpret_cast<const f32x4_t*>(row + k + 16) : kNothing);
   } else if constexpr (PIECE == 2) {  // for many tiles: with a piece a value 300 rows of 8192 x 100 take 27.5 us, 22.7 so
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
-      const float2 x = *reinterpret_cast<const float2*>(row + (k + i < K ? k + i : 0));
-      v[i >> 2][i & 3] = whole || k + i < K ? x.x : 0.f;
-      v[i >> 2][(i & 3) + 1] = whole || k + i < K ? x.y : 0.f;
+      const int at = k + i + (i < 4 ? 0 : 12);
+      const float2 x = *reinterpret_cast<const float2*>(row + (at < K ? at : 0));
+      v[i >> 2][i & 3] = whole || at < K ? x.x : 0.f;
+      v[i >> 2][(i & 3) + 1] = whole || at < K ? x.y : 0.f;
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i >> 2][i & 3] = k + i < K ? row[k + i] : 0.f;
+    for (int i = 0; i < 8; ++i) {
+      const int at = k + i + (i < 4 ? 0 : 12);
+      v[i >> 2][i & 3] = at < K ? row[at] : 0.f;
+    }
   }
+}
+
+// Eight float32 values as sums of three bfloat16 values, rounded to nearest one after the other: 24 significand bits
+// in three times eight, so nothing is left over (down to 2^-133, the least that bfloat16 holds).
+struct split_t {
+  bf16x8_t part[3];
+};
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ split_t split8(const f32x4_t* v) {
+  u32x4_t out[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // two values at a time: one conversion makes both halves of a register
+    f32x2_t x = {v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
+      out[p][i] = bits;
+      if (p < 2) {
+        x[0] -= __uint_as_float(bits << 16);
+        x[1] -= __uint_as_float(bits & 0xffff0000u);
+      }
+    }
+  }
+  split_t s;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) s.part[p] = __builtin_bit_cast(bf16x8_t, out[p]);
+  return s;
+}
+
+// acc += the sums over a chunk of w x a, the smallest of the six products that float32 can tell first (what is left
+// out is below 2^-26 of a product).
+constexpr int kOrder[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+template <int NT, int MT>
+__device__ __forceinline__ void multiply(f32x4_t (&acc)[NT][MT], const split_t* w, const split_t* a) {
+#pragma unroll
+  for (int p = 0; p < 6; ++p)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n].part[kOrder[p][0]], a[m].part[kOrder[p][1]], acc[n][m], 0, 0, 0);
+}
+
+// Four sums that lie side by side in C, as they leave.  A value beyond float32, an infinity or a NaN among the operands
+// leaves a sum that is not finite, and operands below 2^-110 lose what bfloat16 cannot hold (what is below 2^-134), of
+// which sums below 2^-90 could tell: such an element is summed again, in index order with fused multiply-adds.  A sum of
+// zero stays, so that rows and weights of zeros cost nothing.
+__device__ __forceinline__ void leave(f32x4_t v, float* __restrict__ C, const float* __restrict__ A,
+                                      const float* __restrict__ W, const float* __restrict__ bias, int row, int col, int N,
+                                      int K, int64_t lda, int64_t ldc) {
+  // 0 x each: a NaN unless all are finite
+  const float none = fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f)));
+  const float least = fminf(fminf(fabsf(v[0]), fabsf(v[1])), fminf(fabsf(v[2]), fabsf(v[3])));
+  if (none != none || least < 0x1p-90f) {
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      float x = v[0];  // by hand: a register is not indexed
+      x = i == 1 ? v[1] : i == 2 ? v[2] : i == 3 ? v[3] : x;
+      if (col + i < N && (!(fabsf(x) < INFINITY) || (x != 0.f && fabsf(x) < 0x1p-90f))) {
+        const float* a = A + static_cast<int64_t>(row) * lda;
+        const float* w = W + static_cast<int64_t>(col + i) * K;
+        x = 0.f;
+#pragma unroll 1
+        for (int k = 0; k < K; ++k) x = fmaf(a[k], w[k], x);
+      }
+      v[0] = i == 0 ? x : v[0];
+      v[1] = i == 1 ? x : v[1];
+      v[2] = i == 2 ? x : v[2];
+      v[3] = i == 3 ? x : v[3];
+    }
+  }
+  if (bias != nullptr) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += bias[col + i < N ? col + i : N - 1];
+  }
+  store4<float>(C + static_cast<int64_t>(row) * ldc + col, v, N - col);
 }
 
 template <int NT, int MT, int AHEAD, int PIECE>
@@ -74,9 +155,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict
     for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int chunks = (K + kChunk - 1) / kChunk;
   f32x4_t wv[AHEAD][NT][2], av[AHEAD][MT][2];
-  // no branch around the loads: a chunk that is not there is one that reads zeros
-  auto fetch = [&](int slot, int c) {
-    const int k = c * kChunk + 8 * lk;
+  auto fetch = [&](int slot, int c) {  // a chunk that is not there is one that reads zeros
+    const int k = c * kChunk + 4 * lk;
     const bool whole = (c + 1) * kChunk <= K;
 #pragma unroll
     for (int n = 0; n < NT; ++n) load8<PIECE>(wv[slot][n], wp[n], k, K, whole);
@@ -84,23 +164,24 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict
     for (int m = 0; m < MT; ++m) load8<PIECE>(av[slot][m], ap[m], k, K, whole);
   };
 #pragma unroll
-  for (int s = 0; s < AHEAD; ++s) fetch(s, wave + kWaves * s);
-  for (int c = wave; c < chunks; c += kWaves * AHEAD) {  // scalar
+  for (int s = 0; s < AHEAD; ++s) {
+    fetch(s, wave + kWaves * s);
+    __builtin_amdgcn_sched_barrier(0);  // in the order of their use, which the waits count on
+  }
+  for (int c = wave; c < chunks; c += kWaves * AHEAD) {  // scalar; no branch inside, which would drain the loads
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s) {
-      f32x4_t w[NT][2], a[MT][2];
+      split_t w[NT], a[MT];
 #pragma unroll
-      for (int n = 0; n < NT; ++n) w[n][0] = wv[s][n][0], w[n][1] = wv[s][n][1];
+      for (int n = 0; n < NT; ++n) w[n] = split8(wv[s][n]);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) a[m][0] = av[s][m][0], a[m][1] = av[s][m][1];
+      for (int m = 0; m < MT; ++m) a[m] = split8(av[s][m]);
+      // the loads leave after the registers that they fill have been read (or they would fill others and be copied,
+      // which waits for them) and before the products
+      __builtin_amdgcn_sched_barrier(0);
       fetch(s, c + kWaves * (s + AHEAD));
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-          for (int m = 0; m < MT; ++m)
-            acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n][j >> 2][j & 3], a[m][j >> 2][j & 3], acc[n][m], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply<NT, MT>(acc, w, a);
     }
   }
   // the waves' sums, 16 columns at a time: lane holds row li, columns 4 lk .. of its tiles
@@ -116,12 +197,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict
 #pragma unroll
       for (int w = 1; w < kWaves; ++w) v += part[w][m][l];
       const int row = m0 + 16 * m + (l & 15), col = n0 + 16 * n + 4 * (l >> 4);
-      if (row >= M || col >= N) continue;
-      if (bias != nullptr) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += bias[col + i < N ? col + i : N - 1];
-      }
-      store4<float>(C + static_cast<int64_t>(row) * ldc + col, v, N - col);
+      if (row < M && col < N) leave(v, C, A, W, bias, row, col, N, K, lda, ldc);
     }
   }
 }
@@ -151,7 +227,7 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
 #pragma unroll
     for (int m = 0; m < MT; ++m) sum[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   auto fetch = [&](int c) {  // a chunk that is not there is one that reads zeros
-    const int k = c * kChunk + 8 * lk;
+    const int k = c * kChunk + 4 * lk;
     const bool whole = (c + 1) * kChunk <= K;
 #pragma unroll
     for (int n = 0; n < NT; ++n) load8<PIECE>(wv[n], wp[n], k, K, whole);
@@ -160,23 +236,22 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
   };
   fetch(0);
   for (int c = 0; c * kChunk < K; ++c) {  // scalar
-    f32x4_t w[NT][2], a[MT][2], acc[NT][MT];
+    split_t w[NT], a[MT];
+    f32x4_t acc[NT][MT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) w[n][0] = wv[n][0], w[n][1] = wv[n][1];
+    for (int n = 0; n < NT; ++n) w[n] = split8(wv[n]);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) a[m][0] = av[m][0], a[m][1] = av[m][1];
+    for (int m = 0; m < MT; ++m) {
+      a[m] = split8(av[m]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     fetch(c + 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[n][j >> 2][j & 3], a[m][j >> 2][j & 3], acc[n][m], 0, 0, 0);
+    multiply<NT, MT>(acc, w, a);
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -190,22 +265,196 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const int col = n0 + 16 * n + 4 * lk;
-      if (col >= N) continue;
-      f32x4_t v = sum[n][m];
-      if (bias != nullptr) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] += bias[col + i < N ? col + i : N - 1];
-      }
-      store4<float>(C + static_cast<int64_t>(row) * ldc + col, v, N - col);
+      if (col < N) leave(sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
     }
   }
 }
 
+// The same for more rows than a wave's registers take at a time: the waves of a block take 16 NT columns each of 16 MT
+// rows, whose chunk along K goes through LDS, split by the threads that fetch it and laid out as the matrix
+// instructions want it (a wave's load is one contiguous kilobyte); a wave splits the weights of its own columns in
+// registers.  The eight chains of K are walked one after the other, each from zero, and added in order, or (where C
+// has too few tiles for the chip) dealt out to gridDim.z blocks, which leave every chain's sums in `parts`
+// [chain][M][round4(N)] for gemm_f32_parts_kernel.  The bits are those of the kernels above.
+//
+// Bound by the matrix and the vector instructions of a wave together (a step of 4 x 2 tiles is 48 matrix instructions of
+// 16 cycles beside the split of 24 values a lane, 5.5 instructions each; with every operand hot in the cache the kernel is
+// 5 to 10% faster, no more).  With the float32 matrix instructions on operands straight from the cache and now: 122 rows of
+// 16384 x 2048 115 and 64 us (128 TFLOP/s), of 2048 x 8192 62 and 39, of 3072 x 2048 35 and 24, of 2048 x 2048 18.9 and 16.9;
+// 1,000 rows of 2048 x 2048 110 and 58, 2,048 rows of 16384 x 2048 1,668 and 824 (167 TFLOP/s).  Tiles of 128 rows and one
+// column block a wave read LDS twice as often: 74, 38, 24, 18, 68 and 860 us.
+template <int MT, int NT, bool LEAVE>
+__global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
+    float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
+    float* __restrict__ parts, int M, int N, int K, int64_t lda, int64_t ldc) {
+  constexpr int UN = MT / 4;  // pieces of 16 rows that a wave brings
+  __shared__ u32x4_t rows_s[2][MT][3][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int n0 = (blockIdx.x * 4 + wave) * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int chunks = K / kChunk;
+  const int per = kWaves / gridDim.z;
+  const int first = blockIdx.z * per, last = first + per;  // this block's chains
+  // columns and rows beyond the matrix read its last ones and are not stored
+  const float* wp[NT];
+  const float* ap[UN];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+    wp[n] = W + static_cast<int64_t>(n0 + 16 * n + li < N ? n0 + 16 * n + li : N - 1) * K + 4 * lk;
+#pragma unroll
+  for (int u = 0; u < UN; ++u) {
+    const int row = m0 + 16 * (wave + 4 * u) + li;
+    ap[u] = A + static_cast<int64_t>(row < M ? row : M - 1) * lda + 4 * lk;
+  }
+  f32x4_t wv[2][NT][2], av[2][UN][2];
+  split_t ws[2][NT];
+  auto fetch = [&](int slot, int c) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) av[slot][u][i] = *reinterpret_cast<const f32x4_t*>(ap[u] + c * kChunk + 16 * i);
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) wv[slot][n][i] = *reinterpret_cast<const f32x4_t*>(wp[n] + c * kChunk + 16 * i);
+  };
+  auto stash = [&](int slot) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const split_t s = split8(av[slot][u]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) rows_s[slot][wave + 4 * u][p][lane] = __builtin_bit_cast(u32x4_t, s.part[p]);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) ws[slot][n] = split8(wv[slot][n]);
+  };
+  // the chunk after c: the next of its chain, or the first of the next chain, or (at the end) any
+  auto after = [&](int c) {
+    const int next = (c & (kWaves - 1)) + 1;
+    return c + kWaves < chunks ? c + kWaves : next < last ? next : first;
+  };
+  f32x4_t acc[NT][MT], sum[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = sum[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int ahead = first;  // the chunk to be fetched next
+  fetch(0, ahead);
+  __builtin_amdgcn_sched_barrier(0);  // in the order of their use, which the waits count on
+  ahead = after(ahead);
+  fetch(1, ahead);
+  __builtin_amdgcn_sched_barrier(0);
+  stash(0);
+  ahead = after(ahead);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(0, ahead);
+  for (int chain = first; chain < last; ++chain) {
+    for (int c = chain; c < chunks; c += 2 * kWaves) {  // scalar; no branch inside, which would drain the loads
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        __syncthreads();  // this chunk's rows are in LDS buffer s, the other buffer has been read by all
+        split_t a[MT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+#pragma unroll
+          for (int p = 0; p < 3; ++p) a[m].part[p] = __builtin_bit_cast(bf16x8_t, rows_s[s][m][p][lane]);
+        }
+#pragma unroll
+        for (int g = 0; g < MT / 2; ++g)
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+              for (int i = 0; i < 2; ++i)
+                acc[n][2 * g + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[s][n].part[kOrder[p][0]], a[2 * g + i].part[kOrder[p][1]],
+                                                                            acc[n][2 * g + i], 0, 0, 0);
+        stash(s ^ 1);
+        ahead = after(ahead);
+        // after the registers that they fill have been read, or they would fill others and be copied, which waits for them
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(s ^ 1, ahead);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        if constexpr (LEAVE) {
+          const int row = m0 + 16 * m + li, col = n0 + 16 * n + 4 * lk, wide = (N + 3) & ~3;
+          if (row < M && col < N)
+            *reinterpret_cast<f32x4_t*>(parts + (static_cast<int64_t>(chain) * M + row) * wide + col) = acc[n][m];
+        } else {
+          sum[n][m] = chain == first ? acc[n][m] : sum[n][m] + acc[n][m];
+        }
+        acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  if constexpr (LEAVE) return;
+  // lane holds row li, columns 4 lk .. of its tiles
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int row = m0 + 16 * m + li;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const int col = n0 + 16 * n + 4 * lk;
+      if (row < M && col < N) leave(sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
+    }
+  }
+}
+
+// Adds up what the blocks above left: a thread four columns.
+__global__ __launch_bounds__(256) void gemm_f32_parts_kernel(float* __restrict__ C, const float* __restrict__ A,
+                                                             const float* __restrict__ W, const float* __restrict__ bias,
+                                                             const float* __restrict__ parts, int chains, int M, int N, int K,
+                                                             int64_t lda, int64_t ldc) {
+  const int quads = (N + 3) >> 2;
+  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (idx >= static_cast<int64_t>(M) * quads) return;
+  const int row = static_cast<int>(idx / quads), col = 4 * static_cast<int>(idx - static_cast<int64_t>(row) * quads);
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(parts) + idx;
+  const int64_t step = static_cast<int64_t>(M) * quads;
+  f32x4_t v[kWaves];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) v[w] = p[(w < chains ? w : 0) * step];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w)
+    if (w < chains) v[0] += v[w];  // scalar
+  leave(v[0], C, A, W, bias, row, col, N, K, lda, ldc);
+}
+
+// How the sizes of a call are dealt out to the kernel with rows in LDS: column blocks of 16 a wave, chains to how many
+// blocks; nt 0: not at all.
+constexpr int kSharedRows = 4;  // row blocks of 16 a block
+struct SharedShape {
+  int nt, groups;
+};
+SharedShape shared_shape(int M, int N, int K) {
+  if (M <= 32 || K % (2 * kWaves * kChunk)) return {0, 0};
+  const int64_t units = kvc_device_compute_units();
+  // 64 rows a block; 128 columns, or 64 where those give every unit a block and 128 do not (64 rows of 16384 x 2048 52 and
+  // 43 us).  Where neither does, the chains go to several blocks: of 128 columns if eight times as many fill the chip
+  // (122 rows of 2048 x 8192: 64 columns 46 us, 128 columns 39), of 64 otherwise (64 rows of it 28 and 37)
+  SharedShape s{2, 1};
+  const int64_t row_blocks = (M + 63) / 64, wide = (N + 127) / 128 * row_blocks, narrow = (N + 63) / 64 * row_blocks;
+  if (wide < units && (narrow >= units || kWaves * wide < units)) s.nt = 1;
+  while (s.groups < kWaves && (s.nt == 1 ? narrow : wide) * s.groups < units) s.groups *= 2;
+  return s;
+}
+
 }  // namespace
 
+extern "C" int64_t kvc_gemm_f32_parts_floats(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || shared_shape(M, N, K).groups < 2) return 0;
+  return static_cast<int64_t>(kWaves) * M * ((static_cast<int64_t>(N) + 3) & ~3);
+}
+
 extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const float* bias, int M,
-                            int N, int K, int64_t lda, int64_t ldc, kvc_stream stream) {
+                            int N, int K, int64_t lda, int64_t ldc, float* parts, int64_t parts_floats, kvc_stream stream) {
   if (M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N) return kvc_fail("kvc_gemm_f32: bad sizes");
+  if (parts_floats < kvc_gemm_f32_parts_floats(M, N, K) || (reinterpret_cast<uintptr_t>(parts) & 15) != 0)
+    return kvc_fail("kvc_gemm_f32: the workspace is too small or not 16-byte aligned");
   if (M == 0) return 0;
   const int64_t units = kvc_device_compute_units();
   const uintptr_t ends = reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W);
@@ -219,10 +468,10 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
   const int64_t tiles = static_cast<int64_t>((N + 15) / 16) * ((M + 15) / 16);
   const int from = chunks > 6 || (piece != 8 && chunks > 1) ? 24 : chunks > 2 ? 5 : chunks > 1 ? 3 : 0;
   if (chunks <= kWaves && tiles >= from * units) {
-    // 64 rows a wave where the operands' way to it counts and two blocks a unit are left: 4,096 rows of 8192 x 100 209 ->
-    // 157 us, of 8192 x 256 196 -> 189; of 8192 x 32, bound by C, 46 -> 55
+    // 64 rows a wave where the operands' way to it counts and two blocks a unit are left: 4,096 rows of 8192 x 256 185 ->
+    // 172 us (in smaller pieces, of 8192 x 100, 146 -> 167)
     int mt = M <= 16 ? 1 : 2, nt = 4;
-    if (chunks > 2 && static_cast<int64_t>((N + 255) / 256) * ((M + 63) / 64) >= 2 * units) mt = 4;
+    if (piece == 8 && chunks > 2 && static_cast<int64_t>((N + 255) / 256) * ((M + 63) / 64) >= 2 * units) mt = 4;
     auto short_blocks = [&]() { return static_cast<int64_t>((N + 64 * nt - 1) / (64 * nt)) * ((M + 16 * mt - 1) / (16 * mt)); };
     while (nt > 1 && short_blocks() < 2 * units) nt /= 2;
     const dim3 grid((N + 64 * nt - 1) / (64 * nt), (M + 16 * mt - 1) / (16 * mt));
@@ -242,9 +491,31 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
       else if (nt == 2) KVC_F32(2, 2);
       else KVC_F32(1, 2);
     } else {
-      KVC_F32(4, 4);  // blocks enough
+      KVC_F32_LAUNCH((gemm_f32_short_kernel<4, 4, 8>), 256);  // blocks enough
     }
 #undef KVC_F32
+    return kvc_check_launch("kvc_gemm_f32");
+  }
+  const SharedShape shape = piece == 8 ? shared_shape(M, N, K) : SharedShape{0, 0};
+  if (shape.nt) {
+    const int cols = 64 * shape.nt, rows = 16 * kSharedRows;
+    const dim3 grid((N + cols - 1) / cols, (M + rows - 1) / rows, shape.groups);
+    if (grid.y > 65535) return kvc_fail("kvc_gemm_f32: M too large for one launch");
+    const bool left = shape.groups > 1;
+#define KVC_F32_SHARED(NT, LEAVE)                                                                                           \
+  hipLaunchKernelGGL((gemm_f32_shared_kernel<kSharedRows, NT, LEAVE>), grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), \
+                     C, A, W, bias, parts, M, N, K, lda, ldc)
+    if (left && shape.nt == 2) KVC_F32_SHARED(2, true);
+    else if (left) KVC_F32_SHARED(1, true);
+    else if (shape.nt == 2) KVC_F32_SHARED(2, false);
+    else KVC_F32_SHARED(1, false);
+#undef KVC_F32_SHARED
+    if (left) {
+      const int64_t quads = static_cast<int64_t>(M) * ((N + 3) / 4);
+      hipLaunchKernelGGL(gemm_f32_parts_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0,
+                         reinterpret_cast<hipStream_t>(stream), C, A, W, bias, parts, chunks < kWaves ? chunks : kWaves, M, N,
+                         K, lda, ldc);
+    }
     return kvc_check_launch("kvc_gemm_f32");
   }
   // tiles of 64 x 64 where they give every compute unit a block, narrower ones otherwise (122 rows of 2048 x 2048

@@ -477,10 +477,12 @@ int kvc_hyper_step(void* out, int out_dtype, float* streams, const void* y, int 
 // streams[t, c, :] = rows[t, :] for every copy c.
 int kvc_spread_streams(float* streams, const float* rows, int T, int H, int copies, kvc_stream stream);
 
-// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float32 with float32 products and sums;
+// C[M, N] = A[M, K] * W[N, K]^T (+ bias[N]) in float32 with products and sums of 24 bits;
 // each element is the sum of eight running sums over fixed parts of K, whatever M is.
+// parts: a workspace of kvc_gemm_f32_parts_floats, which is 0 (and parts may be null) for most sizes.
+int64_t kvc_gemm_f32_parts_floats(int M, int N, int K);
 int kvc_gemm_f32(float* C, const float* A, const float* W, const float* bias, int M, int N,
-                 int K, int64_t lda, int64_t ldc, kvc_stream stream);
+                 int K, int64_t lda, int64_t ldc, float* parts, int64_t parts_floats, kvc_stream stream);
 
 // The same product for 17 to 192 rows, where the waves of a block share the rows of A through
 // LDS (K a multiple of 512).  mode 0: C = A W^T (+ bias), float32 (out_dtype 0) or bfloat16

@@ -99,7 +99,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_prefill_attention_supported": [I, I, I, I, I, I],
         "kvc_gemm_mid_slices": [I, I],
         "kvc_gemm_mid_bf16": [P, P, P, P, P, I, I, I, L, L, I, I, F, F, F, I, P],
-        "kvc_gemm_f32": [P, P, P, P, I, I, I, L, L, P],
+        "kvc_gemm_f32": [P, P, P, P, I, I, I, L, L, P, L, P],
         "kvc_gemm_skinny_bf16": [P, P, P, P, I, I, I, L, L, I, I, P],
         "kvc_gemm_skinny_act_bf16": [P, P, P, P, I, I, I, L, L, I, I, P],
         "kvc_gemm_skinny_silu_mul_bf16": [P, P, P, P, I, I, I, L, L, I, P],
@@ -133,6 +133,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.kvc_ssm_scan_max_state.argtypes = []
     lib.kvc_fixed_decay_chunk_tokens.restype = c_int
     lib.kvc_fixed_decay_chunk_tokens.argtypes = []
+    lib.kvc_gemm_f32_parts_floats.restype = c_int64
+    lib.kvc_gemm_f32_parts_floats.argtypes = [c_int] * 3
     lib.kvc_gated_chunk_floats.restype = c_int64
     lib.kvc_gated_chunk_floats.argtypes = [c_int] * 4
     lib.kvc_channel_chunk_floats.restype = c_int64
@@ -881,9 +883,13 @@ def gemm_f32(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: torch.Te
     for t, name in ((a, "a"), (out, "out")):
         if t.dtype != torch.float32 or not t.is_cuda:
             raise KernelError(f"gemm_f32: {name} must be a float32 GPU tensor")
-    _check(load().kvc_gemm_f32(out.data_ptr(), a.data_ptr(), _dev(w, "w", torch.float32),
-                               None if bias is None else _dev(bias, "bias", torch.float32),
-                               M, N, K, a.stride(0), out.stride(0), _stream()), "kvc_gemm_f32")
+    lib = load()
+    floats = lib.kvc_gemm_f32_parts_floats(M, N, K)
+    parts = torch.empty(floats, dtype=torch.float32, device=a.device) if floats else None
+    _check(lib.kvc_gemm_f32(out.data_ptr(), a.data_ptr(), _dev(w, "w", torch.float32),
+                            None if bias is None else _dev(bias, "bias", torch.float32),
+                            M, N, K, a.stride(0), out.stride(0), None if parts is None else parts.data_ptr(), floats,
+                            _stream()), "kvc_gemm_f32")
 
 
 SKINNY_MAX_ROWS = 64

@@ -159,6 +159,61 @@ def test_gemm_f32_of_short_rows_gives_the_same_bits(ops, M, N, K):
             assert torch.equal(single[0], out[i, :N])
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 100, 512), (64, 16384, 512), (65, 515, 1024), (122, 2048, 2048), (130, 8200, 1536),
+                                   (300, 33000, 512)])
+def test_gemm_f32_of_many_rows_gives_the_same_bits(ops, M, N, K):
+    """Rows through LDS (from 33 on, K a multiple of 512), with the chains of K in one block or in several: the sums of a
+    64-bit product, and a row's bits as it has them alone."""
+    a, w, b = rnd(M, K, seed=4), rnd(N, K, seed=5), rnd(N, seed=6)
+    wide_in, wide_out = torch.full((M, K + 4), 3.0, device=DEV), torch.full((M, N + 3), 7.0, device=DEV)
+    wide_in[:, :K] = a
+    ops.gemm_f32(wide_out[:, :N], wide_in[:, :K], w, b)
+    assert (wide_out[:, N:] == 7.0).all()
+    out = wide_out[:, :N]
+    want = a.double() @ w.double().T + b.double()
+    bound = 4 * math.sqrt(K) * 2 ** -24 * (a.double().abs() @ w.double().abs().T + b.double().abs())
+    assert ((out.double() - want).abs() <= bound + 1e-7).all()
+    single = torch.empty(1, N, device=DEV)
+    for i in {0, M // 2, M - 1}:
+        ops.gemm_f32(single, a[i:i + 1].contiguous(), w, b)
+        assert torch.equal(single[0], out[i])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 33, 64), (20, 40, 100), (20, 40, 99), (40, 70, 512), (2100, 1100, 64), (2100, 1100, 30)])
+def test_gemm_f32_of_values_at_the_ends_of_float32(ops, M, N, K):
+    """Infinities, NaN, the largest and the smallest numbers, in every kernel: what a chain of float32 gives."""
+    a, w = rnd(M, K, seed=4), rnd(N, K, seed=5)
+    out = torch.empty(M, N, device=DEV)
+
+    def check(a, w):
+        ops.gemm_f32(out, a, w, None)
+        want = a.double() @ w.double().T
+        # plus what float32 cannot hold of a product or a sum of subnormal size; operands are held to 2^-134 (subnormals that
+        # bfloat16 does not have) where the sum comes out as zero
+        bound = 4 * math.sqrt(K) * 2 ** -24 * (a.double().abs() @ w.double().abs().T) + K * 2.0 ** -149
+        bound += (out == 0) * 2.0 ** -134 * (a.double().abs().sum(1)[:, None] + w.double().abs().sum(1)[None])
+        assert torch.equal(out.isnan(), want.isnan())
+        inf = want.abs() > 3.40282351e38
+        assert torch.equal(out.isinf(), inf) and torch.equal(out[inf].sign().double(), want[inf].sign())
+        fine = ~(inf | want.isnan())
+        assert ((out.double() - want).abs() <= bound)[fine].all()
+
+    for value in (math.inf, -math.inf, math.nan, 3.4028234e38, -3.4e38):  # the last two round to infinity in bfloat16
+        x, y = a.clone(), w.clone()
+        x[M // 2] *= 1e-3
+        x[M // 2, K - 1] = value
+        check(x, y.clamp(-0.5, 0.5))  # a sum of the largest times at most a half stays in float32
+        if M < 100:
+            y[N // 3, 0] = value
+            check(a.clamp(-0.5, 0.5), y * torch.where(y.abs() > 1e30, 1.0, 1e-3))
+    if M < 100:  # products and sums of subnormal size, and operands that bfloat16 holds in part only
+        check(a * 1e-37, w)
+        check(a * 1e-30, w * 1e-8)
+        check(a * 1e-42, w)
+        check(a * 1e-20, w * 1e-25)
+    check(torch.zeros_like(a), w)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (5, 100, 200), (8, 4096, 4096), (16, 130, 1032),
                                    (17, 6144, 512), (33, 48, 14336), (64, 1000, 2048),
                                    # the longest sum and the widest output of the 70B shape
