@@ -340,9 +340,11 @@ int kvc_head_rmsnorm_gate(void* out, int out_dtype, const float* o, const void* 
 int kvc_moe_route(int32_t* choice, float* weight, const float* logits, int T, int E, int top,
                   int groups, int keep, int score_fn, const float* bias, const float* correction,
                   int group_best, int renormalize, float weight_scale, kvc_stream stream);
-// Tiles hold up to tile_rows rows, 16, 64 or 128 (kvc_moe_tile_rows says which a step's size and the experts'
-// matrices, [I, H] or gated [2 I, H] and [H, I], ask for; 64 and 128 are for bfloat16 with K a multiple of 32).
+// Tiles hold up to tile_rows rows, 16, 64, 128 or 384.  kvc_moe_tile_rows says which of the first three a step's size and the
+// experts' matrices, [I, H] or gated [2 I, H] and [H, I], ask for (64 and 128 are for bfloat16 with K a multiple of 32);
+// kvc_moe_wide_tile_rows gives 384 where that serves the step better still (bfloat16, K a multiple of 64), otherwise 0.
 int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated);
+int kvc_moe_wide_tile_rows(int pairs, int E, int H, int I, int gated);
 // The router's logits (x [T, H] of x_dtype times router [E, H] float32, float32 sums in one fixed order)
 // and the choice of kvc_moe_route in one kernel.  With gate [T] (may be null) the matrix is [E + 1, H]
 // and gate[t] = sigmoid(x[t] . its last row).

@@ -52,6 +52,11 @@ namespace {
 constexpr int kTileRows = 16;
 constexpr int kMidTileRows = 64;
 constexpr int kBigTileRows = 128;
+constexpr int kWideTileRows = 384;
+
+bool known_tile_rows(int rows) {
+  return rows == kTileRows || rows == kMidTileRows || rows == kBigTileRows || rows == kWideTileRows;
+}
 
 // What happens to the sums of an ungated product on their way out (the codes of kvc_activation; -1: nothing).
 __device__ __forceinline__ float plain_act(float v, int act) {
@@ -428,9 +433,8 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
   }
   __syncthreads();
   // an expert's rows in as few tiles as hold them, all of about one size (in sixteens): no tile is left with a few
-  const int shift = 31 - __clz(tile_rows);
   auto rows_each = [&](int n) {
-    const int tiles_of = (n + tile_rows - 1) >> shift;
+    const int tiles_of = (n + tile_rows - 1) / tile_rows;
     return tiles_of < 2 ? tile_rows : ((n + tiles_of - 1) / tiles_of + 15) & ~15;
   };
   auto list = [&](int e, int n, int each, int at, int nt) {
@@ -440,14 +444,13 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
       tiles[3 * nt + 1] = at + r;
       tiles[3 * nt + 2] = (n - r < each) ? n - r : each;
     }
-    if (e == E - 1) *num_tiles = nt;
   };
-  if (E <= kWave) {  // a lane an expert: running sums over the lanes
+  if (E <= kWave) {  // a lane an expert
     if (threadIdx.x < kWave) {
       const int e = threadIdx.x;
       const int n = e < E ? count[e] : 0;
       const int each = rows_each(n), mine = (n + each - 1) / each;
-      int at = n, nt = mine;
+      int at = n, nt = mine;  // running sums over the lanes
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) {
         const int pa = __shfl_up(at, o, kWave), pt = __shfl_up(nt, o, kWave);
@@ -456,7 +459,21 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
           nt += pt;
         }
       }
-      if (e < E) list(e, n, each, at - n, nt - mine);
+      if (e == E - 1) *num_tiles = nt < max_tiles ? nt : max_tiles;
+      nt -= mine;
+      if (tile_rows == kWideTileRows) {
+        // Blocks of tiles of up to 384 rows have a compute unit to themselves: experts with more rows a tile come first (the
+        // lower index among equals), each one's tiles side by side, so that the last blocks the chip takes up are the short
+        // ones.  Smaller tiles fetch weights in the experts' order (8 rows an expert, 32 gated experts of 2048 x 2048 in
+        // tiles of 64 rows: 95.3 us, in the other order 98.3).
+        const int rows = n < each ? n : each;
+        nt = 0;
+        for (int p = 0; p < E; ++p) {
+          const int pt = __builtin_amdgcn_readlane(mine, p), pr = __builtin_amdgcn_readlane(rows, p);
+          nt += pr > rows || (pr == rows && p < e) ? pt : 0;
+        }
+      }
+      if (e < E) list(e, n, each, at - n, nt);
     }
   } else {
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
@@ -471,6 +488,7 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
         nt += cursor[p];
       }
       list(e, count[e], rows_each(count[e]), at, nt);
+      if (e == E - 1) *num_tiles = nt + cursor[e] < max_tiles ? nt + cursor[e] : max_tiles;
     }
     __syncthreads();
   }
@@ -772,6 +790,60 @@ __device__ __forceinline__ TilePlace place(int id, int tiles, int cols) {
   const int col = at / tiles;
   return {at - col * tiles, col};
 }
+// clamped_glu with the division as a reciprocal and one correction of the quotient: within a rounding of the quotient in
+// float32, a third of the instructions of the division that is rounded correctly, of which a block of 256 x 128 gated values
+// took 6 us.
+__device__ __forceinline__ float tile_glu(float g, float u, float limit, float alpha, float shift) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  const float d = 1.f + expf(-alpha * g);
+  const float r = __builtin_amdgcn_rcpf(d), q = g * r, left = fmaf(-d, q, g);
+  return (left == left ? fmaf(left, r, q) : q) * (u + shift);  // no number where q or d is infinite: q is right then
+}
+
+// The way out of a tile's sums: lane (li, lk) holds NR rows (`row_of`) and of each NF times four columns from n + 16 f on.
+// The pairs and scales of all rows are asked for before the first store: a load behind it would wait for the store too,
+// which cost a block of 256 rows 9 us.
+template <int GATED, int NF, int NR, typename TO, typename RowOf, typename Acc, typename Acc2>
+__device__ __forceinline__ void store_tile(TO* out, int64_t out_stride, RowOf row_of, int nr, int n, int N, int r0,
+                                           const int32_t* sorted, int out_sorted, const float* row_scale, float limit,
+                                           float alpha, float shift, int act, Acc acc_of, Acc2 acc2_of) {
+  int pair[NR];
+  float scale[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) pair[r] = row_of(r) < nr ? r0 + row_of(r) : r0;
+  const bool by_place = out_sorted && row_scale == nullptr;  // the same for the whole grid
+  int place_of[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    place_of[r] = pair[r];
+    if (!by_place) pair[r] = sorted[pair[r]];
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) scale[r] = row_scale != nullptr ? row_scale[pair[r]] : 1.f;
+  constexpr int kBytes = 4 * sizeof(TO);
+  const bool whole = N % 4 == 0 && (reinterpret_cast<uintptr_t>(out) % kBytes) == 0 && out_stride % 4 == 0;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (row_of(r) >= nr) continue;
+    TO* to = out + static_cast<int64_t>(out_sorted ? place_of[r] : pair[r]) * out_stride + n;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      f32x4_t v = acc_of(f, r);
+      const f32x4_t v2 = acc2_of(f, r);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = GATED ? tile_glu(v[i] * scale[r], v2[i] * scale[r], limit, alpha, shift) : plain_act(v[i] * scale[r], act);
+      if (n + 16 * f >= N) continue;
+      if (whole) {
+        store4_whole(to + 16 * f, v);
+      } else {  // rare: kept from becoming a second copy of all of this
+#pragma unroll 1
+        for (int i = 0; i < 4 && n + 16 * f + i < N; ++i) to[16 * f + i] = from_float<TO>(i == 0 ? v[0] : i == 1 ? v[1] : i == 2 ? v[2] : v[3]);
+      }
+    }
+  }
+}
 
 template <int GATED, int NR, typename TO, int PACKED>
 __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
@@ -904,24 +976,178 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
   }
   if (!wave_live) return;
   // lane holds row 16 r + li of the tile, columns n0 + 16 f + 4 lk + i
+  store_tile<GATED, NF, NR, TO>(
+      out, out_stride, [&](int r) { return 16 * r + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale, limit, alpha, shift, act,
+      [&](int f, int r) { return acc[f][r]; }, [&](int f, int r) { return acc2[GATED ? f : 0][r]; });
+}
+
+// bfloat16, tiles of up to 384 rows: a block of eight waves takes the tile's rows and 256 columns (gated: 128 of gate and
+// the 128 of up beside them), one block a compute unit.
+// Both operands go straight into LDS (`global_load_lds`, 16 bytes a lane) in stages of 32 values of K: one is multiplied, one
+// has landed so that its first operands are read before the barrier, the others are on their way (five stages of 32 KB
+// up to 256 rows, four of 40 KB above).  A row block's stage is a kilobyte of 16 rows x 64 bytes; a lane's place in LDS is
+// fixed, so the lanes swap 16-byte pieces within a row on the way in such that the lanes that read operands together
+// meet all banks.  Wave (wr, wc) takes the row blocks of parity wr, so that a tile that is not full is dealt evenly, and 64
+// columns.
+// Packed, 32 experts of 2048 x 2048, gated and ungated, 8,192 pairs: tiles of 128 rows 202 and 122 us, these 168 and 90 (0.82
+// PFLOP/s; the weights alone take 83 and 41 us).  384 rows and not 256: experts of 256 rows in the mean have up to some 330, and
+// with tiles of 256 a third of them had two (175 and 115 us).  One expert of 8,192 rows in tiles of 256: 1.0 PFLOP/s, 1.18
+// without the way in and out of a block (some 10 us of 60); a stage of 256 rows takes 1,490 cycles at 1.8 GHz, of which the
+// matrix instructions are 1,024; without the loads 1,340 at 2.05 GHz: the chip's power, not their latency, is what they cost.
+constexpr int kWideBlocks = kWideTileRows / 32;  // row blocks a wave at most
+constexpr int kWideLds = 163840;
+
+// 64 lanes x 16 bytes, lane i's to lds + 16 i (a scalar byte address of LDS).  In text: where the compiler sees such a
+// load it waits for all of them before the next read of LDS, also of another buffer.  The waits are the kernel's own
+// (no register waits for these loads, and waits for others only get stricter).
+__device__ __forceinline__ void to_lds16(const void* from, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "memory", "m0");
+}
+
+// The wave's loads but the youngest N have landed; past the barrier that holds for all waves.
+template <int N>
+__device__ __forceinline__ void landed() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// R: how many row blocks a wave multiplies: the tile has at most 32 R rows
+template <int PACKED, int R>
+__device__ __forceinline__ void wide_walk(const char* lds, const char* const (&xp)[3], const char* const (&wp)[2], int wave,
+                                          int lane, const int (&wt)[4], int stages, int turn,
+                                          f32x4_t (&acc)[4][kWideBlocks]) {
+  constexpr int P = (R + 1) / 2;                      // row blocks go two at a time
+  constexpr int XL = R > 8 ? 3 : R > 4 ? 2 : 1;       // loads of rows a wave and stage, 8 KB for all waves
+  constexpr int LOADS = XL + 2;
+  constexpr int kW = XL > 2 ? 24576 : 16384;          // where a stage's weights begin
+  constexpr int kStage = kW + 16384;
+  constexpr int kStages = XL > 2 ? 4 : 5;
+  static_assert(kStage * kStages <= kWideLds, "");
+  const int li = lane & 15, lk = lane >> 4, wr = wave & 1;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)lds));
+  const int at = li * 64 + 16 * (lk ^ ((li >> 1) & 3));  // the lane's place in a row or column block
+  auto round = [&](int s) { return s + turn < stages ? s + turn : s + turn - stages; };
+  auto load = [&](int j, int64_t s, uint32_t buffer) {
+    if (j < XL) to_lds16(xp[j] + 64 * s, buffer + (wave + 8 * j) * 1024);
+    else to_lds16(wp[j - XL] + (PACKED ? 1024 : 64) * s, buffer + kW + (wave + 8 * (j - XL)) * 1024);
+  };
+  auto x_operand = [&](const char* stage, int r) {
+    return *reinterpret_cast<const bf16x8_t*>(stage + (2 * r + wr) * 1024 + at);
+  };
+  auto w_operand = [&](const char* stage, int f) { return *reinterpret_cast<const bf16x8_t*>(stage + kW + wt[f] + at); };
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    const int row = 16 * r + li;
-    if (row >= nr) continue;
-    const int pair = sorted[r0 + row];
-    const int64_t out_row = out_sorted ? r0 + row : pair;
-    const float scale = row_scale != nullptr ? row_scale[pair] : 1.f;
+  for (int s = 0; s < kStages - 1; ++s)
+    if (s < stages)  // scalar, as all that follow
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      f32x4_t v = acc[f][r];
+      for (int j = 0; j < LOADS; ++j) load(j, round(s), lds0 + s * kStage);
+  if (stages >= kStages - 1) landed<(kStages - 3) * LOADS>();
+  else landed<0>();
+  bf16x8_t a[4], b[2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = GATED ? clamped_glu(v[i] * scale, acc2[GATED ? f : 0][r][i] * scale, limit, alpha, shift)
-                     : plain_act(v[i] * scale, act);
-      const int nf = n0 + 16 * f + 4 * lk;
-      if (nf < N) store4<TO>(out + out_row * out_stride + nf, v, N - nf);
+  for (int f = 0; f < 4; ++f) a[f] = w_operand(lds, f);
+#pragma unroll
+  for (int i = 0; i < (R < 2 ? R : 2); ++i) b[i] = x_operand(lds, i);
+  int now = 0;  // byte offset of the stage's buffer
+  for (int s = 0; s < stages; ++s) {
+    const int next = now == (kStages - 1) * kStage ? 0 : now + kStage;
+    const int free = now == 0 ? (kStages - 1) * kStage : now - kStage;  // every wave has read it
+    const bool more = s + kStages - 1 < stages;
+    const int64_t from = round(s + kStages - 1);
+    bf16x8_t a_next[4];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      // a load, the operands of the next eight products, the eight products; the loads dealt over the stage, as a wave that
+      // asks for all of them at once waits until they are taken
+      if (more)
+#pragma unroll
+        for (int j = p * LOADS / P; j < (p + 1) * LOADS / P; ++j) load(j, from, lds0 + free);
+      bf16x8_t b_next[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (p + 1 < P && 2 * p + 2 + i < R) b_next[i] = x_operand(lds + now, 2 * p + 2 + i);
+        if (p + 1 == P && i < R) b_next[i] = x_operand(lds + next, i);
+      }
+      if (p == P - 1)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) a_next[f] = w_operand(lds + next, f);
+#pragma unroll
+      for (int i = 0; i < 2 && 2 * p + i < R; ++i)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+          acc[f][2 * p + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[f], b[i], acc[f][2 * p + i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) b[i] = b_next[i];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) a[f] = a_next[f];
+    // the stage after the next has landed where only those after it are on their way
+    if (more) landed<(kStages - 3) * LOADS>();
+    else if (kStages > 4 && s + kStages - 2 < stages) landed<LOADS>();
+    else landed<0>();
+    now = next;
+  }
+}
+
+template <int GATED, typename TO, int PACKED>
+__global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
+    TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
+    const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
+    const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
+    int act, const float* __restrict__ row_scale) {
+  constexpr int COLS = GATED ? 128 : 256;  // a block's columns of the result
+  __shared__ __attribute__((aligned(1024))) char lds[kWideLds];
+  const TilePlace at = place(blockIdx.x, *num_tiles, (N + COLS - 1) / COLS);
+  if (at.tile < 0) return;
+  const int e = tiles[3 * at.tile], r0 = tiles[3 * at.tile + 1];
+  const int nr = __builtin_amdgcn_readfirstlane(tiles[3 * at.tile + 2]);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int li = lane & 15, lk = lane >> 4, wr = wave & 1, wc = wave >> 1;
+  const int c0 = at.col * COLS, n0 = c0 + wc * (COLS / 4);
+  const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
+  // what the lane fetches of row blocks wave, wave + 8 and wave + 16 and of column blocks
+  // wave and wave + 8 (gated: the second is up's)
+  const int part = 16 * ((lane & 3) ^ ((lane >> 3) & 3));
+  const char *xp[3], *wp[2];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int row = 16 * (wave + 8 * j) + (lane >> 2);
+    const int safe = row < nr ? row : 0;  // a row that is not there reads the tile's first and is dropped
+    const int64_t in_row = in_div > 0 ? sorted[r0 + safe] / in_div : r0 + safe;
+    xp[j] = reinterpret_cast<const char*>(x + in_row * x_stride) + part;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int64_t first = static_cast<int64_t>(e) * rows_per_expert + (GATED && j == 1 ? N : 0);
+    if (PACKED) {  // pieces of 16 rows x 32 values
+      const int n = c0 + 16 * (GATED ? wave : wave + 8 * j);
+      wp[j] = reinterpret_cast<const char*>(w) + ((first + (n < N ? n : N - 16)) >> 4) * (K / 32) * 1024 + 64 * (lane >> 2) + part;
+    } else {
+      const int n = c0 + 16 * (GATED ? wave : wave + 8 * j) + (lane >> 2);
+      wp[j] = reinterpret_cast<const char*>(w + (first + (n < N ? n : N - 1)) * K) + part;
     }
   }
+  int wt[4];  // the wave's column blocks, in bytes
+#pragma unroll
+  for (int f = 0; f < 4; ++f) wt[f] = 1024 * (GATED ? 8 * (f >> 1) + 2 * wc + (f & 1) : 4 * wc + f);
+  f32x4_t acc[4][kWideBlocks];  // gated: [0..1] gate, [2..3] up
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int r = 0; r < kWideBlocks; ++r) acc[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // every block walks K round from a place of its own, as in the kernel for tiles of 128 rows, and from the same one
+  const int turn = (e * 5 + at.col * 11) % (K / 64) * 2;
+  switch ((nr + 31) >> 5) {  // scalar
+#define KVC_WALK(R) case R: wide_walk<PACKED, R>(lds, xp, wp, wave, lane, wt, K / 32, turn, acc); break
+    KVC_WALK(1); KVC_WALK(2); KVC_WALK(3); KVC_WALK(4); KVC_WALK(5); KVC_WALK(6); KVC_WALK(7);
+    KVC_WALK(8); KVC_WALK(9); KVC_WALK(10); KVC_WALK(11);
+#undef KVC_WALK
+    default: wide_walk<PACKED, kWideBlocks>(lds, xp, wp, wave, lane, wt, K / 32, turn, acc);
+  }
+  if (n0 >= N) return;  // the whole wave
+  // lane holds row 16 (2 r + wr) + li of the tile, columns n0 + 16 f + 4 lk + i
+  store_tile<GATED, GATED ? 2 : 4, kWideBlocks, TO>(
+      out, out_stride, [&](int r) { return 16 * (2 * r + wr) + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale, limit, alpha,
+      shift, act, [&](int f, int r) { return acc[f][r]; }, [&](int f, int r) { return acc[GATED ? f + 2 : 0][r]; });
 }
 
 // Any operand type and any sizes: a thread a (row, column) pair of the tile, float32 sums in index
@@ -1062,8 +1288,8 @@ extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* so
   if (T > kRouterSpread || E > kWave) return kvc_fail("kvc_moe_router_spread: at most 1024 tokens and 64 experts");
   if (score_fn < 0 || score_fn > 2 || (group_best != 1 && group_best != 2))
     return kvc_fail("kvc_moe_router_spread: scores by softmax (0), sigmoid (1) or logit (2); a group is worth its best 1 or 2");
-  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
-    return kvc_fail("kvc_moe_router_spread: tiles of 16, 64 or 128 rows");
+  if (!known_tile_rows(tile_rows))
+    return kvc_fail("kvc_moe_router_spread: tiles of 16, 64, 128 or 384 rows");
   if (max_tiles < kvc_moe_max_tiles(T * top, E, tile_rows))
     return kvc_fail("kvc_moe_router_spread: room for fewer tiles than the routing may need");
   if (parts_floats < kvc_moe_router_spread_floats(T, E) || (reinterpret_cast<uintptr_t>(parts) & 15) != 0)
@@ -1135,10 +1361,30 @@ extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
   return blocks >= 300 && (each >= 150 || (each >= 40 && each < 104)) ? kBigTileRows : kMidTileRows;
 }
 
+// Whether tiles of up to 384 rows (the answer; otherwise 0) serve such a step better.  A block of theirs has a compute unit to
+// itself, so the first product needs a block a unit and the second one every other unit (an expert has more than one tile only
+// from where nearly all do: rows vary by some three times their root), and below 104 rows an expert they are no faster than
+// the smaller tiles.  Both products in us, the best of the smaller tiles / these, by rows an expert, gated:
+//   32 experts of 2048 x 2048     90  178 / 174  130  237 / 196  180  242 / 218  256  324 / 259  330  371 / 304  500  523 / 444
+//   16 experts of 2048 x 2048     90   97 / 102  130  133 / 115  180  129 / 129  256  187 / 152  330  200 / 182  500  289 / 217
+//   64 experts of 1024 x 512      90   56 /  57  130   77 /  64  180   76 /  73  256  115 /  87  330  120 / 103  500  174 / 144
+//   128 experts of 1024 x 384     90   94 /  99  130  110 / 110  180  127 / 127  256  158 / 151  330  192 / 178  500  277 / 241
+// not gated:
+//   32 experts of 2048 x 2048     90  122 / 123  130  162 / 136  256  230 / 182
+// and where the blocks do not fill the units:
+//   16 experts of 1024 x 1024    256   69 /  83  400   74 /  97  500   98 /  82 (two tiles an expert)
+//   8 experts of 2048 x 1024     256   73 /  97  500  101 /  98
+extern "C" int kvc_moe_wide_tile_rows(int pairs, int E, int H, int I, int gated) {
+  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || H % 64 || I % 64) return 0;
+  const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
+  const double tiles = E * fmax(1.0, ceil((each - 3 * sqrt(each)) / kWideTileRows));
+  const int first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, down_cols = (H + 255) / 256;
+  return each >= 104 && tiles * first_cols >= units && 2 * tiles * down_cols >= units ? kWideTileRows : 0;
+}
+
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
                              int pairs, int E, int max_tiles, int tile_rows, kvc_stream stream) {
-  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
-    return kvc_fail("kvc_moe_align: tiles of 16, 64 or 128 rows");
+  if (!known_tile_rows(tile_rows)) return kvc_fail("kvc_moe_align: tiles of 16, 64, 128 or 384 rows");
   if (pairs < 0 || E <= 0 || max_tiles < kvc_moe_max_tiles(pairs, E, tile_rows))
     return kvc_fail("kvc_moe_align: bad sizes, or room for fewer tiles than the routing may need");
   const size_t lds = sizeof(int32_t) * 3 * E;
@@ -1155,8 +1401,7 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
                             const float* row_scale, int packed, kvc_stream stream) {
   if (max_tiles < 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N)
     return kvc_fail("kvc_moe_gemm: bad sizes");
-  if (tile_rows != kTileRows && tile_rows != kMidTileRows && tile_rows != kBigTileRows)
-    return kvc_fail("kvc_moe_gemm: tiles of 16, 64 or 128 rows");
+  if (!known_tile_rows(tile_rows)) return kvc_fail("kvc_moe_gemm: tiles of 16, 64, 128 or 384 rows");
   if (act < -1 || act > 0 || (gated && act != -1))
     return kvc_fail("kvc_moe_gemm: an ungated product has no activation (-1) or the square of relu (0)");
   if (max_tiles == 0) return 0;
@@ -1172,7 +1417,8 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
     const bool vectors = K % 8 == 0 && x_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(w) & 15) == 0;
     if (tile_rows != kTileRows) {
-      if (!vectors || K % 32) return kvc_fail("kvc_moe_gemm: tiles of 64 and 128 rows need K to be a multiple of 32");
+      if (!vectors || K % 32) return kvc_fail("kvc_moe_gemm: tiles of 64 rows and more need K to be a multiple of 32");
+      if (tile_rows == kWideTileRows && K % 64) return kvc_fail("kvc_moe_gemm: tiles of 384 rows need K to be a multiple of 64");
       if (packed && (N % 16 || K % 64))
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
       const int64_t cols = gated ? (N + 127) / 128 : (N + 255) / 256;
@@ -1186,7 +1432,23 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
     else if (out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, NR, bf16_t, PACKED>), bf16_t, bf16_t);    \
     else KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<0, NR, float, PACKED>), bf16_t, float);                          \
   } while (0)
-      if (tile_rows == kBigTileRows) {
+      if (tile_rows == kWideTileRows) {
+#define KVC_MOE_WIDE(GATED, TO, PACKED)                                                                           \
+  hipLaunchKernelGGL((moe_gemm_wide_kernel<GATED, TO, PACKED>), grid, dim3(512), 0, S(stream),                     \
+                     static_cast<TO*>(out), out_stride, static_cast<const bf16_t*>(x), x_stride,                  \
+                     static_cast<const bf16_t*>(w), KVC_MOE_ARGS)
+#define KVC_MOE_WIDE_OF(PACKED)                                  \
+  do {                                                           \
+    if (gated && out_dtype == 1) KVC_MOE_WIDE(1, bf16_t, PACKED); \
+    else if (gated) KVC_MOE_WIDE(1, float, PACKED);              \
+    else if (out_dtype == 1) KVC_MOE_WIDE(0, bf16_t, PACKED);    \
+    else KVC_MOE_WIDE(0, float, PACKED);                         \
+  } while (0)
+        if (packed) KVC_MOE_WIDE_OF(1);
+        else KVC_MOE_WIDE_OF(0);
+#undef KVC_MOE_WIDE_OF
+#undef KVC_MOE_WIDE
+      } else if (tile_rows == kBigTileRows) {
         if (packed) KVC_MOE_TILED(8, 1);
         else KVC_MOE_TILED(8, 0);
       } else {
@@ -1200,7 +1462,7 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
       // A whole K a wave where a share of it is at most two passes and there are waves enough without: one a compute unit
       // up to K of 256, three up to 512.  Shares / whole: 64 experts of 2048 x 512 down, 8 rows each, 36.7 / 26.2 us; 8
       // experts of 512 x 512 gated, 1 row each (256 waves), 5.4 / 6.6 us, 32 rows (768 waves) 9.5 / 8.3; 4 experts of
-      // 256 x 320 gated, 48 rows (320 waves), 7.1 / 5.8; 16 experts of 1024 x 1024 (sixteen passes), 64 rows, 27 / 33 us.
+      // 256 x 384 gated, 48 rows (384 waves), 7.1 / 5.8; 16 experts of 1024 x 1024 (sixteen passes), 64 rows, 27 / 33 us.
       const int64_t waves = static_cast<int64_t>(max_tiles) * ((N + 15) / 16);
       const bool whole = K <= 512 && waves >= (K <= 256 ? 1 : 3) * static_cast<int64_t>(kvc_device_compute_units());
       kvc_note_variant(kVariantMoeGemm, whole ? "moe_gemm_few_kernel, whole K" : "moe_gemm_few_kernel, shares of K");

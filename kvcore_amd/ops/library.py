@@ -76,6 +76,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_moe_router_spread_floats": [I, I],
         "kvc_moe_max_tiles": [I, I, I],
         "kvc_moe_tile_rows": [I, I, I, I, I],
+        "kvc_moe_wide_tile_rows": [I, I, I, I, I],
         "kvc_moe_align": [P, P, P, P, I, I, I, I, P],
         "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, I, P],
         "kvc_moe_combine": [P, P, P, I, P, I, P, P, I, I, I, P],
@@ -2097,6 +2098,14 @@ def moe_tile_rows(pairs: int, experts: int, x: torch.Tensor | None = None, k_siz
     if x is None or x.dtype != torch.bfloat16 or any(k % 32 for k in k_sizes):
         return 16
     return int(load().kvc_moe_tile_rows(pairs, experts, *k_sizes, int(gated)))
+
+
+def moe_wide_tile_rows(pairs: int, experts: int, x: torch.Tensor, k_sizes: tuple[int, int], gated: bool = True) -> int:
+    """384 where tiles of up to that many rows serve a step of this size better than those of :func:`moe_tile_rows`
+    and the operands allow (bfloat16, every K a multiple of 64), else 0."""
+    if x.dtype != torch.bfloat16:
+        return 0
+    return int(load().kvc_moe_wide_tile_rows(pairs, experts, *k_sizes, int(gated)))
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16) -> int:

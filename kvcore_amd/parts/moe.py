@@ -151,8 +151,9 @@ class RoutedExperts(FeedForward):
                     renormalize=self.renormalize)
         cap = ctx.buffers.token_capacity
         sorted_pairs = ctx.buffers.get(f"moe_sorted:{top}", pairs, 1, torch.int32, reserve=cap * top).view(-1)
-        # what is the faster for this many rows an expert and matrices of these sizes: see kvc_moe_tile_rows
-        tile_rows = ops.moe_tile_rows(pairs, E, x, (H, I), self.gated)
+        # what is the faster for this many rows an expert and matrices of these sizes: see the two kernels' files
+        tile_rows = (ops.moe_wide_tile_rows(pairs, E, x, (H, I), self.gated)
+                     or ops.moe_tile_rows(pairs, E, x, (H, I), self.gated))
         max_tiles = ops.moe_max_tiles(pairs, E, tile_rows)
         tiles = ctx.buffers.get(f"moe_tiles:{top}:{E}", max_tiles, 3, torch.int32,
                                 reserve=ops.moe_max_tiles(cap * top, E, 16))

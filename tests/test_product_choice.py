@@ -85,6 +85,19 @@ def test_rows_a_tile_of_few_rows_and_without_a_gate():
             assert ops.moe_tile_rows(each * E, E, x, (H, I), False) == tile, (E, H, I, each)
 
 
+def test_tiles_of_384_rows_need_rows_and_blocks_for_every_unit():
+    from kvcore_amd.ops import library as ops
+
+    x = torch.empty(1, 8, dtype=torch.bfloat16)
+    for (E, H, I), rows in {(32, 2048, 2048): {64: 0, 103: 0, 104: 384, 256: 384, 512: 384},
+                            (16, 2048, 2048): {96: 0, 130: 384}, (16, 1024, 1024): {256: 0, 400: 0, 500: 384},
+                            (8, 2048, 1024): {256: 0, 500: 0}, (128, 1024, 384): {130: 384}, (32, 2048, 2016): {256: 0}}.items():
+        for each, tile in rows.items():
+            assert ops.moe_wide_tile_rows(each * E, E, x, (H, I)) == tile, (E, H, I, each)
+    assert ops.moe_wide_tile_rows(256 * 32, 32, x.float(), (2048, 2048)) == 0
+    assert ops.moe_wide_tile_rows(0, 32, x, (2048, 2048)) == 0
+
+
 def _mixers():
     from kvcore_amd.parts.linear_attention import GatedLinearAttention, MaxGatedMatrixMemory
     from kvcore_amd.parts.recurrent import StateSpaceMixer

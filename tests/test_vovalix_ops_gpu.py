@@ -560,6 +560,85 @@ def test_products_of_experts_over_tiles_of_many_rows(tile_rows, packed, gated, N
 
 
 @pytest.mark.parametrize("packed", [False, True], ids=["rows", "packed"])
+@pytest.mark.parametrize("gated,N,K,out_dtype", [(True, 256, 64, torch.bfloat16), (True, 176, 192, torch.float32),
+                                                 (False, 512, 128, torch.float32), (False, 304, 320, torch.bfloat16),
+                                                 (True, 42, 64, torch.bfloat16), (False, 301, 448, torch.float32)])
+def test_products_of_experts_over_tiles_of_384_rows(packed, gated, N, K, out_dtype):
+    """Tiles at each number of row blocks a wave takes, and at its edges; two, four and more stages along K, so that the
+    last ones find nothing left to fetch; columns that end inside a wave's, and results that four at a time do not
+    divide; the same bits as tiles of 128 rows."""
+    from kvcore_amd.ops import library as ops
+
+    if packed and N % 16:
+        pytest.skip("a packed matrix has experts of a multiple of 16 rows")
+    gen = torch.Generator().manual_seed(N + K)
+    counts = [0, 1, 31, 32, 33, 65, 100, 129, 160, 192, 223, 225, 256, 257, 288, 289, 320, 321, 352, 353, 384, 385, 800]
+    E, T = len(counts), sum(counts)
+    choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=gen)]
+    x = torch.randn(T, K, generator=gen).to(torch.bfloat16)
+    w = (torch.randn(E * N * (2 if gated else 1), K, generator=gen) * K ** -0.5).to(torch.bfloat16)
+    scale = torch.rand(T, generator=gen) + 0.5
+    xg, wg, i32 = gpu(x, torch.bfloat16), gpu(w, torch.bfloat16), dict(dtype=torch.int32, device=DEV)
+    if packed:
+        ops.pack_weight(wg)
+    outs = []
+    for tile_rows in (384, 128):
+        sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+        tiles = torch.empty(ops.moe_max_tiles(T, E, tile_rows), 3, **i32)
+        ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32).view(T, 1), E, tile_rows)
+        listed = tiles[: int(num)].tolist()
+        assert all(1 <= n <= tile_rows for _, _, n in listed)
+        assert [sum(n for e, _, n in listed if e == which) for which in range(E)] == counts
+        out = torch.full((T, N + 3), float("nan"), dtype=out_dtype, device=DEV)
+        ops.moe_gemm(out[:, :N], xg, wg, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1, out_sorted=False,
+                     gated=gated, limit=1.2, alpha=1.702, up_shift=1.0, tile_rows=tile_rows, row_scale=gpu(scale),
+                     act=None if gated else "relu_squared")
+        assert out[:, N:].isnan().all()
+        outs.append(out[:, :N])
+    assert torch.equal(*outs)
+    want = torch.empty(T, N, dtype=torch.float64)
+    per = w.double().view(E, -1, K)
+    for e in range(E):
+        at = choice == e
+        y = (x[at].double() @ per[e].T) * scale[at, None].double()
+        if gated:
+            g, u = y[:, :N].clamp(max=1.2), y[:, N:].clamp(-1.2, 1.2)
+            want[at] = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            want[at] = y.clamp(min=0) ** 2
+    # float32 sums of exact products; a bfloat16 result adds one rounding of 2^-9
+    assert rel(outs[0], want) < (2e-6 if out_dtype == torch.float32 else 3e-3)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_experts_results_of_infinite_and_missing_sums(gated):
+    """Sums that are infinite or no number leave tiles of 64, 128 and 384 rows as the activation says, a sum whose
+    exponential overflows as zero."""
+    from kvcore_amd.ops import library as ops
+
+    T, N, K = 7, 16, 64
+    rows = torch.zeros(T, K, dtype=torch.bfloat16)
+    rows[:, 0] = torch.tensor([1.0, -1.0, 300.0, -300.0, float("inf"), float("-inf"), float("nan")])
+    w = torch.zeros(N * (2 if gated else 1), K, dtype=torch.bfloat16)
+    w[:, 0] = 1.0
+    i32 = dict(dtype=torch.int32, device=DEV)
+    zero = torch.zeros(T, 1, **i32)
+    for tile_rows in (64, 128, 384):
+        sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+        tiles = torch.empty(ops.moe_max_tiles(T, 1, tile_rows), 3, **i32)
+        ops.moe_align(sorted_pairs, tiles, num, zero, 1, tile_rows)
+        out = torch.empty(T, N, device=DEV)
+        ops.moe_gemm(out, gpu(rows, torch.bfloat16), gpu(w, torch.bfloat16), sorted_pairs, tiles, num, pairs=T, experts=1,
+                     in_div=1, out_sorted=False, gated=gated, limit=float("inf"), alpha=1.0, up_shift=0.0,
+                     tile_rows=tile_rows, act=None if gated else "relu_squared")
+        v = rows[:, 0].float()
+        limit = torch.tensor(float("inf"))  # the clamps take the limit for what is no number
+        g, u = torch.fmin(v, limit), torch.fmin(torch.fmax(v, -limit), limit)
+        want = g / (1.0 + torch.exp(-g)) * u if gated else torch.fmax(v, torch.zeros(())) ** 2
+        assert torch.allclose(out[:, 0].cpu(), want, rtol=1e-6, atol=1e-30, equal_nan=True)
+
+
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "packed"])
 @pytest.mark.parametrize("gated,N,K,whole", [
     (True, 64, 2048, False),    # 32 passes of 64: eight a wave, more than are on their way at once
     (False, 48, 1088, False),   # 17 passes
