@@ -116,6 +116,35 @@ def test_delta_rule_whole_in_steps_and_beside_others(heads, qk_heads, dim, vdim)
     assert rel(out, want) < 5e-6
 
 
+@pytest.mark.parametrize("rule", ["decay", "delta", "gates"])
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 32, 16), (2, 64, 40), (1, 128, 130), (70, 32, 64)])
+def test_whole_stages_of_tokens_give_the_bits_of_single_ones(rule, heads, dim, vdim):
+    """Stages of sixteen tokens keep a token's values in registers ahead of the work; one token at a time is the way without: the same
+    products and sums in the same order."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(dim + vdim)
+    T = 48
+    unit = lambda: gpu(plain.unit_vector(torch.randn(T, heads, dim, generator=gen, dtype=torch.float64)).reshape(T, -1))
+    q, k = unit(), unit()
+    v = gpu(torch.randn(T, heads * vdim, generator=gen))
+    beta = gpu(torch.rand(T, heads, generator=gen))
+    decay = gpu(torch.rand(T, heads * (dim if rule == "decay" else 1), generator=gen) * 0.3 + 0.7)
+
+    def scan(state, first, n):
+        batch, _ = batch_tensors([(0, first, n)])
+        out = torch.full((n, heads * vdim), float("nan"), device=DEV)
+        at = slice(first, first + n)
+        ops.linear_state_scan(out, q[at], k[at], v[at], decay[at], None if rule == "decay" else beta[at], state, heads=heads,
+                              qk_heads=heads, dim=dim, vdim=vdim, delta_rule=rule == "delta", scalar_gates=rule == "gates", **batch)
+        return out
+
+    whole, single = new_state(1, heads, dim, vdim), new_state(1, heads, dim, vdim)
+    out = scan(whole, 0, T)
+    assert torch.equal(out, torch.cat([scan(single, t, 1) for t in range(T)]))
+    assert torch.equal(whole, single)
+
+
 def test_a_token_written_six_hundred_tokens_ago_is_still_read():
     """A decay of almost one: the first token's value, written at a key of its own, comes back
     for a query of that key 600 tokens later (in one step, and token by token), scaled by the
