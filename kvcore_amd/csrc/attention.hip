@@ -175,6 +175,176 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void paged_attention_wave_ke
   }
 }
 
+// float32, heads of D = 64 or 128 whose values are as wide, pages of a multiple of four keys: a block takes one token and GH
+// (1, 2 or 4) query heads of one kv head.  The keys a token sees, from the last multiple of four at or before the first of them, go
+// in tiles of 64; eight chains take the tiles c, c + 8, ..., and their sums are joined in order through LDS, so what a
+// token's sums look like depends on its position (and the window's or chunk's start) alone, not on how many waves (W) deal the chains
+// out among them: eight where a step has few blocks, two where the chip is full (more would hold places of others'
+// waves, with nothing to do for a token near its prompt's start: 15.5 us where two take 10.0).
+// A wave's lanes take a key each for the scores (a key's row read once for all GH heads) and a channel each for the weighted
+// sums, whose values come in runs of four keys, half a tile's asked for without a branch.  The kernel above reads a key and
+// then a value at a time, one wave a head: bound by that chain, some 0.2 us a key.  32 heads of 64 over 8: two portions of 61
+// tokens 27.3 -> 10.0 us, of 512 1,255 -> 119; one token behind 1,500 335 -> 25, 16 behind 1,000 240 -> 21.
+constexpr int kChains = 8;
+
+template <int D, int GH, int W>
+__global__ __launch_bounds__(W* kWave) void paged_attention_tiles_kernel(
+    float* __restrict__ out, const float* __restrict__ q, int64_t q_stride, const float* __restrict__ k_cache,
+    const float* __restrict__ v_cache, const int32_t* __restrict__ table, int table_stride,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req, const int32_t* __restrict__ slots, int nh,
+    int nkv, int page_size, int num_pages, float scale, int window, const float* __restrict__ slopes, int chunk,
+    const float* __restrict__ sinks, float softcap, const float* __restrict__ gate, int64_t gate_stride) {
+  constexpr int E = D / kWave;  // channels a lane
+  __shared__ __attribute__((aligned(16))) float q_s[GH][D];
+  __shared__ __attribute__((aligned(16))) float p_s[W][GH][kWave];
+  __shared__ float acc_s[kChains][GH][D];
+  __shared__ float ml_s[kChains][GH][2];
+  const int t = blockIdx.x, group = nh / nkv, parts = (group + GH - 1) / GH;
+  const int hk = blockIdx.y / parts, g0 = (blockIdx.y - hk * parts) * GH;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const int h0 = hk * group + g0, heads = group - g0 < GH ? group - g0 : GH;
+  const int64_t o0 = (static_cast<int64_t>(t) * nh + h0) * D;
+  const int req = token_req[t];
+  if (req < 0) {  // padding token: the whole block takes this branch
+    for (int i = threadIdx.x; i < heads * D; i += W * kWave) out[o0 + i] = 0.f;
+    return;
+  }
+  const int pos = positions[t];
+  int first = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+  if (chunk > 0 && (pos / chunk) * chunk > first) first = (pos / chunk) * chunk;
+  const int start = first & ~3;
+  const int tiles = (pos - start) / kWave + 1;
+  const int32_t* row = table + static_cast<int64_t>(slots[req]) * table_stride;
+  for (int i = threadIdx.x; i < GH * D; i += W * kWave)  // a head that is not there is the last one again
+    q_s[i / D][i % D] = q[static_cast<int64_t>(t) * q_stride + static_cast<int64_t>(h0 + (i / D < heads ? i / D : heads - 1)) * D + i % D];
+  __syncthreads();
+  const int64_t page_elems = static_cast<int64_t>(nkv) * page_size * D;
+  const int64_t head_off = static_cast<int64_t>(hk) * page_size * D;
+  const int live = tiles < kChains ? tiles : kChains;
+  for (int chain = wave; chain < live; chain += W) {  // scalar
+    float m[GH], l[GH], acc[GH][E];
+#pragma unroll
+    for (int g = 0; g < GH; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.f;
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[g][e] = 0.f;
+    }
+    for (int tile = chain; tile < tiles; tile += kChains) {  // scalar
+      const int key = start + tile * kWave + lane;
+      const bool seen = key >= first && key <= pos;
+      const int at = key <= pos ? key : pos;
+      const int page = row[at / page_size];
+      const bool there = page > 0 && page < num_pages;
+      const bool valid = seen && there;
+      const int page_safe = there ? page : 0;  // the null page: read and not used
+      const int in_page = at % page_size;
+      const float* kr = k_cache + page_safe * page_elems + head_off + static_cast<int64_t>(in_page) * D;
+      float dot[GH];
+#pragma unroll
+      for (int g = 0; g < GH; ++g) dot[g] = 0.f;
+#pragma unroll 8
+      for (int i = 0; i < D; i += 4) {
+        const float4 kv = *reinterpret_cast<const float4*>(kr + i);
+#pragma unroll
+        for (int g = 0; g < GH; ++g) {
+          const float4 qv = *reinterpret_cast<const float4*>(&q_s[g][i]);
+          dot[g] = fmaf(qv.x, kv.x, dot[g]);
+          dot[g] = fmaf(qv.y, kv.y, dot[g]);
+          dot[g] = fmaf(qv.z, kv.z, dot[g]);
+          dot[g] = fmaf(qv.w, kv.w, dot[g]);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < GH; ++g) {
+        const float slope = slopes != nullptr ? slopes[h0 + (g < heads ? g : heads - 1)] : 0.f;
+        float s = dot[g] * scale - slope * static_cast<float>(pos - key);
+        if (softcap > 0.f) s = softcap * tanhf(s / softcap);  // the same for the whole grid
+        s = valid ? s : -INFINITY;
+        const float m_new = fmaxf(m[g], wave_max(s));
+        // a tile with no readable key (pages given back behind a window) leaves the state alone
+        const float p = s == -INFINITY ? 0.f : expf(s - m_new);
+        const float alpha = m[g] == -INFINITY ? 0.f : expf(m[g] - m_new);
+        l[g] = l[g] * alpha + wave_sum(p);
+        m[g] = m_new;
+        p_s[wave][g][lane] = p;
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[g][e] *= alpha;
+      }
+      __builtin_amdgcn_wave_barrier();  // the wave's own values: LDS keeps a wave's order
+      const uint64_t ok = __ballot(valid);
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        if (half == 1 && (ok >> 32) == 0) break;  // scalar
+        float4 v[8][E];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int from = 32 * half + 4 * j;
+          // lane `from` knows where its run is; one that lies behind the last key repeats that key's page: inside the cache, and not used
+          const int vp = __builtin_amdgcn_readlane(page_safe, from);
+          const int vi = __builtin_amdgcn_readlane(in_page, from) & ~3;
+          const float* vr = v_cache + vp * page_elems + head_off + vi;
+#pragma unroll
+          for (int e = 0; e < E; ++e) v[j][e] = *reinterpret_cast<const float4*>(vr + static_cast<int64_t>(lane + kWave * e) * page_size);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t okj = static_cast<uint32_t>(ok >> (32 * half + 4 * j)) & 15u;
+          if (okj == 0) continue;  // scalar
+          if (okj != 15u) {        // scalar; a value that may not be read may be no number
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              v[j][e].x = (okj & 1u) ? v[j][e].x : 0.f;
+              v[j][e].y = (okj & 2u) ? v[j][e].y : 0.f;
+              v[j][e].z = (okj & 4u) ? v[j][e].z : 0.f;
+              v[j][e].w = (okj & 8u) ? v[j][e].w : 0.f;
+            }
+          }
+#pragma unroll
+          for (int g = 0; g < GH; ++g) {
+            const float4 p = *reinterpret_cast<const float4*>(&p_s[wave][g][32 * half + 4 * j]);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+              acc[g][e] = fmaf(p.x, v[j][e].x, acc[g][e]);
+              acc[g][e] = fmaf(p.y, v[j][e].y, acc[g][e]);
+              acc[g][e] = fmaf(p.z, v[j][e].z, acc[g][e]);
+              acc[g][e] = fmaf(p.w, v[j][e].w, acc[g][e]);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int g = 0; g < GH; ++g) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc_s[chain][g][lane + kWave * e] = acc[g][e];
+      if (lane == 0) {
+        ml_s[chain][g][0] = m[g];
+        ml_s[chain][g][1] = l[g];
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < heads * D; i += W * kWave) {
+    const int g = i / D, e = i % D;
+    // a sink is one more logit in the denominator that brings no value along
+    const float sink = sinks != nullptr ? sinks[h0 + g] : -INFINITY;
+    float top = sink;
+    for (int w = 0; w < live; ++w) top = fmaxf(top, ml_s[w][g][0]);
+    float sum = sink == -INFINITY ? 0.f : expf(sink - top), y = 0.f;
+    for (int w = 0; w < live; ++w) {
+      const float mw = ml_s[w][g][0];
+      const float f = mw == -INFINITY ? 0.f : expf(mw - top);
+      sum = fmaf(ml_s[w][g][1], f, sum);
+      y = fmaf(acc_s[w][g][e], f, y);
+    }
+    y *= sum > 0.f ? 1.f / sum : 0.f;
+    if (gate != nullptr) y *= sigmoid_of(gate[t * gate_stride + static_cast<int64_t>(h0 + g) * D + e]);
+    out[o0 + i] = y;
+  }
+}
+
 }  // namespace
 
 extern "C" int kvc_paged_attention(void* out, const void* q, int64_t q_stride, const void* k_cache,
@@ -199,6 +369,40 @@ extern "C" int kvc_paged_attention(void* out, const void* q, int64_t q_stride, c
   if (gate != nullptr && gate_stride < static_cast<int64_t>(nh) * dv)
     return kvc_fail("kvc_paged_attention: gate rows too short");
   if (T == 0) return 0;
+  if (dtype == 0 && dv == d && (d == 64 || d == 128) && page_size % 4 == 0 &&
+      ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) & 15) == 0) {
+    const int group = nh / nkv, gh = group == 1 ? 1 : group == 2 ? 2 : 4;
+    const int64_t rows = static_cast<int64_t>(nkv) * ((group + gh - 1) / gh);
+    if (rows <= 65535) {
+      #define KVC_TILES(D, GH, W)                                                                                       \
+  hipLaunchKernelGGL((paged_attention_tiles_kernel<D, GH, W>), dim3(T, static_cast<unsigned>(rows)),              \
+                     dim3(W * kWave), 0, reinterpret_cast<hipStream_t>(stream), static_cast<float*>(out), \
+                     static_cast<const float*>(q), q_stride, static_cast<const float*>(k_cache),                  \
+                     static_cast<const float*>(v_cache), table, table_stride, positions, token_req, slots, nh, nkv, \
+                     page_size, num_pages, scale, window, slopes, chunk, sinks, softcap,                          \
+                     static_cast<const float*>(gate), gate_stride)
+#define KVC_TILES_W(D, GH)              \
+  do {                                  \
+    if (few) KVC_TILES(D, GH, 8);       \
+    else KVC_TILES(D, GH, 2);           \
+  } while (0)
+#define KVC_TILES_OF(D)                \
+  do {                                 \
+    if (gh == 1) KVC_TILES_W(D, 1);    \
+    else if (gh == 2) KVC_TILES_W(D, 2); \
+    else KVC_TILES_W(D, 4);            \
+  } while (0)
+      const bool few = T * rows < 2 * static_cast<int64_t>(kvc_device_compute_units());
+      kvc_note_variant(kVariantPagedAttention, few ? "paged_attention_tiles_kernel, 8 waves" : "paged_attention_tiles_kernel, 2 waves");
+      if (d == 64) KVC_TILES_OF(64);
+      else KVC_TILES_OF(128);
+#undef KVC_TILES_W
+#undef KVC_TILES_OF
+#undef KVC_TILES
+      return kvc_check_launch("kvc_paged_attention");
+    }
+  }
+  kvc_note_variant(kVariantPagedAttention, "paged_attention_wave_kernel");
   const dim3 grid(T, (nh + kWavesPerBlock - 1) / kWavesPerBlock);
   if (d > kUsualHeadDim || dv > kUsualHeadDim) {
     KVC_DISPATCH_DTYPE(

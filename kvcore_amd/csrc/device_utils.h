@@ -136,5 +136,5 @@ int kvc_device_compute_units(void);
 // which one they launched (kvc_note_variant), and kvc_last_variant() tells the caller's thread:
 // for tests and tuning that must know which code ran.
 enum { kVariantPrefillAttention = 0, kVariantRopeKvWrite = 1, kVariantDecodeAttention = 2, kVariantMoeGemm = 3,
-       kVariantFamilies = 4 };
+       kVariantPagedAttention = 4, kVariantFamilies = 5 };
 void kvc_note_variant(int family, const char* name);

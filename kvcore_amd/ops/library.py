@@ -658,7 +658,8 @@ def decode_attention_supported(nh: int, nkv: int, d: int, page_size: int, dtype:
                                                       DTYPE_CODE.get(dtype, -1)))
 
 
-KERNEL_FAMILIES = {"prefill_attention": 0, "rope_kv_write": 1, "decode_attention": 2, "moe_gemm": 3}
+KERNEL_FAMILIES = {"prefill_attention": 0, "rope_kv_write": 1, "decode_attention": 2, "moe_gemm": 3,
+                   "paged_attention": 4}
 
 
 def last_variant(family: str) -> str:

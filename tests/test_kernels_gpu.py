@@ -829,6 +829,60 @@ def test_paged_attention_mixed_batch(ops, dtype, nh, nkv, d, page):
         t += ql
 
 
+@pytest.mark.parametrize("nh,nkv,d,page", [(32, 8, 64, 16), (3, 3, 64, 4), (6, 3, 128, 12), (5, 1, 128, 16), (3, 1, 64, 32)])
+@pytest.mark.parametrize("option", ["plain", "window", "chunk", "sinks", "slopes", "softcap", "gate"])
+def test_paged_attention_of_float32_over_tiles_of_keys(ops, nh, nkv, d, page, option):
+    """Positions at the edges of the runs of four keys, the tiles of 64 and the rounds of eight tiles, under each option,
+    against float64; what a token may not read is no number, and its bits do not depend on the batch."""
+    seq_lens = [1, 4, 5, 63, 64, 65, 130, 511, 513, 700]
+    kc, vc, table, dense = paged_setup(seq_lens, nkv, d, page, torch.float32, seed=d + nh)
+    window = 70 if option == "window" else 0
+    chunk = 90 if option == "chunk" else 0
+    gen = torch.Generator().manual_seed(nh)
+    sinks = torch.randn(nh, generator=gen).to(DEV) if option == "sinks" else None
+    slopes = (torch.rand(nh, generator=gen) * 0.1).to(DEV) if option == "slopes" else None
+    softcap = 2.0 if option == "softcap" else 0.0
+    spans = [(r, p) for r, n in enumerate(seq_lens) for p in sorted({0, n // 2, n - 1})]
+    T = len(spans)
+    q = rnd(T, nh * d, dtype=torch.float32, seed=7) * 2
+    gate = rnd(T, nh * d, dtype=torch.float32, seed=8) if option == "gate" else None
+    scale = d ** -0.5
+    def run(which):
+        pos = torch.tensor([spans[i][1] for i in which], dtype=torch.int32, device=DEV)
+        req = torch.tensor([spans[i][0] for i in which], dtype=torch.int32, device=DEV)
+        out = torch.empty(len(which), nh * d, device=DEV)
+        ops.paged_attention(out, q[which], kc, vc, table=table, positions=pos, token_req=req,
+                            slots=torch.arange(1, len(seq_lens) + 1, dtype=torch.int32, device=DEV), nh=nh, nkv=nkv, d=d,
+                            scale=scale, window=window, chunk=chunk, sinks=sinks, slopes=slopes, softcap=softcap,
+                            gate=None if gate is None else gate[which])
+        few = len(which) * nkv * -(-(nh // nkv) // 4) < 2 * ops.compute_units()
+        assert ops.last_variant("paged_attention") == f"paged_attention_tiles_kernel, {8 if few else 2} waves"
+        return out
+
+    out = run(list(range(T)))
+    assert torch.equal(run(list(range(T)) * 24).view(24, T, -1), out.expand(24, -1, -1))  # two waves a block
+    for i, (r, p) in enumerate(spans):
+        k, v = dense[r][0].double()[: p + 1], dense[r][1].double()[: p + 1]
+        key = torch.arange(p + 1)
+        first = max(p - window + 1 if window else 0, p // chunk * chunk if chunk else 0)
+        for h in range(nh):
+            s = k[:, h // (nh // nkv)] @ q[i, h * d:(h + 1) * d].double().cpu() * scale
+            if slopes is not None:
+                s = s - float(slopes[h]) * (p - key)
+            if softcap:
+                s = softcap * torch.tanh(s / softcap)
+            s = s.masked_fill(key < first, -torch.inf)
+            if sinks is not None:
+                s = torch.cat([s, sinks[h].double().cpu()[None]])
+            y = torch.softmax(s, 0)[: p + 1] @ v[:, h // (nh // nkv)]
+            if gate is not None:
+                y = y * torch.sigmoid(gate[i, h * d:(h + 1) * d].double().cpu())
+            # sums of at most 700 weighted values and dots of 128 terms in float32
+            assert torch.allclose(out[i, h * d:(h + 1) * d].double().cpu(), y, atol=1e-5, rtol=1e-5), (r, p, h)
+    some = [T - 1, 3, T - 2]
+    assert torch.equal(run(some), out[some])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_paged_attention_finds_one_far_key_among_hundreds(ops, dtype):
     """Random keys would hide a skipped key.  One key (in turn: the first, one at a page's
