@@ -72,7 +72,9 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(
 
 // The same for up to 8 taps, eight consecutive tokens a thread: the taps' weights are fetched
 // once, and the window of the last K inputs slides along in registers, so that a token costs
-// one load of x and one store.
+// one load of x and one store.  Where all eight and the K - 1 inputs before them are one request's of this
+// step, as nearly everywhere in a prompt, all inputs are asked for at once: token by token, each behind the
+// loads of its request and position, 2,048 tokens of 6,144 channels took 33 us, this way 25 (75 MB: 12 us).
 constexpr int kConvTokens = 8, kConvMaxTaps = 8;
 template <typename TI, typename TO>
 __global__ __launch_bounds__(256) void causal_conv_window_kernel(
@@ -91,6 +93,26 @@ __global__ __launch_bounds__(256) void causal_conv_window_kernel(
     h[j] = 0.f;
   }
   const float b0 = bias != nullptr ? bias[c] : 0.f;
+  if (t0 + kConvTokens <= T) {
+    const int r = token_req[t0];  // the same for the whole block, as all that decides here
+    if (r >= 0 && t0 - (K - 1) >= q_start[r] && t0 + kConvTokens <= q_start[r + 1]) {
+      float in[kConvTokens + kConvMaxTaps - 1];  // the last input first
+      const TI* xc = x + static_cast<int64_t>(t0 + kConvTokens - 1) * x_stride + c;
+      const int n = kConvTokens + K - 1;
+#pragma unroll
+      for (int j = 0; j < kConvTokens + kConvMaxTaps - 1; ++j)  // what no tap reads repeats the first
+        in[j] = to_float(xc[-static_cast<int64_t>(j < n ? j : n - 1) * x_stride]);
+#pragma unroll
+      for (int tt = 0; tt < kConvTokens; ++tt) {
+        float acc = b0;
+#pragma unroll
+        for (int j = 0; j < kConvMaxTaps; ++j) acc = fmaf(wr[j], j < K ? in[kConvTokens - 1 - tt + j] : 0.f, acc);
+        if (act == 1) acc = silu_f(acc);
+        out[static_cast<int64_t>(t0 + tt) * out_stride + c] = from_float<TO>(acc);
+      }
+      return;
+    }
+  }
   bool sliding = false;  // h holds the window of the token before
   for (int tt = 0; tt < kConvTokens && t0 + tt < T; ++tt) {
     const int t = t0 + tt;
@@ -492,6 +514,8 @@ __global__ __launch_bounds__(256) void rglru_scan_segments_kernel(
   }
   const float* sums = ws + static_cast<int64_t>(r) * (segs + 1) * 2 * W + c;
   float s = sums[static_cast<int64_t>(segs) * 2 * W];
+  // (the sums of eight segments on their way at a time: one by one, 2,048 tokens of 2,560 channels 39 us, so 34)
+#pragma unroll 8
   for (int j = 0; j < sg; ++j) s = fmaf(sums[static_cast<int64_t>(j) * 2 * W], s, sums[static_cast<int64_t>(j) * 2 * W + W]);
 #pragma unroll 8
   for (int t = t0; t < t1; ++t) {

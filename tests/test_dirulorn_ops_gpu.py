@@ -424,6 +424,34 @@ def attention_setup(ops, T_cap, nkv, d, dv, page, dtype, planes=1):
     return kc, vc[0] if planes == 1 else vc
 
 
+@pytest.mark.parametrize("K", [1, 2, 4, 8])
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.bfloat16])
+def test_convolution_of_groups_of_tokens_at_requests_edges(ops, K, x_dtype):
+    """Eight tokens a thread, all inputs at once where one request of the step holds them: requests that begin and end
+    inside such a group or at its edge, with and without a state before them, give the bits of one token at a time."""
+    C, cuts = 70, [(1, 0, 8), (2, 3, 9), (3, 0, 24), (4, 20, 1), (5, 1, 30), (6, 0, 16)]
+    gen = torch.Generator().manual_seed(K)
+    batch, T = batch_tensors(cuts)
+    x = torch.randn(T, C, generator=gen).to(x_dtype).to(DEV)
+    w, bias = torch.randn(C, K, generator=gen).to(DEV), torch.randn(C, generator=gen).to(DEV)
+    state0 = torch.randn(8, K - 1, C, generator=gen).to(DEV)
+
+    def run(xs, st, batch):
+        out = torch.full((xs.shape[0], C), float("nan"), device=DEV)
+        ops.causal_conv(out, xs, w, bias, st, act="silu", update_state=True, **batch)
+        return out
+
+    state = state0.clone()
+    out = run(x, state, batch)
+    single, at = state0.clone(), 0
+    for slot, first, n in cuts:
+        for i in range(n):
+            one, _ = batch_tensors([(slot, first + i, 1)])
+            assert torch.equal(run(x[at + i: at + i + 1], single, one)[0], out[at + i]), (slot, i)
+        at += n
+    assert torch.equal(state, single)
+
+
 def run_attention_in_steps(ops, qkv, cuts, nh, nkv, d, dv, scale, freqs, interleaved, gains, eps, page, dtype,
                            table_pages, planes=1):
     """Norm, rotation, cache write and attention of one request cut at ``cuts``; pages in the
