@@ -11,7 +11,9 @@
 //   S^T[16 keys, 16 rows]  = K[16 keys, d]   * Q^T[d, 16 rows]        (16x16x32, per key block)
 //   O^T[dv, 16 rows]      += V^T[dv, 32 keys] * P^T[32 keys, 16 rows] (16x16x32, per two key blocks)
 //
-// with value heads as wide as the keys or half as wide.
+// with value heads as wide as the keys or half as wide, or, on keys of 64, values of 128 that lie in two planes of
+// 64 (their two halves against one set of scores: 2,048 tokens of 32 heads over 8, 43 us a plane and a copy of 16 us that
+// laid the planes side by side, 56 us this way).
 //
 // A lane's four accumulator values of S^T for key blocks a and b are the eight values of
 // the B operand of the second product, if the product's k index 8*quad + e stands for key
@@ -87,7 +89,7 @@ constexpr int tile_bytes() {
 template <int D, int DV, int CT, int KB, int W, int CAP_GATE>
 __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_kernel(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, int64_t q_stride,
-    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_first, const bf16_t* __restrict__ v_second,
     const int32_t* __restrict__ table, int table_stride, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ q_start, const int32_t* __restrict__ slots, int num_reqs, int nh,
     int nkv, int page_size, int num_pages, float scale_log2e, int window,
@@ -98,6 +100,7 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
   constexpr int kKeyBlocks = KB;
   constexpr int NJ = DV / 16;
   constexpr int NC = D / 32;
+  constexpr int DVP = DV > D ? D : DV;  // a plane's share of a value head
   // padded K row in LDS (elements): with 32 bytes of padding the operand reads (16 rows x 4
   // pieces of 16 bytes a wave) meet no bank conflict; with 16 they took 1.45 times as long
   constexpr int KROW = D + 16;
@@ -315,9 +318,12 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
 #pragma unroll
   for (int i = 0; i < K_PER_THREAD; ++i)
     k_off[i] = ((i * ROWS_PER_STEP + k_row0) & 15) * D + k_piece * 8;
+  // which plane a thread's row of the head lies in (the same for its wave)
+  const bool v_behind = DV > DVP && __builtin_amdgcn_readfirstlane(v_rem >> 1) >= DVP;
+  const bf16_t* const v_cache = v_behind ? v_second : v_first;
 #pragma unroll
   for (int i = 0; i < V_PER_THREAD; ++i) {
-    v_off[i] = (v_rem >> 1) * page_size + (v_rem & 1) * 8;
+    v_off[i] = ((v_rem >> 1) - (v_behind ? DVP : 0)) * page_size + (v_rem & 1) * 8;
   }
   // Where the key blocks of a tile lie.  Lane i of every wave looks up key block kb0 + i of
   // the tile with one vector load (`lookup_issue`), one tile before the tile is fetched; the
@@ -330,8 +336,8 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
   const int sub_shift = (blocks_per_page & sub_mask) == 0 ? __builtin_ctz(blocks_per_page) : -1;
   const int64_t page_elems = static_cast<int64_t>(nkv) * page_size * D;  // of the keys' plane
   const int64_t head_elems = static_cast<int64_t>(hk) * page_size * D;
-  const int64_t v_page_elems = static_cast<int64_t>(nkv) * page_size * DV;
-  const int64_t v_head_elems = static_cast<int64_t>(hk) * page_size * DV;
+  const int64_t v_page_elems = static_cast<int64_t>(nkv) * page_size * DVP;
+  const int64_t v_head_elems = static_cast<int64_t>(hk) * page_size * DVP;
   const int lk_lane = lane & 15;
   int lk_page = 0, lk_sub = 0;
   auto lookup_issue = [&](int kb0) {
@@ -687,7 +693,7 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
 
 template <int D, int DV, int CT, int W, int CAP_GATE>
 int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t* k_cache,
-                      const bf16_t* v_cache, const int32_t* table, int table_stride,
+                      const bf16_t* v_cache, const bf16_t* v_second, const int32_t* table, int table_stride,
                       const int32_t* positions, const int32_t* q_start, const int32_t* slots, int T,
                       int R, int nh, int nkv, int page_size, int num_pages, float scale, int window,
                       const float* slopes, int chunk, const float* sinks, float* part_o, float* part_ml, int nsplit, int single,
@@ -720,7 +726,7 @@ int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16
            single ? " one tile a block" : "", nsplit);
   kvc_note_variant(kVariantPrefillAttention, variant);
   hipLaunchKernelGGL((prefill_attention_kernel<D, DV, CT, KB, W, CAP_GATE>), dim3(static_cast<unsigned>(wide), 1, nsplit), dim3(W * 64),
-                     lds_bytes, stream, out, q, q_stride, k_cache, v_cache, table, table_stride, positions,
+                     lds_bytes, stream, out, q, q_stride, k_cache, v_cache, v_second, table, table_stride, positions,
                      q_start, slots, R, nh, nkv, page_size, num_pages, (softcap > 0.f ? softcap : scale) * kLog2e, window,
                      slopes, chunk, sinks, part_o, part_ml, single, cos_tab, sin_tab, rot_dim, interleaved,
                      softcap > 0.f ? 2.f * kLog2e * scale / softcap : 0.f, gate, out_f32);
@@ -731,7 +737,7 @@ int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16
 
 template <int D, int DV>
 int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t* k_cache,
-                   const bf16_t* v_cache, const int32_t* table, int table_stride,
+                   const bf16_t* v_cache, const bf16_t* v_second, const int32_t* table, int table_stride,
                    const int32_t* positions, const int32_t* q_start, const int32_t* slots, int T,
                    int R, int nh, int nkv, int page_size, int num_pages, float scale, int window,
                    const float* slopes, int chunk, const float* sinks, float* part_o, float* part_ml, int nsplit,
@@ -793,19 +799,20 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   if (DV < 64) waves = 4;  // eight waves would stage the values of more key blocks than a tile has
   if (g > 16 * waves * ct) return kvc_fail("kvc_prefill_attention: too many query heads per kv head");
 #define KVC_LAUNCH_PREFILL(CT_, W_)                                                                      \
-  return softcap > 0.f || gate.gate != nullptr ? LAUNCH_WITH(CT_, W_, 1) : LAUNCH_WITH(CT_, W_, 0)
+  if constexpr (DV > D) return LAUNCH_WITH(CT_, W_, 0);                                                  \
+  else return softcap > 0.f || gate.gate != nullptr ? LAUNCH_WITH(CT_, W_, 1) : LAUNCH_WITH(CT_, W_, 0)
 #define LAUNCH_WITH(CT_, W_, CAP_GATE_)                                                                  \
-  launch_prefill_ct<D, DV, CT_, W_, CAP_GATE_>(out, q, q_stride, k_cache, v_cache, table, table_stride, positions, \
+  launch_prefill_ct<D, DV, CT_, W_, CAP_GATE_>(out, q, q_stride, k_cache, v_cache, v_second, table, table_stride, positions, \
                                        q_start, slots, T, R, nh, nkv, page_size, num_pages, scale, window, \
                                        slopes, chunk, sinks, part_o, part_ml, nsplit, single, cos_tab, sin_tab, rot_dim,     \
                                        interleaved, softcap, gate, out_f32, stream)
   if constexpr (DV >= 64) {
     if (waves == 8) {
-      if (ct == 2) KVC_LAUNCH_PREFILL(2, 8);
+      if (ct == 2) { KVC_LAUNCH_PREFILL(2, 8); }
       KVC_LAUNCH_PREFILL(1, 8);
     }
   }
-  if (ct == 2) KVC_LAUNCH_PREFILL(2, 4);
+  if (ct == 2) { KVC_LAUNCH_PREFILL(2, 4); }
   KVC_LAUNCH_PREFILL(1, 4);
 #undef KVC_LAUNCH_PREFILL
 #undef LAUNCH_WITH
@@ -822,7 +829,7 @@ extern "C" int kvc_prefill_attention_supported(int nh, int nkv, int d, int dv, i
 }
 
 extern "C" int kvc_prefill_attention(void* out, const void* q, int64_t q_stride,
-                                     const void* k_cache, const void* v_cache,
+                                     const void* k_cache, const void* v_cache, const void* v_second,
                                      const int32_t* table, int table_stride,
                                      const int32_t* positions, const int32_t* q_start,
                                      const int32_t* slots, int T, int R, int nh, int nkv, int d, int dv,
@@ -830,7 +837,10 @@ extern "C" int kvc_prefill_attention(void* out, const void* q, int64_t q_stride,
                                      const float* slopes, int chunk, const float* sinks, void* part_o, void* part_ml, int nsplit, const float* cos_tab,
                                      const float* sin_tab, int rot_dim, int interleaved, float softcap,
                                      const void* gate_rows, int64_t gate_stride, int out_f32, kvc_stream stream) {
-  if (!kvc_prefill_attention_supported(nh, nkv, d, dv, page_size, 1))
+  const bool two = v_second != nullptr;
+  if (two && (d != 64 || dv != 128 || softcap > 0.f || gate_rows != nullptr))
+    return kvc_fail("kvc_prefill_attention: values in two planes are 128 wide on keys of 64, without a cap or a gate");
+  if (!kvc_prefill_attention_supported(nh, nkv, d, two ? d : dv, page_size, 1))
     return kvc_fail("kvc_prefill_attention: unsupported shape (bfloat16, head size 64 or 128, values as "
                     "wide or half as wide, at most 64 query heads per kv head, page size a multiple of 16)");
   if (T < 0 || R <= 0 || nkv > 65535 || table_stride <= 0 || num_pages <= 0)
@@ -860,11 +870,13 @@ extern "C" int kvc_prefill_attention(void* out, const void* q, int64_t q_stride,
   const bf16_t* qq = static_cast<const bf16_t*>(q);
   const bf16_t* kc = static_cast<const bf16_t*>(k_cache);
   const bf16_t* vc = static_cast<const bf16_t*>(v_cache);
+  const bf16_t* vc2 = static_cast<const bf16_t*>(v_second);
 #define KVC_PREFILL(D_, DV_)                                                                                      \
-  return launch_prefill<D_, DV_>(static_cast<bf16_t*>(out), qq, q_stride, kc, vc, table, table_stride, positions, \
+  return launch_prefill<D_, DV_>(static_cast<bf16_t*>(out), qq, q_stride, kc, vc, vc2, table, table_stride, positions, \
                                  q_start, slots, T, R, nh, nkv, page_size, num_pages, scale, window, slopes, chunk, \
                                  sinks, po, pml, nsplit, cos_tab, sin_tab, rot_dim, interleaved, softcap, gate, out_f32, s)
   if (d == 64) {
+    if (two) KVC_PREFILL(64, 128);
     if (dv == d) KVC_PREFILL(64, 64);
     KVC_PREFILL(64, 32);
   }

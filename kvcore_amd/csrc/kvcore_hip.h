@@ -420,10 +420,11 @@ int kvc_decode_attention(void* out, void* part_o, void* part_ml, const void* qkv
 // kernel joins their results; values have dv elements, d or d / 2; part_o [T*nh*nsplit, dv] and part_ml [T*nh*nsplit, 2] float32
 // are its workspace.  With cos_tab and sin_tab [T, rot_dim / 2] the queries come unrotated
 // and are rotated on their way in, as kvc_rope_kv_write would have (rot_dim a multiple of 64,
-// or of 32 when interleaved); without, they are taken as they are.
+// or of 32 when interleaved); without, they are taken as they are.  With v_second values have 128 elements on keys of 64, the
+// first 64 in v_cache and the others in v_second, pages of both alike (no softcap, no gate).
 int kvc_prefill_attention_supported(int nh, int nkv, int d, int dv, int page_size, int dtype);
 int kvc_prefill_attention(void* out, const void* q, int64_t q_stride, const void* k_cache,
-                          const void* v_cache, const int32_t* table, int table_stride,
+                          const void* v_cache, const void* v_second, const int32_t* table, int table_stride,
                           const int32_t* positions, const int32_t* q_start, const int32_t* slots,
                           int T, int R, int nh, int nkv, int d, int dv, int page_size, int num_pages,
                           float scale, int window, const float* slopes, int chunk, const float* sinks, void* part_o,

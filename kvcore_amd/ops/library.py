@@ -95,7 +95,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_decode_attention_waves": [I, I, I],
         "kvc_decode_attention_max_table": [I, I, I],
         "kvc_decode_attention_supported": [I, I, I, I, I, I],
-        "kvc_prefill_attention": [P, P, L, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, P, I, P, P, P, I,
+        "kvc_prefill_attention": [P, P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, P, I, P, P, P, I,
                                   P, P, I, I, F, P, L, I, P],
         "kvc_prefill_attention_supported": [I, I, I, I, I, I],
         "kvc_gemm_mid_slices": [I, I],
@@ -806,6 +806,11 @@ def prefill_attention_supported(nh: int, nkv: int, d: int, page_size: int, dtype
                                                        DTYPE_CODE.get(dtype, -1)))
 
 
+def prefill_attention_two_planes(d: int, plane: int, planes: int) -> bool:
+    """Whether :func:`prefill_attention` takes values of this many planes of this size at once."""
+    return d == 64 and plane == 64 and planes == 2
+
+
 def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       *, table: torch.Tensor, positions: torch.Tensor, q_start: torch.Tensor,
                       slots: torch.Tensor, num_reqs: int, nh: int, nkv: int, d: int, scale: float,
@@ -814,11 +819,12 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                       sin: torch.Tensor | None = None, rot_dim: int = 0, interleaved: bool = False,
                       slopes: torch.Tensor | None = None, chunk: int = 0,
                       sinks: torch.Tensor | None = None, dv: int | None = None, softcap: float = 0.0,
-                      gate: torch.Tensor | None = None) -> None:
+                      gate: torch.Tensor | None = None, v_second: torch.Tensor | None = None) -> None:
     """bfloat16 attention of portions of prompts on the matrix cores (see the C header).
     ``nsplit > 1`` deals every tile's keys to that many blocks; ``part_o`` (float32,
     ``T*nh*nsplit*dv`` values) and ``part_ml`` (``T*nh*nsplit*2``) are then the workspace.
-    ``dv``: the size of a value head, ``d`` (the default) or half of it.  ``softcap`` and ``gate`` as for
+    ``dv``: the size of a value head, ``d`` (the default) or half of it, or with ``v_second`` (a plane like ``v_cache``, which
+    holds the other half of every value head; keys of 64, no cap, no gate) twice.  ``softcap`` and ``gate`` as for
     :func:`paged_attention` (the gate's rows 8-byte aligned).
     With ``cos`` and ``sin`` (``[T, rot_dim / 2]`` float32) the queries come unrotated and
     the kernel rotates them (``prefill_attention_rotates`` says for which shapes)."""
@@ -828,7 +834,9 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         raise KernelError("prefill_attention: out must be contiguous bfloat16 (or float32) [T, nh*dv]")
     if q.shape[0] != T or q.stride(1) != 1 or q.shape[1] < nh * d or q.dtype != torch.bfloat16:
         raise KernelError("prefill_attention: q does not fit")
-    num_pages, page_size = _check_cache(k_cache, v_cache, nkv, d, "prefill_attention", dv)
+    num_pages, page_size = _check_cache(k_cache, v_cache, nkv, d, "prefill_attention", dv if v_second is None else dv // 2)
+    if v_second is not None:
+        _check_cache(k_cache, v_second, nkv, d, "prefill_attention", dv // 2)
     if k_cache.dtype != q.dtype:
         raise KernelError("prefill_attention: cache dtype differs from the queries'")
     if positions.numel() < T or q_start.numel() < num_reqs + 1 or slots.numel() < num_reqs:
@@ -847,7 +855,7 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         cs, sn = _dev(cos, "cos", torch.float32), _dev(sin, "sin", torch.float32)
     _check(load().kvc_prefill_attention(
         out.data_ptr(), q.data_ptr(), q.stride(0), _dev(k_cache, "k_cache"), _dev(v_cache, "v_cache"),
-        _dev(table, "table", torch.int32), table.shape[1], _dev(positions, "positions", torch.int32),
+        None if v_second is None else _dev(v_second, "v_second"), _dev(table, "table", torch.int32), table.shape[1], _dev(positions, "positions", torch.int32),
         _dev(q_start, "q_start", torch.int32), _dev(slots, "slots", torch.int32), T, num_reqs,
         nh, nkv, d, dv, page_size, num_pages, float(scale), int(window), _slopes(slopes, nh), int(chunk),
         _sinks(sinks, nh), po, pml, int(nsplit), cs, sn, int(rot_dim) if cs is not None else 0, int(interleaved),

@@ -380,6 +380,10 @@ class PagedAttention(Mixer):
         if self.v_planes == 1:
             self._attend(attn, qkv, k_cache, v_planes[0], ctx, call, group, cos, sin, rot_dim, interleaved, prepared,
                          q_gain, k_gain, gate if gate_inside else None)
+        elif (ctx.max_query_len > 1 and self.softcap == 0.0 and self._prefill_kernel(group.page_size, qkv.dtype)
+              and ops.prefill_attention_two_planes(self.head_dim, self.v_plane_dim, self.v_planes)):
+            self._attend(attn, qkv, k_cache, v_planes[0], ctx, call, group, cos, sin, rot_dim, interleaved, prepared,
+                         q_gain, k_gain, v_second=v_planes[1])
         else:
             # the same scores against each plane of the values; the planes' results, each [T, heads
             # * plane size], are then laid side by side within every head
@@ -407,8 +411,8 @@ class PagedAttention(Mixer):
         return out
 
     def _attend(self, attn, qkv, k_cache, v_cache, ctx, call, group, cos, sin, rot_dim, interleaved, prepared,
-                q_gain=None, k_gain=None, gate=None):
-        """The attention itself into ``attn [T, heads * plane size]`` over one plane of values,
+                q_gain=None, k_gain=None, gate=None, v_second=None):
+        """The attention itself into ``attn [T, heads * plane size]`` over one plane of values (portions: over two at once),
         by the kernel that serves the step's shape.  ``prepared``: q is ready and the cache is
         written; otherwise the kernels chosen here rotate and write on their way."""
         common = dict(table=group.table, positions=ctx.positions, token_req=ctx.token_req,
@@ -456,23 +460,24 @@ class PagedAttention(Mixer):
                 # portions of prompts (single tokens may ride along): tiles of query rows per
                 # block, and several blocks per tile where few rows meet many keys
                 T = ctx.num_tokens
+                dv = self.v_plane_dim if v_second is None else 2 * self.v_plane_dim
                 nsplit = prefill_splits(T, self.num_kv_heads, self.num_heads // self.num_kv_heads,
                                         ctx.max_query_len, ctx.max_seq_len, reach, ctx.num_reqs)
                 part_o = part_ml = None
                 if nsplit > 1:
                     # asked for at their largest at once: a buffer that grows drops the graphs
                     most = prefill_split_rows(self.num_kv_heads, self.num_heads // self.num_kv_heads) * self.num_heads
-                    part_o = ctx.buffers.get(_sized("attn_prefill_part_o", self.v_plane_dim, self.shared_buffers),
+                    part_o = ctx.buffers.get(_sized("attn_prefill_part_o", dv, self.shared_buffers),
                                              T * self.num_heads * nsplit,
-                                             self.v_plane_dim, torch.float32, reserve=most)
+                                             dv, torch.float32, reserve=most)
                     part_ml = ctx.buffers.get("attn_prefill_part_ml", T * self.num_heads * nsplit, 2,
                                               torch.float32, reserve=most)
                 ops.prefill_attention(attn, qkv, k_cache, v_cache, table=group.table,
                                       positions=ctx.positions, q_start=ctx.q_start, slots=ctx.slots,
                                       num_reqs=ctx.num_reqs, nh=self.num_heads, nkv=self.num_kv_heads,
-                                      d=self.head_dim, dv=self.v_plane_dim, scale=self.scale, window=self.window,
+                                      d=self.head_dim, dv=dv, scale=self.scale, window=self.window,
                                       slopes=self._slopes, chunk=self.chunk, sinks=sinks, softcap=self.softcap, gate=gate,
-                                      nsplit=nsplit, part_o=part_o, part_ml=part_ml,
+                                      nsplit=nsplit, part_o=part_o, part_ml=part_ml, v_second=v_second,
                                       **(dict(cos=cos, sin=sin, rot_dim=rot_dim, interleaved=interleaved)
                                          if rotates else {}))
             else:

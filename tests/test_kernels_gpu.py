@@ -883,6 +883,43 @@ def test_paged_attention_of_float32_over_tiles_of_keys(ops, nh, nkv, d, page, op
     assert torch.equal(run(some), out[some])
 
 
+@pytest.mark.parametrize("nh,nkv,page", [(32, 8, 16), (6, 2, 32), (5, 1, 48)])
+@pytest.mark.parametrize("spans", [[(0, 45), (30, 1), (100, 70)], [(0, 600)], [(700, 20)], [(0, 1500), (5, 1100)]])
+def test_portions_over_two_planes_of_values_at_once(ops, nh, nkv, page, spans):
+    """Values of 128 on keys of 64 in two planes: the bits of a call a plane, under every option that both take, with and
+    without splits, rounded or not."""
+    d, gen = 64, torch.Generator().manual_seed(nh)
+    kc, vc, table, _ = paged_setup([p + n for p, n in spans], nkv, d, page, torch.bfloat16, seed=nh)
+    second = vc * 0.7 + 0.1  # what is not there is no number here either
+    T, R = sum(n for _, n in spans), len(spans)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    q = rnd(T, nh * d, dtype=torch.bfloat16, seed=3)
+    starts = [0]
+    for _, n in spans:
+        starts.append(starts[-1] + n)
+    common = dict(table=table, positions=torch.cat([torch.arange(p, p + n) for p, n in spans]).to(**i32),
+                  q_start=torch.tensor(starts, **i32), slots=torch.arange(1, R + 1, **i32), num_reqs=R, nh=nh, nkv=nkv, d=d,
+                  scale=d ** -0.5)
+    options = [{}, {"window": 50}, {"chunk": 64}, {"sinks": torch.randn(nh, generator=gen).to(DEV)},
+               {"slopes": (torch.rand(nh, generator=gen) * 0.1).to(DEV)}]
+    for option in options:
+        for nsplit in (1, 3):
+            for out_dtype in (torch.bfloat16, torch.float32):
+                def run(planes):
+                    dv = 64 * len(planes)
+                    work = {} if nsplit == 1 else dict(nsplit=nsplit, part_o=torch.empty(T * nh * nsplit, dv, device=DEV),
+                                                       part_ml=torch.empty(T * nh * nsplit, 2, device=DEV))
+                    out = torch.empty(T, nh * dv, dtype=out_dtype, device=DEV)
+                    ops.prefill_attention(out, q, kc, planes[0], dv=dv, v_second=planes[1] if len(planes) > 1 else None,
+                                          **work, **option, **common)
+                    return out.view(T, nh, -1)
+
+                assert torch.equal(run([vc, second]), torch.cat([run([vc]), run([second])], -1)), (option, nsplit)
+    out = torch.empty(T, nh * 128, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ops.KernelError, match="without a cap"):
+        ops.prefill_attention(out, q, kc, vc, dv=128, v_second=second, softcap=2.0, **common)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_paged_attention_finds_one_far_key_among_hundreds(ops, dtype):
     """Random keys would hide a skipped key.  One key (in turn: the first, one at a page's
