@@ -1,0 +1,45 @@
+// Float32 operands of the bfloat16 matrix instructions: each value the sum of three bfloat16 parts, and the six products of
+// parts that float32 can tell, for kernels whose sums must not be less precise than on the float32 matrix instructions.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "gemm_common.h"
+
+namespace kvc {
+
+// Eight float32 values as sums of three bfloat16 values, rounded to nearest one after the other: 24 significand bits
+// in three times eight, so nothing is left over (down to 2^-133, the least that bfloat16 holds).
+struct split_t {
+  bf16x8_t part[3];
+};
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ split_t split8(const f32x4_t* v) {
+  u32x4_t out[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // two values at a time: one conversion makes both halves of a register
+    f32x2_t x = {v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));
+      out[p][i] = bits;
+      if (p < 2) {
+        x[0] -= __uint_as_float(bits << 16);
+        x[1] -= __uint_as_float(bits & 0xffff0000u);
+      }
+    }
+  }
+  split_t s;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) s.part[p] = __builtin_bit_cast(bf16x8_t, out[p]);
+  return s;
+}
+
+// Which parts the six products take, the smallest first (what is left out is below 2^-26 of a product).
+constexpr int kOrder[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+
+}  // namespace kvc

@@ -14,6 +14,7 @@
 #include <cmath>
 
 #include "device_utils.h"
+#include "float_parts.h"
 #include "kvcore_hip.h"
 
 using namespace kvc;
@@ -177,18 +178,15 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
 // a = exp(log a), and the driven input sqrt(1 - a^2) i u, with 1 - a^2 taken as
 // -expm1(2 log a).
 //
-// A wave takes 16 outputs of both matrices x TT tiles of 16 tokens along the whole of a channel
-// block, on the float32 matrix instructions (float32 products, float32 sums), its operands from
-// memory to registers AHEAD chunks of 32 inputs ahead (a lane 32 contiguous bytes).  A result is
-// made in the same order whatever the tile: chunk by chunk, and within one eight 16 x 16 x 4
-// instructions, of which number j takes the inputs k + j, k + 8 + j, k + 16 + j, k + 24 + j.
-// A block's waves are neighbours along the tokens and share the matrices' rows through the
-// cache.  2,048 tokens of 2,560 channels in blocks of 256: 92 us, of which the products take 34
-// at the matrix rate and the exponentials, quotients and roots of the results some 30 (blocks
-// of 16 channels, 38 us); two tiles of outputs or four of tokens a wave 89 to 160 us, with the
-// fewer waves in flight that their registers leave no better over other sizes.  Through LDS with
-// a multiply and an add a step it took 129 us.
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
+// Float32 values as three bfloat16 parts on the bfloat16 matrix instructions (a chunk of 32 inputs six instructions of 16
+// cycles, not eight of 32, and a smaller error: float_parts.h), float32 sums.  A result is made in the same order whatever the
+// tile: two chains, one of the even chunks and one of the odd ones, added at the end; a sum that is not finite is made again
+// in float32, input by input.
+//
+// Many tokens: a wave takes 32 tokens x 32 outputs of both matrices; its tokens' values come straight from memory, the
+// matrices' parts are made by the block's threads and shared through LDS.  2,048 tokens of 2,560 channels in blocks of
+// 256: 99 us on the float32 matrix instructions with 16 outputs a wave, which read the matrices and the tokens twice as often,
+// 55 us this way, of which the exponentials, quotients and roots of the results are some 30.
 constexpr int GT = 16, GK = 32;
 
 // The results for one channel of a token from its two sums (biases added), softplus(lam) and its input.
@@ -209,97 +207,124 @@ __device__ __forceinline__ void gate_load8(f32x4_t* v, const float* row, int k, 
   if (k >= bw) v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 }
 
-template <int TT, int AHEAD>
-__global__ __launch_bounds__(256) void rglru_gates_kernel(
+// acc += the sums over a chunk of one tile of outputs and one of tokens
+__device__ __forceinline__ void gate_multiply(f32x4_t& acc, const bf16x8_t* w, const bf16x8_t* u) {
+#pragma unroll
+  for (int p = 0; p < 6; ++p) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kOrder[p][0]], u[kOrder[p][1]], acc, 0, 0, 0);
+}
+
+// The two sums of a result, again in float32 where one is not finite (an infinity splits into parts that cancel).
+__device__ __forceinline__ void gate_sums_again(float& a, float& i, const float* u, const float* wa, const float* wi, int bw) {
+  if (fmaf(a, 0.f, i * 0.f) == 0.f) return;
+  a = i = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < bw; ++k) {
+    a = fmaf(wa[k], u[k], a);
+    i = fmaf(wi[k], u[k], i);
+  }
+}
+
+constexpr int kGateTokens = 128, kGateOuts = 32;  // of a block of many tokens
+
+__global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
     int bw, int out_tiles, int token_tiles) {
+  __shared__ bf16x8_t w_s[2][2][2][3][64];  // buffer, matrix, tile of outputs, part, lane
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
   const int channel_tile = blockIdx.x / token_tiles;
-  const int token_tile = blockIdx.x - channel_tile * token_tiles;
-  const int t0 = (token_tile * 4 + wave) * 16 * TT;
-  if (t0 >= T) return;
+  const int t0 = (blockIdx.x - channel_tile * token_tiles) * kGateTokens + wave * 32;
   const int blk = channel_tile / out_tiles;
-  const int o0 = (channel_tile - blk * out_tiles) * 16;
-  // outputs and tokens beyond the last read the last one and are not stored
-  const int64_t row = (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
-  const float *wa_row = wa + row, *wi_row = wi + row, *u_row[TT];
+  const int o0 = (channel_tile - blk * out_tiles) * kGateOuts;
+  // outputs and tokens beyond the last read the last one and are not stored; a wave without tokens still shares its part
+  const float* u_row[2];
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
+  for (int t = 0; t < 2; ++t) {
     const int tok = t0 + 16 * t + li;
     u_row[t] = u + static_cast<int64_t>(tok < T ? tok : T - 1) * W + blk * bw;
   }
-  f32x4_t acc_a[TT], acc_i[TT];
+  // the thread's piece of the matrices: eight inputs of one row of one of them
+  const int my_k = 8 * (threadIdx.x & 3), my_row = (threadIdx.x >> 2) & 31, my_mat = threadIdx.x >> 7;
+  const float* w_row = (my_mat ? wi : wa) + (static_cast<int64_t>(blk) * bw + (o0 + my_row < bw ? o0 + my_row : bw - 1)) * bw;
+  const int my_lane = (threadIdx.x & 3) * 16 + (my_row & 15);
+  f32x4_t acc[2][2][2][2];  // chain, matrix, tile of outputs, tile of tokens
 #pragma unroll
-  for (int t = 0; t < TT; ++t) acc_a[t] = acc_i[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  f32x4_t av[AHEAD][2], iv[AHEAD][2], uv[AHEAD][TT][2];
-  auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
-    const int k = k0 + 8 * lk;
-    gate_load8(av[slot], wa_row, k, bw);
-    gate_load8(iv[slot], wi_row, k, bw);
+  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][(i >> 1) & 1][i & 1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t wv[2], uv[2][2];
+  auto fetch = [&](int k0) {  // chunks that are not there arrive as zeros
+    gate_load8(wv, w_row, k0 + my_k, bw);
 #pragma unroll
-    for (int t = 0; t < TT; ++t) gate_load8(uv[slot][t], u_row[t], k, bw);
+    for (int t = 0; t < 2; ++t) gate_load8(uv[t], u_row[t], k0 + 8 * lk, bw);
   };
+  fetch(0);
+  for (int k0 = 0; k0 < bw; k0 += 2 * GK) {
 #pragma unroll
-  for (int s = 0; s < AHEAD; ++s) fetch(s, GK * s);
-  for (int k0 = 0; k0 < bw; k0 += GK * AHEAD) {
+    for (int s = 0; s < 2; ++s) {  // the even chunk and the odd one, each with a buffer and a chain of its own
+      if (k0 + GK * s >= bw) break;  // scalar
+      const split_t w_parts = split8(wv);
 #pragma unroll
-    for (int s = 0; s < AHEAD; ++s) {
-      f32x4_t a_now[2], i_now[2], u_now[TT][2];
+      for (int p = 0; p < 3; ++p) w_s[s][my_mat][my_row >> 4][p][my_lane] = w_parts.part[p];
+      split_t u_parts[2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        a_now[h] = av[s][h];
-        i_now[h] = iv[s][h];
+      for (int t = 0; t < 2; ++t) u_parts[t] = split8(uv[t]);
+      fetch(k0 + GK * (s + 1));
+      __syncthreads();
 #pragma unroll
-        for (int t = 0; t < TT; ++t) u_now[t][h] = uv[s][t][h];
-      }
-      fetch(s, k0 + GK * (s + AHEAD));
+      for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
+        for (int n = 0; n < 2; ++n) {
+          bf16x8_t w[3];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) {
-          acc_a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_a[t], 0, 0, 0);
-          acc_i[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(i_now[j >> 2][j & 3], u_now[t][j >> 2][j & 3], acc_i[t], 0, 0, 0);
+          for (int p = 0; p < 3; ++p) w[p] = w_s[s][m][n][p][lane];
+#pragma unroll
+          for (int t = 0; t < 2; ++t) gate_multiply(acc[s][m][n][t], w, u_parts[t].part);
         }
     }
   }
   // a lane holds token li, outputs 4 lk .. of its tiles
-  const int out = o0 + 4 * lk;
-  if (out >= bw) return;
-  const int c = blk * bw + out;
-  float sp[4], b_a[4], b_i[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    sp[e] = softplus_f(lam[c + e]);
-    b_a[e] = ba[c + e];
-    b_i[e] = bi[c + e];
-  }
+  for (int n = 0; n < 2; ++n) {
+    const int out = o0 + 16 * n + 4 * lk;
+    if (out >= bw) continue;
+    const int c = blk * bw + out;
+    float sp[4], b_a[4], b_i[4];
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    const int tok = t0 + 16 * t + li;
-    if (tok >= T) continue;
-    const int64_t at = static_cast<int64_t>(tok) * W + c;
-    const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(u + at);
-    float a4[4], d4[4];
+    for (int e = 0; e < 4; ++e) {
+      sp[e] = softplus_f(lam[c + e]);
+      b_a[e] = ba[c + e];
+      b_i[e] = bi[c + e];
+    }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) gate_results(a4[e], d4[e], acc_a[t][e] + b_a[e], acc_i[t][e] + b_i[e], sp[e], c_decay, u4[e]);
-    *reinterpret_cast<f32x4_t*>(a_out + at) = f32x4_t{a4[0], a4[1], a4[2], a4[3]};
-    *reinterpret_cast<f32x4_t*>(drive + at) = f32x4_t{d4[0], d4[1], d4[2], d4[3]};
+    for (int t = 0; t < 2; ++t) {
+      const int tok = t0 + 16 * t + li;
+      if (tok >= T) continue;
+      const int64_t at = static_cast<int64_t>(tok) * W + c;
+      const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(u + at);
+      float a4[4], d4[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float sum_a = acc[0][0][n][t][e] + acc[1][0][n][t][e], sum_i = acc[0][1][n][t][e] + acc[1][1][n][t][e];
+        gate_sums_again(sum_a, sum_i, u + at - out, wa + static_cast<int64_t>(c + e) * bw, wi + static_cast<int64_t>(c + e) * bw, bw);
+        gate_results(a4[e], d4[e], sum_a + b_a[e], sum_i + b_i[e], sp[e], c_decay, u4[e]);
+      }
+      *reinterpret_cast<f32x4_t*>(a_out + at) = f32x4_t{a4[0], a4[1], a4[2], a4[3]};
+      *reinterpret_cast<f32x4_t*>(drive + at) = f32x4_t{d4[0], d4[1], d4[2], d4[3]};
+    }
   }
 }
 
-// The same, with the same bits, for few blocks of 16 tokens x 16 outputs: the block's first wave takes one matrix, the
-// second the other, four chunks on their way, and then every thread the results of one channel of one token.  Where one
-// wave made all 256 of them, 8 tokens of 10 blocks of 32 channels took 5.8 us, this way 3.7, of 256 channels 8.2 and 6.1.
+// The same, with the same bits, for few blocks of 16 tokens x 16 outputs: a wave takes one chain of one matrix, four chunks
+// on their way, and then every thread the results of one channel of one token.  Where one wave made all 256 of them, 8
+// tokens of 10 blocks of 32 channels took 5.8 us, so 3.2, of 256 channels 8.2 and 5.1.
 __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
     int bw, int out_tiles, int token_tiles) {
   constexpr int AHEAD = 4, kRow = 20;
-  __shared__ __attribute__((aligned(16))) float sums[2][16 * kRow];
+  __shared__ __attribute__((aligned(16))) float sums[4][16 * kRow];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int channel_tile = blockIdx.x / token_tiles;
   const int t0 = (blockIdx.x - channel_tile * token_tiles) * 16;
@@ -311,10 +336,10 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
   const int c = blk * bw + (mine ? o0 + my_out : 0);
   const int64_t at = static_cast<int64_t>(mine ? t0 + my_tok : 0) * W + c;
   const float sp = softplus_f(lam[c]), b_a = ba[c], b_i = bi[c], my_u = u[at];
-  if (wave < 2) {  // scalar
-    const int li = lane & 15, lk = lane >> 4;
+  {
+    const int li = lane & 15, lk = lane >> 4, odd = wave >> 1;
     // outputs and tokens beyond the last read the last one and are not stored
-    const float* w_row = (wave ? wi : wa) + (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
+    const float* w_row = ((wave & 1) ? wi : wa) + (static_cast<int64_t>(blk) * bw + (o0 + li < bw ? o0 + li : bw - 1)) * bw;
     const float* u_row = u + static_cast<int64_t>(t0 + li < T ? t0 + li : T - 1) * W + blk * bw;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, wv[AHEAD][2], uv[AHEAD][2];
     auto fetch = [&](int slot, int k0) {  // chunks that are not there arrive as zeros
@@ -322,18 +347,14 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
       gate_load8(uv[slot], u_row, k0 + 8 * lk, bw);
     };
 #pragma unroll
-    for (int s = 0; s < AHEAD; ++s) fetch(s, GK * s);
-    for (int k0 = 0; k0 < bw; k0 += GK * AHEAD) {
+    for (int s = 0; s < AHEAD; ++s) fetch(s, GK * (odd + 2 * s));
+    for (int k0 = GK * odd; k0 < bw; k0 += 2 * GK * AHEAD) {
 #pragma unroll
       for (int s = 0; s < AHEAD; ++s) {
-        if (k0 + GK * s >= bw) break;  // scalar
-        f32x4_t w_now[2], u_now[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) w_now[h] = wv[s][h], u_now[h] = uv[s][h];
-        fetch(s, k0 + GK * (s + AHEAD));
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w_now[j >> 2][j & 3], u_now[j >> 2][j & 3], acc, 0, 0, 0);
+        if (k0 + 2 * GK * s >= bw) break;  // scalar
+        const split_t w_now = split8(wv[s]), u_now = split8(uv[s]);
+        fetch(s, k0 + 2 * GK * (s + AHEAD));
+        gate_multiply(acc, w_now.part, u_now.part);
       }
     }
     *reinterpret_cast<f32x4_t*>(sums[wave] + li * kRow + 4 * lk) = acc;  // token li, outputs 4 lk ..
@@ -341,7 +362,9 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
   __syncthreads();
   if (!mine) return;
   const int s = my_tok * kRow + my_out;
-  gate_results(a_out[at], drive[at], sums[0][s] + b_a, sums[1][s] + b_i, sp, c_decay, my_u);
+  float sum_a = sums[0][s] + sums[2][s], sum_i = sums[1][s] + sums[3][s];
+  gate_sums_again(sum_a, sum_i, u + at - (o0 + my_out), wa + static_cast<int64_t>(c) * bw, wi + static_cast<int64_t>(c) * bw, bw);
+  gate_results(a_out[at], drive[at], sum_a + b_a, sum_i + b_i, sp, c_decay, my_u);
 }
 
 // Channel blocks of any width and alignment: 256 threads take 16 tokens x GO outputs and walk the inputs 32 at a time
@@ -947,26 +970,27 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
     return kvc_check_launch("kvc_rglru_gates");
   }
   const int out_tiles = (bw + 15) / 16;
-  // Small blocks or large, whichever an estimate in us says: small ones share the units, a large one has its walk along
-  // the inputs to itself and a second on the same unit costs most of another.  Large / small blocks, both measured:
-  // 10 blocks of 256 channels, 64 tokens, 11.9 / 10.7 us, 100 tokens 14.8 / 15.1, 256 tokens 24.8 / 27.1; one block
-  // of 128, 256 tokens, 10.2 / 4.7, 2,048 tokens 10.7 / 8.1, 4,096 tokens 11.4 / 13.4; 10 blocks of 160, 256 tokens
-  // 13.5 / 14.3, 257 tokens 19.8 / 14.9.
+  // Small blocks or large, whichever an estimate in us says: small ones share the units, of large ones a unit takes one
+  // after the other.  Small / large, both measured: 10 blocks of 256 channels, 100 tokens 14.0 / 17.2, 160 tokens 17.4 / 17.8,
+  // 256 tokens 22.6 / 17.8, 2,048 tokens 147 / 54; 10 blocks of 160, 256 tokens 12.1 / 14.9, 400 tokens 16.2 / 15.6; 10 blocks of
+  // 64, 1,024 tokens 10.8 / 11.9, 2,048 tokens 18.4 / 16.9; one block of 128, 4,096 tokens 12.7 / 13.7; 8 blocks of 512, 64 tokens
+  // 19.7 / 23.8, 100 tokens 30.4 / 26.0.
   const double units = kvc_device_compute_units();
   const int64_t few_blocks = static_cast<int64_t>((T + 15) / 16) * nb * out_tiles;
-  const int64_t big_blocks = static_cast<int64_t>((T + 127) / 128) * nb * out_tiles;
-  const double few_us = 4 + few_blocks / units * (0.6 + 0.0065 * bw);
-  const double big_us = 4 + (0.25 + 0.75 * ceil(big_blocks / units)) * (4.5 + 0.029 * bw);
+  const int big_out_tiles = (bw + kGateOuts - 1) / kGateOuts;
+  const int64_t big_blocks = static_cast<int64_t>((T + kGateTokens - 1) / kGateTokens) * nb * big_out_tiles;
+  const double few_us = 3 + 0.008 * bw + few_blocks / units * (0.4 + 0.0055 * bw);
+  const double big_us = 5.5 + 0.008 * bw + ceil(big_blocks / units) * (4.4 + 0.02 * bw);
   const bool few = few_us <= big_us;
-  const int token_tiles = few ? (T + 15) / 16 : (T + 127) / 128;
+  const int token_tiles = few ? (T + 15) / 16 : (T + kGateTokens - 1) / kGateTokens;
   const int64_t blocks = few ? few_blocks : big_blocks;
   if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");
   if (few)
     hipLaunchKernelGGL(rglru_gates_few_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out, drive,
                        u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles, token_tiles);
   else
-    hipLaunchKernelGGL((rglru_gates_kernel<2, 2>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out,
-                       drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles, token_tiles);
+    hipLaunchKernelGGL(rglru_gates_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out,
+                       drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, big_out_tiles, token_tiles);
   return kvc_check_launch("kvc_rglru_gates");
 }
 

@@ -305,6 +305,28 @@ def test_gates_in_long_portions_are_those_of_short_steps(ops, W, nb):
             assert torch.equal(got, want[first: first + n]), (first, n)
 
 
+@pytest.mark.parametrize("T", [20, 1500])
+def test_gates_of_values_that_are_not_finite_or_tiny(ops, T):
+    """An infinity among a token's values or a matrix's reaches its sums as in float32 (parts of it would cancel to no
+    number), values below what bfloat16 parts can hold leave finite results, and other rows are as if alone."""
+    W, nb = 512, 2
+    bw = W // nb
+    u = rnd(T, W, seed=1)
+    u[3, 5], u[4, 300], u[5] = float("inf"), float("nan"), 1e-39
+    d = [rnd(nb, bw, bw, seed=s, std=bw ** -0.5) for s in (2, 3)]
+    d[0][0, 7, 9] = float("-inf")
+    d += [rnd(nb, bw, seed=4), rnd(nb, bw, seed=5), rnd(W, seed=6)]
+    a, drive = torch.empty(T, W, device=DEV), torch.empty(T, W, device=DEV)
+    ops.rglru_gates(a, drive, u.to(DEV), *(t.to(DEV) for t in d), 8.0)
+    ud = u.double().view(T, nb, bw)
+    r, g = (torch.sigmoid((torch.stack([ud[:, i] @ w[i].double().T for i in range(nb)], 1) + b.double()).view(T, W))
+            for w, b in ((d[0], d[2]), (d[1], d[3])))
+    log_a = -8.0 * r * torch.nn.functional.softplus(d[4].double())
+    want_a, want_d = log_a.exp(), torch.sqrt(-torch.expm1(2 * log_a)) * g * u.double()
+    for got, want in ((a, want_a), (drive, want_d)):
+        assert torch.allclose(got.double().cpu(), want, atol=1e-5, rtol=1e-5, equal_nan=True)
+
+
 def test_long_portions_are_scanned_in_segments_side_by_side(ops):
     """With a workspace, requests longer than a segment are cut into segments that are scanned
     side by side and joined in order: the same results, whatever the portions, beside short
