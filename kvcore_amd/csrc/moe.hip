@@ -433,8 +433,10 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
   }
   __syncthreads();
   // an expert's rows in as few tiles as hold them, all of about one size (in sixteens): no tile is left with a few
+  const bool wide = tile_rows == kWideTileRows;  // the others are powers of two
+  const int shift = 31 - __clz(tile_rows);
   auto rows_each = [&](int n) {
-    const int tiles_of = (n + tile_rows - 1) / tile_rows;
+    const int tiles_of = wide ? (n + kWideTileRows - 1) / kWideTileRows : (n + tile_rows - 1) >> shift;
     return tiles_of < 2 ? tile_rows : ((n + tiles_of - 1) / tiles_of + 15) & ~15;
   };
   auto list = [&](int e, int n, int each, int at, int nt) {
@@ -461,16 +463,18 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
       }
       if (e == E - 1) *num_tiles = nt < max_tiles ? nt : max_tiles;
       nt -= mine;
-      if (tile_rows == kWideTileRows) {
+      if (wide) {
         // Blocks of tiles of up to 384 rows have a compute unit to themselves: experts with more rows a tile come first (the
         // lower index among equals), each one's tiles side by side, so that the last blocks the chip takes up are the short
         // ones.  Smaller tiles fetch weights in the experts' order (8 rows an expert, 32 gated experts of 2048 x 2048 in
         // tiles of 64 rows: 95.3 us, in the other order 98.3).
-        const int rows = n < each ? n : each;
+        const int key = (n < each ? n : each) * kWave + kWave - 1 - e;
         nt = 0;
-        for (int p = 0; p < E; ++p) {
-          const int pt = __builtin_amdgcn_readlane(mine, p), pr = __builtin_amdgcn_readlane(rows, p);
-          nt += pr > rows || (pr == rows && p < e) ? pt : 0;
+#pragma unroll
+        for (int p = 0; p < kWave; ++p) {  // lanes beyond E have no tiles
+          if (p == kWave / 2 && E <= kWave / 2) break;  // scalar
+          const int pt = __builtin_amdgcn_readlane(mine, p);
+          nt += __builtin_amdgcn_readlane(key, p) > key ? pt : 0;
         }
       }
       if (e < E) list(e, n, each, at - n, nt);
