@@ -309,6 +309,25 @@ def test_the_layers_run_the_kernels_they_are_meant_to(models):
             setattr(ops, n, fn)
 
 
+@pytest.mark.parametrize("first", [95, 96])
+def test_two_planes_of_values_on_either_side_of_their_line(models, monkeypatch, first):
+    """The layer whose values lie in two planes takes a launch a plane below the line and one for both from there on: the
+    oracle's logits either way, also for the shorter portion behind."""
+    from kvcore_amd.ops import library as ops
+    from kvcore_amd.parts.attention import TWO_PLANES_TOKENS
+
+    assert TWO_PLANES_TOKENS == 96
+    folder, cfg, weights, page = models["B"]
+    seconds: list = []
+    real = ops.prefill_attention
+    monkeypatch.setattr(ops, "prefill_attention",
+                        lambda *a, **k: (seconds.append(k.get("v_second") is not None), real(*a, **k))[1])
+    tokens = random_tokens(first + 20, cfg["vocab"], 9)
+    got = replay(session_for(folder, torch.bfloat16, page, 128), {"a": tokens}, [[("a", first)], [("a", 20)]])
+    compare(got, {"a": oracle(f"planes {first}", cfg, weights, tokens, torch.bfloat16)}, torch.bfloat16, excused=10)
+    assert sum(seconds) == (first >= 96) and len(seconds) == (15 if first >= 96 else 16)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
 @pytest.mark.parametrize("name", ["A", "B", "C"])
 def test_greedy_generation_through_the_engine(models, name, dtype):
