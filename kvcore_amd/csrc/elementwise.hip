@@ -256,13 +256,12 @@ __device__ __forceinline__ void store8(float* p, const float* v) {
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
   *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
 }
+// (the conversion in hardware: to nearest, ties to even, as f32_to_bf16_bits)
 __device__ __forceinline__ void store8(bf16_t* p, const float* v) {
-  uint4 a;
-  a.x = f32_to_bf16_bits(v[0]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[1])) << 16);
-  a.y = f32_to_bf16_bits(v[2]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[3])) << 16);
-  a.z = f32_to_bf16_bits(v[4]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[5])) << 16);
-  a.w = f32_to_bf16_bits(v[6]) | (static_cast<uint32_t>(f32_to_bf16_bits(v[7])) << 16);
-  *reinterpret_cast<uint4*>(p) = a;
+  typedef float f32x8_t __attribute__((ext_vector_type(8)));
+  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+  const f32x8_t x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+  *reinterpret_cast<bf16x8_t*>(p) = __builtin_convertvector(x, bf16x8_t);
 }
 
 template <typename T, int NCH>
@@ -509,19 +508,21 @@ __global__ void silu_mul_kernel(T* __restrict__ out, const T* __restrict__ gate_
   out[idx] = from_float<T>(gate_join(g, u, rule));
 }
 
+// Eight channels a thread.  A launch has fewer than 2^32 threads, so the token is found in 32 bits: that division in 64 bits and
+// the one in the gate held the pass back (2,048 rows of 8,192 channels 21.1 us, this way 18.7; of 14,336 channels 33 and 29; their
+// bytes alone: 16 and 27).
 template <typename T>
-__global__ void silu_mul_vec_kernel(T* __restrict__ out, const T* __restrict__ gate_up, int I8,
-                                    int64_t n8, GateRule rule) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void silu_mul_vec_kernel(T* __restrict__ out, const T* __restrict__ gate_up, uint32_t I8,
+                                                           uint32_t n8, GateRule rule) {
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
   if (idx >= n8) return;
-  const int64_t t = idx / I8;
-  const int64_t i = (idx - t * I8) * 8;
-  const int64_t I = static_cast<int64_t>(I8) * 8;
+  const uint32_t row = idx / I8;
+  const int64_t t = row, I = static_cast<int64_t>(I8) * 8, i = static_cast<int64_t>(idx - row * I8) * 8;
   float g[8], u[8], y[8];
   load8(gate_up + t * 2 * I + i, g);
   load8(gate_up + t * 2 * I + I + i, u);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) y[e] = gate_join(g[e], u[e], rule);
+  for (int e = 0; e < 8; ++e) y[e] = gate_join<true>(g[e], u[e], rule);
   store8(out + t * I + i, y);
 }
 
@@ -537,14 +538,14 @@ extern "C" int kvc_gate_mul(void* out, const void* gate_up, int T, int I, int ac
   const GateRule rule{act, limit, alpha, up_shift};
   const int64_t n = static_cast<int64_t>(T) * I;
   if (n == 0) return 0;
+  const int64_t n8 = n / 8, vblocks = (n8 + 255) / 256;
   if (I % 8 == 0 && (reinterpret_cast<uintptr_t>(out) % 16) == 0 &&
       (reinterpret_cast<uintptr_t>(gate_up) % 16) == 0) {
-    const int64_t n8 = n / 8;
-    const unsigned vblocks = static_cast<unsigned>((n8 + 255) / 256);
+    if (vblocks >= int64_t{1} << 24) return kvc_fail("kvc_gate_mul: more values than one launch takes");
     KVC_DISPATCH_DTYPE(dtype, Tp,
-                       hipLaunchKernelGGL(silu_mul_vec_kernel<Tp>, dim3(vblocks), dim3(256), 0,
-                                          S(stream), static_cast<Tp*>(out),
-                                          static_cast<const Tp*>(gate_up), I / 8, n8, rule));
+                       hipLaunchKernelGGL(silu_mul_vec_kernel<Tp>, dim3(static_cast<unsigned>(vblocks)), dim3(256), 0,
+                                          S(stream), static_cast<Tp*>(out), static_cast<const Tp*>(gate_up),
+                                          static_cast<uint32_t>(I / 8), static_cast<uint32_t>(n8), rule));
     return kvc_check_launch("kvc_gate_mul");
   }
   const unsigned blocks = static_cast<unsigned>((n + 255) / 256);

@@ -794,17 +794,6 @@ __device__ __forceinline__ TilePlace place(int id, int tiles, int cols) {
   const int col = at / tiles;
   return {at - col * tiles, col};
 }
-// clamped_glu with the division as a reciprocal and one correction of the quotient: within a rounding of the quotient in
-// float32, a third of the instructions of the division that is rounded correctly, of which a block of 256 x 128 gated values
-// took 6 us.
-__device__ __forceinline__ float tile_glu(float g, float u, float limit, float alpha, float shift) {
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  const float d = 1.f + expf(-alpha * g);
-  const float r = __builtin_amdgcn_rcpf(d), q = g * r, left = fmaf(-d, q, g);
-  return (left == left ? fmaf(left, r, q) : q) * (u + shift);  // no number where q or d is infinite: q is right then
-}
-
 // The way out of a tile's sums: lane (li, lk) holds NR rows (`row_of`) and of each NF times four columns from n + 16 f on.
 // The pairs and scales of all rows are asked for before the first store: a load behind it would wait for the store too,
 // which cost a block of 256 rows 9 us.
@@ -837,7 +826,7 @@ __device__ __forceinline__ void store_tile(TO* out, int64_t out_stride, RowOf ro
       const f32x4_t v2 = acc2_of(f, r);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        v[i] = GATED ? tile_glu(v[i] * scale[r], v2[i] * scale[r], limit, alpha, shift) : plain_act(v[i] * scale[r], act);
+        v[i] = GATED ? clamped_glu<true>(v[i] * scale[r], v2[i] * scale[r], limit, alpha, shift) : plain_act(v[i] * scale[r], act);
       if (n + 16 * f >= N) continue;
       if (whole) {
         store4_whole(to + 16 * f, v);

@@ -87,6 +87,25 @@ def test_silu_mul(ops, dtype):
     assert torch.allclose(out.double(), plain.silu_and_mul(gu.double()), **tol(dtype))
 
 
+@pytest.mark.parametrize("T,I", [(1, 8), (3, 24), (257, 8), (2, 2056), (65, 1408)])
+def test_gates_of_any_size_eight_channels_a_thread(ops, T, I):
+    """float32 against 64 bits: the quotient (half an ulp and the ties that the reciprocal's correction misses), the
+    exponential (an ulp, and |g| halves of one from the rounding of its argument where it counts) and two products: 6 ulp.
+    Gates beyond the exponential's range give zero (below 1e-35), the gate itself or no number, as the formula does."""
+    gu = rnd(T, 2 * I, dtype=torch.float32, seed=T) * 4
+    far = torch.tensor([-200.0, -88.6, -87.9, 88.6, 200.0, float("inf"), float("-inf"), float("nan")], device=DEV)
+    gu[T - 1, I - 8: I] = far
+    gu[T - 1, 2 * I - 8:] = 1.5
+    out = torch.empty(T, I, device=DEV)
+    ops.silu_mul(out, gu)
+    g, u = gu.double().chunk(2, -1)
+    want = g * torch.sigmoid(g) * u
+    want[T - 1, I - 2] = float("nan")  # -inf times zero
+    near = torch.where(g.abs() < 1e30, g.abs(), torch.zeros_like(g))
+    ok = (out.double() - want).abs() <= (6 + near.clamp(max=100)) * 2.0 ** -24 * want.abs() + 1e-35
+    assert bool((ok | (out.double() == want) | (out.isnan() & want.isnan())).all())
+
+
 def test_gather_rows_and_to_float(ops):
     src = rnd(10, 50)
     rows = torch.tensor([9, 0, 3, 3], dtype=torch.int32, device=DEV)
