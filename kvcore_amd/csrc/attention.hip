@@ -1,6 +1,7 @@
-// Paged attention, general kernel: one 64-lane wave per (token, query head).
+// Paged attention: float32 heads of 64 and 128 in tiles of keys (paged_attention_tiles_kernel below), and the general
+// kernel, one 64-lane wave per (token, query head).
 //
-// Serves every batch shape (portions of prompts beside single decoded tokens), both
+// The general kernel serves every batch shape (portions of prompts beside single decoded tokens), both
 // storage types and every head size up to 512 (heads above 256 in instances of their own).  A token at
 // position p reads keys first..p of its request through the block table, 64 keys a
 // tile: each lane scores one key (a float32 dot product over the head in index

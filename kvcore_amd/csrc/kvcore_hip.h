@@ -23,7 +23,8 @@ int kvc_compute_units(void);
 // "prefill_attention_kernel<128,1,8,8> x1" (head size, column tiles, key blocks a tile, waves,
 // then the number of splits) or "rope_kv_write_tile_kernel"; "" if the family has not been
 // launched.  Families: 0 attention over portions of prompts, 1 rotation with the cache write, 2
-// attention of single tokens, 3 experts' products in bfloat16 over tiles of 16 rows.
+// attention of single tokens, 3 experts' products in bfloat16 over tiles of 16 rows, 4
+// paged attention (the one-wave kernel or tiles of keys).
 const char* kvc_last_variant(int family);
 
 // Measurement only (peaks.hip).  kvc_peak_read: `blocks` blocks of 256 threads read `bytes` bytes
