@@ -1,5 +1,6 @@
-// Float32 operands of the bfloat16 matrix instructions: each value the sum of three bfloat16 parts, and the six products of
-// parts that float32 can tell, for kernels whose sums must not be less precise than on the float32 matrix instructions.
+// Float32 operands of the bfloat16 matrix instructions: each value the sum of three bfloat16 parts, and six of the nine products
+// of parts, for kernels whose sums must not be less precise than on the float32 matrix instructions.  (Splitting a number
+// into parts of a shorter format goes back to Dekker 1971; with bfloat16 parts: Henry, Tang and Heinecke 2019.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -10,8 +11,14 @@
 
 namespace kvc {
 
-// Eight float32 values as sums of three bfloat16 values, rounded to nearest one after the other: 24 significand bits
-// in three times eight, so nothing is left over (down to 2^-133, the least that bfloat16 holds).
+// Eight float32 values times 2^16 as sums of three bfloat16 values, rounded to nearest one after the other: 24 significand bits
+// in three times eight, and the least bit of float32, 2^-149, comes to the least of bfloat16, 2^-133, so nothing is left over
+// of any value below 2^111.  (Without the factor values below 2^-110 lost bits, which a large value on the other side
+// showed: 1e-38 x 1e36 was off by 3e-3.  The factor costs 122 rows of 16384 x 2048 67 -> 70 us; with v_dot2c_f32_bf16, which takes
+// out a part and subtracts it in one instruction and gives the same bits, they took 74.)  Sums of products are to be
+// multiplied by kPartsUnscale; what goes beyond float32 on the way, operands from 2^111 or sums from 2^96 on, comes out as no
+// finite number and is to be summed again without parts.
+constexpr float kPartsScale = 0x1p16f, kPartsUnscale = 0x1p-32f;
 struct split_t {
   bf16x8_t part[3];
 };
@@ -22,7 +29,7 @@ __device__ __forceinline__ split_t split8(const f32x4_t* v) {
   u32x4_t out[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {  // two values at a time: one conversion makes both halves of a register
-    f32x2_t x = {v[i >> 1][2 * (i & 1)], v[i >> 1][2 * (i & 1) + 1]};
+    f32x2_t x = {v[i >> 1][2 * (i & 1)] * kPartsScale, v[i >> 1][2 * (i & 1) + 1] * kPartsScale};
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       const uint32_t bits = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2_t));

@@ -1,5 +1,5 @@
 // C[M, N] = A[M, K] * W[N, K]^T (+ bias) in float32, its products on the bfloat16 matrix instructions: an operand is
-// the sum of three bfloat16 values, and the six products of parts that float32 can tell are added up in float32.  That
+// the sum of three bfloat16 values, and the six largest products of parts are added up in float32 (float_parts.h).  That
 // is no mode of reduced precision: over 1 to 2,048 rows and K of 64 to 8,192 the error against 64 bits is 0.43 to 0.89 of
 // what the float32 matrix instructions leave (122 rows of 16384 x 2048: 2.4e-7 and 2.9e-7 of the result, of 2048 x 8192
 // 5.1e-7 and 5.7e-7), and a chunk of 32 values takes 96 cycles of a matrix core, not 256.
@@ -55,8 +55,7 @@ __device__ __forceinline__ void load8(f32x4_t* v, const float* row, int k, int K
   }
 }
 
-// acc += the sums over a chunk of w x a, the smallest of the six products that float32 can tell first (what is left
-// out is below 2^-26 of a product).
+// acc += the sums over a chunk of w x a, the smallest of the six products first.
 template <int NT, int MT>
 __device__ __forceinline__ void multiply(f32x4_t (&acc)[NT][MT], const split_t* w, const split_t* a) {
 #pragma unroll
@@ -68,22 +67,21 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[NT][MT], const split_t* 
         acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n].part[kOrder[p][0]], a[m].part[kOrder[p][1]], acc[n][m], 0, 0, 0);
 }
 
-// Four sums that lie side by side in C, as they leave.  A value beyond float32, an infinity or a NaN among the operands
-// leaves a sum that is not finite, and operands below 2^-110 lose what bfloat16 cannot hold (what is below 2^-134), of
-// which sums below 2^-90 could tell: such an element is summed again, in index order with fused multiply-adds.  A sum of
-// zero stays, so that rows and weights of zeros cost nothing.
+// Four sums of parts' products that lie side by side in C, as they leave.  A value beyond what the parts hold, an infinity or a
+// NaN among the operands leaves a sum that is not finite: such an element is summed again, in index order with fused
+// multiply-adds.
 __device__ __forceinline__ void leave(f32x4_t v, float* __restrict__ C, const float* __restrict__ A,
                                       const float* __restrict__ W, const float* __restrict__ bias, int row, int col, int N,
                                       int K, int64_t lda, int64_t ldc) {
+  v *= kPartsUnscale;
   // 0 x each: a NaN unless all are finite
   const float none = fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f)));
-  const float least = fminf(fminf(fabsf(v[0]), fabsf(v[1])), fminf(fabsf(v[2]), fabsf(v[3])));
-  if (none != none || least < 0x1p-90f) {
+  if (none != none) {
 #pragma unroll 1
     for (int i = 0; i < 4; ++i) {
       float x = v[0];  // by hand: a register is not indexed
       x = i == 1 ? v[1] : i == 2 ? v[2] : i == 3 ? v[3] : x;
-      if (col + i < N && (!(fabsf(x) < INFINITY) || (x != 0.f && fabsf(x) < 0x1p-90f))) {
+      if (col + i < N && !(fabsf(x) < INFINITY)) {
         const float* a = A + static_cast<int64_t>(row) * lda;
         const float* w = W + static_cast<int64_t>(col + i) * K;
         x = 0.f;
@@ -249,11 +247,12 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
 // [chain][M][round4(N)] for gemm_f32_parts_kernel.  The bits are those of the kernels above.
 //
 // Bound by the matrix and the vector instructions of a wave together (a step of 4 x 2 tiles is 48 matrix instructions of
-// 16 cycles beside the split of 24 values a lane, 5.5 instructions each; with every operand hot in the cache the kernel is
+// 16 cycles beside the split of 24 values a lane, 6.5 instructions each; with every operand hot in the cache the kernel is
 // 5 to 10% faster, no more).  With the float32 matrix instructions on operands straight from the cache and now: 122 rows of
-// 16384 x 2048 115 and 64 us (128 TFLOP/s), of 2048 x 8192 62 and 39, of 3072 x 2048 35 and 24, of 2048 x 2048 18.9 and 16.9;
-// 1,000 rows of 2048 x 2048 110 and 58, 2,048 rows of 16384 x 2048 1,668 and 824 (167 TFLOP/s).  Tiles of 128 rows and one
-// column block a wave read LDS twice as often: 74, 38, 24, 18, 68 and 860 us.
+// 16384 x 2048 115 and 70 us (117 TFLOP/s), of 2048 x 8192 62 and 40, of 3072 x 2048 35 and 25, of 2048 x 2048 18.9 and 17.9;
+// 1,000 rows of 2048 x 2048 110 and 69, 2,048 rows of 16384 x 2048 1,668 and 834 (165 TFLOP/s).  Tiles of 128 rows and one
+// column block a wave read LDS twice as often: 74, 38, 24, 18, 68 and 860 us before an operand's factor (float_parts.h), where
+// these took 64, 39, 24, 17, 58 and 824.
 template <int MT, int NT, bool LEAVE>
 __global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
     float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,

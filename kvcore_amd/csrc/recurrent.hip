@@ -305,7 +305,8 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
       float a4[4], d4[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float sum_a = acc[0][0][n][t][e] + acc[1][0][n][t][e], sum_i = acc[0][1][n][t][e] + acc[1][1][n][t][e];
+        float sum_a = (acc[0][0][n][t][e] + acc[1][0][n][t][e]) * kPartsUnscale;
+        float sum_i = (acc[0][1][n][t][e] + acc[1][1][n][t][e]) * kPartsUnscale;
         gate_sums_again(sum_a, sum_i, u + at - out, wa + static_cast<int64_t>(c + e) * bw, wi + static_cast<int64_t>(c + e) * bw, bw);
         gate_results(a4[e], d4[e], sum_a + b_a[e], sum_i + b_i[e], sp[e], c_decay, u4[e]);
       }
@@ -362,7 +363,7 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
   __syncthreads();
   if (!mine) return;
   const int s = my_tok * kRow + my_out;
-  float sum_a = sums[0][s] + sums[2][s], sum_i = sums[1][s] + sums[3][s];
+  float sum_a = (sums[0][s] + sums[2][s]) * kPartsUnscale, sum_i = (sums[1][s] + sums[3][s]) * kPartsUnscale;
   gate_sums_again(sum_a, sum_i, u + at - (o0 + my_out), wa + static_cast<int64_t>(c) * bw, wi + static_cast<int64_t>(c) * bw, bw);
   gate_results(a_out[at], drive[at], sum_a + b_a, sum_i + b_i, sp, c_decay, my_u);
 }

@@ -327,6 +327,25 @@ def test_gates_of_values_that_are_not_finite_or_tiny(ops, T):
         assert torch.allclose(got.double().cpu(), want, atol=1e-5, rtol=1e-5, equal_nan=True)
 
 
+@pytest.mark.parametrize("T", [20, 1500])
+@pytest.mark.parametrize("tiny,large", [(1e-37, 1e36), (1e-41, 1e32)])
+def test_gates_of_tiny_values_behind_large_matrices(ops, T, tiny, large):
+    """Values that bfloat16 holds in part only, or not at all, times matrices that make ordinary sums of them."""
+    W, nb = 512, 2
+    bw = W // nb
+    u = rnd(T, W, seed=1, std=tiny)
+    d = [rnd(nb, bw, bw, seed=s, std=large * bw ** -0.5) for s in (2, 3)]
+    d += [rnd(nb, bw, seed=4), rnd(nb, bw, seed=5), rnd(W, seed=6)]
+    a, drive = torch.empty(T, W, device=DEV), torch.empty(T, W, device=DEV)
+    ops.rglru_gates(a, drive, u.to(DEV), *(t.to(DEV) for t in d), 8.0)
+    ud = u.double().view(T, nb, bw)
+    r, g = (torch.sigmoid((torch.stack([ud[:, i] @ w[i].double().T for i in range(nb)], 1) + b.double()).view(T, W))
+            for w, b in ((d[0], d[2]), (d[1], d[3])))
+    log_a = -8.0 * r * torch.nn.functional.softplus(d[4].double())
+    close(a, log_a.exp(), 1e-5)
+    close(drive, torch.sqrt(-torch.expm1(2 * log_a)) * g * u.double(), 2.0 ** -148)
+
+
 def test_long_portions_are_scanned_in_segments_side_by_side(ops):
     """With a workspace, requests longer than a segment are cut into segments that are scanned
     side by side and joined in order: the same results, whatever the portions, beside short

@@ -207,10 +207,8 @@ def test_gemm_f32_of_values_at_the_ends_of_float32(ops, M, N, K):
     def check(a, w):
         ops.gemm_f32(out, a, w, None)
         want = a.double() @ w.double().T
-        # plus what float32 cannot hold of a product or a sum of subnormal size; operands are held to 2^-134 (subnormals that
-        # bfloat16 does not have) where the sum comes out as zero
+        # plus what float32 cannot hold of a product or a sum of subnormal size
         bound = 4 * math.sqrt(K) * 2 ** -24 * (a.double().abs() @ w.double().abs().T) + K * 2.0 ** -149
-        bound += (out == 0) * 2.0 ** -134 * (a.double().abs().sum(1)[:, None] + w.double().abs().sum(1)[None])
         assert torch.equal(out.isnan(), want.isnan())
         inf = want.abs() > 3.40282351e38
         assert torch.equal(out.isinf(), inf) and torch.equal(out[inf].sign().double(), want[inf].sign())
@@ -225,11 +223,13 @@ def test_gemm_f32_of_values_at_the_ends_of_float32(ops, M, N, K):
         if M < 100:
             y[N // 3, 0] = value
             check(a.clamp(-0.5, 0.5), y * torch.where(y.abs() > 1e30, 1.0, 1e-3))
-    if M < 100:  # products and sums of subnormal size, and operands that bfloat16 holds in part only
-        check(a * 1e-37, w)
-        check(a * 1e-30, w * 1e-8)
-        check(a * 1e-42, w)
-        check(a * 1e-20, w * 1e-25)
+    # products and sums of subnormal size, operands that bfloat16 holds in part only or not at all, and such operands times
+    # large ones, whose sums are ordinary numbers
+    for x, y in ((1e-37, 1), (1e-30, 1e-8), (1e-42, 1), (1e-20, 1e-25), (1e-37, 1e20), (1e-36, 1e30), (1e-38, 1e32), (1e-42, 1e32)):
+        check(a * x, w * y)
+        check(a * y, w * x)
+    few = torch.arange(N, device=DEV)[:, None] % 3 == 0  # beside columns of ordinary values
+    check(a * 1e-38, torch.where(few, w * 1e31, w))
     check(torch.zeros_like(a), w)
 
 
