@@ -233,6 +233,18 @@ def test_gemm_f32_of_values_at_the_ends_of_float32(ops, M, N, K):
     check(torch.zeros_like(a), w)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 8), (20, 40, 100), (40, 70, 512), (122, 2048, 2048), (2100, 1100, 64)])
+def test_gemm_f32_of_the_products_whose_parts_leave_most_out(ops, M, N, K):
+    """Operands of one size and sign whose left-out products of parts are as large as they get, 2^-24 of the product."""
+    value = 0x100ff8 / 0x100000
+    out = torch.empty(M, N, device=DEV)
+    ops.gemm_f32(out, torch.full((M, K), value, device=DEV), torch.full((N, K), value, device=DEV), None)
+    # 2^-24 of each product, and one rounding of at most 2^-24 of the sum so far for each of a chunk's six instructions
+    # along a chain, and for each of the chains' eight sums
+    steps = 1 + 6 * -(-K // 256) + 8
+    assert ((out.double() - K * value * value).abs() <= steps * 2 ** -24 * K * value * value).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (5, 100, 200), (8, 4096, 4096), (16, 130, 1032),
                                    (17, 6144, 512), (33, 48, 14336), (64, 1000, 2048),
                                    # the longest sum and the widest output of the 70B shape
