@@ -67,33 +67,38 @@ __device__ __forceinline__ void multiply(f32x4_t (&acc)[NT][MT], const split_t* 
         acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n].part[kOrder[p][0]], a[m].part[kOrder[p][1]], acc[n][m], 0, 0, 0);
 }
 
-// Four sums of parts' products that lie side by side in C, as they leave.  A value beyond what the parts hold, an infinity or a
-// NaN among the operands leaves a sum that is not finite: such an element is summed again, in index order with fused
-// multiply-adds.
-__device__ __forceinline__ void leave(f32x4_t v, float* __restrict__ C, const float* __restrict__ A,
+// Four sums of parts' products that lie side by side in C, as they leave; every lane of a wave comes here, `live` or not.  A value
+// beyond what the parts hold, an infinity or a NaN among the operands leaves a sum that is not finite: such an element is
+// summed again by the wave, or, where its row holds a NaN (which is looked up once a row), is one.
+__device__ __forceinline__ void leave(bool live, f32x4_t v, float* __restrict__ C, const float* __restrict__ A,
                                       const float* __restrict__ W, const float* __restrict__ bias, int row, int col, int N,
                                       int K, int64_t lda, int64_t ldc) {
   v *= kPartsUnscale;
   // 0 x each: a NaN unless all are finite
   const float none = fmaf(v[0], 0.f, fmaf(v[1], 0.f, fmaf(v[2], 0.f, v[3] * 0.f)));
-  if (none != none) {
-#pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-      float x = v[0];  // by hand: a register is not indexed
-      x = i == 1 ? v[1] : i == 2 ? v[2] : i == 3 ? v[3] : x;
-      if (col + i < N && !(fabsf(x) < INFINITY)) {
-        const float* a = A + static_cast<int64_t>(row) * lda;
-        const float* w = W + static_cast<int64_t>(col + i) * K;
-        x = 0.f;
-#pragma unroll 1
-        for (int k = 0; k < K; ++k) x = fmaf(a[k], w[k], x);
+  uint64_t todo = __ballot(live && none != none);
+  while (todo != 0) {  // scalar, as all that decides here
+    const int r = __builtin_amdgcn_readlane(row, __builtin_ctzll(todo));
+    const float* a = A + static_cast<int64_t>(r) * lda;
+    const bool nan = wave_holds_nan(a, K);
+    uint64_t same = __ballot(row == r) & todo;
+    todo &= ~same;
+    for (; same != 0; same &= same - 1) {
+      const int lane = __builtin_ctzll(same), c = __builtin_amdgcn_readlane(col, lane);
+      float sum[4] = {NAN, NAN, NAN, NAN};
+      if (!nan) {
+        const float* w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = W + static_cast<int64_t>(c + i < N ? c + i : N - 1) * K;
+        wave_products<4>(sum, a, w, K);
       }
-      v[0] = i == 0 ? x : v[0];
-      v[1] = i == 1 ? x : v[1];
-      v[2] = i == 2 ? x : v[2];
-      v[3] = i == 3 ? x : v[3];
+      if ((threadIdx.x & 63) == lane) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = fabsf(v[i]) < INFINITY ? v[i] : sum[i];
+      }
     }
   }
+  if (!live) return;
   if (bias != nullptr) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] += bias[col + i < N ? col + i : N - 1];
@@ -166,7 +171,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict
 #pragma unroll
       for (int w = 1; w < kWaves; ++w) v += part[w][m][l];
       const int row = m0 + 16 * m + (l & 15), col = n0 + 16 * n + 4 * (l >> 4);
-      if (row < M && col < N) leave(v, C, A, W, bias, row, col, N, K, lda, ldc);
+      leave(row < M && col < N, v, C, A, W, bias, row, col, N, K, lda, ldc);
     }
   }
 }
@@ -230,11 +235,10 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     const int row = m0 + 16 * m + li;
-    if (row >= M) continue;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const int col = n0 + 16 * n + 4 * lk;
-      if (col < N) leave(sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
+      leave(row < M && col < N, sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
     }
   }
 }
@@ -369,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const int col = n0 + 16 * n + 4 * lk;
-      if (row < M && col < N) leave(sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
+      leave(row < M && col < N, sum[n][m], C, A, W, bias, row, col, N, K, lda, ldc);
     }
   }
 }
@@ -381,9 +385,9 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(float* __restrict__
                                                              int64_t lda, int64_t ldc) {
   const int quads = (N + 3) >> 2;
   const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (idx >= static_cast<int64_t>(M) * quads) return;
+  const bool live = idx < static_cast<int64_t>(M) * quads;
   const int row = static_cast<int>(idx / quads), col = 4 * static_cast<int>(idx - static_cast<int64_t>(row) * quads);
-  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(parts) + idx;
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(parts) + (live ? idx : 0);
   const int64_t step = static_cast<int64_t>(M) * quads;
   f32x4_t v[kWaves];
 #pragma unroll
@@ -391,7 +395,7 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(float* __restrict__
 #pragma unroll
   for (int w = 1; w < kWaves; ++w)
     if (w < chains) v[0] += v[w];  // scalar
-  leave(v[0], C, A, W, bias, row, col, N, K, lda, ldc);
+  leave(live, v[0], C, A, W, bias, row, col, N, K, lda, ldc);
 }
 
 // How the sizes of a call are dealt out to the kernel with rows in LDS: column blocks of 16 a wave, chains to how many

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
 // Float32 values as three bfloat16 parts on the bfloat16 matrix instructions (a chunk of 32 inputs six instructions of 16
 // cycles, not eight of 32, and a smaller error: float_parts.h), float32 sums.  A result is made in the same order whatever the
 // tile: two chains, one of the even chunks and one of the odd ones, added at the end; a sum that is not finite is made again
-// in float32, input by input.
+// in float32.
 //
 // Many tokens: a wave takes 32 tokens x 32 outputs of both matrices; its tokens' values come straight from memory, the
 // matrices' parts are made by the block's threads and shared through LDS.  2,048 tokens of 2,560 channels in blocks of
@@ -213,14 +213,41 @@ __device__ __forceinline__ void gate_multiply(f32x4_t& acc, const bf16x8_t* w, c
   for (int p = 0; p < 6; ++p) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[kOrder[p][0]], u[kOrder[p][1]], acc, 0, 0, 0);
 }
 
-// The two sums of a result, again in float32 where one is not finite (an infinity splits into parts that cancel).
-__device__ __forceinline__ void gate_sums_again(float& a, float& i, const float* u, const float* wa, const float* wi, int bw) {
-  if (fmaf(a, 0.f, i * 0.f) == 0.f) return;
-  a = i = 0.f;
-#pragma unroll 1
-  for (int k = 0; k < bw; ++k) {
-    a = fmaf(wa[k], u[k], a);
-    i = fmaf(wi[k], u[k], i);
+// The sums of E neighbouring results a lane, from `out` of a channel block on, again in float32 where one is not finite (an
+// infinity splits into parts that cancel); every lane of a wave comes here, `live` or not.  u, wa and wi: the block's own.
+template <int E>
+__device__ __forceinline__ void gate_sums_again(bool live, float (&a)[E], float (&i)[E], const float* __restrict__ u,
+                                                const float* __restrict__ wa, const float* __restrict__ wi, int tok, int out,
+                                                int W, int bw) {
+  float none = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; ++e) none = fmaf(a[e], 0.f, fmaf(i[e], 0.f, none));
+  uint64_t todo = __ballot(live && none != none);
+  while (todo != 0) {  // scalar, as all that decides here
+    const int t = __builtin_amdgcn_readlane(tok, __builtin_ctzll(todo));
+    const float* row = u + static_cast<int64_t>(t) * W;
+    const bool nan = wave_holds_nan(row, bw);
+    uint64_t same = __ballot(tok == t) & todo;
+    todo &= ~same;
+    for (; same != 0; same &= same - 1) {
+      const int lane = __builtin_ctzll(same), o = __builtin_amdgcn_readlane(out, lane);
+      float sum[2 * E];
+      const float* w[2 * E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        w[e] = wa + static_cast<int64_t>(o + e) * bw;
+        w[E + e] = wi + static_cast<int64_t>(o + e) * bw;
+        sum[e] = sum[E + e] = NAN;
+      }
+      if (!nan) wave_products<2 * E>(sum, row, w, bw);
+      if ((threadIdx.x & 63) == lane) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          a[e] = fabsf(a[e]) < INFINITY ? a[e] : sum[e];
+          i[e] = fabsf(i[e]) < INFINITY ? i[e] : sum[E + e];
+        }
+      }
+    }
   }
 }
 
@@ -287,8 +314,7 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
     const int out = o0 + 16 * n + 4 * lk;
-    if (out >= bw) continue;
-    const int c = blk * bw + out;
+    const int c = blk * bw + (out < bw ? out : 0);
     float sp[4], b_a[4], b_i[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -299,17 +325,21 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int tok = t0 + 16 * t + li;
-      if (tok >= T) continue;
+      const bool live = out < bw && tok < T;
+      float sum_a[4], sum_i[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sum_a[e] = (acc[0][0][n][t][e] + acc[1][0][n][t][e]) * kPartsUnscale;
+        sum_i[e] = (acc[0][1][n][t][e] + acc[1][1][n][t][e]) * kPartsUnscale;
+      }
+      gate_sums_again<4>(live, sum_a, sum_i, u + blk * bw, wa + static_cast<int64_t>(blk) * bw * bw,
+                         wi + static_cast<int64_t>(blk) * bw * bw, tok, out, W, bw);
+      if (!live) continue;
       const int64_t at = static_cast<int64_t>(tok) * W + c;
       const f32x4_t u4 = *reinterpret_cast<const f32x4_t*>(u + at);
       float a4[4], d4[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float sum_a = (acc[0][0][n][t][e] + acc[1][0][n][t][e]) * kPartsUnscale;
-        float sum_i = (acc[0][1][n][t][e] + acc[1][1][n][t][e]) * kPartsUnscale;
-        gate_sums_again(sum_a, sum_i, u + at - out, wa + static_cast<int64_t>(c + e) * bw, wi + static_cast<int64_t>(c + e) * bw, bw);
-        gate_results(a4[e], d4[e], sum_a + b_a[e], sum_i + b_i[e], sp[e], c_decay, u4[e]);
-      }
+      for (int e = 0; e < 4; ++e) gate_results(a4[e], d4[e], sum_a[e] + b_a[e], sum_i[e] + b_i[e], sp[e], c_decay, u4[e]);
       *reinterpret_cast<f32x4_t*>(a_out + at) = f32x4_t{a4[0], a4[1], a4[2], a4[3]};
       *reinterpret_cast<f32x4_t*>(drive + at) = f32x4_t{d4[0], d4[1], d4[2], d4[3]};
     }
@@ -361,11 +391,11 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
     *reinterpret_cast<f32x4_t*>(sums[wave] + li * kRow + 4 * lk) = acc;  // token li, outputs 4 lk ..
   }
   __syncthreads();
-  if (!mine) return;
   const int s = my_tok * kRow + my_out;
-  float sum_a = (sums[0][s] + sums[2][s]) * kPartsUnscale, sum_i = (sums[1][s] + sums[3][s]) * kPartsUnscale;
-  gate_sums_again(sum_a, sum_i, u + at - (o0 + my_out), wa + static_cast<int64_t>(c) * bw, wi + static_cast<int64_t>(c) * bw, bw);
-  gate_results(a_out[at], drive[at], sum_a + b_a, sum_i + b_i, sp, c_decay, my_u);
+  float sum_a[1] = {(sums[0][s] + sums[2][s]) * kPartsUnscale}, sum_i[1] = {(sums[1][s] + sums[3][s]) * kPartsUnscale};
+  gate_sums_again<1>(mine, sum_a, sum_i, u + blk * bw, wa + static_cast<int64_t>(blk) * bw * bw,
+                     wi + static_cast<int64_t>(blk) * bw * bw, t0 + my_tok, o0 + my_out, W, bw);
+  if (mine) gate_results(a_out[at], drive[at], sum_a[0] + b_a, sum_i[0] + b_i, sp, c_decay, my_u);
 }
 
 // Channel blocks of any width and alignment: 256 threads take 16 tokens x GO outputs and walk the inputs 32 at a time

@@ -233,6 +233,36 @@ def test_gemm_f32_of_values_at_the_ends_of_float32(ops, M, N, K):
     check(torch.zeros_like(a), w)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 8192), (20, 4096, 8192), (122, 2048, 8192), (1000, 2048, 2048), (2100, 1100, 256)])
+@pytest.mark.parametrize("value,most", [(math.nan, 5), (math.inf, 50)])
+def test_gemm_f32_of_a_row_that_is_not_finite_is_no_chain_of_waits(ops, M, N, K, value, most):
+    """One NaN or infinity in one row: a NaN is looked up once a row, and behind an infinity a wave shares every element of the
+    row that is made again (one lane alone took up to 115 times the product either way); the other rows are as without it."""
+    a, w = rnd(M, K, seed=4), rnd(N, K, seed=5).abs()
+    clean, out = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+
+    def best(a, out):
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(4):
+                ops.gemm_f32(out, a, w, None)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    before = best(a, clean)
+    a[M // 2, K - 3] = value
+    after = best(a, out)
+    want = a[M // 2].double() @ w.double().T
+    assert torch.equal(out[M // 2].isnan(), want.isnan()) and torch.equal(out[M // 2].isinf(), want.isinf())
+    rest = torch.arange(M, device=DEV) != M // 2
+    assert torch.equal(out[rest], clean[rest])
+    assert after < most * before, (before, after)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (20, 40, 100), (40, 70, 512), (122, 2048, 2048), (2100, 1100, 64)])
 def test_gemm_f32_of_the_products_whose_parts_leave_most_out(ops, M, N, K):
     """Operands of one size and sign whose left-out products of parts are as large as they get, 2^-24 of the product."""
