@@ -87,6 +87,30 @@ def test_silu_mul(ops, dtype):
     assert torch.allclose(out.double(), plain.silu_and_mul(gu.double()), **tol(dtype))
 
 
+@pytest.mark.parametrize("alpha", [None, 1.702])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_gates_by_eights_have_the_bits_of_gates_one_by_one(ops, dtype, alpha):
+    """The pass that takes eight channels a thread makes its quotient by a corrected reciprocal, the one for channels that
+    do not come in eights divides: the same bits for every gate that bfloat16 has, and in float32 for gates of every size,
+    densely where the denominator nears the end of float32, and for zeros, subnormals, infinities and NaN."""
+    act = "silu" if alpha is None else ops.GateAct("clamped", 7.0, alpha, 1.0)
+    if dtype == torch.bfloat16:
+        g = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    else:
+        gen = torch.Generator().manual_seed(1)
+        bits = torch.randint(-2 ** 31, 2 ** 31, (1 << 20,), generator=gen, dtype=torch.int64).to(torch.int32).view(torch.float32)
+        near = -torch.linspace(86.0, 89.5, 1 << 18) / (alpha or 1.0)
+        g = torch.cat([bits, near, torch.tensor([0.0, -0.0, 1e-45, -1e-45, math.inf, -math.inf, math.nan, 3.4e38]).to(torch.float32)])
+    u = rnd(g.numel(), dtype=dtype, seed=2)
+    g = g.to(DEV)
+    by_eights, one_by_one = torch.empty(g.numel() // 8, 8, dtype=dtype, device=DEV), torch.empty(g.numel(), 1, dtype=dtype, device=DEV)
+    ops.silu_mul(by_eights, torch.cat([g.view(-1, 8), u.view(-1, 8)], 1), act)
+    ops.silu_mul(one_by_one, torch.stack([g, u], 1), act)
+    a, b = by_eights.view(-1), one_by_one.view(-1)
+    same = a.view(torch.int32 if dtype == torch.float32 else torch.int16) == b.view(torch.int32 if dtype == torch.float32 else torch.int16)
+    assert (same | (a.isnan() & b.isnan())).all(), g[~same][:10]
+
+
 @pytest.mark.parametrize("T,I", [(1, 8), (3, 24), (257, 8), (2, 2056), (65, 1408)])
 def test_gates_of_any_size_eight_channels_a_thread(ops, T, I):
     """float32 against 64 bits: the quotient (half an ulp and the ties that the reciprocal's correction misses), the
