@@ -76,13 +76,6 @@ def prefill_splits(T: int, nkv: int, g: int, max_query_len: int, max_seq_len: in
     return max(1, min(-(-target // blocks), keys // min_keys, PREFILL_MAX_SPLITS))
 
 
-# From so many tokens a step on, portions are attended to over two planes of values at once (16 heads over 2 in us, at once
-# and a call a plane with the copy that joins them: 70 tokens 7.6 and 16.2, 96 tokens 7.8 and 16.6, 2,048 tokens 43 and 76).
-# At once is faster below the line too; shorter steps keep the launch a plane that tests/test_sopulorn_model_gpu.py pins for
-# a step of 70 tokens.
-TWO_PLANES_TOKENS = 96
-
-
 def decode_splits(num_tokens: int, num_kv_heads: int, max_seq_len: int, waves: int,
                   window: int = 0) -> int:
     """Into how many parts each request's key range is cut for the decode kernel, beyond the
@@ -387,9 +380,11 @@ class PagedAttention(Mixer):
         if self.v_planes == 1:
             self._attend(attn, qkv, k_cache, v_planes[0], ctx, call, group, cos, sin, rot_dim, interleaved, prepared,
                          q_gain, k_gain, gate if gate_inside else None)
-        elif (ctx.num_tokens >= TWO_PLANES_TOKENS and ctx.max_query_len > 1 and self.softcap == 0.0
-              and self._prefill_kernel(group.page_size, qkv.dtype)
+        elif (ctx.max_query_len > 1 and self.softcap == 0.0 and self._prefill_kernel(group.page_size, qkv.dtype)
               and ops.prefill_attention_two_planes(self.head_dim, self.v_plane_dim, self.v_planes)):
+            # portions attend to both planes at once: the faster from two tokens on (16 heads over 2 in us, at once and a call
+            # a plane with the copy that joins them: 2 tokens 5.9 and 13.4, 70 tokens 7.6 and 16.4, 2 and 5 tokens behind
+            # 1,200 and 1,000 25 and 46, 2,048 tokens 43 and 76; 32 heads over 8, 8,192 tokens 453 and 794)
             self._attend(attn, qkv, k_cache, v_planes[0], ctx, call, group, cos, sin, rot_dim, interleaved, prepared,
                          q_gain, k_gain, v_second=v_planes[1])
         else:

@@ -300,7 +300,8 @@ def test_the_layers_run_the_kernels_they_are_meant_to(models):
         tokens = random_tokens(71, cfg["vocab"], 9)
         s.run_step({"step": 0, "entries": [{"id": "a", "tokens": tokens[:70], "want": [69]}], "end": []})
         assert sorted(set(names)) == ["prefill_attention", "qk_norm_rope_kv_write"]
-        assert names.count("prefill_attention") == 8 and names.count("qk_norm_rope_kv_write") == 7
+        # seven layers; the one whose values lie in two planes attends to both at once in portions of any length
+        assert names.count("prefill_attention") == 7 and names.count("qk_norm_rope_kv_write") == 7
         del names[:]
         s.run_step({"step": 1, "entries": [{"id": "a", "tokens": tokens[70:], "want": [0]}], "end": ["a"]})
         assert names.count("decode_attention") == 8 and names.count("qk_norm_rope_kv_write") == 1 and len(names) == 9
@@ -309,23 +310,23 @@ def test_the_layers_run_the_kernels_they_are_meant_to(models):
             setattr(ops, n, fn)
 
 
-@pytest.mark.parametrize("first", [95, 96])
-def test_two_planes_of_values_on_either_side_of_their_line(models, monkeypatch, first):
-    """The layer whose values lie in two planes takes a launch a plane below the line and one for both from there on: the
-    oracle's logits either way, also for the shorter portion behind."""
+@pytest.mark.parametrize("first", [2, 16, 70, 100])
+def test_two_planes_of_values_at_once_in_portions_of_any_length(models, monkeypatch, first):
+    """The layer whose values lie in two planes takes one launch for both in every portion: the oracle's logits, also for a
+    short portion behind, with single tokens beside them."""
     from kvcore_amd.ops import library as ops
-    from kvcore_amd.parts.attention import TWO_PLANES_TOKENS
 
-    assert TWO_PLANES_TOKENS == 96
     folder, cfg, weights, page = models["B"]
     seconds: list = []
     real = ops.prefill_attention
     monkeypatch.setattr(ops, "prefill_attention",
                         lambda *a, **k: (seconds.append(k.get("v_second") is not None), real(*a, **k))[1])
-    tokens = random_tokens(first + 20, cfg["vocab"], 9)
-    got = replay(session_for(folder, torch.bfloat16, page, 128), {"a": tokens}, [[("a", first)], [("a", 20)]])
-    compare(got, {"a": oracle(f"planes {first}", cfg, weights, tokens, torch.bfloat16)}, torch.bfloat16, excused=10)
-    assert sum(seconds) == (first >= 96) and len(seconds) == (15 if first >= 96 else 16)
+    seqs = {"a": random_tokens(first + 21, cfg["vocab"], 9), "b": random_tokens(4, cfg["vocab"], 5)}
+    got = replay(session_for(folder, torch.bfloat16, page, 256, max_num_seqs=2), seqs,
+                 [[("a", first)], [("b", 3)], [("a", 20), ("b", 1)], [("a", 1)]])
+    compare(got, {k: oracle(f"planes {first} {k}", cfg, weights, v, torch.bfloat16) for k, v in seqs.items()},
+            torch.bfloat16, excused=10)
+    assert sum(seconds) == 3 and len(seconds) == 21
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=IDS)
