@@ -504,8 +504,10 @@ def test_the_feed_forward_of_routed_experts(dtype, E, top, groups, keep, H, I, s
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("E,top,groups,keep,H,T,score,gated", [
     (32, 4, 8, 4, 2048, 8, "softmax", False), (64, 8, 1, 1, 520, 64, "logit", True), (33, 5, 3, 2, 100, 17, "sigmoid", True),
-    (2, 2, 2, 1, 8, 1, "sigmoid", False), (40, 3, 10, 9, 2040, 256, "softmax", True), (1, 1, 1, 1, 32, 16, "logit", False), (16, 2, 4, 2, 64, 1000, "softmax", False)])
-def test_spread_router_and_tiles_are_those_of_the_two_kernels(dtype, E, top, groups, keep, H, T, score, gated):
+    (2, 2, 2, 1, 8, 1, "sigmoid", False), (40, 3, 10, 9, 2040, 256, "softmax", True), (1, 1, 1, 1, 32, 16, "logit", False), (16, 2, 4, 2, 64, 1000, "softmax", False),
+    (3, 2, 1, 1, 64, 1000, "softmax", False)])
+@pytest.mark.parametrize("tile_rows", [16, 384])
+def test_spread_router_and_tiles_are_those_of_the_two_kernels(dtype, E, top, groups, keep, H, T, score, gated, tile_rows):
     """The same bits for choices, weights and gates, and the same tiles; a tile's pairs may stand in any order."""
     from kvcore_amd.ops import library as ops
 
@@ -523,13 +525,13 @@ def test_spread_router_and_tiles_are_those_of_the_two_kernels(dtype, E, top, gro
         choice, weight = torch.full((T, top), -1, **i32), torch.full((T, top), float("nan"), device=DEV)
         gate = torch.full((T,), float("nan"), device=DEV) if gated else None
         sorted_pairs, num = torch.full((T * top,), -1, **i32), torch.empty(1, **i32)
-        tiles = torch.full((ops.moe_max_tiles(T * top, E, 16), 3), -1, **i32)
+        tiles = torch.full((ops.moe_max_tiles(T * top, E, tile_rows), 3), -1, **i32)
         if few:
             work = torch.full((ops.moe_router_spread_floats(T, E),), float("nan"), device=DEV)
-            ops.moe_router_spread(choice, weight, sorted_pairs, tiles, num, x, w, work, tile_rows=16, gate=gate, **rule)
+            ops.moe_router_spread(choice, weight, sorted_pairs, tiles, num, x, w, work, tile_rows=tile_rows, gate=gate, **rule)
         else:
             ops.moe_router(choice, weight, x, w, gate=gate, **rule)
-            ops.moe_align(sorted_pairs, tiles, num, choice, E, 16)
+            ops.moe_align(sorted_pairs, tiles, num, choice, E, tile_rows)
         listed = tiles[: int(num)].tolist()
         pairs = sorted_pairs.tolist()
         starts = {e: min(a for f, a, _ in listed if f == e) for e, _, _ in listed}
@@ -637,6 +639,38 @@ def test_products_of_experts_over_tiles_of_384_rows(packed, gated, N, K, out_dty
             want[at] = y.clamp(min=0) ** 2
     # float32 sums of exact products; a bfloat16 result adds one rounding of 2^-9
     assert rel(outs[0], want) < (2e-6 if out_dtype == torch.float32 else 3e-3)
+
+
+@pytest.mark.parametrize("E", [1, 31, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("counts_of", ["equal", "edges", "drawn"])
+def test_tiles_of_384_rows_hold_every_pair_once(E, counts_of):
+    """The list of tiles for up to 32, up to 64 and more experts, with equal counts, without rows and with up to three tiles
+    an expert: as many tiles as the rows ask for, each pair in one of them, no row beyond an expert's own, and up to 64
+    experts those with more rows a tile first."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(E)
+    edges = [0, 1, 383, 384, 385, 768, 769, 1000, 384, 0, 1, 16, 17]
+    counts = {"equal": [200] * E, "edges": [edges[i % len(edges)] for i in range(E)],
+              "drawn": torch.randint(0, 500, (E,), generator=gen).tolist()}[counts_of]
+    if not sum(counts):
+        counts[0] = 5
+    pairs = sum(counts)
+    choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(pairs, generator=gen)]
+    i32 = dict(dtype=torch.int32, device=DEV)
+    sorted_pairs, num = torch.full((pairs,), -1, **i32), torch.empty(1, **i32)
+    tiles = torch.full((ops.moe_max_tiles(pairs, E, 384), 3), -1, **i32)
+    ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32).view(pairs, 1), E, 384)
+    assert int(num) == sum(-(-n // 384) for n in counts)
+    assert (tiles[int(num):] == -1).all()
+    listed, order = tiles[: int(num)].tolist(), sorted_pairs.tolist()
+    rows = [r for _, first, n in listed for r in range(first, first + n)]
+    assert sorted(rows) == list(range(pairs)) and sorted(order) == list(range(pairs))
+    for e, first, n in listed:
+        assert 1 <= n <= 384 and all(choice[order[r]] == e for r in range(first, first + n))
+    if E <= 64:
+        most = {e: max(n for f, _, n in listed if f == e) for e, _, _ in listed}
+        assert [e for e, _, _ in listed] == sorted((e for e, _, _ in listed), key=lambda e: (-most[e], e))
 
 
 @pytest.mark.parametrize("gated", [True, False])
