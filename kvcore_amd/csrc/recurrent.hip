@@ -183,10 +183,10 @@ __global__ __launch_bounds__(256) void conv_state_kernel(
 // tile: two chains, one of the even chunks and one of the odd ones, added at the end; a sum that is not finite is made again
 // in float32.
 //
-// Many tokens: a wave takes 32 tokens x 32 outputs of both matrices; its tokens' values come straight from memory, the
-// matrices' parts are made by the block's threads and shared through LDS.  2,048 tokens of 2,560 channels in blocks of
-// 256: 99 us on the float32 matrix instructions with 16 outputs a wave, which read the matrices and the tokens twice as often,
-// 55 us this way, of which the exponentials, quotients and roots of the results are some 30.
+// Many tokens: a wave takes 32 tokens x 32 outputs of both matrices (16 outputs where that deals out better); its tokens'
+// values come straight from memory, the matrices' parts are made by the block's threads and shared through LDS.  2,048
+// tokens of 2,560 channels in blocks of 256: 91 us on the float32 matrix instructions with 16 outputs a wave, which read the
+// matrices and the tokens twice as often, 55 us this way, of which the exponentials, quotients and roots of the results are some 30.
 constexpr int GT = 16, GK = 32;
 
 // The results for one channel of a token from its two sums (biases added), softplus(lam) and its input.
@@ -251,20 +251,21 @@ __device__ __forceinline__ void gate_sums_again(bool live, float (&a)[E], float 
   }
 }
 
-constexpr int kGateTokens = 128, kGateOuts = 32;  // of a block of many tokens
+constexpr int kGateTokens = 128;  // of a block of many tokens
 
+template <int NT>  // tiles of 16 outputs
 __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
     int bw, int out_tiles, int token_tiles) {
-  __shared__ bf16x8_t w_s[2][2][2][3][64];  // buffer, matrix, tile of outputs, part, lane
+  __shared__ bf16x8_t w_s[2][2][NT][3][64];  // buffer, matrix, tile of outputs, part, lane
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
   const int channel_tile = blockIdx.x / token_tiles;
   const int t0 = (blockIdx.x - channel_tile * token_tiles) * kGateTokens + wave * 32;
   const int blk = channel_tile / out_tiles;
-  const int o0 = (channel_tile - blk * out_tiles) * kGateOuts;
+  const int o0 = (channel_tile - blk * out_tiles) * 16 * NT;
   // outputs and tokens beyond the last read the last one and are not stored; a wave without tokens still shares its part
   const float* u_row[2];
 #pragma unroll
@@ -272,16 +273,17 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
     const int tok = t0 + 16 * t + li;
     u_row[t] = u + static_cast<int64_t>(tok < T ? tok : T - 1) * W + blk * bw;
   }
-  // the thread's piece of the matrices: eight inputs of one row of one of them
-  const int my_k = 8 * (threadIdx.x & 3), my_row = (threadIdx.x >> 2) & 31, my_mat = threadIdx.x >> 7;
+  // the thread's piece of the matrices: eight inputs of one row of one of them (with one tile of outputs every other wave)
+  const int my_k = 8 * (threadIdx.x & 3), my_row = (threadIdx.x >> 2) & (16 * NT - 1), my_mat = threadIdx.x >> 7;
+  const bool brings = NT == 2 || (wave & 1) == 0;  // scalar
   const float* w_row = (my_mat ? wi : wa) + (static_cast<int64_t>(blk) * bw + (o0 + my_row < bw ? o0 + my_row : bw - 1)) * bw;
   const int my_lane = (threadIdx.x & 3) * 16 + (my_row & 15);
-  f32x4_t acc[2][2][2][2];  // chain, matrix, tile of outputs, tile of tokens
+  f32x4_t acc[2][2][NT][2];  // chain, matrix, tile of outputs, tile of tokens
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][(i >> 1) & 1][i & 1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 8 * NT; ++i) acc[i / (4 * NT)][i / (2 * NT) & 1][i / 2 % NT][i & 1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   f32x4_t wv[2], uv[2][2];
   auto fetch = [&](int k0) {  // chunks that are not there arrive as zeros
-    gate_load8(wv, w_row, k0 + my_k, bw);
+    if (brings) gate_load8(wv, w_row, k0 + my_k, bw);
 #pragma unroll
     for (int t = 0; t < 2; ++t) gate_load8(uv[t], u_row[t], k0 + 8 * lk, bw);
   };
@@ -290,9 +292,11 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
 #pragma unroll
     for (int s = 0; s < 2; ++s) {  // the even chunk and the odd one, each with a buffer and a chain of its own
       if (k0 + GK * s >= bw) break;  // scalar
-      const split_t w_parts = split8(wv);
+      if (brings) {
+        const split_t w_parts = split8(wv);
 #pragma unroll
-      for (int p = 0; p < 3; ++p) w_s[s][my_mat][my_row >> 4][p][my_lane] = w_parts.part[p];
+        for (int p = 0; p < 3; ++p) w_s[s][my_mat][my_row >> 4][p][my_lane] = w_parts.part[p];
+      }
       split_t u_parts[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) u_parts[t] = split8(uv[t]);
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
+        for (int n = 0; n < NT; ++n) {
           bf16x8_t w[3];
 #pragma unroll
           for (int p = 0; p < 3; ++p) w[p] = w_s[s][m][n][p][lane];
@@ -312,7 +316,7 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
   }
   // a lane holds token li, outputs 4 lk .. of its tiles
 #pragma unroll
-  for (int n = 0; n < 2; ++n) {
+  for (int n = 0; n < NT; ++n) {
     const int out = o0 + 16 * n + 4 * lk;
     const int c = blk * bw + (out < bw ? out : 0);
     float sp[4], b_a[4], b_i[4];
@@ -348,13 +352,15 @@ __global__ __launch_bounds__(256, 2) void rglru_gates_kernel(
 
 // The same, with the same bits, for few blocks of 16 tokens x 16 outputs: a wave takes one chain of one matrix, four chunks
 // on their way, and then every thread the results of one channel of one token.  Where one wave made all 256 of them, 8
-// tokens of 10 blocks of 32 channels took 5.8 us, so 3.2, of 256 channels 8.2 and 5.1.
+// tokens of 10 blocks of 32 channels took 5.8 us, so 3.2, of 256 channels 8.2 and 5.1.  AHEAD is one where a chain has one chunk
+// (1,024 tokens of 10 blocks of 32 channels 6.1 us with four, 5.5 so).
+template <int AHEAD>
 __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
     float* __restrict__ a_out, float* __restrict__ drive, const float* __restrict__ u,
     const float* __restrict__ wa, const float* __restrict__ wi, const float* __restrict__ ba,
     const float* __restrict__ bi, const float* __restrict__ lam, float c_decay, int T, int W,
     int bw, int out_tiles, int token_tiles) {
-  constexpr int AHEAD = 4, kRow = 20;
+  constexpr int kRow = 20;
   __shared__ __attribute__((aligned(16))) float sums[4][16 * kRow];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int channel_tile = blockIdx.x / token_tiles;
@@ -384,7 +390,7 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
       for (int s = 0; s < AHEAD; ++s) {
         if (k0 + 2 * GK * s >= bw) break;  // scalar
         const split_t w_now = split8(wv[s]), u_now = split8(uv[s]);
-        fetch(s, k0 + 2 * GK * (s + AHEAD));
+        if (AHEAD > 1) fetch(s, k0 + 2 * GK * (s + AHEAD));  // otherwise a chain has one chunk
         gate_multiply(acc, w_now.part, u_now.part);
       }
     }
@@ -1001,27 +1007,34 @@ extern "C" int kvc_rglru_gates(float* a_out, float* drive, const float* u, const
     return kvc_check_launch("kvc_rglru_gates");
   }
   const int out_tiles = (bw + 15) / 16;
-  // Small blocks or large, whichever an estimate in us says: small ones share the units, of large ones a unit takes one
-  // after the other.  Small / large, both measured: 10 blocks of 256 channels, 100 tokens 14.0 / 17.2, 160 tokens 17.4 / 17.8,
-  // 256 tokens 22.6 / 17.8, 2,048 tokens 147 / 54; 10 blocks of 160, 256 tokens 12.1 / 14.9, 400 tokens 16.2 / 15.6; 10 blocks of
-  // 64, 1,024 tokens 10.8 / 11.9, 2,048 tokens 18.4 / 16.9; one block of 128, 4,096 tokens 12.7 / 13.7; 8 blocks of 512, 64 tokens
-  // 19.7 / 23.8, 100 tokens 30.4 / 26.0.
+  // Small blocks, large ones of half the outputs or large ones, whichever an estimate in us says: small ones share the units, of
+  // large ones a unit takes one after the other, and half the outputs leave half as much for the last round and read the
+  // tokens twice as often.  All three measured: 10 blocks of 32 channels, 1,024 tokens 5.5 / 6.9 / 10.3, 2,048 tokens
+  // 8.9 / 9.0 / 10.8, 4,096 tokens 14.9 / 12.7 / 15.1; 32 blocks of 32, 683 tokens 9.5 / 9.2 / 10.9; 10 blocks of 64, 1,024 tokens
+  // 10.6 / 10.3 / 11.6, 2,048 tokens 17.6 / 14.3 / 16.8, 8,192 tokens 55 / 36 / 35; one block of 128, 4,096 tokens 12.6 / 9.9 / 13.5; 10
+  // blocks of 160, 256 tokens 12.7 / 10.5 / 14.7, 1,500 tokens 48.5 / 30.1 / 28.9; 10 blocks of 256, 100 tokens 13.5 / 12.5 / 16.6, 160
+  // tokens 17.1 / 17.3 / 17.7, 2,048 tokens 147 / 65 / 55; 8 blocks of 512, 100 tokens 30.5 / 20.2 / 25.1.
   const double units = kvc_device_compute_units();
   const int64_t few_blocks = static_cast<int64_t>((T + 15) / 16) * nb * out_tiles;
-  const int big_out_tiles = (bw + kGateOuts - 1) / kGateOuts;
-  const int64_t big_blocks = static_cast<int64_t>((T + kGateTokens - 1) / kGateTokens) * nb * big_out_tiles;
-  const double few_us = 3 + 0.008 * bw + few_blocks / units * (0.4 + 0.0055 * bw);
-  const double big_us = 5.5 + 0.008 * bw + ceil(big_blocks / units) * (4.4 + 0.02 * bw);
-  const bool few = few_us <= big_us;
-  const int token_tiles = few ? (T + 15) / 16 : (T + kGateTokens - 1) / kGateTokens;
-  const int64_t blocks = few ? few_blocks : big_blocks;
+  const int big_out_tiles = (bw + 31) / 32, token_blocks = (T + kGateTokens - 1) / kGateTokens;
+  const int64_t big_blocks = static_cast<int64_t>(token_blocks) * nb * big_out_tiles;
+  const int64_t half_blocks = static_cast<int64_t>(token_blocks) * nb * out_tiles;
+  const double few_us = 3 + 0.008 * bw + few_blocks / units * (bw <= 2 * GK ? 0.46 + 0.0035 * bw : 0.5 + 0.0048 * bw);
+  const double half_us = 3.9 + 0.011 * bw + ceil(half_blocks / units) * (2.3 + 0.015 * bw);
+  const double big_us = 4.8 + 0.008 * bw + ceil(big_blocks / units) * (4.4 + 0.02 * bw);
+  const bool few = few_us <= big_us && few_us <= half_us, half = !few && half_us < big_us;
+  const int token_tiles = few ? (T + 15) / 16 : token_blocks;
+  const int64_t blocks = few ? few_blocks : half ? half_blocks : big_blocks;
   if (blocks > 0x7fffffff) return kvc_fail("kvc_rglru_gates: too many blocks");
-  if (few)
-    hipLaunchKernelGGL(rglru_gates_few_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out, drive,
-                       u, wa, wi, ba, bi, lam, c_decay, T, W, bw, out_tiles, token_tiles);
-  else
-    hipLaunchKernelGGL(rglru_gates_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, S(stream), a_out,
-                       drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, big_out_tiles, token_tiles);
+  const dim3 grid(static_cast<unsigned>(blocks));
+#define KVC_GATES(KERNEL, OUT_TILES)                                                                                     \
+  hipLaunchKernelGGL((KERNEL), grid, dim3(256), 0, S(stream), a_out, drive, u, wa, wi, ba, bi, lam, c_decay, T, W, bw, \
+                     OUT_TILES, token_tiles)
+  if (few && bw <= 2 * GK) KVC_GATES(rglru_gates_few_kernel<1>, out_tiles);
+  else if (few) KVC_GATES(rglru_gates_few_kernel<4>, out_tiles);
+  else if (half) KVC_GATES(rglru_gates_kernel<1>, out_tiles);
+  else KVC_GATES(rglru_gates_kernel<2>, big_out_tiles);
+#undef KVC_GATES
   return kvc_check_launch("kvc_rglru_gates");
 }
 

@@ -279,7 +279,8 @@ def test_gates_of_a_token_do_not_depend_on_the_step(ops, W, nb):
             assert torch.equal(got, want[first: first + n])
 
 
-@pytest.mark.parametrize("W,nb", [(512, 2), (512, 8), (520, 13), (60, 2)])
+@pytest.mark.parametrize("W,nb", [(512, 2), (512, 8), (520, 13), (60, 2),  # the first three in large blocks of half the outputs
+                                  (1000, 5), (2560, 10)])                   # in large blocks
 def test_gates_in_long_portions_are_those_of_short_steps(ops, W, nb):
     """Steps long enough for the larger blocks, tokens that do not fill them and channels that do not fill tiles of
     16: 64-bit results, and the bits of the same rows in steps that take the small ones."""
@@ -305,7 +306,7 @@ def test_gates_in_long_portions_are_those_of_short_steps(ops, W, nb):
             assert torch.equal(got, want[first: first + n]), (first, n)
 
 
-@pytest.mark.parametrize("T", [20, 1500])
+@pytest.mark.parametrize("T", [20, 1000, 1500])  # small blocks, large ones of half the outputs, large ones
 def test_gates_of_values_that_are_not_finite_or_tiny(ops, T):
     """An infinity among a token's values or a matrix's reaches its sums as in float32 (parts of it would cancel to no
     number), values below what bfloat16 parts can hold leave finite results, and other rows are as if alone."""
@@ -327,7 +328,7 @@ def test_gates_of_values_that_are_not_finite_or_tiny(ops, T):
         assert torch.allclose(got.double().cpu(), want, atol=1e-5, rtol=1e-5, equal_nan=True)
 
 
-@pytest.mark.parametrize("T", [20, 1500])
+@pytest.mark.parametrize("T", [20, 1000, 1500])
 @pytest.mark.parametrize("tiny,large", [(1e-37, 1e36), (1e-41, 1e32)])
 def test_gates_of_tiny_values_behind_large_matrices(ops, T, tiny, large):
     """Values that bfloat16 holds in part only, or not at all, times matrices that make ordinary sums of them."""
