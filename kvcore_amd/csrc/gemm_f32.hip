@@ -106,7 +106,9 @@ __device__ __forceinline__ void leave(bool live, f32x4_t v, float* __restrict__ 
   store4<float>(C + static_cast<int64_t>(row) * ldc + col, v, N - col);
 }
 
-template <int NT, int MT, int AHEAD, int PIECE>
+// ONCE: K is at most kWaves * AHEAD chunks, so all of it is on its way from the start and nothing is asked for behind it (one row
+// of 4096 x 512 5.7 us with four chunks ahead and loads of nothing behind the two that there are, 4.5 so)
+template <int NT, int MT, int AHEAD, int PIECE, bool ONCE>
 __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict__ C, const float* __restrict__ A,
                                                                const float* __restrict__ W,
                                                                const float* __restrict__ bias, int M, int N, int K,
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_f32_kernel(float* __restrict
       // the loads leave after the registers that they fill have been read (or they would fill others and be copied,
       // which waits for them) and before the products
       __builtin_amdgcn_sched_barrier(0);
-      fetch(s, c + kWaves * (s + AHEAD));
+      if (!ONCE) fetch(s, c + kWaves * (s + AHEAD));
       __builtin_amdgcn_sched_barrier(0);
       multiply<NT, MT>(acc, w, a);
     }
@@ -398,8 +400,36 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(float* __restrict__
   leave(live, v[0], C, A, W, bias, row, col, N, K, lda, ldc);
 }
 
+// Tiles of 16 columns and 16 rows a block of gemm_f32_kernel: 64 x 64 where they give every compute unit a block, narrower ones
+// otherwise (122 rows of 2048 x 2048 are 64 blocks of 64 x 64 and 256 of 32 x 32); rows in sixteens up to the batch's size.
+struct FewShape {
+  int nt, mt;
+  int64_t blocks;
+};
+FewShape few_shape(int M, int N) {
+  const int64_t units = kvc_device_compute_units();
+  int nt = 4, mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+  if (mt == 4 && M < 256 && (M + 63) / 64 * 64 >= M + 32) mt = 2;  // the last 64 rows would be half empty
+  auto blocks = [&]() { return (static_cast<int64_t>(N) + 16 * nt - 1) / (16 * nt) * ((M + 16 * mt - 1) / (16 * mt)); };
+  while (blocks() < units && (nt > 1 || mt > 2)) {  // from (2, 4) on to (2, 2)
+    if (nt >= mt && nt > 1) nt /= 2;
+    else if (mt > 2) mt /= 2;
+    else nt /= 2;
+  }
+  return {nt, mt, blocks()};
+}
+
 // How the sizes of a call are dealt out to the kernel with rows in LDS: column blocks of 16 a wave, chains to how many
-// blocks; nt 0: not at all.
+// blocks; nt 0: not at all.  By an estimate in us of each way, fitted to 155 sizes (33 to 1,500 rows, N of 256 to 16,384, K of
+// 512 to 8,192; weights that no cache holds) within some 6%: a round of blocks on the units has a start and its share of K, and chains left
+// in memory cost another kernel and their bytes.  gemm_f32_kernel / here, 64 columns, chains in one block / 128 columns in one /
+// the better of those dealt out, in us:
+//   64 rows of 2048 x 512     6.1 / 13.1 / 21.1 /  9.6      122 of 2048 x 2048    18.6 / 37 / 62 / 18.5
+//   64 rows of 8192 x 512    10.4 / 13.6 / 21.2 / 18.5      64 of 16384 x 2048    42 / 47 / 69 / 52
+//   256 of 2048 x 1024       15.8 / 22.1 / 36.0 / 22.1      128 of 3072 x 8192    93 / 133 / 223 / 58
+//   400 of 2048 x 1024       28.6 / 22.4 / 36.7 / 30.1      400 of 3072 x 4096   124 / 119 / 121 / 93
+//   100 of 16384 x 512       26.2 / 21.2 / 23.8 / 41.4      200 of 8192 x 8192   347 / 261 / 257 / 229
+// Chains are dealt out up to the workspace that 64 x 128 of C a unit need.
 constexpr int kSharedRows = 4;  // row blocks of 16 a block
 struct SharedShape {
   int nt, groups;
@@ -407,14 +437,22 @@ struct SharedShape {
 SharedShape shared_shape(int M, int N, int K) {
   if (M <= 32 || K % (2 * kWaves * kChunk)) return {0, 0};
   const int64_t units = kvc_device_compute_units();
-  // 64 rows a block; 128 columns, or 64 where those give every unit a block and 128 do not (64 rows of 16384 x 2048 52 and
-  // 43 us).  Where neither does, the chains go to several blocks: of 128 columns if eight times as many fill the chip
-  // (122 rows of 2048 x 8192: 64 columns 46 us, 128 columns 39), of 64 otherwise (64 rows of it 28 and 37)
-  SharedShape s{2, 1};
-  const int64_t row_blocks = (M + 63) / 64, wide = (N + 127) / 128 * row_blocks, narrow = (N + 63) / 64 * row_blocks;
-  if (wide < units && (narrow >= units || kWaves * wide < units)) s.nt = 1;
-  while (s.groups < kWaves && (s.nt == 1 ? narrow : wide) * s.groups < units) s.groups *= 2;
-  return s;
+  auto rounds = [&](int64_t blocks) { return static_cast<double>((blocks + units - 1) / units); };
+  const FewShape few = few_shape(M, N);
+  const int live = few.mt < (M + 15) / 16 ? few.mt : (M + 15) / 16;  // row blocks that are not copies of the last
+  double least = 2.7 + rounds(few.blocks) * (0.3 * few.nt * few.mt + 0.45 * (K / (kWaves * kChunk)) * (few.nt + live));
+  SharedShape best{0, 0};
+  for (int nt = 1; nt <= 2; ++nt) {
+    const int64_t blocks = (static_cast<int64_t>(N) + 64 * nt - 1) / (64 * nt) * ((M + 63) / 64);
+    for (int groups = 1; groups <= kWaves; groups *= 2) {
+      if (groups > 1 && static_cast<int64_t>(M) * N > units * 64 * 128) break;
+      const double r = rounds(blocks * groups);
+      double us = 5.3 + 0.8 * r + K / kChunk / groups * (nt == 1 ? 0.49 + 0.45 * (r - 1) : 0.89 + 0.735 * (r - 1));
+      if (groups > 1) us += 1.1 + 12e-6 * M * N;
+      if (us < least) least = us, best = {nt, groups};
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -492,25 +530,17 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
     }
     return kvc_check_launch("kvc_gemm_f32");
   }
-  // tiles of 64 x 64 where they give every compute unit a block, narrower ones otherwise (122 rows of 2048 x 2048
-  // are 64 blocks of 64 x 64 and 256 of 32 x 32); rows in sixteens up to the batch's size
-  int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-  if (mt == 4 && M < 256 && (M + 63) / 64 * 64 >= M + 32) mt = 2;  // the last 64 rows would be half empty
-  int nt = 4;
-  auto blocks = [&]() { return static_cast<int64_t>((N + 16 * nt - 1) / (16 * nt)) * ((M + 16 * mt - 1) / (16 * mt)); };
-  while (blocks() < units && (nt > 1 || mt > 2)) {
-    if (nt >= mt && nt > 1) nt /= 2;
-    else if (mt > 2) mt /= 2;
-    else nt /= 2;
-  }
+  const FewShape few = few_shape(M, N);
+  const int nt = few.nt, mt = few.mt;
   const dim3 grid((N + 16 * nt - 1) / (16 * nt), (M + 16 * mt - 1) / (16 * mt));
   if (grid.y > 65535) return kvc_fail("kvc_gemm_f32: M too large for one launch");
-#define KVC_F32(NT, MT, AHEAD)                                                                      \
-  do {                                                                                              \
-    if (piece == 8) KVC_F32_LAUNCH((gemm_f32_kernel<NT, MT, AHEAD, 8>), kWaves * 64);               \
-    else KVC_F32_LAUNCH((gemm_f32_kernel<NT, MT, 1, 1>), kWaves * 64);                              \
+#define KVC_F32(NT, MT, AHEAD)                                                                                        \
+  do {                                                                                                                \
+    if (piece != 8) KVC_F32_LAUNCH((gemm_f32_kernel<NT, MT, 1, 1, false>), kWaves * 64);                              \
+    else if (chunks <= kWaves * AHEAD) KVC_F32_LAUNCH((gemm_f32_kernel<NT, MT, AHEAD, 8, true>), kWaves * 64);        \
+    else KVC_F32_LAUNCH((gemm_f32_kernel<NT, MT, AHEAD, 8, false>), kWaves * 64);                                     \
   } while (0)
-  if (mt == 4) {  // from (2, 4) the loop above goes on to (2, 2)
+  if (mt == 4) {
     if (nt == 4) KVC_F32(4, 4, 1);
     else KVC_F32(2, 4, 1);
   } else if (mt == 2) {
@@ -520,6 +550,7 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
   } else {
     if (nt == 4) KVC_F32(4, 1, 2);
     else if (nt == 2) KVC_F32(2, 1, 2);
+    else if (chunks <= 2 * kWaves) KVC_F32(1, 1, 2);
     else KVC_F32(1, 1, 4);
   }
 #undef KVC_F32

@@ -165,7 +165,9 @@ def test_gemm_f32_is_true_float32_and_does_not_depend_on_the_batch(ops, M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (2, 4100, 2048), (16, 17, 264), (17, 8200, 520), (33, 2048, 1024),
-                                   (65, 515, 2056), (122, 2048, 8192), (122, 16384, 264), (130, 100, 40), (300, 1000, 72)])
+                                   (65, 515, 2056), (122, 2048, 8192), (122, 16384, 264), (130, 100, 40), (300, 1000, 72),
+                                   # all of K on its way from the start: two and four chunks a wave, every width of tile
+                                   (2, 300, 1000), (16, 515, 512), (3, 8300, 392), (4, 16400, 512), (20, 4100, 512), (33, 2048, 512)])
 def test_gemm_f32_tiles_give_the_same_bits(ops, M, N, K):
     """Every tile shape that the sizes choose: the sums of a 64-bit product, and a row's bits as it has them alone."""
     a, w = rnd(M, K, seed=4), rnd(N, K, seed=5)
@@ -203,9 +205,12 @@ def test_gemm_f32_of_short_rows_gives_the_same_bits(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(33, 100, 512), (64, 16384, 512), (65, 515, 1024), (122, 2048, 2048), (130, 8200, 1536),
-                                   (300, 33000, 512)])
+                                   (300, 33000, 512),
+                                   # 64 columns a block and 128, with the chains of K in one block, in two, in four and in eight
+                                   (65, 6150, 512), (1030, 130, 1024), (33, 70, 1536), (450, 2052, 512), (33, 4100, 1024), (33, 2052, 1024)])
 def test_gemm_f32_of_many_rows_gives_the_same_bits(ops, M, N, K):
-    """Rows through LDS (from 33 on, K a multiple of 512), with the chains of K in one block or in several: the sums of a
+    """Rows through LDS (from 33 on, K a multiple of 512, where an estimate says so), with the chains of K in one block or in
+    several, and sizes on the estimate's other side: the sums of a
     64-bit product, and a row's bits as it has them alone."""
     a, w, b = rnd(M, K, seed=4), rnd(N, K, seed=5), rnd(N, seed=6)
     wide_in, wide_out = torch.full((M, K + 4), 3.0, device=DEV), torch.full((M, N + 3), 7.0, device=DEV)
