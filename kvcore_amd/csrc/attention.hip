@@ -185,7 +185,9 @@ __global__ __launch_bounds__(kWavesPerBlock* kWave) void paged_attention_wave_ke
 // A wave's lanes take a key each for the scores (a key's row read once for all GH heads) and a channel each for the weighted
 // sums, whose values come in runs of four keys, half a tile's asked for without a branch.  The kernel above reads a key and
 // then a value at a time, one wave a head: bound by that chain, some 0.2 us a key.  32 heads of 64 over 8: two portions of 61
-// tokens 27.3 -> 10.0 us, of 512 1,255 -> 119; one token behind 1,500 335 -> 25, 16 behind 1,000 240 -> 21.
+// tokens 27.3 -> 10.0 us, of 512 1,255 -> 119; one token behind 1,500 335 -> 25, 16 behind 1,000 240 -> 21.  A token that sees
+// fewer than some ten keys pays for a whole tile: the first token 4.9 -> 6.9, one behind three 5.4 -> 6.8, one behind 20 8.7 -> 7.2.
+// (Values asked for before the scores, with all of a key's row at once, take registers that spill: 7 -> 10 us, 1,500 keys 2.2 times as long.)
 constexpr int kChains = 8;
 
 template <int D, int GH, int W>
