@@ -1354,25 +1354,33 @@ extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
   return blocks >= 300 && (each >= 150 || (each >= 40 && each < 104)) ? kBigTileRows : kMidTileRows;
 }
 
-// Whether tiles of up to 384 rows (the answer; otherwise 0) serve such a step better.  A block of theirs has a compute unit to
-// itself, so the first product needs a block a unit and the second one every other unit (an expert has more than one tile only
-// from where nearly all do: rows vary by some three times their root), and below 104 rows an expert they are no faster than
-// the smaller tiles.  Both products in us, the best of the smaller tiles / these, by rows an expert, gated:
-//   32 experts of 2048 x 2048     90  178 / 174  130  237 / 196  180  242 / 218  256  324 / 259  330  371 / 304  500  523 / 444
-//   16 experts of 2048 x 2048     90   97 / 102  130  133 / 115  180  129 / 129  256  187 / 152  330  200 / 182  500  289 / 217
-//   64 experts of 1024 x 512      90   56 /  57  130   77 /  64  180   76 /  73  256  115 /  87  330  120 / 103  500  174 / 144
-//   128 experts of 1024 x 384     90   94 /  99  130  110 / 110  180  127 / 127  256  158 / 151  330  192 / 178  500  277 / 241
+// Whether tiles of up to 384 rows (the answer; otherwise 0) serve such a step better, also where the experts' rows are uneven, which
+// no launch knows.  A block of theirs has a compute unit to itself, and the largest one (three times the mean and more rows soon
+// make it full) lasts as long as two or three in the mean: with one round of blocks the units wait for it, with two, the
+// largest first, they do not.  So the first product needs two blocks a unit and the second one a block, experts wide enough
+// that a block's way in and out counts little, and 104 rows an expert; or one block a unit and every other one, where the
+// experts' rows fill two thirds of a tile in the mean and K is long; or (an expert has more than one tile only from where nearly all do, as
+// rows vary by some three times their root) two tiles an expert.  Both products and the list in us, the best of the smaller tiles /
+// these, experts of the same chance, and of chances by which the fullest has 2 to 3, 4 to 5 and 7 to 15 times the mean, gated:
+//   32 experts of 2048 x 2048   110  220 / 193  228 / 203  220 / 217  226 / 203    256  324 / 275  337 / 306  334 / 294  337 / 284
+//   64 experts of 2048 x 1024   110  234 / 211  230 / 208  228 / 215  219 / 191    256  342 / 297  341 / 328  347 / 313  358 / 319
+//   16 experts of 2048 x 2048   256  191 / 160  192 / 183  192 / 170  196 / 176    500  296 / 220  293 / 243  308 / 239  294 / 242
+//   64 experts of 1024 x 512    500  209 / 181  208 / 192  208 / 193  208 / 198
 // not gated:
-//   32 experts of 2048 x 2048     90  122 / 123  130  162 / 136  256  230 / 182
-// and where the blocks do not fill the units:
-//   16 experts of 1024 x 1024    256   69 /  83  400   74 /  97  500   98 /  82 (two tiles an expert)
-//   8 experts of 2048 x 1024     256   73 /  97  500  101 /  98
+//   32 experts of 2048 x 2048   256  243 / 198  245 / 240  244 / 210  232 / 205
+// and not taken:
+//   16 experts of 2048 x 2048   130  139 / 122  136 / 154  133 / 162  130 / 147    180  133 / 135  138 / 178  146 / 164  140 / 157
+//   64 experts of 1024 x 512    130   86 /  76   87 / 114   86 / 124   83 / 121    256  131 / 109  131 / 157  130 / 148  131 / 155
+//   64 experts of 1024 x 1024   130  139 / 124  134 / 139  137 / 143  134 / 136    180  149 / 142  154 / 177  154 / 172  151 / 173
+//   128 experts of 1024 x 384   130  132 / 136  134 / 156  135 / 161  133 / 160    256  197 / 193  198 / 214  196 / 207  190 / 204
 extern "C" int kvc_moe_wide_tile_rows(int pairs, int E, int H, int I, int gated) {
   if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || H % 64 || I % 64) return 0;
   const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
-  const double tiles = E * fmax(1.0, ceil((each - 3 * sqrt(each)) / kWideTileRows));
-  const int first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, down_cols = (H + 255) / 256;
-  return each >= 104 && tiles * first_cols >= units && 2 * tiles * down_cols >= units ? kWideTileRows : 0;
+  const double of_one = fmax(1.0, ceil((each - 3 * sqrt(each)) / kWideTileRows)), tiles = E * of_one;
+  const double first = tiles * (gated ? (I + 127) / 128 : (I + 255) / 256) / units, down = tiles * ((H + 255) / 256) / units;
+  const bool two_rounds = first >= 2 && down >= 1 && (H + I >= 3072 || of_one > 1);
+  const bool full = first >= 1 && down >= 0.5 && each >= 230 && H >= 2048 && I >= 2048;
+  return each >= 104 && (two_rounds || full) ? kWideTileRows : 0;
 }
 
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,

@@ -90,8 +90,11 @@ def test_tiles_of_384_rows_need_rows_and_blocks_for_every_unit():
 
     x = torch.empty(1, 8, dtype=torch.bfloat16)
     for (E, H, I), rows in {(32, 2048, 2048): {64: 0, 103: 0, 104: 384, 256: 384, 512: 384},
-                            (16, 2048, 2048): {96: 0, 130: 384}, (16, 1024, 1024): {256: 0, 400: 0, 500: 384},
-                            (8, 2048, 1024): {256: 0, 500: 0}, (128, 1024, 384): {130: 384}, (32, 2048, 2016): {256: 0}}.items():
+                            # one block a unit: rows enough for uneven experts not to be waited for, and a long K
+                            (16, 2048, 2048): {130: 0, 229: 0, 230: 384, 500: 384}, (64, 1024, 512): {130: 0, 256: 0, 500: 384},
+                            (128, 1024, 384): {130: 0, 256: 0, 500: 384}, (64, 1024, 1024): {256: 0, 500: 384},
+                            (64, 2048, 1024): {103: 0, 104: 384}, (16, 1024, 1024): {256: 0, 400: 0, 500: 0},
+                            (8, 2048, 1024): {256: 0, 500: 0}, (32, 2048, 2016): {256: 0}}.items():
         for each, tile in rows.items():
             assert ops.moe_wide_tile_rows(each * E, E, x, (H, I)) == tile, (E, H, I, each)
     assert ops.moe_wide_tile_rows(256 * 32, 32, x.float(), (2048, 2048)) == 0
