@@ -10,7 +10,7 @@
 //
 // Few rows: a block takes NT x MT tiles of 16 columns x 16 rows of C and all its waves take all of them, each a chain
 // of K: the operands go from memory to registers (the four lanes of a row read 64 contiguous bytes at a time).  Bound by
-// reading W (one row of 16384 x 2048 31 us, 4.4 TB/s).  More than 32 rows: gemm_f32_shared_kernel.
+// reading W (one row of 16384 x 2048 31 us, 4.4 TB/s).  More than 32 rows: these, or gemm_f32_shared_kernel (shared_shape).
 
 #include <hip/hip_runtime.h>
 
