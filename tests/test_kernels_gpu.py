@@ -182,6 +182,33 @@ def test_gemm_f32_tiles_give_the_same_bits(ops, M, N, K):
         assert torch.equal(single[0], out[i])
 
 
+def test_gemm_f32_with_its_chains_in_memory_replays_from_a_graph(ops):
+    """Two products one after the other whose chains go to several blocks: their workspaces come and go inside the graph, and
+    each replay has the bits of eager calls on the inputs of that time."""
+    M, N, K = 64, 2048, 8192
+    a, w, v = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5), rnd(K, N, seed=3, scale=N ** -0.5)
+    first, second = torch.empty(M, N, device=DEV), torch.empty(M, K, device=DEV)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        ops.gemm_f32(first, a, w, None)
+        ops.gemm_f32(second, first, v, None)
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            ops.gemm_f32(first, a, w, None)
+            ops.gemm_f32(second, first, v, None)
+    torch.cuda.synchronize()
+    for seed in range(4):
+        a.copy_(rnd(M, K, seed=10 + seed))
+        graph.replay()
+        torch.cuda.synchronize()
+        want, then = torch.empty_like(first), torch.empty_like(second)
+        ops.gemm_f32(want, a, w, None)
+        ops.gemm_f32(then, want, v, None)
+        assert torch.equal(first, want) and torch.equal(second, then)
+        torch.full((1 << 22,), float("nan"), device=DEV)  # what eager work between replays leaves in freed memory
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 70000, 8), (16, 140003, 16), (16, 100, 32), (70, 515, 24), (2100, 4100, 30), (800, 1000, 64),
                                    (2100, 5000, 96), (2100, 800, 100), (2100, 801, 99), (1030, 6200, 130), (1030, 2052, 192),
                                    (2100, 2052, 256), (2100, 2052, 255), (2100, 2052, 257)])
