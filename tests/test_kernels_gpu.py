@@ -1205,6 +1205,77 @@ def test_decode_attention_rotates_and_writes_like_the_separate_kernels(ops, nh, 
     assert torch.equal(bits(kc3), bits(kc1)) and torch.equal(bits(vc3), bits(vc1))
 
 
+@pytest.mark.parametrize("nh,nkv,d,dv,page", [(4, 1, 32, 32, 16), (4, 2, 64, 32, 16), (8, 2, 64, 64, 48),
+                                              (8, 2, 128, 128, 16), (4, 1, 128, 64, 32), (3, 3, 224, 224, 16),
+                                              (2, 2, 256, 128, 16)])
+@pytest.mark.parametrize("window", [0, 1, 17, 32, 33])
+@pytest.mark.parametrize("nsplit", [1, 2])
+def test_decode_attention_at_every_place_of_its_units_of_keys(ops, nh, nkv, d, dv, page, window, nsplit):
+    """Tokens at each of 100 positions: the token's own key at every place of a unit of 32 keys, ranges
+    that begin and end at every place of one, in a wave's first, second and later unit.  Pages that a token
+    does not see are not in its row of the table, and the null page holds NaN."""
+    dtype, n = torch.bfloat16, 100
+    kc, vc, table, _ = paged_setup([n], nkv, d, page, dtype, seed=d + page)
+    vc = vc[:, :, :dv].contiguous()
+    kc[0], vc[0] = float("nan"), float("nan")
+    rows = table[1].repeat(n, 1)
+    for pos in range(n):
+        first = max(0, pos - window + 1) if window else 0
+        rows[pos, : first // page] = 0
+        rows[pos, pos // page + 1:] = 0
+    qkv = rnd(n, nh * d + nkv * (d + dv), dtype=dtype, seed=3)
+    order = torch.arange(n, dtype=torch.int32, device=DEV)
+    part_o = torch.full((n * nh * nsplit, dv), float("nan"), device=DEV)
+    part_ml = torch.full((n * nh * nsplit, 2), float("nan"), device=DEV)
+    # every token sees the keys before it as they are in the cache and its own as it brings it
+    outs = []
+    for pos in range(n):  # a token at a time, so that no other writes into what it reads
+        out = torch.full((1, nh * dv), float("nan"), dtype=dtype, device=DEV)
+        ops.decode_attention(out, qkv[pos:pos + 1], kc.clone(), vc.clone(), table=rows, positions=order[pos:pos + 1],
+                             token_req=order[:1], slots=order[pos:pos + 1], nh=nh, nkv=nkv, d=d, dv=dv,
+                             scale=d ** -0.5, window=window, nsplit=nsplit, part_o=part_o, part_ml=part_ml, write_kv=True)
+        outs.append(out)
+    got = torch.cat(outs).double().cpu().view(n, nh, dv)
+    pg, off = table[1, torch.arange(n) // page].long(), torch.arange(n, device=DEV) % page
+    k = kc[pg, :, off].double().cpu()
+    v = vc[pg, :, :, off].double().cpu()
+    q = qkv.double().cpu()
+    for pos in range(n):
+        first = max(0, pos - window + 1) if window else 0
+        kk, vv = k[first: pos + 1].clone(), v[first: pos + 1].clone()
+        kk[-1] = q[pos, nh * d: (nh + nkv) * d].view(nkv, d)
+        vv[-1] = q[pos, (nh + nkv) * d:].view(nkv, dv)
+        g = nh // nkv
+        p = torch.softmax(torch.einsum("hd,khd->hk", q[pos, : nh * d].view(nh, d),
+                                       kk.repeat_interleave(g, 1)) * d ** -0.5, -1)
+        want = torch.einsum("hk,khd->hd", p, vv.repeat_interleave(g, 1))
+        # p and the result are rounded to bfloat16: half of 2^-8 of a sum of |v| <= 4.5, twice
+        assert torch.allclose(got[pos], want, atol=2e-2, rtol=1e-2), pos
+
+
+def test_decode_attention_keeps_infinite_values_and_the_bits_of_its_probabilities(ops):
+    """A value of infinity comes out as itself, not as no number; float32 results hold the probabilities to
+    16 bits: 2^-16 of sums of |v| of about one, against 64 bits."""
+    dtype, nh, nkv, d, page, n = torch.bfloat16, 4, 2, 64, 16, 75
+    kc, vc, table, dense = paged_setup([n], nkv, d, page, dtype, seed=5)
+    q = rnd(1, nh * d, dtype=dtype, seed=6)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    args = dict(table=table, positions=torch.tensor([n - 1], **i32), token_req=torch.zeros(1, **i32),
+                slots=torch.ones(1, **i32), nh=nh, nkv=nkv, d=d, scale=d ** -0.5)
+    out = torch.empty(1, nh * d, device=DEV)
+    ops.decode_attention(out, q, kc, vc, **args)
+    full_q = torch.zeros(n, nh, d, dtype=torch.float64)
+    full_q[n - 1] = q.double().cpu().view(nh, d)
+    want = plain.causal_gqa_attention(full_q, dense[0][0].double(), dense[0][1].double(), d ** -0.5)[n - 1]
+    assert float((out.double().cpu().view(nh, d) - want).abs().max()) < 2.0 ** -16
+    for key, value in ((3, float("inf")), (40, float("-inf")), (n - 1, float("inf"))):
+        vc2 = vc.clone()
+        vc2[int(table[1, key // page]), :, 7, key % page] = value
+        ops.decode_attention(out, q, kc, vc2, **args)
+        assert torch.all(out.view(nh, d)[:, 7] == value)
+        assert torch.isfinite(out.view(nh, d)[:, 8:]).all()
+
+
 @pytest.mark.parametrize("nsplit", [1, 5])
 def test_decode_attention_far_key_and_window(ops, nsplit):
     dtype = torch.bfloat16
