@@ -33,6 +33,7 @@
 #include <cstdlib>
 
 #include "attention_combine.h"
+#include "attention_decode_block.h"
 #include "device_utils.h"
 #include "kvcore_hip.h"
 
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
     const float* __restrict__ slopes, int chunk, const float* __restrict__ sinks, float* __restrict__ part_o,
     float* __restrict__ part_ml, int single,
     const float* __restrict__ cos_tab, const float* __restrict__ sin_tab, int rot_dim, int interleaved,
-    float cap_rate, const GateRows gate, int out_f32) {
+    float cap_rate, const GateRows gate, int out_f32, int single_pages, unsigned page_magic) {
   constexpr int kKeyBlocks = KB;
   constexpr int NJ = DV / 16;
   constexpr int NC = D / 32;
@@ -147,25 +148,82 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
   // tiles see many keys and its early tiles few, so a block takes tile n-1-p and then tile p
   // (p < n/2; the middle tile of an odd count once): every block of a request then walks
   // about the same number of key tiles.  Pairs are numbered request by request.
+  // A lane looks at one request, 16 at once: request by request, with two loads and a wait each, 29 single tokens
+  // before the block's own request cost it some 8 us.
   int req = -1, pair = 0, n_tiles = 0, q_begin = 0, q_end = 0;
-  {
+  if (num_reqs == 1) {  // scalar: one request needs no search (half a microsecond of 7 for 64 tokens)
+    q_begin = q_start[0];
+    q_end = q_start[1];
+    n_tiles = (q_end - q_begin + bq - 1) / bq;
+    pair = block_index;
+    req = pair < (single ? n_tiles : (n_tiles + 1) / 2) ? 0 : -1;
+  } else {
     int idx = block_index;
-    for (int r = 0; r < num_reqs; ++r) {
+    for (int r0 = 0; r0 < num_reqs; r0 += 16) {
+      const int r = r0 + col < num_reqs ? r0 + col : num_reqs - 1;
       const int b = q_start[r], e = q_start[r + 1];
       const int tiles_r = (e - b + bq - 1) / bq;
-      const int pairs_r = single ? tiles_r : (tiles_r + 1) / 2;
-      if (idx < pairs_r) {
-        req = r;
-        pair = idx;
-        n_tiles = tiles_r;
-        q_begin = b;
-        q_end = e;
+      const int pairs_r = r0 + col >= num_reqs ? 0 : single ? tiles_r : (tiles_r + 1) / 2;
+      int upto = pairs_r;  // pairs of this lane's request and those before it, among 16 lanes
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, true);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, true);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, true);
+      upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, true);
+      const unsigned long long beyond = __ballot(upto > idx);
+      if (beyond != 0) {
+        const int at = __builtin_ctzll(beyond);
+        req = r0 + at;
+        pair = idx - __builtin_amdgcn_readlane(upto - pairs_r, at);
+        n_tiles = __builtin_amdgcn_readlane(tiles_r, at);
+        q_begin = __builtin_amdgcn_readlane(b, at);
+        q_end = __builtin_amdgcn_readlane(e, at);
         break;
       }
-      idx -= pairs_r;
+      idx -= __builtin_amdgcn_readlane(upto, 15);
     }
   }
   if (req < 0) return;  // the grid is an upper bound on the number of pairs
+  // A request that brings one token has g rows, of the 16 a wave has room for, and its keys would be walked by one wave:
+  // its blocks work as those of the kernel for single tokens do, all waves on the keys.
+  if constexpr (DV <= D) {
+    if (q_end - q_begin == 1 && positions[q_begin] / page_size + 2 <= single_pages) {
+      decode::DecodeArgs one = {};
+      one.out = out;
+      one.out_f32 = out_f32;
+      one.part_o = part_o;
+      one.part_ml = part_ml;
+      one.qkv = q;
+      one.qkv_stride = q_stride;
+      one.k_cache = const_cast<bf16_t*>(k_cache);  // read only: write_kv is 0
+      one.v_cache = const_cast<bf16_t*>(v_first);
+      one.table = table;
+      one.table_stride = table_stride;
+      one.positions = positions;
+      one.cos_tab = cos_tab;
+      one.sin_tab = sin_tab;
+      one.rot_dim = cos_tab != nullptr ? rot_dim : 0;
+      one.interleaved = interleaved;
+      one.nh = nh;
+      one.nkv = nkv;
+      one.page_size = page_size;
+      one.num_pages = num_pages;
+      one.scale_log2e = scale_log2e;
+      if (CAP_GATE) {
+        one.cap_rate = cap_rate;
+        one.cap_log2e = scale_log2e;
+        one.gate = gate;
+      }
+      one.window = window;
+      one.slopes = slopes;
+      one.chunk = chunk;
+      one.sinks = sinks;
+      one.page_magic = page_magic;
+      one.nsplit = gridDim.z;
+      one.lds_pages = single_pages;
+      decode::decode_block<D, DV>(one, q_begin, hk, blockIdx.z, slots[req], reinterpret_cast<unsigned char*>(tiles));
+      return;
+    }
+  }
   const int32_t* row_table = table + static_cast<int64_t>(slots[req]) * table_stride;
   for (int turn = 0; turn < 2; ++turn) {
   const int tile = (turn == 0) ? n_tiles - 1 - pair : pair;
@@ -723,6 +781,9 @@ int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16
   const int64_t wide = (8 % nkv == 0) ? static_cast<int64_t>((max_pairs + 8 / nkv - 1) / (8 / nkv)) * 8
                                       : (static_cast<int64_t>(max_pairs) * nkv + 7) / 8 * 8;
   if (wide > 0x7fffffff) return kvc_fail("kvc_prefill_attention: too many blocks");
+  // page ids that a request of one token finds room for in LDS (more: it is walked like any other)
+  const int single_pages = g <= 16 && DV <= D ? (lds_bytes - static_cast<int>(decode::lds_total(W, g, D, 0))) / 4 : 0;
+  const unsigned page_magic = decode::page_magic_of(page_size);
   char variant[64];
   snprintf(variant, sizeof(variant), "prefill_attention_kernel<%d,%d,%d,%d>%s x%d", D, CT, KB, W,
            single ? " one tile a block" : "", nsplit);
@@ -731,7 +792,7 @@ int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16
                      lds_bytes, stream, out, q, q_stride, k_cache, v_cache, v_second, table, table_stride, positions,
                      q_start, slots, R, nh, nkv, page_size, num_pages, (softcap > 0.f ? softcap : scale) * kLog2e, window,
                      slopes, chunk, sinks, part_o, part_ml, single, cos_tab, sin_tab, rot_dim, interleaved,
-                     softcap > 0.f ? 2.f * kLog2e * scale / softcap : 0.f, gate, out_f32);
+                     softcap > 0.f ? 2.f * kLog2e * scale / softcap : 0.f, gate, out_f32, single_pages, page_magic);
   if (nsplit > 1)
     return launch_attention_combine(out, part_o, part_ml, static_cast<int64_t>(T) * nh, DV, nsplit, out_f32, gate, stream);
   return kvc_check_launch("kvc_prefill_attention");
@@ -744,52 +805,86 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
                    int R, int nh, int nkv, int page_size, int num_pages, float scale, int window,
                    const float* slopes, int chunk, const float* sinks, float* part_o, float* part_ml, int nsplit,
                    const float* cos_tab, const float* sin_tab,
-                   int rot_dim, int interleaved, float softcap, const GateRows& gate, int out_f32, hipStream_t stream) {
+                   int rot_dim, int interleaved, float softcap, const GateRows& gate, int out_f32, int singles,
+                   int context, hipStream_t stream) {
   const int g = nh / nkv;
-  // Blocks of four waves lie two to a compute unit, blocks of eight waves one.  Tiles of 64
-  // query rows, two a block one after the other (a late and an early one), are the fastest as
-  // long as all their blocks find room at once; more rows than that take tiles of 128 rows,
-  // which stage each key tile for twice the rows (and so does a launch that splits the keys,
-  // unless its rows are very few: its caller splits until there are blocks enough).  Few rows
-  // take one tile of 64 a block, for twice the blocks.  Where the requests are long, blocks of
-  // eight waves (tiles of 128 or 256 rows) halve the loads and LDS writes per row once more.
-  // Measured at 32 heads over 8 kv heads of 128, one request, four waves against eight:
-  // 1,024 tokens 36 against 38 us, 1,536 tokens 64 against 56, 2,048 tokens 83 against 77,
-  // 3,072 tokens 149 against 144, 8,192 tokens 699 against 672; four requests of 512 tokens 29
-  // (tiles of 64 rows) and 33 (tiles of 128) against 40 (eight waves, tiles of 256).  Heads
-  // of 64: 1,024 tokens 27 against 23, 2,048 tokens 54 against 43, 8,192 tokens 445 against 393.
-  // (every request but one may add a ragged tile)
+  // Blocks of four waves lie two to a compute unit, blocks of eight waves one.  A wave takes 16 query rows of a tile of keys
+  // at a time (ct 1) or 32 (ct 2, cheaper per key); a block takes one tile of its rows (single) or two, a late one and
+  // then an early one.  What decides is how many tiles of 64 rows the portions have (blocks: times the kv heads) against
+  // the compute units, and whether all blocks find room at once.  Single tokens are blocks of their own kind that take a
+  // place for a short while.  Measured over 1,000 launches of 1 to 8 portions of 30 to 2,048 tokens, from position 0 and
+  // behind 200 to 1,200 tokens, alone and beside 24 single tokens, against the best of all ways:
+  // Up to cu blocks one tile of 64 rows a block (others 1.05 to 1.6).  Up to 2 cu tiles of 128 rows, eight waves, from 11/8 cu
+  // on, where they and the single tokens' blocks find a unit each (0.79 to 1.04 of tiles of 64 rows; below 11/8 cu, which
+  // leaves them too few, 0.89 to 1.3); else four (beside many single tokens 1.00 to
+  // 1.03, eight waves 1.04 to 1.18).
+  //
+  // Whole prompts of more: their early tiles see few keys and their late ones many, so a block takes two.  At 32 heads over 8
+  // kv heads of 128, one request, four waves against eight: 2,048 tokens 83 against
+  // 77, 3,072 tokens 149 against 144, 8,192 tokens 699 against 672; four requests of 512 tokens 29 (tiles of 64 rows)
+  // and 33 (tiles of 128) against 40 (eight waves, tiles of 256).  Heads of 64: 2,048 tokens 54
+  // against 43, 8,192 tokens 445 against 393.
+  //
+  // Portions behind a context, or beside single tokens, have tiles of like lengths (two a block 1.1 to 1.45 below 4 cu): up
+  // to 4 cu heads of 64 four waves (1.00 to 1.05), two tiles a block of eight waves where those just fill the chip (1.06 to
+  // 1.09); heads of 128 32 rows a wave (1.00 to 1.08), except that long requests pair their tiles.
+  //
+  // With splits of the keys: one tile of 64 rows a block up to cu (1.00 to 1.07; 32 rows a wave and two tiles a block 1.2 to
+  // 1.75), on heads of 64 up to 3 cu (1.00 to 1.08; with values of 128 up to 2 cu), else 32 rows a wave, one tile a block
+  // on heads of 128 (1.00 to 1.02).
+  const int ones = g <= 16 && DV <= D ? singles : 0;  // single tokens that are blocks of their own kind
+  const int T1 = T - ones, R1 = R - ones > 1 ? R - ones : 1;
   const int bq1 = 64 / g > 0 ? 64 / g : 1;
-  const int tiles1 = (T + bq1 - 1) / bq1 + (R - 1);
-  const int64_t pairs1 = static_cast<int64_t>((tiles1 + 1) / 2) * nkv;
-  const int64_t small_tiles = static_cast<int64_t>(tiles1) * nkv;
-  const bool long_requests = T / R >= (D == 64 ? 512 : 1024);
-  // the thresholds below were measured on 256 compute units and are kept as multiples of them
+  const int tiles1 = (T1 + bq1 - 1) / bq1 + (R1 - 1);  // every request but one may add a ragged tile
+  const int64_t blocks = static_cast<int64_t>(tiles1) * nkv;
+  const int64_t pairs = static_cast<int64_t>((tiles1 + 1) / 2) * nkv;
+  const int64_t single_blocks = static_cast<int64_t>(ones) * nkv;
+  const bool long_requests = T1 / R1 >= (D == 64 ? 512 : 1024);
+  const bool whole_prompts = ones == 0 && 4 * static_cast<int64_t>(context) < T1 / R1;
+  // the thresholds were measured on 256 compute units and are kept as multiples of them
   const int cu = kvc_device_compute_units();
-  int ct = 1, single = 0, waves = 4;
+  int ct = 1, single = 1, waves = 4;
   if (g > 64) {
     ct = 2;
+    single = 0;
   } else if (nsplit > 1) {
-    // very few rows: small tiles one a block reach the blocks wanted with a quarter of the
-    // splits (128 rows at 1,024 keys: 21 against 39 us)
-    if (small_tiles <= cu / 2) {
-      single = 1;
-    } else {
-      ct = 2;
-      if (long_requests) waves = 8;  // 2,048 tokens after 30,000: 1.38 against 1.32 ms
+    if (blocks > (DV > D ? 2 : D == 64 ? 3 : 1) * cu) ct = 2;
+    if (D == 64 && ct == 2) {  // 2,048 tokens behind 1,200: two tiles a block of eight waves 0.97, one of four 1.09
+      single = 0;
+      if (long_requests) waves = 8;
     }
-  } else if (pairs1 > 2 * cu) {
-    ct = 2;
-    if (long_requests) waves = 8;
-  } else if (pairs1 > cu) {
-    if (long_requests) {
+  } else if (blocks <= cu) {
+  } else if (DV <= D && blocks <= 2 * cu) {
+    if (blocks / 2 + single_blocks <= cu && 8 * blocks > 11 * cu) waves = 8;
+  } else if (whole_prompts || DV > D) {
+    if (pairs > 2 * cu) {
+      ct = 2;
+      single = 0;
+      if (long_requests) waves = 8;
+    } else if (pairs > cu) {
+      if (long_requests) waves = 8;
+      single = long_requests && pairs <= 7 * cu / 4;
+    } else if (long_requests && ((D == 64 && pairs > cu / 2) || (D == 128 && DV < D))) {
       waves = 8;
-      single = pairs1 <= 7 * cu / 4;
+    }
+  } else if (blocks <= 4 * cu + nkv) {
+    if (D == 64) {
+      if (blocks > 3 * cu && blocks / 4 + single_blocks <= cu + nkv) {
+        waves = 8;
+        single = 0;
+      }
+    } else if (blocks > 3 * cu && long_requests) {
+      waves = 8;
+      single = 0;
+    } else if (blocks <= 3 * cu && single_blocks == 0) {
+      waves = 8;
+    } else if (2 * blocks > 5 * cu) {
+      ct = 2;
     }
   } else {
-    single = 1;
-    // keys of 128 with values of 64, one request: 2,048 tokens 45.8 against 40.8 us (16 heads over 4)
-    if (long_requests && ((D == 64 && pairs1 > cu / 2) || (D == 128 && DV < D))) waves = 8;
+    ct = 2;
+    single = 0;
+    if (long_requests) waves = 8;
   }
   // KVC_PREFILL_MODE = 1p | 1s | 2p | 2s, then 4 or 8 (waves), overrides the choice for tuning
   static const char* mode = getenv("KVC_PREFILL_MODE");
@@ -838,14 +933,15 @@ extern "C" int kvc_prefill_attention(void* out, const void* q, int64_t q_stride,
                                      int page_size, int num_pages, float scale, int window,
                                      const float* slopes, int chunk, const float* sinks, void* part_o, void* part_ml, int nsplit, const float* cos_tab,
                                      const float* sin_tab, int rot_dim, int interleaved, float softcap,
-                                     const void* gate_rows, int64_t gate_stride, int out_f32, kvc_stream stream) {
+                                     const void* gate_rows, int64_t gate_stride, int out_f32, int singles,
+                                     int context, kvc_stream stream) {
   const bool two = v_second != nullptr;
   if (two && (d != 64 || dv != 128 || softcap > 0.f || gate_rows != nullptr))
     return kvc_fail("kvc_prefill_attention: values in two planes are 128 wide on keys of 64, without a cap or a gate");
   if (!kvc_prefill_attention_supported(nh, nkv, d, two ? d : dv, page_size, 1))
     return kvc_fail("kvc_prefill_attention: unsupported shape (bfloat16, head size 64 or 128, values as "
                     "wide or half as wide, at most 64 query heads per kv head, page size a multiple of 16)");
-  if (T < 0 || R <= 0 || nkv > 65535 || table_stride <= 0 || num_pages <= 0)
+  if (T < 0 || R <= 0 || nkv > 65535 || table_stride <= 0 || num_pages <= 0 || singles < 0 || singles > R || context < 0)
     return kvc_fail("kvc_prefill_attention: bad sizes");
   if (!(scale > 0.f)) return kvc_fail("kvc_prefill_attention: the scale must be positive");
   if (q_stride % 8) return kvc_fail("kvc_prefill_attention: q rows must be 16-byte aligned");
@@ -876,7 +972,8 @@ extern "C" int kvc_prefill_attention(void* out, const void* q, int64_t q_stride,
 #define KVC_PREFILL(D_, DV_)                                                                                      \
   return launch_prefill<D_, DV_>(static_cast<bf16_t*>(out), qq, q_stride, kc, vc, vc2, table, table_stride, positions, \
                                  q_start, slots, T, R, nh, nkv, page_size, num_pages, scale, window, slopes, chunk, \
-                                 sinks, po, pml, nsplit, cos_tab, sin_tab, rot_dim, interleaved, softcap, gate, out_f32, s)
+                                 sinks, po, pml, nsplit, cos_tab, sin_tab, rot_dim, interleaved, softcap, gate, out_f32, \
+                                 singles, context, s)
   if (d == 64) {
     if (two) KVC_PREFILL(64, 128);
     if (dv == d) KVC_PREFILL(64, 64);

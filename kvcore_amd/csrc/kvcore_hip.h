@@ -423,6 +423,8 @@ int kvc_decode_attention(void* out, void* part_o, void* part_ml, const void* qkv
 // and are rotated on their way in, as kvc_rope_kv_write would have (rot_dim a multiple of 64,
 // or of 32 when interleaved); without, they are taken as they are.  With v_second values have 128 elements on keys of 64, the
 // first 64 in v_cache and the others in v_second, pages of both alike (no softcap, no gate).
+// singles: how many of the requests bring one token, context: how many tokens lie behind the others in the mean (0: not
+// known), which decide with T and R how the launch is cut.
 int kvc_prefill_attention_supported(int nh, int nkv, int d, int dv, int page_size, int dtype);
 int kvc_prefill_attention(void* out, const void* q, int64_t q_stride, const void* k_cache,
                           const void* v_cache, const void* v_second, const int32_t* table, int table_stride,
@@ -431,7 +433,8 @@ int kvc_prefill_attention(void* out, const void* q, int64_t q_stride, const void
                           float scale, int window, const float* slopes, int chunk, const float* sinks, void* part_o,
                           void* part_ml, int nsplit,
                           const float* cos_tab, const float* sin_tab, int rot_dim, int interleaved,
-                          float softcap, const void* gate, int64_t gate_stride, int out_f32, kvc_stream stream);
+                          float softcap, const void* gate, int64_t gate_stride, int out_f32, int singles,
+                          int context, kvc_stream stream);
 
 // ---- norms after a sublayer, norms over a whole projection, gates per head (norm_ops.hip)
 // residual[t, :] += post_gain * delta[t, :] / sqrt(mean(delta[t, :]^2) + eps), and then, if out is

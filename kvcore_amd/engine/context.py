@@ -127,6 +127,17 @@ class StepContext:
     scratch: dict = field(default_factory=dict)  # per-step values parts share (rotary tables)
     token_rows: torch.Tensor | None = None
 
+    @property
+    def portion_counts(self) -> dict[str, int]:
+        """How many of the step's requests bring one token (``singles``) and how many tokens the others have
+        behind them in the mean (``context``); counted once a step."""
+        got = self.scratch.get("portion_counts")
+        if got is None:
+            behind = [n - q for q, n in zip(self.host_query_lens, self.host_seq_lens) if q > 1]
+            got = self.scratch["portion_counts"] = dict(singles=len(self.host_query_lens) - len(behind),
+                                                        context=sum(behind) // max(len(behind), 1))
+        return got
+
     def buf(self, name: str, cols: int, dtype: torch.dtype | None = None, rows: int | None = None) -> torch.Tensor:
         return self.buffers.get(name, self.num_tokens if rows is None else rows, cols,
                                 self.dtype if dtype is None else dtype,

@@ -96,7 +96,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_decode_attention_max_table": [I, I, I],
         "kvc_decode_attention_supported": [I, I, I, I, I, I],
         "kvc_prefill_attention": [P, P, L, P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, P, I, P, P, P, I,
-                                  P, P, I, I, F, P, L, I, P],
+                                  P, P, I, I, F, P, L, I, I, I, P],
         "kvc_prefill_attention_supported": [I, I, I, I, I, I],
         "kvc_gemm_mid_slices": [I, I],
         "kvc_gemm_mid_bf16": [P, P, P, P, P, I, I, I, L, L, I, I, F, F, F, I, P],
@@ -819,7 +819,7 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
                       sin: torch.Tensor | None = None, rot_dim: int = 0, interleaved: bool = False,
                       slopes: torch.Tensor | None = None, chunk: int = 0,
                       sinks: torch.Tensor | None = None, dv: int | None = None, softcap: float = 0.0,
-                      gate: torch.Tensor | None = None, v_second: torch.Tensor | None = None) -> None:
+                      gate: torch.Tensor | None = None, v_second: torch.Tensor | None = None, singles: int = 0, context: int = 0) -> None:
     """bfloat16 attention of portions of prompts on the matrix cores (see the C header).
     ``nsplit > 1`` deals every tile's keys to that many blocks; ``part_o`` (float32,
     ``T*nh*nsplit*dv`` values) and ``part_ml`` (``T*nh*nsplit*2``) are then the workspace.
@@ -827,7 +827,9 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
     holds the other half of every value head; keys of 64, no cap, no gate) twice.  ``softcap`` and ``gate`` as for
     :func:`paged_attention` (the gate's rows 8-byte aligned).
     With ``cos`` and ``sin`` (``[T, rot_dim / 2]`` float32) the queries come unrotated and
-    the kernel rotates them (``prefill_attention_rotates`` says for which shapes)."""
+    the kernel rotates them (``prefill_attention_rotates`` says for which shapes).
+    ``singles``: how many of the requests bring one token, ``context``: how many tokens the others have behind
+    them in the mean; both for the choice of the launch alone (0 where they are not known)."""
     T = out.shape[0]
     dv = d if dv is None else dv
     if out.shape != (T, nh * dv) or not out.is_contiguous() or out.dtype not in (torch.bfloat16, torch.float32):
@@ -859,7 +861,8 @@ def prefill_attention(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor,
         _dev(q_start, "q_start", torch.int32), _dev(slots, "slots", torch.int32), T, num_reqs,
         nh, nkv, d, dv, page_size, num_pages, float(scale), int(window), _slopes(slopes, nh), int(chunk),
         _sinks(sinks, nh), po, pml, int(nsplit), cs, sn, int(rot_dim) if cs is not None else 0, int(interleaved),
-        float(softcap), *_gate(gate, T, nh * dv, torch.bfloat16), int(out.dtype == torch.float32), _stream()),
+        float(softcap), *_gate(gate, T, nh * dv, torch.bfloat16), int(out.dtype == torch.float32), int(singles), int(context),
+        _stream()),
         "kvc_prefill_attention")
 
 

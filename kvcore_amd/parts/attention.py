@@ -47,11 +47,9 @@ PREFILL_MAX_SPLITS = 32
 def prefill_splits(T: int, nkv: int, g: int, max_query_len: int, max_seq_len: int, window: int,
                    num_reqs: int = 1) -> int:
     """How many blocks share the keys of one tile of query rows in the kernel for portions
-    of prompts.  A compute unit holds two of its blocks, so a launch wants some 512.  The
-    kernel has tiles of 64 rows (one or two a block) and of 128 (two a block, cheaper per
-    key); with splits it takes the small tiles one a block for very few rows and the large
-    ones otherwise (`launch_prefill` in csrc/attention_prefill.hip, which must agree with
-    this on where "very few" ends).  Measured on the 8B shape: splits pay when the rows are
+    of prompts.  A compute unit holds two of its blocks, so a launch wants some 512; the
+    kernel's own choice of tiles is `launch_prefill` in csrc/attention_prefill.hip.
+    Measured on the 8B shape: splits pay when the rows are
     few and every block still has a few hundred keys to walk, a thousand for steps of a
     thousand tokens (a row sees ``max_seq_len`` keys at most and, under the causal mask,
     about half a portion fewer on average).  Every request but one may add a ragged tile."""
@@ -481,6 +479,7 @@ class PagedAttention(Mixer):
                                       d=self.head_dim, dv=dv, scale=self.scale, window=self.window,
                                       slopes=self._slopes, chunk=self.chunk, sinks=sinks, softcap=self.softcap, gate=gate,
                                       nsplit=nsplit, part_o=part_o, part_ml=part_ml, v_second=v_second,
+                                      **ctx.portion_counts,
                                       **(dict(cos=cos, sin=sin, rot_dim=rot_dim, interleaved=interleaved)
                                          if rotates else {}))
             else:

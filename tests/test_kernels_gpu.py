@@ -1702,6 +1702,64 @@ def test_decode_attention_long_context(ops, nsplit):
             assert torch.allclose(got[r, h], want, atol=1e-2, rtol=1e-2), (n, h)
 
 
+@pytest.mark.parametrize("nh,nkv,d,dv,page", [(8, 2, 128, 128, 16), (8, 2, 64, 64, 32), (4, 4, 64, 32, 16),
+                                              (16, 1, 128, 64, 48), (40, 2, 64, 64, 16)])
+@pytest.mark.parametrize("extra", ["none", "rotated", "interleaved", "window", "chunk", "slopes", "sinks", "capped", "gated"])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_prefill_attention_of_single_tokens_beside_portions(ops, nh, nkv, d, dv, page, extra, nsplit):
+    """Requests that bring one token are blocks of another kind than portions: more of them than one look at the
+    requests covers, before, between and behind portions, at edges of units of keys and pages, with every option, against
+    the general kernel.  (With 20 query heads a kv head they are walked as portions are.)"""
+    dtype = torch.bfloat16
+    spans = [(0, 1), (15, 1), (16, 1), (30, 40), (31, 1), (32, 1), (33, 1), (640, 1), (0, 70)] + [(90 + i, 1) for i in range(20)]
+    seq_lens = [p + n for p, n in spans]
+    kc, vc, table, _ = paged_setup(seq_lens, nkv, d, page, dtype, seed=d + nsplit)
+    vc = vc[:, :, :dv].contiguous()
+    R, T = len(spans), sum(n for _, n in spans)
+    positions = torch.tensor([p + i for p, n in spans for i in range(n)], dtype=torch.int32, device=DEV)
+    token_req = torch.tensor([r for r, (_, n) in enumerate(spans) for _ in range(n)], dtype=torch.int32, device=DEV)
+    q_start = torch.tensor([0] + [sum(n for _, n in spans[:r + 1]) for r in range(R)], dtype=torch.int32, device=DEV)
+    slots = torch.arange(1, R + 1, dtype=torch.int32, device=DEV)
+    q = rnd(T, nh * d, dtype=dtype, seed=4)
+    options, turn = {}, {}
+    if extra in ("rotated", "interleaved"):
+        cos, sin = torch.empty(T, d // 2, device=DEV), torch.empty(T, d // 2, device=DEV)
+        ops.rope_table(cos, sin, positions, plain.rope_inv_freq(d, 10000.0).float().to(DEV))
+        turn = dict(cos=cos, sin=sin, rot_dim=d, interleaved=extra == "interleaved")
+    elif extra == "window":
+        options["window"] = 33
+    elif extra == "chunk":
+        options["chunk"] = 48
+    elif extra == "slopes":
+        options["slopes"] = torch.linspace(0.01, 0.3, nh, device=DEV)
+    elif extra == "sinks":
+        options["sinks"] = torch.linspace(-2, 2, nh, device=DEV)
+    elif extra == "capped":
+        options["softcap"] = 5.0
+    elif extra == "gated":
+        options["gate"] = rnd(T, nh * dv, dtype=dtype, seed=8)
+    common = dict(table=table, positions=positions, slots=slots, nh=nh, nkv=nkv, d=d, dv=dv, scale=d ** -0.5, **options)
+    out = torch.full((T, nh * dv), float("nan"), dtype=dtype, device=DEV)
+    ops.prefill_attention(out, q, kc, vc, q_start=q_start, num_reqs=R, nsplit=nsplit, singles=R - 2, context=15,
+                          part_o=torch.full((T * nh * nsplit, dv), float("nan"), device=DEV),
+                          part_ml=torch.full((T * nh * nsplit, 2), float("nan"), device=DEV), **turn, **common)
+    if turn:  # the general kernel takes queries that are turned
+        qkv = torch.cat([q, torch.zeros(T, nkv * (d + dv), dtype=dtype, device=DEV)], 1)
+        x = qkv[:, : nh * d].float().view(T, nh, d)
+        if extra == "interleaved":
+            a, b = x[..., 0::2], x[..., 1::2]
+        else:
+            a, b = x[..., : d // 2], x[..., d // 2:]
+        c, s = cos[:, None], sin[:, None]
+        turned = torch.stack([a * c - b * s, b * c + a * s], -1) if extra == "interleaved" else \
+            torch.cat([a * c - b * s, b * c + a * s], -1)
+        q = turned.reshape(T, nh * d).to(dtype)
+    ref = torch.empty_like(out)
+    ops.paged_attention(ref, q, kc, vc, token_req=token_req, **common)
+    # both round p and the result to bfloat16: half of 2^-8 of sums of |v| <= 4.5, twice each
+    assert torch.allclose(out.float(), ref.float(), atol=2e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("nh,nkv,d,whole,nsplit", [(8, 2, 128, 2100, 1), (8, 1, 64, 2100, 1), (32, 8, 128, 4200, 1),
                                                    (8, 2, 128, 2100, 7), (8, 1, 64, 2100, 2),
                                                    (16, 4, 128, 2100, 1), (16, 4, 128, 3100, 1),
