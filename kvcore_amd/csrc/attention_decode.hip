@@ -26,13 +26,13 @@
 // from a block's start to its end are 0.9 until the token's row is known, 0.5 for its pages, 3.2 for
 // the burst of keys and values of all blocks (a unit's loads are all in flight together), 0.6 for the
 // rotation behind them, 0.5 for scores and values, 0.8 for the merge; 64 tokens of 450 keys read
-// 118 MB at 4.4 TB/s.  A compute unit draws some 45 GB/s, so few blocks of many keys are the slower
+// 118 MB at 4.8 TB/s.  A compute unit draws some 45 GB/s, so few blocks of many keys are the slower
 // ones.  Every load is asked for as early as its address is known and waits for nothing else: the
 // queries before the pages, units only where there are some, and barriers that do not wait for
 // global memory.  Before (units of 16 keys, barriers that did, the merge's reads one by one) and now,
-// in a graph: 8 tokens x 512 keys of 128 in four splits 14.2 -> 11.7 us, of 64 11.7 -> 9.7; one token, 512 keys of
-// 64 in eight splits 10.5 -> 8.8; 64 tokens x 450 keys of 128 34.9 -> 29.7, of 64 21.8 -> 18.5; 4 tokens x 1,024 of
-// 256 in eight splits 19.9 -> 15.3.
+// in a graph: 8 tokens x 512 keys of 128 in four splits 14.2 -> 11.0 us, of 64 11.7 -> 9.6; one token, 512 keys of
+// 64 in eight splits 10.5 -> 9.0; 64 tokens x 450 keys of 128 34.9 -> 27.9, of 64 21.8 -> 17.3; 4 tokens x 1,024 of
+// 256 in eight splits 19.9 -> 15.8 (with loads marked as streaming ones, `read8`: 11.7, 9.7, 8.8, 29.7, 18.5 and 15.3 without).
 //
 // The block first rotates the group's query heads into LDS.  The block whose range holds
 // the token's own position also rotates the key, stores key and value in their cache slot

@@ -9,12 +9,10 @@
 
 #include "attention_combine.h"
 #include "device_utils.h"
+#include "gemm_common.h"
 
 namespace kvc {
 namespace decode {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kMaxWaves = 8;
@@ -219,7 +217,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) un.k[h][c] = *reinterpret_cast<const bf16x8_t*>(krow + h * 4 * D + 32 * c);
+      for (int c = 0; c < NC; ++c) un.k[h][c] = once8(krow + h * 4 * D + 32 * c);
   };
   auto issue_values = [&](Unit& un, int u) {
     int64_t base[2];
@@ -229,7 +227,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
     const int64_t v0 = base[0] * DV * page_size + sub[0], v1 = base[1] * DV * page_size + sub[1];
     const bf16_t* vrow = a.v_cache + (quad >= 2 ? v1 : v0) + (col * page_size + 8 * (quad & 1));
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) un.v[j] = *reinterpret_cast<const bf16x8_t*>(vrow + j * 16 * page_size);
+    for (int j = 0; j < NJ; ++j) un.v[j] = once8(vrow + j * 16 * page_size);
   };
 
   // the first unit of this wave is asked for at once, before anything else waits

@@ -13,6 +13,19 @@ namespace kvc {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
+// Sixteen bytes; ONCE: of a matrix that the whole launch reads once.  Such loads are marked as streaming ones: 512 MB in
+// runs of 64 KB a wave are read at 6.6 TB/s with the mark and at 6.25 without (the caches need not make room for
+// them, and keep the rows).  Steps with them in the products of few and of some dozen rows, in the experts' tiles and on
+// keys and values of single tokens: 8B shape, 8 tokens 3,478 -> 3,271 us, 64 tokens 5,005 -> 4,835, 1B, one token 901 ->
+// 856.  Where several blocks share a matrix through the L2 the mark costs more than it brings.
+template <bool ONCE>
+__device__ __forceinline__ bf16x8_t read8(const void* p) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  const u32x4_t* from = static_cast<const u32x4_t*>(p);
+  return __builtin_bit_cast(bf16x8_t, ONCE ? __builtin_nontemporal_load(from) : *from);
+}
+__device__ __forceinline__ bf16x8_t once8(const void* p) { return read8<true>(p); }
+
 __device__ __forceinline__ bf16x8_t zero8() {
   bf16x8_t z;
 #pragma unroll

@@ -112,8 +112,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mid_kernel(
     const int k = 64 * where(step);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      wbuf[stage][rt][0] = *reinterpret_cast<const bf16x8_t*>(wp[rt] + k * ks);
-      wbuf[stage][rt][1] = *reinterpret_cast<const bf16x8_t*>(wp[rt] + (k + 32) * ks);
+      wbuf[stage][rt][0] = once8(wp[rt] + k * ks);
+      wbuf[stage][rt][1] = once8(wp[rt] + (k + 32) * ks);
     }
   };
   auto fetch_chunk = [&](int slot, int chunk) {

@@ -131,8 +131,8 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
     const int k = k_begin + 64 * step;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      abuf[stage][rt][0] = *reinterpret_cast<const bf16x8_t*>(wp[rt] + static_cast<int64_t>(k) * ks);
-      abuf[stage][rt][1] = *reinterpret_cast<const bf16x8_t*>(wp[rt] + static_cast<int64_t>(k + 32) * ks);
+      abuf[stage][rt][0] = once8(wp[rt] + static_cast<int64_t>(k) * ks);
+      abuf[stage][rt][1] = once8(wp[rt] + static_cast<int64_t>(k + 32) * ks);
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
   for (; k < k_full; k += 32) {
     bf16x8_t a[RT], b[NT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) a[rt] = *reinterpret_cast<const bf16x8_t*>(wp[rt] + static_cast<int64_t>(k) * ks);
+    for (int rt = 0; rt < RT; ++rt) a[rt] = once8(wp[rt] + static_cast<int64_t>(k) * ks);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b[nt] = *reinterpret_cast<const bf16x8_t*>(ap[nt] + k);
 #pragma unroll
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
     bf16x8_t a[RT], b[NT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
-      a[rt] = valid ? *reinterpret_cast<const bf16x8_t*>(wp[rt] + static_cast<int64_t>(k_full) * ks) : zero8();
+      a[rt] = valid ? once8(wp[rt] + static_cast<int64_t>(k_full) * ks) : zero8();
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       b[nt] = valid ? *reinterpret_cast<const bf16x8_t*>(ap[nt] + k_full) : zero8();

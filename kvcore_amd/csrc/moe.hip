@@ -38,6 +38,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "device_utils.h"
 #include "gemm_common.h"
@@ -653,6 +654,13 @@ __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
 // passes long a share of it is one or two, and with many tiles four times the blocks cost more than they bring
 // (kvc_moe_gemm has the line): 128 experts of 1024 x 384, 8 rows each, down 37.0 us with WK 4, 20.8 with WK 1
 // (two passes on their way: with four 22.6).
+// An expert that has one tile has its matrices read once, with loads that say so (`read8`): eight tokens 64 and 34 ->
+// 57 and 30 us (6.0 TB/s), 256 pairs 93 and 49 -> 83 and 46.  Where two tiles share a matrix through the L2 such loads cost
+// more than they bring (256 pairs, half of them with few experts, 160 -> 196 us), so those keep the others.
+__device__ __forceinline__ bool only_tile(const int32_t* tiles, int tile, int num_tiles) {  // an expert's are side by side
+  const int e = tiles[3 * tile];
+  return (tile == 0 || tiles[3 * tile - 3] != e) && (tile + 1 >= num_tiles || tiles[3 * tile + 3] != e);
+}
 template <int GATED, typename TO, int PACKED, int WK>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
@@ -686,6 +694,9 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   const int passes = K / 64;
   // blocks walk K round from places of their own, as in the kernel for more rows
   const int turn = passes > 0 ? (e * 5 + (n0 >> 4) * 3) % passes : 0;
+  // ONCE: this tile holds all rows of its expert, so nothing else reads the matrix (see `once8`)
+  auto walk = [&](auto once) {
+  constexpr bool ONCE = decltype(once)::value;
   bf16x8_t an[kStages][2], a2n[kStages][2], bn[kStages][2];
   auto fetch = [&](int slot, int pass) {  // no branch around the loads: a pass that is not there repeats the last
     int p = pass < passes ? pass + turn : passes - 1 + turn;
@@ -693,8 +704,8 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int64_t wo = PACKED ? static_cast<int64_t>(2 * p + h) * 512 : 64 * p + 8 * h;
-      an[slot][h] = *reinterpret_cast<const bf16x8_t*>(wr + wo);
-      if (GATED) a2n[slot][h] = *reinterpret_cast<const bf16x8_t*>(wr2 + wo);
+      an[slot][h] = read8<ONCE>(wr + wo);
+      if (GATED) a2n[slot][h] = read8<ONCE>(wr2 + wo);
       bn[slot][h] = *reinterpret_cast<const bf16x8_t*>(xr + 64 * p + (PACKED ? 32 : 8) * h);
     }
   };
@@ -721,6 +732,9 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
       }
     }
   }
+  };
+  if (only_tile(tiles, tile, *num_tiles)) walk(std::true_type{});
+  else walk(std::false_type{});
   const int k_main = 64 * passes;
   if (wave == 0 && k_main < K) {  // a ragged end along K (a multiple of 8): element by element, zeros beyond
     bf16x8_t a[2], a2[2], b[2];
@@ -771,7 +785,8 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
 // (NF blocks of 16 columns, for gate and for up), one chunk ahead of the products.  Bound by the weights' way to
 // the compute units: a fetched weight meets 16 NR rows, a row 128 or 256 columns, and the blocks that read the
 // same weights or the same rows run on one die at the same time (see `place`), so its L2 is asked twice and
-// memory once.  Packed, 32 experts of 2048 x 2048, gated and ungated: 8,192 pairs 397 and 232 us with tiles of 64
+// memory once, or, where the expert has no other tile, with loads that say so (`read8`: 256 pairs 94 and 46 -> 86 and 43 us,
+// 1,184 pairs 101 and 51.5 -> 90 and 50; 2,880 pairs, two tiles an expert, in that way 121 -> 150).  Packed, 32 experts of 2048 x 2048, gated and ungated: 8,192 pairs 397 and 232 us with tiles of 64
 // rows dealt to the dies in turn, 202 and 123 us this way (0.68 PFLOP/s); 1,200 pairs 226 and 143 us in tiles of 16
 // rows, 102 and 52 us here (5.3 TB/s of weights); 256 pairs 113 and 61 us, 95 and 46 us (5.8 TB/s), of which
 // 14 and 7 us are the turn that every block starts K at.
@@ -893,6 +908,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
       x_next[c] = *reinterpret_cast<const uint4*>(xp + k + 8 * c - (k + col < K ? 0 : 32));
     }
   };
+  auto walk = [&](auto once) {
+  constexpr bool ONCE = decltype(once)::value;
   auto fetch_w = [&](int k) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -900,8 +917,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
         const int64_t wo = PACKED ? static_cast<int64_t>(kk / 32) * 512 : kk;
-        w_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + wo);
-        if (GATED) w2_next[h][f] = *reinterpret_cast<const bf16x8_t*>(wp[f] + up_off + wo);
+        w_next[h][f] = read8<ONCE>(wp[f] + wo);
+        if (GATED) w2_next[h][f] = read8<ONCE>(wp[f] + up_off + wo);
       }
     }
   };
@@ -967,6 +984,9 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
       __syncthreads();  // this chunk has been read by every wave, the next one is there
     }
   }
+  };
+  if (only_tile(tiles, at.tile, *num_tiles)) walk(std::true_type{});
+  else walk(std::false_type{});
   if (!wave_live) return;
   // lane holds row 16 r + li of the tile, columns n0 + 16 f + 4 lk + i
   store_tile<GATED, NF, NR, TO>(
@@ -1319,7 +1339,8 @@ extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
 // How many rows a tile holds, for experts of matrices [I, H] ([2 I, H] if gated) and [H, I], by an estimate of both
 // products in us, for tokens that choose their experts at random.  Tiles of 16: the matrices of the experts that are
 // chosen at 6.6 TB/s, and again for each further tile, of which there are some from 4.5 rows an expert on.  Tiles of 64:
-// one fetch, at 6.1 TB/s gated and 7.2 otherwise, but columns of 128 (ungated 256) a block, so a product is no faster than
+// one fetch, at 6.1 TB/s gated and 7.2 otherwise (before loads marked as streaming ones, which read a tenth more in
+// either kind of tile: 8 rows 129 / 130 us for the first line's 146 / 139, 16 rows 162 / 132), but columns of 128 (ungated 256) a block, so a product is no faster than
 // a block's walk along K (1.05 us a pass of 64), and blocks that come out uneven on the units wait for the last.  Both
 // products, tiles of 16 / 64, by rows an expert, gated:
 //   32 experts of 2048 x 2048     1   90 / 101 us    4  141 / 139    8  146 / 139   16  177 / 145
