@@ -73,7 +73,7 @@ __global__ __launch_bounds__(max_waves<D>() * 64) void decode_attention_kernel(c
     const int req = a.token_req[t];
     trow_idx = req < 0 ? -1 : a.slots[req];
   }
-  decode_block<D, DV>(a, t, blockIdx.y, blockIdx.z, __builtin_amdgcn_readfirstlane(trow_idx), lds);
+  decode_block<D, DV, true>(a, t, blockIdx.y, blockIdx.z, __builtin_amdgcn_readfirstlane(trow_idx), lds);
 }
 
 // out[t, head, :] = sum_s w_s * part_o[s] / sum_s w_s * l_s with w_s = exp2(m_s - max m).
@@ -223,6 +223,7 @@ extern "C" int kvc_decode_attention(void* out, void* part_o, void* part_ml, cons
   args.qkv_stride = qkv_stride;
   args.k_cache = static_cast<bf16_t*>(k_cache);
   args.v_cache = static_cast<bf16_t*>(v_cache);
+  args.v_second = nullptr;
   args.table = table;
   args.table_stride = table_stride;
   args.page_magic = page_magic_of(page_size);

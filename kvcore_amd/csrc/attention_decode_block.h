@@ -29,6 +29,7 @@ struct DecodeArgs {
   int64_t qkv_stride;
   bf16_t* k_cache;
   bf16_t* v_cache;
+  const bf16_t* v_second;  // the other half of every value head, where it is twice as wide as a key head (not written)
   const int32_t* table;
   int table_stride;
   const int32_t* positions;
@@ -96,8 +97,10 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // One block's work: token t (its row of the block table: trow_idx), kv head hk, one split of the keys; lds: lds_total()
-// bytes of it, 16-byte aligned.  D: the size of a query and key head; DV: the size of a value head.
-template <int D, int DV>
+// bytes of it, 16-byte aligned.  D: the size of a query and key head; DV: the size of a value head, at most D, or 2 D in two
+// planes.  STREAM: keys and values come by loads marked as streaming ones (`read8`).  They bring more where blocks fill
+// the chip, and take longer where a block walks many keys with few beside it (one token's 2,048 keys of 128, unsplit, 25 -> 32 us).
+template <int D, int DV, bool STREAM>
 __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk, int split, int trow_idx, unsigned char* lds) {
   const int tid = threadIdx.x;
   const int nthreads = blockDim.x;
@@ -110,6 +113,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
   const int g = nh / nkv;
   const bool head_live = col < g;
   constexpr int NJ = DV / 16;  // output row blocks
+  constexpr int DVP = DV > D ? D : DV;  // a plane's share of a value head
   constexpr int NC = D / 32;  // 32-wide chunks of the head for Q.K
 
   bf16_t* sq = reinterpret_cast<bf16_t*>(lds);                       // [g][D + kQPad]
@@ -214,20 +218,23 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
     half_of(u, 1, un.page[1], base[1], sub[1]);
     const int64_t k0 = (base[0] * page_size + sub[0]) * D, k1 = (base[1] * page_size + sub[1]) * D;
     const bf16_t* krow = a.k_cache + (col >= 8 ? k1 : k0) + (key_row * D + 8 * quad);
+    // keys and values are read once (see read8); rows of wide heads are several loads' way from whole lines: 8 tokens x 1,024
+    // keys of 128 14.4 -> 13.6 us marked (values alone 14.1), of 256 16.0 -> 16.6 (values alone 15.8)
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) un.k[h][c] = once8(krow + h * 4 * D + 32 * c);
+      for (int c = 0; c < NC; ++c) un.k[h][c] = read8<(STREAM && D <= 128)>(krow + h * 4 * D + 32 * c);
   };
   auto issue_values = [&](Unit& un, int u) {
     int64_t base[2];
     int sub[2];
     half_of(u, 0, un.page[0], base[0], sub[0]);
     half_of(u, 1, un.page[1], base[1], sub[1]);
-    const int64_t v0 = base[0] * DV * page_size + sub[0], v1 = base[1] * DV * page_size + sub[1];
-    const bf16_t* vrow = a.v_cache + (quad >= 2 ? v1 : v0) + (col * page_size + 8 * (quad & 1));
+    const int64_t v0 = base[0] * DVP * page_size + sub[0], v1 = base[1] * DVP * page_size + sub[1];
+    const int64_t at = (quad >= 2 ? v1 : v0) + (col * page_size + 8 * (quad & 1));
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) un.v[j] = once8(vrow + j * 16 * page_size);
+    for (int j = 0; j < NJ; ++j)
+      un.v[j] = read8<STREAM>((j < DVP / 16 ? a.v_cache : a.v_second) + at + j % (DVP / 16) * 16 * page_size);
   };
 
   // the first unit of this wave is asked for at once, before anything else waits

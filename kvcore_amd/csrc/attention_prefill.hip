@@ -185,44 +185,43 @@ __global__ __launch_bounds__(W * 64, (W == 4) ? 2 : 1) void prefill_attention_ke
   if (req < 0) return;  // the grid is an upper bound on the number of pairs
   // A request that brings one token has g rows, of the 16 a wave has room for, and its keys would be walked by one wave:
   // its blocks work as those of the kernel for single tokens do, all waves on the keys.
-  if constexpr (DV <= D) {
-    if (q_end - q_begin == 1 && positions[q_begin] / page_size + 2 <= single_pages) {
-      decode::DecodeArgs one = {};
-      one.out = out;
-      one.out_f32 = out_f32;
-      one.part_o = part_o;
-      one.part_ml = part_ml;
-      one.qkv = q;
-      one.qkv_stride = q_stride;
-      one.k_cache = const_cast<bf16_t*>(k_cache);  // read only: write_kv is 0
-      one.v_cache = const_cast<bf16_t*>(v_first);
-      one.table = table;
-      one.table_stride = table_stride;
-      one.positions = positions;
-      one.cos_tab = cos_tab;
-      one.sin_tab = sin_tab;
-      one.rot_dim = cos_tab != nullptr ? rot_dim : 0;
-      one.interleaved = interleaved;
-      one.nh = nh;
-      one.nkv = nkv;
-      one.page_size = page_size;
-      one.num_pages = num_pages;
-      one.scale_log2e = scale_log2e;
-      if (CAP_GATE) {
-        one.cap_rate = cap_rate;
-        one.cap_log2e = scale_log2e;
-        one.gate = gate;
-      }
-      one.window = window;
-      one.slopes = slopes;
-      one.chunk = chunk;
-      one.sinks = sinks;
-      one.page_magic = page_magic;
-      one.nsplit = gridDim.z;
-      one.lds_pages = single_pages;
-      decode::decode_block<D, DV>(one, q_begin, hk, blockIdx.z, slots[req], reinterpret_cast<unsigned char*>(tiles));
-      return;
+  if (q_end - q_begin == 1 && positions[q_begin] / page_size + 2 <= single_pages) {
+    decode::DecodeArgs one = {};
+    one.out = out;
+    one.out_f32 = out_f32;
+    one.part_o = part_o;
+    one.part_ml = part_ml;
+    one.qkv = q;
+    one.qkv_stride = q_stride;
+    one.k_cache = const_cast<bf16_t*>(k_cache);  // read only: write_kv is 0
+    one.v_cache = const_cast<bf16_t*>(v_first);
+    one.v_second = v_second;
+    one.table = table;
+    one.table_stride = table_stride;
+    one.positions = positions;
+    one.cos_tab = cos_tab;
+    one.sin_tab = sin_tab;
+    one.rot_dim = cos_tab != nullptr ? rot_dim : 0;
+    one.interleaved = interleaved;
+    one.nh = nh;
+    one.nkv = nkv;
+    one.page_size = page_size;
+    one.num_pages = num_pages;
+    one.scale_log2e = scale_log2e;
+    if (CAP_GATE) {
+      one.cap_rate = cap_rate;
+      one.cap_log2e = scale_log2e;
+      one.gate = gate;
     }
+    one.window = window;
+    one.slopes = slopes;
+    one.chunk = chunk;
+    one.sinks = sinks;
+    one.page_magic = page_magic;
+    one.nsplit = gridDim.z;
+    one.lds_pages = single_pages;
+    decode::decode_block<D, DV, false>(one, q_begin, hk, blockIdx.z, slots[req], reinterpret_cast<unsigned char*>(tiles));
+    return;
   }
   const int32_t* row_table = table + static_cast<int64_t>(slots[req]) * table_stride;
   for (int turn = 0; turn < 2; ++turn) {
@@ -782,7 +781,7 @@ int launch_prefill_ct(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16
                                       : (static_cast<int64_t>(max_pairs) * nkv + 7) / 8 * 8;
   if (wide > 0x7fffffff) return kvc_fail("kvc_prefill_attention: too many blocks");
   // page ids that a request of one token finds room for in LDS (more: it is walked like any other)
-  const int single_pages = g <= 16 && DV <= D ? (lds_bytes - static_cast<int>(decode::lds_total(W, g, D, 0))) / 4 : 0;
+  const int single_pages = g <= 16 ? (lds_bytes - static_cast<int>(decode::lds_total(W, g, DV > D ? DV : D, 0))) / 4 : 0;
   const unsigned page_magic = decode::page_magic_of(page_size);
   char variant[64];
   snprintf(variant, sizeof(variant), "prefill_attention_kernel<%d,%d,%d,%d>%s x%d", D, CT, KB, W,
@@ -826,13 +825,14 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   // against 43, 8,192 tokens 445 against 393.
   //
   // Portions behind a context, or beside single tokens, have tiles of like lengths (two a block 1.1 to 1.45 below 4 cu): up
-  // to 4 cu heads of 64 four waves (1.00 to 1.05), two tiles a block of eight waves where those just fill the chip (1.06 to
-  // 1.09); heads of 128 32 rows a wave (1.00 to 1.08), except that long requests pair their tiles.
+  // to 4 cu heads of 64 four waves (1.00 to 1.05; long portions alone up to 3 cu eight, as over two planes four take 63 us
+  // where those take 53), two tiles a block of eight waves where those just fill the chip (1.06 to 1.09); heads of 128 32 rows
+  // a wave (1.00 to 1.08), except that long requests pair their tiles.
   //
   // With splits of the keys: one tile of 64 rows a block up to cu (1.00 to 1.07; 32 rows a wave and two tiles a block 1.2 to
-  // 1.75), on heads of 64 up to 3 cu (1.00 to 1.08; with values of 128 up to 2 cu), else 32 rows a wave, one tile a block
-  // on heads of 128 (1.00 to 1.02).
-  const int ones = g <= 16 && DV <= D ? singles : 0;  // single tokens that are blocks of their own kind
+  // 1.75), on heads of 64 up to 2 cu (1.00 to 1.08), else 32 rows a wave, one tile a block on heads of 128 (1.00 to 1.02).
+  // (The rules know nothing of the values, so that one call over two planes and a call for each take the same tiles.)
+  const int ones = g <= 16 ? singles : 0;  // single tokens that are blocks of their own kind
   const int T1 = T - ones, R1 = R - ones > 1 ? R - ones : 1;
   const int bq1 = 64 / g > 0 ? 64 / g : 1;
   const int tiles1 = (T1 + bq1 - 1) / bq1 + (R1 - 1);  // every request but one may add a ragged tile
@@ -848,15 +848,15 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
     ct = 2;
     single = 0;
   } else if (nsplit > 1) {
-    if (blocks > (DV > D ? 2 : D == 64 ? 3 : 1) * cu) ct = 2;
+    if (blocks > (D == 64 ? 2 : 1) * cu) ct = 2;
     if (D == 64 && ct == 2) {  // 2,048 tokens behind 1,200: two tiles a block of eight waves 0.97, one of four 1.09
       single = 0;
       if (long_requests) waves = 8;
     }
   } else if (blocks <= cu) {
-  } else if (DV <= D && blocks <= 2 * cu) {
+  } else if (blocks <= 2 * cu) {
     if (blocks / 2 + single_blocks <= cu && 8 * blocks > 11 * cu) waves = 8;
-  } else if (whole_prompts || DV > D) {
+  } else if (whole_prompts) {
     if (pairs > 2 * cu) {
       ct = 2;
       single = 0;
@@ -869,7 +869,9 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
     }
   } else if (blocks <= 4 * cu + nkv) {
     if (D == 64) {
-      if (blocks > 3 * cu && blocks / 4 + single_blocks <= cu + nkv) {
+      if (blocks <= 3 * cu) {
+        if (single_blocks == 0 && long_requests) waves = 8;
+      } else if (blocks / 4 + single_blocks <= cu + nkv) {
         waves = 8;
         single = 0;
       }
