@@ -17,7 +17,8 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // runs of 64 KB a wave are read at 6.6 TB/s with the mark and at 6.25 without (the caches need not make room for
 // them, and keep the rows).  Steps with them in the products of few and of some dozen rows, in the experts' tiles and on
 // keys and values of single tokens: 8B shape, 8 tokens 3,478 -> 3,271 us, 64 tokens 5,005 -> 4,835, 1B, one token 901 ->
-// 856.  Where several blocks share a matrix through the L2 the mark costs more than it brings.
+// 856.  Where several blocks share a matrix through the L2, or a load takes
+// part of a line whose rest comes with another, the mark costs more than it brings.
 template <bool ONCE>
 __device__ __forceinline__ bf16x8_t read8(const void* p) {
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));

@@ -45,11 +45,11 @@ constexpr int kKMultiple = 512;         // what callers are promised: K is a mul
 constexpr int kMaxRows = 192;           // rows of A: up to twelve 16-row tiles a wave (sixteen were measured slower than the vendor's product)
 static_assert(kKMultiple % kRound == 0, "every K that is accepted must be whole rounds");
 
-template <int WAVES, int RT, int NT, bool GATED, typename OutT>
+template <int WAVES, int RT, int NT, bool GATED, typename OutT, bool PACKED>  // PACKED: see gemm_skinny_kernel
 __global__ __launch_bounds__(WAVES * 64) void gemm_mid_kernel(
     OutT* __restrict__ C, float* __restrict__ partial, const bf16_t* __restrict__ A,
     const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias, int M, int N, int K, int64_t lda,
-    int64_t ldc, int k_per_block, int packed, GateRule rule) {
+    int64_t ldc, int k_per_block, GateRule rule) {
   static_assert(!GATED || RT == 2, "the gated form pairs one gate tile with one up tile");
   static_assert(kStages % (2 * kChunkSteps) == 0, "a round of stages must cover whole pairs of chunks");
   __shared__ __attribute__((aligned(16))) bf16_t a_lds[2][NT * 16 * kRowElems];
@@ -69,14 +69,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mid_kernel(
   const int k_end = (k_begin + k_per_block < K) ? k_begin + k_per_block : K;
   const int n_steps = (k_end - k_begin) / 64;  // the host makes slices whole rounds of steps
 
-  const int ks = packed ? 16 : 1;
+  constexpr int ks = PACKED ? 16 : 1;
   const bf16_t* wp[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int r = GATED ? n0 + col : n0 + rt * 16 + col;
     const int64_t row = (r < N ? r : N - 1) + ((GATED && rt == 1) ? N : 0);
     // packed: what kvc_pack_weight made of W (tiles of 16 rows x 32 k, 1 KB each, along K)
-    wp[rt] = packed ? W + (row >> 4) * (static_cast<int64_t>(K) * 16) + (row & 15) * 32 +
+    wp[rt] = PACKED ? W + (row >> 4) * (static_cast<int64_t>(K) * 16) + (row & 15) * 32 +
                           static_cast<int64_t>(k_begin) * 16 + 8 * quad
                     : W + row * K + k_begin + 8 * quad;
   }
@@ -112,8 +112,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_mid_kernel(
     const int k = 64 * where(step);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      wbuf[stage][rt][0] = once8(wp[rt] + k * ks);
-      wbuf[stage][rt][1] = once8(wp[rt] + (k + 32) * ks);
+      wbuf[stage][rt][0] = read8<PACKED>(wp[rt] + k * ks);
+      wbuf[stage][rt][1] = read8<PACKED>(wp[rt] + (k + 32) * ks);
     }
   };
   auto fetch_chunk = [&](int slot, int chunk) {
@@ -315,8 +315,13 @@ void launch_mid(OutT* C, float* partial, const bf16_t* A, const bf16_t* W, const
                 int N, int K, int64_t lda, int64_t ldc, const MidPlan& p, hipStream_t stream) {
   const int cols_per_block = WAVES * (GATED ? 16 : 16 * RT);
   const dim3 grid((N + cols_per_block - 1) / cols_per_block, p.slices), block(WAVES * 64);
-  hipLaunchKernelGGL((gemm_mid_kernel<WAVES, RT, NT, GATED, OutT>), grid, block, 0, stream, C,
-                     p.slices > 1 ? partial : nullptr, A, W, bias, M, N, K, lda, ldc, p.k_per_block, p.packed, p.rule);
+  float* parts = p.slices > 1 ? partial : nullptr;
+  if (p.packed)
+    hipLaunchKernelGGL((gemm_mid_kernel<WAVES, RT, NT, GATED, OutT, true>), grid, block, 0, stream, C, parts, A, W, bias, M, N,
+                       K, lda, ldc, p.k_per_block, p.rule);
+  else
+    hipLaunchKernelGGL((gemm_mid_kernel<WAVES, RT, NT, GATED, OutT, false>), grid, block, 0, stream, C, parts, A, W, bias, M, N,
+                       K, lda, ldc, p.k_per_block, p.rule);
 }
 
 template <bool GATED, typename OutT>

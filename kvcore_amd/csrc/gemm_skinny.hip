@@ -53,11 +53,13 @@ struct SkinnyExtras {
 // FOLD: bit 0, the rows of A carry a scale factor still to be applied (ex.in_ss); bit 1, the
 // result goes into the residual stream (ex.residual).  Kernels without these keep their
 // register count, on which the number of waves in flight depends.
-template <int RT, int NT, int U, int MAXW, typename OutT, bool GATED, int FOLD = 0>
+// PACKED: W is what kvc_pack_weight made of the matrix, and read as a stream (`read8`).  Row-major, a load takes half a
+// line of each of 16 rows, which the next load must still find in the cache: marked so, 28672 x 4096 took 45 -> 48 us.
+template <int RT, int NT, int U, int MAXW, typename OutT, bool GATED, int FOLD, bool PACKED>
 __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict__ C, const bf16_t* __restrict__ A,
                                    const bf16_t* __restrict__ W, const bf16_t* __restrict__ bias,
                                    int M, int N, int K, int64_t lda, int64_t ldc, int k_per_wave,
-                                   const SkinnyExtras ex, int packed) {
+                                   const SkinnyExtras ex) {
   static_assert(!GATED || RT == 2, "the gated form pairs one gate tile with one up tile");
   extern __shared__ float red[];  // [waves - 1][RT * NT][64][4], then 16 row scales and [16][256] parts of their sums if FOLD & 1
   // wave-uniform values are made scalar on purpose: a condition on them becomes a scalar
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
   const int k_begin = wave * k_per_wave;
   const int k_end = (k_begin + k_per_wave < K) ? k_begin + k_per_wave : K;
 
-  const int ks = packed ? 16 : 1;  // elements between a row's 32-wide steps, in units of 32
+  constexpr int ks = PACKED ? 16 : 1;  // elements between a row's 32-wide steps, in units of 32
   const bf16_t* wp[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
     const int64_t row = (r < N ? r : N - 1) + ((GATED && rt == 1) ? N : 0);
     // packed: tiles of 16 rows x 32 k stored one after the other along K, so that the 64 lanes
     // of a load read 1 KB in one piece (see kvc_pack_weight)
-    wp[rt] = packed ? W + (row >> 4) * (static_cast<int64_t>(K) * 16) + (row & 15) * 32 + 8 * quad
+    wp[rt] = PACKED ? W + (row >> 4) * (static_cast<int64_t>(K) * 16) + (row & 15) * 32 + 8 * quad
                     : W + row * K + 8 * quad;
   }
   const bf16_t* ap[NT];
@@ -131,8 +133,8 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
     const int k = k_begin + 64 * step;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      abuf[stage][rt][0] = once8(wp[rt] + static_cast<int64_t>(k) * ks);
-      abuf[stage][rt][1] = once8(wp[rt] + static_cast<int64_t>(k + 32) * ks);
+      abuf[stage][rt][0] = read8<PACKED>(wp[rt] + static_cast<int64_t>(k) * ks);
+      abuf[stage][rt][1] = read8<PACKED>(wp[rt] + static_cast<int64_t>(k + 32) * ks);
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
   for (; k < k_full; k += 32) {
     bf16x8_t a[RT], b[NT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) a[rt] = once8(wp[rt] + static_cast<int64_t>(k) * ks);
+    for (int rt = 0; rt < RT; ++rt) a[rt] = read8<PACKED>(wp[rt] + static_cast<int64_t>(k) * ks);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) b[nt] = *reinterpret_cast<const bf16x8_t*>(ap[nt] + k);
 #pragma unroll
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(MAXW * 64) void gemm_skinny_kernel(OutT* __restrict
     bf16x8_t a[RT], b[NT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
-      a[rt] = valid ? once8(wp[rt] + static_cast<int64_t>(k_full) * ks) : zero8();
+      a[rt] = valid ? read8<PACKED>(wp[rt] + static_cast<int64_t>(k_full) * ks) : zero8();
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       b[nt] = valid ? *reinterpret_cast<const bf16x8_t*>(ap[nt] + k_full) : zero8();
@@ -409,9 +411,15 @@ void launch(OutT* C, const bf16_t* A, const bf16_t* W, const bf16_t* bias, int M
   const int rows_per_block = GATED ? 16 : 16 * RT;
   const dim3 grid((N + rows_per_block - 1) / rows_per_block), block(waves * 64);
   const int fold = (ex.in_ss != nullptr ? 1 : 0) | (ex.residual != nullptr ? 2 : 0);
-#define KVC_SKINNY_LAUNCH(FOLD_)                                                                   \
-  hipLaunchKernelGGL((gemm_skinny_kernel<RT, NT, STAGES, MAXW, OutT, GATED, FOLD_>), grid, block, \
-                     lds, stream, C, A, W, bias, M, N, K, lda, ldc, k_per_wave, ex, packed)
+  constexpr bool MAY_PACK = RT == 1 || GATED;  // pick_shape gives other shapes to row-major matrices alone
+#define KVC_SKINNY_OF(FOLD_, PACKED_)                                                                       \
+  hipLaunchKernelGGL((gemm_skinny_kernel<RT, NT, STAGES, MAXW, OutT, GATED, FOLD_, PACKED_>), grid, block, \
+                     lds, stream, C, A, W, bias, M, N, K, lda, ldc, k_per_wave, ex)
+#define KVC_SKINNY_LAUNCH(FOLD_)                                          \
+  do {                                                                    \
+    if (MAY_PACK && packed) KVC_SKINNY_OF(FOLD_, MAY_PACK);               \
+    else KVC_SKINNY_OF(FOLD_, false);                                     \
+  } while (0)
   if constexpr (NT == 1 && sizeof(OutT) == 2) {  // folded norms are for steps of few rows
     switch (fold) {
       case 0: KVC_SKINNY_LAUNCH(0); break;
@@ -423,6 +431,7 @@ void launch(OutT* C, const bf16_t* A, const bf16_t* W, const bf16_t* bias, int M
     KVC_SKINNY_LAUNCH(0);
   }
 #undef KVC_SKINNY_LAUNCH
+#undef KVC_SKINNY_OF
 }
 
 // The launch shape is a function of N and K alone, so that a row's sums do not depend on
@@ -449,6 +458,7 @@ inline void pick_shape(int N, int K, int packed, int* rt_out, int* waves_out) {
   if (const char* e = getenv("KVC_SKINNY_RT")) rt = atoi(e);
   if (const char* e = getenv("KVC_SKINNY_WAVES")) waves = atoi(e);
   if (rt != 1 && rt != 2) rt = 1;
+  if (packed) rt = 1;
   const int max_waves = (rt >= 2) ? 4 : 8;
   if (waves < 1) waves = 1;
   if (waves > max_waves) waves = max_waves;

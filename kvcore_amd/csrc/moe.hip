@@ -654,7 +654,7 @@ __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
 // passes long a share of it is one or two, and with many tiles four times the blocks cost more than they bring
 // (kvc_moe_gemm has the line): 128 experts of 1024 x 384, 8 rows each, down 37.0 us with WK 4, 20.8 with WK 1
 // (two passes on their way: with four 22.6).
-// An expert that has one tile has its matrices read once, with loads that say so (`read8`): eight tokens 64 and 34 ->
+// An expert that has one tile has its (packed) matrices read once, with loads that say so (`read8`): eight tokens 64 and 34 ->
 // 57 and 30 us (6.0 TB/s), 256 pairs 93 and 49 -> 83 and 46.  Where two tiles share a matrix through the L2 such loads cost
 // more than they bring (256 pairs, half of them with few experts, 160 -> 196 us), so those keep the others.
 __device__ __forceinline__ bool only_tile(const int32_t* tiles, int tile, int num_tiles) {  // an expert's are side by side
@@ -733,7 +733,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     }
   }
   };
-  if (only_tile(tiles, tile, *num_tiles)) walk(std::true_type{});
+  if (PACKED && only_tile(tiles, tile, *num_tiles)) walk(std::integral_constant<bool, PACKED != 0>{});
   else walk(std::false_type{});
   const int k_main = 64 * passes;
   if (wave == 0 && k_main < K) {  // a ragged end along K (a multiple of 8): element by element, zeros beyond
@@ -985,7 +985,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
     }
   }
   };
-  if (only_tile(tiles, at.tile, *num_tiles)) walk(std::true_type{});
+  if (PACKED && only_tile(tiles, at.tile, *num_tiles)) walk(std::integral_constant<bool, PACKED != 0>{});
   else walk(std::false_type{});
   if (!wave_live) return;
   // lane holds row 16 r + li of the tile, columns n0 + 16 f + 4 lk + i
