@@ -259,18 +259,27 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(float* __restrict__
 // 1,000 rows of 2048 x 2048 110 and 69, 2,048 rows of 16384 x 2048 1,668 and 834 (165 TFLOP/s).  Tiles of 128 rows and one
 // column block a wave read LDS twice as often: 74, 38, 24, 18, 68 and 860 us before an operand's factor (float_parts.h), where
 // these took 64, 39, 24, 17, 58 and 824.
-template <int MT, int NT, bool LEAVE>
-__global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
+// HALVES 2: a block of eight waves whose halves walk every other chain each, with LDS of their own for the rows; the second
+// half's sums go to the first by LDS after each chain and are added in the same order.  Where the launch gives a unit one
+// block of four waves, a SIMD has a single one, whose splits, reads of LDS and products wait for one another (122 rows of 16384 x
+// 2048: 57 of 60 us remain without five of the six products); with two they overlap: 69 -> 60 us.  Where a unit has two
+// blocks of four waves anyway, those do it better (700 rows 306 and 317 us).
+template <int MT, int NT, bool LEAVE, int HALVES>
+__global__ __launch_bounds__(256 * HALVES, 2) void gemm_f32_shared_kernel(
     float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias,
     float* __restrict__ parts, int M, int N, int K, int64_t lda, int64_t ldc) {
   constexpr int UN = MT / 4;  // pieces of 16 rows that a wave brings
-  __shared__ u32x4_t rows_s[2][MT][3][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  __shared__ u32x4_t all_rows_s[HALVES][2][MT][3][64];
+  __shared__ f32x4_t meet_s[HALVES == 2 ? 4 * NT * MT : 1][64];
+  static_assert(HALVES == 1 || !LEAVE, "chains that stay in memory need not meet");
+  const int of_block = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wave = of_block & 3, second = HALVES == 2 ? of_block >> 2 : 0;
+  u32x4_t(&rows_s)[2][MT][3][64] = all_rows_s[second];
   const int li = lane & 15, lk = lane >> 4;
   const int n0 = (blockIdx.x * 4 + wave) * 16 * NT, m0 = blockIdx.y * 16 * MT;
-  const int chunks = K / kChunk;
+  const int chunks = K / kChunk;  // a multiple of 16: both halves of a block make the same steps
   const int per = kWaves / gridDim.z;
-  const int first = blockIdx.z * per, last = first + per;  // this block's chains
+  const int first = blockIdx.z * per + second, last = blockIdx.z * per + per;  // this half's chains, HALVES apart
   // columns and rows beyond the matrix read its last ones and are not stored
   const float* wp[NT];
   const float* ap[UN];
@@ -306,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
   };
   // the chunk after c: the next of its chain, or the first of the next chain, or (at the end) any
   auto after = [&](int c) {
-    const int next = (c & (kWaves - 1)) + 1;
+    const int next = (c & (kWaves - 1)) + HALVES;
     return c + kWaves < chunks ? c + kWaves : next < last ? next : first;
   };
   f32x4_t acc[NT][MT], sum[NT][MT];
@@ -324,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
   ahead = after(ahead);
   __builtin_amdgcn_sched_barrier(0);
   fetch(0, ahead);
-  for (int chain = first; chain < last; ++chain) {
+  for (int chain = first; chain < last; chain += HALVES) {
     for (int c = chain; c < chunks; c += 2 * kWaves) {  // scalar; no branch inside, which would drain the loads
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -361,13 +370,24 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_shared_kernel(
           const int row = m0 + 16 * m + li, col = n0 + 16 * n + 4 * lk, wide = (N + 3) & ~3;
           if (row < M && col < N)
             *reinterpret_cast<f32x4_t*>(parts + (static_cast<int64_t>(chain) * M + row) * wide + col) = acc[n][m];
+        } else if (second) {
+          meet_s[(wave * NT + n) * MT + m][lane] = acc[n][m];
         } else {
           sum[n][m] = chain == first ? acc[n][m] : sum[n][m] + acc[n][m];
         }
         acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
+    if constexpr (HALVES == 2) {
+      __syncthreads();
+      if (!second) {  // read before this half comes to the next chain's first barrier, and so before it is written again
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) sum[n][m] += meet_s[(wave * NT + n) * MT + m][lane];
+      }
+    }
   }
-  if constexpr (LEAVE) return;
+  if (LEAVE || second) return;
   // lane holds row li, columns 4 lk .. of its tiles
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -432,16 +452,16 @@ FewShape few_shape(int M, int N) {
 // Chains are dealt out up to the workspace that 64 x 128 of C a unit need.
 constexpr int kSharedRows = 4;  // row blocks of 16 a block
 struct SharedShape {
-  int nt, groups;
+  int nt, groups, halves;
 };
 SharedShape shared_shape(int M, int N, int K) {
-  if (M <= 32 || K % (2 * kWaves * kChunk)) return {0, 0};
+  if (M <= 32 || K % (2 * kWaves * kChunk)) return {0, 0, 1};
   const int64_t units = kvc_device_compute_units();
   auto rounds = [&](int64_t blocks) { return static_cast<double>((blocks + units - 1) / units); };
   const FewShape few = few_shape(M, N);
   const int live = few.mt < (M + 15) / 16 ? few.mt : (M + 15) / 16;  // row blocks that are not copies of the last
   double least = 2.7 + rounds(few.blocks) * (0.3 * few.nt * few.mt + 0.45 * (K / (kWaves * kChunk)) * (few.nt + live));
-  SharedShape best{0, 0};
+  SharedShape best{0, 0, 1};
   for (int nt = 1; nt <= 2; ++nt) {
     const int64_t blocks = (static_cast<int64_t>(N) + 64 * nt - 1) / (64 * nt) * ((M + 63) / 64);
     for (int groups = 1; groups <= kWaves; groups *= 2) {
@@ -449,7 +469,11 @@ SharedShape shared_shape(int M, int N, int K) {
       const double r = rounds(blocks * groups);
       double us = 5.3 + 0.8 * r + K / kChunk / groups * (nt == 1 ? 0.49 + 0.45 * (r - 1) : 0.89 + 0.735 * (r - 1));
       if (groups > 1) us += 1.1 + 12e-6 * M * N;
-      if (us < least) least = us, best = {nt, groups};
+      if (us < least) least = us, best = {nt, groups, 1};
+      if (groups == 1 && nt == 2 && r == 1) {
+        us = 7.4 + K / kChunk * 0.79;
+        if (us < least) least = us, best = {nt, groups, 2};
+      }
     }
   }
   return best;
@@ -508,19 +532,20 @@ extern "C" int kvc_gemm_f32(float* C, const float* A, const float* W, const floa
 #undef KVC_F32
     return kvc_check_launch("kvc_gemm_f32");
   }
-  const SharedShape shape = piece == 8 ? shared_shape(M, N, K) : SharedShape{0, 0};
+  const SharedShape shape = piece == 8 ? shared_shape(M, N, K) : SharedShape{0, 0, 1};
   if (shape.nt) {
     const int cols = 64 * shape.nt, rows = 16 * kSharedRows;
     const dim3 grid((N + cols - 1) / cols, (M + rows - 1) / rows, shape.groups);
     if (grid.y > 65535) return kvc_fail("kvc_gemm_f32: M too large for one launch");
     const bool left = shape.groups > 1;
-#define KVC_F32_SHARED(NT, LEAVE)                                                                                           \
-  hipLaunchKernelGGL((gemm_f32_shared_kernel<kSharedRows, NT, LEAVE>), grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), \
-                     C, A, W, bias, parts, M, N, K, lda, ldc)
-    if (left && shape.nt == 2) KVC_F32_SHARED(2, true);
-    else if (left) KVC_F32_SHARED(1, true);
-    else if (shape.nt == 2) KVC_F32_SHARED(2, false);
-    else KVC_F32_SHARED(1, false);
+#define KVC_F32_SHARED(NT, LEAVE, HALVES)                                                                                   \
+  hipLaunchKernelGGL((gemm_f32_shared_kernel<kSharedRows, NT, LEAVE, HALVES>), grid, dim3(256 * HALVES), 0,                 \
+                     reinterpret_cast<hipStream_t>(stream), C, A, W, bias, parts, M, N, K, lda, ldc)
+    if (left && shape.nt == 2) KVC_F32_SHARED(2, true, 1);
+    else if (left) KVC_F32_SHARED(1, true, 1);
+    else if (shape.nt == 2 && shape.halves == 2) KVC_F32_SHARED(2, false, 2);
+    else if (shape.nt == 2) KVC_F32_SHARED(2, false, 1);
+    else KVC_F32_SHARED(1, false, 1);
 #undef KVC_F32_SHARED
     if (left) {
       const int64_t quads = static_cast<int64_t>(M) * ((N + 3) / 4);
