@@ -233,6 +233,43 @@ def new_memory(slots, H, d, dv):
             torch.full((slots, H), float("nan"), device=DEV))
 
 
+@pytest.mark.parametrize("H", [1, 16, 17, 40])
+@pytest.mark.parametrize("n", [3, 63, 64, 65, 129, 1000])
+def test_running_maxima_of_portions(H, n):
+    """Requests of lengths around the 64 runs that a portion is cut into, a padded one between, heads around the 16
+    that a block takes, against the recurrence in 64 bits."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(H * n)
+    reqs = [(2, 0, n), None, (1, 5, n + 1), (0, 0, 2)]
+    batch, T = batch_tensors(reqs)
+    raw = torch.randn(T, 2 * H, generator=gen) * 3
+    bi, bf = torch.randn(H, generator=gen), torch.randn(H, generator=gen) + 3
+    state = torch.randn(3, H, generator=gen)
+    keep, take, mx = (torch.full((T, H), float("nan"), device=DEV) for _ in range(3))
+    got = state.to(DEV)
+    ops.max_gates(keep, take, mx, raw[:, :H].to(DEV).contiguous(), raw[:, H:].to(DEV).contiguous(), bi.to(DEV), bf.to(DEV),
+                  15.0, got, **batch)
+    at = 0
+    for item in reqs:
+        if item is None:
+            assert float(keep[at].abs().max() + take[at].abs().max() + mx[at].abs().max()) == 0
+            at += 1
+            continue
+        slot, start, count = item
+        m = torch.zeros(H, dtype=F64) if start == 0 else state[slot].double()
+        for t in range(at, at + count):
+            i = 15 * torch.tanh((raw[t, :H].double() + bi.double()) / 15)
+            f = torch.nn.functional.logsigmoid(15 * torch.tanh((raw[t, H:].double() + bf.double()) / 15))
+            new = torch.maximum(f + m, i)
+            # sums of up to 1,000 float32 logarithms of some 1, and what their exponentials make of that
+            for a, b in ((keep[t], torch.exp(f + m - new)), (take[t], torch.exp(i - new)), (mx[t], new)):
+                assert float((a.cpu().double() - b).abs().max()) < 2e-4
+            m = new
+        assert float((got[slot].cpu().double() - m).abs().max()) < 2e-4
+        at += count
+
+
 @pytest.mark.parametrize("H,d,dv,cap", [(3, 24, 40, 15.0), (1, 8, 1, 1.0), (2, 200, 80, 20.0), (4, 64, 64, 8.0),
                                         (2, 64, 127, 12.0), (6, 20, 16, 3.0)])
 def test_matrix_memory_whole_in_steps_and_beside_others(H, d, dv, cap):
