@@ -237,33 +237,6 @@ __global__ void add_rmsnorm_kernel(T* __restrict__ out, float* __restrict__ resi
 // in registers, so residual and delta are read once, with 16- and 32-byte accesses that
 // are all in flight together.  The order of the additions in the sum of squares is
 // fixed by the width alone.
-__device__ __forceinline__ void load8(const float* p, float* v) {
-  const float4 a = *reinterpret_cast<const float4*>(p);
-  const float4 b = *reinterpret_cast<const float4*>(p + 4);
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-  v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
-__device__ __forceinline__ void load8(const bf16_t* p, float* v) {
-  const uint4 a = *reinterpret_cast<const uint4*>(p);
-  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = __uint_as_float(w[i] << 16);
-    v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-  }
-}
-__device__ __forceinline__ void store8(float* p, const float* v) {
-  *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
-}
-// (the conversion in hardware: to nearest, ties to even, as f32_to_bf16_bits)
-__device__ __forceinline__ void store8(bf16_t* p, const float* v) {
-  typedef float f32x8_t __attribute__((ext_vector_type(8)));
-  typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-  const f32x8_t x = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-  *reinterpret_cast<bf16x8_t*>(p) = __builtin_convertvector(x, bf16x8_t);
-}
-
 template <typename T, int NCH>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(T* __restrict__ out,
                                                               float* __restrict__ residual,

@@ -13,6 +13,7 @@ using namespace kvc;
 namespace {
 
 inline hipStream_t S(kvc_stream s) { return reinterpret_cast<hipStream_t>(s); }
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // One block per row.  residual += delta; mean; mean of the squared deviations; then
 // (x - mean) / sqrt(var + eps) * weight + bias.  Three passes over a row that stays in cache.
@@ -99,6 +100,59 @@ __global__ __launch_bounds__(256) void add_layernorm_regs_kernel(T* __restrict__
   }
 }
 
+// The same for rows of a multiple of 8 values up to 2048 * NCH, 16-byte aligned: eight neighbouring values a load.
+// Bound by its bytes: 2,048 rows of 2,048, bfloat16 (50 MB), value by value 13.4 us, 12.1 this way.
+template <typename T, int NCH>
+__global__ __launch_bounds__(256) void add_layernorm_vec_kernel(T* __restrict__ out, float* __restrict__ residual,
+                                                                const T* __restrict__ delta, const float* __restrict__ weight,
+                                                                const float* __restrict__ bias, float eps, int H) {
+  __shared__ float scratch[16];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * H;
+  float v[NCH][8], w[NCH][8], sh[NCH][8];  // gain and shift come with the row: one trip to memory in all
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int e = (c * 256 + threadIdx.x) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[c][i] = w[c][i] = sh[c][i] = 0.f;
+    if (e < H) {
+      load8(residual + base + e, v[c]);
+      load8(weight + e, w[c]);
+      if (bias != nullptr) load8(bias + e, sh[c]);
+      if (delta != nullptr) {
+        float d[8];
+        load8(delta + base + e, d);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[c][i] += d[i];
+        store8(residual + base + e, v[c]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum += v[c][i];
+    }
+  }
+  const float mean = block_sum(sum, scratch) / static_cast<float>(H);
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    if ((c * 256 + threadIdx.x) * 8 < H)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[c][i] -= mean;
+        ss = fmaf(v[c][i], v[c][i], ss);
+      }
+  }
+  const float inv = 1.f / sqrtf(block_sum(ss, scratch) / static_cast<float>(H) + eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int e = (c * 256 + threadIdx.x) * 8;
+    if (e < H) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[c][i] = fmaf(v[c][i] * inv, w[c][i], sh[c][i]);
+      store8(out + base + e, v[c]);
+    }
+  }
+}
+
 constexpr int kMaxBranches = 4;
 struct Branches {
   const float* x[kMaxBranches];
@@ -107,8 +161,9 @@ struct Branches {
 
 // out[t] = (1 / n) * sum_b gain_b * x_b[t] / sqrt(mean(x_b[t]^2) + eps).  One block per row.
 // REGS: the rows (up to 256 * 8 values) and the gains are fetched once, all at the start, and
-// kept in registers; otherwise a row is read twice.
-template <typename T, bool REGS>
+// kept in registers; otherwise a row is read twice.  VEC (with REGS): a multiple of 8 values, 16-byte aligned, eight
+// neighbouring ones a thread (2,048 rows of 2,048, two branches, 40 MB: 13.4 us value by value, 10.8 so).
+template <typename T, bool REGS, bool VEC>
 __global__ __launch_bounds__(256) void rms_branches_mean_kernel(T* __restrict__ out, Branches br,
                                                                 int n, float eps, int H) {
   __shared__ float scratch[16];
@@ -120,13 +175,25 @@ __global__ __launch_bounds__(256) void rms_branches_mean_kernel(T* __restrict__ 
 #pragma unroll
     for (int b = 0; b < kMaxBranches; ++b) {
       ss[b] = 0.f;
+      if constexpr (VEC) {
+        const int c = threadIdx.x * 8;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int c = threadIdx.x + i * 256;
-        const bool ok = b < n && c < H;
-        x[b][i] = ok ? br.x[b][base + c] : 0.f;
-        gn[b][i] = ok ? br.gain[b][c] : 0.f;
-        ss[b] = fmaf(x[b][i], x[b][i], ss[b]);
+        for (int i = 0; i < NV; ++i) x[b][i] = gn[b][i] = 0.f;
+        if (b < n && c < H) {
+          load8(br.x[b] + base + c, x[b]);
+          load8(br.gain[b] + c, gn[b]);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; ++i) ss[b] = fmaf(x[b][i], x[b][i], ss[b]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          const int c = threadIdx.x + i * 256;
+          const bool ok = b < n && c < H;
+          x[b][i] = ok ? br.x[b][base + c] : 0.f;
+          gn[b][i] = ok ? br.gain[b][c] : 0.f;
+          ss[b] = fmaf(x[b][i], x[b][i], ss[b]);
+        }
       }
     }
     float acc[NV];
@@ -140,10 +207,16 @@ __global__ __launch_bounds__(256) void rms_branches_mean_kernel(T* __restrict__ 
         for (int i = 0; i < NV; ++i) acc[i] = fmaf(x[b][i] * inv, gn[b][i], acc[i]);
       }
     }
+    if constexpr (VEC) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = threadIdx.x + i * 256;
-      if (c < H) out[base + c] = from_float<T>(acc[i] * share);
+      for (int i = 0; i < NV; ++i) acc[i] *= share;
+      if (threadIdx.x * 8 < H) store8(out + base + threadIdx.x * 8, acc);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int c = threadIdx.x + i * 256;
+        if (c < H) out[base + c] = from_float<T>(acc[i] * share);
+      }
     }
   } else {
     float inv[kMaxBranches];
@@ -185,6 +258,17 @@ extern "C" int kvc_add_layernorm(void* out, float* residual, const void* delta, 
                                  kvc_stream stream) {
   if (T < 0 || H <= 0) return kvc_fail("kvc_add_layernorm: bad sizes");
   if (T == 0) return 0;
+  if (H % 8 == 0 && H <= 2048 * 4 && aligned16(out) && aligned16(residual) && aligned16(weight) && aligned16(bias) && aligned16(delta)) {
+#define KVC_LAYERNORM(NCH)                                                                                            \
+  KVC_DISPATCH_DTYPE(dtype, Tp, hipLaunchKernelGGL((add_layernorm_vec_kernel<Tp, NCH>), dim3(T), dim3(256), 0, S(stream), \
+                                                   static_cast<Tp*>(out), residual, static_cast<const Tp*>(delta),    \
+                                                   weight, bias, eps, H))
+    if (H <= 2048) KVC_LAYERNORM(1);
+    else if (H <= 4096) KVC_LAYERNORM(2);
+    else KVC_LAYERNORM(4);
+#undef KVC_LAYERNORM
+    return kvc_check_launch("kvc_add_layernorm");
+  }
   if (H <= 256 * 8) {
     KVC_DISPATCH_DTYPE(dtype, Tp,
                        hipLaunchKernelGGL((add_layernorm_regs_kernel<Tp, 8>), dim3(T), dim3(256), 0, S(stream),
@@ -213,17 +297,23 @@ extern "C" int kvc_rms_branches_mean(void* out, const float* const* host_x,
     return kvc_fail("kvc_rms_branches_mean: bad sizes (one to four branches)");
   if (T == 0) return 0;
   Branches br{};
+  bool vec = H % 8 == 0 && aligned16(out);
   for (int b = 0; b < n; ++b) {
     br.x[b] = host_x[b];
     br.gain[b] = host_gain[b];
+    vec = vec && aligned16(host_x[b]) && aligned16(host_gain[b]);
   }
-  if (H <= 256 * 8)
+  if (H <= 256 * 8 && vec)
     KVC_DISPATCH_DTYPE(dtype, Tp,
-                       hipLaunchKernelGGL((rms_branches_mean_kernel<Tp, true>), dim3(T), dim3(256), 0,
+                       hipLaunchKernelGGL((rms_branches_mean_kernel<Tp, true, true>), dim3(T), dim3(256), 0,
+                                          S(stream), static_cast<Tp*>(out), br, n, eps, H));
+  else if (H <= 256 * 8)
+    KVC_DISPATCH_DTYPE(dtype, Tp,
+                       hipLaunchKernelGGL((rms_branches_mean_kernel<Tp, true, false>), dim3(T), dim3(256), 0,
                                           S(stream), static_cast<Tp*>(out), br, n, eps, H));
   else
     KVC_DISPATCH_DTYPE(dtype, Tp,
-                       hipLaunchKernelGGL((rms_branches_mean_kernel<Tp, false>), dim3(T), dim3(256), 0,
+                       hipLaunchKernelGGL((rms_branches_mean_kernel<Tp, false, false>), dim3(T), dim3(256), 0,
                                           S(stream), static_cast<Tp*>(out), br, n, eps, H));
   return kvc_check_launch("kvc_rms_branches_mean");
 }

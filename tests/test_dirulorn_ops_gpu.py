@@ -58,6 +58,29 @@ def test_layer_norm_with_the_residual_sum(ops, H, dtype):
     close(out, plain.layer_norm(total, w.double(), torch.zeros(H, dtype=torch.float64), 1e-5), **tol)
 
 
+@pytest.mark.parametrize("H", [8, 2040, 2048, 2056, 4096, 4104, 8192, 8200])
+def test_norms_of_rows_read_eight_values_at_a_time(ops, H):
+    """Widths around those at which a thread takes one, two or four pieces of eight values, and rows that lie four
+    bytes off 16: both take a row's values in another order, which is all that may differ."""
+    T, dtype = 3, torch.bfloat16
+    res, delta = rnd(T, H, seed=1) * 3 + 5.0, rnd(T, H, seed=2).to(dtype)
+    w, b = rnd(H, seed=3) + 1, rnd(H, seed=4)
+    total = res.double() + delta.double()
+    want = plain.layer_norm(total, w.double(), b.double(), 1e-5)
+    for shift in (0, 1):
+        space = torch.full((T * H + 1,), float("nan"), device=DEV)
+        r = space[shift: shift + T * H].view(T, H)
+        r.copy_(res)
+        out = torch.empty(T, H, dtype=dtype, device=DEV)
+        ops.add_layernorm(out, r, delta.to(DEV), w.to(DEV), b.to(DEV), 1e-5)
+        close(r, total, 1e-6)
+        close(out, want, 1e-2, 8e-3)  # one rounding to 8 bits
+        out = torch.empty(T, H, device=DEV)
+        ops.rms_branches_mean(out, [(r, w.to(DEV)), (r * 2, b.to(DEV))], 1e-6)
+        unit = plain.rms_unit(total, 1e-6)
+        close(out, (unit * w.double() + unit * b.double()) / 2, 1e-5)
+
+
 @pytest.mark.parametrize("n", [1, 2, 3])
 def test_mean_of_branches_each_over_its_root_mean_square(ops, n):
     T, H = 5, 72
