@@ -1002,7 +1002,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
 // fixed, so the lanes swap 16-byte pieces within a row on the way in such that the lanes that read operands together
 // meet all banks.  Wave (wr, wc) takes the row blocks of parity wr, so that a tile that is not full is dealt evenly, and 64
 // columns.
-// Packed, 32 experts of 2048 x 2048, gated and ungated, 8,192 pairs: tiles of 128 rows 202 and 122 us, these 168 and 90 (0.82
+// Packed, 32 experts of 2048 x 2048, gated and ungated, 8,192 pairs: tiles of 128 rows 202 and 122 us, these 166 and 89 (0.82
 // PFLOP/s; the weights alone take 83 and 41 us).  384 rows and not 256: experts of 256 rows in the mean have up to some 330, and
 // with tiles of 256 a third of them had two (175 and 115 us).  One expert of 8,192 rows in tiles of 256: 1.0 PFLOP/s, 1.18
 // without the way in and out of a block (some 10 us of 60); a stage of 256 rows takes 1,490 cycles at 1.8 GHz, of which the
@@ -1017,14 +1017,18 @@ __device__ __forceinline__ void to_lds16(const void* from, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(from) : "memory", "m0");
 }
 
+__device__ __forceinline__ void to_lds16_once(const void* from, uint32_t lds) {  // marked as a streaming load, as `read8`'s
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(from) : "memory", "m0");
+}
+
 // The wave's loads but the youngest N have landed; past the barrier that holds for all waves.
 template <int N>
 __device__ __forceinline__ void landed() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// R: how many row blocks a wave multiplies: the tile has at most 32 R rows
-template <int PACKED, int R>
+// R: how many row blocks a wave multiplies: the tile has at most 32 R rows.  ONCE: no other block reads these weights
+template <int PACKED, int R, bool ONCE>
 __device__ __forceinline__ void wide_walk(const char* lds, const char* const (&xp)[3], const char* const (&wp)[2], int wave,
                                           int lane, const int (&wt)[4], int stages, int turn,
                                           f32x4_t (&acc)[4][kWideBlocks]) {
@@ -1041,6 +1045,7 @@ __device__ __forceinline__ void wide_walk(const char* lds, const char* const (&x
   auto round = [&](int s) { return s + turn < stages ? s + turn : s + turn - stages; };
   auto load = [&](int j, int64_t s, uint32_t buffer) {
     if (j < XL) to_lds16(xp[j] + 64 * s, buffer + (wave + 8 * j) * 1024);
+    else if (ONCE) to_lds16_once(wp[j - XL] + (PACKED ? 1024 : 64) * s, buffer + kW + (wave + 8 * (j - XL)) * 1024);
     else to_lds16(wp[j - XL] + (PACKED ? 1024 : 64) * s, buffer + kW + (wave + 8 * (j - XL)) * 1024);
   };
   auto x_operand = [&](const char* stage, int r) {
@@ -1101,6 +1106,29 @@ __device__ __forceinline__ void wide_walk(const char* lds, const char* const (&x
   }
 }
 
+// As `place`, but a tile's column blocks all go to one die, tiles in turn, where experts have a tile each (up to a quarter
+// more tiles than that): the die's L2 holds the tile's rows for them, and no die reads every tile's.  The kernel is bound by
+// what it draws through the fabric, and rows read by eight dies are a third of that.  Microseconds of the first and the second
+// product, packed, columns dealt to the dies and plain loads / tiles and streaming loads (weights are read once then):
+//   32 experts of 2048 x 2048, 245 rows 176 + 93 / 164 + 85, 138 rows 132 + 72 / 120 + 62, every other expert's twice as many
+//   176 + 102 / 170 + 98; 25 of them, 240 rows 144 + 73 / 127 + 67; 12 of them 70 + 59 / 68 + 58;
+//   64 of 2048 x 1024, 125 rows 127 + 83 / 109 + 66; 16 of 2048 x 2048, 256 rows 89 + 67 / 78 + 66.
+// With two tiles an expert (500 rows) the dies would read the weights twice: 296 + 150 / 304 + 157.  Tiles that leave dies idle
+// or the fullest die (32 blocks a round) more rounds than an even split stay with it too: 4 experts of 2048 x 2048 61 + 56 /
+// 63 + 58, of 2048 x 8192 80 + 181 / 127 + 180.
+__device__ __forceinline__ TilePlace place_wide(int id, const int32_t* tiles, int num_tiles, int cols, int lane) {
+  const int turns = (num_tiles + 7) / 8;  // tiles of the fullest die
+  int again = 0;                          // tiles behind the first of their expert
+  for (int t0 = 0; t0 < num_tiles; t0 += kWave) {
+    const int t = t0 + lane;
+    again += __popcll(__ballot(t + 1 < num_tiles && tiles[3 * t] == tiles[3 * t + 3]));
+  }
+  if (num_tiles < 8 || (turns * cols + 31) / 32 > (num_tiles * cols + 255) / 256 || 4 * again > num_tiles)
+    return place(id, num_tiles, cols);
+  const int idx = id >> 3, turn = idx / cols, tile = 8 * turn + (id & 7);
+  return {tile < num_tiles ? tile : -1, idx - turn * cols};
+}
+
 template <int GATED, typename TO, int PACKED>
 __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
@@ -1109,11 +1137,11 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
     int act, const float* __restrict__ row_scale) {
   constexpr int COLS = GATED ? 128 : 256;  // a block's columns of the result
   __shared__ __attribute__((aligned(1024))) char lds[kWideLds];
-  const TilePlace at = place(blockIdx.x, *num_tiles, (N + COLS - 1) / COLS);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+  const TilePlace at = place_wide(blockIdx.x, tiles, *num_tiles, (N + COLS - 1) / COLS, lane);
   if (at.tile < 0) return;
   const int e = tiles[3 * at.tile], r0 = tiles[3 * at.tile + 1];
   const int nr = __builtin_amdgcn_readfirstlane(tiles[3 * at.tile + 2]);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   const int li = lane & 15, lk = lane >> 4, wr = wave & 1, wc = wave >> 1;
   const int c0 = at.col * COLS, n0 = c0 + wc * (COLS / 4);
   const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
@@ -1149,12 +1177,22 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
     for (int r = 0; r < kWideBlocks; ++r) acc[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // every block walks K round from a place of its own, as in the kernel for tiles of 128 rows, and from the same one
   const int turn = (e * 5 + at.col * 11) % (K / 64) * 2;
+  // an expert of more tiles than one has some 200 rows in each
+  constexpr bool kStream = PACKED != 0;
+  const bool alone = kStream && only_tile(tiles, at.tile, *num_tiles);
   switch ((nr + 31) >> 5) {  // scalar
-#define KVC_WALK(R) case R: wide_walk<PACKED, R>(lds, xp, wp, wave, lane, wt, K / 32, turn, acc); break
-    KVC_WALK(1); KVC_WALK(2); KVC_WALK(3); KVC_WALK(4); KVC_WALK(5); KVC_WALK(6); KVC_WALK(7);
-    KVC_WALK(8); KVC_WALK(9); KVC_WALK(10); KVC_WALK(11);
+#define KVC_WALK_OF(R, ONCE) wide_walk<PACKED, R, ONCE>(lds, xp, wp, wave, lane, wt, K / 32, turn, acc)
+#define KVC_WALK(R) case R: KVC_WALK_OF(R, kStream); break
+#define KVC_WALK2(R)                       \
+  case R:                                  \
+    if (alone) KVC_WALK_OF(R, kStream);    \
+    else KVC_WALK_OF(R, false);            \
+    break
+    KVC_WALK(1); KVC_WALK(2); KVC_WALK(3); KVC_WALK(4); KVC_WALK(5); KVC_WALK2(6); KVC_WALK2(7);
+    KVC_WALK2(8); KVC_WALK2(9); KVC_WALK2(10); KVC_WALK2(11); KVC_WALK2(12);
+#undef KVC_WALK2
 #undef KVC_WALK
-    default: wide_walk<PACKED, kWideBlocks>(lds, xp, wp, wave, lane, wt, K / 32, turn, acc);
+#undef KVC_WALK_OF
   }
   if (n0 >= N) return;  // the whole wave
   // lane holds row 16 (2 r + wr) + li of the tile, columns n0 + 16 f + 4 lk + i
@@ -1444,7 +1482,9 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
       if (packed && (N % 16 || K % 64))
         return kvc_fail("kvc_moe_gemm: a packed matrix has experts of a multiple of 16 rows of a multiple of 64");
       const int64_t cols = gated ? (N + 127) / 128 : (N + 255) / 256;
-      const int64_t blocks = 8 * ((cols * max_tiles + 7) / 8);  // every die gets its share of the pairs
+      // every die gets its share of the pairs, or (384 rows) of the tiles
+      const int64_t blocks = tile_rows == kWideTileRows ? 8 * (cols * ((static_cast<int64_t>(max_tiles) + 7) / 8))
+                                                        : 8 * ((cols * max_tiles + 7) / 8);
       if (blocks > 0x7fffffff) return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
       grid = dim3(static_cast<unsigned>(blocks));
 #define KVC_MOE_TILED(NR, PACKED)                                                                               \

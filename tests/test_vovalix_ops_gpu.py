@@ -641,6 +641,33 @@ def test_products_of_experts_over_tiles_of_384_rows(packed, gated, N, K, out_dty
     assert rel(outs[0], want) < (2e-6 if out_dtype == torch.float32 else 3e-3)
 
 
+@pytest.mark.parametrize("gated,N", [(True, 176), (False, 272), (True, 4224)])
+@pytest.mark.parametrize("counts", [[300] * 7, [300] * 8, [40, 385] * 4 + [0, 200], [500] * 5, [33] * 67, [20] * 60 + [385] * 8,
+                                    [390, 10] * 33], ids=lambda c: f"{len(c)}x{c[0]}")
+def test_tiles_of_384_rows_dealt_to_the_dies_by_tile_and_by_column(counts, gated, N):
+    """Fewer tiles than dies, as many, more than a wave looks at at once; one tile an expert, a few of two, all of two;
+    one column block, two, and more than a die takes in a round: the same bits as tiles of 128 rows."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(N + len(counts))
+    E, T, K = len(counts), sum(counts), 64
+    i32 = dict(dtype=torch.int32, device=DEV)
+    choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=gen)].to(**i32)
+    xg = gpu(torch.randn(T, K, generator=gen), torch.bfloat16)
+    wg = gpu(torch.randn(E * N * (2 if gated else 1), K, generator=gen), torch.bfloat16)
+    ops.pack_weight(wg)
+    outs = []
+    for tile_rows in (384, 128):
+        sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+        tiles = torch.empty(ops.moe_max_tiles(T, E, tile_rows), 3, **i32)
+        ops.moe_align(sorted_pairs, tiles, num, choice.view(T, 1), E, tile_rows)
+        out = torch.full((T, N), float("nan"), dtype=torch.float32, device=DEV)
+        ops.moe_gemm(out, xg, wg, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1, out_sorted=False, gated=gated,
+                     tile_rows=tile_rows)
+        outs.append(out)
+    assert torch.equal(*outs) and outs[0].isfinite().all()
+
+
 @pytest.mark.parametrize("E", [1, 31, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("counts_of", ["equal", "edges", "drawn"])
 def test_tiles_of_384_rows_hold_every_pair_once(E, counts_of):
