@@ -376,6 +376,10 @@ int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const void* x, in
 int kvc_moe_combine(float* out, const float* y, const float* weight, int top, const void* add0,
                     int add0_dtype, const float* add1, const float* add1_gate, int T, int H, int accumulate,
                     kvc_stream stream);
+// kvc_moe_combine into residual (float32 add0), then x (of x_dtype) = gain * residual / rms(residual), eps inside the root.
+int kvc_moe_combine_norm(void* x, int x_dtype, float* residual, const float* y, const float* weight, int top,
+                         const float* add0, const float* add1, const float* add1_gate, const float* gain, float eps,
+                         int T, int H, kvc_stream stream);
 
 // The same attention for bfloat16 steps of single tokens on the matrix cores, a block of
 // several waves per (token, kv head, split), which also does what kvc_rope_kv_write does for

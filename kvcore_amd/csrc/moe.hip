@@ -34,6 +34,7 @@
 //   kvc_moe_combine  out[t] = sum_c weight[t, c] * y[t * top + c] (without weights: the plain sum) (+ up to two more row sets, the second
 //                    times a number a token where one is given), float32, in the order of the
 //                    choices; or added into out (the residual stream).
+//   kvc_moe_combine_norm  the same added into the residual stream, and the RMS norm of its new rows
 
 #include <hip/hip_runtime.h>
 
@@ -1269,6 +1270,63 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ ou
   *o = accumulate ? *o + acc : acc;
 }
 
+// The same into the residual stream, a block a token, which has the new row in registers and leaves its norm for the next layer:
+// in few rows a launch is all that the norm by itself takes, in many its row read again.  Every sum in the order of the two
+// kernels (`add_rmsnorm_vec_kernel` has the norm's), so with their bits.  2,048 columns, four choices and two more rows, float32 to
+// bfloat16, in a graph, two kernels / this one: 1 token 5.1 / 3.5 us, 8 5.3 / 3.7, 64 6.2 / 4.1, 300 8.2 / 6.2, 2,048 31.4 / 27.0 (5.6 TB/s).
+template <typename TO, int NCH>
+__global__ __launch_bounds__(256) void moe_combine_norm_kernel(
+    TO* __restrict__ x, float* __restrict__ residual, const float* __restrict__ y, const float* __restrict__ weight, int top,
+    const float* __restrict__ add0, const float* __restrict__ add1, const float* __restrict__ add1_gate,
+    const float* __restrict__ gain, float eps, int H) {
+  __shared__ float scratch[16];
+  const int64_t t = blockIdx.x, base = t * H;
+  float v[NCH][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int e = (c * 256 + threadIdx.x) * 8;
+    if (e >= H) continue;
+    const float* yt = y + t * top * H + e;
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, u[8];
+#pragma unroll 4
+    for (int j = 0; j < top; ++j) {
+      const float w = weight != nullptr ? weight[t * top + j] : 1.f;
+      load8(yt + static_cast<int64_t>(j) * H, u);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = fmaf(w, u[i], acc[i]);
+    }
+    if (add0 != nullptr) {
+      load8(add0 + base + e, u);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] += u[i];
+    }
+    if (add1 != nullptr) {
+      load8(add1 + base + e, u);
+      const float g = add1_gate != nullptr ? add1_gate[t] : 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] = add1_gate != nullptr ? fmaf(g, u[i], acc[i]) : acc[i] + u[i];
+    }
+    load8(residual + base + e, v[c]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[c][i] += acc[i];
+    store8(residual + base + e, v[c]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += v[c][i] * v[c][i];
+  }
+  const float inv = rsqrtf(block_sum(ss, scratch) / static_cast<float>(H) + eps);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int e = (c * 256 + threadIdx.x) * 8;
+    if (e >= H) continue;
+    float w[8], o[8];
+    load8(gain + e, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = w[i] * (v[c][i] * inv);
+    store8(x + base + e, o);
+  }
+}
+
 }  // namespace
 
 extern "C" int kvc_moe_route(int32_t* choice, float* weight, const float* logits, int T, int E, int top,
@@ -1584,4 +1642,35 @@ extern "C" int kvc_moe_combine(float* out, const float* y, const float* weight, 
   }
 #undef KVC_COMBINE
   return kvc_check_launch("kvc_moe_combine");
+}
+
+extern "C" int kvc_moe_combine_norm(void* x, int x_dtype, float* residual, const float* y, const float* weight, int top,
+                                    const float* add0, const float* add1, const float* add1_gate, const float* gain,
+                                    float eps, int T, int H, kvc_stream stream) {
+  if (T < 0 || H <= 0 || top < 0) return kvc_fail("kvc_moe_combine_norm: bad sizes");
+  if (x_dtype != 0 && x_dtype != 1) return kvc_fail("kvc_moe_combine_norm: unknown dtype code");
+  if (T == 0) return 0;
+  const uintptr_t places = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(residual) |
+                           reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(add0) |
+                           reinterpret_cast<uintptr_t>(add1) | reinterpret_cast<uintptr_t>(gain);
+  if (H % 8 || H > 8 * 2048 || (places & 15)) {  // no vectors, or more than a block's registers hold: one after the other
+    const int bad = kvc_moe_combine(residual, y, weight, top, add0, 0, add1, add1_gate, T, H, 1, stream);
+    return bad ? bad : kvc_add_rmsnorm(x, residual, nullptr, gain, eps, T, H, x_dtype, stream);
+  }
+  const int nch = (H + 2047) / 2048;
+#define KVC_COMBINE_NORM(TO, NCH)                                                                              \
+  hipLaunchKernelGGL((moe_combine_norm_kernel<TO, NCH>), dim3(T), dim3(256), 0, S(stream), static_cast<TO*>(x), \
+                     residual, y, weight, top, add0, add1, add1_gate, gain, eps, H)
+#define KVC_COMBINE_NORM_OF(TO)               \
+  do {                                        \
+    if (nch <= 1) KVC_COMBINE_NORM(TO, 1);      \
+    else if (nch <= 2) KVC_COMBINE_NORM(TO, 2); \
+    else if (nch <= 4) KVC_COMBINE_NORM(TO, 4); \
+    else KVC_COMBINE_NORM(TO, 8);               \
+  } while (0)
+  if (x_dtype == 1) KVC_COMBINE_NORM_OF(bf16_t);
+  else KVC_COMBINE_NORM_OF(float);
+#undef KVC_COMBINE_NORM_OF
+#undef KVC_COMBINE_NORM
+  return kvc_check_launch("kvc_moe_combine_norm");
 }

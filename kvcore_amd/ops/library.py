@@ -80,6 +80,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_moe_align": [P, P, P, P, I, I, I, I, P],
         "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, I, P],
         "kvc_moe_combine": [P, P, P, I, P, I, P, P, I, I, I, P],
+        "kvc_moe_combine_norm": [P, I, P, P, P, I, P, P, P, P, F, I, I, P],
         "kvc_qk_norm_rope_kv_write": [P, L, P, P, I, P, P, F, P, P, I, I, P, I, I, I, I, I, I, I, I, I, P],
         "kvc_add_layernorm": [P, P, P, P, P, F, I, I, I, P],
         "kvc_rms_branches_mean": [P, P, P, I, F, I, I, I, P],
@@ -2187,6 +2188,21 @@ def moe_combine(out: torch.Tensor, y: torch.Tensor, weight: torch.Tensor | None,
                                   None if add1 is None else _dev(add1, "add1", torch.float32),
                                   None if add1_gate is None else _dev(add1_gate, "add1_gate", torch.float32), T, H,
                                   int(bool(accumulate)), _stream()), "kvc_moe_combine")
+
+
+def moe_combine_norm(x: torch.Tensor, residual: torch.Tensor, rows: "WeightedRows", gain: torch.Tensor, eps: float,
+                     add: torch.Tensor | None = None) -> None:
+    """:func:`moe_combine` of ``rows`` and ``add`` (float32) into the stream ``residual``, and ``x = gain * residual /
+    rms(residual)`` (eps inside the root): the next layer's norm in the kernel that adds the experts up."""
+    T, H = residual.shape
+    top = rows.check(T, H)
+    if x.shape != (T, H) or gain.shape != (H,) or (add is not None and add.shape != (T, H)):
+        raise KernelError("moe_combine_norm: shapes do not match")
+    opt = [None if t is None else _dev(t, "a row set", torch.float32) for t in (rows.weight, add, rows.add, rows.add_gate)]
+    _check(load().kvc_moe_combine_norm(_dev(x, "x"), _code(x, "x"), _dev(residual, "residual", torch.float32),
+                                       _dev(rows.data, "rows", torch.float32), opt[0], top, *opt[1:],
+                                       _dev(gain, "gain", torch.float32), float(eps), T, H, _stream()),
+           "kvc_moe_combine_norm")
 
 
 def clamped_glu(out: torch.Tensor, gate_up: torch.Tensor, limit: float, alpha: float) -> None:

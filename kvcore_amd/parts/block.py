@@ -104,7 +104,8 @@ class PreNormBlock(Block):
 class ParallelResidualBlock(Block):
     """``r += delta; h = norm(r); r += mixer(h) + ffn(h)``: one norm a layer, both branches read
     its output, and both sums go straight into the float32 stream (nothing stays pending, so the
-    branches may hand over float32 rows).  With a feed-forward of kind ``none`` the mixer is
+    branches may hand over float32 rows), with the norm of a parallel block behind it where the feed-forward's
+    last kernel can make it.  With a feed-forward of kind ``none`` the mixer is
     the layer."""
 
     def __init__(self, *, mixer: Mixer, ffn: FeedForward, norms: dict[str, Norm],
@@ -126,13 +127,22 @@ class ParallelResidualBlock(Block):
         if isinstance(delta, (ops.ScaledRows, ops.NormedRows)):
             raise RuntimeError("a parallel block takes its input from the stream, not from folded norms")
         x = ctx.buf("block_x", residual.shape[1])
-        self.norms[self.norm_name].forward_fused(x, residual, delta)
+        if ctx.scratch.pop("stream_normed", None) != call.exec_index:  # else the block before left the norm there
+            self.norms[self.norm_name].forward_fused(x, residual, delta)
         a = self.mixer.forward(x, ctx, call)
         if self.mixer_only:
             ops.residual_add(residual, a)
         elif a.dtype == torch.float32 and hasattr(self.ffn, "forward_into"):
-            # a feed-forward whose last kernel can add into the stream takes the mixer's rows along
-            self.ffn.forward_into(residual, x, ctx, call, add=a)
+            # a feed-forward whose last kernel can add into the stream takes the mixer's rows along, and
+            # has the next layer's first norm at hand
+            gain = None
+            if isinstance(next_block, ParallelResidualBlock) and hasattr(self.ffn, "forward_into_normed"):
+                gain = next_block.norms[next_block.norm_name].as_gain()
+            if gain is None:
+                self.ffn.forward_into(residual, x, ctx, call, add=a)
+            else:  # into x, which nothing reads any more by then
+                self.ffn.forward_into_normed(x, residual, x, ctx, call, *gain, add=a)
+                ctx.scratch["stream_normed"] = call.exec_index + 1
         else:
             f = self.ffn.forward(x, ctx, call)
             ops.residual_add2(residual, a, f)

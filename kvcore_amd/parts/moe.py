@@ -130,6 +130,10 @@ class RoutedExperts(FeedForward):
         experts: what a block calls that would otherwise add the result into the stream itself."""
         self.forward(x, ctx, call, into=residual, add=add)
 
+    def forward_into_normed(self, out, residual, x, ctx, call, gain, eps, add=None):
+        """:meth:`forward_into`, and ``out`` gets the RMS norm of the new rows of the stream (the next layer's)."""
+        ops.moe_combine_norm(out, residual, self.forward_weighted(x, ctx, call), gain, eps, add=add)
+
     def forward(self, x, ctx, call, sink=None, into=None, add=None):
         rows = self.forward_weighted(x, ctx, call)
         out = ctx.buf("ffn_out_f32", self.hidden_size, torch.float32) if into is None else into

@@ -668,6 +668,26 @@ def test_tiles_of_384_rows_dealt_to_the_dies_by_tile_and_by_column(counts, gated
     assert torch.equal(*outs) and outs[0].isfinite().all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,top", [(1, 8, 1), (3, 2048, 4), (67, 2056, 3), (2, 4096, 8), (5, 16384, 5), (5, 16392, 2), (4, 2047, 4)])
+def test_experts_sums_with_the_next_norm(T, H, top, dtype):
+    """Rows of one chunk a block, a few, all that its registers hold, and those that take two kernels: the bits of the
+    two kernels, with and without weights, a further row and its gate, and the mixer's rows."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(T + H)
+    draw = lambda *shape: gpu(torch.randn(*shape, generator=gen))  # noqa: E731
+    y, gain, start = draw(T * top, H), draw(H), draw(T, H)
+    for weight, shared, gate, other in ((draw(T, top), draw(T, H), draw(T, 1), draw(T, H)), (None, None, None, None),
+                                        (draw(T, top), draw(T, H), None, None), (None, None, None, draw(T, H))):
+        want, got = start.clone(), start.clone()
+        rows, x = (torch.empty(T, H, dtype=dtype, device=DEV) for _ in range(2))
+        ops.moe_combine(want, y, weight, other, shared, accumulate=True, add1_gate=gate, count=top)
+        ops.add_rmsnorm(rows, want, None, gain, 1e-5)
+        ops.moe_combine_norm(x, got, ops.WeightedRows(y, weight, shared, gate, count=top), gain, 1e-5, add=other)
+        assert torch.equal(got, want) and torch.equal(x, rows)
+
+
 @pytest.mark.parametrize("E", [1, 31, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("counts_of", ["equal", "edges", "drawn"])
 def test_tiles_of_384_rows_hold_every_pair_once(E, counts_of):
