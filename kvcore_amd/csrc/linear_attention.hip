@@ -104,13 +104,16 @@ __global__ __launch_bounds__(256) void linear_state_scan_kernel(
   float s[NPT];
   if (!fresh) {  // the same for the whole block
     // every row is asked for with no branch between the loads (a row or column that is not there
-    // reads one that is, and is then set to zero), so that all of them are in flight together
+    // reads one that is, and is then set to zero), so that all of them are in flight together; marked as streaming
+    // ones, as the stores are (a launch reads and writes a state once, and the layers' states of a full batch are more than
+    // the caches hold): 64 requests at one token, 16 heads of 128 x 128 (134 MB) 49.3 -> 47.2 us, of 64 x 128 (67 MB) 21.8 -> 19.6,
+    // and a step of 64 over four and eight such layers 4,032 -> 3,979 us, of 8 2,341 -> 2,331
     const int c_safe = c_ok ? c : dv - 1;
 #pragma unroll
     for (int i = 0; i < NPT; ++i) {
       const int n = ns + NSL * i;
       const int n_safe = (FULL || n < d) ? n : 0;
-      s[i] = st[(static_cast<int64_t>(n_safe >> 2) * dv + c_safe) * 4 + (n_safe & 3)];
+      s[i] = __builtin_nontemporal_load(st + (static_cast<int64_t>(n_safe >> 2) * dv + c_safe) * 4 + (n_safe & 3));
     }
 #pragma unroll
     for (int i = 0; i < NPT; ++i)
@@ -377,7 +380,7 @@ __global__ __launch_bounds__(256) void linear_state_scan_kernel(
 #pragma unroll
   for (int i = 0; i < NPT; ++i) {
     const int n = ns + NSL * i;
-    if (n < d) st[st_at(n)] = s[i];
+    if (n < d) __builtin_nontemporal_store(s[i], st + st_at(n));
   }
 }
 

@@ -737,11 +737,13 @@ __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(
   const int g = h / (nh / G);
   float* st = state + (static_cast<int64_t>(slots[r]) * nh + h) * N * P;
   const bool fresh = positions[b] == 0;
+  // a launch reads and writes a state once: streaming loads and stores.  64 requests at one token, 268 MB: 61.3 -> 55.3 us, the step of
+  // eight such layers 2,924 -> 2,796 us (of 8 requests 1,462 -> 1,441)
   float s[NPT];
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int n = ns * NPT + k;
-    s[k] = (!fresh && p_ok && n < N) ? st[static_cast<int64_t>(n) * P + p] : 0.f;
+    s[k] = (!fresh && p_ok && n < N) ? __builtin_nontemporal_load(st + static_cast<int64_t>(n) * P + p) : 0.f;
   }
   const float neg_a = -expf(a_log[h]);
   const float bias = dt_bias[h];
@@ -830,7 +832,7 @@ __global__ __launch_bounds__(256) void ssm_scan_wide_kernel(
 #pragma unroll
   for (int k = 0; k < NPT; ++k) {
     const int n = ns * NPT + k;
-    if (n < N) st[static_cast<int64_t>(n) * P + p] = s[k];
+    if (n < N) __builtin_nontemporal_store(s[k], st + static_cast<int64_t>(n) * P + p);
   }
 }
 
