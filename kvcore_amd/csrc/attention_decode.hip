@@ -131,9 +131,9 @@ template <int D, int DV>
 int launch_decode(DecodeArgs& args, int T, hipStream_t stream) {
   const int g = args.nh / args.nkv;
   // a split's range of pages always fits: the table's width cut into nsplit parts, and slack, as a split is whole
-  // units of two blocks; all of them may end one page behind the table
-  args.lds_pages = (args.table_stride + args.nsplit - 1) / args.nsplit + 4;
-  if (args.lds_pages > args.table_stride + 1) args.lds_pages = args.table_stride + 1;
+  // units of 32 keys (not more than two pages, also where a page is half a unit, as none behind the token's own counts)
+  args.lds_pages = (args.table_stride + args.nsplit - 1) / args.nsplit + 2;
+  if (args.lds_pages > args.table_stride) args.lds_pages = args.table_stride;
   int waves = decode_waves(g, D);
   // more blocks than compute units: smaller blocks pack better
   if (static_cast<int64_t>(T) * args.nkv * args.nsplit > kvc_device_compute_units() && waves > 4) waves = 4;

@@ -177,7 +177,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
   const int unit_own = unit_end - 1;  // the unit of the token's own key
   const int blk_own = pos / 16;
   const bool owner = a.write_kv && u0 <= unit_own && unit_own < u1;
-  // page that holds 16-key block b; the host keeps b below 2^27 and the division exact
+  // page that holds 16-key block b (exact: see page_magic_of)
   auto page_index = [&](int b) {
     return a.page_magic == 0 ? b : static_cast<int>(__umulhi(static_cast<unsigned>(b), a.page_magic));
   };
@@ -185,7 +185,9 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
 
   // the page ids of the range go to LDS, where the walk below reads them
   const int page_lo = page_index(2 * u0);
-  const int n_range_pages = (u1 > u0) ? page_index(2 * u1 - 1) - page_lo + 1 : 0;
+  // of a unit's second half only where the token sees it, so that no page behind the token's own has a place
+  auto second_page = [&](int u) { return page_index(2 * u + 1 < blk_own ? 2 * u + 1 : blk_own) - page_lo; };
+  const int n_range_pages = (u1 > u0) ? second_page(u1 - 1) + 1 : 0;
   for (int i = tid; i < n_range_pages && i < a.lds_pages; i += nthreads)
     spage[i] = (page_lo + i < a.table_stride) ? row[page_lo + i] : 0;
 
@@ -435,7 +437,7 @@ __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk,
   if (has_work) {
     auto next_pages = [&](Unit& un, int u) {
       set_pages(un, u, __builtin_amdgcn_readfirstlane(spage[page_index(2 * u) - page_lo]),
-                __builtin_amdgcn_readfirstlane(spage[page_index(2 * u + 1) - page_lo]));
+                __builtin_amdgcn_readfirstlane(spage[second_page(u)]));
     };
     int u = u_wave;
     if constexpr (two_units<D, DV>()) {

@@ -1276,6 +1276,36 @@ def test_decode_attention_keeps_infinite_values_and_the_bits_of_its_probabilitie
         assert torch.isfinite(out.view(nh, d)[:, 8:]).all()
 
 
+@pytest.mark.parametrize("nsplit", [1, 2, 5])
+@pytest.mark.parametrize("page", [16, 48])
+def test_decode_attention_over_the_widest_tables(ops, nsplit, page):
+    """A split has room for its share of the table and two pages more: tables of as many entries as that allows are served
+    up to the last token's key.  Five pages of keys again and again, so that each of their keys has a known weight."""
+    dtype, nh, nkv, d = torch.bfloat16, 2, 1, 32
+    widest = ops.decode_attention_max_table(nh, nkv, d)
+    width = widest + 2 if nsplit == 1 else widest * nsplit
+    i32 = dict(dtype=torch.int32, device=DEV)
+    kc, vc = rnd(6, nkv, page, d, dtype=dtype, seed=1), rnd(6, nkv, d, page, dtype=dtype, seed=2)
+    q = rnd(1, nh * d, dtype=dtype, seed=3)
+    table = torch.zeros(2, width, **i32)
+    table[1] = torch.arange(width, **i32) % 5 + 1
+    out = torch.full((1, nh * d), float("nan"), device=DEV)
+    parts = torch.full((nh * nsplit * d,), float("nan"), device=DEV), torch.full((nh * nsplit * 2,), float("nan"), device=DEV)
+    ops.decode_attention(out, q, kc, vc, table=table, positions=torch.tensor([width * page - 1], **i32),
+                         token_req=torch.zeros(1, **i32), slots=torch.ones(1, **i32), nh=nh, nkv=nkv, d=d, scale=d ** -0.5,
+                         nsplit=nsplit, part_o=parts[0], part_ml=parts[1])
+    times = torch.bincount(table[1].long().cpu(), minlength=6).double()[1:]
+    k, v = kc[1:, 0].double().cpu(), vc[1:, 0].double().cpu()
+    w = torch.exp(torch.einsum("hd,pkd->hpk", q.double().cpu().view(nh, d), k) * d ** -0.5) * times[:, None]
+    want = torch.einsum("hpk,pdk->hd", w / w.sum((1, 2), keepdim=True), v)
+    # probabilities of 16 bits, and a wave's 4,000 sums one after the other in float32, of |v| of about one
+    assert float((out.double().cpu().view(nh, d) - want).abs().max()) < 2.0 ** -16 + 4000 * 2.0 ** -24
+    with pytest.raises(ops.KernelError):
+        ops.decode_attention(out, q, kc, vc, table=torch.zeros(2, width + 2 * nsplit, **i32), positions=torch.zeros(1, **i32),
+                             token_req=torch.zeros(1, **i32), slots=torch.ones(1, **i32), nh=nh, nkv=nkv, d=d,
+                             scale=d ** -0.5, nsplit=nsplit, part_o=parts[0], part_ml=parts[1])
+
+
 @pytest.mark.parametrize("nsplit", [1, 5])
 def test_decode_attention_far_key_and_window(ops, nsplit):
     dtype = torch.bfloat16
