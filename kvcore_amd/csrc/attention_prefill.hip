@@ -829,8 +829,13 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   // where those take 53), two tiles a block of eight waves where those just fill the chip (1.06 to 1.09); heads of 128 32 rows
   // a wave (1.00 to 1.08), except that long requests pair their tiles.
   //
-  // With splits of the keys: one tile of 64 rows a block up to cu (1.00 to 1.07; 32 rows a wave and two tiles a block 1.2 to
-  // 1.75), on heads of 64 up to 2 cu (1.00 to 1.08), else 32 rows a wave, one tile a block on heads of 128 (1.00 to 1.02).
+  // With splits of the keys: one tile of 64 rows a block as long as the blocks of all splits find room at once, two a unit
+  // (heads of 64: three), else 32 rows a wave, one tile a block, which stages each key for twice the rows; two tiles a block
+  // are never the best.  512 tokens behind 2,000 in four splits 60 and 52 us, behind 8,000 in eight 145 and 111 (two tiles a
+  // block 112), 300 behind 1,000 in three 34 and 35.  Long requests of heads of 64, or with narrow values: eight waves (512
+  // behind 16,000 in eight 130 and 113; 4,096 of 128 / 64 behind 8,000 in two 339 and 295).
+  // Over 850 launches with splits 1.03 of the best of all ways; one tile of 64 rows up to cu blocks whatever the splits
+  // 1.05, and for some long contexts 1.5.
   // (The rules know nothing of the values, so that one call over two planes and a call for each take the same tiles.)
   const int ones = g <= 16 ? singles : 0;  // single tokens that are blocks of their own kind
   const int T1 = T - ones, R1 = R - ones > 1 ? R - ones : 1;
@@ -848,10 +853,9 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
     ct = 2;
     single = 0;
   } else if (nsplit > 1) {
-    if (blocks > (D == 64 ? 2 : 1) * cu) ct = 2;
-    if (D == 64 && ct == 2) {  // 2,048 tokens behind 1,200: two tiles a block of eight waves 0.97, one of four 1.09
-      single = 0;
-      if (long_requests) waves = 8;
+    if (blocks * nsplit > (D == 64 ? 3 : 2) * cu) {
+      ct = 2;
+      if (long_requests && (D == 64 || DV < D)) waves = 8;
     }
   } else if (blocks <= cu) {
   } else if (blocks <= 2 * cu) {

@@ -1790,6 +1790,61 @@ def test_prefill_attention_of_single_tokens_beside_portions(ops, nh, nkv, d, dv,
     assert torch.allclose(out.float(), ref.float(), atol=2e-2, rtol=1e-2)
 
 
+def prefill_beside(ops, nh, nkv, d, portions, singles, nsplit=1, planes=1, dv=None, far=None):
+    """Portions ``[(start, tokens)]`` with single tokens (``singles`` of them, their positions 3 to 400) before, between and
+    behind, by the kernel for portions and by the general one -> ``(variant, result, reference)``.  ``far``: one of the
+    single tokens sits at this position, behind its keys' pages again and again."""
+    dtype, page, dv = torch.bfloat16, 16, dv or d
+    ones = [(3 + 397 * i // max(singles, 1), 1) for i in range(singles)]
+    spans = ones[: singles // 3] + [portions[0]] + ones[singles // 3: singles * 2 // 3] + portions[1:] + ones[singles * 2 // 3:]
+    if far is not None:
+        spans[spans.index(ones[singles // 2])] = (160, 1)  # as far as its pages are concerned
+    kc, vc, table, _ = paged_setup([p + n for p, n in spans], nkv, d, page, dtype, seed=nh + d)
+    vcs = [vc[:, :, :dv].contiguous(), rnd(*vc[:, :, :dv].shape, dtype=dtype, seed=5)][:planes]
+    positions = torch.tensor([p + i for p, n in spans for i in range(n)], dtype=torch.int32, device=DEV)
+    starts = [sum(n for _, n in spans[:r]) for r in range(len(spans) + 1)]
+    if far is not None:
+        r = spans.index((160, 1))
+        wide = torch.zeros(table.shape[0], far // page + 1, dtype=torch.int32, device=DEV)
+        wide[:, : table.shape[1]] = table
+        wide[r + 1] = table[r + 1, torch.arange(wide.shape[1], device=DEV) % 10]
+        table, positions[starts[r]] = wide, far
+    token_req = torch.tensor([r for r, (_, n) in enumerate(spans) for _ in range(n)], dtype=torch.int32, device=DEV)
+    T, R = starts[-1], len(spans)
+    q = rnd(T, nh * d, dtype=dtype, seed=4)
+    common = dict(table=table, positions=positions, slots=torch.arange(1, R + 1, dtype=torch.int32, device=DEV), nh=nh, nkv=nkv,
+                  d=d, scale=d ** -0.5)
+    out = torch.full((T, nh * dv * planes), float("nan"), dtype=dtype, device=DEV)
+    ops.prefill_attention(out, q, kc, vcs[0], q_start=torch.tensor(starts, dtype=torch.int32, device=DEV), num_reqs=R,
+                          nsplit=nsplit, singles=singles, context=sum(p for p, _ in portions) // len(portions), dv=dv * planes,
+                          v_second=vcs[1] if planes == 2 else None,
+                          part_o=torch.full((T * nh * nsplit, dv * planes), float("nan"), device=DEV),
+                          part_ml=torch.full((T * nh * nsplit, 2), float("nan"), device=DEV), **common)
+    refs = []
+    for v in vcs:
+        refs.append(torch.empty(T, nh, dv, dtype=dtype, device=DEV))
+        ops.paged_attention(refs[-1].view(T, -1), q, kc, v, token_req=token_req, dv=dv, **common)
+    return ops.last_variant("prefill_attention"), out.float(), torch.cat(refs, -1).view(T, -1).float()
+
+
+SHAPES_OF_PREFILL = {"128": (32, 8, 128), "64": (32, 8, 64), "128/64": (16, 4, 128)}
+
+
+@pytest.mark.parametrize("shape,tokens,portions,nsplit,way", [
+    ("128", 512, 1, 2, "1s4"), ("128", 512, 1, 3, "2s4"), ("64", 512, 1, 3, "1s4"), ("64", 512, 1, 4, "2s8"),
+    ("64", 300, 2, 4, "2s4"), ("128/64", 1100, 1, 3, "2s8"), ("128/64", 500, 1, 4, "1s4"), ("128/64", 520, 1, 5, "2s4")])
+@pytest.mark.parametrize("singles", [0, 5])
+def test_prefill_attention_with_splits_takes_small_tiles_while_all_blocks_find_room(ops, shape, tokens, portions, nsplit, way, singles):
+    """Tiles of 64 rows as long as the blocks of all splits find room at once (two a unit, three of heads of 64), else
+    32 rows a wave, on eight waves for long requests of narrow heads; either side of the line, beside single tokens and alone."""
+    nh, nkv, d = SHAPES_OF_PREFILL[shape]
+    variant, out, ref = prefill_beside(ops, nh, nkv, d, [(40, tokens)] * portions, singles, nsplit, dv=64 if "/" in shape else d)
+    assert variant.startswith(f"prefill_attention_kernel<{d},{way[0]},") and f",{way[2]}>" in variant, variant
+    assert variant.endswith(f"x{nsplit}") and ("one tile a block" in variant) == (way[1] == "s"), variant
+    # both round p and the result to bfloat16: half of 2^-8 of sums of |v| <= 4.5, twice each
+    assert torch.allclose(out, ref, atol=2e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("nh,nkv,d,whole,nsplit", [(8, 2, 128, 2100, 1), (8, 1, 64, 2100, 1), (32, 8, 128, 4200, 1),
                                                    (8, 2, 128, 2100, 7), (8, 1, 64, 2100, 2),
                                                    (16, 4, 128, 2100, 1), (16, 4, 128, 3100, 1),
