@@ -813,10 +813,11 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   // the compute units, and whether all blocks find room at once.  Single tokens are blocks of their own kind that take a
   // place for a short while.  Measured over 1,000 launches of 1 to 8 portions of 30 to 2,048 tokens, from position 0 and
   // behind 200 to 1,200 tokens, alone and beside 24 single tokens, against the best of all ways:
-  // Up to cu blocks one tile of 64 rows a block (others 1.05 to 1.6).  Up to 2 cu tiles of 128 rows, eight waves, from 11/8 cu
-  // on, where they and the single tokens' blocks find a unit each (0.79 to 1.04 of tiles of 64 rows; below 11/8 cu, which
-  // leaves them too few, 0.89 to 1.3); else four (beside many single tokens 1.00 to
-  // 1.03, eight waves 1.04 to 1.18).
+  // Up to 2 cu blocks one tile of 64 rows a block (others 1.05 to 1.6), or, where all blocks, single tokens' among them, then
+  // find a unit each, tiles of 128 rows on eight waves: from 11/8 cu on (0.79 to 1.04; below, which leaves them too few, 0.89 to
+  // 1.3, and with fewer than some 128 keys a row 1.2), and long requests of heads of 64, or with narrow values, at any
+  // number (0.88 to 1.03 over 480 launches; 700 tokens over 8 of 64 behind 600 27.5 and 25.7 us, 1,300 over 4 of 128 / 64 43.2 and
+  // 39.1).  Where they do not find one each 1.04 to 1.3.
   //
   // Whole prompts of more: their early tiles see few keys and their late ones many, so a block takes two.  At 32 heads over 8
   // kv heads of 128, one request, four waves against eight: 2,048 tokens 83 against
@@ -826,7 +827,9 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   //
   // Portions behind a context, or beside single tokens, have tiles of like lengths (two a block 1.1 to 1.45 below 4 cu): up
   // to 4 cu heads of 64 four waves (1.00 to 1.05; long portions alone up to 3 cu eight, as over two planes four take 63 us
-  // where those take 53), two tiles a block of eight waves where those just fill the chip (1.06 to 1.09); heads of 128 32 rows
+  // where those take 53), above 3 cu 32 rows a wave for short requests, whose tiles of 128 rows are ragged (eight of 240
+  // tokens 38 us with two of those a block, 27 so), and for long ones two tiles a block of eight waves where those just fill the
+  // chip (1.06 to 1.09), below 7/2 cu one (24 heads of 64, 2,048 tokens 44 and 39); heads of 128 32 rows
   // a wave (1.00 to 1.08), except that long requests pair their tiles.
   //
   // With splits of the keys: one tile of 64 rows a block as long as the blocks of all splits find room at once, two a unit
@@ -857,9 +860,10 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
       ct = 2;
       if (long_requests && (D == 64 || DV < D)) waves = 8;
     }
-  } else if (blocks <= cu) {
   } else if (blocks <= 2 * cu) {
-    if (blocks / 2 + single_blocks <= cu && 8 * blocks > 11 * cu) waves = 8;
+    const bool few_keys = static_cast<int64_t>(T1 / R1) + context < 128;
+    if (blocks / 2 + single_blocks <= cu && ((long_requests && (D == 64 || DV < D)) || (8 * blocks > 11 * cu && !few_keys)))
+      waves = 8;
   } else if (whole_prompts) {
     if (pairs > 2 * cu) {
       ct = 2;
@@ -876,8 +880,12 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
       if (blocks <= 3 * cu) {
         if (single_blocks == 0 && long_requests) waves = 8;
       } else if (blocks / 4 + single_blocks <= cu + nkv) {
-        waves = 8;
-        single = 0;
+        if (long_requests) {
+          waves = 8;
+          single = 2 * blocks <= 7 * cu;
+        } else {
+          ct = 2;
+        }
       }
     } else if (blocks > 3 * cu && long_requests) {
       waves = 8;

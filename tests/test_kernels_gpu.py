@@ -1845,6 +1845,43 @@ def test_prefill_attention_with_splits_takes_small_tiles_while_all_blocks_find_r
     assert torch.allclose(out, ref, atol=2e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("shape,portions,singles,planes,way", [
+    # up to twice the units in small tiles: eight waves where all blocks find a unit each ...
+    ("128", [(100, 720)], 3, 1, "1s8"), ("128", [(100, 700)], 3, 1, "1s4"), ("128", [(100, 720)], 12, 1, "1s4"),
+    ("64 over 8", [(0, 57)] * 8, 0, 1, "1s4"), ("64 over 8", [(100, 57)] * 8, 0, 1, "1s8"),  # few keys a row, more
+    # ... and for long requests of narrow heads at any number
+    ("64", [(100, 600)], 2, 1, "1s8"), ("64", [(100, 600)], 14, 1, "1s4"), ("64", [(100, 600)], 2, 2, "1s8"),
+    ("128/64", [(0, 1030)], 4, 1, "1s8"), ("128/64", [(0, 1000)], 4, 1, "1s4"),
+    # whole prompts
+    ("128", [(0, 1100)], 0, 1, "1s8"), ("128", [(0, 300)] * 4, 0, 1, "1p4"), ("128", [(0, 2200)], 0, 1, "2p8"),
+    ("64", [(0, 2000)], 0, 2, "1p8"),
+    # behind a context or beside single tokens, up to four times the units
+    ("64", [(700, 1200)], 0, 1, "1s8"), ("64", [(50, 1200)], 2, 1, "1s4"), ("64", [(50, 120)] * 14, 2, 1, "2s4"),
+    ("64", [(20, 1900)], 2, 1, "1p8"), ("64", [(20, 1650)], 2, 1, "1s8"), ("64", [(20, 1650)], 2, 2, "1s8"),
+    ("64", [(20, 1650)], 12, 1, "1s4"),
+    ("128", [(400, 1100)], 0, 1, "1s8"), ("128", [(50, 1100)], 2, 1, "1s4"), ("128", [(50, 1400)], 2, 1, "2s4"),
+    ("128", [(50, 1900)], 2, 1, "1p8"),
+    # and more
+    ("128", [(50, 2200)], 2, 1, "2p8"), ("128", [(50, 400)] * 6, 5, 1, "2p4"), ("64", [(50, 400)] * 6, 5, 2, "2p4")])
+def test_prefill_attention_takes_the_tiles_that_its_launch_has_room_for(ops, shape, portions, singles, planes, way):
+    """Every way that a launch without splits is cut in, on either side of its line, single tokens before, between and
+    behind the portions, against the general kernel."""
+    nh, nkv, d = dict(SHAPES_OF_PREFILL, **{"64 over 8": (64, 8, 128)})[shape]
+    variant, out, ref = prefill_beside(ops, nh, nkv, d, portions, singles, planes=planes, dv=64 if "/" in shape else d)
+    assert variant.startswith(f"prefill_attention_kernel<{d},{way[0]},") and f",{way[2]}>" in variant, variant
+    assert ("one tile a block" in variant) == (way[1] == "s"), variant
+    # both round p and the result to bfloat16: half of 2^-8 of sums of |v| <= 4.5, twice each
+    assert torch.allclose(out, ref, atol=2e-2, rtol=1e-2)
+
+
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_prefill_attention_of_a_single_token_with_more_pages_than_a_block_has_room_for(ops, nsplit):
+    """160 KB hold 40,960 page ids at most: a single token behind 41,000 pages is walked as portions are, beside others whose
+    blocks are of their own kind."""
+    _, out, ref = prefill_beside(ops, 8, 2, 64, [(50, 70), (0, 20)], 5, nsplit, far=41000 * 16 + 15)
+    assert torch.allclose(out, ref, atol=2e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("nh,nkv,d,whole,nsplit", [(8, 2, 128, 2100, 1), (8, 1, 64, 2100, 1), (32, 8, 128, 4200, 1),
                                                    (8, 2, 128, 2100, 7), (8, 1, 64, 2100, 2),
                                                    (16, 4, 128, 2100, 1), (16, 4, 128, 3100, 1),
