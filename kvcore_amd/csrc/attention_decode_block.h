@@ -81,12 +81,12 @@ inline size_t lds_total(int waves, int g, int d, int lds_pages) {
 template <int D>
 constexpr int max_waves() { return D > 128 ? 4 : kMaxWaves; }
 
-// whether a wave's registers hold two units of keys and values beside queries and results
-// (128 / 128 with two spills: 8 tokens of 512 keys 15.4 us unsplit, with one 13.4; 64 tokens of 1,024 keys 70 us and 57)
+// Whether a wave has two units of keys and values on their way.  Two bring 1 to 2% of a launch of few blocks of 64 / 64 (one
+// token of 100 keys 6.4 us, with one unit 6.5); their registers cost a place on the unit, or spill, wherever heads are wider and where
+// values are half as wide: one, two and one again, 64 requests of 40 keys, 16 heads of 128 / 64 16.1, 14.8 and 10.1 us; 128 requests of 8 keys, 3
+// of 224 / 112 9.1, 14.1 and 8.6, 16 of 96 20.0, 26.2 and 17.5, 12 of 64 / 32 9.9, 12.0 and 11.3 (units of 16 keys, of 32, and now).
 template <int D, int DV>
-constexpr bool two_units() {
-  return 2 * (D / 4 + DV / 4) + DV / 4 + D / 8 <= (max_waves<D>() == 4 ? 270 : 140);
-}
+constexpr bool two_units() { return D == 64 && DV >= 64; }
 
 // A barrier for what the block's waves exchange through LDS alone: __syncthreads would also wait for every load and
 // store in flight to global memory, here the first keys and values and the cache's new entries.
