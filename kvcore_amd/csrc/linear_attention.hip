@@ -557,15 +557,17 @@ __global__ __launch_bounds__(256) void max_gates_kernel(
 // The same for portions of prompts, whose log gates are there (log_gates_kernel): a block a request and 16 heads, a thread a
 // run of tokens of one head, 64 runs a request, so that a wave's loads and stores are four runs' 64 contiguous bytes (with a
 // wave a head and a lane a run every one of them touched 64 lines: two requests of 1,000 tokens, 16 heads 22.7 us, 14.3 this
-// way).  The runs' joins are made in the same order by one lane a head, so the bits are those of the kernel above.
+// way).  A block has threads for `heads` of them, a power of two: with 16 whatever nh is, one head left every wave four lanes (8,000
+// tokens 83.4 us, 53.9 so, with a wave a head 55.0; four heads 81.4, 58.4 and 130).  The runs' joins are made in the same order by one lane a head, so the bits are
+// those of the kernel above.
 constexpr int kRuns = 64, kRunHeads = 16;
 __global__ __launch_bounds__(kRuns * kRunHeads) void max_gates_runs_kernel(
     float* __restrict__ keep, float* __restrict__ take, float* __restrict__ m_out, float* __restrict__ m_state,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_req, const int32_t* __restrict__ q_start,
-    const int32_t* __restrict__ slots, int nh) {
+    const int32_t* __restrict__ slots, int nh, int heads) {
   __shared__ float a_s[kRuns][kRunHeads + 1], b_s[kRuns][kRunHeads + 1];
-  const int r = blockIdx.x, of = threadIdx.x / kRunHeads;
-  const int h = blockIdx.y * kRunHeads + threadIdx.x % kRunHeads;
+  const int r = blockIdx.x, of = threadIdx.x / heads, mine_h = threadIdx.x & (heads - 1);
+  const int h = blockIdx.y * heads + mine_h;
   const bool live = h < nh;
   const int b = q_start[r], e = q_start[r + 1];
   if (e <= b) return;
@@ -595,8 +597,8 @@ __global__ __launch_bounds__(kRuns * kRunHeads) void max_gates_runs_kernel(
       B = fmaxf(B + gf[i], gi[i]);
     }
   }
-  a_s[of][threadIdx.x % kRunHeads] = A;
-  b_s[of][threadIdx.x % kRunHeads] = B;
+  a_s[of][mine_h] = A;
+  b_s[of][mine_h] = B;
   __syncthreads();
   if (of == 0 && live) {
     float* ms = m_state + static_cast<int64_t>(slots[r]) * nh + h;
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(kRuns * kRunHeads) void max_gates_runs_kernel(
     *ms = m;
   }
   __syncthreads();
-  float mine = a_s[of][threadIdx.x % kRunHeads];
+  float mine = a_s[of][mine_h];
   for (int t0 = lo; t0 < hi; t0 += 8) {
     float gf[8], gi[8];
     fetch(t0, gf, gi);
@@ -688,8 +690,10 @@ extern "C" int kvc_max_gates(float* keep, float* take, float* m_out, const float
     const int64_t total = static_cast<int64_t>(T) * nh;
     hipLaunchKernelGGL(log_gates_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, S(stream),
                        keep, take, i_raw, i_stride, f_raw, f_stride, i_bias, f_bias, cap, total, nh);
-    hipLaunchKernelGGL(max_gates_runs_kernel, dim3(R, (nh + kRunHeads - 1) / kRunHeads), dim3(kRuns * kRunHeads), 0, S(stream),
-                       keep, take, m_out, m_state, positions, token_req, q_start, slots, nh);
+    int heads = 1;
+    while (heads < nh && heads < kRunHeads) heads *= 2;
+    hipLaunchKernelGGL(max_gates_runs_kernel, dim3(R, (nh + heads - 1) / heads), dim3(kRuns * heads), 0, S(stream),
+                       keep, take, m_out, m_state, positions, token_req, q_start, slots, nh, heads);
     return kvc_check_launch("kvc_max_gates");
   }
   // four waves a block, a wave a (request, head)

@@ -270,6 +270,27 @@ def test_running_maxima_of_portions(H, n):
         at += count
 
 
+@pytest.mark.parametrize("H", [1, 2, 3, 5, 8, 9, 18])
+def test_running_maxima_do_not_depend_on_the_heads_beside_them(H):
+    """Blocks of 1, 2, 4, 8 and 16 heads: every head's values are those that it has alone."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(H)
+    batch, T = batch_tensors([(2, 0, 3), (1, 5, 200), (0, 0, 700)])
+    raw = [torch.randn(T, H, generator=gen).to(DEV) * 3 for _ in range(2)]
+    bias = [torch.randn(H, generator=gen).to(DEV) for _ in range(2)]
+    state = torch.randn(3, H, generator=gen)
+
+    def run(h):
+        n = h.stop - h.start
+        out = [torch.full((T, n), float("nan"), device=DEV) for _ in range(3)] + [state[:, h].contiguous().to(DEV)]
+        ops.max_gates(*out[:3], raw[0][:, h], raw[1][:, h], bias[0][h], bias[1][h], 15.0, out[3], **batch)
+        return out
+
+    for whole, *alone in zip(run(slice(0, H)), *(run(slice(h, h + 1)) for h in range(H))):
+        assert torch.equal(whole, torch.cat(alone, 1)) and whole.isfinite().all()
+
+
 @pytest.mark.parametrize("H,d,dv,cap", [(3, 24, 40, 15.0), (1, 8, 1, 1.0), (2, 200, 80, 20.0), (4, 64, 64, 8.0),
                                         (2, 64, 127, 12.0), (6, 20, 16, 3.0)])
 def test_matrix_memory_whole_in_steps_and_beside_others(H, d, dv, cap):
