@@ -81,6 +81,21 @@ def test_norms_of_rows_read_eight_values_at_a_time(ops, H):
         close(out, (unit * w.double() + unit * b.double()) / 2, 1e-5)
 
 
+@pytest.mark.parametrize("H", [8, 1016, 1024, 1032, 2048, 2056, 3080, 8192])
+@pytest.mark.parametrize("delta", [True, False])
+def test_layer_norm_of_float32_rows_read_four_values_at_a_time(ops, H, delta):
+    """Widths around those at which a thread's second and further pieces begin, with and without rows to add and a bias."""
+    T = 3
+    res, more = rnd(T, H, seed=1) * 3 + 5.0, rnd(T, H, seed=2)
+    w, b = rnd(H, seed=3) + 1, rnd(H, seed=4)
+    total = res.double() + more.double() if delta else res.double()
+    r, out = res.to(DEV), torch.full((T, H), float("nan"), device=DEV)
+    ops.add_layernorm(out, r, more.to(DEV) if delta else None, w.to(DEV), b.to(DEV) if delta else None, 1e-5)
+    close(r, total, 1e-6)
+    # a mean of some 5 and deviations of some 3, each off by a few roundings of 2^-24
+    close(out, plain.layer_norm(total, w.double(), b.double() if delta else torch.zeros(H, dtype=torch.float64), 1e-5), 1e-5)
+
+
 @pytest.mark.parametrize("n", [1, 2, 3])
 def test_mean_of_branches_each_over_its_root_mean_square(ops, n):
     T, H = 5, 72
