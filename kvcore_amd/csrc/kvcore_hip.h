@@ -330,7 +330,8 @@ int kvc_head_rmsnorm_gate(void* out, int out_dtype, const float* o, const void* 
 // `gated` [E, 2N, K] (gate rows, then up rows) and the activation applied; a sorted row i reads
 // x row sorted[i] / in_div (in_div 0: row i itself) and writes out row i (out_sorted) or
 // sorted[i].  dtype is that of x and w.  packed: w is the copy kvc_pack_weight makes of the whole
-// stacked matrix (bfloat16, N a multiple of 16, K of 64).  act, of a product that is not gated: -1 none, 0 the
+// stacked matrix (bfloat16, N a multiple of 16, K of 64); 2: and most experts have one tile (for the choice of the kernel
+// alone).  act, of a product that is not gated: -1 none, 0 the
 // square of relu.  row_scale [pairs] (or null): multiplies a pair's sums before any activation, which is
 // what multiplying its input does.
 // bias [E] (or null) joins the logits.  score_fn 0: softmax over the experts, 1: sigmoid of each logit,

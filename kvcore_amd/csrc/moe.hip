@@ -695,7 +695,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   const int passes = K / 64;
   // blocks walk K round from places of their own, as in the kernel for more rows
   const int turn = passes > 0 ? (e * 5 + (n0 >> 4) * 3) % passes : 0;
-  // ONCE: this tile holds all rows of its expert, so nothing else reads the matrix (see `once8`)
+  // ONCE: this tile holds all rows of its expert, so nothing else reads the matrix (see `read8`)
   auto walk = [&](auto once) {
   constexpr bool ONCE = decltype(once)::value;
   bf16x8_t an[kStages][2], a2n[kStages][2], bn[kStages][2];
@@ -898,6 +898,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
       acc[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (GATED) acc2[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
+  auto walk = [&](auto once) {  // ONCE: loads marked as streaming ones (PACKED 2: see kvc_moe_gemm)
+  constexpr bool ONCE = decltype(once)::value;
   uint4 x_next[CH];
   bf16x8_t w_next[2][NF], w2_next[2][GATED ? NF : 1];
   // a pass's second half may lie beyond K (K a multiple of 32 only): the first half is then read
@@ -909,8 +911,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
       x_next[c] = *reinterpret_cast<const uint4*>(xp + k + 8 * c - (k + col < K ? 0 : 32));
     }
   };
-  auto walk = [&](auto once) {
-  constexpr bool ONCE = decltype(once)::value;
   auto fetch_w = [&](int k) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -923,10 +923,11 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
       }
     }
   };
-  auto stash = [&](int buffer) {
+  auto stash = [&](int buffer) {  // the choice word by word: of a whole piece it became a branch that waited for every load
 #pragma unroll
     for (int c = 0; c < CH; ++c)
-      *reinterpret_cast<uint4*>(x_s[buffer] + srow * KROW + 8 * (CH * spart + c)) = srow_ok ? x_next[c] : uint4{0u, 0u, 0u, 0u};
+      *reinterpret_cast<uint4*>(x_s[buffer] + srow * KROW + 8 * (CH * spart + c)) =
+          uint4{srow_ok ? x_next[c].x : 0u, srow_ok ? x_next[c].y : 0u, srow_ok ? x_next[c].z : 0u, srow_ok ? x_next[c].w : 0u};
   };
   // Every block walks K round from a place of its own (which its expert and columns decide, so a row's sums do
   // not depend on its tile): blocks that start at the same place of rows that lie a power of two apart would ask
@@ -986,8 +987,12 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
     }
   }
   };
-  if (PACKED && only_tile(tiles, at.tile, *num_tiles)) walk(std::integral_constant<bool, PACKED != 0>{});
-  else walk(std::false_type{});
+  if constexpr (PACKED == 2) {
+    if (only_tile(tiles, at.tile, *num_tiles)) walk(std::true_type{});
+    else walk(std::false_type{});
+  } else {
+    walk(std::false_type{});
+  }
   if (!wave_live) return;
   // lane holds row 16 r + li of the tile, columns n0 + 16 f + 4 lk + i
   store_tile<GATED, NF, NR, TO>(
@@ -1107,8 +1112,8 @@ __device__ __forceinline__ void wide_walk(const char* lds, const char* const (&x
   }
 }
 
-// As `place`, but a tile's column blocks all go to one die, tiles in turn, where experts have a tile each (up to a quarter
-// more tiles than that): the die's L2 holds the tile's rows for them, and no die reads every tile's.  The kernel is bound by
+// As `place`, but a tile's column blocks all go to one die, tiles in turn, where experts have a tile each (or up to a quarter
+// of all tiles are further ones): the die's L2 holds the tile's rows for them, and no die reads every tile's.  The kernel is bound by
 // what it draws through the fabric, and rows read by eight dies are a third of that.  Microseconds of the first and the second
 // product, packed, columns dealt to the dies and plain loads / tiles and streaming loads (weights are read once then):
 //   32 experts of 2048 x 2048, 245 rows 176 + 93 / 164 + 85, 138 rows 132 + 72 / 120 + 62, every other expert's twice as many
@@ -1545,6 +1550,11 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
                                                         : 8 * ((cols * max_tiles + 7) / 8);
       if (blocks > 0x7fffffff) return kvc_fail("kvc_moe_gemm: too many tiles for one launch");
       grid = dim3(static_cast<unsigned>(blocks));
+      // Streaming loads have a kernel of their own with a second walk for experts of more tiles, which takes some registers more
+      // (tiles of 64 rows 172, and so two blocks a unit for three): where most experts have more, all take the kernel without (4
+      // experts of 2048 x 2048, 200 rows each, down 31.0 us, 29.4 so, 28.9 before there were such loads).  Short walks are not faster with
+      // such loads (128 experts of 1024 x 384, 44 rows each, down 31.0 us with and 28.4 without).
+      const bool stream_tiles = packed == 2 && K >= 512;
 #define KVC_MOE_TILED(NR, PACKED)                                                                               \
   do {                                                                                                          \
     if (gated && out_dtype == 1) KVC_MOE_LAUNCH((moe_gemm_tiled_kernel<1, NR, bf16_t, PACKED>), bf16_t, bf16_t); \
@@ -1569,10 +1579,12 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
 #undef KVC_MOE_WIDE_OF
 #undef KVC_MOE_WIDE
       } else if (tile_rows == kBigTileRows) {
-        if (packed) KVC_MOE_TILED(8, 1);
+        if (stream_tiles) KVC_MOE_TILED(8, 2);
+        else if (packed) KVC_MOE_TILED(8, 1);
         else KVC_MOE_TILED(8, 0);
       } else {
-        if (packed) KVC_MOE_TILED(4, 1);
+        if (stream_tiles) KVC_MOE_TILED(4, 2);
+        else if (packed) KVC_MOE_TILED(4, 1);
         else KVC_MOE_TILED(4, 0);
       }
 #undef KVC_MOE_TILED

@@ -2158,6 +2158,8 @@ def moe_gemm(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, sorted_pairs: 
     max_tiles = min(tiles.shape[0], moe_max_tiles(pairs, experts, tile_rows))
     # the bfloat16 kernels read the packed twin of the experts' matrix where the model keeps one
     w_ptr, packed = (_streamed(w, N) if N % 16 == 0 and K % 64 == 0 else (_dev(w, "w"), 0))
+    if packed and pairs <= experts * tile_rows:
+        packed = 2  # most experts have one tile, whose loads may then be streaming ones
     _check(load().kvc_moe_gemm(out.data_ptr(), out.stride(0), _code(out, "out"), x.data_ptr(), x.stride(0),
                                w_ptr, _code(x, "x"), _dev(sorted_pairs, "sorted", torch.int32),
                                _dev(tiles, "tiles", torch.int32), _dev(num_tiles, "num_tiles", torch.int32),

@@ -668,6 +668,45 @@ def test_tiles_of_384_rows_dealt_to_the_dies_by_tile_and_by_column(counts, gated
     assert torch.equal(*outs) and outs[0].isfinite().all()
 
 
+@pytest.mark.parametrize("tile_rows", [64, 128])
+@pytest.mark.parametrize("gated,N,K", [(True, 176, 448), (False, 304, 512), (True, 2064, 576)])
+def test_tiles_of_experts_with_and_without_streaming_loads(tile_rows, gated, N, K):
+    """Sums shorter, as long and longer than those from which the experts' tiles are read by streaming loads; experts with
+    one tile in the mean (some of none, of two and of three among them) and with more, whose kernel has no such loads; from a
+    packed matrix and from rows, which give the same bits."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(N + K)
+    counts = [0, 1, tile_rows // 3, tile_rows, tile_rows + 1, 3, 2 * tile_rows + 5, tile_rows // 4]
+    i32 = dict(dtype=torch.int32, device=DEV)
+    for counts in (counts, [n + tile_rows for n in counts]):
+        E, T = len(counts), sum(counts)
+        choice = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=gen)]
+        x = torch.randn(T, K, generator=gen).to(torch.bfloat16)
+        w = (torch.randn(E * N * (2 if gated else 1), K, generator=gen) * K ** -0.5).to(torch.bfloat16)
+        sorted_pairs, num = torch.empty(T, **i32), torch.empty(1, **i32)
+        tiles = torch.empty(ops.moe_max_tiles(T, E, tile_rows), 3, **i32)
+        ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32).view(T, 1), E, tile_rows)
+        outs = []
+        for packed in (False, True):
+            wg = gpu(w, torch.bfloat16)
+            if packed:
+                ops.pack_weight(wg)
+            outs.append(torch.full((T, N), float("nan"), device=DEV))
+            ops.moe_gemm(outs[-1], gpu(x, torch.bfloat16), wg, sorted_pairs, tiles, num, pairs=T, experts=E, in_div=1,
+                         out_sorted=False, gated=gated, limit=1.2, alpha=1.702, tile_rows=tile_rows)
+        assert torch.equal(*outs)
+        per = w.double().view(E, -1, K)
+        want = torch.empty(T, N, dtype=torch.float64)
+        for e in range(E):
+            y = x[choice == e].double() @ per[e].T
+            if gated:
+                g, u = y[:, :N].clamp(max=1.2), y[:, N:].clamp(-1.2, 1.2)
+                y = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+            want[choice == e] = y
+        assert rel(outs[0], want) < 2e-6  # float32 sums of exact products
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,H,top", [(1, 8, 1), (3, 2048, 4), (67, 2056, 3), (2, 4096, 8), (5, 16384, 5), (5, 16392, 2), (4, 2047, 4)])
 def test_experts_sums_with_the_next_norm(T, H, top, dtype):
