@@ -25,7 +25,6 @@ __device__ __forceinline__ bf16x8_t read8(const void* p) {
   const u32x4_t* from = static_cast<const u32x4_t*>(p);
   return __builtin_bit_cast(bf16x8_t, ONCE ? __builtin_nontemporal_load(from) : *from);
 }
-__device__ __forceinline__ bf16x8_t once8(const void* p) { return read8<true>(p); }
 
 __device__ __forceinline__ bf16x8_t zero8() {
   bf16x8_t z;
