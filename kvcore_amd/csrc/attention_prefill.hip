@@ -839,7 +839,7 @@ int launch_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t*
   // behind 16,000 in eight 130 and 113; 4,096 of 128 / 64 behind 8,000 in two 339 and 295).
   // Over 850 launches with splits 1.03 of the best of all ways; one tile of 64 rows up to cu blocks whatever the splits
   // 1.05, and for some long contexts 1.5.
-  // (The rules know nothing of the values, so that one call over two planes and a call for each take the same tiles.)
+  // (On keys of 64 the rules know nothing of the values, so that one call over two planes and a call for each take the same tiles.)
   const int ones = g <= 16 ? singles : 0;  // single tokens that are blocks of their own kind
   const int T1 = T - ones, R1 = R - ones > 1 ? R - ones : 1;
   const int bq1 = 64 / g > 0 ? 64 / g : 1;

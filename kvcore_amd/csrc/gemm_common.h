@@ -17,7 +17,10 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // runs of 64 KB a wave are read at 6.6 TB/s with the mark and at 6.25 without (the caches need not make room for
 // them, and keep the rows).  Steps with them in the products of few and of some dozen rows, in the experts' tiles and on
 // keys and values of single tokens: 8B shape, 8 tokens 3,478 -> 3,271 us, 64 tokens 5,005 -> 4,835, 1B, one token 901 ->
-// 856.  Where several blocks share a matrix through the L2, or a load takes
+// 856.  A model's size does not matter much: matrices of up to 256 MB in all, which the memory-side cache holds, read one after
+// the other by nothing but these products take 1.04 to 1.2 times as long with the mark (2048 x 2048 in 128 MB, one row 4.05 -> 4.48 us),
+// but whole decode steps of six models with 60 to 200 MB 0.95 to 1.01 up to 16 tokens and 0.97 to 1.04 at 32 and 64.
+// Where several blocks share a matrix through the L2, or a load takes
 // part of a line whose rest comes with another, the mark costs more than it brings.
 template <bool ONCE>
 __device__ __forceinline__ bf16x8_t read8(const void* p) {
