@@ -61,7 +61,7 @@ using namespace kvc::decode;
 constexpr size_t kLdsLimit = 64 * 1024;
 constexpr int kMaxLdsPages = 1024;  // what the choice of waves per block leaves room for
 
-template <int D, int DV>
+template <int D, int DV, bool STREAM>
 __global__ __launch_bounds__(max_waves<D>() * 64) void decode_attention_kernel(const DecodeArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int t = blockIdx.x;
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(max_waves<D>() * 64) void decode_attention_kernel(c
     const int req = a.token_req[t];
     trow_idx = req < 0 ? -1 : a.slots[req];
   }
-  decode_block<D, DV, true>(a, t, blockIdx.y, blockIdx.z, __builtin_amdgcn_readfirstlane(trow_idx), lds);
+  decode_block<D, DV, STREAM>(a, t, blockIdx.y, blockIdx.z, __builtin_amdgcn_readfirstlane(trow_idx), lds);
 }
 
 // out[t, head, :] = sum_s w_s * part_o[s] / sum_s w_s * l_s with w_s = exp2(m_s - max m).
@@ -128,7 +128,7 @@ int decode_waves(int g, int d) {
 }
 
 template <int D, int DV>
-int launch_decode(DecodeArgs& args, int T, hipStream_t stream) {
+int launch_decode(DecodeArgs& args, int T, bool stream_keys, hipStream_t stream) {
   const int g = args.nh / args.nkv;
   // a split's range of pages always fits: the table's width cut into nsplit parts, and slack, as a split is whole
   // units of 32 keys (not more than two pages, also where a page is half a unit, as none behind the token's own counts)
@@ -141,8 +141,10 @@ int launch_decode(DecodeArgs& args, int T, hipStream_t stream) {
   if (lds_total(waves, g, D, args.lds_pages) > kLdsLimit)
     return kvc_fail("kvc_decode_attention: the block table is wider than kvc_decode_attention_max_table "
                     "allows for one split");
-  hipLaunchKernelGGL((decode_attention_kernel<D, DV>), dim3(T, args.nkv, args.nsplit), dim3(waves * 64),
-                     lds_total(waves, g, D, args.lds_pages), stream, args);
+  const dim3 grid(T, args.nkv, args.nsplit), block(waves * 64);
+  const size_t lds = lds_total(waves, g, D, args.lds_pages);
+  if (stream_keys) hipLaunchKernelGGL((decode_attention_kernel<D, DV, true>), grid, block, lds, stream, args);
+  else hipLaunchKernelGGL((decode_attention_kernel<D, DV, false>), grid, block, lds, stream, args);
   if (args.nsplit > 1)
     hipLaunchKernelGGL(decode_combine_kernel, dim3(T * args.nh), dim3((DV + 63) / 64 * 64), 0, stream,
                        args.out, args.part_o, args.part_ml, DV, args.nsplit, args.out_f32, args.gate);
@@ -192,11 +194,11 @@ extern "C" int kvc_decode_attention(void* out, void* part_o, void* part_ml, cons
                                     int nkv, int d, int dv, int page_size, int num_pages, float scale,
                                     int window, const float* slopes, int chunk, const float* sinks, float softcap,
                                     const void* gate, int64_t gate_stride, int values_are_keys,
-                                    int nsplit, int out_f32, kvc_stream stream) {
+                                    int nsplit, int longest, int out_f32, kvc_stream stream) {
   if (!kvc_decode_attention_supported(nh, nkv, d, dv, page_size, 1))
     return kvc_fail("kvc_decode_attention: unsupported shape (bfloat16, head size a multiple of 32 "
                     "up to 256, values as wide or half as wide, at most 16 query heads per kv head, page size a multiple of 16)");
-  if (T < 0 || nsplit < 1 || nsplit > kMaxSplits || nkv > 65535 || table_stride <= 0 || num_pages <= 0)
+  if (T < 0 || nsplit < 1 || nsplit > kMaxSplits || longest < 0 || nkv > 65535 || table_stride <= 0 || num_pages <= 0)
     return kvc_fail("kvc_decode_attention: bad sizes (at most 64 splits)");
   if (values_are_keys && dv != d) return kvc_fail("kvc_decode_attention: values that are the keys have the keys' size");
   if (softcap < 0.f || (softcap > 0.f && slopes != nullptr))
@@ -254,9 +256,16 @@ extern "C" int kvc_decode_attention(void* out, void* part_o, void* part_ml, cons
   args.sinks = sinks;
   args.nsplit = nsplit;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  kvc_note_variant(kVariantDecodeAttention, nsplit > 1 ? "decode_attention_kernel with splits" : "decode_attention_kernel");
+  // Streaming loads, but not where few blocks walk many keys each: they give a block some 10% fewer keys a second, which counts
+  // where blocks do not fill the chip.  Steps of 16 layers with them and without, one token, 8 heads over 1 of 128 in 32
+  // parts: 8,000 tokens 815 and 820 us, 32,000 972 and 938, 60,000 1,174 and 1,151, 120,000 1,576 and 1,480; 16 over 4 of
+  // 128 / 64 32,000 1,391 and 1,448, 60,000 1,577 and 1,558, 120,000 1,948 and 1,847; 256 blocks of 4,096 keys 1,438 and 1,532.
+  // (The kernel by itself, over and over on keys that the caches hold, is up to 12% faster without at any length.)
+  const bool stream_keys = static_cast<int64_t>(T) * nkv * nsplit >= kvc_device_compute_units() || longest / nsplit < 2048;
+  kvc_note_variant(kVariantDecodeAttention, !stream_keys ? "decode_attention_kernel, plain loads"
+                                            : nsplit > 1 ? "decode_attention_kernel with splits" : "decode_attention_kernel");
 #define KVC_DECODE(D_) \
-  case D_: return dv == d ? launch_decode<D_, D_>(args, T, s) : launch_decode<D_, D_ / 2>(args, T, s)
+  case D_: return dv == d ? launch_decode<D_, D_>(args, T, stream_keys, s) : launch_decode<D_, D_ / 2>(args, T, stream_keys, s)
   switch (d) {
     KVC_DECODE(32);
     KVC_DECODE(64);

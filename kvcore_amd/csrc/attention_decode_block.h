@@ -99,7 +99,8 @@ __device__ __forceinline__ void lds_barrier() {
 // One block's work: token t (its row of the block table: trow_idx), kv head hk, one split of the keys; lds: lds_total()
 // bytes of it, 16-byte aligned.  D: the size of a query and key head; DV: the size of a value head, at most D, or 2 D in two
 // planes.  STREAM: keys and values come by loads marked as streaming ones (`read8`).  They bring more where blocks fill
-// the chip, and take longer where a block walks many keys with few beside it (one token's 2,048 keys of 128, unsplit, 25 -> 32 us).
+// the chip, and take longer where a block walks many keys with few beside it (one token's 2,048 keys of 128, unsplit, 25 -> 32 us;
+// kvc_decode_attention has the line).
 template <int D, int DV, bool STREAM>
 __device__ __forceinline__ void decode_block(const DecodeArgs& a, int t, int hk, int split, int trow_idx, unsigned char* lds) {
   const int tid = threadIdx.x;

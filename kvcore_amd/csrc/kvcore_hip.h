@@ -403,7 +403,8 @@ int kvc_moe_combine_norm(void* x, int x_dtype, float* residual, const float* y, 
 // they are built.
 // slopes, sinks (float32 [nh] or null), chunk, softcap and gate (here bfloat16) as for kvc_paged_attention; the
 // kernel for portions (kvc_prefill_attention) takes them too (gate rows 8-byte aligned).  values_are_keys as
-// for kvc_qk_norm_rope_kv_write: rows of qkv end with the k heads, which are the values too.
+// for kvc_qk_norm_rope_kv_write: rows of qkv end with the k heads, which are the values too.  longest: how many keys the
+// launch is planned for (0: not known), for the choice of the kernel alone.
 int kvc_decode_attention_supported(int nh, int nkv, int d, int dv, int page_size, int dtype);
 int kvc_decode_attention_waves(int nh, int nkv, int d);
 int kvc_decode_attention_max_table(int nh, int nkv, int d);
@@ -415,7 +416,7 @@ int kvc_decode_attention(void* out, void* part_o, void* part_ml, const void* qkv
                          const float* k_gain, float norm_eps, int write_kv, int T,
                          int nh, int nkv, int d, int dv, int page_size, int num_pages, float scale,
                          int window, const float* slopes, int chunk, const float* sinks, float softcap,
-                         const void* gate, int64_t gate_stride, int values_are_keys, int nsplit, int out_f32,
+                         const void* gate, int64_t gate_stride, int values_are_keys, int nsplit, int longest, int out_f32,
                          kvc_stream stream);
 
 // The same attention for bfloat16 portions of prompts on the matrix cores: a block per

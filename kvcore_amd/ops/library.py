@@ -92,7 +92,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_ssm_scan": [P, P, L, P, L, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P],
         "kvc_gated_group_rmsnorm": [P, I, P, P, L, I, P, F, I, I, I, P],
         "kvc_decode_attention": [P, P, P, P, L, P, P, P, I, P, P, P, P, P, P, I, I, P, P, F, I, I, I, I, I, I,
-                                 I, I, F, I, P, I, P, F, P, L, I, I, I, P],
+                                 I, I, F, I, P, I, P, F, P, L, I, I, I, I, P],
         "kvc_decode_attention_waves": [I, I, I],
         "kvc_decode_attention_max_table": [I, I, I],
         "kvc_decode_attention_supported": [I, I, I, I, I, I],
@@ -744,7 +744,7 @@ def decode_attention(out: torch.Tensor, qkv: torch.Tensor, k_cache: torch.Tensor
                      sinks: torch.Tensor | None = None, dv: int | None = None,
                      q_gain: torch.Tensor | None = None, k_gain: torch.Tensor | None = None,
                      eps: float = 0.0, softcap: float = 0.0, gate: torch.Tensor | None = None,
-                     values_are_keys: bool = False) -> None:
+                     values_are_keys: bool = False, longest: int = 0) -> None:
     """bfloat16 attention of single tokens on the matrix cores (see the C header), with the
     rotation of each token's query and key and the write of its key and value into the cache
     (``write_kv``) in the same kernel; ``qkv`` is not changed.  With ``rot_dim = 0`` and
@@ -755,7 +755,8 @@ def decode_attention(out: torch.Tensor, qkv: torch.Tensor, k_cache: torch.Tensor
     it.  ``q_gain`` and ``k_gain`` (float32 ``[d]``): every query head, and the key head that is
     written, is divided by its root mean square (``eps`` inside the root) and multiplied by the
     gain before the rotation.  ``softcap`` and ``gate`` as for :func:`paged_attention`.
-    ``values_are_keys``: the rows of ``qkv`` hold no values; the keys as they are become the values."""
+    ``values_are_keys``: the rows of ``qkv`` hold no values; the keys as they are become the values.
+    ``longest``: how many keys the launch is planned for (0: not known), for the choice of the kernel alone."""
     T = out.shape[0]
     dv = d if dv is None else dv
     if out.shape != (T, nh * dv) or not out.is_contiguous() or out.dtype not in (torch.bfloat16, torch.float32):
@@ -796,7 +797,7 @@ def decode_attention(out: torch.Tensor, qkv: torch.Tensor, k_cache: torch.Tensor
         None if k_gain is None else _dev(k_gain, "k_gain", torch.float32), float(eps),
         int(bool(write_kv)), T, nh, nkv, d, dv, page_size, num_pages, float(scale),
         int(window), _slopes(slopes, nh), int(chunk), _sinks(sinks, nh), float(softcap),
-        *_gate(gate, T, nh * dv, torch.bfloat16), int(bool(values_are_keys)), int(nsplit),
+        *_gate(gate, T, nh * dv, torch.bfloat16), int(bool(values_are_keys)), int(nsplit), int(longest),
         int(out.dtype == torch.float32), _stream()),
         "kvc_decode_attention")
 

@@ -452,8 +452,8 @@ class PagedAttention(Mixer):
                                          torch.float32, reserve=most)
                 part_ml = ctx.buffers.get("attn_part_ml", T * self.num_heads * nsplit, 2, torch.float32,
                                           reserve=most)
-            ops.decode_attention(attn, qkv, k_cache, v_cache, nsplit=nsplit, part_o=part_o,
-                                 part_ml=part_ml, cos=cos, sin=sin, rot_dim=rot_dim,
+            ops.decode_attention(attn, qkv, k_cache, v_cache, nsplit=nsplit,
+                                 longest=min(reach or ctx.max_seq_len, ctx.max_seq_len), part_o=part_o, part_ml=part_ml, cos=cos, sin=sin, rot_dim=rot_dim,
                                  interleaved=interleaved, write_kv=call.write_cache and self.own_kv and not prepared,
                                  token_rows=ctx.token_rows, values_are_keys=self.keys_serve_as_values, **({} if prepared or not self.head_norm else dict(
                                      q_gain=q_gain, k_gain=k_gain, eps=self.qk_norm_eps)), **common)

@@ -1306,6 +1306,37 @@ def test_decode_attention_over_the_widest_tables(ops, nsplit, page):
                              scale=d ** -0.5, nsplit=nsplit, part_o=parts[0], part_ml=parts[1])
 
 
+@pytest.mark.parametrize("d,dv", [(32, 32), (64, 64), (64, 32), (96, 96), (128, 128), (128, 64), (224, 112), (256, 256)])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_decode_attention_takes_plain_loads_where_few_blocks_walk_many_keys(ops, d, dv, nsplit):
+    """Planned for 2,048 keys a block and more, and fewer blocks than compute units: another kernel, the same bits."""
+    dtype, nh, nkv, T, page = torch.bfloat16, 4, 2, 3, 16
+    lens = [1, 77, 700]
+    width = 700 // page + 1
+    i32 = dict(dtype=torch.int32, device=DEV)
+    kc, vc = rnd(T * width + 1, nkv, page, d, dtype=dtype, seed=1), rnd(T * width + 1, nkv, dv, page, dtype=dtype, seed=2)
+    qkv = rnd(T, (nh + nkv) * d + nkv * dv, dtype=dtype, seed=3)
+    table = (torch.randperm(T * width, device=DEV) + 1).view(T, width).to(torch.int32)
+    positions, ids = torch.tensor([n - 1 for n in lens], **i32), torch.arange(T, **i32)
+    angle = rnd(T, d // 2, seed=4).float()
+    outs = []
+    for longest, plain in ((0, False), (2048 * nsplit - 1, False), (2048 * nsplit, True)):
+        out = torch.full((T, nh * dv), float("nan"), device=DEV)
+        parts = torch.empty(T * nh * nsplit * dv, device=DEV), torch.empty(T * nh * nsplit * 2, device=DEV)
+        ops.decode_attention(out, qkv, kc, vc, table=table, positions=positions, token_req=ids, slots=ids, nh=nh, nkv=nkv, d=d,
+                             dv=dv, scale=d ** -0.5, nsplit=nsplit, part_o=parts[0], part_ml=parts[1], cos=angle.cos(),
+                             sin=angle.sin(), rot_dim=d, write_kv=True, longest=longest)
+        assert ops.last_variant("decode_attention").endswith("plain loads") == plain
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]) and outs[0].isfinite().all()
+    many = ops.compute_units() // nkv // nsplit + 1  # blocks for every unit
+    out, ids = torch.empty(many, nh * dv, device=DEV), torch.zeros(many, **i32)
+    parts = torch.empty(many * nh * nsplit * dv, device=DEV), torch.empty(many * nh * nsplit * 2, device=DEV)
+    ops.decode_attention(out, qkv[:1].repeat(many, 1), kc, vc, table=table, positions=ids, token_req=ids, slots=ids, nh=nh, nkv=nkv,
+                         d=d, dv=dv, scale=d ** -0.5, nsplit=nsplit, part_o=parts[0], part_ml=parts[1], longest=100000)
+    assert not ops.last_variant("decode_attention").endswith("plain loads")
+
+
 @pytest.mark.parametrize("nsplit", [1, 5])
 def test_decode_attention_far_key_and_window(ops, nsplit):
     dtype = torch.bfloat16
