@@ -333,7 +333,12 @@ int kvc_head_rmsnorm_gate(void* out, int out_dtype, const float* o, const void* 
 // stacked matrix (bfloat16, N a multiple of 16, K of 64); 2: and most experts have one tile (for the choice of the kernel
 // alone).  act, of a product that is not gated: -1 none, 0 the
 // square of relu.  row_scale [pairs] (or null): multiplies a pair's sums before any activation, which is
-// what multiplying its input does.
+// what multiplying its input does (not beside w_shared).
+// An expert that every token runs, of the others' sizes, joins the launches: with shared_rows (0: none) kvc_moe_align and
+// kvc_moe_router_spread list its tiles first (room for ceil(shared_rows / tile_rows) more) and behind `pairs` its pairs pairs + t, row t of x
+// where in_div > 0; its matrix is w_shared (stored as w is), shared_first is `pairs`, and
+// shared_limit is its limit.  kvc_moe_shared_tile_rows says whether that is the faster for T tokens, and in tiles of how many rows
+// (0: it is not), where the routed experts alone would take tile_rows.
 // bias [E] (or null) joins the logits.  score_fn 0: softmax over the experts, 1: sigmoid of each logit,
 // 2: the logit itself, the weights then being the softmax over the chosen logits.  correction [E] (or
 // null) is added to the scores for the choice alone.  group_best 1 or 2: a group is worth its best choice score, or
@@ -359,18 +364,19 @@ int kvc_moe_router(int32_t* choice, float* weight, const void* x, int64_t x_stri
 int kvc_moe_router_spread_tokens(void);
 int kvc_moe_router_spread_floats(int T, int E);
 int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32_t* tiles, int32_t* num_tiles,
-                       int max_tiles, int tile_rows, float* parts, int64_t parts_floats, const void* x,
+                       int max_tiles, int tile_rows, int shared_rows, float* parts, int64_t parts_floats, const void* x,
                        int64_t x_stride, int x_dtype, const float* router, float* gate, int T, int H, int E,
                        int top, int groups, int keep, int score_fn, const float* bias, const float* correction,
                        int group_best, int renormalize, float weight_scale, kvc_stream stream);
 int kvc_moe_max_tiles(int pairs, int E, int tile_rows);
+int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows);
 int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
-                  int pairs, int E, int max_tiles, int tile_rows, kvc_stream stream);
+                  int pairs, int E, int max_tiles, int tile_rows, int shared_rows, kvc_stream stream);
 int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const void* x, int64_t x_stride,
                  const void* w, int dtype, const int32_t* sorted, const int32_t* tiles,
                  const int32_t* num_tiles, int max_tiles, int tile_rows, int N, int K, int in_div, int out_sorted,
-                 int gated, float limit, float alpha, float up_shift, int act, const float* row_scale, int packed,
-                 kvc_stream stream);
+                 int gated, float limit, float alpha, float up_shift, int act, const float* row_scale, const void* w_shared,
+                 int shared_first, float shared_limit, int packed, kvc_stream stream);
 // out[t] = sum_c weight[t, c] * y[t * top + c] (weight null: ones) + add0[t] + add1[t] (either may be null; add0 of
 // dtype add0_dtype, add1 float32), float32.  add1_gate [T] (or null): add1[t] is multiplied by it.
 // accumulate: the sum is added into out instead of stored.

@@ -97,6 +97,15 @@ struct RouteRule {
   float weight_scale;
 };
 
+// The expert that every token runs, multiplied in the routed experts' launches: its tiles name kSharedExpert, its pair of
+// token t is first_pair + t, and its matrix (of their sizes and their order of storage) lies at w.
+constexpr int kSharedExpert = -1;
+struct SharedExpert {
+  const void* w;
+  int first_pair;
+  float limit;
+};
+
 // One token's choice by one wave: z [E] logits (global or LDS), sc [E], pk [E] and gs [groups] LDS
 // scratch (sc may be z itself).
 __device__ __forceinline__ void route_one(int32_t* __restrict__ choice, float* __restrict__ weight, const float* z,
@@ -423,7 +432,7 @@ __global__ __launch_bounds__(kRouterWaves * 64) void moe_router_kernel(
 // One block.  counts -> offsets and tiles (a thread an expert) -> sorted pairs.  `ilds`: [3 E] in LDS.
 __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
                                             int32_t* __restrict__ num_tiles, const int32_t* choice, int pairs, int E,
-                                            int max_tiles, int tile_rows, int32_t* ilds) {
+                                            int max_tiles, int tile_rows, int shared_rows, int32_t* ilds) {
   int32_t* count = ilds;           // [E]
   int32_t* offset = count + E;     // [E]
   int32_t* cursor = offset + E;    // [E]; at first the experts' numbers of tiles
@@ -441,6 +450,15 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
     const int tiles_of = wide ? (n + kWideTileRows - 1) / kWideTileRows : (n + tile_rows - 1) >> shift;
     return tiles_of < 2 ? tile_rows : ((n + tiles_of - 1) / tiles_of + 15) & ~15;
   };
+  // the shared expert's tiles come first (its rows fill them), its pairs behind the others
+  const int shared_each = rows_each(shared_rows), shared_tiles = (shared_rows + shared_each - 1) / shared_each;
+  for (int i = threadIdx.x; i < shared_tiles; i += blockDim.x) {
+    const int r = i * shared_each;
+    tiles[3 * i] = kSharedExpert;
+    tiles[3 * i + 1] = pairs + r;
+    tiles[3 * i + 2] = shared_rows - r < shared_each ? shared_rows - r : shared_each;
+  }
+  for (int i = threadIdx.x; i < shared_rows; i += blockDim.x) sorted[pairs + i] = pairs + i;
   auto list = [&](int e, int n, int each, int at, int nt) {
     offset[e] = at;
     for (int r = 0; r < n && nt < max_tiles; r += each, ++nt) {
@@ -463,6 +481,7 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
           nt += pt;
         }
       }
+      nt += shared_tiles;
       if (e == E - 1) *num_tiles = nt < max_tiles ? nt : max_tiles;
       nt -= mine;
       if (wide) {
@@ -471,7 +490,7 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
         // ones.  Smaller tiles fetch weights in the experts' order (8 rows an expert, 32 gated experts of 2048 x 2048 in
         // tiles of 64 rows: 95.3 us, in the other order 98.3).
         const int key = (n < each ? n : each) * kWave + kWave - 1 - e;
-        nt = 0;
+        nt = shared_tiles;
 #pragma unroll
         for (int p = 0; p < kWave; ++p) {  // lanes beyond E have no tiles
           if (p == kWave / 2 && E <= kWave / 2) break;  // scalar
@@ -488,7 +507,7 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
     }
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      int at = 0, nt = 0;
+      int at = 0, nt = shared_tiles;
       for (int p = 0; p < e; ++p) {
         at += count[p];
         nt += cursor[p];
@@ -513,9 +532,9 @@ __device__ __forceinline__ void align_pairs(int32_t* __restrict__ sorted, int32_
 __global__ __launch_bounds__(1024) void moe_align_kernel(int32_t* __restrict__ sorted, int32_t* __restrict__ tiles,
                                                          int32_t* __restrict__ num_tiles,
                                                          const int32_t* __restrict__ choice, int pairs, int E,
-                                                         int max_tiles, int tile_rows) {
+                                                         int max_tiles, int tile_rows, int shared_rows) {
   extern __shared__ int32_t ilds[];
-  align_pairs(sorted, tiles, num_tiles, choice, pairs, E, max_tiles, tile_rows, ilds);
+  align_pairs(sorted, tiles, num_tiles, choice, pairs, E, max_tiles, tile_rows, shared_rows, ilds);
 }
 
 // The router spread over the chip (at most kRouterSpread tokens and 64 experts), with the arrangement of its pairs.
@@ -631,7 +650,7 @@ __global__ __launch_bounds__(256) void moe_choose_kernel(int32_t* __restrict__ c
 __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
     int32_t* __restrict__ choice, float* __restrict__ weight, float* __restrict__ gate, int32_t* __restrict__ sorted,
     int32_t* __restrict__ tiles, int32_t* __restrict__ num_tiles, const float* __restrict__ parts, int T_, int E,
-    int max_tiles, int tile_rows, RouteRule rule) {
+    int max_tiles, int tile_rows, int shared_rows, RouteRule rule) {
   extern __shared__ int32_t ilds[];  // [T top] choices, then [3 E]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
   if (wave < T_)  // scalar
@@ -640,7 +659,7 @@ __global__ __launch_bounds__(1024) void moe_choose_align_kernel(
   __syncthreads();
   const int pairs = T_ * rule.top;
   for (int i = threadIdx.x; i < pairs; i += blockDim.x) choice[i] = ilds[i];
-  align_pairs(sorted, tiles, num_tiles, ilds, pairs, E, max_tiles, tile_rows, ilds + pairs);
+  align_pairs(sorted, tiles, num_tiles, ilds, pairs, E, max_tiles, tile_rows, shared_rows, ilds + pairs);
 }
 
 // bfloat16, few rows: a wave takes one tile of up to 16 rows and 16 columns (gated: of gate and of up).  WK 4: the
@@ -662,12 +681,22 @@ __device__ __forceinline__ bool only_tile(const int32_t* tiles, int tile, int nu
   const int e = tiles[3 * tile];
   return (tile == 0 || tiles[3 * tile - 3] != e) && (tile + 1 >= num_tiles || tiles[3 * tile + 3] != e);
 }
+// Where a pair's input row lies (in_div 0: the products of its own place), its expert's matrix, and what the expert adds to
+// the place at which a block begins its walk along K.
+__device__ __forceinline__ int64_t input_row(int pair, int place, int in_div, int e, const SharedExpert& shared) {
+  return in_div == 0 ? place : e == kSharedExpert ? pair - shared.first_pair : pair / in_div;
+}
+template <typename T>
+__device__ __forceinline__ const T* expert_weights(const T* w, int e, int64_t elems, const SharedExpert& shared) {
+  return e == kSharedExpert ? static_cast<const T*>(shared.w) : w + e * elems;
+}
+__device__ __forceinline__ int turn_of(int e) { return e == kSharedExpert ? 0 : e * 5; }
 template <int GATED, typename TO, int PACKED, int WK>
 __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
-    int act, const float* __restrict__ row_scale) {
+    int act, const float* __restrict__ row_scale, SharedExpert shared) {
   constexpr int kStages = WK == 1 ? 2 : 4;
   const int tile = blockIdx.z * gridDim.y + blockIdx.y;  // more tiles than a grid's second dimension takes
   if (tile >= *num_tiles) return;
@@ -680,7 +709,7 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   // B operand: token row li of the tile; A operand: the expert's row n0 + li
   const bool row_ok = li < nr;
   const int pair = sorted[r0 + (row_ok ? li : 0)];  // a row that is not there reads the tile's first and is dropped
-  const int64_t in_row = in_div > 0 ? pair / in_div : r0 + (row_ok ? li : 0);
+  const int64_t in_row = input_row(pair, r0 + (row_ok ? li : 0), in_div, e, shared);
   // PACKED: w is the copy that `kvc_pack_weight` makes, tiles of 16 rows x 32 values of K in one
   // piece of 1 KB each, so a wave's load of an operand is one contiguous kilobyte instead of 128 bytes
   // from each of 16 rows that lie 2 K bytes apart (which meet in the same memory channels); the lanes
@@ -688,13 +717,14 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   const bf16_t* xr = x + in_row * x_stride + (PACKED ? 8 : 16) * lk;
   const int wrow = n0 + li < N ? n0 + li : N - 1;
   const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
-  const bf16_t* wr = PACKED ? w + ((static_cast<int64_t>(e) * rows_per_expert + n0) >> 4) * (K / 32) * 512 + li * 32 + lk * 8
-                            : w + (static_cast<int64_t>(e) * rows_per_expert + wrow) * K + 16 * lk;
+  const bf16_t* we = expert_weights(w, e, rows_per_expert * K, shared);
+  const bf16_t* wr = PACKED ? we + static_cast<int64_t>(n0 >> 4) * (K / 32) * 512 + li * 32 + lk * 8
+                            : we + static_cast<int64_t>(wrow) * K + 16 * lk;
   const bf16_t* wr2 = wr + static_cast<int64_t>(N) * K;  // the up rows follow the gate rows (in either order of storage)
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
   const int passes = K / 64;
   // blocks walk K round from places of their own, as in the kernel for more rows
-  const int turn = passes > 0 ? (e * 5 + (n0 >> 4) * 3) % passes : 0;
+  const int turn = passes > 0 ? (turn_of(e) + (n0 >> 4) * 3) % passes : 0;
   // ONCE: this tile holds all rows of its expert, so nothing else reads the matrix (see `read8`)
   auto walk = [&](auto once) {
   constexpr bool ONCE = decltype(once)::value;
@@ -773,7 +803,8 @@ __global__ __launch_bounds__(256) void moe_gemm_few_kernel(
   const float scale = row_scale != nullptr ? row_scale[pair] : 1.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    acc[i] = GATED ? clamped_glu(acc[i] * scale, acc2[i] * scale, limit, alpha, shift) : plain_act(acc[i] * scale, act);
+    acc[i] = GATED ? clamped_glu(acc[i] * scale, acc2[i] * scale, e == kSharedExpert ? shared.limit : limit, alpha, shift)
+                   : plain_act(acc[i] * scale, act);
   const int64_t out_row = out_sorted ? r0 + li : pair;
   const int nf = n0 + 4 * lk;
   if (nf < N) store4<TO>(out + out_row * out_stride + nf, acc, N - nf);
@@ -859,7 +890,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
-    int act, const float* __restrict__ row_scale) {
+    int act, const float* __restrict__ row_scale, SharedExpert shared) {
   constexpr int NF = GATED ? 2 : 4;   // column blocks of 16 a wave
   constexpr int KC = 64;              // values of K a pass (two matrix instructions deep)
   constexpr int KROW = KC + 8;        // a row's chunk in LDS, padded against bank conflicts
@@ -877,17 +908,18 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
   const int srow = threadIdx.x / (8 / CH), spart = threadIdx.x % (8 / CH);
   const bool srow_ok = srow < nr;
   const int srow_safe = srow_ok ? srow : 0;  // a row that is not there reads the tile's first, and is set to zero
-  const int64_t in_row = in_div > 0 ? sorted[r0 + srow_safe] / in_div : r0 + srow_safe;
+  const int64_t in_row = in_div > 0 ? input_row(sorted[r0 + srow_safe], 0, in_div, e, shared) : r0 + srow_safe;
   const bf16_t* xp = x + in_row * x_stride + 8 * CH * spart;
   const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
+  const bf16_t* we = expert_weights(w, e, rows_per_expert * K, shared);
   const bf16_t* wp[NF];
 #pragma unroll
   for (int f = 0; f < NF; ++f) {
     const int wrow = n0 + 16 * f + li < N ? n0 + 16 * f + li : N - 1;
     // PACKED (N a multiple of 16): the copy in pieces of 16 rows x 32 values, one contiguous kilobyte a load
     const int ntile = n0 + 16 * f < N ? n0 + 16 * f : N - 16;
-    wp[f] = PACKED ? w + ((static_cast<int64_t>(e) * rows_per_expert + ntile) >> 4) * (K / 32) * 512 + li * 32 + lk * 8
-                   : w + (static_cast<int64_t>(e) * rows_per_expert + wrow) * K + 8 * lk;
+    wp[f] = PACKED ? we + static_cast<int64_t>(ntile >> 4) * (K / 32) * 512 + li * 32 + lk * 8
+                   : we + static_cast<int64_t>(wrow) * K + 8 * lk;
   }
   const int64_t up_off = static_cast<int64_t>(N) * K;
   f32x4_t acc[NF][NR], acc2[GATED ? NF : 1][NR];
@@ -932,7 +964,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
   // Every block walks K round from a place of its own (which its expert and columns decide, so a row's sums do
   // not depend on its tile): blocks that start at the same place of rows that lie a power of two apart would ask
   // the same memory channels at the same time.
-  const int turn = K % KC == 0 ? (e * 5 + at.col * 11) % (K / KC) * KC : 0;
+  const int turn = K % KC == 0 ? (turn_of(e) + at.col * 11) % (K / KC) * KC : 0;
   auto round = [&](int k) { return k + turn < K ? k + turn : k + turn - K; };
   fetch_x(round(0));
   fetch_w(round(0));
@@ -996,8 +1028,9 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_tiled_kernel(
   if (!wave_live) return;
   // lane holds row 16 r + li of the tile, columns n0 + 16 f + 4 lk + i
   store_tile<GATED, NF, NR, TO>(
-      out, out_stride, [&](int r) { return 16 * r + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale, limit, alpha, shift, act,
-      [&](int f, int r) { return acc[f][r]; }, [&](int f, int r) { return acc2[GATED ? f : 0][r]; });
+      out, out_stride, [&](int r) { return 16 * r + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale,
+      e == kSharedExpert ? shared.limit : limit, alpha, shift, act, [&](int f, int r) { return acc[f][r]; },
+      [&](int f, int r) { return acc2[GATED ? f : 0][r]; });
 }
 
 // bfloat16, tiles of up to 384 rows: a block of eight waves takes the tile's rows and 256 columns (gated: 128 of gate and
@@ -1140,7 +1173,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
     TO* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ x, int64_t x_stride,
     const bf16_t* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
-    int act, const float* __restrict__ row_scale) {
+    int act, const float* __restrict__ row_scale, SharedExpert shared) {
   constexpr int COLS = GATED ? 128 : 256;  // a block's columns of the result
   __shared__ __attribute__((aligned(1024))) char lds[kWideLds];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
@@ -1154,23 +1187,24 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
   // what the lane fetches of row blocks wave, wave + 8 and wave + 16 and of column blocks
   // wave and wave + 8 (gated: the second is up's)
   const int part = 16 * ((lane & 3) ^ ((lane >> 3) & 3));
+  const bf16_t* we = expert_weights(w, e, rows_per_expert * K, shared);
   const char *xp[3], *wp[2];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
     const int row = 16 * (wave + 8 * j) + (lane >> 2);
     const int safe = row < nr ? row : 0;  // a row that is not there reads the tile's first and is dropped
-    const int64_t in_row = in_div > 0 ? sorted[r0 + safe] / in_div : r0 + safe;
+    const int64_t in_row = in_div > 0 ? input_row(sorted[r0 + safe], 0, in_div, e, shared) : r0 + safe;
     xp[j] = reinterpret_cast<const char*>(x + in_row * x_stride) + part;
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
-    const int64_t first = static_cast<int64_t>(e) * rows_per_expert + (GATED && j == 1 ? N : 0);
+    const int64_t first = GATED && j == 1 ? N : 0;
     if (PACKED) {  // pieces of 16 rows x 32 values
       const int n = c0 + 16 * (GATED ? wave : wave + 8 * j);
-      wp[j] = reinterpret_cast<const char*>(w) + ((first + (n < N ? n : N - 16)) >> 4) * (K / 32) * 1024 + 64 * (lane >> 2) + part;
+      wp[j] = reinterpret_cast<const char*>(we) + ((first + (n < N ? n : N - 16)) >> 4) * (K / 32) * 1024 + 64 * (lane >> 2) + part;
     } else {
       const int n = c0 + 16 * (GATED ? wave : wave + 8 * j) + (lane >> 2);
-      wp[j] = reinterpret_cast<const char*>(w + (first + (n < N ? n : N - 1)) * K) + part;
+      wp[j] = reinterpret_cast<const char*>(we + (first + (n < N ? n : N - 1)) * K) + part;
     }
   }
   int wt[4];  // the wave's column blocks, in bytes
@@ -1182,7 +1216,7 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
 #pragma unroll
     for (int r = 0; r < kWideBlocks; ++r) acc[f][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // every block walks K round from a place of its own, as in the kernel for tiles of 128 rows, and from the same one
-  const int turn = (e * 5 + at.col * 11) % (K / 64) * 2;
+  const int turn = (turn_of(e) + at.col * 11) % (K / 64) * 2;
   // an expert of more tiles than one has some 200 rows in each
   constexpr bool kStream = PACKED != 0;
   const bool alone = kStream && only_tile(tiles, at.tile, *num_tiles);
@@ -1203,8 +1237,9 @@ __global__ __launch_bounds__(512) void moe_gemm_wide_kernel(
   if (n0 >= N) return;  // the whole wave
   // lane holds row 16 (2 r + wr) + li of the tile, columns n0 + 16 f + 4 lk + i
   store_tile<GATED, GATED ? 2 : 4, kWideBlocks, TO>(
-      out, out_stride, [&](int r) { return 16 * (2 * r + wr) + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale, limit, alpha,
-      shift, act, [&](int f, int r) { return acc[f][r]; }, [&](int f, int r) { return acc[GATED ? f + 2 : 0][r]; });
+      out, out_stride, [&](int r) { return 16 * (2 * r + wr) + li; }, nr, n0 + 4 * lk, N, r0, sorted, out_sorted, row_scale,
+      e == kSharedExpert ? shared.limit : limit, alpha, shift, act, [&](int f, int r) { return acc[f][r]; },
+      [&](int f, int r) { return acc[GATED ? f + 2 : 0][r]; });
 }
 
 // Any operand type and any sizes: a thread a (row, column) pair of the tile, float32 sums in index
@@ -1214,19 +1249,19 @@ __global__ __launch_bounds__(256) void moe_gemm_plain_kernel(
     TO* __restrict__ out, int64_t out_stride, const TI* __restrict__ x, int64_t x_stride,
     const TI* __restrict__ w, const int32_t* __restrict__ sorted, const int32_t* __restrict__ tiles,
     const int32_t* __restrict__ num_tiles, int N, int K, int in_div, int out_sorted, float limit, float alpha, float shift,
-    int act, const float* __restrict__ row_scale) {
+    int act, const float* __restrict__ row_scale, SharedExpert shared) {
   const int tile = blockIdx.x;
   if (tile >= *num_tiles) return;
   const int e = tiles[3 * tile], r0 = tiles[3 * tile + 1], nr = tiles[3 * tile + 2];
   const int li = threadIdx.x & 15, col = threadIdx.x >> 4;  // 16 rows x 16 columns a pass
   if (li >= nr) return;
   const int pair = sorted[r0 + li];
-  const int64_t in_row = in_div > 0 ? pair / in_div : r0 + li;
+  const int64_t in_row = input_row(pair, r0 + li, in_div, e, shared);
   const TI* xr = x + in_row * x_stride;
   const int64_t rows_per_expert = GATED ? 2 * static_cast<int64_t>(N) : N;
   const int64_t out_row = out_sorted ? r0 + li : pair;
   for (int n = blockIdx.y * 64 + col; n < N && n < (blockIdx.y + 1) * 64; n += 16) {
-    const TI* wr = w + (static_cast<int64_t>(e) * rows_per_expert + n) * K;
+    const TI* wr = expert_weights(w, e, rows_per_expert * K, shared) + static_cast<int64_t>(n) * K;
     float acc = 0.f, acc2 = 0.f;
     for (int k = 0; k < K; ++k) {
       const float xv = to_float(xr[k]);
@@ -1235,7 +1270,8 @@ __global__ __launch_bounds__(256) void moe_gemm_plain_kernel(
     }
     const float scale = row_scale != nullptr ? row_scale[pair] : 1.f;
     out[out_row * out_stride + n] = from_float<TO>(
-        GATED ? clamped_glu(acc * scale, acc2 * scale, limit, alpha, shift) : plain_act(acc * scale, act));
+        GATED ? clamped_glu(acc * scale, acc2 * scale, e == kSharedExpert ? shared.limit : limit, alpha, shift)
+              : plain_act(acc * scale, act));
   }
 }
 
@@ -1388,11 +1424,14 @@ extern "C" int kvc_moe_router(int32_t* choice, float* weight, const void* x, int
   return kvc_check_launch("kvc_moe_router");
 }
 
+// how many tiles the rows of an expert that every token runs take at most
+static int shared_tiles(int rows, int tile_rows) { return (rows + tile_rows - 1) / tile_rows; }
+
 extern "C" int kvc_moe_router_spread_tokens(void) { return kRouterSpread; }
 extern "C" int kvc_moe_router_spread_floats(int T, int E) { return kRouterWaves * T * router_part_row(E); }
 
 extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32_t* tiles, int32_t* num_tiles,
-                                  int max_tiles, int tile_rows, float* parts, int64_t parts_floats, const void* x,
+                                  int max_tiles, int tile_rows, int shared_rows, float* parts, int64_t parts_floats, const void* x,
                                   int64_t x_stride, int x_dtype, const float* router, float* gate, int T, int H, int E,
                                   int top, int groups, int keep, int score_fn, const float* bias, const float* correction,
                                   int group_best, int renormalize, float weight_scale, kvc_stream stream) {
@@ -1404,7 +1443,7 @@ extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* so
     return kvc_fail("kvc_moe_router_spread: scores by softmax (0), sigmoid (1) or logit (2); a group is worth its best 1 or 2");
   if (!known_tile_rows(tile_rows))
     return kvc_fail("kvc_moe_router_spread: tiles of 16, 64, 128 or 384 rows");
-  if (max_tiles < kvc_moe_max_tiles(T * top, E, tile_rows))
+  if (shared_rows < 0 || max_tiles < kvc_moe_max_tiles(T * top, E, tile_rows) + shared_tiles(shared_rows, tile_rows))
     return kvc_fail("kvc_moe_router_spread: room for fewer tiles than the routing may need");
   if (parts_floats < kvc_moe_router_spread_floats(T, E) || (reinterpret_cast<uintptr_t>(parts) & 15) != 0)
     return kvc_fail("kvc_moe_router_spread: the workspace is too small or not 16-byte aligned");
@@ -1425,11 +1464,11 @@ extern "C" int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* so
 #undef KVC_PARTS
   if (T <= kChooseInOne) {
     hipLaunchKernelGGL(moe_choose_align_kernel, dim3(1), dim3(1024), sizeof(int32_t) * (T * top + 3 * E), S(stream),
-                       choice, weight, gate, sorted, tiles, num_tiles, parts, T, E, max_tiles, tile_rows, rule);
+                       choice, weight, gate, sorted, tiles, num_tiles, parts, T, E, max_tiles, tile_rows, shared_rows, rule);
     return kvc_check_launch("kvc_moe_router_spread");
   }
   hipLaunchKernelGGL(moe_choose_kernel, dim3((T + 3) / 4), dim3(256), 0, S(stream), choice, weight, gate, parts, T, E, rule);
-  return kvc_moe_align(sorted, tiles, num_tiles, choice, T * top, E, max_tiles, tile_rows, stream);
+  return kvc_moe_align(sorted, tiles, num_tiles, choice, T * top, E, max_tiles, tile_rows, shared_rows, stream);
 }
 
 extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
@@ -1456,22 +1495,36 @@ extern "C" int kvc_moe_max_tiles(int pairs, int E, int tile_rows) {
 // 64 rows: the second of two blocks a unit keeps the matrix cores busy): 32 experts of 2048 x 2048, 64 rows each,
 // 188 / 165 us, 16 experts of 1024 x 1024 41 / 53.  From 104 to 150 rows many an expert has a few more than 128, and two
 // tiles of half the size cost more than smaller ones: 128 rows 227 us in tiles of 64, 249 in tiles of 128.
-extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
-  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0) return kTileRows;
-  const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
-  const double used = E * -expm1(-each);  // experts with rows
-  const int first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, down_cols = (H + 255) / 256;
+struct TileEstimate {
+  double each, used, mb, mid;  // rows an expert, experts with rows, megabytes of an expert, us in tiles of 64
+  int first_cols, down_cols;
+};
+static TileEstimate estimate_tiles(int pairs, int E, int H, int I, int gated) {
+  TileEstimate t;
+  const double units = kvc_device_compute_units();
+  t.each = static_cast<double>(pairs) / E;
+  t.used = E * -expm1(-t.each);
+  t.first_cols = gated ? (I + 127) / 128 : (I + 255) / 256, t.down_cols = (H + 255) / 256;
   const double down_mb = 2e-6 * H * I, first_mb = gated ? 2 * down_mb : down_mb;
-  const double again = each > 4.5 ? (each - 4.5) / 16 * E : 0;
-  const double few = 10 + (first_mb + down_mb) * (used / 6.6 + again / 6.5);
-  const double mid_tiles = used + (each > 32 ? (each - 32) / 64 * E : 0);
+  t.mb = first_mb + down_mb;
+  const double mid_tiles = t.used + (t.each > 32 ? (t.each - 32) / 64 * E : 0);
   auto product = [&](double mb, double rate, int k, int cols) {
     const double a_unit = mid_tiles * cols / units;
     const double uneven = a_unit > 1 ? ceil(a_unit) / a_unit : 1;
-    return 5 + fmax(1.05 * k / 64, used * mb / rate * uneven);
+    return 5 + fmax(1.05 * k / 64, t.used * mb / rate * uneven);
   };
-  const double mid = product(first_mb, gated ? 6.1 : 7.2, H, first_cols) + product(down_mb, 7.2, I, down_cols);
-  if (each <= 64 && few <= mid) return kTileRows;
+  t.mid = product(first_mb, gated ? 6.1 : 7.2, H, t.first_cols) + product(down_mb, 7.2, I, t.down_cols);
+  return t;
+}
+
+extern "C" int kvc_moe_tile_rows(int pairs, int E, int H, int I, int gated) {
+  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0) return kTileRows;
+  const TileEstimate est = estimate_tiles(pairs, E, H, I, gated);
+  const double each = est.each;
+  const int first_cols = est.first_cols, down_cols = est.down_cols;
+  const double again = each > 4.5 ? (each - 4.5) / 16 * E : 0;
+  const double few = 10 + est.mb * (est.used / 6.6 + again / 6.5);
+  if (each <= 64 && few <= est.mid) return kTileRows;
   const double blocks = (pairs / 64.0 + E / 2.0) * (first_cols < down_cols ? first_cols : down_cols);
   return blocks >= 300 && (each >= 150 || (each >= 40 && each < 104)) ? kBigTileRows : kMidTileRows;
 }
@@ -1505,15 +1558,49 @@ extern "C" int kvc_moe_wide_tile_rows(int pairs, int E, int H, int I, int gated)
   return each >= 104 && (two_rounds || full) ? kWideTileRows : 0;
 }
 
+// Whether the expert that every one of T tokens runs joins the routed experts' launches, and in tiles of how many rows all of
+// them then go (0: it stays with products of its own), where tile_rows is what they would take alone.
+// In tiles of 16 it is one more expert whose rows fill its tiles, at the rate at which weights stream, where two products of
+// its own take 13 us up to 16 tokens and some 30 beyond for 25 MB.  Larger tiles are few blocks a unit: it joins them where the
+// launches' blocks a unit, rounded up, stay what they are, as a unit with one block more makes the whole chip wait (32 experts of 2048 x
+// 2048, 64 tokens of four, two blocks a unit and 16 more 95 -> 111 us).  So small tiles are worth more with it than without, up to where
+// experts of random tokens begin to have more rows than one holds.
+// A step of 15 layers of 32 experts of 2048 x 2048, four a token, alone / joined in tiles of 16 / of 64 / of 128 rows, us:
+//   1 token 1167 / 1065 / 1502   16 tokens 2587 / 2439 / 2543   32 2960 / 2831 / 3111   64 3365 / 3119 / 3496
+//   100 tokens 3600 / 3577 / 3605 / 3730   180 3746 / 4887 / 3743 / 3923   300 4018 / - / 3883 / 4121   500 4268 / - / 4267 / 4467
+//   800 5720 / - / 5166 / 5141
+extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows) {
+  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || T <= 0 || !known_tile_rows(tile_rows)) return 0;
+  constexpr int kMost = 128;  // tokens whose tiles of 16 find the weights in the L2
+  if (tile_rows == kTileRows) return T <= kMost ? kTileRows : 0;
+  const TileEstimate est = estimate_tiles(pairs, E, H, I, gated);
+  const double units = kvc_device_compute_units();
+  const double tiles = tile_rows == kWideTileRows
+                           ? est.used * fmax(1.0, ceil((est.each - 3 * sqrt(est.each)) / kWideTileRows))
+                           : est.used + (est.each > tile_rows / 2.0 ? (est.each / tile_rows - 0.5) * E : 0);
+  auto room = [&](int cols) {
+    return ceil((tiles + shared_tiles(T, tile_rows)) * cols / units) <= ceil(tiles * cols / units);
+  };
+  const bool joins = room(est.first_cols) && room(est.down_cols);
+  if (T <= kMost && est.each <= 16 && tile_rows == kMidTileRows) {
+    const double again = 0.5 * E * erfc((16.5 - est.each) / sqrt(2 * est.each));  // experts with more than 16 rows
+    const double few = 10 + est.mb * ((est.used + 1) / 6.6 + again / 6.5);
+    const double own = T <= 16 ? 8.6 + est.mb / 6.4 : 20 + est.mb / 2.8;
+    if (few <= est.mid + (joins ? est.mb / 6.5 : own)) return kTileRows;
+  }
+  return joins ? tile_rows : 0;
+}
+
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
-                             int pairs, int E, int max_tiles, int tile_rows, kvc_stream stream) {
+                             int pairs, int E, int max_tiles, int tile_rows, int shared_rows, kvc_stream stream) {
   if (!known_tile_rows(tile_rows)) return kvc_fail("kvc_moe_align: tiles of 16, 64, 128 or 384 rows");
-  if (pairs < 0 || E <= 0 || max_tiles < kvc_moe_max_tiles(pairs, E, tile_rows))
+  if (pairs < 0 || E <= 0 || shared_rows < 0 ||
+      max_tiles < kvc_moe_max_tiles(pairs, E, tile_rows) + shared_tiles(shared_rows, tile_rows))
     return kvc_fail("kvc_moe_align: bad sizes, or room for fewer tiles than the routing may need");
   const size_t lds = sizeof(int32_t) * 3 * E;
   if (lds > 60000) return kvc_fail("kvc_moe_align: too many experts");
   hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), lds, S(stream), sorted, tiles, num_tiles, choice,
-                     pairs, E, max_tiles, tile_rows);
+                     pairs, E, max_tiles, tile_rows, shared_rows);
   return kvc_check_launch("kvc_moe_align");
 }
 
@@ -1521,7 +1608,11 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
                             const void* w, int dtype, const int32_t* sorted, const int32_t* tiles,
                             const int32_t* num_tiles, int max_tiles, int tile_rows, int N, int K, int in_div,
                             int out_sorted, int gated, float limit, float alpha, float up_shift, int act,
-                            const float* row_scale, int packed, kvc_stream stream) {
+                            const float* row_scale, const void* w_shared, int shared_first, float shared_limit, int packed,
+                            kvc_stream stream) {
+  const SharedExpert shared{w_shared, shared_first, shared_limit};
+  if (w_shared != nullptr && row_scale != nullptr)
+    return kvc_fail("kvc_moe_gemm: no scale a pair beside an expert that every token runs");
   if (max_tiles < 0 || N <= 0 || K <= 0 || x_stride < K || out_stride < N)
     return kvc_fail("kvc_moe_gemm: bad sizes");
   if (!known_tile_rows(tile_rows)) return kvc_fail("kvc_moe_gemm: tiles of 16, 64, 128 or 384 rows");
@@ -1530,7 +1621,7 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
   if (max_tiles == 0) return 0;
   dim3 grid(max_tiles, (N + 63) / 64);
   if (grid.y > 65535u) return kvc_fail("kvc_moe_gemm: too many columns");
-#define KVC_MOE_ARGS sorted, tiles, num_tiles, N, K, in_div, out_sorted, limit, alpha, up_shift, act, row_scale
+#define KVC_MOE_ARGS sorted, tiles, num_tiles, N, K, in_div, out_sorted, limit, alpha, up_shift, act, row_scale, shared
 #define KVC_MOE_LAUNCH(KERNEL, TI, TO)                                                                          \
   hipLaunchKernelGGL(KERNEL, grid, dim3(256), 0, S(stream), static_cast<TO*>(out), out_stride,                   \
                      static_cast<const TI*>(x), x_stride, static_cast<const TI*>(w), KVC_MOE_ARGS)
@@ -1538,7 +1629,7 @@ extern "C" int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const 
   if (dtype == 1) {
     // the matrix cores read 16 bytes at a time: rows of a multiple of 8 values, 16-byte aligned
     const bool vectors = K % 8 == 0 && x_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-                         (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+                         ((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w_shared)) & 15) == 0;
     if (tile_rows != kTileRows) {
       if (!vectors || K % 32) return kvc_fail("kvc_moe_gemm: tiles of 64 rows and more need K to be a multiple of 32");
       if (tile_rows == kWideTileRows && K % 64) return kvc_fail("kvc_moe_gemm: tiles of 384 rows need K to be a multiple of 64");

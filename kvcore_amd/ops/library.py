@@ -72,13 +72,14 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_head_rmsnorm_gate": [P, I, P, P, L, I, P, F, I, I, I, I, P],
         "kvc_moe_route": [P, P, P, I, I, I, I, I, I, P, P, I, I, F, P],
         "kvc_moe_router": [P, P, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
-        "kvc_moe_router_spread": [P, P, P, P, P, I, I, P, L, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
+        "kvc_moe_router_spread": [P, P, P, P, P, I, I, I, P, L, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
         "kvc_moe_router_spread_floats": [I, I],
         "kvc_moe_max_tiles": [I, I, I],
+        "kvc_moe_shared_tile_rows": [I, I, I, I, I, I, I],
         "kvc_moe_tile_rows": [I, I, I, I, I],
         "kvc_moe_wide_tile_rows": [I, I, I, I, I],
-        "kvc_moe_align": [P, P, P, P, I, I, I, I, P],
-        "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, I, P],
+        "kvc_moe_align": [P, P, P, P, I, I, I, I, I, P],
+        "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, P, I, F, I, P],
         "kvc_moe_combine": [P, P, P, I, P, I, P, P, I, I, I, P],
         "kvc_moe_combine_norm": [P, I, P, P, P, I, P, P, P, P, F, I, I, P],
         "kvc_qk_norm_rope_kv_write": [P, L, P, P, I, P, P, F, P, P, I, I, P, I, I, I, I, I, I, I, I, I, P],
@@ -2085,7 +2086,8 @@ def moe_router_spread(choice: torch.Tensor, weight: torch.Tensor, sorted_pairs: 
                    num_tiles: torch.Tensor, x: torch.Tensor, router: torch.Tensor, work: torch.Tensor, *, top: int,
                    tile_rows: int, groups: int = 1, keep: int = 1, score: str = "softmax",
                    correction: torch.Tensor | None = None, group_best: int = 1, weight_scale: float = 1.0,
-                   bias: torch.Tensor | None = None, gate: torch.Tensor | None = None, renormalize: bool = True) -> None:
+                   bias: torch.Tensor | None = None, gate: torch.Tensor | None = None, renormalize: bool = True,
+                   shared_rows: int = 0) -> None:
     """:func:`moe_router` and :func:`moe_align` where ``moe_router_spread_supported``, with the same results; ``work`` float32, ``moe_router_spread_floats`` values."""
     T, H = x.shape
     E = router.shape[0] - (1 if gate is not None else 0)
@@ -2093,11 +2095,11 @@ def moe_router_spread(choice: torch.Tensor, weight: torch.Tensor, sorted_pairs: 
         raise KernelError("moe_router_spread: a gate value a token")
     if router.dim() != 2 or router.shape[1] != H or E < 1 or choice.shape != (T, top) or weight.shape != (T, top) or x.stride(1) != 1:
         raise KernelError("moe_router_spread: shapes do not match")
-    if sorted_pairs.numel() < T * top or tiles.dim() != 2 or tiles.shape[1] != 3 or num_tiles.numel() < 1:
+    if sorted_pairs.numel() < T * top + shared_rows or tiles.dim() != 2 or tiles.shape[1] != 3 or num_tiles.numel() < 1:
         raise KernelError("moe_router_spread: buffers too small")
     _check(load().kvc_moe_router_spread(
         _dev(choice, "choice", torch.int32), _dev(weight, "weight", torch.float32), _dev(sorted_pairs, "sorted", torch.int32),
-        _dev(tiles, "tiles", torch.int32), _dev(num_tiles, "num_tiles", torch.int32), tiles.shape[0], tile_rows,
+        _dev(tiles, "tiles", torch.int32), _dev(num_tiles, "num_tiles", torch.int32), tiles.shape[0], tile_rows, int(shared_rows),
         _dev(work, "work", torch.float32), work.numel(), x.data_ptr(), x.stride(0), _code(x, "x"),
         _dev(router, "router", torch.float32), None if gate is None else _dev(gate, "gate", torch.float32), T, H, E, top,
         groups, keep, *_route_rule(E, score, bias, correction, group_best, weight_scale, renormalize), _stream()),
@@ -2122,43 +2124,65 @@ def moe_wide_tile_rows(pairs: int, experts: int, x: torch.Tensor, k_sizes: tuple
     return int(load().kvc_moe_wide_tile_rows(pairs, experts, *k_sizes, int(gated)))
 
 
-def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16) -> int:
-    return int(load().kvc_moe_max_tiles(pairs, experts, tile_rows))
+def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16, shared_rows: int = 0) -> int:
+    return int(load().kvc_moe_max_tiles(pairs, experts, tile_rows)) + -(-shared_rows // tile_rows)
+
+
+def moe_shared_fits(w: torch.Tensor, shared: torch.Tensor, experts: int) -> bool:
+    """Whether the matrix of an expert that every token runs may join a launch over the routed experts' stacked ones
+    (:func:`moe_gemm`'s ``shared``): bfloat16, of an expert's size, and stored in the same order."""
+    return (w.dtype == torch.bfloat16 and shared.dtype == torch.bfloat16
+            and w.shape == (experts * shared.shape[0], shared.shape[1])
+            and (getattr(w, "kvc_packed", None) is None) == (getattr(shared, "kvc_packed", None) is None))
+
+
+def moe_shared_tile_rows(pairs: int, experts: int, k_sizes: tuple[int, int], gated: bool, tokens: int, tile_rows: int) -> int:
+    """Rows a tile of the experts' products holds where the expert that every one of ``tokens`` tokens runs joins them,
+    or 0 where it is the faster by itself; ``tile_rows``: what the routed experts take alone."""
+    return int(load().kvc_moe_shared_tile_rows(pairs, experts, *k_sizes, int(gated), tokens, tile_rows))
 
 
 def moe_align(sorted_pairs: torch.Tensor, tiles: torch.Tensor, num_tiles: torch.Tensor, choice: torch.Tensor,
-              experts: int, tile_rows: int = 16) -> None:
+              experts: int, tile_rows: int = 16, shared_rows: int = 0) -> None:
     """(token, choice) pairs sorted by expert, and the list of row tiles (``tiles [>= max_tiles, 3]``)
-    of up to ``tile_rows`` rows."""
+    of up to ``tile_rows`` rows.  ``shared_rows``: so many tokens' rows of an expert that every token runs join
+    them (:func:`moe_gemm`'s ``shared``): its tiles first, its pairs last."""
     pairs = choice.numel()
-    if sorted_pairs.numel() < pairs or tiles.dim() != 2 or tiles.shape[1] != 3 or num_tiles.numel() < 1:
+    if sorted_pairs.numel() < pairs + shared_rows or tiles.dim() != 2 or tiles.shape[1] != 3 or num_tiles.numel() < 1:
         raise KernelError("moe_align: buffers too small")
     _check(load().kvc_moe_align(_dev(sorted_pairs, "sorted", torch.int32), _dev(tiles, "tiles", torch.int32),
                                 _dev(num_tiles, "num_tiles", torch.int32), _dev(choice, "choice", torch.int32),
-                                pairs, experts, tiles.shape[0], tile_rows, _stream()), "kvc_moe_align")
+                                pairs, experts, tiles.shape[0], tile_rows, int(shared_rows), _stream()), "kvc_moe_align")
 
 
 def moe_gemm(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, sorted_pairs: torch.Tensor, tiles: torch.Tensor,
              num_tiles: torch.Tensor, *, pairs: int, experts: int, in_div: int, out_sorted: bool, gated: bool,
              limit: float = 0.0, alpha: float = 0.0, up_shift: float = 1.0, tile_rows: int = 16,
-             act: str | None = None, row_scale: torch.Tensor | None = None) -> None:
+             act: str | None = None, row_scale: torch.Tensor | None = None, shared: torch.Tensor | None = None,
+             shared_rows: int = 0, shared_limit: float = 0.0) -> None:
     """Every expert's product over its own rows.  ``w`` is ``[experts * N, K]`` (``experts * 2N``
     rows when ``gated``: each expert's gate rows, then its up rows); ``out [pairs, N]``.  The gated
     form stores ``min(g, limit) * sigmoid(alpha * g) * (clamp(u, -limit, limit) + up_shift)``; without a gate
     ``act`` may name one of :data:`ACTIVATIONS`.  ``row_scale`` (float32, a value a pair) multiplies a pair's
-    input: its sums, before any activation."""
+    input: its sums, before any activation.  ``shared`` (``moe_shared_fits``): the matrix of an expert of the same
+    size that every token runs, with a limit of its own; ``out`` has ``shared_rows`` more rows for it behind the
+    ``pairs``, and so has ``x`` where ``in_div`` is 0."""
     N = out.shape[1]
     K = x.shape[1]
     rows = experts * N * (2 if gated else 1)
-    if w.shape != (rows, K) or out.shape[0] < pairs or x.dtype != w.dtype or out.stride(1) != 1 or x.stride(1) != 1:
+    if w.shape != (rows, K) or out.shape[0] < pairs + shared_rows or x.dtype != w.dtype or out.stride(1) != 1 or x.stride(1) != 1:
         raise KernelError("moe_gemm: shapes do not match")
     if act is not None and (gated or act not in ACTIVATIONS):
         raise KernelError(f"moe_gemm: activation {act!r} of a product without a gate (known: {sorted(ACTIVATIONS)})")
     if row_scale is not None and row_scale.numel() < pairs:
         raise KernelError("moe_gemm: a scale a pair")
-    max_tiles = min(tiles.shape[0], moe_max_tiles(pairs, experts, tile_rows))
+    if (shared is None) != (shared_rows == 0) or (shared is not None and (
+            not moe_shared_fits(w, shared, experts) or x.shape[0] < (pairs if in_div == 0 else 0) + shared_rows)):
+        raise KernelError("moe_gemm: the expert that every token runs does not fit the others")
+    max_tiles = min(tiles.shape[0], moe_max_tiles(pairs, experts, tile_rows, shared_rows))
     # the bfloat16 kernels read the packed twin of the experts' matrix where the model keeps one
     w_ptr, packed = (_streamed(w, N) if N % 16 == 0 and K % 64 == 0 else (_dev(w, "w"), 0))
+    shared_ptr = None if shared is None else _dev(shared.kvc_packed if packed else shared, "shared")
     if packed and pairs <= experts * tile_rows:
         packed = 2  # most experts have one tile, whose loads may then be streaming ones
     _check(load().kvc_moe_gemm(out.data_ptr(), out.stride(0), _code(out, "out"), x.data_ptr(), x.stride(0),
@@ -2166,8 +2190,8 @@ def moe_gemm(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, sorted_pairs: 
                                _dev(tiles, "tiles", torch.int32), _dev(num_tiles, "num_tiles", torch.int32),
                                max_tiles, tile_rows, N, K, int(in_div), int(bool(out_sorted)), int(bool(gated)),
                                float(limit), float(alpha), float(up_shift), -1 if act is None else ACTIVATIONS[act],
-                               None if row_scale is None else _dev(row_scale, "row_scale", torch.float32), packed,
-                               _stream()), "kvc_moe_gemm")
+                               None if row_scale is None else _dev(row_scale, "row_scale", torch.float32), shared_ptr,
+                               int(pairs), float(shared_limit), packed, _stream()), "kvc_moe_gemm")
 
 
 def moe_combine(out: torch.Tensor, y: torch.Tensor, weight: torch.Tensor | None, add0: torch.Tensor | None = None,

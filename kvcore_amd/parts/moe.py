@@ -154,32 +154,41 @@ class RoutedExperts(FeedForward):
                     group_best=self.group_best, weight_scale=self.weight_scale, bias=p.get("router.bias"), gate=gate,
                     renormalize=self.renormalize)
         cap = ctx.buffers.token_capacity
-        sorted_pairs = ctx.buffers.get(f"moe_sorted:{top}", pairs, 1, torch.int32, reserve=cap * top).view(-1)
         # what is the faster for this many rows an expert and matrices of these sizes: see the two kernels' files
         tile_rows = (ops.moe_wide_tile_rows(pairs, E, x, (H, I), self.gated)
                      or ops.moe_tile_rows(pairs, E, x, (H, I), self.gated))
-        max_tiles = ops.moe_max_tiles(pairs, E, tile_rows)
+        # a shared expert of the routed ones' size may run in their launches: as one more expert, of every token
+        fits = (self.shared_size == I and not self.weight_on_input
+                and ops.moe_shared_fits(p[f"experts.{self.first}"], p[f"shared.{self.first}"], E)
+                and ops.moe_shared_fits(p["experts.down"], p["shared.down"], E))
+        joined = ops.moe_shared_tile_rows(pairs, E, (H, I), self.gated, T, tile_rows) if fits else 0
+        tile_rows, also = (joined, T) if joined else (tile_rows, 0)
+        room = cap * (top + 1) if fits else cap * top
+        sorted_pairs = ctx.buffers.get(f"moe_sorted:{top}", pairs + also, 1, torch.int32, reserve=room).view(-1)
+        max_tiles = ops.moe_max_tiles(pairs, E, tile_rows, also)
         tiles = ctx.buffers.get(f"moe_tiles:{top}:{E}", max_tiles, 3, torch.int32,
-                                reserve=ops.moe_max_tiles(cap * top, E, 16))
+                                reserve=ops.moe_max_tiles(cap * top, E, 16, cap if fits else 0))
         num_tiles = ctx.buffers.get("moe_num_tiles", 1, 1, torch.int32).view(-1)
         if ops.moe_router_spread_supported(T, E):
             work = ctx.buffers.get(f"moe_router_parts:{E}", T, ops.moe_router_spread_floats(1, E), torch.float32,
                                    reserve=min(cap, ops.moe_router_spread_tokens()))
             ops.moe_router_spread(choice, weight, sorted_pairs, tiles, num_tiles, x, p["router.weight"], work,
-                               tile_rows=tile_rows, **rule)
+                               tile_rows=tile_rows, shared_rows=also, **rule)
         else:
             ops.moe_router(choice, weight, x, p["router.weight"], **rule)
-            ops.moe_align(sorted_pairs, tiles, num_tiles, choice, E, tile_rows)
-        act = ctx.buffers.get(f"moe_act:{I}", pairs, I, ctx.dtype, reserve=cap * top)
+            ops.moe_align(sorted_pairs, tiles, num_tiles, choice, E, tile_rows, also)
+        act = ctx.buffers.get(f"moe_act:{I}", pairs + also, I, ctx.dtype, reserve=room)
         ops.moe_gemm(act, x, p[f"experts.{self.first}"], sorted_pairs, tiles, num_tiles, pairs=pairs, experts=E,
                      in_div=top, out_sorted=True, gated=self.gated, limit=self.limit, alpha=self.alpha,
                      up_shift=self.up_shift, act=self.activation, row_scale=weight if self.weight_on_input else None,
-                     tile_rows=tile_rows)
-        y = ctx.buffers.get(f"moe_y:{H}", pairs, H, torch.float32, reserve=cap * top)
+                     tile_rows=tile_rows, shared=p[f"shared.{self.first}"] if joined else None, shared_rows=also,
+                     shared_limit=self.shared_limit)
+        y = ctx.buffers.get(f"moe_y:{H}", pairs + also, H, torch.float32, reserve=room)
         ops.moe_gemm(y, act, p["experts.down"], sorted_pairs, tiles, num_tiles, pairs=pairs, experts=E,
-                     in_div=0, out_sorted=False, gated=False, tile_rows=tile_rows)
-        shared = None
-        if self.shared_size:
+                     in_div=0, out_sorted=False, gated=False, tile_rows=tile_rows, shared=p["shared.down"] if joined else None,
+                     shared_rows=also)
+        shared = y[pairs:] if joined else None
+        if self.shared_size and not joined:
             S = self.shared_size
             sact = ctx.buf(f"moe_shared_act:{S}", S)
             if self.gated:

@@ -101,6 +101,19 @@ def test_tiles_of_384_rows_need_rows_and_blocks_for_every_unit():
     assert ops.moe_wide_tile_rows(0, 32, x, (2048, 2048)) == 0
 
 
+def test_when_an_expert_of_every_token_joins_the_others():
+    """In tiles of 16 up to some hundred tokens, in larger ones where no unit gets one block more; never where it does."""
+    from kvcore_amd.ops import library as ops
+
+    x = torch.empty(1, 8, dtype=torch.bfloat16)
+    E, top, sizes = 32, 4, (2048, 2048)
+    for T, want in {1: 16, 32: 16, 64: 16, 100: 16, 120: 0, 180: 0, 300: 64, 500: 0, 800: 128, 831: 0, 1962: 0}.items():
+        alone = ops.moe_wide_tile_rows(T * top, E, x, sizes) or ops.moe_tile_rows(T * top, E, x, sizes)
+        assert ops.moe_shared_tile_rows(T * top, E, sizes, True, T, alone) == want, T
+    assert ops.moe_shared_tile_rows(0, E, sizes, True, 0, 16) == 0
+    assert ops.moe_shared_tile_rows(129 * 2, 64, sizes, True, 129, 16) == 0
+
+
 def _mixers():
     from kvcore_amd.parts.linear_attention import GatedLinearAttention, MaxGatedMatrixMemory
     from kvcore_amd.parts.recurrent import StateSpaceMixer

@@ -759,6 +759,56 @@ def test_tiles_of_384_rows_hold_every_pair_once(E, counts_of):
         assert [e for e, _, _ in listed] == sorted((e for e, _, _ in listed), key=lambda e: (-most[e], e))
 
 
+@pytest.mark.parametrize("packed", [False, True], ids=["rows", "packed"])
+@pytest.mark.parametrize("gated", [True, False], ids=["gated", "plain"])
+@pytest.mark.parametrize("tile_rows,E,T", [(16, 5, 1), (16, 70, 33), (64, 5, 65), (64, 64, 128), (128, 3, 129), (384, 5, 385), (384, 70, 30)])
+def test_an_expert_of_every_token_in_the_others_launches(tile_rows, E, T, gated, packed):
+    """Both products with the shared expert as one more expert: its rows (one tile, a tile and one row, whole tiles) against
+    64-bit sums with its own limit, and the routed experts' rows, which have the bits that they have without it."""
+    from kvcore_amd.ops import library as ops
+
+    H, I, top = 192, 128, 2
+    gen = torch.Generator().manual_seed(T)
+    choice = torch.randint(0, E, (T, top), generator=gen)
+    x = torch.randn(T, H, generator=gen).to(torch.bfloat16)
+    branches = 2 if gated else 1
+    weights = [(torch.randn(*shape, generator=gen) * shape[1] ** -0.5).to(torch.bfloat16)
+               for shape in ((E * branches * I, H), (E * H, I), (branches * I, H), (H, I))]
+    on = [gpu(w, torch.bfloat16) for w in weights]
+    if packed:
+        for w in on:
+            ops.pack_weight(w)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    pairs = T * top
+
+    def products(also):
+        sorted_pairs, num = torch.full((pairs + also,), -1, **i32), torch.empty(1, **i32)
+        tiles = torch.full((ops.moe_max_tiles(pairs, E, tile_rows, also), 3), -7, **i32)
+        ops.moe_align(sorted_pairs, tiles, num, choice.to(**i32), E, tile_rows, also)
+        listed = tiles[: int(num)].tolist()
+        assert sorted(r for _, f, n in listed for r in range(f, f + n)) == list(range(pairs + also))
+        assert sum(n for e, _, n in listed if e < 0) == also
+        act = torch.full((pairs + also, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+        y = torch.full((pairs + also, H), float("nan"), device=DEV)
+        ops.moe_gemm(act, gpu(x, torch.bfloat16), on[0], sorted_pairs, tiles, num, pairs=pairs, experts=E, in_div=top,
+                     out_sorted=True, gated=gated, limit=1.2, alpha=1.702, tile_rows=tile_rows,
+                     act=None if gated else "relu_squared", shared=on[2] if also else None, shared_rows=also, shared_limit=0.7)
+        ops.moe_gemm(y, act, on[1], sorted_pairs, tiles, num, pairs=pairs, experts=E, in_div=0, out_sorted=False, gated=False,
+                     tile_rows=tile_rows, shared=on[3] if also else None, shared_rows=also)
+        return y
+
+    y, alone = products(T), products(0)
+    assert torch.equal(y[:pairs], alone)
+    h = x.double() @ weights[2].double().T
+    if gated:
+        g, u = h[:, :I].clamp(max=0.7), h[:, I:].clamp(-0.7, 0.7)
+        h = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+    else:
+        h = h.clamp(min=0) ** 2
+    # one rounding of the activations to bfloat16, float32 sums
+    assert rel(y[pairs:], h @ weights[3].double().T) < 3e-3
+
+
 @pytest.mark.parametrize("gated", [True, False])
 def test_experts_results_of_infinite_and_missing_sums(gated):
     """Sums that are infinite or no number leave tiles of 64, 128 and 384 rows as the activation says, a sum whose
