@@ -1581,7 +1581,10 @@ extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gate
   auto room = [&](int cols) {
     return ceil((tiles + shared_tiles(T, tile_rows)) * cols / units) <= ceil(tiles * cols / units);
   };
-  const bool joins = room(est.first_cols) && room(est.down_cols);
+  // where the last round has but begun, few units wait for it (tiles of 128 rows, 583 tokens 4,520 / 4,600, 650 5,003 / 4,738)
+  const double rounds = tiles * est.first_cols / units;
+  const bool begun = rounds - floor(rounds) >= (tile_rows == kMidTileRows ? 0.1 : 0.25);
+  const bool joins = begun && room(est.first_cols) && room(est.down_cols);
   if (T <= kMost && est.each <= 16 && tile_rows == kMidTileRows) {
     const double again = 0.5 * E * erfc((16.5 - est.each) / sqrt(2 * est.each));  // experts with more than 16 rows
     const double few = 10 + est.mb * ((est.used + 1) / 6.6 + again / 6.5);

@@ -34,7 +34,14 @@ from kvcore_amd.ops import library as ops
 from kvcore_amd.parts.base import RunLimits
 from kvcore_amd.registry import resolve_architecture
 
-from .context import CacheGroupView, StepBuffers, StepContext
+from .context import CacheGroupView, SideStream, StepBuffers, StepContext
+
+
+# Tokens from which a step that is not captured runs two branches of a layer side by side.  A fork and a join cost the host some
+# 35 us a layer, so that a step that waits for its launches gets slower; layers of linear attention or window attention beside 32 routed
+# experts, off / on, ms: 300 tokens 4.64 / 4.87, 700 6.04 / 5.10, 1,000 6.69 / 6.05, 2,048 10.4 / 9.0, three prompts of 683 9.3 / 8.2.  In a
+# captured step they cost a few us and it is always done: 1 token 1,127 / 991 us, 8 2,200 / 2,021, 64 3,701 / 3,427.
+SIDE_TOKENS = 640
 
 
 @dataclass
@@ -149,6 +156,11 @@ class ModelRunner:
 
         self.buffers = StepBuffers(self.device, token_capacity=max_num_tokens, on_grow=drop_graphs,
                                    seq_capacity=max_num_seqs)
+
+        # a second stream, where a layer has two branches that may run side by side
+        self._side = None
+        if self.device.type == "cuda" and any(block.has_branches for block in model.blocks):
+            self._side = SideStream(self.device)
 
         # host mirror of what each slot's table rows hold: (request id, entries synced,
         # leading entries nulled) per group
@@ -453,7 +465,7 @@ class ModelRunner:
         return StepOutput(ids, logits, owners, T)
 
     def _context(self, T: int, R: int, q_lens: list[int], seq_lens: list[int], max_q: int,
-                 max_seq: int) -> StepContext:
+                 max_seq: int, graph: bool = False) -> StepContext:
         return StepContext(
             num_tokens=T, num_reqs=R,
             token_ids=self._dev["token_ids"], positions=self._dev["positions"],
@@ -464,6 +476,7 @@ class ModelRunner:
             dtype=self.dtype, device=self.device,
             host_query_lens=q_lens, host_seq_lens=seq_lens,
             max_query_len=max_q, max_seq_len=max_seq,
+            side=self._side if graph or T >= SIDE_TOKENS else None,
         )
 
     def _run_decode_bucket(self, bucket: int, num_live: int, max_seq_len: int) -> torch.Tensor:
@@ -481,7 +494,7 @@ class ModelRunner:
         key = (bucket, plan_len)
 
         def run(keep: list | None = None) -> torch.Tensor:
-            ctx = self._context(bucket, bucket, [1] * bucket, [plan_len] * bucket, 1, plan_len)
+            ctx = self._context(bucket, bucket, [1] * bucket, [plan_len] * bucket, 1, plan_len, graph=True)
             hidden = self.model.forward(ctx)
             logits = self.model.compute_logits(ctx, hidden, self._dev["logit_rows"], bucket, every_row=True)
             if keep is not None:  # nothing made in here dies before the capture has ended

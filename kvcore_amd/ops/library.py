@@ -712,6 +712,12 @@ def measure_peaks(device: str | torch.device = "cuda:0") -> dict[str, float]:
     return {"read_bytes_per_s": read_rate, "mfma_bf16_flops_per_s": best}
 
 
+def keep_busy(device: torch.device) -> None:
+    """Some four milliseconds of work on one compute unit, on the current stream (matrix products on registers)."""
+    out = torch.empty(256, dtype=torch.float32, device=device)
+    _check(load().kvc_peak_mfma_bf16(out.data_ptr(), 1, 60000, _stream()), "kvc_peak_mfma_bf16")
+
+
 _COMPUTE_UNITS: int | None = None
 
 

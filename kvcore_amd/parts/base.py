@@ -301,7 +301,10 @@ class FeedForward(Part):
 class Block(Part):
     """An arrangement of norms, mixer and feed-forward around the residual stream.
     ``forward`` takes the pending ``delta`` (output of the previous block not yet added,
-    or None) and the float32 ``residual``, and returns the new pending delta."""
+    or None) and the float32 ``residual``, and returns the new pending delta.  ``has_branches``: the
+    block runs two branches side by side where the step has a second stream (``ctx.side``)."""
+
+    has_branches = False
 
     def __init__(self, *, mixer: Mixer, ffn: FeedForward, norms: dict[str, Norm]) -> None:
         self.mixer = mixer

@@ -116,6 +116,9 @@ class ParallelResidualBlock(Block):
             raise ValueError(f"a parallel block needs its one norm; asked for {norm!r}, given {list(norms)}")
         self.mixer_only = bool(getattr(ffn, "absent", False))
         self.mixer_name, self.ffn_name = mixer_name, ffn_name
+        # experts that add up float32 rows run beside such a mixer where the step has a second stream for it
+        self.has_branches = bool(ffn.gives_weighted_rows and hasattr(ffn, "forward_into")
+                                 and getattr(mixer, "float32_result", False))
 
     def children(self) -> dict[str, Part]:
         out = {self.norm_name: self.norms[self.norm_name], self.mixer_name: self.mixer}
@@ -129,7 +132,15 @@ class ParallelResidualBlock(Block):
         x = ctx.buf("block_x", residual.shape[1])
         if ctx.scratch.pop("stream_normed", None) != call.exec_index:  # else the block before left the norm there
             self.norms[self.norm_name].forward_fused(x, residual, delta)
-        a = self.mixer.forward(x, ctx, call)
+        rows = None
+        if self.has_branches and ctx.side is not None:
+            mixed = []
+            rows = self.ffn.forward_weighted(x, ctx, call, beside=lambda: mixed.append(
+                ctx.side.branch(lambda: self.mixer.forward(x, ctx, call))))
+            ctx.side.join()
+            a = mixed[0]
+        else:
+            a = self.mixer.forward(x, ctx, call)
         if self.mixer_only:
             ops.residual_add(residual, a)
         elif a.dtype == torch.float32 and hasattr(self.ffn, "forward_into"):
@@ -139,9 +150,9 @@ class ParallelResidualBlock(Block):
             if isinstance(next_block, ParallelResidualBlock) and hasattr(self.ffn, "forward_into_normed"):
                 gain = next_block.norms[next_block.norm_name].as_gain()
             if gain is None:
-                self.ffn.forward_into(residual, x, ctx, call, add=a)
+                self.ffn.forward_into(residual, x, ctx, call, add=a, rows=rows)
             else:  # into x, which nothing reads any more by then
-                self.ffn.forward_into_normed(x, residual, x, ctx, call, *gain, add=a)
+                self.ffn.forward_into_normed(x, residual, x, ctx, call, *gain, add=a, rows=rows)
                 ctx.scratch["stream_normed"] = call.exec_index + 1
         else:
             f = self.ffn.forward(x, ctx, call)

@@ -353,3 +353,35 @@ def test_command_lines(models, tmp_path):
            ("x", 12): torch.from_numpy(np.fromfile(out_dir / "0.f32", dtype="<f4").reshape(2, -1)[1]).double(),
            ("x", 20): torch.from_numpy(np.fromfile(out_dir / "2.f32", dtype="<f4").reshape(1, -1)[0]).double()}
     compare(got, {"x": want}, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16"])
+@pytest.mark.parametrize("name", ["A", "B"])
+def test_branches_side_by_side_give_the_bits_of_one_after_the_other(models, name, dtype):
+    """Mixer and experts of a layer on two streams, in a prompt beyond the line from which that is done and in captured
+    steps of two requests (launched, captured and replayed, work of the test's own between the replays), against the same
+    steps on one stream."""
+    from kvcore_amd.engine.runner import SIDE_TOKENS
+
+    folder, cfg, weights, page = models[name]
+    tokens = random_tokens(SIDE_TOKENS + 45, cfg["vocab"], 9)
+    short = random_tokens(30, cfg["vocab"], 10)
+    got = []
+    for beside in (True, False):
+        s = session_for(folder, dtype, page, 1536)
+        assert s.runner._side is not None
+        if not beside:
+            s.runner._side = None
+        steps = [{"step": 0, "entries": [{"id": "a", "tokens": tokens[:SIDE_TOKENS + 9], "want": [0, SIDE_TOKENS]},
+                                         {"id": "b", "tokens": short[:3], "want": [2]}], "end": []}]
+        rows = collect(s, steps)
+        for i in range(8):
+            out = s.run_step({"step": 1 + i, "entries": [
+                {"id": "a", "tokens": [tokens[SIDE_TOKENS + 9 + i]], "want": [0]}, {"id": "b", "tokens": [short[3 + i]], "want": [0]}]})
+            rows[("decode", i)] = out.logits.clone().cpu().double()
+            torch.randn(256, 256, device="cuda").mm(torch.randn(256, 256, device="cuda"))
+        assert s.runner.graph_replays >= 6
+        got.append(rows)
+    assert got[0].keys() == got[1].keys()
+    for key, row in got[0].items():
+        assert torch.isfinite(row).all() and torch.equal(row, got[1][key]), key
