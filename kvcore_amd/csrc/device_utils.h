@@ -76,9 +76,6 @@ __device__ __forceinline__ float rotate_second(float x0, float x1, float c, floa
   return __builtin_fmaf(x0, s, x1 * c);
 }
 
-__device__ __forceinline__ float sigmoid_of(float x) { return 1.f / (1.f + expf(-x)); }
-__device__ __forceinline__ float silu_of(float x) { return x / (1.f + expf(-x)); }
-
 // A soft cap on attention scores inside the matrix-core kernels: cap * tanh(scale * raw / cap) in units of
 // cap, from the raw score and rate = 2 * log2(e) * scale / cap.  tanh(y) = 1 - 2 / (1 + e^(2y)) with the
 // hardware's exponential and reciprocal: an absolute error of some 1e-7 of the cap.
@@ -90,7 +87,7 @@ __device__ __forceinline__ float capped_unit(float raw, float rate) {
 // division's instructions (an elementwise pass over a gate and a tile of gated results spent more time in the division than
 // on their bytes).  The reciprocal is taken of a quarter of d, as that of a d beyond 2^126 would be subnormal and come out
 // as zero.  For d = 1 + exp(-alpha g) the bits are the division's for all 2^32 values of g with alpha 0.5, 1, 1.702 and 3, tried out
-// one by one (with alpha 0.001 two differ, in the last bit).
+// one by one (with alpha 0.001 two differ, in the last bit), and so they are for 1 / d with alpha 1.
 template <bool QUICK>
 __device__ __forceinline__ float quotient(float g, float d) {
   if (!QUICK) return g / d;
@@ -98,6 +95,10 @@ __device__ __forceinline__ float quotient(float g, float d) {
   return fabsf(left) > 0.f ? __builtin_fmaf(left, r, q) : q;  // q is right where nothing is left (a zero keeps its sign) and
                                                               // where q or d is infinite and what is left no number
 }
+
+// (the bits of the divisions, see above)
+__device__ __forceinline__ float sigmoid_of(float x) { return quotient<true>(1.f, 1.f + expf(-x)); }
+__device__ __forceinline__ float silu_of(float x) { return quotient<true>(x, 1.f + expf(-x)); }
 
 // min(g, limit) * sigmoid(alpha * min(g, limit)) * (clamp(u, -limit, limit) + shift)
 template <bool QUICK = false>

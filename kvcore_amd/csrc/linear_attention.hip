@@ -31,8 +31,8 @@ namespace {
 
 constexpr int LSC = 16;  // tokens a stage
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
-__device__ __forceinline__ float silu_ff(float x) { return x / (1.f + expf(-x)); }
+__device__ __forceinline__ float sigmoid_f(float x) { return sigmoid_of(x); }
+__device__ __forceinline__ float silu_ff(float x) { return silu_of(x); }
 // log(1 + e^x) without a threshold: max(x, 0) + log1p(e^-|x|)
 __device__ __forceinline__ float softplus_ff(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 // log(sigmoid(x)) = -softplus(-x)

@@ -23,7 +23,7 @@ namespace {
 
 inline hipStream_t S(kvc_stream s) { return reinterpret_cast<hipStream_t>(s); }
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
+__device__ __forceinline__ float sigmoid_f(float x) { return sigmoid_of(x); }
 __device__ __forceinline__ float silu_f(float x) { return x * sigmoid_f(x); }
 // log(1 + e^x) with no threshold: max(x, 0) + log1p(e^-|x|)
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
@@ -75,9 +75,11 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(
 // once, and the window of the last K inputs slides along in registers, so that a token costs
 // one load of x and one store.  Where all eight and the K - 1 inputs before them are one request's of this
 // step, as nearly everywhere in a prompt, all inputs are asked for at once: token by token, each behind the
-// loads of its request and position, 2,048 tokens of 6,144 channels took 33 us, this way 25 (75 MB: 12 us).
+// loads of its request and position, 2,048 tokens of 6,144 channels took 33 us, this way 25, and with four taps known
+// to the compiler and the division of silu as a reciprocal and a correction (device_utils.h) 22 (75 MB: 12 us).
 constexpr int kConvTokens = 8, kConvMaxTaps = 8;
-template <typename TI, typename TO>
+// TAPS: as many as there are; 0: up to kConvMaxTaps.
+template <typename TI, typename TO, int TAPS>
 __global__ __launch_bounds__(256) void causal_conv_window_kernel(
     TO* __restrict__ out, int64_t out_stride, const TI* __restrict__ x, int64_t x_stride,
     const float* __restrict__ w, const float* __restrict__ bias, const float* __restrict__ state,
@@ -97,17 +99,18 @@ __global__ __launch_bounds__(256) void causal_conv_window_kernel(
   if (t0 + kConvTokens <= T) {
     const int r = token_req[t0];  // the same for the whole block, as all that decides here
     if (r >= 0 && t0 - (K - 1) >= q_start[r] && t0 + kConvTokens <= q_start[r + 1]) {
-      float in[kConvTokens + kConvMaxTaps - 1];  // the last input first
+      constexpr int kTaps = TAPS ? TAPS : kConvMaxTaps;
+      float in[kConvTokens + kTaps - 1];  // the last input first
       const TI* xc = x + static_cast<int64_t>(t0 + kConvTokens - 1) * x_stride + c;
       const int n = kConvTokens + K - 1;
 #pragma unroll
-      for (int j = 0; j < kConvTokens + kConvMaxTaps - 1; ++j)  // what no tap reads repeats the first
-        in[j] = to_float(xc[-static_cast<int64_t>(j < n ? j : n - 1) * x_stride]);
+      for (int j = 0; j < kConvTokens + kTaps - 1; ++j)  // what no tap reads repeats the first
+        in[j] = to_float(xc[-static_cast<int64_t>(TAPS || j < n ? j : n - 1) * x_stride]);
 #pragma unroll
       for (int tt = 0; tt < kConvTokens; ++tt) {
         float acc = b0;
 #pragma unroll
-        for (int j = 0; j < kConvMaxTaps; ++j) acc = fmaf(wr[j], j < K ? in[kConvTokens - 1 - tt + j] : 0.f, acc);
+        for (int j = 0; j < kTaps; ++j) acc = fmaf(wr[j], TAPS || j < K ? in[kConvTokens - 1 - tt + j] : 0.f, acc);
         if (act == 1) acc = silu_f(acc);
         out[static_cast<int64_t>(t0 + tt) * out_stride + c] = from_float<TO>(acc);
       }
@@ -573,15 +576,40 @@ __global__ __launch_bounds__(256) void rglru_scan_segments_kernel(
     return;
   }
   const float* sums = ws + static_cast<int64_t>(r) * (segs + 1) * 2 * W + c;
+  // Sixteen tokens at a time, the next ones on their way while these are worked on, the first while the segments before are
+  // added up: 2,048 tokens of 2,560 channels 35 -> 25 us (eight at a time, none ahead; segments of 32 or blocks of 64 threads: 25).
+  constexpr int kBatch = 16;
+  float av[kBatch], dv[kBatch], yv[kBatch];
+  auto fetch = [&](int t) {  // tokens beyond the segment repeat its last
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int64_t tok = t + i < t1 ? t + i : t1 - 1;
+      av[i] = a[tok * W + c];
+      dv[i] = drive[tok * W + c];
+      yv[i] = to_float(y[tok * y_stride + c]);
+    }
+  };
+  fetch(t0);
   float s = sums[static_cast<int64_t>(segs) * 2 * W];
   // (the sums of eight segments on their way at a time: one by one, 2,048 tokens of 2,560 channels 39 us, so 34)
 #pragma unroll 8
   for (int j = 0; j < sg; ++j) s = fmaf(sums[static_cast<int64_t>(j) * 2 * W], s, sums[static_cast<int64_t>(j) * 2 * W + W]);
-#pragma unroll 8
-  for (int t = t0; t < t1; ++t) {
-    const int64_t at = static_cast<int64_t>(t) * W + c;
-    s = fmaf(a[at], s, drive[at]);
-    out[at] = from_float<TO>(s * gelu_tanh_f(to_float(y[static_cast<int64_t>(t) * y_stride + c])));
+  for (int t = t0; t < t1; t += kBatch) {
+    float g[kBatch], ds[kBatch], as[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      as[i] = av[i];
+      ds[i] = dv[i];
+      g[i] = yv[i];
+    }
+    if (t + kBatch < t1) fetch(t + kBatch);
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      if (t + i < t1) {  // the same for the whole block
+        s = fmaf(as[i], s, ds[i]);
+        out[static_cast<int64_t>(t + i) * W + c] = from_float<TO>(s * gelu_tanh_f(g[i]));
+      }
+    }
   }
   if (t1 == e) state[static_cast<int64_t>(slots[r]) * W + c] = s;
 }
@@ -964,11 +992,14 @@ extern "C" int kvc_causal_conv(void* out, int64_t out_stride, int out_dtype, con
     // portions of prompts (several tokens a request): eight tokens a thread, the window in
     // registers; single tokens of many requests would refill the window at every token
     const dim3 tiles((T + kConvTokens - 1) / kConvTokens, (C + 255) / 256);
-    KVC_DISPATCH_2(x_dtype, TI, out_dtype, TO,
-                   hipLaunchKernelGGL((causal_conv_window_kernel<TI, TO>), tiles, dim3(256), 0, S(stream),
-                                      static_cast<TO*>(out), out_stride, static_cast<const TI*>(x),
-                                      x_stride, weight, bias, state, positions, token_req, q_start,
-                                      slots, T, C, K, act));
+#define KVC_WINDOW(TAPS)                                                                                       \
+  KVC_DISPATCH_2(x_dtype, TI, out_dtype, TO,                                                                   \
+                 hipLaunchKernelGGL((causal_conv_window_kernel<TI, TO, TAPS>), tiles, dim3(256), 0, S(stream), \
+                                    static_cast<TO*>(out), out_stride, static_cast<const TI*>(x), x_stride,    \
+                                    weight, bias, state, positions, token_req, q_start, slots, T, C, K, act))
+    if (K == 4) KVC_WINDOW(4);
+    else KVC_WINDOW(0);
+#undef KVC_WINDOW
   } else {
     KVC_DISPATCH_2(x_dtype, TI, out_dtype, TO,
                    hipLaunchKernelGGL((causal_conv_kernel<TI, TO>), grid, dim3(256), 0, S(stream),
