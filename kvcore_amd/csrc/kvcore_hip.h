@@ -368,6 +368,7 @@ int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32
                        int64_t x_stride, int x_dtype, const float* router, float* gate, int T, int H, int E,
                        int top, int groups, int keep, int score_fn, const float* bias, const float* correction,
                        int group_best, int renormalize, float weight_scale, kvc_stream stream);
+int kvc_moe_one_tile_rows(int pairs, int E, int H, int I, int gated);
 int kvc_moe_max_tiles(int pairs, int E, int tile_rows);
 int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows);
 int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,

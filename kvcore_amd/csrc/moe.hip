@@ -1558,6 +1558,31 @@ extern "C" int kvc_moe_wide_tile_rows(int pairs, int E, int H, int I, int gated)
   return each >= 104 && (two_rounds || full) ? kWideTileRows : 0;
 }
 
+// Tiles of up to 384 rows (the answer; otherwise 0) for fewer rows an expert than the rule above asks for: where the first product
+// has two blocks a unit and the second one a block if every expert is one tile, none is waited for, and an expert with more rows
+// than its share fetches its weights once, where tiles of 128 rows fetch them again for every tile.  Both products and the
+// list in us, the best of the smaller tiles / these, experts of the same chance, and of chances by which the fullest has 2 to 3, and
+// 3.5 to 6 times the mean, gated:
+//   32 experts of 2048 x 2048    56  153 / 152  167 / 157  164 / 170    72  157 / 155  200 / 174  193 / 199    100  172 / 164  201 / 175  202 / 207
+//   64 experts of 2048 x 1024    56  166 / 163  177 / 163  180 / 167    72  173 / 169  206 / 173  196 / 184    100  192 / 175  223 / 189  215 / 192
+//   64 experts of 2048 x 2048    56  303 / 294  320 / 296  332 / 302    72  315 / 301  356 / 310  353 / 340    100  346 / 316  387 / 336  383 / 360
+//   48 experts of 2048 x 1536    56  193 / 192  189 / 185  204 / 182    72  212 / 201  214 / 197  213 / 197    100  230 / 221  235 / 216  244 / 210
+//   32 experts of 4096 x 2048    56  300 / 288  330 / 293  341 / 306    72  314 / 294  368 / 315  361 / 340    100  339 / 306  382 / 319  384 / 361
+//   128 experts of 2048 x 1024   56  326 / 310  349 / 323  341 / 331    72  343 / 319  361 / 365  374 / 353    100  371 / 343  408 / 367  414 / 370
+// not gated:
+//   64 experts of 2048 x 2048    56  209 / 200  223 / 201  239 / 211    72  218 / 204  263 / 213  252 / 233    100  241 / 214  283 / 235  269 / 246
+// A step over 15 layers of 32 experts of 2048 x 2048, four a token, beside an expert that every token runs: 450 tokens 4,220 ->
+// 4,165 us, 600 4,730 -> 4,565, 700 4,925 -> 4,745, 820 5,830 -> 5,055.
+// At 40 rows they are level where experts have the same chance (148 / 148, 155 / 159, 286 / 289), and an expert that every token
+// runs costs in them what it does not in tiles of 64 (177 / 193).
+extern "C" int kvc_moe_one_tile_rows(int pairs, int E, int H, int I, int gated) {
+  if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || H % 64 || I % 64) return 0;
+  const double each = static_cast<double>(pairs) / E, units = kvc_device_compute_units();
+  const double first = E * static_cast<double>(gated ? (I + 127) / 128 : (I + 255) / 256) / units;
+  const double down = E * static_cast<double>((H + 255) / 256) / units;
+  return each >= 48 && each < 104 && first >= 2 && down >= 1 && H + I >= 3072 ? kWideTileRows : 0;
+}
+
 // Whether the expert that every one of T tokens runs joins the routed experts' launches, and in tiles of how many rows all of
 // them then go (0: it stays with products of its own), where tile_rows is what they would take alone.
 // In tiles of 16 it is one more expert whose rows fill its tiles, at the rate at which weights stream, where two products of

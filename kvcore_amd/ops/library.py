@@ -78,6 +78,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_moe_shared_tile_rows": [I, I, I, I, I, I, I],
         "kvc_moe_tile_rows": [I, I, I, I, I],
         "kvc_moe_wide_tile_rows": [I, I, I, I, I],
+        "kvc_moe_one_tile_rows": [I, I, I, I, I],
         "kvc_moe_align": [P, P, P, P, I, I, I, I, I, P],
         "kvc_moe_gemm": [P, L, I, P, L, P, I, P, P, P, I, I, I, I, I, I, I, F, F, F, I, P, P, I, F, I, P],
         "kvc_moe_combine": [P, P, P, I, P, I, P, P, I, I, I, P],
@@ -2128,6 +2129,14 @@ def moe_wide_tile_rows(pairs: int, experts: int, x: torch.Tensor, k_sizes: tuple
     if x.dtype != torch.bfloat16:
         return 0
     return int(load().kvc_moe_wide_tile_rows(pairs, experts, *k_sizes, int(gated)))
+
+
+def moe_one_tile_rows(pairs: int, experts: int, x: torch.Tensor, k_sizes: tuple[int, int], gated: bool = True) -> int:
+    """384 where such tiles serve experts of fewer rows than :func:`moe_wide_tile_rows` asks for, nearly every expert in one of
+    them, and the operands allow (bfloat16, every K a multiple of 64), else 0."""
+    if x.dtype != torch.bfloat16:
+        return 0
+    return int(load().kvc_moe_one_tile_rows(pairs, experts, *k_sizes, int(gated)))
 
 
 def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16, shared_rows: int = 0) -> int:

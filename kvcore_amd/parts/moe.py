@@ -153,8 +153,11 @@ class RoutedExperts(FeedForward):
         plan = ctx.scratch.get(key)
         if plan is None:
             pairs, cap = T * top, ctx.buffers.token_capacity
-            # what is the faster for this many rows an expert and matrices of these sizes: see the two kernels' files
+            # what is the faster for this many rows an expert and matrices of these sizes: see the two kernels' files.  Beside another
+            # branch experts of less than 104 rows keep smaller tiles, whose blocks leave room on the units for the branch's (32 experts
+            # of 2048 x 2048, 650 tokens of four 4,650 / 5,170 us, 820 5,070 / 5,300)
             tile_rows = (ops.moe_wide_tile_rows(pairs, E, x, (H, I), self.gated)
+                         or (not beside and ops.moe_one_tile_rows(pairs, E, x, (H, I), self.gated))
                          or ops.moe_tile_rows(pairs, E, x, (H, I), self.gated))
             joined = ops.moe_shared_tile_rows(pairs, E, (H, I), self.gated, T, tile_rows) if fits else 0
             if beside and fits and not joined:

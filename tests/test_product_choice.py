@@ -101,6 +101,20 @@ def test_tiles_of_384_rows_need_rows_and_blocks_for_every_unit():
     assert ops.moe_wide_tile_rows(0, 32, x, (2048, 2048)) == 0
 
 
+def test_tiles_of_384_rows_for_experts_in_one_tile_need_blocks_for_every_unit():
+    from kvcore_amd.ops import library as ops
+
+    x = torch.empty(1, 8, dtype=torch.bfloat16)
+    for (E, H, I, gated), rows in {(32, 2048, 2048, True): {47: 0, 48: 384, 103: 384, 104: 0}, (64, 2048, 1024, True): {47: 0, 48: 384},
+                                   (32, 2048, 2048, False): {100: 0}, (64, 2048, 2048, False): {47: 0, 48: 384},
+                                   (31, 2048, 2048, True): {100: 0}, (64, 1024, 1024, True): {100: 0},
+                                   (32, 2048, 2016, True): {100: 0}}.items():
+        for each, tile in rows.items():
+            assert ops.moe_one_tile_rows(each * E, E, x, (H, I), gated) == tile, (E, H, I, gated, each)
+    assert ops.moe_one_tile_rows(100 * 32, 32, x.float(), (2048, 2048)) == 0
+    assert ops.moe_one_tile_rows(0, 32, x, (2048, 2048)) == 0
+
+
 def test_when_an_expert_of_every_token_joins_the_others():
     """In tiles of 16 up to some hundred tokens, in larger ones where no unit gets one block more; never where it does."""
     from kvcore_amd.ops import library as ops
