@@ -98,9 +98,9 @@ class StepBuffers:
 
 
 class SideStream:
-    """A second stream on which a step runs one of two branches that do not need each other.  ``branch`` starts
-    work there behind what the current stream holds, ``join`` makes the current stream wait for it; between the two neither
-    branch writes what the other one touches.  In a captured step they become branches of the graph.
+    """A second stream on which a step runs one of two branches that do not need each other.  ``fork`` marks what the
+    current stream holds, ``branch`` starts work behind it on the other one, ``join`` makes the current stream wait for that; between
+    fork and join neither branch writes what the other one touches.  In a captured step they become branches of the graph.
 
     The runtime deals its streams to a few hardware queues, and work on two streams of one queue runs one after the
     other: so the stream is the first of some that is seen to work while the current one is busy (a prompt of 2,048 tokens
@@ -132,9 +132,11 @@ class SideStream:
         busy.synchronize()
         return beside
 
+    def fork(self) -> None:
+        self._forked.record(torch.cuda.current_stream(self.device))
+
     def branch(self, work):
         current = torch.cuda.current_stream(self.device)
-        self._forked.record(current)
         self._forked.wait(self.stream)
         torch.cuda.set_stream(self.stream)
         try:

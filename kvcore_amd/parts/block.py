@@ -135,7 +135,7 @@ class ParallelResidualBlock(Block):
         rows = None
         if self.has_branches and ctx.side is not None:
             mixed = []
-            rows = self.ffn.forward_weighted(x, ctx, call, beside=lambda: mixed.append(
+            rows = self.ffn.forward_weighted(x, ctx, call, fork=ctx.side.fork, beside=lambda: mixed.append(
                 ctx.side.branch(lambda: self.mixer.forward(x, ctx, call))))
             ctx.side.join()
             a = mixed[0]

@@ -35,6 +35,15 @@ from .base import FeedForward, ParamSource, ParamSpec, register_feed_forward
 
 GLU_ALPHA = 1.702
 
+# Weights of a step's experts from which they are the longer of a layer's two branches.  The branch that is launched first goes on in
+# the queue that the layer before ran in; the other one's first kernel waits some 6 us for a signal, and so does the kernel behind
+# both for its last one where that is the later.  So the longer branch is launched first: a mixer of few tokens takes some 38 us, in which
+# this many bytes are read.  Captured steps of 16 layers of 32 experts of 2048 x 2048, mixer / router first: 1 token 948 / 990 us, 2 (203 MB)
+# 1,165 / 1,187, 3 (277 MB) 1,383 / 1,343, 4 1,512 / 1,464, 8 2,015 / 1,897, 16 2,568 / 2,424, 32 2,907 / 2,830, 64 3,490 / 3,250,
+# 128 3,957 / 3,763; the mixer only behind the experts' products 8 1,923, 64 3,322.  Steps that are not captured do not care (three prompts of 683
+# 7,700 / 7,700).
+LONG_BRANCH_BYTES = 240e6
+
 
 class RoutedExperts(FeedForward):
     """``experts`` experts of ``expert_size`` hidden units, ``top`` a token; ``groups`` and
@@ -143,9 +152,10 @@ class RoutedExperts(FeedForward):
                         accumulate=into is not None, add1_gate=rows.add_gate, count=rows.count)
         return out
 
-    def _plan(self, x, ctx, fits: bool, beside: bool) -> tuple[int, bool, int, int, int]:
+    def _plan(self, x, ctx, fits: bool, beside: bool) -> tuple[int, bool, int, int, int, bool]:
         """What a step's size decides, once for all layers of these sizes: rows a tile, whether the shared expert joins, how many
-        tiles there may be in this step and in any, and the floats a token that the spread router wants (0: the other one).
+        tiles there may be in this step and in any, the floats a token that the spread router wants (0: the other one), and whether
+        the experts are the longer of two branches.
         ``beside`` another branch it always joins, as products of its own would have to come before the fork: three prompts of
         683 tokens 8,580 -> 8,127 us, two of 700 7,317 -> 6,452, one of 1,500 8,511 -> 7,374 (8,468 on one stream)."""
         E, H, I, top, T = self.experts, self.hidden_size, self.expert_size, self.top, ctx.num_tokens
@@ -163,16 +173,18 @@ class RoutedExperts(FeedForward):
             if beside and fits and not joined:
                 joined = tile_rows
             tile_rows = joined or tile_rows
+            read = (E * -math.expm1(-pairs / E) + (joined != 0)) * (3 if self.gated else 2) * H * I * x.element_size()
             plan = ctx.scratch[key] = (
                 tile_rows, joined != 0, ops.moe_max_tiles(pairs, E, tile_rows, T if joined else 0),
                 ops.moe_max_tiles(cap * top, E, 16, cap if fits else 0),
-                ops.moe_router_spread_floats(1, E) if ops.moe_router_spread_supported(T, E) else 0)
+                ops.moe_router_spread_floats(1, E) if ops.moe_router_spread_supported(T, E) else 0,
+                read >= LONG_BRANCH_BYTES)
         return plan
 
-    def forward_weighted(self, x, ctx, call, beside=None) -> "ops.WeightedRows":
+    def forward_weighted(self, x, ctx, call, fork=None, beside=None) -> "ops.WeightedRows":
         """The experts' results with their weights, and the shared expert's with its gate.  ``beside`` launches what may
-        run at the same time on another stream: from then on this part launches kernels of this library alone, as the vendor
-        library's products on two streams might share memory of its own."""
+        run at the same time on another stream, behind what ``fork`` marks: from the mark on this part launches kernels of this
+        library alone, as the vendor library's products on two streams might share memory of its own."""
         p, H, E, I, top = self.params, self.hidden_size, self.experts, self.expert_size, self.top
         T = ctx.num_tokens
         pairs = T * top
@@ -188,7 +200,7 @@ class RoutedExperts(FeedForward):
         fits = (self.shared_size == I and not self.weight_on_input
                 and ops.moe_shared_fits(p[f"experts.{self.first}"], p[f"shared.{self.first}"], E)
                 and ops.moe_shared_fits(p["experts.down"], p["shared.down"], E))
-        tile_rows, joined, max_tiles, most_tiles, spread = self._plan(x, ctx, fits, beside is not None)
+        tile_rows, joined, max_tiles, most_tiles, spread, longer = self._plan(x, ctx, fits, beside is not None)
         also = T if joined else 0
         room = cap * (top + 1) if fits else cap * top
         shared = None
@@ -203,7 +215,9 @@ class RoutedExperts(FeedForward):
             shared = ctx.buf(f"moe_shared_out:{H}", H, torch.float32)
             ops.linear(shared, sact, p["shared.down"])
         if beside is not None:
-            beside()
+            fork()
+            if not longer:
+                beside()
         sorted_pairs = ctx.buffers.get(f"moe_sorted:{top}", pairs + also, 1, torch.int32, reserve=room).view(-1)
         tiles = ctx.buffers.get(f"moe_tiles:{top}:{E}", max_tiles, 3, torch.int32, reserve=most_tiles)
         num_tiles = ctx.buffers.get("moe_num_tiles", 1, 1, torch.int32).view(-1)
@@ -215,6 +229,8 @@ class RoutedExperts(FeedForward):
         else:
             ops.moe_router(choice, weight, x, p["router.weight"], **rule)
             ops.moe_align(sorted_pairs, tiles, num_tiles, choice, E, tile_rows, also)
+        if beside is not None and longer:
+            beside()
         act = ctx.buffers.get(f"moe_act:{I}", pairs + also, I, ctx.dtype, reserve=room)
         ops.moe_gemm(act, x, p[f"experts.{self.first}"], sorted_pairs, tiles, num_tiles, pairs=pairs, experts=E,
                      in_div=top, out_sorted=True, gated=self.gated, limit=self.limit, alpha=self.alpha,

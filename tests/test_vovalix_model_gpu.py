@@ -385,3 +385,10 @@ def test_branches_side_by_side_give_the_bits_of_one_after_the_other(models, name
     assert got[0].keys() == got[1].keys()
     for key, row in got[0].items():
         assert torch.isfinite(row).all() and torch.equal(row, got[1][key]), key
+
+
+@pytest.mark.parametrize("name", ["A", "B"])
+def test_branches_side_by_side_with_the_experts_launched_first(models, name, monkeypatch):
+    """The same where the experts are taken for the longer branch, as they are in larger models."""
+    monkeypatch.setattr("kvcore_amd.parts.moe.LONG_BRANCH_BYTES", 0)
+    test_branches_side_by_side_give_the_bits_of_one_after_the_other(models, name, torch.bfloat16)
