@@ -99,7 +99,8 @@ class StepBuffers:
 
 class SideStream:
     """A second stream on which a step runs one of two branches that do not need each other.  ``fork`` marks what the
-    current stream holds, ``branch`` starts work behind it on the other one, ``join`` makes the current stream wait for that; between
+    current stream holds, ``branch`` starts work behind it on the other one, ``join`` makes the current stream wait for that (and
+    does nothing where no branch has been started, so that it may stand in a ``finally``); between
     fork and join neither branch writes what the other one touches.  In a captured step they become branches of the graph.
 
     The runtime deals its streams to a few hardware queues, and work on two streams of one queue runs one after the
@@ -114,6 +115,7 @@ class SideStream:
                 if self._works_beside():
                     break
         self._forked, self._done = torch.cuda.Event(), torch.cuda.Event()
+        self._started = False
 
     def _works_beside(self) -> bool:
         """Whether a kernel of the stream ends while a longer one (some milliseconds on one compute unit) holds the current
@@ -138,6 +140,7 @@ class SideStream:
     def branch(self, work):
         current = torch.cuda.current_stream(self.device)
         self._forked.wait(self.stream)
+        self._started = True
         torch.cuda.set_stream(self.stream)
         try:
             return work()
@@ -146,7 +149,9 @@ class SideStream:
             torch.cuda.set_stream(current)
 
     def join(self) -> None:
-        self._done.wait(torch.cuda.current_stream(self.device))
+        if self._started:
+            self._started = False
+            self._done.wait(torch.cuda.current_stream(self.device))
 
 
 @dataclass

@@ -135,9 +135,11 @@ class ParallelResidualBlock(Block):
         rows = None
         if self.has_branches and ctx.side is not None:
             mixed = []
-            rows = self.ffn.forward_weighted(x, ctx, call, fork=ctx.side.fork, beside=lambda: mixed.append(
-                ctx.side.branch(lambda: self.mixer.forward(x, ctx, call))))
-            ctx.side.join()
+            try:
+                rows = self.ffn.forward_weighted(x, ctx, call, fork=ctx.side.fork, beside=lambda: mixed.append(
+                    ctx.side.branch(lambda: self.mixer.forward(x, ctx, call))))
+            finally:  # whoever catches an error and goes on is behind the mixer's kernels, too
+                ctx.side.join()
             a = mixed[0]
         else:
             a = self.mixer.forward(x, ctx, call)

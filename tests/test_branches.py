@@ -1,0 +1,127 @@
+"""A layer's two branches side by side, on the CPU: what a parallel block hands to its parts, and what orders the streams."""
+
+from __future__ import annotations
+
+import contextlib
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from kvcore_amd.engine.context import LayerCall, SideStream
+from kvcore_amd.parts.base import Mixer, Norm
+from kvcore_amd.parts.block import ParallelResidualBlock
+from kvcore_amd.parts.moe import RoutedExperts
+
+
+class CopyNorm(Norm):
+    def forward_fused(self, out, residual, delta):
+        out.copy_(residual)
+
+    def as_gain(self):
+        return torch.ones(4), 1e-5
+
+
+class DoublingMixer(Mixer):
+    float32_result = True
+
+    def __init__(self, log):
+        self.log = log
+
+    def forward(self, x, ctx, call, sink=None):
+        self.log.append("mixer")
+        return 2.0 * x
+
+
+class Side:
+    """In the place of a ``SideStream``: notes what it is asked."""
+
+    def __init__(self, log):
+        self.log = log
+
+    def fork(self):
+        self.log.append("fork")
+
+    def branch(self, work):
+        self.log.append("branch")
+        return work()
+
+    def join(self):
+        self.log.append("join")
+
+
+def experts(log, fails=False):
+    part = RoutedExperts(hidden_size=4, experts=2, top=1, expert_size=4, limit=None)
+
+    def forward_weighted(x, ctx, call, fork=None, beside=None):
+        if beside is not None:
+            fork()
+            beside()
+        log.append("experts")
+        if fails:
+            raise RuntimeError("no room")
+        return "rows"
+
+    part.forward_weighted = forward_weighted
+    part.forward_into = lambda residual, x, ctx, call, add=None, rows=None: (log.append(("into", rows)), residual.add_(add))
+    return part
+
+
+def step(ffn, log, side=True, next_block=None):
+    block = ParallelResidualBlock(mixer=DoublingMixer(log), ffn=ffn, norms={"n": CopyNorm()})
+    ctx = SimpleNamespace(side=Side(log) if side else None, scratch={}, buf=lambda name, cols: torch.zeros(3, cols))
+    residual = torch.ones(3, 4)
+    block.forward(None, residual, ctx, LayerCall(0, 0), next_block=next_block)
+    return residual
+
+
+def test_the_streams_are_joined_when_the_experts_raise():
+    log = []
+    with pytest.raises(RuntimeError, match="no room"):
+        step(experts(log, fails=True), log)
+    assert log == ["fork", "branch", "mixer", "experts", "join"]
+
+
+def test_a_join_waits_for_the_branch_that_was_started_last_and_for_nothing_else(monkeypatch):
+    log = []
+
+    class Event:
+        def __init__(self, name):
+            self.name = name
+
+        def record(self, stream=None):
+            log.append((self.name, "record", stream))
+
+        def wait(self, stream=None):
+            log.append((self.name, "wait", stream))
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: "main")
+    monkeypatch.setattr(torch.cuda, "set_stream", lambda stream: log.append(stream))
+    monkeypatch.setattr(SideStream, "_works_beside", lambda self: True)
+    monkeypatch.setattr(torch.cuda, "Stream", lambda device=None: "side")
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    events = iter((Event("forked"), Event("done")))
+    monkeypatch.setattr(torch.cuda, "Event", lambda: next(events))
+    side = SideStream(torch.device("cpu"))
+
+    def fails():
+        raise ValueError("in the branch")
+
+    side.fork()
+    side.join()  # an error before the branch: an event that this step has not recorded is not waited for
+    assert log == [("forked", "record", "main")]
+    log.clear()
+    with pytest.raises(ValueError, match="in the branch"):
+        side.branch(fails)
+    side.join()
+    side.join()
+    assert log == [("forked", "wait", "side"), "side", ("done", "record", "side"), "main", ("done", "wait", "main")]
+
+
+def test_experts_beside_a_mixer_take_the_rows_that_they_have_made():
+    log = []
+    assert torch.equal(step(experts(log), log), torch.full((3, 4), 3.0))
+    assert log == ["fork", "branch", "mixer", "experts", "join", ("into", "rows")]
+    log.clear()
+    step(experts(log), log, side=False)
+    assert log == ["mixer", ("into", None)]
