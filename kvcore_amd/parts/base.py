@@ -286,13 +286,17 @@ class StreamOp(Part):
 
 class FeedForward(Part):
     """``takes_scaled_rows``, ``takes_sink`` and ``takes_slice_sink`` as for :class:`Mixer`.
-    ``gives_weighted_rows``: the part has a method ``forward_weighted`` that returns its result as
-    ``ops.WeightedRows``, for a block whose next kernel adds them up."""
+    ``gives_weighted_rows``: the part has a method ``forward_weighted(x, ctx, call)`` that returns its result as
+    ``ops.WeightedRows``, for a block whose next kernel adds them up.  ``runs_beside``: that method also takes ``fork`` and
+    ``beside``, calls the one and then the other, which launches another branch on a second stream behind what ``fork`` marks, and
+    launches nothing of the vendor library's from there on; and ``forward_into`` and ``forward_into_normed`` take
+    the ``rows`` that it returned.  A part that says nothing is handed none of these."""
 
     takes_scaled_rows = False
     takes_sink = False
     takes_slice_sink = False
     gives_weighted_rows = False
+    runs_beside = False
 
     def forward(self, x: torch.Tensor, ctx: "StepContext", call: "LayerCall") -> torch.Tensor:
         raise NotImplementedError

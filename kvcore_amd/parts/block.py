@@ -117,8 +117,7 @@ class ParallelResidualBlock(Block):
         self.mixer_only = bool(getattr(ffn, "absent", False))
         self.mixer_name, self.ffn_name = mixer_name, ffn_name
         # experts that add up float32 rows run beside such a mixer where the step has a second stream for it
-        self.has_branches = bool(ffn.gives_weighted_rows and hasattr(ffn, "forward_into")
-                                 and getattr(mixer, "float32_result", False))
+        self.has_branches = bool(getattr(ffn, "runs_beside", False) and getattr(mixer, "float32_result", False))
 
     def children(self) -> dict[str, Part]:
         out = {self.norm_name: self.norms[self.norm_name], self.mixer_name: self.mixer}
@@ -132,11 +131,11 @@ class ParallelResidualBlock(Block):
         x = ctx.buf("block_x", residual.shape[1])
         if ctx.scratch.pop("stream_normed", None) != call.exec_index:  # else the block before left the norm there
             self.norms[self.norm_name].forward_fused(x, residual, delta)
-        rows = None
+        made = {}  # the feed-forward's rows, where it ran beside the mixer
         if self.has_branches and ctx.side is not None:
             mixed = []
             try:
-                rows = self.ffn.forward_weighted(x, ctx, call, fork=ctx.side.fork, beside=lambda: mixed.append(
+                made["rows"] = self.ffn.forward_weighted(x, ctx, call, fork=ctx.side.fork, beside=lambda: mixed.append(
                     ctx.side.branch(lambda: self.mixer.forward(x, ctx, call))))
             finally:  # whoever catches an error and goes on is behind the mixer's kernels, too
                 ctx.side.join()
@@ -152,9 +151,9 @@ class ParallelResidualBlock(Block):
             if isinstance(next_block, ParallelResidualBlock) and hasattr(self.ffn, "forward_into_normed"):
                 gain = next_block.norms[next_block.norm_name].as_gain()
             if gain is None:
-                self.ffn.forward_into(residual, x, ctx, call, add=a, rows=rows)
+                self.ffn.forward_into(residual, x, ctx, call, add=a, **made)
             else:  # into x, which nothing reads any more by then
-                self.ffn.forward_into_normed(x, residual, x, ctx, call, *gain, add=a, rows=rows)
+                self.ffn.forward_into_normed(x, residual, x, ctx, call, *gain, add=a, **made)
                 ctx.scratch["stream_normed"] = call.exec_index + 1
         else:
             f = self.ffn.forward(x, ctx, call)

@@ -61,6 +61,13 @@ class RoutedExperts(FeedForward):
     pattern with ``{e}``), shared, shared_gate, gate, up, down)."""
 
     gives_weighted_rows = True
+    runs_beside = True
+
+    def __init_subclass__(cls, **kwargs) -> None:
+        # a class that brings one of these methods along says by itself whether it takes what another branch needs
+        super().__init_subclass__(**kwargs)
+        if "runs_beside" not in vars(cls) and vars(cls).keys() & {"forward", "forward_weighted", "forward_into", "forward_into_normed"}:
+            cls.runs_beside = False
 
     def __init__(self, *, hidden_size: int, experts: int, top: int, expert_size: int, limit: float | None,
                  groups: int = 1, keep: int = 1, shared_size: int = 0, shared_limit: float | None = None,

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from kvcore_amd.engine.context import LayerCall, SideStream
-from kvcore_amd.parts.base import Mixer, Norm
+from kvcore_amd.parts.base import FeedForward, Mixer, Norm
 from kvcore_amd.parts.block import ParallelResidualBlock
 from kvcore_amd.parts.moe import RoutedExperts
 
@@ -125,3 +125,67 @@ def test_experts_beside_a_mixer_take_the_rows_that_they_have_made():
     log.clear()
     step(experts(log), log, side=False)
     assert log == ["mixer", ("into", None)]
+
+
+class AddingFeedForward(FeedForward):
+    """As the documented signatures have it, and no more."""
+
+    gives_weighted_rows = True
+
+    def __init__(self, log):
+        self.log = log
+
+    def forward_weighted(self, x, ctx, call):
+        raise AssertionError("not this block's")
+
+    def forward_into(self, residual, x, ctx, call, add=None):
+        self.log.append("into")
+        residual.add_(add).add_(x)
+
+
+class NormedFeedForward(AddingFeedForward):
+    def forward_into_normed(self, out, residual, x, ctx, call, gain, eps, add=None):
+        self.log.append("normed")
+        residual.add_(add).add_(x)
+
+
+class OwnExperts(RoutedExperts):
+    """Experts with a ``forward_weighted`` of the three arguments that a block without a second stream passes."""
+
+    def forward_weighted(self, x, ctx, call):
+        self.log.append("weighted")
+        return "rows"
+
+    def forward_into(self, residual, x, ctx, call, add=None):
+        assert self.forward_weighted(x, ctx, call) == "rows"
+        residual.add_(add).add_(x)
+
+
+@pytest.mark.parametrize("side", [False, True], ids=["one stream", "a second stream"])
+@pytest.mark.parametrize("kind", ["into", "normed", "experts"])
+def test_a_feed_forward_that_knows_nothing_of_branches(kind, side):
+    """A registered part with the documented methods is called with their arguments, on one stream."""
+    log = []
+    following = None
+    if kind == "experts":
+        ffn = OwnExperts(hidden_size=4, experts=2, top=1, expert_size=4, limit=None)
+        ffn.log = log
+    else:
+        ffn = (NormedFeedForward if kind == "normed" else AddingFeedForward)(log)
+        following = ParallelResidualBlock(mixer=DoublingMixer(log), ffn=ffn, norms={"n": CopyNorm()})
+        assert not following.has_branches
+    assert torch.equal(step(ffn, log, side, following), torch.full((3, 4), 4.0))
+    assert log == ["mixer", {"into": "into", "normed": "normed", "experts": "weighted"}[kind]]
+
+
+def test_a_subclass_of_the_experts_that_says_so_runs_beside():
+    class Same(RoutedExperts):
+        pass
+
+    class Own(RoutedExperts):
+        runs_beside = True
+
+        def forward_weighted(self, x, ctx, call, fork=None, beside=None):
+            return super().forward_weighted(x, ctx, call, fork, beside)
+
+    assert RoutedExperts.runs_beside and Same.runs_beside and Own.runs_beside and not OwnExperts.runs_beside
