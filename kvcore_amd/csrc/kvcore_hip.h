@@ -251,13 +251,16 @@ int kvc_gated_group_rmsnorm(void* out, int out_dtype, const float* y, const void
 // values a head and column dv - 1 of every head takes a one for each token: a normaliser that is
 // gated and read like the matrix, out[t, h, dv - 1] being its product with the query.  silu_in: q, k and v
 // pass through silu on their way in (q before its scale; delta_rule 2 without beta only).  below > 0: requests of
-// that many tokens and more in the step are left alone (so for kvc_ssm_scan).
+// that many tokens and more in the step are left alone (so for kvc_ssm_scan).  chains: so many requests bring many tokens while
+// another stream's kernels may run beside (0: none do); speed alone depends on it.
 int kvc_linear_state_scan(float* out, const float* q, int64_t q_stride, const float* k,
                           int64_t k_stride, const float* v, int64_t v_stride, const float* decay,
                           int64_t decay_stride, const float* beta, int64_t beta_stride, float* state,
                           const int32_t* positions, const int32_t* token_req, const int32_t* q_start,
                           const int32_t* slots, int R, int nh, int nqk, int d, int dv, int delta_rule,
-                          float q_scale, int ones_column, int silu_in, int below, kvc_stream stream);
+                          float q_scale, int ones_column, int silu_in, int below, int chains, kvc_stream stream);
+// The bytes of LDS that a block asks for at least where so many of them walk many tokens beside another stream.
+int kvc_linear_state_scan_lds(int64_t blocks);
 // delta_rule 2 with a fixed decay per head (decay [nh], no beta) over portions of prompts, in chunks of
 // kvc_fixed_decay_chunk_tokens() tokens side by side (chunked_state.hip): the same results as the scan's, up to
 // the order of sums.  work: work_chunks >= min(T, T / chunk + R) chunks of nh * dpad * dv floats each.

@@ -728,13 +728,28 @@ extern "C" int kvc_max_gated_finish(void* out, int out_dtype, const float* o, co
   return kvc_check_launch("kvc_max_gated_finish");
 }
 
+// What a block of a scan asks for of a unit's LDS at least where another stream's kernels may run beside it and `blocks` of its blocks walk
+// many tokens.  Such a block is a serial chain, and blocks on one unit slow each other's; alone on the chip they are spread, but where
+// another stream's kernels hold the units, one that such a kernel leaves takes as many blocks as find room.  Beside the routed
+// experts' widest tiles (all of a unit's LDS) four piled up: a prompt of 3,500 tokens, 16 heads of 128 x 128, 1,227 us for the 700
+// that it takes alone.  So where the chains fill half the units a block asks for more than half of the LDS, where they fill all of
+// them for more than a third: one and two a unit, and the rest of the units is the other stream's.  Steps over 12 layers of key decay
+// or attention and four of the delta rule beside 32 experts of 2048 x 2048, one stream / side by side with 35 KB a block / so: 1 x 1,024
+// tokens 6,690 / 6,235 / 5,930 us, 1 x 2,048 10,150 / 9,400 / 9,005, 1 x 4,096 17,960 / 19,100 / 16,700, 2 x 1,024 9,390 / 8,580 / 8,370,
+// 2 x 2,048 16,150 / 15,940 / 15,220; one a unit for two requests 8,440 and 15,520.  More chains stay as they are (3 x 683 7,975;
+// two a unit 8,080, one 8,340), and so do single tokens; beside four of them a prompt of 3,500 takes 14,750 us (one stream 16,430).
+extern "C" int kvc_linear_state_scan_lds(int64_t blocks) {
+  const int64_t units = kvc_device_compute_units();
+  return 2 * blocks <= units ? 82 * 1024 : blocks <= units ? 64 * 1024 : 0;
+}
+
 extern "C" int kvc_linear_state_scan(float* out, const float* q, int64_t q_stride, const float* k,
                                      int64_t k_stride, const float* v, int64_t v_stride,
                                      const float* decay, int64_t decay_stride, const float* beta,
                                      int64_t beta_stride, float* state, const int32_t* positions,
                                      const int32_t* token_req, const int32_t* q_start,
                                      const int32_t* slots, int R, int nh, int nqk, int d, int dv,
-                                     int rule, float q_scale, int ones_column, int silu_in, int below,
+                                     int rule, float q_scale, int ones_column, int silu_in, int below, int chains,
                                      kvc_stream stream) {
   ones_column = ones_column ? 1 : 0;
   if (rule < 0 || rule > 2) return kvc_fail("kvc_linear_state_scan: the rule is 0 (key decay), 1 (delta) or 2 (scalar gates)");
@@ -762,11 +777,19 @@ extern "C" int kvc_linear_state_scan(float* out, const float* q, int64_t q_strid
   const size_t lds = sizeof(float) * (2 * LSC * d + LSC * (delta_rule ? 2 : d) + LSC * VT);
   const int per_thread = (d + NSL - 1) / NSL;
   static const bool no_pf = getenv("KVC_LSCAN_NOPF") != nullptr;  // for tuning
+  const size_t least = chains > 0 ? kvc_linear_state_scan_lds(static_cast<int64_t>(chains) * grid.y * grid.z) : 0;
 #define KVC_LSCAN_F(NPT, DELTA, NSL_, FULL_, PF_)                                                             \
-  hipLaunchKernelGGL((linear_state_scan_kernel<NPT, DELTA, NSL_, FULL_, PF_>), grid, dim3(256),               \
-                     lds*(PF_ ? 2 : 1), S(stream), out, q, q_stride, k, k_stride, v, v_stride, decay,         \
-                     decay_stride, beta, beta_stride, state, positions, token_req, q_start, slots, nh, nqk, d, \
-                     dv, q_scale, ones_column, silu_in, below > 0 ? below : 0x7fffffff)
+  do {                                                                                                        \
+    const auto kernel = &linear_state_scan_kernel<NPT, DELTA, NSL_, FULL_, PF_>;                              \
+    const size_t bytes = lds * (PF_ ? 2 : 1) > least ? lds * (PF_ ? 2 : 1) : least;                           \
+    if (bytes > 64 * 1024 &&                                                                                  \
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                            static_cast<int>(bytes)) != hipSuccess)                                           \
+      return kvc_fail("kvc_linear_state_scan: the kernel's LDS size was refused");                            \
+    hipLaunchKernelGGL(kernel, grid, dim3(256), bytes, S(stream), out, q, q_stride, k, k_stride, v, v_stride, \
+                       decay, decay_stride, beta, beta_stride, state, positions, token_req, q_start, slots,   \
+                       nh, nqk, d, dv, q_scale, ones_column, silu_in, below > 0 ? below : 0x7fffffff);        \
+  } while (0)
   // two sets of LDS buffers (the next stage fetched while one is worked on) where a stage's values
   // deal out evenly to the threads and both sets fit the 64 KB a block may take
 #define KVC_LSCAN(NPT, DELTA, NSL_)                                                  \

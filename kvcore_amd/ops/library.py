@@ -61,7 +61,8 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_kv_slots": [P, P, P, P, P, I, I, I, I, P],
         "kvc_rope_kv_write": [P, P, P, P, P, I, I, P, I, I, I, I, I, I, I, I, P],
         "kvc_paged_attention": [P, P, L, P, P, P, I, P, P, P, I, I, I, I, I, I, I, F, I, P, I, P, F, P, L, I, I, P],
-        "kvc_linear_state_scan": [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, I, I, P],
+        "kvc_linear_state_scan_lds": [L],
+        "kvc_linear_state_scan": [P, P, L, P, L, P, L, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, I, I, I, P],
         "kvc_fixed_decay_chunks": [P, P, L, P, L, P, L, P, P, P, L, P, P, P, P, I, I, I, I, I, I, F, I, P],
         "kvc_scalar_gate_chunks": [P, P, L, P, L, P, L, P, L, P, L, P, P, L, P, P, P, P, I, I, I, I, I, I, I, F, I, P],
         "kvc_channel_gate_chunks": [P, P, L, P, L, P, L, P, L, P, P, L, P, P, P, P, I, I, I, I, I, I, I, F, P],
@@ -1750,7 +1751,7 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
                       slots: torch.Tensor, num_reqs: int, heads: int, qk_heads: int, dim: int,
                       vdim: int, delta_rule: bool = False, q_scale: float = 1.0,
                       scalar_gates: bool = False, ones_column: bool = False, silu_in: bool = False,
-                      below: int = 0) -> None:
+                      below: int = 0, chains: int = 0) -> None:
     """The recurrence of a matrix state per head (see the C header): ``q, k [T, qk_heads * dim]``,
     ``v [T, heads * vdim]``, all float32 rows (column views are fine); ``decay [T, heads * dim]``
     (a factor per key channel) or, with ``delta_rule``, ``decay`` and ``beta [T, heads]``; with
@@ -1760,7 +1761,9 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
     columns takes a one for every token (a normaliser beside the matrix);
     ``state [slots, heads, linear_state_rows(dim), vdim]`` float32, in an order of the kernel's own;
     ``out [T, heads * vdim]`` float32.  ``q_scale``
-    multiplies every q on its way in.  ``below`` > 0: requests of that many tokens and more are left alone."""
+    multiplies every q on its way in.  ``below`` > 0: requests of that many tokens and more are left alone.
+    ``chains``: so many requests walk many tokens while another stream's kernels may run beside; their blocks then share a
+    compute unit with few others (the same bits)."""
     T = out.shape[0]
     if out.shape != (T, heads * vdim) or not out.is_contiguous() or out.dtype != torch.float32:
         raise KernelError("linear_state_scan: out must be contiguous float32 [T, heads * vdim]")
@@ -1790,7 +1793,7 @@ def linear_state_scan(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
         _dev(positions, "positions", torch.int32), _dev(token_req, "token_req", torch.int32),
         _dev(q_start, "q_start", torch.int32), _dev(slots, "slots", torch.int32), num_reqs, heads,
         qk_heads, dim, vdim, 2 if scalar_gates else int(bool(delta_rule)), float(q_scale), int(bool(ones_column)),
-        int(bool(silu_in)), below, _stream()),
+        int(bool(silu_in)), below, int(chains), _stream()),
         "kvc_linear_state_scan")
 
 

@@ -42,6 +42,8 @@ CHUNKED_FROM = 48
 # cut into steps
 GATED_CHUNKED_FROM = 128
 CHANNEL_CHUNKED_FROM = 160
+# from so many tokens on a scan's blocks are chains that must not crowd a unit beside another stream (some 60 us)
+CHAIN_TOKENS = 256
 
 
 def _chunk_start(lengths, start: int, floats: int, many: int, ahead: int) -> int:
@@ -97,6 +99,13 @@ class _MatrixStateMixer(Mixer):
     def _batch(ctx) -> dict:
         return dict(positions=ctx.positions, token_req=ctx.token_req, q_start=ctx.q_start,
                     slots=ctx.slots, num_reqs=ctx.num_reqs)
+
+    @staticmethod
+    def _chains(ctx, below: int = 0) -> int:
+        """Requests that a scan walks for many tokens beside another stream (``below`` > 0: those of fewer tokens alone)."""
+        if ctx.side is None:
+            return 0
+        return sum(n >= CHAIN_TOKENS and (below == 0 or n < below) for n in ctx.host_query_lens)
 
 
 class GatedLinearAttention(_MatrixStateMixer):
@@ -167,7 +176,8 @@ class GatedLinearAttention(_MatrixStateMixer):
         if start:
             ops.channel_gate_chunks(o, *rows, decay, state, work, chunks=chunks, start=start, **sizes)
         if not start or min(ctx.host_query_lens) < start:
-            ops.linear_state_scan(o, *rows, decay, None, state, delta_rule=False, below=start, **sizes)
+            ops.linear_state_scan(o, *rows, decay, None, state, delta_rule=False, below=start, chains=self._chains(ctx, start),
+                                  **sizes)
         return self._finish(o, proj[:, 2 * qk + inner:], ctx)
 
 
@@ -238,7 +248,8 @@ class GatedDeltaRule(_MatrixStateMixer):
         ops.decay_and_write_gates(g, beta, proj[:, at:at + nh], proj[:, at + nh:], p["A_log"], p["dt_bias"])
         o = ctx.buf(f"ms_o:{inner}", inner, torch.float32)
         ops.linear_state_scan(o, qkv[:, :qk], qkv[:, qk:2 * qk], qkv[:, 2 * qk:], g, beta, state, heads=nh,
-                              qk_heads=self.qk_heads, dim=self.dim, vdim=self.vdim, delta_rule=True, **batch)
+                              qk_heads=self.qk_heads, dim=self.dim, vdim=self.vdim, delta_rule=True,
+                              chains=self._chains(ctx), **batch)
         return self._finish(o, proj[:, self.conv_dim: self.conv_dim + inner], ctx)
 
 

@@ -189,3 +189,14 @@ def test_a_subclass_of_the_experts_that_says_so_runs_beside():
             return super().forward_weighted(x, ctx, call, fork, beside)
 
     assert RoutedExperts.runs_beside and Same.runs_beside and Own.runs_beside and not OwnExperts.runs_beside
+
+
+def test_the_requests_whose_scans_leave_units_to_the_other_stream():
+    from kvcore_amd.parts.linear_attention import CHAIN_TOKENS, GatedDeltaRule
+
+    lengths = [3500, 1, CHAIN_TOKENS, CHAIN_TOKENS - 1]
+    beside = SimpleNamespace(side=object(), host_query_lens=lengths)
+    assert GatedDeltaRule._chains(beside) == 2
+    assert GatedDeltaRule._chains(beside, below=300) == 1  # the longer ones go in chunks
+    assert GatedDeltaRule._chains(SimpleNamespace(side=None, host_query_lens=lengths)) == 0
+    assert GatedDeltaRule._chains(SimpleNamespace(side=object(), host_query_lens=[1] * 8)) == 0

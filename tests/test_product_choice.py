@@ -160,3 +160,13 @@ def test_which_requests_are_cut_into_chunks(kind, lengths, cut):
     """By the tokens of the requests, by how far they are ahead of those that stay with the scan, and by how full of
     scans the chip is: the side that was measured to be the faster."""
     assert _mixers()[kind].chunk_start(lengths) == cut
+
+
+def test_a_scan_s_blocks_leave_units_to_another_stream():
+    """Up to half as many blocks as units: one a unit; up to as many: two; they never ask for more than a unit has."""
+    from kvcore_amd.ops import library as ops
+
+    unit = 160 * 1024
+    for blocks, each in {1: 1, 128: 1, 129: 2, 256: 2}.items():
+        assert unit // ops.load().kvc_linear_state_scan_lds(blocks) == each, blocks
+    assert ops.load().kvc_linear_state_scan_lds(257) == 0 and ops.load().kvc_linear_state_scan_lds(1 << 40) == 0

@@ -145,6 +145,34 @@ def test_whole_stages_of_tokens_give_the_bits_of_single_ones(rule, heads, dim, v
     assert torch.equal(whole, single)
 
 
+@pytest.mark.parametrize("rule", ["decay", "delta", "gates"])
+@pytest.mark.parametrize("dim", [64, 256])
+def test_chains_that_leave_room_for_one_two_and_more_on_a_unit(rule, dim):
+    """128, 256 and 384 blocks ask for different shares of a unit's LDS: the first request has the same bits in each, and without any."""
+    from kvcore_amd.ops import library as ops
+
+    gen = torch.Generator().manual_seed(dim)
+    heads, vdim, n = 16, 128, 37
+    asked = [ops.load().kvc_linear_state_scan_lds(128 * R) for R in (1, 2, 3)]
+    assert asked[0] > asked[1] > asked[2] == 0
+    unit = lambda: gpu(plain.unit_vector(torch.randn(3 * n, heads, dim, generator=gen, dtype=torch.float64)).reshape(3 * n, -1))
+    q, k = unit(), unit()
+    v = gpu(torch.randn(3 * n, heads * vdim, generator=gen))
+    beta = gpu(torch.rand(3 * n, heads, generator=gen))
+    decay = gpu(torch.rand(3 * n, heads * (dim if rule == "decay" else 1), generator=gen) * 0.3 + 0.7)
+    got = []
+    for R, chains in ((1, 0), (1, 1), (2, 2), (3, 3), (3, 1)):
+        batch, T = batch_tensors([(r, 0, n) for r in range(R)])
+        state = new_state(3, heads, dim, vdim)
+        out = torch.full((T, heads * vdim), float("nan"), device=DEV)
+        ops.linear_state_scan(out, q[:T], k[:T], v[:T], decay[:T], None if rule == "decay" else beta[:T], state, heads=heads,
+                              qk_heads=heads, dim=dim, vdim=vdim, delta_rule=rule == "delta", scalar_gates=rule == "gates", chains=chains, **batch)
+        got.append((out[:n], state[0]))
+    assert torch.isfinite(got[0][0]).all()
+    for out, state in got[1:]:
+        assert torch.equal(out, got[0][0]) and torch.equal(state, got[0][1])
+
+
 def test_a_token_written_six_hundred_tokens_ago_is_still_read():
     """A decay of almost one: the first token's value, written at a key of its own, comes back
     for a query of that key 600 tokens later (in one step, and token by token), scaled by the
