@@ -1583,22 +1583,34 @@ extern "C" int kvc_moe_one_tile_rows(int pairs, int E, int H, int I, int gated) 
   return each >= 48 && each < 104 && first >= 2 && down >= 1 && H + I >= 3072 ? kWideTileRows : 0;
 }
 
+// us that the expert of every one of T tokens takes in tiles of 16 beside the routed ones: its matrices once, at the rate of theirs,
+// and again for every further tile (a die's L2 holds less than they are); and in two products of its own.
+static double shared_in_few_us(double mb, int T) { return mb / 6.6 + (shared_tiles(T, kTileRows) - 1) * mb / 6.2; }
+static double shared_alone_us(double mb, int T) { return T <= 16 ? 8.6 + mb / 6.4 : 20 + mb / 2.8; }
+
 // Whether the expert that every one of T tokens runs joins the routed experts' launches, and in tiles of how many rows all of
 // them then go (0: it stays with products of its own), where tile_rows is what they would take alone.
 // In tiles of 16 it is one more expert whose rows fill its tiles, at the rate at which weights stream, where two products of
 // its own take 13 us up to 16 tokens and some 30 beyond for 25 MB.  Larger tiles are few blocks a unit: it joins them where the
 // launches' blocks a unit, rounded up, stay what they are, as a unit with one block more makes the whole chip wait (32 experts of 2048 x
 // 2048, 64 tokens of four, two blocks a unit and 16 more 95 -> 111 us).  So small tiles are worth more with it than without, up to where
-// experts of random tokens begin to have more rows than one holds.
-// A step of 15 layers of 32 experts of 2048 x 2048, four a token, alone / joined in tiles of 16 / of 64 / of 128 rows, us:
-//   1 token 1167 / 1065 / 1502   16 tokens 2587 / 2439 / 2543   32 2960 / 2831 / 3111   64 3365 / 3119 / 3496
-//   100 tokens 3600 / 3577 / 3605 / 3730   180 3746 / 4887 / 3743 / 3923   300 4018 / - / 3883 / 4121   500 4268 / - / 4267 / 4467
-//   800 5720 / - / 5166 / 5141
+// experts of random tokens begin to have more rows than one holds, or its own tiles have read its matrices too often.
+// Captured steps, us a layer with it alone / joined in tiles of 16 / of what the others take alone (64 where not said); where this rule
+// counted no second reading, it took tiles of 16 up to 128 tokens in all of these:
+//   32 of 2048 x 2048, 4 a token  24 tokens 179 / 170 (16)   48 216 / 196 / 203   64 219 / 205 / 207   96 231 / 235 / 231   128 245 / 267 / 241
+//   64 of 2048 x 2048, 4 a token  64 tokens 320 / 306 (16)   96 351 / 339 / 332   128 373 / 369 / 355   160 378 / 399 / 375
+//   24 of 3072 x 3072, 4 a token  64 tokens 368 / 360 (16)   96 402 / 432 / 354   128 425 / 507 / 371
+//   16 of 4096 x 4096, 2 a token  32 tokens 342 / 340 (16)   48 380 / 374 / 374   64 396 / 414 / 404    96 425 / 498 / 441   128 461 / 582 / 456
+//   64 of 4096 x 2048, 4 a token  64 tokens 570 / 560 (16)   96 639 / 618 / 597   128 681 / 688 / 651
+//   16 of 1024 x 1024, 4 a token  32 tokens 92 / 80 (16)     64 121 / 103 (16)    96 127 / 111 / 103
+// A step of 15 layers of 32 experts of 2048 x 2048, four a token, alone / joined in tiles of 64 / of 128 rows, us:
+//   300 tokens 4018 / 3883 / 4121   500 4268 / 4267 / 4467
 extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows) {
   if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || T <= 0 || !known_tile_rows(tile_rows)) return 0;
-  constexpr int kMost = 128;  // tokens whose tiles of 16 find the weights in the L2
-  if (tile_rows == kTileRows) return T <= kMost ? kTileRows : 0;
+  constexpr int kMost = 128;  // tokens up to which tiles of 16 were measured
   const TileEstimate est = estimate_tiles(pairs, E, H, I, gated);
+  const double in_few = shared_in_few_us(est.mb, T), own = shared_alone_us(est.mb, T);
+  if (tile_rows == kTileRows) return T <= kMost && in_few <= own ? kTileRows : 0;
   const double units = kvc_device_compute_units();
   const double tiles = tile_rows == kWideTileRows
                            ? est.used * fmax(1.0, ceil((est.each - 3 * sqrt(est.each)) / kWideTileRows))
@@ -1606,14 +1618,14 @@ extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gate
   auto room = [&](int cols) {
     return ceil((tiles + shared_tiles(T, tile_rows)) * cols / units) <= ceil(tiles * cols / units);
   };
-  // where the last round has but begun, few units wait for it (tiles of 128 rows, 583 tokens 4,520 / 4,600, 650 5,003 / 4,738)
+  // where the last round has but begun, few units wait for it (alone / joined, 32 experts of 2048 x 2048 in tiles of 128 rows, 583
+  // tokens 4,520 / 4,600, 650 5,003 / 4,738; tiles of 384 take these numbers of tokens since, but not those of smaller experts)
   const double rounds = tiles * est.first_cols / units;
   const bool begun = rounds - floor(rounds) >= (tile_rows == kMidTileRows ? 0.1 : 0.25);
   const bool joins = begun && room(est.first_cols) && room(est.down_cols);
   if (T <= kMost && est.each <= 16 && tile_rows == kMidTileRows) {
     const double again = 0.5 * E * erfc((16.5 - est.each) / sqrt(2 * est.each));  // experts with more than 16 rows
-    const double few = 10 + est.mb * ((est.used + 1) / 6.6 + again / 6.5);
-    const double own = T <= 16 ? 8.6 + est.mb / 6.4 : 20 + est.mb / 2.8;
+    const double few = 10 + est.mb * (est.used / 6.6 + again / 6.5) + in_few;
     if (few <= est.mid + (joins ? est.mb / 6.5 : own)) return kTileRows;
   }
   return joins ? tile_rows : 0;

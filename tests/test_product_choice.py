@@ -115,17 +115,33 @@ def test_tiles_of_384_rows_for_experts_in_one_tile_need_blocks_for_every_unit():
     assert ops.moe_one_tile_rows(0, 32, x, (2048, 2048)) == 0
 
 
-def test_when_an_expert_of_every_token_joins_the_others():
-    """In tiles of 16 up to some hundred tokens, in larger ones where no unit gets one block more; never where it does."""
+@pytest.mark.parametrize("E,top,H,I,wanted", [
+    (32, 4, 2048, 2048, {1: 16, 32: 16, 64: 16, 72: 16, 96: 0, 128: 0, 180: 0, 300: 64, 500: 0, 800: 0, 831: 0, 1962: 0}),
+    (24, 4, 3072, 3072, {1: 16, 64: 16, 96: 64, 128: 64, 300: 384, 800: 384}),
+    (16, 2, 4096, 4096, {1: 16, 48: 16, 64: 0, 96: 0, 128: 0}),
+    (64, 4, 2048, 2048, {1: 16, 64: 16, 128: 16, 160: 0}),
+    (64, 4, 4096, 2048, {1: 16, 96: 16, 128: 0}),
+    (256, 8, 2048, 512, {1: 16, 128: 16, 129: 0})])
+def test_when_an_expert_of_every_token_joins_the_others(E, top, H, I, wanted):
+    """In tiles of 16 up to some hundred tokens, fewer where its own tiles would read large matrices again and again; in larger tiles where
+    no unit gets one block more; never where it does.  Asked as a step on one stream asks."""
     from kvcore_amd.ops import library as ops
 
     x = torch.empty(1, 8, dtype=torch.bfloat16)
-    E, top, sizes = 32, 4, (2048, 2048)
-    for T, want in {1: 16, 32: 16, 64: 16, 100: 16, 120: 0, 180: 0, 300: 64, 500: 0, 800: 128, 831: 0, 1962: 0}.items():
-        alone = ops.moe_wide_tile_rows(T * top, E, x, sizes) or ops.moe_tile_rows(T * top, E, x, sizes)
-        assert ops.moe_shared_tile_rows(T * top, E, sizes, True, T, alone) == want, T
-    assert ops.moe_shared_tile_rows(0, E, sizes, True, 0, 16) == 0
-    assert ops.moe_shared_tile_rows(129 * 2, 64, sizes, True, 129, 16) == 0
+    for T, want in wanted.items():
+        sizes = (T * top, E, x, (H, I))
+        alone = ops.moe_wide_tile_rows(*sizes) or ops.moe_one_tile_rows(*sizes) or ops.moe_tile_rows(*sizes)
+        assert ops.moe_shared_tile_rows(T * top, E, (H, I), True, T, alone) == want, T
+
+
+def test_tiles_of_16_for_an_expert_of_every_token():
+    from kvcore_amd.ops import library as ops
+
+    assert ops.moe_shared_tile_rows(0, 32, (2048, 2048), True, 0, 16) == 0
+    assert ops.moe_shared_tile_rows(129 * 2, 64, (2048, 2048), True, 129, 16) == 0
+    # two tiles of any matrix cost less than products of its own, eight tiles of 100 MB do not
+    assert ops.moe_shared_tile_rows(32, 128, (4096, 4096), True, 32, 16) == 16
+    assert ops.moe_shared_tile_rows(128, 128, (4096, 4096), True, 128, 16) == 0
 
 
 def _mixers():
