@@ -341,7 +341,7 @@ int kvc_head_rmsnorm_gate(void* out, int out_dtype, const float* o, const void* 
 // kvc_moe_router_spread list its tiles first (room for ceil(shared_rows / tile_rows) more) and behind `pairs` its pairs pairs + t, row t of x
 // where in_div > 0; its matrix is w_shared (stored as w is), shared_first is `pairs`, and
 // shared_limit is its limit.  kvc_moe_shared_tile_rows says whether that is the faster for T tokens, and in tiles of how many rows
-// (0: it is not), where the routed experts alone would take tile_rows.
+// (0: it is not), where the routed experts alone would take tile_rows; beside: while another branch's kernels run on another stream.
 // bias [E] (or null) joins the logits.  score_fn 0: softmax over the experts, 1: sigmoid of each logit,
 // 2: the logit itself, the weights then being the softmax over the chosen logits.  correction [E] (or
 // null) is added to the scores for the choice alone.  group_best 1 or 2: a group is worth its best choice score, or
@@ -373,7 +373,7 @@ int kvc_moe_router_spread(int32_t* choice, float* weight, int32_t* sorted, int32
                        int group_best, int renormalize, float weight_scale, kvc_stream stream);
 int kvc_moe_one_tile_rows(int pairs, int E, int H, int I, int gated);
 int kvc_moe_max_tiles(int pairs, int E, int tile_rows);
-int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows);
+int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows, int beside);
 int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,
                   int pairs, int E, int max_tiles, int tile_rows, int shared_rows, kvc_stream stream);
 int kvc_moe_gemm(void* out, int64_t out_stride, int out_dtype, const void* x, int64_t x_stride,

@@ -1605,12 +1605,21 @@ static double shared_alone_us(double mb, int T) { return T <= 16 ? 8.6 + mb / 6.
 //   16 of 1024 x 1024, 4 a token  32 tokens 92 / 80 (16)     64 121 / 103 (16)    96 127 / 111 / 103
 // A step of 15 layers of 32 experts of 2048 x 2048, four a token, alone / joined in tiles of 64 / of 128 rows, us:
 //   300 tokens 4018 / 3883 / 4121   500 4268 / 4267 / 4467
-extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows) {
+// `beside` another branch's kernels it joins more often, as products of its own come before the branches part: in tiles of 16 wherever these
+// cost less than its own products, in larger ones up to 64 MB an expert, or up to 511 tokens.  Steps of eight layers (16 of the first sizes)
+// beside mixers, own products / joined, us:
+//   32 of 2048 x 2048 (25 MB)    400 tokens 5,620 / 5,230   1,000 6,287 / 6,126   1,500 8,251 / 7,243   2,048 9,385 / 8,889   4,096 17,040 / 16,640
+//   64 of 4096 x 1024 (25 MB)    400 tokens 4,135 / 3,940   640 3,840 / 3,745     1,500 5,345 / 5,070   4,096 10,500 / 10,180
+//   128 of 2048 x 1024 (13 MB), 8 a token  160 tokens 3,495 / 3,377   640 3,695 / 3,557   2,048 6,097 / 5,920
+//   24 of 3072 x 3072 (57 MB)    256 tokens 3,275 / 3,275   640 3,840 / 3,845     1,250 5,300 / 5,350   3,000 11,550 / 11,070
+//   16 of 4096 x 4096 (100 MB), 2 a token  64 tokens 3,105 / 3,270   160 3,607 / 3,397   400 4,535 / 4,240   820 5,000 / 4,620   1,000 5,050 / 5,480   1,500 6,270 / 6,600
+//   16 of 2048 x 8192 (100 MB), 2 a token  160 tokens 3,977 / 3,537   400 4,810 / 4,560   650 4,885 / 5,050   1,000 6,370 / 6,050   4,096 13,050 / 13,410
+extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gated, int T, int tile_rows, int beside) {
   if (pairs <= 0 || E <= 0 || H <= 0 || I <= 0 || T <= 0 || !known_tile_rows(tile_rows)) return 0;
   constexpr int kMost = 128;  // tokens up to which tiles of 16 were measured
   const TileEstimate est = estimate_tiles(pairs, E, H, I, gated);
   const double in_few = shared_in_few_us(est.mb, T), own = shared_alone_us(est.mb, T);
-  if (tile_rows == kTileRows) return T <= kMost && in_few <= own ? kTileRows : 0;
+  if (tile_rows == kTileRows) return (beside || T <= kMost) && in_few <= own ? kTileRows : 0;
   const double units = kvc_device_compute_units();
   const double tiles = tile_rows == kWideTileRows
                            ? est.used * fmax(1.0, ceil((est.each - 3 * sqrt(est.each)) / kWideTileRows))
@@ -1628,7 +1637,7 @@ extern "C" int kvc_moe_shared_tile_rows(int pairs, int E, int H, int I, int gate
     const double few = 10 + est.mb * (est.used / 6.6 + again / 6.5) + in_few;
     if (few <= est.mid + (joins ? est.mb / 6.5 : own)) return kTileRows;
   }
-  return joins ? tile_rows : 0;
+  return joins || (beside && (est.mb <= 64 || T < 512)) ? tile_rows : 0;
 }
 
 extern "C" int kvc_moe_align(int32_t* sorted, int32_t* tiles, int32_t* num_tiles, const int32_t* choice,

@@ -76,7 +76,7 @@ def _declare(lib: ctypes.CDLL) -> None:
         "kvc_moe_router_spread": [P, P, P, P, P, I, I, I, P, L, P, L, I, P, P, I, I, I, I, I, I, I, P, P, I, I, F, P],
         "kvc_moe_router_spread_floats": [I, I],
         "kvc_moe_max_tiles": [I, I, I],
-        "kvc_moe_shared_tile_rows": [I, I, I, I, I, I, I],
+        "kvc_moe_shared_tile_rows": [I, I, I, I, I, I, I, I],
         "kvc_moe_tile_rows": [I, I, I, I, I],
         "kvc_moe_wide_tile_rows": [I, I, I, I, I],
         "kvc_moe_one_tile_rows": [I, I, I, I, I],
@@ -2154,10 +2154,12 @@ def moe_shared_fits(w: torch.Tensor, shared: torch.Tensor, experts: int) -> bool
             and (getattr(w, "kvc_packed", None) is None) == (getattr(shared, "kvc_packed", None) is None))
 
 
-def moe_shared_tile_rows(pairs: int, experts: int, k_sizes: tuple[int, int], gated: bool, tokens: int, tile_rows: int) -> int:
+def moe_shared_tile_rows(pairs: int, experts: int, k_sizes: tuple[int, int], gated: bool, tokens: int, tile_rows: int,
+                         beside: bool = False) -> int:
     """Rows a tile of the experts' products holds where the expert that every one of ``tokens`` tokens runs joins them,
-    or 0 where it is the faster by itself; ``tile_rows``: what the routed experts take alone."""
-    return int(load().kvc_moe_shared_tile_rows(pairs, experts, *k_sizes, int(gated), tokens, tile_rows))
+    or 0 where it is the faster by itself; ``tile_rows``: what the routed experts take alone; ``beside``: while another branch
+    runs on another stream."""
+    return int(load().kvc_moe_shared_tile_rows(pairs, experts, *k_sizes, int(gated), tokens, tile_rows, int(beside)))
 
 
 def moe_align(sorted_pairs: torch.Tensor, tiles: torch.Tensor, num_tiles: torch.Tensor, choice: torch.Tensor,

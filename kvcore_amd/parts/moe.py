@@ -162,9 +162,8 @@ class RoutedExperts(FeedForward):
     def _plan(self, x, ctx, fits: bool, beside: bool) -> tuple[int, bool, int, int, int, bool]:
         """What a step's size decides, once for all layers of these sizes: rows a tile, whether the shared expert joins, how many
         tiles there may be in this step and in any, the floats a token that the spread router wants (0: the other one), and whether
-        the experts are the longer of two branches.
-        ``beside`` another branch it always joins, as products of its own would have to come before the fork: three prompts of
-        683 tokens 8,580 -> 8,127 us, two of 700 7,317 -> 6,452, one of 1,500 8,511 -> 7,374 (8,468 on one stream)."""
+        the experts are the longer of two branches.  ``beside`` another branch the shared expert joins more often, as products of its
+        own have to come before the fork."""
         E, H, I, top, T = self.experts, self.hidden_size, self.expert_size, self.top, ctx.num_tokens
         key = ("routed_experts", E, H, I, top, self.gated, fits, beside)
         plan = ctx.scratch.get(key)
@@ -176,9 +175,7 @@ class RoutedExperts(FeedForward):
             tile_rows = (ops.moe_wide_tile_rows(pairs, E, x, (H, I), self.gated)
                          or (not beside and ops.moe_one_tile_rows(pairs, E, x, (H, I), self.gated))
                          or ops.moe_tile_rows(pairs, E, x, (H, I), self.gated))
-            joined = ops.moe_shared_tile_rows(pairs, E, (H, I), self.gated, T, tile_rows) if fits else 0
-            if beside and fits and not joined:
-                joined = tile_rows
+            joined = ops.moe_shared_tile_rows(pairs, E, (H, I), self.gated, T, tile_rows, beside) if fits else 0
             tile_rows = joined or tile_rows
             read = (E * -math.expm1(-pairs / E) + (joined != 0)) * (3 if self.gated else 2) * H * I * x.element_size()
             plan = ctx.scratch[key] = (

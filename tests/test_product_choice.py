@@ -144,6 +144,31 @@ def test_tiles_of_16_for_an_expert_of_every_token():
     assert ops.moe_shared_tile_rows(128, 128, (4096, 4096), True, 128, 16) == 0
 
 
+@pytest.mark.parametrize("E,top,H,I,wanted", [
+    (32, 4, 2048, 2048, {1: 16, 64: 16, 96: 64, 180: 64, 500: 128, 831: 128, 1000: 384, 2048: 384}),
+    (128, 8, 2048, 1024, {130: 64, 160: 64, 640: 128, 2048: 384}),
+    (16, 2, 4096, 4096, {48: 16, 64: 64, 511: 128, 800: 0, 1024: 0, 1500: 0}),
+    (256, 8, 2048, 512, {129: 16, 150: 16, 180: 64}),
+    (512, 1, 4096, 4096, {40: 16, 129: 0, 200: 0})])
+def test_when_an_expert_of_every_token_joins_beside_another_branch(E, top, H, I, wanted):
+    """More often than on one stream, but not in tiles of 16 that read its matrices again and again, nor large matrices over many tokens."""
+    from types import SimpleNamespace
+
+    from kvcore_amd.ops import library as ops
+    from kvcore_amd.parts.moe import RoutedExperts
+
+    part = RoutedExperts(hidden_size=H, experts=E, top=top, expert_size=I, limit=None, shared_size=I)
+    x = torch.empty(1, 8, dtype=torch.bfloat16)
+    for T, want in wanted.items():
+        ctx = SimpleNamespace(num_tokens=T, scratch={}, buffers=SimpleNamespace(token_capacity=4096))
+        tile_rows, joined, max_tiles, most_tiles, *_ = part._plan(x, ctx, True, True)
+        assert (tile_rows if joined else 0) == want, T
+        assert max_tiles == ops.moe_max_tiles(T * top, E, tile_rows, T if joined else 0) <= most_tiles
+        alone = part._plan(x, ctx, False, True)
+        assert not alone[1] and alone[3] == ops.moe_max_tiles(4096 * top, E, 16, 0)
+        assert part._plan(x, ctx, True, True) is ctx.scratch[("routed_experts", E, H, I, top, True, True, True)]
+
+
 def _mixers():
     from kvcore_amd.parts.linear_attention import GatedLinearAttention, MaxGatedMatrixMemory
     from kvcore_amd.parts.recurrent import StateSpaceMixer
