@@ -1584,9 +1584,11 @@ extern "C" int kvc_moe_one_tile_rows(int pairs, int E, int H, int I, int gated) 
 }
 
 // us that the expert of every one of T tokens takes in tiles of 16 beside the routed ones: its matrices once, at the rate of theirs,
-// and again for every further tile (a die's L2 holds less than they are); and in two products of its own.
+// and again for every further tile (a die's L2 holds less than they are); and in two products of its own, which reach
+// the memory's rate where matrices are large (taken for 20 + mb / 2.8 us throughout, 48 tokens of 16 experts of 2048 x 8192 joined in tiles
+// of 16 for 360 us a layer, 350 alone).
 static double shared_in_few_us(double mb, int T) { return mb / 6.6 + (shared_tiles(T, kTileRows) - 1) * mb / 6.2; }
-static double shared_alone_us(double mb, int T) { return T <= 16 ? 8.6 + mb / 6.4 : 20 + mb / 2.8; }
+static double shared_alone_us(double mb, int T) { return T <= 16 ? 8.6 + mb / 6.4 : fmin(20 + mb / 2.8, 28 + mb / 6); }
 
 // Whether the expert that every one of T tokens runs joins the routed experts' launches, and in tiles of how many rows all of
 // them then go (0: it stays with products of its own), where tile_rows is what they would take alone.
@@ -1601,6 +1603,7 @@ static double shared_alone_us(double mb, int T) { return T <= 16 ? 8.6 + mb / 6.
 //   64 of 2048 x 2048, 4 a token  64 tokens 320 / 306 (16)   96 351 / 339 / 332   128 373 / 369 / 355   160 378 / 399 / 375
 //   24 of 3072 x 3072, 4 a token  64 tokens 368 / 360 (16)   96 402 / 432 / 354   128 425 / 507 / 371
 //   16 of 4096 x 4096, 2 a token  32 tokens 342 / 340 (16)   48 380 / 374 / 374   64 396 / 414 / 404    96 425 / 498 / 441   128 461 / 582 / 456
+//   16 of 2048 x 8192, 2 a token  40 tokens 340 / 349 (16)   48 350 / 360 (16)    96 438 / 464 / 412   128 455 / 557 / 423
 //   64 of 4096 x 2048, 4 a token  64 tokens 570 / 560 (16)   96 639 / 618 / 597   128 681 / 688 / 651
 //   16 of 1024 x 1024, 4 a token  32 tokens 92 / 80 (16)     64 121 / 103 (16)    96 127 / 111 / 103
 // A step of 15 layers of 32 experts of 2048 x 2048, four a token, alone / joined in tiles of 64 / of 128 rows, us:

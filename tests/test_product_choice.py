@@ -118,6 +118,7 @@ def test_tiles_of_384_rows_for_experts_in_one_tile_need_blocks_for_every_unit():
 @pytest.mark.parametrize("E,top,H,I,wanted", [
     (32, 4, 2048, 2048, {1: 16, 32: 16, 64: 16, 72: 16, 96: 0, 128: 0, 180: 0, 300: 64, 500: 0, 800: 0, 831: 0, 1962: 0}),
     (24, 4, 3072, 3072, {1: 16, 64: 16, 96: 64, 128: 64, 300: 384, 800: 384}),
+    (16, 2, 2048, 8192, {1: 16, 32: 16, 40: 0, 48: 0, 96: 0}),
     (16, 2, 4096, 4096, {1: 16, 48: 16, 64: 0, 96: 0, 128: 0}),
     (64, 4, 2048, 2048, {1: 16, 64: 16, 128: 16, 160: 0}),
     (64, 4, 4096, 2048, {1: 16, 96: 16, 128: 0}),
@@ -149,7 +150,7 @@ def test_tiles_of_16_for_an_expert_of_every_token():
     (128, 8, 2048, 1024, {130: 64, 160: 64, 640: 128, 2048: 384}),
     (16, 2, 4096, 4096, {48: 16, 64: 64, 511: 128, 800: 0, 1024: 0, 1500: 0}),
     (256, 8, 2048, 512, {129: 16, 150: 16, 180: 64}),
-    (512, 1, 4096, 4096, {40: 16, 129: 0, 200: 0})])
+    (512, 1, 4096, 4096, {32: 16, 40: 0, 129: 0, 200: 0})])
 def test_when_an_expert_of_every_token_joins_beside_another_branch(E, top, H, I, wanted):
     """More often than on one stream, but not in tiles of 16 that read its matrices again and again, nor large matrices over many tokens."""
     from types import SimpleNamespace
