@@ -37,11 +37,33 @@ from kvcore_amd.registry import resolve_architecture
 from .context import CacheGroupView, SideStream, StepBuffers, StepContext
 
 
-# Tokens from which a step that is not captured runs two branches of a layer side by side.  A fork and a join cost the host some
-# 35 us a layer, so that a step that waits for its launches gets slower; layers of linear attention or window attention beside 32 routed
-# experts, off / on, ms: 300 tokens 4.64 / 4.87, 700 6.04 / 5.10, 1,000 6.69 / 6.05, 2,048 10.4 / 9.0, three prompts of 683 9.3 / 8.2.  In a
-# captured step they cost a few us and it is always done: 1 token 1,127 / 991 us, 8 2,200 / 2,021, 64 3,701 / 3,427.
+# Where a step runs two branches of a layer side by side.
+# Not captured: a fork and a join cost the host some 35 to 80 us a layer, so that a step that waits for its launches gets slower (some
+# 240 us a layer by itself).  It does not from SIDE_TOKENS tokens on where a layer's kernels take SIDE_LAYER us by the estimate of
+# ``branches_pay`` (its rates fit one stream's steps of 640 to 4,096 tokens at the sizes below within some 20%).  One stream / two, ms:
+#   32 experts of 2048 x 2048, 16 layers   300 tokens 4.64 / 4.87, 640 5.66 / 4.62, 1,000 6.70 / 5.93, 2,048 10.1 / 8.9, three prompts of 683 9.2 / 8.1
+#   16 of 1024 x 1024, 8 layers            640 1.65 / 1.97 to 2.3, 1,000 1.88 / 2.0 to 2.3, 1,250 2.07 / 2.34, 1,500 2.50 / 2.42, 2,048 2.83 / 2.43
+#   128 of 2048 x 1024, 8 layers           640 4.40 / 3.56;   16 of 4096 x 4096   640 4.72 / 4.17
+# Captured: a branch waits some 6 us for a signal at either end, which small experts do not bring in: from SIDE_BYTES of their weights
+# a layer on.  us: 16 of 1024 x 1024, one token (31 MB) 388 / 382 to 411, two (46 MB) 414 / 391 to 404, eight 490 / 442, 64 875 / 717;
+# 32 of 2048 x 2048, one token (126 MB) 1,120 / 965, 8 2,190 / 1,895, 64 3,690 / 3,280.
 SIDE_TOKENS = 640
+SIDE_LAYER = 300.0
+SIDE_BYTES = 40e6
+
+
+def branches_pay(blocks, tokens: int, itemsize: int, captured: bool) -> bool:
+    """Whether a step of so many tokens runs the two branches of ``blocks`` that have two side by side: their mean decides."""
+    if not captured and tokens < SIDE_TOKENS:
+        return False
+    costs = [block.ffn.beside_cost(tokens, itemsize) for block in blocks if block.has_branches]
+    if not costs:
+        return False
+    read, ops_done = (sum(part) / len(costs) for part in zip(*costs))
+    if captured:
+        return read >= SIDE_BYTES
+    # small kernels, the experts' weights and operations, and what a mixer takes a token
+    return 70 + read / 5.5e6 + ops_done / 1.2e9 + 0.1 * tokens >= SIDE_LAYER
 
 
 @dataclass
@@ -476,7 +498,7 @@ class ModelRunner:
             dtype=self.dtype, device=self.device,
             host_query_lens=q_lens, host_seq_lens=seq_lens,
             max_query_len=max_q, max_seq_len=max_seq,
-            side=self._side if graph or T >= SIDE_TOKENS else None,
+            side=self._side if self._side is not None and branches_pay(self.model.blocks, T, self.dtype.itemsize, graph) else None,
         )
 
     def _run_decode_bucket(self, bucket: int, num_live: int, max_seq_len: int) -> torch.Tensor:

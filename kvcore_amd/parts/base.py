@@ -290,7 +290,7 @@ class FeedForward(Part):
     ``ops.WeightedRows``, for a block whose next kernel adds them up.  ``runs_beside``: that method also takes ``fork`` and
     ``beside``, calls the one and then the other, which launches another branch on a second stream behind what ``fork`` marks, and
     launches nothing of the vendor library's from there on; and ``forward_into`` and ``forward_into_normed`` take
-    the ``rows`` that it returned.  A part that says nothing is handed none of these."""
+    the ``rows`` that it returned.  A part that says nothing is handed none of these.  ``beside_cost`` is then what a step costs it."""
 
     takes_scaled_rows = False
     takes_sink = False
@@ -300,6 +300,11 @@ class FeedForward(Part):
 
     def forward(self, x: torch.Tensor, ctx: "StepContext", call: "LayerCall") -> torch.Tensor:
         raise NotImplementedError
+
+    def beside_cost(self, tokens: int, itemsize: int) -> tuple[float, float]:
+        """About how many bytes of weights a step of so many tokens reads, of so many bytes a value, and how many operations it does,
+        for whoever decides whether two branches side by side are worth a fork and a join."""
+        return 0.0, 0.0
 
 
 class Block(Part):

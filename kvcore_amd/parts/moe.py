@@ -159,6 +159,11 @@ class RoutedExperts(FeedForward):
                         accumulate=into is not None, add1_gate=rows.add_gate, count=rows.count)
         return out
 
+    def beside_cost(self, tokens: int, itemsize: int) -> tuple[float, float]:
+        E, each = self.experts, (3 if self.gated else 2) * self.hidden_size
+        read = (E * -math.expm1(-tokens * self.top / E)) * self.expert_size + self.shared_size
+        return read * each * itemsize, 2.0 * tokens * each * (self.top * self.expert_size + self.shared_size)
+
     def _plan(self, x, ctx, fits: bool, beside: bool) -> tuple[int, bool, int, int, int, bool]:
         """What a step's size decides, once for all layers of these sizes: rows a tile, whether the shared expert joins, how many
         tiles there may be in this step and in any, the floats a token that the spread router wants (0: the other one), and whether

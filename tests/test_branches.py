@@ -200,3 +200,34 @@ def test_the_requests_whose_scans_leave_units_to_the_other_stream():
     assert GatedDeltaRule._chains(beside, below=300) == 1  # the longer ones go in chunks
     assert GatedDeltaRule._chains(SimpleNamespace(side=None, host_query_lens=lengths)) == 0
     assert GatedDeltaRule._chains(SimpleNamespace(side=object(), host_query_lens=[1] * 8)) == 0
+
+
+def blocks_of(layers):
+    return [ParallelResidualBlock(mixer=DoublingMixer([]), ffn=RoutedExperts(hidden_size=H, experts=E, top=top, expert_size=I, limit=None,
+                                                                             shared_size=I), norms={"n": CopyNorm()})
+            for E, top, H, I in layers]
+
+
+def test_where_two_branches_are_worth_a_fork_and_a_join():
+    """Not captured: where a layer's kernels take longer than the host for its launches and the fork; captured: from some weights on."""
+    from kvcore_amd.engine.runner import SIDE_TOKENS, branches_pay
+
+    small, middle = blocks_of([(16, 4, 1024, 1024)] * 8), blocks_of([(32, 4, 2048, 2048)] * 16)
+    for blocks, wanted in ((small, {640: False, 1000: False, 1250: False, 2048: True, 4096: True}),
+                           (middle, {300: False, SIDE_TOKENS - 1: False, SIDE_TOKENS: True, 2048: True}),
+                           (blocks_of([(128, 8, 2048, 1024)]), {639: False, 640: True}),
+                           (blocks_of([(16, 2, 4096, 4096)]), {640: True})):
+        assert {T: branches_pay(blocks, T, 2, False) for T in wanted} == wanted
+    assert {T: branches_pay(small, T, 2, True) for T in (1, 2, 8, 64)} == {1: False, 2: True, 8: True, 64: True}
+    assert branches_pay(middle, 1, 2, True) and branches_pay(small, 1, 4, True)
+    plain = ParallelResidualBlock(mixer=DoublingMixer([]), ffn=AddingFeedForward([]), norms={"n": CopyNorm()})
+    assert not branches_pay([plain], 4096, 2, False) and not branches_pay([plain], 64, 2, True)
+    assert branches_pay([plain, *middle], 4096, 2, False)  # a block without branches has no say
+
+
+def test_what_a_step_of_routed_experts_reads_and_multiplies():
+    gated = RoutedExperts(hidden_size=8, experts=4, top=2, expert_size=16, limit=None, shared_size=24)
+    read, ops_done = gated.beside_cost(10_000, 2)
+    assert read == pytest.approx(3 * 8 * (4 * 16 + 24) * 2) and ops_done == 2 * 10_000 * 3 * 8 * (2 * 16 + 24)
+    plain = RoutedExperts(hidden_size=8, experts=4, top=2, expert_size=16, limit=None, activation="relu_squared")
+    assert plain.beside_cost(10_000, 4)[0] == pytest.approx(2 * 8 * 4 * 16 * 4)
