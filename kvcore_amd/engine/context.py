@@ -105,14 +105,18 @@ class SideStream:
 
     The runtime deals its streams to a few hardware queues, and work on two streams of one queue runs one after the
     other: so the stream is the first of some that is seen to work while the current one is busy (a prompt of 2,048 tokens
-    over routed experts takes 9.0 ms so, 10.5 with a stream of the same queue and 10.4 without any)."""
+    over routed experts takes 9.0 ms so, 10.5 with a stream of the same queue and 10.4 without any).  Where none is (``apart``
+    False) a step that is not captured runs its branches one after the other on the current stream, as the layers plan them for two: what a
+    step computes depends on its sizes and not on which queue a stream was given."""
 
     def __init__(self, device: torch.device) -> None:
         self.device = device
+        self.apart = False
         with torch.cuda.device(device):
             for _ in range(8):
                 self.stream = torch.cuda.Stream(device)
-                if self._works_beside():
+                self.apart = self._works_beside()
+                if self.apart:
                     break
         self._forked, self._done = torch.cuda.Event(), torch.cuda.Event()
         self._started = False
@@ -134,10 +138,16 @@ class SideStream:
         busy.synchronize()
         return beside
 
+    def _in_line(self) -> bool:
+        return not self.apart and not torch.cuda.is_current_stream_capturing()
+
     def fork(self) -> None:
-        self._forked.record(torch.cuda.current_stream(self.device))
+        if not self._in_line():
+            self._forked.record(torch.cuda.current_stream(self.device))
 
     def branch(self, work):
+        if self._in_line():
+            return work()
         current = torch.cuda.current_stream(self.device)
         self._forked.wait(self.stream)
         self._started = True

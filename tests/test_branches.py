@@ -82,27 +82,34 @@ def test_the_streams_are_joined_when_the_experts_raise():
     assert log == ["fork", "branch", "mixer", "experts", "join"]
 
 
-def test_a_join_waits_for_the_branch_that_was_started_last_and_for_nothing_else(monkeypatch):
-    log = []
+class Event:
+    def __init__(self, name, log):
+        self.name, self.log = name, log
 
-    class Event:
-        def __init__(self, name):
-            self.name = name
+    def record(self, stream=None):
+        self.log.append((self.name, "record", stream))
 
-        def record(self, stream=None):
-            log.append((self.name, "record", stream))
+    def wait(self, stream=None):
+        self.log.append((self.name, "wait", stream))
 
-        def wait(self, stream=None):
-            log.append((self.name, "wait", stream))
 
+def side_stream(monkeypatch, log, beside=True):
+    """A ``SideStream`` over streams and events that only note what is asked of them; the current stream is "main"."""
+    made = []
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: "main")
     monkeypatch.setattr(torch.cuda, "set_stream", lambda stream: log.append(stream))
-    monkeypatch.setattr(SideStream, "_works_beside", lambda self: True)
-    monkeypatch.setattr(torch.cuda, "Stream", lambda device=None: "side")
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: "capturing" in made)
+    monkeypatch.setattr(SideStream, "_works_beside", lambda self: beside)
+    monkeypatch.setattr(torch.cuda, "Stream", lambda device=None: made.append("side") or "side")
     monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
-    events = iter((Event("forked"), Event("done")))
+    events = iter((Event("forked", log), Event("done", log)))
     monkeypatch.setattr(torch.cuda, "Event", lambda: next(events))
-    side = SideStream(torch.device("cpu"))
+    return SideStream(torch.device("cpu")), made
+
+
+def test_a_join_waits_for_the_branch_that_was_started_last_and_for_nothing_else(monkeypatch):
+    log = []
+    side, _ = side_stream(monkeypatch, log)
 
     def fails():
         raise ValueError("in the branch")
@@ -116,6 +123,26 @@ def test_a_join_waits_for_the_branch_that_was_started_last_and_for_nothing_else(
     side.join()
     side.join()
     assert log == [("forked", "wait", "side"), "side", ("done", "record", "side"), "main", ("done", "wait", "main")]
+
+
+def test_where_no_stream_works_beside_the_current_one(monkeypatch):
+    """Branches run in line, one after the other, but for captured steps, whose graph has branches of its own."""
+    log = []
+    side, made = side_stream(monkeypatch, log, beside=False)
+    assert not side.apart and len(made) == 8
+    side.fork()
+    assert side.branch(lambda: log.append("work") or 7) == 7
+    side.join()
+    assert log == ["work"]
+    log.clear()
+    made.append("capturing")
+    side.fork()
+    side.branch(lambda: log.append("work"))
+    side.join()
+    assert log == [("forked", "record", "main"), ("forked", "wait", "side"), "side", "work", ("done", "record", "side"), "main",
+                   ("done", "wait", "main")]
+    side, made = side_stream(monkeypatch, log)
+    assert side.apart and len(made) == 1
 
 
 def test_experts_beside_a_mixer_take_the_rows_that_they_have_made():
