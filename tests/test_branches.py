@@ -93,9 +93,9 @@ class Event:
         self.log.append((self.name, "wait", stream))
 
 
-def side_stream(monkeypatch, log, beside=True):
+def side_stream(monkeypatch, log, beside=True, made=None):
     """A ``SideStream`` over streams and events that only note what is asked of them; the current stream is "main"."""
-    made = []
+    made = [] if made is None else made
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: "main")
     monkeypatch.setattr(torch.cuda, "set_stream", lambda stream: log.append(stream))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: "capturing" in made)
@@ -136,6 +136,7 @@ def test_where_no_stream_works_beside_the_current_one(monkeypatch):
     assert log == ["work"]
     log.clear()
     made.append("capturing")
+    side.begin_capture()
     side.fork()
     side.branch(lambda: log.append("work"))
     side.join()
@@ -143,6 +144,30 @@ def test_where_no_stream_works_beside_the_current_one(monkeypatch):
                    ("done", "wait", "main")]
     side, made = side_stream(monkeypatch, log)
     assert side.apart and len(made) == 1
+
+
+def test_a_process_captures_so_many_steps_with_branches(monkeypatch):
+    log = []
+    monkeypatch.setattr(SideStream, "_graphs", 0)
+    monkeypatch.setattr(SideStream, "MOST_GRAPHS", 2)
+    side, made = side_stream(monkeypatch, log)
+    other, _ = side_stream(monkeypatch, log, made=made)
+    ways = []
+    for s in (side, other, side, other):
+        made.append("capturing")
+        s.begin_capture()
+        log.clear()
+        s.fork()
+        s.branch(lambda: None)
+        s.join()
+        ways.append(bool(log))
+        made.remove("capturing")
+        log.clear()
+        s.fork()  # a step that is not captured
+        s.branch(lambda: None)
+        s.join()
+        assert log
+    assert ways == [True, True, False, False]
 
 
 def test_experts_beside_a_mixer_take_the_rows_that_they_have_made():
