@@ -107,8 +107,8 @@ class SideStream:
     The runtime deals its streams to a few hardware queues, and work on two streams of one queue runs one after the
     other: so the stream is the first of some that is seen to work while the current one is busy (a prompt of 2,048 tokens
     over routed experts takes 9.0 ms so, 10.5 with a stream of the same queue and 10.4 without any).  Where none is (``apart``
-    False) a step that is not captured runs its branches one after the other on the current stream, as the layers plan them for two: what a
-    step computes depends on its sizes and not on which queue a stream was given.
+    False) a step that is not captured runs its branches one after the other on the current stream, as the layers plan them for two (up to 5% more than
+    with the plan for one): what a step computes depends on its sizes and not on which queue a stream was given.
 
     A process captures at most ``MOST_GRAPHS`` steps with branches, further ones in line: a process that had captured, replayed and dropped some 185 of
     them (and 150 without) ended with a segmentation fault, the cause of which is not known; 624 without branches and 84 with passed."""

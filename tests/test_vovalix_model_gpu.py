@@ -11,7 +11,7 @@ import torch
 from tests.helpers import random_tokens
 from tests.plain import vovalix as plain
 from tests.test_cuts_gpu import collect
-from tests.vovalix_helpers import CONFIGS, make_model_dir
+from tests.vovalix_helpers import CONFIG_E, CONFIGS, make_model_dir
 
 pytestmark = pytest.mark.gpu
 
@@ -393,3 +393,57 @@ def test_branches_side_by_side_with_the_experts_launched_first(models, name, mon
     """The same where the experts are taken for the longer branch, as they are in larger models."""
     monkeypatch.setattr("kvcore_amd.parts.moe.LONG_BRANCH_BYTES", 0)
     test_branches_side_by_side_give_the_bits_of_one_after_the_other(models, name, torch.bfloat16, monkeypatch)
+
+
+def joined_in_tiles(monkeypatch, tile_rows):
+    """The rules that choose tiles made to answer so many rows, and the shared expert to join them; the launches that it joined."""
+    from kvcore_amd.ops import library as ops
+
+    monkeypatch.setattr(ops, "moe_wide_tile_rows", lambda *of: 384 if tile_rows == 384 else 0)
+    monkeypatch.setattr(ops, "moe_one_tile_rows", lambda *of: 0)
+    monkeypatch.setattr(ops, "moe_tile_rows", lambda *of: tile_rows)
+    monkeypatch.setattr(ops, "moe_shared_tile_rows", lambda pairs, experts, sizes, gated, tokens, alone, beside=False: alone)
+    product, joined = ops.moe_gemm, []
+
+    def noting(*args, **kwargs):
+        joined.append((kwargs["shared_rows"], kwargs["tile_rows"], torch.cuda.is_current_stream_capturing()))
+        return product(*args, **kwargs)
+
+    monkeypatch.setattr(ops, "moe_gemm", noting)
+    return joined
+
+
+@pytest.mark.parametrize("tile_rows", [16, 64, 128, 384])
+def test_a_shared_expert_joins_the_others_beside_a_mixer(tmp_path, monkeypatch, tile_rows):
+    """A prompt and captured steps of two requests with the shared expert among the routed ones and the mixer on the second stream, against
+    the plain model, and bit by bit against the same steps in line."""
+    from kvcore_amd.engine.context import SideStream
+    from kvcore_amd.engine.runner import SIDE_TOKENS
+
+    folder = make_model_dir(tmp_path / "e", CONFIG_E, seed=71)
+    cfg, weights = plain.load_model_folder(folder)
+    n = SIDE_TOKENS + 61
+    seqs = {"a": random_tokens(n + 6, cfg["vocab"], 9), "b": random_tokens(9, cfg["vocab"], 10)}
+    want = {k: oracle("E", cfg, weights, v) for k, v in seqs.items()}
+    joined = joined_in_tiles(monkeypatch, tile_rows)
+    monkeypatch.setattr("kvcore_amd.engine.runner.branches_pay", lambda *of: True)
+    got = []
+    for beside in (True, False):
+        if not beside:
+            monkeypatch.setattr(SideStream, "MOST_GRAPHS", 0)
+        s = session_for(folder, torch.bfloat16, 16, 1536)
+        if not beside:
+            s.runner._side.apart = False
+        joined.clear()
+        steps = [{"step": 0, "entries": [{"id": "a", "tokens": seqs["a"][:n], "want": [0, 17, 300, n - 1]},
+                                         {"id": "b", "tokens": seqs["b"][:3], "want": [2]}], "end": []}]
+        steps += [{"step": 1 + i, "entries": [{"id": "a", "tokens": [seqs["a"][n + i]], "want": [0]},
+                                              {"id": "b", "tokens": [seqs["b"][3 + i]], "want": [0]}], "end": []} for i in range(6)]
+        got.append(collect(s, steps))
+        assert s.runner.graph_replays >= 4
+        # both products of every layer: the prompt's, a step launched and a step captured
+        assert joined == [(n + 3, tile_rows, False)] * 6 + [(2, tile_rows, False)] * 6 + [(2, tile_rows, True)] * 6
+    compare(got[0], want, torch.bfloat16)
+    assert got[0].keys() == got[1].keys()
+    for key, row in got[0].items():
+        assert torch.equal(row, got[1][key]), key

@@ -253,6 +253,23 @@ def test_small_kernels_around_the_recurrences():
     assert rel(out, gg * torch.sigmoid(1.702 * gg) * (uu + 1)) < 1e-6
 
 
+@pytest.mark.parametrize("act", ["sigmoid", "silu"])
+def test_sigmoid_and_silu_have_the_division_s_bits_for_every_float32(act):
+    """All 2^32 values as gates of rows whose norm is one: a reciprocal and a correction in the kernel, a division here."""
+    from kvcore_amd.ops import library as ops
+
+    T, heads, dim = 65536, 16, 64
+    ones, gain = torch.ones(T, heads * dim, device=DEV), torch.ones(dim, device=DEV)
+    out = torch.empty_like(ones)
+    count = ones.numel()
+    for first in range(-2 ** 31, 2 ** 31, count):
+        gate = torch.arange(first, first + count, dtype=torch.int64, device=DEV).to(torch.int32).view(torch.float32).view(T, -1)
+        ops.head_rmsnorm_gate(out, ones, gate, gain, 0.0, heads, dim, act=act)
+        want = (gate if act == "silu" else ones) / (1.0 + torch.exp(-gate))
+        same = (out.view(torch.int32) == want.view(torch.int32)) | (out.isnan() & want.isnan())
+        assert bool(same.all()), (first, gate[~same][:4].tolist(), out[~same][:4].tolist(), want[~same][:4].tolist())
+
+
 # ------------------------------------------------------------------------- attention
 def paged(q, k, v, page, *, scale, slopes, chunk, dtype, positions=None, shuffle=True, kernel="general"):
     """Attention of ``q [T, H, d]`` (tokens at ``positions``, default 0..T-1) over keys and values
@@ -527,6 +544,69 @@ def test_the_feed_forward_of_routed_experts(dtype, E, top, groups, keep, H, I, s
         perm = torch.randperm(T, generator=gen)
         again = part.forward(gpu(x[perm], dtype), ctx, None)
         assert rel(again, first[perm].double()) < 1e-6
+
+
+@pytest.mark.parametrize("gated", [True, False], ids=["gated", "plain"])
+@pytest.mark.parametrize("tile_rows", [16, 64, 128, 384])
+@pytest.mark.parametrize("T", [1, 129, 700])
+def test_experts_with_a_shared_one_of_their_size_beside_another_branch(monkeypatch, T, tile_rows, gated):
+    """The part with its shared expert in the routed ones' launches, with and without another branch: the same bits, each against the
+    weighted sum in 64 bits; the branch starts behind the mark."""
+    from kvcore_amd.engine.context import StepBuffers, StepContext
+    from kvcore_amd.ops import library as ops
+    from kvcore_amd.parts.base import Runtime
+    from kvcore_amd.parts.moe import RoutedExperts
+
+    E, top, H, I = 6, 2, 192, 128
+    gen = torch.Generator().manual_seed(T + tile_rows)
+    part = RoutedExperts(hidden_size=H, experts=E, top=top, expert_size=I, limit=1.2, shared_size=I, shared_limit=0.8,
+                         activation=None if gated else "relu_squared")
+    part.setup(Runtime(dtype=torch.bfloat16, device=torch.device(DEV)))
+    params = {}
+    for ps in part.param_specs():
+        t = torch.randn(ps.shape, generator=gen) * ps.shape[1] ** -0.5
+        params[ps.name] = gpu(t, torch.float32 if ps.kind == "vector" else torch.bfloat16)
+    part.bind(params)
+    x = gpu(torch.randn(T, H, generator=gen), torch.bfloat16)
+    monkeypatch.setattr(ops, "moe_wide_tile_rows", lambda *of: 384 if tile_rows == 384 else 0)
+    monkeypatch.setattr(ops, "moe_one_tile_rows", lambda *of: 0)
+    monkeypatch.setattr(ops, "moe_tile_rows", lambda *of: tile_rows)
+    monkeypatch.setattr(ops, "moe_shared_tile_rows", lambda pairs, experts, sizes, gated, tokens, alone, beside=False: alone)
+    none = torch.zeros(1, dtype=torch.int32, device=DEV)
+    called, got = [], []
+    for longer in (None, False, True):
+        monkeypatch.setattr("kvcore_amd.parts.moe.LONG_BRANCH_BYTES", 0 if longer else 1e18)
+        ctx = StepContext(num_tokens=T, num_reqs=1, token_ids=none, positions=none, token_req=none, q_start=none,
+                          seq_lens=none, slots=none, groups=[], states=[], buffers=StepBuffers(torch.device(DEV), token_capacity=T),
+                          dtype=torch.bfloat16, device=torch.device(DEV))
+        branch = {} if longer is None else dict(fork=lambda: called.append("fork"), beside=lambda: called.append("beside"))
+        rows = part.forward_weighted(x, ctx, None, **branch)
+        assert rows.data.shape[0] == T * (top + 1) and rows.add.shape == (T, H) and rows.add.data_ptr() == rows.data[T * top:].data_ptr()
+        out = torch.empty(T, H, device=DEV)
+        ops.moe_combine(out, rows.data, rows.weight, None, rows.add, add1_gate=rows.add_gate, count=rows.count)
+        got.append((out, rows.weight.clone(), ctx.buffers.get(f"moe_choice:{top}", T, top, torch.int32)))
+    assert called == ["fork", "beside"] * 2
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][0], got[2][0])
+
+    w = {k: v.double().cpu() for k, v in params.items()}
+    xs = x.double().cpu()
+
+    def expert(rows, first, down, limit):
+        h = rows @ first.T
+        if gated:
+            g, u = h[:, :I].clamp(max=limit), h[:, I:].clamp(-limit, limit)
+            h = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            h = h.clamp(min=0) ** 2
+        return h @ down.T
+
+    want = expert(xs, w[f"shared.{part.first}"], w["shared.down"], 0.8)
+    weight, choice = got[0][1].double().cpu(), got[0][2].cpu()
+    per = w[f"experts.{part.first}"].shape[0] // E
+    for e in range(E):
+        rows = expert(xs, w[f"experts.{part.first}"][e * per:(e + 1) * per], w["experts.down"][e * H:(e + 1) * H], 1.2)
+        want += rows * (weight * (choice == e)).sum(1, keepdim=True)
+    assert rel(got[0][0], want) < 3e-3  # one rounding of the activations to bfloat16, float32 sums
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])

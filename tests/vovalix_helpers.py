@@ -94,6 +94,17 @@ CONFIG_D = {
     ],
 }
 
+# shared experts of the routed ones' size, which may join their launches; widths that tiles of every size serve
+_MOE_E = _moe(8, 3, 64, 2.0, groups=(4, 2), shared=(64, 1.0))
+CONFIG_E = {
+    "architecture": "Vovalix", "vocab": 256, "width": 128, "norm": {"eps": 1e-6}, "logit_scale": 1.0,
+    "layers": [
+        {"type": "delta", "mixer": _delta(2, 2, 64, 64, 4), "mlp": _MOE_E},
+        {"type": "attention", "mixer": _attn(4, 2, 64, 64, 0.125, 48), "mlp": _MOE_E},
+        {"type": "gla", "mixer": _gla(2, 64, 64, 8.0, 16), "mlp": _MOE_E},
+    ],
+}
+
 CONFIGS = {"A": (CONFIG_A, 8), "B": (CONFIG_B, 16), "C": (CONFIG_C, 4), "D": (CONFIG_D, 16)}
 
 
