@@ -75,8 +75,9 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(
 // once, and the window of the last K inputs slides along in registers, so that a token costs
 // one load of x and one store.  Where all eight and the K - 1 inputs before them are one request's of this
 // step, as nearly everywhere in a prompt, all inputs are asked for at once: token by token, each behind the
-// loads of its request and position, 2,048 tokens of 6,144 channels took 33 us, this way 25, and with four taps known
-// to the compiler and the division of silu as a reciprocal and a correction (device_utils.h) 22 (75 MB: 12 us).
+// loads of its request and position, 2,048 tokens of 6,144 channels took 33 us in a step, this way 26.5, and with four taps known
+// to the compiler and the division of silu as a reciprocal and a correction (device_utils.h) 23.3 (75 MB: 12 us; the same rows
+// again and again 18.9, float32 on either side 21.4).
 constexpr int kConvTokens = 8, kConvMaxTaps = 8;
 // TAPS: as many as there are; 0: up to kConvMaxTaps.
 template <typename TI, typename TO, int TAPS>

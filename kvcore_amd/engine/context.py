@@ -105,8 +105,8 @@ class SideStream:
     fork and join neither branch writes what the other one touches.  In a captured step they become branches of the graph.
 
     The runtime deals its streams to a few hardware queues, and work on two streams of one queue runs one after the
-    other: so the stream is the first of some that is seen to work while the current one is busy (a prompt of 2,048 tokens
-    over routed experts takes 9.0 ms so, 10.5 with a stream of the same queue and 10.4 without any).  Where none is (``apart``
+    other: so the stream is the first of some that is seen to work while the current one is busy (prompts of 2,048 tokens
+    over routed experts, back to back, take 8.9 ms so and 10.1 without any; 10.5 was seen with a stream of the same queue).  Where none is (``apart``
     False) a step that is not captured runs its branches one after the other on the current stream, as the layers plan them for two (up to 5% more than
     with the plan for one): what a step computes depends on its sizes and not on which queue a stream was given.
 

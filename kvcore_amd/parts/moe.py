@@ -40,8 +40,10 @@ GLU_ALPHA = 1.702
 # both for its last one where that is the later.  So the longer branch is launched first: a mixer of few tokens takes some 38 us, in which
 # this many bytes are read.  Captured steps of 16 layers of 32 experts of 2048 x 2048, mixer / router first: 1 token 948 / 990 us, 2 (203 MB)
 # 1,165 / 1,187, 3 (277 MB) 1,383 / 1,343, 4 1,512 / 1,464, 8 2,015 / 1,897, 16 2,568 / 2,424, 32 2,907 / 2,830, 64 3,490 / 3,250,
-# 128 3,957 / 3,763; the mixer only behind the experts' products 8 1,923, 64 3,322.  Steps that are not captured do not care (three prompts of 683
-# 7,700 / 7,700).
+# 128 3,957 / 3,763; the mixer only behind the experts' products 8 1,923, 64 3,322.  Eight layers of other sizes: 16 of 1024 x 1024 8 tokens (94 MB)
+# 437 / 459, 160 (107 MB) 806 / 822; 16 of 4096 x 4096, two a token, 1 (302 MB) 780 / 780, 8 1,865 / 1,806, 32 2,740 / 2,653; 128 of 2048 x 1024, eight
+# a token, whose router takes longer, 1 (113 MB) 884 / 828, 4 (378 MB) 1,195 / 1,126, 32 2,500 / 2,435, 64 2,785 / 2,823.  Steps that are not captured do not
+# care (three prompts of 683 7,700 / 7,700).
 LONG_BRANCH_BYTES = 240e6
 
 
