@@ -2148,10 +2148,12 @@ def moe_max_tiles(pairs: int, experts: int, tile_rows: int = 16, shared_rows: in
 
 def moe_shared_fits(w: torch.Tensor, shared: torch.Tensor, experts: int) -> bool:
     """Whether the matrix of an expert that every token runs may join a launch over the routed experts' stacked ones
-    (:func:`moe_gemm`'s ``shared``): bfloat16, of an expert's size, and stored in the same order."""
+    (:func:`moe_gemm`'s ``shared``): bfloat16, of an expert's size, stored in the same order, and rows as the kernels read them
+    (a view of another tensor may lie otherwise; products of its own take it)."""
     return (w.dtype == torch.bfloat16 and shared.dtype == torch.bfloat16
             and w.shape == (experts * shared.shape[0], shared.shape[1])
-            and (getattr(w, "kvc_packed", None) is None) == (getattr(shared, "kvc_packed", None) is None))
+            and (getattr(w, "kvc_packed", None) is None) == (getattr(shared, "kvc_packed", None) is None)
+            and shared.is_contiguous() and shared.data_ptr() % 16 == 0)
 
 
 def moe_shared_tile_rows(pairs: int, experts: int, k_sizes: tuple[int, int], gated: bool, tokens: int, tile_rows: int,

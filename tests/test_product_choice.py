@@ -135,6 +135,23 @@ def test_when_an_expert_of_every_token_joins_the_others(E, top, H, I, wanted):
         assert ops.moe_shared_tile_rows(T * top, E, (H, I), True, T, alone) == want, T
 
 
+def test_which_matrix_of_an_expert_of_every_token_fits_the_others():
+    """Of their type, size and order of storage, contiguous and 16-byte aligned: what is not stays with products of its own."""
+    from kvcore_amd.ops import library as ops
+
+    w = torch.zeros(4 * 32, 64, dtype=torch.bfloat16)
+    shared = torch.zeros(32, 64, dtype=torch.bfloat16)
+    assert ops.moe_shared_fits(w, shared, 4)
+    assert not ops.moe_shared_fits(w, shared.float(), 4) and not ops.moe_shared_fits(w.float(), shared, 4)
+    assert not ops.moe_shared_fits(w, shared[:16], 4) and not ops.moe_shared_fits(w, shared, 5)
+    assert not ops.moe_shared_fits(w, torch.zeros(64, 32, dtype=torch.bfloat16).t(), 4)
+    assert not ops.moe_shared_fits(w, torch.zeros(32, 128, dtype=torch.bfloat16)[:, :64], 4)
+    assert not ops.moe_shared_fits(w, torch.zeros(32 * 64 + 1, dtype=torch.bfloat16)[1:].view(32, 64), 4)
+    packed = shared.clone()
+    packed.kvc_packed = shared
+    assert not ops.moe_shared_fits(w, packed, 4)
+
+
 def test_tiles_of_16_for_an_expert_of_every_token():
     from kvcore_amd.ops import library as ops
 
